@@ -348,6 +348,17 @@ enum RagkEpilogue : int {
   EPI_GLU_CLIP = 9,  // paired columns: clipped gated unit; the bias pointer holds fp32 {limit, alpha, shift}
 };
 
+// Operands of EPI_ROPE_KV (head size 128).
+struct RopeKV {
+  const int* pos;
+  const int* slot;     // < 0: row not cached
+  const float* cos_t;  // [positions][64]
+  const float* sin_t;
+  bf16_t* kc;          // [blocks][Hkv][BS][128]
+  bf16_t* vc;
+  int Hq, Hkv, BS;
+};
+
 // epilogues over packed [64 gate | 64 up] weight rows (one output column per pair)
 constexpr bool epi_pair(int e) { return e == EPI_SILU_MUL || e == EPI_GLU_CLIP; }
 

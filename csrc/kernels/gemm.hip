@@ -1,21 +1,15 @@
-// bf16 GEMM family for gfx950: C[M,N] = A[M,K] . B[N,K]^T  (+ fused epilogue)
+// bf16 GEMMs of decode steps (M <= 64) for gfx950: C[M,N] = A[M,K] . B[N,K]^T  (+ fused epilogue)
 //
 // B is the HF weight layout [out_features, in_features], so both operands are
 // K-contiguous and every MFMA fragment is one 16-byte load.
 //
-// Two kernels:
-//  * gemm_tile   : prefill / encoder GEMMs (M >= 64). 128x128x64 block tile,
-//                  4 waves (2x2) of 64x64, mfma_f32_16x16x32_bf16, operands
-//                  staged global->LDS with global_load_lds (16 B/lane), XOR
-//                  swizzled rows (conflict-free ds_read_b128), double-buffered,
-//                  XCD-aware grouped tile order, LDS-staged vectorised epilogue
-//                  (bias / residual / GELU / SiLU*up fused).
-//  * gemm_skinny : decode GEMMs (M <= 64). Weight-streaming: every weight byte is
+//  * gemm_skinny : weight-streaming: every weight byte is
 //                  read exactly once straight into VGPRs (no LDS round trip), 8
 //                  waves per block split K, MFMA with the activations as the A
 //                  operand, cross-wave reduction through LDS, fused epilogue.
+//  * gemm_gemv   : the same software-pipelined (explicit path 3).
 //
-// Replaces reference ops K3/K7/K8/K9/K10/K11 (SURVEY.md §2.4; the reference
+// Replaces reference ops K3/K7/K8/K9/K10/K11 (the reference
 // runs them as fp32 ATen CPU matmuls inside transformers' LlamaForCausalLM,
 // /root/reference/llm/rag.py:24,172) and encoder ops E2/E4/E5/E6.
 #include <stdlib.h>
@@ -24,177 +18,6 @@
 using namespace ragk;
 
 namespace {
-
-constexpr int BM = 128, BN = 128, BK = 64;
-constexpr int TILE_THREADS = 256;
-constexpr int STAGE_BYTES = (BM + BN) * BK * 2;         // one buffer: A + B = 32 KiB
-constexpr int EPI_LD = BN + 4;                          // padded f32 row (conflict-free C-layout writes)
-constexpr int EPI_BYTES = BM * EPI_LD * 4;              // 67,584 B
-constexpr int TILE_LDS = (2 * STAGE_BYTES > EPI_BYTES) ? 2 * STAGE_BYTES : EPI_BYTES;
-constexpr int GROUP_M = 8;
-
-// 128-byte LDS rows (64 bf16): 8 x 16-B chunks. XOR the chunk with (row>>1)&7 so the
-// 16 lanes of each ds_read_b128 lane-group land on 16 distinct 16-B bank slots.
-__device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
-
-__device__ __forceinline__ void stage_tile(const bf16_t* __restrict__ g, int ld, int row0, int rows_valid,
-                                           int k0, char* lds_tile, int wid, int lane) {
-  // 128 rows x 128 B = 16 x 1 KiB glds pieces, 4 per wave. Lane-linear LDS
-  // destination; the swizzle is applied to the per-lane SOURCE address.
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int q = wid * 4 + i;
-    const int r = q * 8 + (lane >> 3);
-    const int p = lane & 7;
-    const int c = swz(r, p);
-    int gr = row0 + r;
-    gr = gr < rows_valid ? gr : rows_valid - 1;  // clamp: rows past the edge are never stored
-    const bf16_t* src = g + (size_t)gr * ld + k0 + c * 8;
-    glds16(src, lds_tile + q * 1024);
-  }
-}
-
-template <int EPI, bool OUT_F32>
-__global__ __launch_bounds__(TILE_THREADS, 2) void gemm_tile_kernel(
-    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ B, int ldb, void* C, int ldc,
-    const bf16_t* __restrict__ bias, const bf16_t* resid, int ldr, int M, int N, int K) {
-  __shared__ __attribute__((aligned(16))) char smem[TILE_LDS];
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int wr = wid >> 1, wc = wid & 1;
-
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  const int nwg = tiles_m * tiles_n;
-  const int logical = xcd_remap(blockIdx.x, nwg);
-  const int group = logical / (GROUP_M * tiles_n);
-  const int first_m = group * GROUP_M;
-  const int gm = min(tiles_m - first_m, GROUP_M);
-  const int in_group = logical % (GROUP_M * tiles_n);
-  const int tm = first_m + in_group % gm;
-  const int tn = in_group / gm;
-  const int m0 = tm * BM, n0 = tn * BN;
-
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  const int nk = K / BK;
-  const int wid_u = __builtin_amdgcn_readfirstlane(wid);
-
-  stage_tile(A, lda, m0, M, 0, smem, wid_u, lane);
-  stage_tile(B, ldb, n0, N, 0, smem + BM * BK * 2, wid_u, lane);
-  wait_vmcnt0();
-  __syncthreads();
-
-  const int fr = lane & 15, fh = lane >> 4;
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) {
-      char* nxt = smem + (cur ^ 1) * STAGE_BYTES;
-      stage_tile(A, lda, m0, M, (kt + 1) * BK, nxt, wid_u, lane);
-      stage_tile(B, ldb, n0, N, (kt + 1) * BK, nxt + BM * BK * 2, wid_u, lane);
-    }
-    const char* sa = smem + cur * STAGE_BYTES;
-    const char* sb = sa + BM * BK * 2;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      bf16x8 af[4], bfr[4];
-      const int c = 4 * s + fh;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int R = wr * 64 + 16 * i + fr;
-        af[i] = *reinterpret_cast<const bf16x8*>(sa + R * 128 + 16 * swz(R, c));
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int R = wc * 64 + 16 * j + fr;
-        bfr[j] = *reinterpret_cast<const bf16x8*>(sb + R * 128 + 16 * swz(R, c));
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-    }
-    wait_vmcnt0();
-    __syncthreads();
-  }
-
-  // ---- epilogue: accumulators -> padded f32 LDS tile -> 16-B row stores ----
-  float* sC = reinterpret_cast<float*>(smem);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        sC[(wr * 64 + 16 * i + 4 * fh + r) * EPI_LD + wc * 64 + 16 * j + fr] = acc[i][j][r];
-  __syncthreads();
-
-  if constexpr (epi_pair(EPI)) {
-    const GluPar gp = glu_par<EPI>(bias);
-    // packed tile = [64 gate cols | 64 up cols] -> 64 output cols
-    const int ocol0 = tn * 64;
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int v = tid + it * TILE_THREADS;  // 128 rows x 8 vec
-      const int row = v >> 3, c8 = (v & 7) * 8;
-      const int gr = m0 + row;
-      if (gr < M) {
-        float o[8];
-        const float* g = sC + row * EPI_LD + c8;
-        const float* u = g + 64;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = glu_act<EPI>(g[e], u[e], gp);
-        bf16_t* dst = reinterpret_cast<bf16_t*>(C) + (size_t)gr * ldc + ocol0 + c8;
-        *reinterpret_cast<u32x4*>(dst) = pack8(o);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int it = 0; it < 8; ++it) {
-      const int v = tid + it * TILE_THREADS;  // 128 rows x 16 vec
-      const int row = v >> 4, c8 = (v & 15) * 8;
-      const int gr = m0 + row, gc = n0 + c8;
-      if (gr < M && gc < N) {
-        float o[8];
-        const float* s = sC + row * EPI_LD + c8;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = s[e];
-        if constexpr (EPI == EPI_BIAS || EPI == EPI_BIAS_RESID || EPI == EPI_BIAS_GELU ||
-                      EPI == EPI_BIAS_GELU_TANH) {
-          float b[8];
-          unpack8(*reinterpret_cast<const u32x4*>(bias + gc), b);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) o[e] += b[e];
-        }
-        if constexpr (EPI == EPI_RESID || EPI == EPI_BIAS_RESID) {
-          float rr[8];
-          unpack8(*reinterpret_cast<const u32x4*>(resid + (size_t)gr * ldr + gc), rr);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) o[e] += rr[e];
-        }
-        if constexpr (EPI == EPI_BIAS_GELU || EPI == EPI_GELU) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) o[e] = gelu_erf(o[e]);
-        }
-        if constexpr (EPI == EPI_BIAS_GELU_TANH) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) o[e] = gelu_tanh(o[e]);
-        }
-        if constexpr (OUT_F32) {
-          float* dst = reinterpret_cast<float*>(C) + (size_t)gr * ldc + gc;
-          *reinterpret_cast<f32x4*>(dst) = (f32x4){o[0], o[1], o[2], o[3]};
-          *reinterpret_cast<f32x4*>(dst + 4) = (f32x4){o[4], o[5], o[6], o[7]};
-        } else {
-          bf16_t* dst = reinterpret_cast<bf16_t*>(C) + (size_t)gr * ldc + gc;
-          *reinterpret_cast<u32x4*>(dst) = pack8(o);
-        }
-      }
-    }
-  }
-}
 
 // ------------------------------------------------------------------------------------
 // Skinny (decode) GEMM. Block = WAVES waves handling one 16-column output tile; the
@@ -469,16 +292,6 @@ hipError_t dispatch_gemv(const void* X, int ldx, const void* W, int ldw, void* C
 #undef RAGK_GV
 }
 
-template <int EPI, bool F32>
-hipError_t launch_tile(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias,
-                       const void* resid, int ldr, int M, int N, int K, hipStream_t st) {
-  const int nwg = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  hipLaunchKernelGGL((gemm_tile_kernel<EPI, F32>), dim3(nwg), dim3(TILE_THREADS), 0, st,
-                     (const bf16_t*)A, lda, (const bf16_t*)B, ldb, C, ldc, (const bf16_t*)bias,
-                     (const bf16_t*)resid, ldr, M, N, K);
-  return hipGetLastError();
-}
-
 template <int MT, int EPI, bool F32>
 hipError_t launch_skinny(const void* X, int ldx, const void* W, int ldw, void* C, int ldc, const void* bias,
                          const void* resid, int ldr, int M, int N, int K, hipStream_t st) {
@@ -504,30 +317,22 @@ hipError_t dispatch_skinny(const void* X, int ldx, const void* W, int ldw, void*
 }  // namespace
 
 // N here is the number of OUTPUT columns. For EPI_SILU_MUL / EPI_GLU_CLIP the weight has 2*N rows
-// in the packed [64 gate | 64 up] tile layout and N must be a multiple of 64.
+// in the packed [64 gate | 64 up] tile layout and N must be a multiple of 64. M <= 64.
 RAGK_API int ragk_gemm(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias,
                        const void* resid, int ldr, int M, int N, int K, int epi, int out_f32, hipStream_t st) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  if (K % 128 != 0) return (int)hipErrorInvalidValue;
-  const bool skinny = M <= 64;
-  if (epi == EPI_SILU_MUL) {
-    if (N % 64 != 0 || out_f32) return (int)hipErrorInvalidValue;
-    if (skinny) return (int)dispatch_skinny<EPI_SILU_MUL, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
-    return (int)launch_tile<EPI_SILU_MUL, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, 2 * N, K, st);
-  }
+  if (K % 128 != 0 || M > 64) return (int)hipErrorInvalidValue;
+  if (epi_pair(epi) && (N % 64 != 0 || out_f32)) return (int)hipErrorInvalidValue;
+  if (epi == EPI_SILU_MUL)
+    return (int)dispatch_skinny<EPI_SILU_MUL, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
   if (epi == EPI_GLU_CLIP) {
-    if (N % 64 != 0 || out_f32 || !bias) return (int)hipErrorInvalidValue;
-    if (skinny) return (int)dispatch_skinny<EPI_GLU_CLIP, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
-    return (int)launch_tile<EPI_GLU_CLIP, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, 2 * N, K, st);
+    if (!bias) return (int)hipErrorInvalidValue;
+    return (int)dispatch_skinny<EPI_GLU_CLIP, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
   }
-  if (!skinny && N % 8 != 0) return (int)hipErrorInvalidValue;
 #define RAGK_GEMM_CASE(E)                                                                               \
   case E:                                                                                               \
-    if (skinny)                                                                                         \
-      return out_f32 ? (int)dispatch_skinny<E, true>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st) \
-                     : (int)dispatch_skinny<E, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st); \
-    return out_f32 ? (int)launch_tile<E, true>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st)     \
-                   : (int)launch_tile<E, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
+    return out_f32 ? (int)dispatch_skinny<E, true>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st) \
+                   : (int)dispatch_skinny<E, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
   switch (epi) {
     RAGK_GEMM_CASE(EPI_NONE)
     RAGK_GEMM_CASE(EPI_BIAS)
@@ -541,26 +346,20 @@ RAGK_API int ragk_gemm(const void* A, int lda, const void* B, int ldb, void* C, 
 #undef RAGK_GEMM_CASE
 }
 
-// Force a specific path (tests / benchmarks): path 0 = tile, 1 = skinny v1, 3 = pipelined gemv v2.
+// Force a specific path (tests / benchmarks): path 1 = skinny v1, 3 = pipelined gemv v2.
 RAGK_API int ragk_gemm_path(int path, const void* A, int lda, const void* B, int ldb, void* C, int ldc,
                             const void* bias, const void* resid, int ldr, int M, int N, int K, int epi,
                             hipStream_t st) {
-  if (K % 128 != 0) return (int)hipErrorInvalidValue;
-  if (path == 1 || path == 3) {
-    if (M > 64) return (int)hipErrorInvalidValue;
-    if (path == 3) {
-      if (epi == EPI_SILU_MUL) return (int)dispatch_gemv<EPI_SILU_MUL, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
-      if (epi == EPI_NONE) return (int)dispatch_gemv<EPI_NONE, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
-      if (epi == EPI_RESID) return (int)dispatch_gemv<EPI_RESID, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
-      return (int)hipErrorInvalidValue;
-    }
-    if (epi == EPI_SILU_MUL) return (int)dispatch_skinny<EPI_SILU_MUL, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
-    if (epi == EPI_NONE) return (int)dispatch_skinny<EPI_NONE, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
-    if (epi == EPI_RESID) return (int)dispatch_skinny<EPI_RESID, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
+  if (K % 128 != 0 || M > 64) return (int)hipErrorInvalidValue;
+  if (path == 3) {
+    if (epi == EPI_SILU_MUL) return (int)dispatch_gemv<EPI_SILU_MUL, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
+    if (epi == EPI_NONE) return (int)dispatch_gemv<EPI_NONE, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
+    if (epi == EPI_RESID) return (int)dispatch_gemv<EPI_RESID, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
     return (int)hipErrorInvalidValue;
   }
-  if (epi == EPI_SILU_MUL) return (int)launch_tile<EPI_SILU_MUL, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, 2 * N, K, st);
-  if (epi == EPI_NONE) return (int)launch_tile<EPI_NONE, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
-  if (epi == EPI_RESID) return (int)launch_tile<EPI_RESID, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
+  if (path != 1) return (int)hipErrorInvalidValue;
+  if (epi == EPI_SILU_MUL) return (int)dispatch_skinny<EPI_SILU_MUL, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
+  if (epi == EPI_NONE) return (int)dispatch_skinny<EPI_NONE, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
+  if (epi == EPI_RESID) return (int)dispatch_skinny<EPI_RESID, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
   return (int)hipErrorInvalidValue;
 }

@@ -258,15 +258,6 @@ __device__ __forceinline__ void w4_epilogue_full_bf16(const f32x4 (&acc)[8][8], 
 // p / p + 2 of the same lane. q heads: rotated into C; k heads: rotated into C and the paged cache at the
 // row's slot; v heads: C and the cache. Rows two at a time (cos / sin in registers: 64 values), loads
 // never predicated (rows past M clamp; only the stores are guarded).
-struct RopeKV {
-  const int* pos;
-  const int* slot;
-  const float* cos_t;  // [positions][64]
-  const float* sin_t;
-  bf16_t* kc;          // [blocks][Hkv][BS][128]
-  bf16_t* vc;
-  int Hq, Hkv, BS;
-};
 
 template <bool FULL>
 __device__ __forceinline__ void w4_epilogue_rope(const f32x4 (&acc)[8][8], int wr, int wc, int fr, int fh, int m0,

@@ -419,7 +419,7 @@ class NativeBackend(TorchBackend):
     def prefill_nsplit(self, M, w):
         if isinstance(w, Fp8Weight):
             return 1
-        return self.n.prefill_nsplit(M, w.shape[0], w.shape[1])
+        return self.n.slab_count(M, w.shape[0], w.shape[1])
 
     def gemm_splitk(self, x, w, nsplit):
         return self.n.gemm_splitk(x, w, nsplit)

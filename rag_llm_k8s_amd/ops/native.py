@@ -6,6 +6,7 @@ HIP stream, so everything here is capturable in a hipGraph (torch.cuda.CUDAGraph
 """
 from __future__ import annotations
 
+import functools
 import math
 import os
 import threading
@@ -116,7 +117,7 @@ def gemm_rope_kv_ok(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, 
         return False
     M, K = x.shape
     N = w.shape[0]
-    if N != (Hq + 2 * Hkv) * D or N % 256 or w.shape[1] != K or not use_pp(M, N, K, "none"):
+    if N != (Hq + 2 * Hkv) * D or N % 256 or w.shape[1] != K or M <= 64 or K % 64 or K < 192:
         return False
     if PREFILL_BLAS in ("plain", "all"):
         return False
@@ -136,17 +137,24 @@ def gemm_rope_kv_ok(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, 
 
 def gemm_rope_kv(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, Hkv, D, out=None):
     """qkv = x @ w^T with RoPE applied to q and k and the k / v rows written to the paged cache at `slots`
-    (gemm + rope_kv in one launch; callers check gemm_rope_kv_ok first)."""
+    (gemm + rope_kv in gemm's own launches, bit-identical to both; callers check gemm_rope_kv_ok first)."""
     _req(gemm_rope_kv_ok(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, Hkv, D), "gemm_rope_kv operands")
     M, K = x.shape
     N = w.shape[0]
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     _req(out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "gemm_rope_kv out")
-    check(_lib.lib().ragk_gemm_w4_rope_kv(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(),
-                                          out.stride(0), M, K, positions.data_ptr(), slots.data_ptr(),
-                                          cos_t.data_ptr(), sin_t.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-                                          Hq, Hkv, k_cache.shape[2], stream_ptr()), "ragk_gemm_w4_rope_kv")
+    L = _lib.lib()
+    for r0, r1, mi, S in gemm_plan(M, N, K, True, _cu_count()):
+        a = (x.data_ptr() + r0 * x.stride(0) * 2, x.stride(0), w.data_ptr(), w.stride(0),
+             out.data_ptr() + r0 * out.stride(0) * 2, out.stride(0), r1 - r0, K, positions.data_ptr() + 4 * r0,
+             slots.data_ptr() + 4 * r0, cos_t.data_ptr(), sin_t.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), Hq, Hkv,
+             k_cache.shape[2])
+        if mi == 0:
+            check(L.ragk_gemm_w4_rope_kv(*a, stream_ptr()), "ragk_gemm_w4_rope_kv")
+        else:
+            ws = torch.empty(S * (r1 - r0) * N, dtype=torch.float32, device=x.device) if S > 1 else None
+            check(L.ragk_gemm_mid_rope_kv(*a, mi, S, ptr(ws), stream_ptr()), "ragk_gemm_mid_rope_kv")
     return out
 
 
@@ -193,16 +201,25 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
             and ((epi == "none" and PREFILL_BLAS in ("plain", "all"))
                  or (epi == "resid" and PREFILL_BLAS in ("resid", "all")))):
         return _gemm_blas(x, w, resid, out, epi)
-    if path is None and use_pp(M, N, K, epi):
+    if path is None and M > 64:
         rows = w.shape[0]
         # gemm_w4 addresses operands with 32-bit buffer offsets
         fits = x.stride(0) * M * 2 < 2 ** 31 and w.stride(0) * rows * 2 < 2 ** 31
-        if epi == "glu_clip" and not fits:  # gemm_pp has no clipped unit: halve the rows until they fit
-            h = (M // 2 + 127) // 128 * 128
-            gemm(x[:h], w, bias=bias, epi=epi, out=out[:h])
-            gemm(x[h:], w, bias=bias, epi=epi, out=out[h:])
+        if not fits and use_pp(M, N, K, epi):
+            if epi != "glu_clip":
+                path = 2  # gemm_pp (8-wave ping-pong, 64-bit addressing): operands past 2 GiB
+            else:  # which has no clipped unit: halve the rows until they fit
+                h = (M // 2 + 127) // 128 * 128
+                gemm(x[:h], w, bias=bias, epi=epi, out=out[:h])
+                gemm(x[h:], w, bias=bias, epi=epi, out=out[h:])
+                return out
+        else:
+            w4 = fits and K % 64 == 0 and K >= 192 and (N % 128 == 0 if epi in PAIR_EPI else N % 8 == 0)
+            for r0, r1, mi, S in gemm_plan(M, rows, K, w4, _cu_count()):
+                _gemm_rows(x, w, bias, resid, epi, out, out_f32, r0, r1, mi, S)
             return out
-        path = 6 if fits else 2  # gemm_pp (8-wave ping-pong, 64-bit addressing): operands past 2 GiB
+    if path == 0:
+        return gemm_mid(x, w, bias=bias, resid=resid, epi=epi, out=out, out_f32=out_f32)
     if path is None and STREAM_DEFAULT and use_stream(M, N, K, epi):
         path = 5
     if path is None and DEC_DEFAULT and use_dec(M, N, K, epi):
@@ -237,6 +254,89 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
 def gemm_glu(x, w, par):
     """Packed gate/up projection with the clipped gated unit (par: fp32 {limit, alpha, shift} on the device)."""
     return gemm(x, w, bias=par, epi="glu_clip")
+
+
+def gemm_mid(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, mi=4, S=1):
+    """gemm() on the 128-column ring tiles of gemm_mid.hip: tiles of 32 mi rows, K cut into S slabs (S > 1: fp32 slabs in
+    a workspace, summed with the epilogue by a second launch)."""
+    M, K = x.shape
+    N = w.shape[0] // 2 if epi in PAIR_EPI else w.shape[0]
+    _req(mi in MID_US and 1 <= S <= K // 64 and K % 64 == 0 and w.shape[1] == K, "gemm_mid tile or split")
+    _req(out.shape == (M, N) and out.stride(1) == 1, "gemm_mid out")
+    _gemm_rows(x, w, bias, resid, epi, out, out_f32, 0, M, mi, S)
+    return out
+
+
+def _gemm_rows(x, w, bias, resid, epi, out, out_f32, r0, r1, mi, S):
+    """Rows r0 .. r1 of gemm() on gemm_mid (mi > 0) or gemm_w4 (mi == 0); operands checked by the caller."""
+    M, K = r1 - r0, x.shape[1]
+    N = w.shape[0] // 2 if epi in PAIR_EPI else w.shape[0]
+    ldx, ldo = x.stride(0), out.stride(0)
+    ldr = resid.stride(0) if resid is not None else 0
+    px, po = x.data_ptr() + r0 * ldx * 2, out.data_ptr() + r0 * ldo * out.element_size()
+    pr = resid.data_ptr() + r0 * ldr * 2 if resid is not None else None
+    args = (px, ldx, w.data_ptr(), w.stride(0), po, ldo, ptr(bias), pr, ldr, M, N, K, EPI[epi], int(out_f32))
+    if mi == 0:
+        check(_lib.lib().ragk_gemm_w4(*args, stream_ptr()), "ragk_gemm_w4")
+        return
+    ws = torch.empty(S * M * w.shape[0], dtype=torch.float32, device=x.device) if S > 1 else None
+    check(_lib.lib().ragk_gemm_mid(*args, mi, S, ptr(ws), stream_ptr()), "ragk_gemm_mid")
+
+
+# Microseconds that one 64-deep K-tile of an output tile takes with few blocks running, and what a full machine adds
+# (clocks, L2): tiles of gemm_mid by rows / 32, 0 = gemm_w4's 256 x 256. Fitted to M = 90 .. 13762, N = 1024 .. 28672.
+MID_US = {3: (0.29, 0.13), 4: (0.34, 0.17), 5: (0.40, 0.25), 6: (0.48, 0.15), 8: (0.60, 0.23)}
+W4_US = (1.0, 0.36)
+SLAB_US = 8 / 5e6  # one fp32 slab value written and read back
+
+
+def _tiles_us(M, rows, K, mi, S, cus):
+    """Model time of one launch: rounds of tiles over the CUs, each K-tiles long plus an epilogue."""
+    bm, bn = (32 * mi, 128) if mi else (256, 256)
+    items = -(-M // bm) * -(-rows // bn) * S
+    rounds = -(-items // cus)
+    a, b = MID_US[mi] if mi else W4_US
+    return (4.5 if mi else 7.5) + rounds * (-(-(K // 64) // S) * (a + b * items / (rounds * cus)) + 1.0)
+
+
+def _mid_best(M, rows, K, cus, slab_us, launch_us, even=False):
+    """(time, mi, S) of the best gemm_mid launch; a split costs launch_us and slab_us per slab value (even: equal slabs)."""
+    best = (float("inf"), 0, 1)
+    for mi in MID_US:
+        for S in range(1, 17):
+            if S > 1 and K // 64 // S < 4:
+                break
+            if even and K // 64 % S:
+                continue
+            t = _tiles_us(M, rows, K, mi, S, cus) + (launch_us + slab_us * S * M * rows if S > 1 else 0)
+            best = min(best, (t, mi, S))
+    return best
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_plan(M, rows, K, w4, cus):
+    """Launches of one product with M > 64 rows: [(first row, end, mi, S)], mi as in _tiles_us. Candidates: gemm_mid alone;
+    gemm_w4 alone (w4: its operands fit); gemm_w4 on as many rows as fill whole rounds of its tiles and gemm_mid on the
+    rest. Where they meet (us, N = K = 4096): 300 rows 24 against gemm_w4's 69, 1777 rows 54 against 79; at N = 28672 of
+    1777 rows gemm_w4 329 against 365 (its 128 x 128 wave tiles read less LDS per MFMA)."""
+    t, mi, S = _mid_best(M, rows, K, cus, SLAB_US, 3.0)
+    plan = ((0, M, mi, S),)
+    if not w4:
+        return plan
+    full = _tiles_us(M, rows, K, 0, 1, cus)
+    if full < t:
+        t, plan = full, ((0, M, 0, 1),)
+    tn = -(-rows // 256)
+    rounds = -(-M // 256) * tn // cus
+    for r in range(max(1, rounds - 1), rounds + 1):
+        m1 = r * cus // tn * 256
+        if not 0 < m1 < M:
+            continue
+        t2, mi, S = _mid_best(M - m1, rows, K, cus, SLAB_US, 3.0)
+        t2 += _tiles_us(m1, rows, K, 0, 1, cus)
+        if t2 < 0.97 * t:  # two launches have to earn their keep
+            t, plan = t2, ((0, m1, 0, 1), (m1, M, mi, S))
+    return plan
 
 
 PART_MIN_BLOCKS = 512
@@ -399,9 +499,34 @@ def prefill_nsplit(M, N, K):
     return best_s
 
 
+@functools.lru_cache(maxsize=4096)
+def _slab_best(M, N, K, cus):
+    """(S, mi) of the cheapest split whose slabs a row norm sums, (1, 0) if the whole product + a plain norm is cheaper.
+    Per output value the slabs cost 8 B each through memory, the whole product 6 (bf16 write, residual, norm's read).
+    o_proj / down at 300 rows: 28 / 88 us whole, 17 / 42 us as 2 / 4 slabs; at 14076 rows the slabs' traffic (212 us in the
+    norm) is more than the last round that they would fill."""
+    whole = 0.0
+    for r0, r1, mi, S in gemm_plan(M, N, K, K >= 192, cus):
+        whole += _tiles_us(r1 - r0, N, K, mi, S, cus) + (3.0 + SLAB_US * S * (r1 - r0) * N if S > 1 else 0)
+    best, S, mi = min((t - 0.75 * SLAB_US * M * N, S, mi) for t, mi, S in [_mid_best(M, N, K, cus, SLAB_US, 0.0, even=True)])
+    w4 = prefill_nsplit(M, N, K)
+    if w4 > 1:
+        t = _tiles_us(M, N, K, 0, w4, cus) + SLAB_US * (w4 - 0.75) * M * N
+        if t < best:
+            best, S, mi = t, w4, 0
+    return (S, mi) if S > 1 and best < whole else (1, 0)
+
+
+def slab_count(M, N, K):
+    """K-slabs for a prefill projection in front of a row norm (1: the whole product)."""
+    if not PREFILL_SPLITK or M <= 64 or K % 128 or N % 8:
+        return 1
+    return _slab_best(M, N, K, _cu_count())[0]
+
+
 def gemm_splitk(x, w, nsplit, out=None):
-    """fp32 split-K slabs P[nsplit, M, N] with P.sum(0) = x @ w^T, one persistent gemm_w4 launch
-    (csrc/kernels/gemm_w4.hip KSPLIT); consumed by add_partials_rmsnorm (residual add + norm)."""
+    """fp32 split-K slabs P[nsplit, M, N] with P.sum(0) = x @ w^T in one launch, consumed by add_partials_rmsnorm (residual
+    add + norm). gemm_mid or gemm_w4's KSPLIT form, whichever the launch model puts first."""
     _bf16_2d(x, "x")
     _bf16_2d(w, "w")
     M, K = x.shape
@@ -410,8 +535,17 @@ def gemm_splitk(x, w, nsplit, out=None):
     if out is None:
         out = torch.empty((nsplit, M, N), dtype=torch.float32, device=x.device)
     _req(out.dtype == torch.float32 and out.is_contiguous() and out.numel() >= nsplit * M * N, "gemm_splitk out")
-    check(_lib.lib().ragk_gemm_w4_splitk(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), M, N, K,
-                                         nsplit, stream_ptr()), "ragk_gemm_w4_splitk")
+    if M == 0:
+        return out
+    cus = _cu_count()
+    t, mi = min((_tiles_us(M, N, K, m, nsplit, cus), m) for m in MID_US)
+    fits = x.stride(0) * M * 2 < 2 ** 31 and w.stride(0) * N * 2 < 2 ** 31
+    if fits and _tiles_us(M, N, K, 0, nsplit, cus) < t:
+        check(_lib.lib().ragk_gemm_w4_splitk(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), M, N, K,
+                                             nsplit, stream_ptr()), "ragk_gemm_w4_splitk")
+    else:
+        check(_lib.lib().ragk_gemm_mid(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), N, None, None, 0,
+                                       M, N, K, EPI["none"], 2, mi, nsplit, None, stream_ptr()), "ragk_gemm_mid")
     return out
 
 

@@ -1,0 +1,30 @@
+"""The launch rule of products with more than 64 rows: every row once, splits that the kernels take."""
+import random
+
+from rag_llm_k8s_amd.ops import native as n
+
+
+def test_plans_cover_every_row_with_legal_launches():
+    r = random.Random(1)
+    for _ in range(400):
+        M = int(2 ** r.uniform(6.05, 15.5))
+        rows, K = 8 * r.randint(1, 4000), 128 * r.randint(1, 120)
+        for w4 in (False, K >= 192):
+            plan = n.gemm_plan(M, rows, K, w4, 256)
+            at = 0
+            for r0, r1, mi, S in plan:
+                assert r0 == at < r1
+                at = r1
+                assert (mi in n.MID_US or (mi == 0 and w4 and S == 1)) and 1 <= S <= max(1, K // 256)
+            assert at == M
+        S, mi = n._slab_best(M, rows, K, 256)
+        assert S == 1 or (K % (64 * S) == 0 and K // S >= 256 and (mi in n.MID_US or mi == 0))
+
+
+def test_launch_model_prefers_full_rounds():
+    """What the plan is for: few rows split K, one filled round of large tiles stays whole, a ragged last round of gemm_w4's
+    tiles goes to the smaller ones."""
+    assert n.gemm_plan(300, 4096, 14336, True, 256)[0][3] > 1
+    assert n.gemm_plan(4096, 4096, 4096, True, 256) == ((0, 4096, 0, 1),)
+    (a, b) = n.gemm_plan(14076, 4096, 4096, True, 256)
+    assert a == (0, 12288, 0, 1) and b[2] > 0

@@ -1,5 +1,5 @@
 // Memory-bound row kernels for gfx950: RMSNorm, LayerNorm, embedding gathers,
-// fused RoPE + paged-KV write, pooling + L2 normalise, standalone SiLU*up.
+// fused RoPE + paged-KV write, standalone SiLU*up.
 //
 // All loads/stores are 16-byte vectors (8 x bf16) -- hipcc does not vectorise
 // bf16 on its own. Rows map to blocks of 256 threads (4 waves); reductions are
@@ -8,10 +8,9 @@
 // Reference semantics reproduced here:
 //   K1 embed_tokens gather, K2 LlamaRMSNorm (fp32 variance, cast back, *weight),
 //   K4 llama3-scaled RoPE in rotate_half layout, K13 KV-cache append,
-//   E1 BERT/XLM-R embeddings (+LayerNorm), E4/E6 post-LN LayerNorm,
-//   E7 CLS / masked-mean pooling + L2 normalise (sentence-transformers
-//   Normalize(), /root/reference/llm/rag.py:55 normalize_embeddings=True).
+//   E1 BERT/XLM-R embeddings (+LayerNorm), E4/E6 post-LN LayerNorm.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 using namespace ragk;
@@ -66,58 +65,84 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(const bf16_t* x, int ldx, b
   }
 }
 
-// LayerNorm over the last dim (fp32 statistics, two-pass in registers), optional
-// fused residual: y = LN(x + resid) * g + b.
-__global__ __launch_bounds__(NT) void layernorm_kernel(const bf16_t* x, int ldx, const bf16_t* resid, int ldr,
-                                                       const bf16_t* __restrict__ g, const bf16_t* __restrict__ b,
-                                                       bf16_t* out, int ldo, int H, float eps) {
-  __shared__ float red[NT / 64];
-  const int row = blockIdx.x;
-  const bf16_t* xr = x + (size_t)row * ldx;
-  constexpr int MAXV = 4;
-  float v[MAXV][8];
-  const int nvec = H >> 3;
+// LayerNorm of a row held in registers (fp32 statistics, two passes): NV vectors of 8 columns a thread, W waves a row.
+// Encoder rows are 384 to 1024 wide: with a block a row, 48 to 128 of 256 threads had columns, behind two block-wide
+// reductions; one wave a row (up to 2048 columns) takes 11.1 us for 13762 x 1024 (before: 20.1) and 8.6 for 12805 x 384
+// (17.1, launch included). Wider rows stay a block each: 3000 x 4096 takes 11.0 us so, 12.1 in one wave.
+template <int W>
+__device__ __forceinline__ float row_sum(float v) {
+  if constexpr (W == 1) return wave_sum(v);
+  __shared__ float red[W];
+  return block_sum(v, red);
+}
+template <int NV, int W>
+__device__ __forceinline__ void ln_row(float (&v)[NV][8], int nvec, int lane, const bf16_t* __restrict__ g,
+                                       const bf16_t* __restrict__ b, bf16_t* orow, int H, float eps) {
+  u32x4 gr[NV], br[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int vi = min(lane + 64 * W * i, nvec - 1);
+    gr[i] = *reinterpret_cast<const u32x4*>(g + vi * 8);
+    br[i] = *reinterpret_cast<const u32x4*>(b + vi * 8);
+  }
   float s = 0.f;
 #pragma unroll
-  for (int i = 0; i < MAXV; ++i) {
-    const int vi = threadIdx.x + i * NT;
-    if (vi < nvec) {
-      unpack8(*reinterpret_cast<const u32x4*>(xr + vi * 8), v[i]);
-      if (resid) {
-        float r8[8];
-        unpack8(*reinterpret_cast<const u32x4*>(resid + (size_t)row * ldr + vi * 8), r8);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[i][e] += r8[e];
-      }
+  for (int i = 0; i < NV; ++i)
+    if (lane + 64 * W * i < nvec)
 #pragma unroll
       for (int e = 0; e < 8; ++e) s += v[i][e];
-    }
-  }
-  const float mean = block_sum(s, red) / (float)H;
+  const float mean = row_sum<W>(s) / (float)H;
   float sq = 0.f;
 #pragma unroll
-  for (int i = 0; i < MAXV; ++i) {
-    const int vi = threadIdx.x + i * NT;
-    if (vi < nvec)
+  for (int i = 0; i < NV; ++i)
+    if (lane + 64 * W * i < nvec)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float d = v[i][e] - mean;
         sq += d * d;
       }
-  }
-  const float inv = rsqrtf(block_sum(sq, red) / (float)H + eps);
+  const float inv = rsqrtf(row_sum<W>(sq) / (float)H + eps);
 #pragma unroll
-  for (int i = 0; i < MAXV; ++i) {
-    const int vi = threadIdx.x + i * NT;
+  for (int i = 0; i < NV; ++i) {
+    const int vi = lane + 64 * W * i;
     if (vi < nvec) {
       float gv[8], bv[8], o[8];
-      unpack8(*reinterpret_cast<const u32x4*>(g + vi * 8), gv);
-      unpack8(*reinterpret_cast<const u32x4*>(b + vi * 8), bv);
+      unpack8(gr[i], gv);
+      unpack8(br[i], bv);
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = (v[i][e] - mean) * inv * gv[e] + bv[e];
-      *reinterpret_cast<u32x4*>(out + (size_t)row * ldo + vi * 8) = pack8(o);
+      *reinterpret_cast<u32x4*>(orow + vi * 8) = pack8(o);
     }
   }
+}
+
+// y = LN(x [+ resid]) * g + b, 4 / W rows a block
+template <int NV, int W>
+__global__ __launch_bounds__(NT) void layernorm_kernel(const bf16_t* x, int ldx, const bf16_t* resid, int ldr,
+                                                       const bf16_t* __restrict__ g, const bf16_t* __restrict__ b,
+                                                       bf16_t* out, int ldo, int rows, int H, float eps) {
+  const int lane = threadIdx.x & (64 * W - 1), row = blockIdx.x * (NT / 64 / W) + threadIdx.x / (64 * W);
+  if (row >= rows) return;  // (whole rows: never part of a block that reduces together)
+  const int nvec = H >> 3;
+  u32x4 xv[NV], rv[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int vi = min(lane + 64 * W * i, nvec - 1);
+    xv[i] = *reinterpret_cast<const u32x4*>(x + (size_t)row * ldx + vi * 8);
+    if (resid) rv[i] = *reinterpret_cast<const u32x4*>(resid + (size_t)row * ldr + vi * 8);
+  }
+  float v[NV][8];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    unpack8(xv[i], v[i]);
+    if (resid) {
+      float r8[8];
+      unpack8(rv[i], r8);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[i][e] += r8[e];
+    }
+  }
+  ln_row<NV, W>(v, nvec, lane, g, b, out + (size_t)row * ldo, H, eps);
 }
 
 // token embedding gather: out[t] = table[ids[t]]
@@ -143,72 +168,56 @@ __global__ __launch_bounds__(NT) void embed_kernel(int* __restrict__ ids, const 
   for (int i = threadIdx.x; i < (H >> 3); i += NT) dst[i] = src[i];
 }
 
-// BERT / XLM-R embeddings: LN(word[id] + pos[pos_id] + type[type_id]) (+ optional GPT-2 style no-LN)
+// BERT / XLM-R embeddings: LN(word[id] + pos[pos_id] + type[type_id]) (+ optional GPT-2 style no-LN), 4 / W rows a block
+template <int NV, int W>
 __global__ __launch_bounds__(NT) void embed_ln_kernel(const int* __restrict__ ids, const int* __restrict__ pos_ids,
                                                       const bf16_t* __restrict__ word, const bf16_t* __restrict__ pos,
                                                       const bf16_t* __restrict__ type, const bf16_t* __restrict__ g,
-                                                      const bf16_t* __restrict__ b, bf16_t* out, int H, float eps,
+                                                      const bf16_t* __restrict__ b, bf16_t* out, int rows, int H, float eps,
                                                       int do_ln) {
-  __shared__ float red[NT / 64];
-  const int t = blockIdx.x;
+  const int lane = threadIdx.x & (64 * W - 1), t = blockIdx.x * (NT / 64 / W) + threadIdx.x / (64 * W);
+  if (t >= rows) return;
   const bf16_t* wr = word + (size_t)ids[t] * H;
   const bf16_t* pr = pos + (size_t)pos_ids[t] * H;
-  constexpr int MAXV = 4;
-  float v[MAXV][8];
   const int nvec = H >> 3;
-  float s = 0.f;
+  u32x4 wv[NV], pv[NV], tv[NV];
 #pragma unroll
-  for (int i = 0; i < MAXV; ++i) {
-    const int vi = threadIdx.x + i * NT;
-    if (vi < nvec) {
-      float a[8], p[8];
-      unpack8(*reinterpret_cast<const u32x4*>(wr + vi * 8), a);
-      unpack8(*reinterpret_cast<const u32x4*>(pr + vi * 8), p);
+  for (int i = 0; i < NV; ++i) {
+    const int vi = min(lane + 64 * W * i, nvec - 1);
+    wv[i] = *reinterpret_cast<const u32x4*>(wr + vi * 8);
+    pv[i] = *reinterpret_cast<const u32x4*>(pr + vi * 8);
+    if (type) tv[i] = *reinterpret_cast<const u32x4*>(type + vi * 8);
+  }
+  float v[NV][8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[i][e] = a[e] + p[e];
-      if (type) {
-        float ty[8];
-        unpack8(*reinterpret_cast<const u32x4*>(type + vi * 8), ty);
+  for (int i = 0; i < NV; ++i) {
+    float p[8];
+    unpack8(wv[i], v[i]);
+    unpack8(pv[i], p);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[i][e] += ty[e];
-      }
+    for (int e = 0; e < 8; ++e) v[i][e] += p[e];
+    if (type) {
+      unpack8(tv[i], p);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) s += v[i][e];
+      for (int e = 0; e < 8; ++e) v[i][e] += p[e];
     }
   }
-  if (!do_ln) {
+  bf16_t* orow = out + (size_t)t * H;
+  if (do_ln) return ln_row<NV, W>(v, nvec, lane, g, b, orow, H, eps);
 #pragma unroll
-    for (int i = 0; i < MAXV; ++i) {
-      const int vi = threadIdx.x + i * NT;
-      if (vi < nvec) *reinterpret_cast<u32x4*>(out + (size_t)t * H + vi * 8) = pack8(v[i]);
-    }
-    return;
-  }
-  const float mean = block_sum(s, red) / (float)H;
-  float sq = 0.f;
-#pragma unroll
-  for (int i = 0; i < MAXV; ++i) {
-    const int vi = threadIdx.x + i * NT;
-    if (vi < nvec)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float d = v[i][e] - mean;
-        sq += d * d;
-      }
-  }
-  const float inv = rsqrtf(block_sum(sq, red) / (float)H + eps);
-#pragma unroll
-  for (int i = 0; i < MAXV; ++i) {
-    const int vi = threadIdx.x + i * NT;
-    if (vi < nvec) {
-      float gv[8], bv[8], o[8];
-      unpack8(*reinterpret_cast<const u32x4*>(g + vi * 8), gv);
-      unpack8(*reinterpret_cast<const u32x4*>(b + vi * 8), bv);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = (v[i][e] - mean) * inv * gv[e] + bv[e];
-      *reinterpret_cast<u32x4*>(out + (size_t)t * H + vi * 8) = pack8(o);
-    }
-  }
+  for (int i = 0; i < NV; ++i)
+    if (lane + 64 * W * i < nvec) *reinterpret_cast<u32x4*>(orow + (lane + 64 * W * i) * 8) = pack8(v[i]);
+}
+
+// f(NV, W) as constants for a row of H <= 8192 columns
+template <typename F>
+hipError_t by_row(int H, F f) {
+  using std::integral_constant;
+  if (H <= 512) f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+  else if (H <= 1024) f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+  else if (H <= 2048) f(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+  else f(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+  return hipGetLastError();
 }
 
 // Fused RoPE (rotate_half layout, HF bf16 rounding replicated) + paged KV write.
@@ -272,53 +281,6 @@ __global__ __launch_bounds__(NT) void rope_kv_kernel(bf16_t* qkv, int ld, const 
       bf16_t* dst = vc + (((size_t)(slot / BS) * Hkv + kh) * BS + (slot % BS)) * D + v * 8;
       *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(src);
     }
-  }
-}
-
-// out[b] = normalize(pool(hidden[cu[b]:cu[b+1]])) in fp32. mode 0 = CLS (first token),
-// mode 1 = masked mean over the sequence, mode 2 = last token.
-__global__ __launch_bounds__(NT) void pool_l2norm_kernel(const bf16_t* __restrict__ hidden, int ld,
-                                                         const int* __restrict__ cu, float* out, int H, int mode,
-                                                         int normalize) {
-  __shared__ float red[NT / 64];
-  const int b = blockIdx.x;
-  const int s0 = cu[b], s1 = cu[b + 1];
-  const int len = s1 - s0;
-  float ss = 0.f;
-  // each thread owns columns c = threadIdx.x + k*NT
-  constexpr int MAXC = 8;  // H <= 2048
-  float acc[MAXC];
-#pragma unroll
-  for (int k = 0; k < MAXC; ++k) acc[k] = 0.f;
-  if (mode == 1) {
-    for (int t = s0; t < s1; ++t)
-#pragma unroll
-      for (int k = 0; k < MAXC; ++k) {
-        const int c = threadIdx.x + k * NT;
-        if (c < H) acc[k] += bf2f(hidden[(size_t)t * ld + c]);
-      }
-    const float inv = len > 0 ? 1.f / (float)len : 0.f;
-#pragma unroll
-    for (int k = 0; k < MAXC; ++k) acc[k] *= inv;
-  } else {
-    const int t = mode == 0 ? s0 : s1 - 1;
-#pragma unroll
-    for (int k = 0; k < MAXC; ++k) {
-      const int c = threadIdx.x + k * NT;
-      if (c < H) acc[k] = bf2f(hidden[(size_t)t * ld + c]);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < MAXC; ++k) ss += acc[k] * acc[k];
-  float scale = 1.f;
-  if (normalize) {
-    ss = block_sum(ss, red);
-    scale = 1.f / fmaxf(sqrtf(ss), 1e-12f);  // torch.nn.functional.normalize eps
-  }
-#pragma unroll
-  for (int k = 0; k < MAXC; ++k) {
-    const int c = threadIdx.x + k * NT;
-    if (c < H) out[(size_t)b * H + c] = acc[k] * scale;
   }
 }
 
@@ -467,9 +429,12 @@ RAGK_API int ragk_layernorm(const void* x, int ldx, const void* resid, int ldr, 
                             void* out, int ldo, int rows, int H, float eps, hipStream_t st) {
   if (rows <= 0) return 0;
   if (H % 8 || H > 8 * NT * 4) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(layernorm_kernel, dim3(rows), dim3(NT), 0, st, (const bf16_t*)x, ldx, (const bf16_t*)resid,
-                     ldr, (const bf16_t*)g, (const bf16_t*)b, (bf16_t*)out, ldo, H, eps);
-  return (int)hipGetLastError();
+  return (int)by_row(H, [&](auto nv, auto w) {
+    constexpr int R = NT / 64 / decltype(w)::value;
+    hipLaunchKernelGGL((layernorm_kernel<decltype(nv)::value, decltype(w)::value>), dim3((rows + R - 1) / R), dim3(NT), 0, st,
+                       (const bf16_t*)x, ldx, (const bf16_t*)resid, ldr, (const bf16_t*)g, (const bf16_t*)b, (bf16_t*)out, ldo,
+                       rows, H, eps);
+  });
 }
 
 RAGK_API int ragk_embed(const int* ids, const void* table, void* out, int T, int H, int vocab, hipStream_t st) {
@@ -496,10 +461,12 @@ RAGK_API int ragk_embed_ln(const int* ids, const int* pos_ids, const void* word,
                            hipStream_t st) {
   if (T <= 0) return 0;
   if (H % 8 || H > 8 * NT * 4) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(embed_ln_kernel, dim3(T), dim3(NT), 0, st, ids, pos_ids, (const bf16_t*)word,
-                     (const bf16_t*)pos, (const bf16_t*)type, (const bf16_t*)g, (const bf16_t*)b, (bf16_t*)out, H,
-                     eps, do_ln);
-  return (int)hipGetLastError();
+  return (int)by_row(H, [&](auto nv, auto w) {
+    constexpr int R = NT / 64 / decltype(w)::value;
+    hipLaunchKernelGGL((embed_ln_kernel<decltype(nv)::value, decltype(w)::value>), dim3((T + R - 1) / R), dim3(NT), 0, st, ids,
+                       pos_ids, (const bf16_t*)word, (const bf16_t*)pos, (const bf16_t*)type, (const bf16_t*)g,
+                       (const bf16_t*)b, (bf16_t*)out, T, H, eps, do_ln);
+  });
 }
 
 RAGK_API int ragk_rope_kv(void* qkv, int ld, const int* positions, const float* cos_t, const float* sin_t,
@@ -509,15 +476,6 @@ RAGK_API int ragk_rope_kv(void* qkv, int ld, const int* positions, const float* 
   if (D % 16) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(rope_kv_kernel, dim3(T), dim3(NT), 0, st, (bf16_t*)qkv, ld, positions, cos_t, sin_t, slots,
                      (bf16_t*)kc, (bf16_t*)vc, Hq, Hkv, D, BS, apply_rope);
-  return (int)hipGetLastError();
-}
-
-RAGK_API int ragk_pool_l2norm(const void* hidden, int ld, const int* cu, float* out, int B, int H, int mode,
-                              int normalize, hipStream_t st) {
-  if (B <= 0) return 0;
-  if (H > 8 * NT) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(pool_l2norm_kernel, dim3(B), dim3(NT), 0, st, (const bf16_t*)hidden, ld, cu, out, H, mode,
-                     normalize);
   return (int)hipGetLastError();
 }
 

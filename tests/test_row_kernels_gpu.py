@@ -1,0 +1,31 @@
+"""LayerNorm and pooling at the widths where their split changes."""
+import pytest
+import torch
+
+from rag_llm_k8s_amd.ops import reference as R
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("T,H", [(1, 384), (5, 512), (3, 520), (9, 1024), (4, 1032), (2, 2048), (3, 2056), (5, 8192)])
+def test_layernorm_rows(native, T, H):
+    """Widths around the vectors a lane holds and the change from one wave to four a row."""
+    torch.manual_seed(H)
+    x, r = torch.randn(T, H, device=DEV).bfloat16(), torch.randn(T, H, device=DEV).bfloat16()
+    g, b = torch.randn(H, device=DEV).bfloat16(), torch.randn(H, device=DEV).bfloat16()
+    for res in (None, r):
+        ref = R.layernorm(x.double(), g.double(), b.double(), 1e-12, resid=None if res is None else res.double())
+        assert (native.layernorm(x, g, b, 1e-12, resid=res).double() - ref).norm() / ref.norm() < 3e-3
+
+
+@pytest.mark.parametrize("H", [8, 100, 384, 1000, 2048])
+def test_pool_rows(native, H):
+    """Column groups of eight and single columns (odd widths and strides), one row to more rows than row groups."""
+    lens = [1, 3, 200, 17]
+    cu = torch.tensor([0, 1, 4, 204, 221], dtype=torch.int32, device=DEV)
+    h = torch.randn(sum(lens), H + 3, device=DEV).bfloat16()
+    for x in (h[:, :H], h[:, :H].contiguous()):
+        for mode in ("cls", "mean", "last"):
+            ref = R.pool_l2norm(x.float().cpu(), cu.cpu(), mode=mode)
+            assert (native.pool_l2norm(x, cu, mode=mode).cpu() - ref).abs().max().item() < 1e-5

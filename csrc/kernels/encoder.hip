@@ -1,7 +1,23 @@
 // Sentence encoders: pooling + L2 normalise (E7: CLS / masked mean, sentence-transformers Normalize(),
-// /root/reference/llm/rag.py:55 normalize_embeddings=True).
+// /root/reference/llm/rag.py:55 normalize_embeddings=True), and one forward over packed sequences as a single host call.
+//
+// A query's embedding is about 45 launches of 2 to 5 us each (6 layers); issued one by one from Python they took 14 us each and
+// the GPU idled between them. The kernels of the layers are those of gemm*.hip, attention.hip and norm.hip.
 #include "common.h"
 using namespace ragk;
+
+extern "C" {
+int ragk_gemm(const void*, int, const void*, int, void*, int, const void*, const void*, int, int, int, int, int, int, hipStream_t);
+int ragk_gemm_w4(const void*, int, const void*, int, void*, int, const void*, const void*, int, int, int, int, int, int,
+                 hipStream_t);
+int ragk_gemm_mid(const void*, int, const void*, int, void*, int, const void*, const void*, int, int, int, int, int, int, int,
+                  int, float*, hipStream_t);
+int ragk_attn_prefill(const void*, int, const void*, const void*, int, const int*, int, const int*, const int*, const int*,
+                      const int*, int, void*, int, int, int, int, int, int, float, hipStream_t);
+int ragk_layernorm(const void*, int, const void*, int, const void*, const void*, void*, int, int, int, float, hipStream_t);
+int ragk_embed_ln(const int*, const int*, const void*, const void*, const void*, const void*, const void*, void*, int, int,
+                  float, int, hipStream_t);
+}
 
 namespace {
 
@@ -86,6 +102,38 @@ __global__ __launch_bounds__(POOL_NT) void pool_l2norm_kernel(const bf16_t* __re
 }
 
 
+// Launches of one product: rows r0 .. r1 on gemm_mid (tile mi, S slabs), gemm_w4 (mi 0) or the skinny kernel (mi -1).
+struct Piece { int r0, r1, mi, S; };
+struct Plan { int n; Piece p[2]; };
+
+// The arguments of one forward (mirrored by ops/_lib.py EncoderCall).
+struct EncoderCall {
+  const void *word, *pos_table, *type_row, *ln_g, *ln_b;
+  const void* const* layers;  // 12 a layer: wqkv bqkv wo bo ln1_g ln1_b wi bi wo2 bo2 ln2_g ln2_b
+  const int *ids, *pos, *cu, *lens, *tiles, *rows;  // rows: output row of every sequence
+  void *h, *a, *qkv, *attn, *f;
+  float *ws, *out;
+  int n_layers, T, B, H, I, heads, n_tiles, pooling, normalize, ldo;
+  float eps;
+  Plan plans[4];  // qkv, attention output, up, down
+};
+
+int product(const Plan& plan, const void* x, int K, const void* w, int N, const void* bias, const void* resid, void* out, int epi,
+            float* ws, hipStream_t st) {
+  for (int i = 0; i < plan.n; ++i) {
+    const Piece& p = plan.p[i];
+    const char* px = (const char*)x + (size_t)p.r0 * K * 2;
+    const char* pr = resid ? (const char*)resid + (size_t)p.r0 * N * 2 : nullptr;
+    char* po = (char*)out + (size_t)p.r0 * N * 2;
+    const int M = p.r1 - p.r0;
+    const int rc = p.mi < 0    ? ragk_gemm(px, K, w, K, po, N, bias, pr, N, M, N, K, epi, 0, st)
+                   : p.mi == 0 ? ragk_gemm_w4(px, K, w, K, po, N, bias, pr, N, M, N, K, epi, 0, st)
+                               : ragk_gemm_mid(px, K, w, K, po, N, bias, pr, N, M, N, K, epi, 0, p.mi, p.S, ws, st);
+    if (rc) return rc;
+  }
+  return 0;
+}
+
 }  // namespace
 
 // The pooled sequence b goes to row rows[b] of out (rows null: row b), row stride ldo.
@@ -101,4 +149,31 @@ RAGK_API int ragk_pool_l2norm_rows(const void* hidden, int ld, const int* cu, co
 RAGK_API int ragk_pool_l2norm(const void* hidden, int ld, const int* cu, float* out, int B, int H, int mode,
                               int normalize, hipStream_t st) {
   return ragk_pool_l2norm_rows(hidden, ld, cu, nullptr, out, H, B, H, mode, normalize, st);
+}
+
+RAGK_API int ragk_encoder_call_bytes() { return (int)sizeof(EncoderCall); }
+
+RAGK_API int ragk_encoder_forward(const EncoderCall* cp, hipStream_t st) {
+  const EncoderCall& c = *cp;
+  const int H = c.H, D = H / c.heads, T = c.T;
+  if (T <= 0 || c.B <= 0) return 0;
+  const float scale = 1.f / sqrtf((float)D);
+#define RAGK_TRY(x) \
+  if (const int rc = (x)) return rc
+  RAGK_TRY(ragk_embed_ln(c.ids, c.pos, c.word, c.pos_table, c.type_row, c.ln_g, c.ln_b, c.h, T, H, c.eps, 1, st));
+  for (int l = 0; l < c.n_layers; ++l) {
+    const void* const* w = c.layers + 12 * l;
+    RAGK_TRY(product(c.plans[0], c.h, H, w[0], 3 * H, w[1], nullptr, c.qkv, EPI_BIAS, c.ws, st));
+    const char* q = (const char*)c.qkv;
+    RAGK_TRY(ragk_attn_prefill(q, 3 * H, q + 2 * H, q + 4 * H, 3 * H, nullptr, 0, c.cu, c.cu, c.lens, c.tiles, c.n_tiles, c.attn,
+                               H, c.heads, c.heads, D, 0, 0, scale, st));
+    RAGK_TRY(product(c.plans[1], c.attn, H, w[2], H, w[3], c.h, c.a, EPI_BIAS_RESID, c.ws, st));
+    RAGK_TRY(ragk_layernorm(c.a, H, nullptr, 0, w[4], w[5], c.h, H, T, H, c.eps, st));
+    RAGK_TRY(product(c.plans[2], c.h, H, w[6], c.I, w[7], nullptr, c.f, EPI_BIAS_GELU, c.ws, st));
+    RAGK_TRY(product(c.plans[3], c.f, c.I, w[8], H, w[9], c.h, c.a, EPI_BIAS_RESID, c.ws, st));
+    RAGK_TRY(ragk_layernorm(c.a, H, nullptr, 0, w[10], w[11], c.h, H, T, H, c.eps, st));
+  }
+  RAGK_TRY(ragk_pool_l2norm_rows(c.h, H, c.cu, c.rows, c.out, c.ldo, c.B, H, c.pooling, c.normalize, st));
+#undef RAGK_TRY
+  return 0;
 }

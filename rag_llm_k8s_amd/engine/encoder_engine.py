@@ -68,9 +68,7 @@ class EmbeddingEngine:
             j = i + max(1, int(np.searchsorted(csum, self.max_batch_tokens, side="right")))
             rows = order[i:j]
             flat = np.concatenate([ids[starts[r]:starts[r + 1]] for r in rows])
-            t = torch.from_numpy(flat).to(self.device)  # pageable source: a synchronous copy, safe to reuse
-            emb = self.model.forward_packed(t, [int(x) for x in slens[i:j]])
-            out[torch.from_numpy(rows + row0).to(self.device)] = emb
+            self.model.embed_into(flat, slens[i:j], out, rows + row0)
             i = j
         return out
 

@@ -168,10 +168,21 @@ class EncoderModel:
         self.cfg, self.w, self.device = cfg, weights, torch.device(device)
         self.be = get_backend(self.device)
 
-    def position_ids(self, lens):
+    @property
+    def first_position(self):
         """BERT: 0..L-1.  XLM-R: cumsum(mask) + padding_idx -> starts at padding_idx + 1."""
-        off = self.cfg.pad_token_id + 1 if self.cfg.model_type == "xlm-roberta" else 0
+        return self.cfg.pad_token_id + 1 if self.cfg.model_type == "xlm-roberta" else 0
+
+    def position_ids(self, lens):
+        off = self.first_position
         return torch.cat([torch.arange(off, off + L, dtype=torch.int32) for L in lens])
+
+    def embed_into(self, ids, lens, out, rows):
+        """Embeddings of the packed sequences (host ids int32, lens int64) into rows `rows` (int64) of out."""
+        if self.be.encoder_forward(self.cfg, self.w, ids, lens, self.first_position, out, rows):
+            return
+        t = torch.from_numpy(ids).to(self.device)  # pageable source: a synchronous copy, safe to reuse
+        out[torch.from_numpy(rows).to(self.device)] = self.forward_packed(t, lens.tolist())
 
     def forward_packed(self, ids: torch.Tensor, lens):
         """ids: int32 [T] packed token ids (on device), lens: python list of sequence lengths.

@@ -68,6 +68,8 @@ _SIGS = {
     "ragk_embed_ln": [P, P, P, P, P, P, P, P, I, I, F, I, S],
     "ragk_rope_kv": [P, I, P, P, P, P, P, P, I, I, I, I, I, I, S],
     "ragk_pool_l2norm": [P, I, P, P, I, I, I, I, S],
+    "ragk_encoder_call_bytes": [],
+    "ragk_encoder_forward": [P, S],
     "ragk_silu_mul": [P, I, P, I, I, I, S],
     "ragk_gather_rows": [P, I, P, P, I, I, I, S],
     "ragk_attn_prefill_qtile": [I, I],
@@ -233,6 +235,22 @@ def has_symbol(name: str) -> bool:
         return hasattr(lib(), name)
     except NativeLibraryError:
         return False
+
+
+class GemmPiece(ctypes.Structure):
+    _fields_ = [(n, I) for n in ("r0", "r1", "mi", "S")]
+
+
+class GemmPlan(ctypes.Structure):
+    _fields_ = [("n", I), ("p", GemmPiece * 2)]
+
+
+class EncoderCall(ctypes.Structure):
+    """csrc/kernels/encoder.hip EncoderCall."""
+    _fields_ = ([(n, P) for n in ("word", "pos_table", "type_row", "ln_g", "ln_b", "layers", "ids", "pos", "cu", "lens", "tiles",
+                                  "rows", "h", "a", "qkv", "attn", "f", "ws", "out")]
+                + [(n, I) for n in ("n_layers", "T", "B", "H", "I", "heads", "n_tiles", "pooling", "normalize", "ldo")]
+                + [("eps", F), ("plans", GemmPlan * 4)])
 
 
 def stream_ptr(device=None) -> int:

@@ -218,6 +218,10 @@ class TorchBackend:
     def pool_l2norm(self, hidden, cu, mode="cls", normalize=True):
         return R.pool_l2norm(hidden, cu.cpu(), mode=mode, normalize=normalize)
 
+    def encoder_forward(self, cfg, w, ids, lens, first_pos, out, rows):
+        """Whole forward of a packed batch given as host integers, into rows of out; False: not offered here."""
+        return False
+
     # fp32 residual stream, shaped attention, state-space mixers ---------------
     def embed_residual(self, ids, table, carry=None, prev=None, scale=1.0, pos=None, turns=None, n=0):
         """Embedding rows * scale as the fp32 residual stream, plus the sinusoid of `pos` over the first n columns."""
@@ -534,6 +538,14 @@ class NativeBackend(TorchBackend):
 
     def pool_l2norm(self, hidden, cu, mode="cls", normalize=True):
         return self.n.pool_l2norm(hidden, cu, mode=mode, normalize=normalize)
+
+    def encoder_forward(self, cfg, w, ids, lens, first_pos, out, rows):
+        T = int(lens.sum())
+        if (out.dtype != torch.float32 or out.stride(1) != 1 or out.device != w.word.device or T == 0
+                or T * max(3 * cfg.hidden_size, cfg.intermediate_size) * 2 >= 2 ** 31 or not self.n.encoder_forward_ok(cfg, w)):
+            return False
+        self.n.encoder_forward(cfg, w, ids, lens, first_pos, out, rows)
+        return True
 
     def topk_candidates(self, logits, K, vocab_offset=0, max_cand=512, chunks=None):
         return self.n.topk_candidates(logits, K, vocab_offset=vocab_offset, max_cand=max_cand, chunks=chunks)

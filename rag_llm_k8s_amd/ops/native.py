@@ -991,6 +991,64 @@ def pool_l2norm(hidden, cu, mode="cls", normalize=True, out=None):
     return out
 
 
+ENCODER_LAYER = ("wqkv", "bqkv", "wo", "bo", "ln1_g", "ln1_b", "wi", "bi", "wo2", "bo2", "ln2_g", "ln2_b")
+
+
+def encoder_forward_ok(cfg, w):
+    """Whether encoder_forward takes these weights (else: layer by layer through the checked entry points)."""
+    H, I = cfg.hidden_size, cfg.intermediate_size
+    if H % 128 or I % 128 or H > 2048 or max(3 * H, I) >= STREAM_MIN_ROWS or H // cfg.num_attention_heads not in (32, 64, 128):
+        return False
+    sizes = [2 * n for n in (3 * H * H, 3 * H, H * H, H, H, H, I * H, I, H * I, H, H, H)]
+    return (all([L[k].nbytes for k in ENCODER_LAYER] == sizes and L["wqkv"].dtype == torch.bfloat16 for L in w.layers)
+            and w.word.dtype == torch.bfloat16 and w.word.shape[1] == H and w.pos.shape[1] == H and w.type_row.numel() == H)
+
+
+def encoder_forward(cfg, w, ids, lens, first_pos, out, rows):
+    """Embeddings of packed sequences (host int32 ids, int64 lens) into rows `rows` of out (fp32 on the device): one upload
+    of the step's integers, one workspace, one native call for all launches (csrc/kernels/encoder.hip)."""
+    import ctypes
+
+    import numpy as np
+
+    H, I, nh, B, T = cfg.hidden_size, cfg.intermediate_size, cfg.num_attention_heads, len(lens), int(len(ids))
+    _req(out.dtype == torch.float32 and out.is_cuda and out.stride(1) == 1 and out.shape[1] == H, "out fp32 rows")
+    _req(T == int(lens.sum()) and len(rows) == B and 0 <= int(rows.min()) and int(rows.max()) < out.shape[0], "lens, rows")
+    _req(T * max(3 * H, I) * 2 < 2 ** 31, "packed rows past 2 GiB")
+    dev = out.device
+    cu = np.zeros(B + 1, dtype=np.int32)
+    np.cumsum(lens, out=cu[1:])
+    pos = np.arange(first_pos, first_pos + T, dtype=np.int32) - np.repeat(cu[:-1], lens)
+    tiles = build_prefill_tiles(lens, nh, nh).numpy().reshape(-1)
+    parts = [ids, pos, cu, lens, rows, tiles]
+    at = np.cumsum([0] + [len(p) for p in parts]).tolist()
+    ints = torch.from_numpy(np.concatenate(parts).astype(np.int32, copy=False)).to(dev)
+    L, cus, c = _lib.lib(), _cu_count(), _lib.EncoderCall()
+    slab = 0
+    for i, (N, K) in enumerate(((3 * H, H), (H, H), (I, H), (H, I))):
+        plan = ((0, T, -1, 1),) if T <= 64 else gemm_plan(T, N, K, True, cus)
+        c.plans[i].n = len(plan)
+        for j, (r0, r1, mi, S) in enumerate(plan):
+            c.plans[i].p[j] = _lib.GemmPiece(r0, r1, mi, S)
+            slab = max(slab, S * (r1 - r0) * N if S > 1 else 0)
+    # activations in the order h, a, attn, qkv, f, then the slabs
+    sizes = [2 * T * n for n in (H, H, H, 3 * H, I)] + [4 * slab]
+    off = np.cumsum([0] + [-(-n // 256) * 256 for n in sizes]).tolist()
+    buf = torch.empty(off[-1], dtype=torch.uint8, device=dev)
+    p, q = buf.data_ptr(), ints.data_ptr()
+    c.h, c.a, c.attn, c.qkv, c.f, c.ws = (p + o for o in off[:-1])
+    c.ids, c.pos, c.cu, c.lens, c.rows, c.tiles = (q + 4 * o for o in at[:-1])
+    table = [t.data_ptr() for layer in w.layers for t in map(layer.__getitem__, ENCODER_LAYER)]
+    ptrs = (ctypes.c_void_p * len(table))(*table)
+    c.layers = ctypes.addressof(ptrs)
+    c.word, c.pos_table, c.type_row = w.word.data_ptr(), w.pos.data_ptr(), w.type_row.data_ptr()
+    c.ln_g, c.ln_b, c.out, c.ldo = w.ln_g.data_ptr(), w.ln_b.data_ptr(), out.data_ptr(), out.stride(0)
+    c.n_layers, c.T, c.B, c.H, c.I, c.heads, c.n_tiles = len(w.layers), T, B, H, I, nh, len(tiles) // 2
+    c.pooling, c.normalize, c.eps = {"cls": 0, "mean": 1, "last": 2}[cfg.pooling], int(cfg.normalize), float(cfg.layer_norm_eps)
+    check(L.ragk_encoder_forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
+    return out
+
+
 def silu_mul(x, out=None):
     _bf16_2d(x, "x")
     T, I2 = x.shape

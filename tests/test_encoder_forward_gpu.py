@@ -1,0 +1,48 @@
+"""The native encoder forward (csrc/kernels/encoder.hip) against the layer-by-layer path."""
+import numpy as np
+import pytest
+import torch
+
+from rag_llm_k8s_amd.engine.encoder_engine import EmbeddingEngine
+from rag_llm_k8s_amd.models import encoder as E
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def model(pooling, hidden=256, heads=4, inter=512, kind="bert"):
+    cfg = E.EncoderConfig(model_type=kind, vocab_size=500, hidden_size=hidden, num_hidden_layers=2, num_attention_heads=heads,
+                          intermediate_size=inter, max_position_embeddings=512, pooling=pooling,
+                          pad_token_id=1 if kind == "xlm-roberta" else 0)
+    return E.EncoderModel(cfg, E.EncoderWeights.random(cfg, DEV, seed=3), DEV)
+
+
+@pytest.mark.parametrize("pooling,kind", [("cls", "xlm-roberta"), ("mean", "bert")])
+@pytest.mark.parametrize("lens", [[1], [14], [63, 1], [30, 35], [129, 7, 300, 64, 1], [200] * 9])
+def test_native_forward_is_the_layered_one(native, pooling, kind, lens):
+    """Bit for bit, one launch plan in both: few rows (skinny products), past 64 (tiles), rows written where they belong."""
+    m = model(pooling, kind=kind)
+    ids = np.random.RandomState(sum(lens)).randint(0, 500, sum(lens)).astype(np.int32)
+    ref = m.forward_packed(torch.from_numpy(ids).to(DEV), lens)
+    out = torch.full((len(lens) + 2, 256), 9.0, device=DEV)
+    rows = np.random.RandomState(1).permutation(len(lens)) + 1
+    m.embed_into(ids, np.asarray(lens, dtype=np.int64), out, rows)
+    assert native.encoder_forward_ok(m.cfg, m.w)
+    assert torch.equal(out[torch.from_numpy(rows).to(DEV)], ref)
+    assert bool((out[0] == 9.0).all()) and bool((out[-1] == 9.0).all())
+
+
+def test_engine_order_and_odd_outputs(native):
+    """Batches cut by tokens, unsorted lengths; an output that the native call does not take (strided columns) still works."""
+    m = model("mean")
+    eng = EmbeddingEngine(m, None, max_batch_tokens=150)
+    r = np.random.RandomState(0)
+    lists = [r.randint(0, 500, n).tolist() for n in (5, 120, 33, 1, 64, 90)]
+    got = eng.embed_ids(lists)
+    for x, y in zip(lists, got):
+        one = m.forward_packed(torch.tensor(x, dtype=torch.int32, device=DEV), [len(x)])[0]
+        assert torch.nn.functional.cosine_similarity(one, y, dim=0).item() > 0.999
+    cols = torch.zeros(256, len(lists), device=DEV).t()
+    ids, lens = np.concatenate(lists).astype(np.int32), np.array([len(x) for x in lists], dtype=np.int32)
+    eng.embed_flat(ids, lens, cols)
+    assert torch.equal(cols, got)

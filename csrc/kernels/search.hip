@@ -4,8 +4,7 @@
 //
 // The database stays resident in HBM in a COLUMN-major layout xt[d][cap] (cap = row
 // capacity): lane l of a wave reads row r0 + l of one dimension per load, 256 contiguous
-// bytes per wave instruction, no LDS for the data. Queries are staged in LDS in 256-dim
-// chunks and read as broadcasts. Distances are sum((x - q)^2) in fp32 (faiss' exact path).
+// bytes per wave instruction, no LDS for the data. Queries come by scalar loads. Distances are sum((x - q)^2) in fp32 (faiss' exact path).
 //
 // Top-k without sorting the scanned rows: every wave keeps a RUNNING sorted top-64 list per
 // query in its lanes (lane j = j-th best). A tile of 64 fresh distances (one per lane) is
@@ -26,7 +25,7 @@ using namespace ragk;
 namespace {
 
 constexpr int ST = 256;   // threads per block (4 waves)
-constexpr int DCH = 256;  // query dims staged per LDS chunk
+constexpr int DCH = 256;  // dims that the slices of a row tile split between them at a time
 constexpr int UNR = 16;   // dims (independent loads) in flight per lane
 
 // wave_offer for QB queries at once (the same 64 rows, one candidate per lane and query): the QB
@@ -104,53 +103,63 @@ __device__ __forceinline__ void wave_offer_multi(float (&bv)[NQ], int (&bi)[NQ],
     for (int q = 0; q < NQ; ++q) cx(bv[q], bi[q], lane, j, true);
 }
 
-// Distances of rows [rbase, rbase + 64) (one per lane; rows clamped into [0, cap)) over dims
-// [t0, t1) of the staged chunk starting at dim dc, for QB queries.
-template <int QB, int U = (QB <= 2 ? 32 : UNR)>
-__device__ __forceinline__ void scan_dims(const float* __restrict__ xt, size_t cap, int rc, int dc, int t0, int t1,
-                                          const float* qs, float* acc) {
-  const float* col = xt + (size_t)(dc + t0) * cap + rc;
+// Distances of 64 rows (one per lane, at xt + rc) over dims [t0, t1) for QB queries, whose values are wave-uniform: they come
+// by scalar loads (qp[j] = query j, or the last one past the batch), so no LDS, staging or barrier stands between the loads
+// of the rows. U dims in flight.
+template <int QB, int U = (QB <= 2 ? 32 : QB <= 4 ? 16 : 8)>
+__device__ __forceinline__ void scan_dims(const float* __restrict__ xt, size_t cap, int rc, int t0, int t1,
+                                          const float* const (&qp)[QB], float* acc) {
+  const float* col = xt + (size_t)t0 * cap + rc;
   int t = t0;
   for (; t + U <= t1; t += U, col += U * cap) {
     float x[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) x[u] = col[(size_t)u * cap];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int j = 0; j < QB; ++j) {
 #pragma unroll
-      for (int j = 0; j < QB; ++j) {
-        const float df = x[u] - qs[j * DCH + t + u];
+      for (int u = 0; u < U; ++u) {
+        const float df = x[u] - qp[j][t + u];
         acc[j] = fmaf(df, df, acc[j]);
       }
+    }
   }
   for (; t < t1; ++t, col += cap) {
     const float x = *col;
 #pragma unroll
     for (int j = 0; j < QB; ++j) {
-      const float df = x - qs[j * DCH + t];
+      const float df = x - qp[j][t];
       acc[j] = fmaf(df, df, acc[j]);
     }
   }
 }
 
 // Flat scan. Row tile = 64 * (4 / S) rows: wave w scans rows 64 * (w / S) .. +63 of the tile over
-// dim slice w % S of every 256-dim chunk. Block bx handles tiles bx, bx + gridDim.x, ...; its
+// dim slice w % S of every 256-dim chunk. Block bx of G handles tiles bx, bx + G, ...; its
 // queries are q0 = blockIdx.y * QB .. + QB. Output: per query one sorted list of k at [q][bx].
+// Grid (8, query groups, ceil(G / 8)): workgroups go to the XCDs in turn, so the groups that read the same rows are
+// neighbours on one XCD and all but the first find them in its L2: 13 queries of 500000 x 1024 take 528 us, as grid (G, query
+// groups), where each group streams the index from HBM, 724. (Before, with the queries' chunks staged in LDS: 8 queries 710 us
+// and now 408, 13 queries 1032, 32 queries of k = 10 1340 and now 901; 8 of 10000 x 1024: 71 and 37, launches included.)
 template <int QB, int S>
 __global__ __launch_bounds__(ST) void l2_scan_kernel(const float* __restrict__ xt, int cap, int d, int row_begin,
                                                      int row_end, int ntiles, const float* __restrict__ q, int nq,
                                                      int k, float* __restrict__ out_d, int* __restrict__ out_i,
-                                                     const int* __restrict__ ids_map) {
+                                                     const int* __restrict__ ids_map, int G) {
   constexpr int RG = 4 / S;
   constexpr int RB = 64 * RG;
+  const int bx = blockIdx.z * 8 + blockIdx.x;
+  if (bx >= G) return;
   extern __shared__ __attribute__((aligned(16))) float sc_smem[];
-  float* qs = sc_smem;              // [QB][DCH]
-  float* red = sc_smem + QB * DCH;  // [S - 1][RG][QB][64]
+  float* red = sc_smem;  // [S - 1][RG][QB][64]
   __shared__ float mv[4][64];
   __shared__ int mi[4][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = w / S, s = w % S;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = w / S, s = w % S;
   const int q0 = blockIdx.y * QB;
   const int nqb = min(QB, nq - q0);
+  const float* qp[QB];
+#pragma unroll
+  for (int j = 0; j < QB; ++j) qp[j] = q + (size_t)(q0 + min(j, nqb - 1)) * d;
   float bv[QB];
   int bi[QB];
 #pragma unroll
@@ -158,7 +167,7 @@ __global__ __launch_bounds__(ST) void l2_scan_kernel(const float* __restrict__ x
     bv[j] = FLT_MAX;
     bi[j] = -1;
   }
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+  for (int tile = bx; tile < ntiles; tile += G) {
     const int row = row_begin + tile * RB + 64 * g + lane;
     const int rc = min(row, cap - 1);  // rows in [row_end, cap) are valid memory; masked below
     float acc[QB];
@@ -166,17 +175,12 @@ __global__ __launch_bounds__(ST) void l2_scan_kernel(const float* __restrict__ x
     for (int j = 0; j < QB; ++j) acc[j] = 0.f;
     for (int dc = 0; dc < d; dc += DCH) {
       const int dn = min(DCH, d - dc);
-      __syncthreads();  // previous chunk (and the previous tile's slice reduction) consumed
-      for (int e = threadIdx.x; e < QB * DCH; e += ST) {
-        const int j = e / DCH, t = e % DCH;
-        qs[e] = (j < nqb && t < dn) ? q[(size_t)(q0 + j) * d + dc + t] : 0.f;
-      }
-      __syncthreads();
       const int per = (dn + S - 1) / S;
       const int t0 = min(dn, s * per), t1 = min(dn, t0 + per);
-      scan_dims<QB>(xt, (size_t)cap, rc, dc, t0, t1, qs, acc);
+      scan_dims<QB>(xt, (size_t)cap, rc, dc + t0, dc + t1, qp, acc);
     }
     if (S > 1) {
+      __syncthreads();  // the previous tile's slices are summed
       if (s > 0) {
 #pragma unroll
         for (int j = 0; j < QB; ++j) red[(((s - 1) * RG + g) * QB + j) * 64 + lane] = acc[j];
@@ -212,7 +216,7 @@ __global__ __launch_bounds__(ST) void l2_scan_kernel(const float* __restrict__ x
         for (int gg = 1; gg < RG; ++gg) wave_merge64(bv[j], bi[j], mv[gg][lane], mi[gg][lane], lane);
     }
     if (w == 0 && lane < k) {
-      const size_t o = ((size_t)(q0 + j) * gridDim.x + blockIdx.x) * k + lane;
+      const size_t o = ((size_t)(q0 + j) * G + bx) * k + lane;
       out_d[o] = bv[j];
       out_i[o] = bi[j];
     }
@@ -221,60 +225,84 @@ __global__ __launch_bounds__(ST) void l2_scan_kernel(const float* __restrict__ x
 
 // Batched queries (nq >= 16: the BLAS path of faiss' IndexFlatL2): ||x||^2 + ||q||^2 - 2 x.q with the
 // dot products on the exact fp32-input MFMA (v_mfma_f32_16x16x4_f32: a k-ordered fmaf chain), 16 rows x
-// 16 queries per instruction. Block = 4 waves x 64 rows per iteration, QT query tiles of 16 (all of a
-// <= 32-query batch in one block: the index is streamed from HBM once). Lane l of a wave loads
-// x[row0 + 16 rt + (l & 15)][k0 + (l >> 4)] (A fragment) and reads q^T[k0 + (l >> 4)][16 qt + (l & 15)]
-// from LDS (B fragment); its accumulators hold rows 16 rt + 4 (l >> 4) + r of query 16 qt + (l & 15).
-// Selection: every lane keeps a sorted list of the MK best (distance, id) of its query among the rows
-// it sees (MK >= k; a quarter of the rows of its query per wave), and the block merges the 16 lists of
-// each query (4 lanes x 4 waves) -> one sorted list of k per query. Distances clamp at 0 like faiss.
+// 16 queries per instruction, QT query tiles of 16 (all of a <= 32-query batch in one block: the index is streamed
+// from HBM once).
+//
+// The stream bounds it (32 queries: 209 us of MFMA for the 2 GB that take 360 us to read), so nothing may stand between
+// a wave and its next loads: the whole q^T lies in LDS (up to 128 KB, one block of 8 waves a CU), staged once, and each
+// wave walks its own tiles of 16 * RT rows without a barrier, three groups of loads deep. Row RT m + rt of a tile is row m
+// of MFMA rt, so the A operands of the RT MFMAs are one load of RT consecutive rows of a dimension: 16 B a lane at RT = 4.
+// (Before: 4-wave blocks that staged q^T in chunks of 256 dims for every 256 rows, 4-B loads.)
+// 32 queries, 500000 x 1024: 606 -> 387 us; 100000 x 1024: 250 -> 124; 10000 x 384: 40 -> 29 (launches included).
+//
+// Lane l of a wave holds x[rows][k0 + (l >> 4)] (A fragment), reads q^T[k0 + (l >> 4)][16 qt + (l & 15)] (B fragment), and
+// its accumulators hold MFMA rows 4 (l >> 4) + r of query 16 qt + (l & 15).
+// Selection: every lane keeps a sorted list of the MK best (distance, id) of its query among the rows it sees
+// (MK >= k); the four lanes of a query merge theirs, then the block its waves' -> one sorted list of k per query.
+// Distances clamp at 0 like faiss.
 constexpr int MQ_MK = 8;   // k <= 8 on this path
-constexpr int MQ_KU = 8;   // k-steps (of 4 dims) per unrolled group
+constexpr int MQ_KU = 4;   // k-steps (of 4 dims) per group of loads
 constexpr int MQ_DMAX = 1024;
+constexpr int MQ_NW = 8;   // waves of a block
+constexpr int MQ_CAND = MQ_NW * MQ_MK;  // candidates of a query at the block's merge: one a lane
+static_assert(MQ_CAND == 64, "one wave merges a query");
 
-constexpr int MQ_DCH = 256;  // query dims staged per LDS chunk (4 blocks per CU fit)
-// LDS floats of region 0: a q^T chunk during the scan, the candidate lists at the merge (aliased)
-__host__ __device__ inline int mq_region0(int d, int QT) {
-  return max(min(d, MQ_DCH) * 16 * QT, 2 * 16 * QT * 128);
-}
+// LDS floats: q^T during the scan, the candidates (values, ids) at the merge; then ||q||^2 and the waves' ||x||^2
+__host__ __device__ inline int mq_region0(int d, int QT) { return max(d * 16 * QT, 2 * 16 * QT * MQ_CAND); }
+__host__ __device__ inline int mq_floats(int d, int QT) { return mq_region0(d, QT) + 16 * QT + MQ_NW * 64; }
 
 template <int QT, int RT>
-__global__ __launch_bounds__(ST) void l2_mfma_kernel(const float* __restrict__ xt, int cap, int d, int row_begin,
-                                                     int row_end, int ntiles, const float* __restrict__ q, int nq,
-                                                     int k, float* __restrict__ out_d, int* __restrict__ out_i,
-                                                     const int* __restrict__ ids_map) {
+__global__ __launch_bounds__(MQ_NW * 64, 2) void l2_mfma_kernel(const float* __restrict__ xt, int cap, int d, int row_begin,
+                                                             int row_end, int ntiles, const float* __restrict__ q, int nq,
+                                                             int k, float* __restrict__ out_d, int* __restrict__ out_i,
+                                                             const int* __restrict__ ids_map) {
+  constexpr int NQ = 16 * QT, TH = MQ_NW * 64;
+  // RT consecutive rows of a dimension; only 4-byte aligned (cap and row_begin are arbitrary)
+  struct __attribute__((packed, aligned(4))) Rows { float v[RT]; };
   extern __shared__ __attribute__((aligned(16))) float mq_smem[];
-  float* qsT = mq_smem;                              // [MQ_DCH][16 * QT]: q transposed, one dim chunk
-  float* cd = mq_smem;                               // [16 * QT][128] candidates (merge, aliases qsT)
-  int* ci = reinterpret_cast<int*>(mq_smem + 16 * QT * 128);
-  float* qn = mq_smem + mq_region0(d, QT);           // [16 * QT] ||q||^2
-  float* xnl = qn + 16 * QT;                         // [4 waves][16 * RT] ||x||^2 of the wave's rows
+  float* qsT = mq_smem;                              // [d][16][QT]
+  float* cd = mq_smem;                               // [NQ][MQ_CAND] candidates (merge, aliases qsT)
+  int* ci = reinterpret_cast<int*>(mq_smem + NQ * MQ_CAND);
+  float* qn = mq_smem + mq_region0(d, QT);           // [NQ] ||q||^2
+  float* xnl = qn + NQ;                              // [waves][64] ||x||^2 of the wave's rows
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int q0 = blockIdx.y * 16 * QT;
-  const int nqb = min(16 * QT, nq - q0);
-  {
-    // ||q||^2 by the whole block: query j = tid / QP, part p = tid % QP sums dims p, p + QP, ...
-    // (consecutive threads read consecutive floats, 8 loads in flight), parts summed in order by
-    // shuffles. One thread per query walking all d dims with a dependent load each was ~60 us of a
-    // 10k-row search.
-    constexpr int QP = ST / (16 * QT);  // parts per query: 8 (QT 2) or 16 (QT 1)
-    const int j = threadIdx.x / QP, p = threadIdx.x % QP;
-    float sq = 0.f;
-    if (j < nqb) {
-      const float* qr = q + (size_t)(q0 + j) * d;
-      int t = p;
-      for (; t + 7 * QP < d; t += 8 * QP) {
-        float v[8];
+  const int q0 = blockIdx.y * NQ;
+  const int nqb = min(NQ, nq - q0);
+  // consecutive threads take consecutive queries, so the transposed LDS words they write are consecutive; eight loads a
+  // thread in flight
+  struct __attribute__((packed, aligned(4))) Quad { float v[4]; };
+  const int quads = NQ * (d >> 2);
+  for (int e0 = threadIdx.x; e0 < quads; e0 += 8 * TH) {
+    Quad v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = qr[t + u * QP];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) sq = fmaf(v[u], v[u], sq);
-      }
-      for (; t < d; t += QP) sq = fmaf(qr[t], qr[t], sq);
+    for (int u = 0; u < 8; ++u) {
+      const int e = min(e0 + u * TH, quads - 1);
+      v[u] = *reinterpret_cast<const Quad*>(q + (size_t)(q0 + min(e % NQ, nqb - 1)) * d + (e / NQ) * 4);
     }
 #pragma unroll
-    for (int o = 1; o < QP; o <<= 1) sq += __shfl_xor(sq, o, 64);
-    if (p == 0) qn[j] = sq;
+    for (int u = 0; u < 8; ++u) {
+      const int e = e0 + u * TH;
+      if (e < quads) {
+        const int j = e % NQ, t = (e / NQ) * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) qsT[(t + i) * NQ + (j & 15) * QT + (j >> 4)] = j < nqb ? v[u].v[i] : 0.f;
+      }
+    }
+  }
+  __syncthreads();
+  {
+    // ||q||^2: thread (part p, word j) sums dims p, p + P, ...; the parts are added in order
+    constexpr int P = TH / NQ;
+    const int j = threadIdx.x % NQ, p = threadIdx.x / NQ;
+    float sq = 0.f;
+#pragma unroll 8
+    for (int t = p; t < d; t += P) sq = fmaf(qsT[t * NQ + j], qsT[t * NQ + j], sq);
+    xnl[p * NQ + j] = sq;  // TH floats
+    __syncthreads();
+    if (p == 0) {
+      for (int o = 1; o < P; ++o) sq += xnl[o * NQ + j];
+      qn[(j % QT) * 16 + j / QT] = sq;
+    }
   }
   __syncthreads();
   const int fr = lane & 15, fg = lane >> 4;
@@ -291,11 +319,12 @@ __global__ __launch_bounds__(ST) void l2_mfma_kernel(const float* __restrict__ x
   float qnv[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) qnv[qt] = qn[16 * qt + fr];
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int rbase = row_begin + tile * (64 * RT) + 16 * RT * w;
-    int rc[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) rc[rt] = min(rbase + 16 * rt + fr, cap - 1);
+  const float* qb = qsT + fg * NQ + fr * QT;
+  float* xw = xnl + 64 * w;
+  for (int tile = w * gridDim.x + blockIdx.x; tile < ntiles; tile += MQ_NW * gridDim.x) {
+    const int first = row_begin + tile * 16 * RT;
+    // a tile over the store's end moves back (the rows of the tile before it are masked below), so that it loads like any
+    const int rbase = max(0, min(first, cap - 16 * RT));
     f32x4 acc[RT][QT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -304,97 +333,90 @@ __global__ __launch_bounds__(ST) void l2_mfma_kernel(const float* __restrict__ x
     float xs[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) xs[rt] = 0.f;
-    for (int dc = 0; dc < d; dc += MQ_DCH) {
-    const int dn = min(MQ_DCH, d - dc);  // host guarantees d % (4 * MQ_KU) == 0
-    __syncthreads();  // every wave is done with the previous chunk
-    // q^T chunk: consecutive threads read consecutive dims of one query (coalesced; the transposed LDS
-    // writes are the cheap side)
-    // (8 loads per thread in flight: a one-at-a-time loop paid a full L2 latency per element)
-    const int tot = dn * 16 * QT;
-    for (int e0 = threadIdx.x; e0 < tot; e0 += 16 * ST) {
-      float v[16];
+    const int nk = d / 4;  // multiple of MQ_KU
+    auto mma = [&](int t, const Rows& a) __attribute__((always_inline)) {  // k-step t
+      float b[QT];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int e = min(e0 + u * ST, tot - 1);
-        const int j = e / dn, t = e % dn;
-        v[u] = q[(size_t)(q0 + min(j, nqb - 1)) * d + dc + t];
-      }
+      for (int qt = 0; qt < QT; ++qt) b[qt] = qb[4 * t * NQ + qt];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int e = e0 + u * ST;
-        if (e < tot) {
-          const int j = e / dn, t = e % dn;
-          qsT[t * 16 * QT + j] = j < nqb ? v[u] : 0.f;
-        }
-      }
-    }
-    __syncthreads();
-    // index columns of the next group of MQ_KU k-steps are requested before the current group's
-    // MFMAs (two register buffers, loop unrolled by two): one group at a time left every group
-    // waiting a full memory latency (12 round trips per 384-dim tile)
-    const int nk = dn / 4;  // multiple of MQ_KU
-    auto load_grp = [&](int k0, float (&a)[MQ_KU][RT]) {
+      for (int rt = 0; rt < RT; ++rt) {
+        xs[rt] = fmaf(a.v[rt], a.v[rt], xs[rt]);
 #pragma unroll
-      for (int u = 0; u < MQ_KU; ++u) {
-        const float* col = xt + (size_t)(dc + 4 * (k0 + u) + fg) * cap;
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) a[u][rt] = col[rc[rt]];
+        for (int qt = 0; qt < QT; ++qt) acc[rt][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[rt], b[qt], acc[rt][qt], 0, 0, 0);
       }
     };
-    auto mma_grp = [&](int k0, const float (&a)[MQ_KU][RT]) {
+    if (rbase + 16 * RT <= cap) {
+      const float* col = xt + (size_t)fg * cap + rbase + RT * fr;
+      auto load_grp = [&](Rows (&a)[MQ_KU]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int u = 0; u < MQ_KU; ++u) {
-        float b[QT];
+        for (int u = 0; u < MQ_KU; ++u) {
+          a[u] = *reinterpret_cast<const Rows*>(col);
+          col += (size_t)4 * cap;
+        }
+      };
+      auto mma_grp = [&](int k0, const Rows (&a)[MQ_KU]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) b[qt] = qsT[(4 * (k0 + u) + fg) * 16 * QT + 16 * qt + fr];
+        for (int u = 0; u < MQ_KU; ++u) mma(k0 + u, a[u]);
+      };
+      // four register buffers, refilled as soon as their MFMAs are issued (a group's take 0.4 us, the other wave of the SIMD
+      // as long): three groups in flight
+      constexpr int NB = 4;
+      Rows a[NB][MQ_KU];
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-          xs[rt] = fmaf(a[u][rt], a[u][rt], xs[rt]);
+      for (int i = 0; i < NB; ++i)
+        if (i * MQ_KU < nk) load_grp(a[i]);
+#pragma unroll 1
+      for (int k0 = 0; k0 < nk; k0 += NB * MQ_KU) {
 #pragma unroll
-          for (int qt = 0; qt < QT; ++qt)
-            acc[rt][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][rt], b[qt], acc[rt][qt], 0, 0, 0);
+        for (int i = 0; i < NB; ++i) {
+          if (k0 + i * MQ_KU >= nk) break;
+          mma_grp(k0 + i * MQ_KU, a[i]);
+          if (k0 + (i + NB) * MQ_KU < nk) load_grp(a[i]);
         }
       }
-    };
-    // three register buffers, two groups in flight ahead of the MFMAs (a group's 8 k-steps of MFMA
-    // are far shorter than one memory latency)
-    float a0[MQ_KU][RT], a1[MQ_KU][RT], a2[MQ_KU][RT];
-    load_grp(0, a0);
-    if (MQ_KU < nk) load_grp(MQ_KU, a1);
-    for (int k0 = 0; k0 < nk; k0 += 3 * MQ_KU) {
-      if (k0 + 2 * MQ_KU < nk) load_grp(k0 + 2 * MQ_KU, a2);
-      mma_grp(k0, a0);
-      if (k0 + MQ_KU >= nk) break;
-      if (k0 + 3 * MQ_KU < nk) load_grp(k0 + 3 * MQ_KU, a0);
-      mma_grp(k0 + MQ_KU, a1);
-      if (k0 + 2 * MQ_KU >= nk) break;
-      if (k0 + 4 * MQ_KU < nk) load_grp(k0 + 4 * MQ_KU, a1);
-      mma_grp(k0 + 2 * MQ_KU, a2);
+    } else {  // a store smaller than a tile: one row at a time, clamped
+#pragma unroll 1
+      for (int t = 0; t < nk; ++t) {
+        Rows a;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) a.v[rt] = xt[(size_t)(4 * t + fg) * cap + min(rbase + RT * fr + rt, cap - 1)];
+        mma(t, a);
+      }
     }
-    }  // dim chunk
-    // ||x||^2 of row 16 rt + fr: the 4 dim phases (lanes fr, fr+16, fr+32, fr+48) summed in order
+    // ||x||^2 of row RT fr + rt: the 4 dim phases (lanes fr, fr+16, fr+32, fr+48) summed in order
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       float t = xs[rt];
       t += __int_as_float(xor_lane(__float_as_int(t), 16, lane));
       t += __int_as_float(xor_lane(__float_as_int(t), 32, lane));
-      if (fg == 0) xnl[w * 16 * RT + 16 * rt + fr] = t;
+      if (fg == 0) xw[RT * fr + rt] = t;
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's xnl writes landed (wave-local rows)
     __builtin_amdgcn_wave_barrier();
+    // a lane's rows in ascending order: without a map of ids an equal distance stays behind the ones already listed, and
+    // an insertion is one median a slot (l'[m] = med3(l[m - 1], l[m], c)) instead of a chain of compare-exchanges
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int rl = 16 * rt + 4 * fg + r;
+      for (int rt = 0; rt < RT; ++rt) {
+        const int rl = RT * (4 * fg + r) + rt;
         const int row = rbase + rl;
-        const bool ok = row < row_end;
+        const bool ok = row >= first && row < row_end;
         const int id = ok ? (ids_map ? ids_map[row] : row) : -1;
-        const float xn = xnl[w * 16 * RT + rl];
+        const float xn = xw[rl];
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
           const float dv = ok ? fmaxf(xn + qnv[qt] - 2.f * acc[rt][qt][r], 0.f) : FLT_MAX;
-          if (cand_lt(dv, id, lv[qt][MQ_MK - 1], lix[qt][MQ_MK - 1])) {  // insert (rare once warm)
+          if (!ids_map) {
+            if (dv < lv[qt][MQ_MK - 1]) {
+#pragma unroll
+              for (int m = MQ_MK - 1; m >= 0; --m) {
+                const bool here = dv < lv[qt][m], before = m > 0 && dv < lv[qt][m > 0 ? m - 1 : 0];
+                lix[qt][m] = before ? lix[qt][m > 0 ? m - 1 : 0] : (here ? id : lix[qt][m]);
+                lv[qt][m] = m > 0 ? __builtin_amdgcn_fmed3f(lv[qt][m > 0 ? m - 1 : 0], lv[qt][m], dv) : fminf(lv[qt][0], dv);
+              }
+            }
+          } else if (cand_lt(dv, id, lv[qt][MQ_MK - 1], lix[qt][MQ_MK - 1])) {
             float cv = dv;
             int cidx = id;
 #pragma unroll
@@ -413,34 +435,44 @@ __global__ __launch_bounds__(ST) void l2_mfma_kernel(const float* __restrict__ x
       }
     __builtin_amdgcn_wave_barrier();
   }
-  // merge: query j's lists live in lanes with fr == j % 16 of every wave: 4 waves x 4 lane groups x MQ_MK
-  __syncthreads();  // every wave is done reading q^T: the candidate lists reuse its LDS
+  // a query's four lanes (fr, fr + 16, + 32, + 48) emit the best MK of their lists in order: the smallest head goes out,
+  // its lane moves on
+  __syncthreads();  // every wave is done reading q^T: the candidates reuse its LDS
 #pragma unroll
-  for (int qt = 0; qt < QT; ++qt)
+  for (int m = 0; m < MQ_MK; ++m)
 #pragma unroll
-    for (int m = 0; m < MQ_MK; ++m) {
-      const int j = 16 * qt + fr;
-      const int slot = (w * 4 + fg) * MQ_MK + m;  // 0 .. 127
-      cd[(size_t)j * 128 + slot] = lv[qt][m];
-      ci[(size_t)j * 128 + slot] = lix[qt][m];
+    for (int qt = 0; qt < QT; ++qt) {
+      float mv = lv[qt][0];
+      int mi = lix[qt][0];
+#pragma unroll
+      for (int jx = 16; jx < 64; jx <<= 1) {
+        const float ov = __int_as_float(xor_lane(__float_as_int(mv), jx, lane));
+        const int oi = xor_lane(mi, jx, lane);
+        const bool take = cand_lt(ov, oi, mv, mi);
+        mv = take ? ov : mv;
+        mi = take ? oi : mi;
+      }
+      const bool won = (lv[qt][0] == mv) & (lix[qt][0] == mi);
+#pragma unroll
+      for (int n = 0; n < MQ_MK; ++n) {
+        lv[qt][n] = won ? (n + 1 < MQ_MK ? lv[qt][n + 1] : FLT_MAX) : lv[qt][n];
+        lix[qt][n] = won ? (n + 1 < MQ_MK ? lix[qt][n + 1] : -1) : lix[qt][n];
+      }
+      if (fg == 0) {
+        cd[(16 * qt + fr) * MQ_CAND + w * MQ_MK + m] = mv;
+        ci[(16 * qt + fr) * MQ_CAND + w * MQ_MK + m] = mi;
+      }
     }
   __syncthreads();
-  // wave w merges queries w, w + 4, ... (4 * QT of them). A query's 128 candidates are 16 sorted
-  // lists of MQ_MK: lane l holds entries 2 (l >> 4) and 2 (l >> 4) + 1 of list l & 15 (a sorted pair),
-  // and k rounds of a wave-wide argmin over the lanes' first entries emit the top k in order (the
-  // winner shifts its pair). Two full 64-lane bitonic offers per query cost ~3x the steps for k <= 8.
+  // a wave merges queries w, w + MQ_NW, ...: k rounds of a wave-wide argmin over the lanes' candidates, the winner drops out
   {
-    constexpr int NQW = 4 * QT;
-    float v0[NQW], v1[NQW];
-    int i0[NQW], i1[NQW];
-    const int slot = (lane & 15) * MQ_MK + 2 * (lane >> 4);
+    constexpr int NQW = NQ / MQ_NW;
+    float v0[NQW];
+    int i0[NQW];
 #pragma unroll
     for (int t = 0; t < NQW; ++t) {
-      const int j = w + 4 * t;
-      v0[t] = cd[(size_t)j * 128 + slot];
-      i0[t] = ci[(size_t)j * 128 + slot];
-      v1[t] = cd[(size_t)j * 128 + slot + 1];
-      i1[t] = ci[(size_t)j * 128 + slot + 1];
+      v0[t] = cd[(size_t)(w + MQ_NW * t) * MQ_CAND + lane];
+      i0[t] = ci[(size_t)(w + MQ_NW * t) * MQ_CAND + lane];
     }
     for (int r = 0; r < k; ++r) {
       float mv[NQW];
@@ -463,11 +495,9 @@ __global__ __launch_bounds__(ST) void l2_mfma_kernel(const float* __restrict__ x
 #pragma unroll
       for (int t = 0; t < NQW; ++t) {
         const bool won = (v0[t] == mv[t]) & (i0[t] == mi[t]);
-        v0[t] = won ? v1[t] : v0[t];
-        i0[t] = won ? i1[t] : i0[t];
-        v1[t] = won ? FLT_MAX : v1[t];
-        i1[t] = won ? -1 : i1[t];
-        const int j = w + 4 * t;
+        v0[t] = won ? FLT_MAX : v0[t];
+        i0[t] = won ? -1 : i0[t];
+        const int j = w + MQ_NW * t;
         if (j < nqb && lane == 0) {
           const size_t o = ((size_t)(q0 + j) * gridDim.x + blockIdx.x) * k + r;
           out_d[o] = mv[t];
@@ -539,7 +569,7 @@ __global__ __launch_bounds__(ST) void ivf_scan_kernel(const float* __restrict__ 
 
 // in: [nq][G][k] sorted lists -> out: [nq][k] (distances fp32, ids int64). One block of MW waves per query; each wave takes 64
 // candidates at a time (64 / k whole lists per step) and offers them to its running top list; the
-// waves' lists are merged last.
+// waves' lists are merged last, pairwise.
 constexpr int MW = 16;
 __global__ __launch_bounds__(MW * 64) void topk_lists_merge_kernel(const float* __restrict__ in_d,
                                                                    const int* __restrict__ in_i, int G, int k,
@@ -569,15 +599,18 @@ __global__ __launch_bounds__(MW * 64) void topk_lists_merge_kernel(const float* 
     v = vn;
     id = idn;
   }
-  mv[w][lane] = bv;
-  mi[w][lane] = bi;
-  __syncthreads();
-  if (w == 0) {
-    for (int gg = 1; gg < MW; ++gg) wave_merge64(bv, bi, mv[gg][lane], mi[gg][lane], lane);
-    if (lane < k) {
-      out_d[(size_t)qi * k + lane] = bv;
-      out_i[(size_t)qi * k + lane] = bi;  // int64 ids: the caller's final type, no widening launch
-    }
+  // the waves' lists as a tree: four dependent merges instead of fifteen
+#pragma unroll
+  for (int h = MW / 2; h > 0; h >>= 1) {
+    mv[w][lane] = bv;
+    mi[w][lane] = bi;
+    __syncthreads();
+    if (w < h) wave_merge64(bv, bi, mv[w + h][lane], mi[w + h][lane], lane);
+    __syncthreads();
+  }
+  if (w == 0 && lane < k) {
+    out_d[(size_t)qi * k + lane] = bv;
+    out_i[(size_t)qi * k + lane] = bi;  // int64 ids: the caller's final type, no widening launch
   }
 }
 
@@ -737,19 +770,20 @@ __global__ __launch_bounds__(256) void kmeans_assign_kernel(const float* __restr
 static int scan_slices(int n) { return n < 65536 ? 4 : (n < 262144 ? 2 : 1); }
 
 template <int QB, int S>
-static void launch_scan(dim3 grid, size_t lds, hipStream_t st, const float* xt, int cap, int d, int rb, int re,
+static void launch_scan(int G, size_t lds, hipStream_t st, const float* xt, int cap, int d, int rb, int re,
                         int ntiles, const float* q, int nq, int k, float* od, int* oi, const int* ids) {
+  const dim3 grid(8, (nq + QB - 1) / QB, (G + 7) / 8);
   hipLaunchKernelGGL((l2_scan_kernel<QB, S>), grid, dim3(ST), lds, st, xt, cap, d, rb, re, ntiles, q, nq, k, od, oi,
-                     ids);
+                     ids, G);
 }
 
 template <int QB>
-static void launch_scan_s(int S, dim3 grid, hipStream_t st, const float* xt, int cap, int d, int rb, int re,
+static void launch_scan_s(int S, int G, hipStream_t st, const float* xt, int cap, int d, int rb, int re,
                           int ntiles, const float* q, int nq, int k, float* od, int* oi, const int* ids) {
-  const size_t lds = (size_t)QB * DCH * 4 + (size_t)(S - 1) * (4 / S) * QB * 64 * 4;
-  if (S == 4) launch_scan<QB, 4>(grid, lds, st, xt, cap, d, rb, re, ntiles, q, nq, k, od, oi, ids);
-  else if (S == 2) launch_scan<QB, 2>(grid, lds, st, xt, cap, d, rb, re, ntiles, q, nq, k, od, oi, ids);
-  else launch_scan<QB, 1>(grid, lds, st, xt, cap, d, rb, re, ntiles, q, nq, k, od, oi, ids);
+  const size_t lds = (size_t)(S - 1) * (4 / S) * QB * 64 * 4;
+  if (S == 4) launch_scan<QB, 4>(G, lds, st, xt, cap, d, rb, re, ntiles, q, nq, k, od, oi, ids);
+  else if (S == 2) launch_scan<QB, 2>(G, lds, st, xt, cap, d, rb, re, ntiles, q, nq, k, od, oi, ids);
+  else launch_scan<QB, 1>(G, lds, st, xt, cap, d, rb, re, ntiles, q, nq, k, od, oi, ids);
 }
 
 // the MFMA path (batched queries, k <= 8, d % 32 == 0) for nq >= this
@@ -759,10 +793,11 @@ RAGK_API int ragk_l2_search_set_mfma_min_nq(int n) {
   return 0;
 }
 static bool use_mfma(int nq, int k, int d) {
-  return nq >= g_mfma_min_nq && k <= MQ_MK && d % (4 * MQ_KU) == 0 && d <= MQ_DMAX;
+  return nq >= g_mfma_min_nq && k <= MQ_MK && d % 32 == 0 && d <= MQ_DMAX;
 }
-static size_t mfma_lds(int d, int QT) { return ((size_t)mq_region0(d, QT) + 16 * QT + 4 * 64) * 4; }
-static int mfma_rt(int n) { return n < 262144 ? 1 : 4; }  // 16 or 64 rows per wave and tile
+static size_t mfma_lds(int d, int QT) { return (size_t)mq_floats(d, QT) * 4; }
+// rows of a wave's tile / 16: tiles for every wave of the chip before wider loads
+static int mfma_rt(int n) { return n >= 196608 ? 4 : (n >= 65536 ? 2 : 1); }
 
 // Number of partial lists per query the scan of rows [row_begin, row_end) emits (size the
 // partial buffers [nq][G][k] with it).
@@ -779,9 +814,7 @@ RAGK_API int ragk_l2_scan_groups(int row_begin, int row_end, int nq) {
 RAGK_API int ragk_l2_search_groups(int row_begin, int row_end, int nq, int k, int d) {
   if (!use_mfma(nq, k, d)) return ragk_l2_scan_groups(row_begin, row_end, nq);
   const int n = max(0, row_end - row_begin);
-  const int ntiles = (n + 64 * mfma_rt(n) - 1) / (64 * mfma_rt(n));
-  const int qgroups = (nq + 31) / 32;
-  return max(1, min(ntiles, max(1, 2048 / qgroups)));
+  return max(1, min((n + 16 * mfma_rt(n) - 1) / (16 * mfma_rt(n)), 256));  // a block a CU
 }
 
 // Exact top-k (k <= 64) over rows [row_begin, row_end) of xt[d][cap]; part_d / part_i hold
@@ -792,29 +825,31 @@ RAGK_API int ragk_l2_search(const float* xt, int cap, int d, int row_begin, int 
   if (nq <= 0) return 0;
   if (k < 1 || k > 64 || d < 1 || cap < 1 || row_end > cap) return (int)hipErrorInvalidValue;
   if (use_mfma(nq, k, d)) {
-    static bool attr = false;
-    if (!attr) {
-      hipError_t e = hipSuccess;
-      const void* fns[4] = {(const void*)l2_mfma_kernel<1, 1>, (const void*)l2_mfma_kernel<1, 4>,
-                            (const void*)l2_mfma_kernel<2, 1>, (const void*)l2_mfma_kernel<2, 4>};
-      for (int i = 0; i < 4 && e == hipSuccess; ++i)
-        e = hipFuncSetAttribute(fns[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)mfma_lds(MQ_DMAX, 1 + i / 2));
-      if (e != hipSuccess) return (int)e;
-      attr = true;
-    }
+    static const hipError_t attr = [] {
+      const void* fns[6] = {(const void*)l2_mfma_kernel<1, 1>, (const void*)l2_mfma_kernel<1, 2>,
+                            (const void*)l2_mfma_kernel<1, 4>, (const void*)l2_mfma_kernel<2, 1>,
+                            (const void*)l2_mfma_kernel<2, 2>, (const void*)l2_mfma_kernel<2, 4>};
+      for (int i = 0; i < 6; ++i) {
+        const hipError_t e = hipFuncSetAttribute(fns[i], hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int)mfma_lds(MQ_DMAX, 1 + i / 3));
+        if (e != hipSuccess) return e;
+      }
+      return hipSuccess;
+    }();
+    if (attr != hipSuccess) return (int)attr;
     const int n = max(0, row_end - row_begin);
     const int RT = mfma_rt(n);
-    const int ntiles = (n + 64 * RT - 1) / (64 * RT);
+    const int ntiles = (n + 16 * RT - 1) / (16 * RT);
     const int G = ragk_l2_search_groups(row_begin, row_end, nq, k, d);
-    const int QT = nq >= 32 ? 2 : 1;
+    const int QT = nq > 16 ? 2 : 1;
     const dim3 grid(G, (nq + 16 * QT - 1) / (16 * QT));
     const size_t lds = mfma_lds(d, QT);
-#define RAGK_MQ(Q, R) hipLaunchKernelGGL((l2_mfma_kernel<Q, R>), grid, dim3(ST), lds, st, xt, cap, d, row_begin, row_end, \
-                                         ntiles, q, nq, k, part_d, part_i, ids_map)
+#define RAGK_MQ(Q, R) hipLaunchKernelGGL((l2_mfma_kernel<Q, R>), grid, dim3(MQ_NW * 64), lds, st, xt, cap, d, row_begin, \
+                                         row_end, ntiles, q, nq, k, part_d, part_i, ids_map)
     if (QT == 2) {
-      if (RT == 4) RAGK_MQ(2, 4); else RAGK_MQ(2, 1);
+      if (RT == 4) RAGK_MQ(2, 4); else if (RT == 2) RAGK_MQ(2, 2); else RAGK_MQ(2, 1);
     } else {
-      if (RT == 4) RAGK_MQ(1, 4); else RAGK_MQ(1, 1);
+      if (RT == 4) RAGK_MQ(1, 4); else if (RT == 2) RAGK_MQ(1, 2); else RAGK_MQ(1, 1);
     }
 #undef RAGK_MQ
     hipError_t e = hipGetLastError();
@@ -826,15 +861,13 @@ RAGK_API int ragk_l2_search(const float* xt, int cap, int d, int row_begin, int 
   const int S = scan_slices(n);
   const int ntiles = (n + 64 * (4 / S) - 1) / (64 * (4 / S));
   const int G = ragk_l2_search_groups(row_begin, row_end, nq, k, d);
-  // queries per block: up to 16 (32 accumulators + the x[] ring would leave one wave per SIMD);
-  // the last group of the y-dimension may be partial (handled in-kernel)
-  const int QB = nq >= 16 ? 16 : (nq >= 8 ? 8 : (nq >= 4 ? 4 : (nq >= 2 ? 2 : 1)));
-  const dim3 grid(G, (nq + QB - 1) / QB);
-  if (QB == 16) launch_scan_s<16>(S, grid, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
-  else if (QB == 8) launch_scan_s<8>(S, grid, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
-  else if (QB == 4) launch_scan_s<4>(S, grid, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
-  else if (QB == 2) launch_scan_s<2>(S, grid, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
-  else launch_scan_s<1>(S, grid, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
+  // queries per block, padded to the next count below. Twelve or sixteen spill the scalar registers, and one pass of them loses
+  // to two groups of eight that share the L2: 12 queries of 500000 x 1024 594 us, 15 837; in groups of eight 528
+  const int QB = nq > 4 ? 8 : (nq > 2 ? 4 : nq);
+  if (QB == 8) launch_scan_s<8>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
+  else if (QB == 4) launch_scan_s<4>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
+  else if (QB == 2) launch_scan_s<2>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
+  else launch_scan_s<1>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
   hipLaunchKernelGGL(topk_lists_merge_kernel, dim3(nq), dim3(MW * 64), 0, st, part_d, part_i, G, k, out_d, out_i);

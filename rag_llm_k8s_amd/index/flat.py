@@ -79,8 +79,7 @@ class FlatL2Index:
             if self._n is not None:
                 if k > 64:
                     raise ValueError("k <= 64 on the GPU path")
-                D, I = self._n.l2_search(self._xt, self._cap, self.ntotal, q.to(self.device), k)
-                return D.cpu(), I.cpu()
+                return self._n.l2_search(self._xt, self._cap, self.ntotal, q.to(self.device), k, host=True)
             return self._cpu_search(q, k)
 
     def search_device(self, q, k):

@@ -237,9 +237,8 @@ class IVFFlatIndex:
 
                 qd = q.to(self.device, non_blocking=True)
                 pr = self._coarse_device(qd, nprobe)  # stays on the device: one host sync per search
-                D, I = native.ivf_search(self._xt, self._cap, qd, pr, self._start_dev, self._ids_dev, k,
-                                         max_list=int(self._size.max()), ends=self._end_dev)
-                return D.cpu(), I.cpu()
+                return native.ivf_search(self._xt, self._cap, qd, pr, self._start_dev, self._ids_dev, k,
+                                         max_list=int(self._size.max()), ends=self._end_dev, host=True)
             pr = probes(q.to(self.centroids.device), self.centroids, self._cnorm, nprobe).cpu()
             return self._search_host(q, pr, k)
 

@@ -1289,9 +1289,11 @@ _search_ws = {}
 _search_lock = threading.Lock()
 
 
-def _search_out(nq, k, device):
-    """(D fp32 [nq, k], I int64 [nq, k]) as views of ONE allocation (the merge kernel writes int64 ids)."""
-    buf = torch.empty(nq * k * 3, dtype=torch.int32, device=device)
+def _search_views(buf, nq, k, host):
+    """(D fp32 [nq, k], I int64 [nq, k]) as views of the ONE allocation a search writes, int64 ids first; host: of its copy there
+    (a copy of each result waits for the device twice)."""
+    if host:
+        buf = buf.cpu()
     return buf[2 * nq * k:].view(torch.float32).view(nq, k), buf[:2 * nq * k].view(torch.int64).view(nq, k)
 
 
@@ -1307,11 +1309,11 @@ def _search_partials(n_entries, device):
     return ws[:n_entries].view(torch.float32), ws[n_entries:2 * n_entries]
 
 
-def l2_search(xt, cap, n, q, k, row_begin=0, ids_map=None):
+def l2_search(xt, cap, n, q, k, row_begin=0, ids_map=None, host=False):
     """Exact squared-L2 top-k over rows [row_begin, n) of a column-major store xt[d][cap]
     (csrc/kernels/search.hip: l2_scan with wave-resident running top lists + one list merge; batches
     of >= 16 queries with k <= 8 on the fp32-MFMA distance GEMM, faiss' BLAS form).
-    Returns (D fp32 [nq,k], I int64 [nq,k]) with faiss padding semantics (-1, FLT_MAX).
+    Returns (D fp32 [nq,k], I int64 [nq,k]) with faiss padding semantics (-1, FLT_MAX), on the device or (host) in host memory.
     Host cost per call: one output allocation and two ctypes calls (the partial lists live in a
     cached workspace), so a single-query search is not dominated by launch overhead."""
     _req(xt.is_cuda and xt.dtype == torch.float32 and xt.is_contiguous() and xt.dim() == 2, "xt fp32 [d, cap]")
@@ -1323,19 +1325,19 @@ def l2_search(xt, cap, n, q, k, row_begin=0, ids_map=None):
     _req(xt.shape[1] == cap and 0 <= row_begin <= max(row_begin, n) <= cap, "rows within the store")
     _req(ids_map is None or (ids_map.dtype == torch.int32 and ids_map.is_cuda and ids_map.numel() >= n), "ids_map")
     L = _lib.lib()
-    od, oi = _search_out(nq, k, q.device)
+    out = torch.empty(nq * k * 3, dtype=torch.int32, device=q.device)
     if nq == 0:
-        return od, oi
+        return _search_views(out, nq, k, host)
     G = L.ragk_l2_search_groups(row_begin, max(n, row_begin), nq, k, d)
     with _search_lock:
         pd, pi = _search_partials(nq * G * k, q.device)
         check(L.ragk_l2_search(xt.data_ptr(), cap, d, row_begin, max(n, row_begin), q.data_ptr(), nq, k,
-                               ptr(ids_map), pd.data_ptr(), pi.data_ptr(), od.data_ptr(), oi.data_ptr(), stream_ptr()),
-              "ragk_l2_search")
-    return od, oi
+                               ptr(ids_map), pd.data_ptr(), pi.data_ptr(), out.data_ptr() + 8 * nq * k, out.data_ptr(),
+                               stream_ptr()), "ragk_l2_search")
+    return _search_views(out, nq, k, host)
 
 
-def ivf_search(xt, cap, q, probes, offsets, ids_map, k, max_list=None, ends=None):
+def ivf_search(xt, cap, q, probes, offsets, ids_map, k, max_list=None, ends=None, host=False):
     """IVF-Flat scan of the probed lists (one block per (query, probe), wave-resident top lists,
     then one list merge). probes int32 [nq, nprobe] (device; -1 = no list); list i occupies store rows
     [offsets[i], ends[i]) (ends None: packed lists, offsets has nlist+1 entries); ids_map int32 [cap]
@@ -1347,15 +1349,16 @@ def ivf_search(xt, cap, q, probes, offsets, ids_map, k, max_list=None, ends=None
     d = xt.shape[0]
     nq, nprobe = probes.shape
     _req(1 <= k <= 64 and d <= 2048 and nprobe >= 1, "k <= 64, d <= 2048")
-    od, oi = _search_out(nq, k, q.device)
+    out = torch.empty(nq * k * 3, dtype=torch.int32, device=q.device)
     if nq == 0:
-        return od, oi
+        return _search_views(out, nq, k, host)
     with _search_lock:
         pd, pi = _search_partials(nq * nprobe * k, q.device)
         check(_lib.lib().ragk_ivf_search(xt.data_ptr(), cap, d, q.data_ptr(), nq, probes.data_ptr(), nprobe,
                                          offsets.data_ptr(), ptr(ends), ids_map.data_ptr(), k, pd.data_ptr(),
-                                         pi.data_ptr(), od.data_ptr(), oi.data_ptr(), stream_ptr()), "ragk_ivf_search")
-    return od, oi
+                                         pi.data_ptr(), out.data_ptr() + 8 * nq * k, out.data_ptr(), stream_ptr()),
+              "ragk_ivf_search")
+    return _search_views(out, nq, k, host)
 
 
 def kmeans_assign(x, c, cnorm=None, scores=None):

@@ -63,10 +63,12 @@ def _names(raw):
 
 FAMILIES = (
     Family("niduvik", lambda raw: "niduvik" in _names(raw), _niduvik, ("bf16", "float32"),
-           ("gemm.hip", "gemm_mid.hip", "gemm_w4.hip", "gemm_pp.hip", "gemm_stream.hip", "gemm_dec.hip", "gemm_part.hip", "gemm_f32.hip",
+           ("gemm.hip", "gemm_hold.hip", "gemm_mid.hip", "gemm_w4.hip", "gemm_pp.hip", "gemm_stream.hip", "gemm_dec.hip",
+            "gemm_part.hip", "gemm_f32.hip",
             "norm.hip", "residual.hip", "attn_shaped.hip", "ssm.hip", "sampling.hip")),
     Family("rolesun", lambda raw: "rolesun" in _names(raw), _rolesun, ("bf16", "float32"),
-           ("gemm.hip", "gemm_mid.hip", "gemm_w4.hip", "gemm_pp.hip", "gemm_stream.hip", "gemm_dec.hip", "gemm_part.hip", "gemm_f32.hip",
+           ("gemm.hip", "gemm_hold.hip", "gemm_mid.hip", "gemm_w4.hip", "gemm_pp.hip", "gemm_stream.hip", "gemm_dec.hip",
+            "gemm_part.hip", "gemm_f32.hip",
             "norm.hip", "residual.hip", "attn_shaped.hip", "latent.hip", "sampling.hip")),
     Family("gpt2", lambda raw: "gpt2" in _names(raw), _gpt2, ("bf16",)),
     Family("llama", lambda raw: True, _llama, ("bf16", "fp8")),

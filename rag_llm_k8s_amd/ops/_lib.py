@@ -22,6 +22,8 @@ P, I, F, S, U64 = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_void_p
 _SIGS = {
     "ragk_gemm": [P, I, P, I, P, I, P, P, I, I, I, I, I, I, S],
     "ragk_gemm_path": [I, P, I, P, I, P, I, P, P, I, I, I, I, I, S],
+    "ragk_gemm_hold": [P, I, P, I, P, P, I, P, I, I, I, I, I, S],
+    "ragk_gemm_hold_rows": [I, I],
     "ragk_gemm_mid": [P, I, P, I, P, I, P, P, I, I, I, I, I, I, I, I, P, S],
     "ragk_gemm_mid_rope_kv": [P, I, P, I, P, I, I, I, P, P, P, P, P, P, I, I, I, I, I, P, S],
     "ragk_gemm_pp": [P, I, P, I, P, I, P, P, I, I, I, I, I, I, S],

@@ -220,6 +220,8 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
             return out
     if path == 0:
         return gemm_mid(x, w, bias=bias, resid=resid, epi=epi, out=out, out_f32=out_f32)
+    if path is None and use_hold(M, N, K, epi):
+        return gemm_hold(x, w, par=bias, epi=epi, out=out)
     if path is None and STREAM_DEFAULT and use_stream(M, N, K, epi):
         path = 5
     if path is None and DEC_DEFAULT and use_dec(M, N, K, epi):
@@ -820,6 +822,44 @@ def _gemm_stream(x, w, wscale, out, bias, resid, ldr, M, N, K, epi, e, out_f32):
                               cnt.data_ptr(), stream_ptr())
 
 
+def use_hold(M, N, K, epi, fp8=False):
+    """Packed gate/up projections whose activations fit a block's registers go to gemm_hold.hip: 11264 x 2048 bf16 at 12 / 50
+    rows 14.7 / 24 -> 11.8 / 17 us against the register-streaming kernel, 28672 x 4096 fp8 at 11 / 32 rows 38 / 37 -> 27.5 / 33
+    (gemm_fp8_dec / gemm_stream). Not where they lose: K of 1024 (a barrier for every 16 KB of weights: 28672 rows 10.3 against
+    8.7); row tiles that leave the last of a CU's few rounds mostly empty (6144 x 3072 bf16, 1.5 rounds: 11.9 against 11.4);
+    bf16 weights that the LDS ring streams without a K-split (28672 x 4096: 43 against 42); and more rows than one launch
+    holds, but for 8192 rows of fp8 and up, whose second launch reads the Infinity Cache while the ring is down to half its
+    depth (14336 x 4096 at 48 rows 51 -> 38, but 7168 x 4096 25 against 28)."""
+    if not 0 < M <= 64 or K < 2048 or epi not in PAIR_EPI or (fp8 and epi != "silu_mul"):
+        return False
+    per = _lib.lib().ragk_gemm_hold_rows(K, int(fp8))
+    if per == 0 or not (M <= per or (fp8 and 32 < M <= 2 * per and 2 * N >= 8192)):
+        return False
+    tiles, cus = N // 8, _cu_count()
+    if tiles > cus and tiles < (0.6 if fp8 else 0.78) * (-(-tiles // cus) * cus):
+        return False
+    return fp8 or not use_stream(M, N, K, epi) or _lib.lib().ragk_gemm_stream_splits(N, K, EPI[epi], 0) > 1
+
+
+def gemm_hold(x, w, wscale=None, par=None, epi="silu_mul", out=None):
+    """Packed gate/up projection of at most 64 rows with the activations held in registers (gemm_hold.hip); more rows than
+    one launch holds go in equal launches."""
+    L = _lib.lib()
+    M, K = x.shape
+    N = w.shape[0] // 2
+    if out is None:
+        out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    per = L.ragk_gemm_hold_rows(K, int(wscale is not None))
+    _req(per > 0 and w.shape[1] == K and epi in PAIR_EPI and 0 < M <= 64, "gemm_hold shape")
+    per = -(-M // -(-M // per))
+    for r0 in range(0, M, per):
+        xs, os_ = x[r0:r0 + per], out[r0:r0 + per]
+        check(L.ragk_gemm_hold(xs.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), ptr(wscale), os_.data_ptr(),
+                               out.stride(0), ptr(par), xs.shape[0], N, K, EPI[epi], _cu_count(), stream_ptr()),
+              "ragk_gemm_hold")
+    return out
+
+
 # ----------------------------------------------------------------------------- fp8 GEMM
 def quant_fp8_rows(x, q=None, scale=None):
     """bf16 [M,K] -> (e4m3fn [M,K], fp32 [M]) with one dynamic scale per row."""
@@ -865,6 +905,8 @@ def gemm_fp8(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False):
     if M == 0:
         return out
     ldr = resid.stride(0) if resid is not None else 0
+    if use_hold(M, N, K, epi, fp8=True):
+        return gemm_hold(x, w8, sw, epi=epi, out=out)
     if M <= DEC_MAX_M and FP8_DEC_STREAM and use_stream(M, N, K, epi, fp8=True):
         rc = _gemm_stream(x, w8, sw, out, bias, resid, ldr, M, N, K, epi, e, out_f32)
     elif M <= DEC_MAX_M:

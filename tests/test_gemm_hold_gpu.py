@@ -1,0 +1,42 @@
+"""Gate/up projections of a few rows with held activations."""
+import pytest
+import torch
+
+from rag_llm_k8s_amd.ops.fp8 import quantize_weight
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _glu(x, w, act):
+    z = (x.double() @ w.double().t()).view(x.shape[0], -1, 2, 64)
+    return act(z[:, :, 0].reshape(x.shape[0], -1), z[:, :, 1].reshape(x.shape[0], -1))
+
+
+@pytest.mark.parametrize("rows", [128, 2816, 8320, 16384])  # one tile group; less than a tile a CU; uneven shares; even ones
+@pytest.mark.parametrize("K", [1024, 2048, 3072, 4096, 5120])
+def test_gemm_hold(native, rows, K):
+    """Row counts around the 16-row fragments and the launch's limit, both weight types, strided activations and output."""
+    g = torch.Generator(device=DEV).manual_seed(rows + K)
+    w = (torch.randn(rows, K, device=DEV, generator=g) * K ** -0.5).bfloat16()
+    w8 = quantize_weight(w)
+    par = torch.tensor([1.0, 1.7, 1.0], device=DEV)
+    X = torch.randn(64, K + 8, device=DEV, generator=g).bfloat16()[:, :K]
+    for M in (1, 15, 16, 17, 33, 64):
+        x, out = X[:M], torch.full((M + 1, rows // 2 + 64), 7.0, device=DEV).bfloat16()
+        cases = [(w8.w8, w8.scale, None, "silu_mul", w8.w8.double() * w8.scale.double()[:, None]),
+                 (w, None, None, "silu_mul", w), (w, None, par, "glu_clip", w)]
+        for wt, sw, p, epi, wd in cases:
+            if native._lib.lib().ragk_gemm_hold_rows(K, int(sw is not None)) == 0:
+                continue
+            native.gemm_hold(x, wt, sw, p, epi, out=out[:M, :rows // 2])
+
+            def act(a, b):
+                if epi == "silu_mul":
+                    return a * torch.sigmoid(a) * b
+                a = a.clamp(max=1.0)
+                return a * torch.sigmoid(1.7 * a) * (b.clamp(-1.0, 1.0) + 1.0)
+            ref = _glu(x, wd, act)
+            # one rounding to the 8 bits of bf16: at most 2^-8 of each value (1.6e-3 in the mean square); fp32 sums are far below
+            assert (out[:M, :rows // 2].double() - ref).norm() / ref.norm() < 2.0 ** -8, (M, epi)
+            assert out[M:].eq(7.0).all() and out[:, rows // 2:].eq(7.0).all()

@@ -86,6 +86,15 @@ def use_stream(M, N, K, epi, fp8=False):
     return M > 16 if fp8 else True
 
 
+def use_vocab(M, N, K, epi):
+    """fp32 logits go to the slab form of the stream GEMM with one slab: its 64-row tiles keep two blocks a CU and no K-split
+    ends in a reduction (32000 x 4096, 4 / 32 rows: stream GEMM 64 / 64 us -> 49 / 48; 32768 x 4096, 11 rows: register-streaming
+    kernel, which reads the activations for every 16 columns, 58.6 -> 48.3, 32 rows: 65.7 -> 49.6). The register-streaming
+    kernel keeps vocabularies from 32768 on below 8 rows (128256 x 4096 at 5 rows: 173 us against 184, at 8: 191 against 182)."""
+    return (epi == "none" and (1 if N < 32768 else 8) <= M <= 64 and N >= STREAM_MIN_ROWS and N % 4 == 0
+            and K % 64 == 0)
+
+
 def use_pp(M, N, K, epi):
     """Large-M GEMMs go to a 256x256 MFMA kernel: gemm_w4.hip (default, 4 waves x 128x128, 9-16 %
     faster on the Llama-8B prefill shapes, profiles/gemm_w4_r1.txt) or the 8-wave ping-pong gemm_pp.hip."""
@@ -222,6 +231,8 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
         return gemm_mid(x, w, bias=bias, resid=resid, epi=epi, out=out, out_f32=out_f32)
     if path is None and use_hold(M, N, K, epi):
         return gemm_hold(x, w, par=bias, epi=epi, out=out)
+    if path is None and use_vocab(M, N, K, epi) and out_f32 and out.stride(0) == N:
+        return gemm_stream_part(x, w, out=out, rows=64, S=1)
     if path is None and STREAM_DEFAULT and use_stream(M, N, K, epi):
         path = 5
     if path is None and DEC_DEFAULT and use_dec(M, N, K, epi):
@@ -409,6 +420,15 @@ def stream_part_cfg(M, N, K):
     # into 8-step slices) stays on gemm_part, whose 64-column blocks split finer
     if best[2] < 0.5 * cus:
         return 0, 0
+    # half the chip, or slices as short as the ring is deep: 64-row tiles at one block a CU instead, with as many slabs or half
+    # of them (12 rows: 2048 x 5632 8.9 -> 7.1 us, 4096 x 4096 9.3 -> 8.3, 4096 x 7168 12.5 -> 12.2; from 16 steps a slice on
+    # the wider tile is ahead: 4096 x 8192 14.3 against 16.4)
+    if best[0] == 128 and (best[2] < cus or steps // best[1] < 16):
+        tiles, S = -(-N // 64), 1
+        while tiles * S * 2 <= cus and steps % (S * 2) == 0 and steps // (S * 2) >= 8 and S * 2 <= STREAM_PART_MAX_S:
+            S *= 2
+        if 0.9 * cus <= tiles * S <= cus:
+            return 64, S
     return best[0], best[1]
 
 

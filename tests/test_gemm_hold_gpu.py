@@ -1,4 +1,4 @@
-"""Gate/up projections of a few rows with held activations."""
+"""Decode projections of a few rows: gate/up with held activations, logits and split-K slabs of the weight ring."""
 import pytest
 import torch
 
@@ -40,3 +40,24 @@ def test_gemm_hold(native, rows, K):
             # one rounding to the 8 bits of bf16: at most 2^-8 of each value (1.6e-3 in the mean square); fp32 sums are far below
             assert (out[:M, :rows // 2].double() - ref).norm() / ref.norm() < 2.0 ** -8, (M, epi)
             assert out[M:].eq(7.0).all() and out[:, rows // 2:].eq(7.0).all()
+
+
+@pytest.mark.parametrize("N,K", [(16384, 1024), (32000, 256), (32772, 2048), (50304, 384)])
+def test_logits_rows(native, N, K):
+    """Vocabularies of a ragged last tile, on both sides of the row count where the kernel changes."""
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    for M in (1, 7, 8, 17, 64):
+        x = torch.randn(M, K, device=DEV).bfloat16()
+        got = native.gemm(x, w, out_f32=True)
+        ref = x.double() @ w.double().t()
+        # fp32 sums of K products of size K^-0.5
+        assert (got.double() - ref).abs().max().item() < K * 2.0 ** -24 * 8
+
+
+@pytest.mark.parametrize("N,K", [(2048, 5632), (4096, 4096), (4096, 7168), (4096, 8192), (6144, 4096)])
+def test_stream_slabs(native, N, K):
+    """The split-K slabs sum to the product whichever tile and split the rule takes."""
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    for M in (5, 17, 64):
+        x = torch.randn(M, K, device=DEV).bfloat16()
+        assert (native.gemm_part(x, w).double().sum(0) - x.double() @ w.double().t()).abs().max().item() < K * 2.0 ** -24 * 8

@@ -308,7 +308,7 @@ def attn_decode(P, bias, spec, table, slots, kc, vc, meta, out, v_first=None, la
 
 # ------------------------------------------------------------------------------------- latent attention
 KEY_PAD = 64  # zero rows behind packed key rows: attention reads whole 64-row groups
-LATENT_TARGET_BLOCKS = 256  # a decode block fills a CU's LDS
+LATENT_TARGET_BLOCKS = 256  # at most: a decode block fills a CU's LDS (20 rows of 13 blocks took 23.1 us, of 12 18.9)
 LATENT_MIN_TOKENS = 128  # of a partition
 LATENT_MAX_PARTS = 64
 
@@ -361,7 +361,7 @@ def latent_split(spec, max_kv_len, batch):
     most = min(-(-tiles // latent_min_tiles(spec)), LATENT_MAX_PARTS)
     wide = spec.rp <= 512 and spec.heads > 16 and batch * -(-spec.heads // 32) * most >= LATENT_TARGET_BLOCKS
     heads = 32 if wide else 16
-    return min(-(-LATENT_TARGET_BLOCKS // (batch * -(-spec.heads // heads))), most), heads
+    return max(1, min(LATENT_TARGET_BLOCKS // (batch * -(-spec.heads // heads)), most)), heads
 
 
 def latent_parts(spec, max_kv_len, batch):

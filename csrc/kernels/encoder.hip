@@ -14,6 +14,9 @@ int ragk_gemm_mid(const void*, int, const void*, int, void*, int, const void*, c
                   int, float*, hipStream_t);
 int ragk_attn_prefill(const void*, int, const void*, const void*, int, const int*, int, const int*, const int*, const int*,
                       const int*, int, void*, int, int, int, int, int, int, float, hipStream_t);
+int ragk_gemm_part(const void*, int, const void*, int, float*, int, int, int, int, hipStream_t);
+int ragk_layernorm_slabs(const float*, int, const void*, const void*, int, const void*, const void*, void*, int, int, int, float,
+                         hipStream_t);
 int ragk_layernorm(const void*, int, const void*, int, const void*, const void*, void*, int, int, int, float, hipStream_t);
 int ragk_embed_ln(const int*, const int*, const void*, const void*, const void*, const void*, const void*, void*, int, int,
                   float, int, hipStream_t);
@@ -102,9 +105,9 @@ __global__ __launch_bounds__(POOL_NT) void pool_l2norm_kernel(const bf16_t* __re
 }
 
 
-// Launches of one product: rows r0 .. r1 on gemm_mid (tile mi, S slabs), gemm_w4 (mi 0) or the skinny kernel (mi -1).
+// Launches of one product: rows r0 .. r1 on gemm_mid (tile mi, S slabs), gemm_w4 (mi 0) or the decode kernels (mi -1).
 struct Piece { int r0, r1, mi, S; };
-struct Plan { int n; Piece p[2]; };
+struct Plan { int n, slabs; Piece p[2]; };  // slabs: p[0].S fp32 slabs of all rows for the norm behind it
 
 // The arguments of one forward (mirrored by ops/_lib.py EncoderCall).
 struct EncoderCall {
@@ -132,6 +135,20 @@ int product(const Plan& plan, const void* x, int K, const void* w, int N, const 
     if (rc) return rc;
   }
   return 0;
+}
+
+// norm(x . w^T + bias + h) into h
+int product_norm(const EncoderCall& c, const Plan& plan, const void* x, int K, const void* w, const void* bias, const void* g,
+                 const void* b, hipStream_t st) {
+  const Piece& p = plan.p[0];
+  if (!plan.slabs) {
+    const int rc = product(plan, x, K, w, c.H, bias, c.h, c.a, EPI_BIAS_RESID, c.ws, st);
+    return rc ? rc : ragk_layernorm(c.a, c.H, nullptr, 0, g, b, c.h, c.H, c.T, c.H, c.eps, st);
+  }
+  const int rc = p.mi < 0 ? ragk_gemm_part(x, K, w, K, c.ws, c.T, c.H, K, K / 64 / p.S, st)
+                          : ragk_gemm_mid(x, K, w, K, c.ws, c.H, nullptr, nullptr, 0, c.T, c.H, K, EPI_NONE, 2, p.mi, p.S,
+                                          nullptr, st);
+  return rc ? rc : ragk_layernorm_slabs(c.ws, p.S, bias, c.h, c.H, g, b, c.h, c.H, c.T, c.H, c.eps, st);
 }
 
 }  // namespace
@@ -167,11 +184,9 @@ RAGK_API int ragk_encoder_forward(const EncoderCall* cp, hipStream_t st) {
     const char* q = (const char*)c.qkv;
     RAGK_TRY(ragk_attn_prefill(q, 3 * H, q + 2 * H, q + 4 * H, 3 * H, nullptr, 0, c.cu, c.cu, c.lens, c.tiles, c.n_tiles, c.attn,
                                H, c.heads, c.heads, D, 0, 0, scale, st));
-    RAGK_TRY(product(c.plans[1], c.attn, H, w[2], H, w[3], c.h, c.a, EPI_BIAS_RESID, c.ws, st));
-    RAGK_TRY(ragk_layernorm(c.a, H, nullptr, 0, w[4], w[5], c.h, H, T, H, c.eps, st));
+    RAGK_TRY(product_norm(c, c.plans[1], c.attn, H, w[2], w[3], w[4], w[5], st));
     RAGK_TRY(product(c.plans[2], c.h, H, w[6], c.I, w[7], nullptr, c.f, EPI_BIAS_GELU, c.ws, st));
-    RAGK_TRY(product(c.plans[3], c.f, c.I, w[8], H, w[9], c.h, c.a, EPI_BIAS_RESID, c.ws, st));
-    RAGK_TRY(ragk_layernorm(c.a, H, nullptr, 0, w[10], w[11], c.h, H, T, H, c.eps, st));
+    RAGK_TRY(product_norm(c, c.plans[3], c.f, c.I, w[8], w[9], w[10], w[11], st));
   }
   RAGK_TRY(ragk_pool_l2norm_rows(c.h, H, c.cu, c.rows, c.out, c.ldo, c.B, H, c.pooling, c.normalize, st));
 #undef RAGK_TRY

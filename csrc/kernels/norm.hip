@@ -145,6 +145,48 @@ __global__ __launch_bounds__(NT) void layernorm_kernel(const bf16_t* x, int ldx,
   ln_row<NV, W>(v, nvec, lane, g, b, out + (size_t)row * ldo, H, eps);
 }
 
+// y = LN(sum_s P[s] + bias + resid) * g + b from the fp32 split-K slabs P[s][rows][H] of the product that precedes the norm
+// (slab S_stride floats apart), 4 / W rows a block: the sum that a reduction launch and its bf16 result would have carried.
+template <int NV, int W>
+__global__ __launch_bounds__(NT) void layernorm_slabs_kernel(const float* __restrict__ P, int S, size_t slab,
+                                                             const bf16_t* __restrict__ bias, const bf16_t* resid, int ldr,
+                                                             const bf16_t* __restrict__ g, const bf16_t* __restrict__ b,
+                                                             bf16_t* out, int ldo, int rows, int H, float eps) {
+  const int lane = threadIdx.x & (64 * W - 1), row = blockIdx.x * (NT / 64 / W) + threadIdx.x / (64 * W);
+  if (row >= rows) return;
+  const int nvec = H >> 3;
+  float v[NV][8];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int vi = min(lane + 64 * W * i, nvec - 1);
+    float r8[8], b8[8];
+    unpack8(*reinterpret_cast<const u32x4*>(resid + (size_t)row * ldr + vi * 8), r8);
+    unpack8(*reinterpret_cast<const u32x4*>(bias + vi * 8), b8);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[i][e] = 0.f;
+    const float* p = P + (size_t)row * H + vi * 8;
+    int s = 0;
+    for (; s + 4 <= S; s += 4) {  // four slabs' loads in flight
+      f32x4 t[4][2];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        t[u][0] = *reinterpret_cast<const f32x4*>(p + (s + u) * slab);
+        t[u][1] = *reinterpret_cast<const f32x4*>(p + (s + u) * slab + 4);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[i][e] += t[u][e >> 2][e & 3];
+    }
+    for (; s < S; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[i][e] += p[s * slab + e];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[i][e] += b8[e] + r8[e];
+  }
+  ln_row<NV, W>(v, nvec, lane, g, b, out + (size_t)row * ldo, H, eps);
+}
+
 // token embedding gather: out[t] = table[ids[t]]
 // carry (optional, asynchronous decode): carry[t] >= 0 takes the token id from prev[carry[t]] (the
 // previous decode step's sampled tokens, still on the device) instead of ids[t]; the resolved id is
@@ -434,6 +476,19 @@ RAGK_API int ragk_layernorm(const void* x, int ldx, const void* resid, int ldr, 
     hipLaunchKernelGGL((layernorm_kernel<decltype(nv)::value, decltype(w)::value>), dim3((rows + R - 1) / R), dim3(NT), 0, st,
                        (const bf16_t*)x, ldx, (const bf16_t*)resid, ldr, (const bf16_t*)g, (const bf16_t*)b, (bf16_t*)out, ldo,
                        rows, H, eps);
+  });
+}
+
+// P: S slabs of rows x H floats, one after the other; bias [H]; resid bf16 rows.
+RAGK_API int ragk_layernorm_slabs(const float* P, int S, const void* bias, const void* resid, int ldr, const void* g,
+                                  const void* b, void* out, int ldo, int rows, int H, float eps, hipStream_t st) {
+  if (rows <= 0) return 0;
+  if (H % 8 || H > 8 * NT * 4 || S < 1) return (int)hipErrorInvalidValue;
+  return (int)by_row(H, [&](auto nv, auto w) {
+    constexpr int R = NT / 64 / decltype(w)::value;
+    hipLaunchKernelGGL((layernorm_slabs_kernel<decltype(nv)::value, decltype(w)::value>), dim3((rows + R - 1) / R), dim3(NT), 0,
+                       st, P, S, (size_t)rows * H, (const bf16_t*)bias, (const bf16_t*)resid, ldr, (const bf16_t*)g,
+                       (const bf16_t*)b, (bf16_t*)out, ldo, rows, H, eps);
   });
 }
 

@@ -204,9 +204,7 @@ class EncoderModel:
         for L in w.layers:
             qkv = be.gemm(h, L["wqkv"], bias=L["bqkv"], epi="bias")
             be.attn_encoder(qkv, cu, lens, tiles, attn, nh, D)
-            a = be.gemm(attn, L["wo"], bias=L["bo"], resid=h, epi="bias_resid")
-            h = be.layernorm(a, L["ln1_g"], L["ln1_b"], c.layer_norm_eps)
+            h = be.gemm_layernorm(attn, L["wo"], L["bo"], h, L["ln1_g"], L["ln1_b"], c.layer_norm_eps)
             f = be.gemm(h, L["wi"], bias=L["bi"], epi="bias_gelu")
-            a = be.gemm(f, L["wo2"], bias=L["bo2"], resid=h, epi="bias_resid")
-            h = be.layernorm(a, L["ln2_g"], L["ln2_b"], c.layer_norm_eps)
+            h = be.gemm_layernorm(f, L["wo2"], L["bo2"], h, L["ln2_g"], L["ln2_b"], c.layer_norm_eps)
         return be.pool_l2norm(h, cu, mode=c.pooling, normalize=c.normalize)

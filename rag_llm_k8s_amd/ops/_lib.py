@@ -22,6 +22,7 @@ P, I, F, S, U64 = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_void_p
 _SIGS = {
     "ragk_gemm": [P, I, P, I, P, I, P, P, I, I, I, I, I, I, S],
     "ragk_gemm_path": [I, P, I, P, I, P, I, P, P, I, I, I, I, I, S],
+    "ragk_layernorm_slabs": [P, I, P, P, I, P, P, P, I, I, I, F, S],
     "ragk_gemm_hold": [P, I, P, I, P, P, I, P, I, I, I, I, I, S],
     "ragk_gemm_hold_rows": [I, I],
     "ragk_gemm_mid": [P, I, P, I, P, I, P, P, I, I, I, I, I, I, I, I, P, S],
@@ -244,7 +245,7 @@ class GemmPiece(ctypes.Structure):
 
 
 class GemmPlan(ctypes.Structure):
-    _fields_ = [("n", I), ("p", GemmPiece * 2)]
+    _fields_ = [("n", I), ("slabs", I), ("p", GemmPiece * 2)]
 
 
 class EncoderCall(ctypes.Structure):

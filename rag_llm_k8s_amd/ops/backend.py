@@ -75,6 +75,10 @@ class TorchBackend:
             return out
         return y
 
+    def gemm_layernorm(self, x, w, bias, resid, g, b, eps):
+        """LN(x @ w^T + bias + resid) * g + b: the output projections of an encoder layer."""
+        return self.layernorm(self.gemm(x, w, bias=bias, resid=resid, epi="bias_resid"), g, b, eps)
+
     def embed(self, ids, table, out=None, carry=None, prev=None):
         if carry is not None:
             c = carry[:ids.numel()].long()
@@ -345,6 +349,9 @@ class NativeBackend(TorchBackend):
 
     def layernorm(self, x, g, b, eps, out=None, resid=None):
         return self.n.layernorm(x, g, b, eps, out=out, resid=resid)
+
+    def gemm_layernorm(self, x, w, bias, resid, g, b, eps):
+        return self.n.gemm_layernorm(x, w, bias, resid, g, b, eps)
 
     def embed(self, ids, table, out=None, carry=None, prev=None):
         return self.n.embed(ids, table, out=out, carry=carry, prev=prev)

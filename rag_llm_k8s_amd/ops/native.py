@@ -1088,8 +1088,9 @@ def encoder_forward(cfg, w, ids, lens, first_pos, out, rows):
     L, cus, c = _lib.lib(), _cu_count(), _lib.EncoderCall()
     slab = 0
     for i, (N, K) in enumerate(((3 * H, H), (H, H), (I, H), (H, I))):
-        plan = ((0, T, -1, 1),) if T <= 64 else gemm_plan(T, N, K, True, cus)
-        c.plans[i].n = len(plan)
+        S, mi = ln_slabs(T, N, K) if i in (1, 3) else (1, 0)
+        plan = ((0, T, mi, S),) if S > 1 else ((0, T, -1, 1),) if T <= 64 else gemm_plan(T, N, K, True, cus)
+        c.plans[i].n, c.plans[i].slabs = len(plan), int(S > 1)
         for j, (r0, r1, mi, S) in enumerate(plan):
             c.plans[i].p[j] = _lib.GemmPiece(r0, r1, mi, S)
             slab = max(slab, S * (r1 - r0) * N if S > 1 else 0)
@@ -1109,6 +1110,51 @@ def encoder_forward(cfg, w, ids, lens, first_pos, out, rows):
     c.pooling, c.normalize, c.eps = {"cls": 0, "mean": 1, "last": 2}[cfg.pooling], int(cfg.normalize), float(cfg.layer_norm_eps)
     check(L.ragk_encoder_forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
     return out
+
+
+def layernorm_slabs(P, bias, resid, g, b, eps, out=None):
+    """LN(P.sum(0) + bias + resid) * g + b of a product's fp32 split-K slabs P [S, T, H]."""
+    S, T, H = P.shape
+    _req(P.dtype == torch.float32 and P.is_cuda and P.is_contiguous(), "slabs fp32")
+    _req(H % 8 == 0 and H <= 8192 and resid.shape == (T, H) and bias.numel() == H, "H")
+    _bf16_2d(resid, "resid")
+    out = torch.empty((T, H), dtype=torch.bfloat16, device=P.device) if out is None else out
+    check(_lib.lib().ragk_layernorm_slabs(P.data_ptr(), S, bias.data_ptr(), resid.data_ptr(), resid.stride(0), g.data_ptr(),
+                                          b.data_ptr(), out.data_ptr(), out.stride(0), T, H, float(eps), stream_ptr()),
+          "ragk_layernorm_slabs")
+    return out
+
+
+def ln_slabs(M, N, K):
+    """(slabs, tile) of a product whose bias, residual and LayerNorm follow as one launch over its split-K slabs (tile -1:
+    gemm_part, else gemm_mid's), (1, 0): the product with its epilogue and a plain LayerNorm. Pairs of launches, us: 1024 x
+    4096 at 30 / 64 rows 15.6 / 23.3 -> 9.5 / 10.8, 384 x 1536 at 16 / 64 7.0 / 11.5 -> 6.5 / 7.6, 1024 x 1024 at 64 9.9 -> 8.3;
+    past 64 rows, where the split ended in a reduction or did not pay for one, 384 x 1536 at 100 rows 11.9 -> 10.2, 1024 x
+    1024 at 200 13.5 -> 11.6, 1024 x 4096 at 400 19.0 -> 17.1. Under 18432 = 12 x 1536 inputs, or a K that gives fewer than
+    four slabs of four K-steps, the register-streaming kernel's epilogue is ahead (1024 x 1024 at 12 rows 6.6 against 7.1)."""
+    if K % 64 or N % 8:
+        return 1, 0
+    if M <= 64:
+        ks = 4 if K <= 3072 else 8  # K-steps of a slab: at most twelve slabs of the shorter ones
+        return (K // (64 * ks), -1) if K >= 1024 and K % (64 * ks) == 0 and M * K >= 18432 else (1, 0)
+    S, mi = _slab_best(M, N, K, _cu_count())
+    return (S, mi) if S > 1 and mi else (1, 0)
+
+
+def gemm_layernorm(x, w, bias, resid, g, b, eps):
+    """LN(x @ w^T + bias + resid) * g + b, the sum kept in fp32 where the product is split (ln_slabs)."""
+    M, K = x.shape
+    N = w.shape[0]
+    S, mi = ln_slabs(M, N, K)
+    if S == 1:
+        return layernorm(gemm(x, w, bias=bias, resid=resid, epi="bias_resid"), g, b, eps)
+    if mi < 0:
+        return layernorm_slabs(gemm_part(x, w, out=torch.empty((S, M, N), dtype=torch.float32, device=x.device), ks=K // 64 // S),
+                               bias, resid, g, b, eps)
+    P = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
+    check(_lib.lib().ragk_gemm_mid(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), P.data_ptr(), N, None, None, 0, M, N, K,
+                                   EPI["none"], 2, mi, S, None, stream_ptr()), "ragk_gemm_mid")
+    return layernorm_slabs(P, bias, resid, g, b, eps)
 
 
 def silu_mul(x, out=None):

@@ -29,3 +29,28 @@ def test_pool_rows(native, H):
         for mode in ("cls", "mean", "last"):
             ref = R.pool_l2norm(x.float().cpu(), cu.cpu(), mode=mode)
             assert (native.pool_l2norm(x, cu, mode=mode).cpu() - ref).abs().max().item() < 1e-5
+
+
+@pytest.mark.parametrize("S", [1, 3, 4, 9])
+@pytest.mark.parametrize("T,H", [(1, 384), (5, 520), (3, 1032), (2, 2056), (5, 8192)])
+def test_layernorm_slabs(native, T, H, S):
+    """Slab counts around the four that are loaded together, widths as above; the residual's rows are overwritten in place."""
+    torch.manual_seed(H + S)
+    P, r = torch.randn(S, T, H, device=DEV), torch.randn(T, H, device=DEV).bfloat16()
+    bias, g, b = (torch.randn(H, device=DEV).bfloat16() for _ in range(3))
+    ref = R.layernorm(P.double().sum(0) + bias.double() + r.double(), g.double(), b.double(), 1e-12)
+    # one rounding to bf16 a value: at most 2^-8 of it
+    assert (native.layernorm_slabs(P, bias, r, g, b, 1e-12, out=r).double() - ref).norm() / ref.norm() < 2.0 ** -8
+
+
+@pytest.mark.parametrize("N,K", [(384, 384), (384, 1536), (1024, 1024), (1024, 4096), (256, 512)])
+def test_gemm_layernorm(native, N, K):
+    """Both forms of the pair, on either side of every line between them."""
+    torch.manual_seed(N + K)
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).bfloat16()
+    bias, g, b = (torch.randn(N, device=DEV).bfloat16() for _ in range(3))
+    for M in (1, 11, 12, 17, 18, 64, 65, 200, 1100):
+        x, r = torch.randn(M, K, device=DEV).bfloat16(), torch.randn(M, N, device=DEV).bfloat16()
+        ref = R.layernorm(x.double() @ w.double().t() + bias.double() + r.double(), g.double(), b.double(), 1e-12)
+        # roundings to bf16, at most 2^-8 of a value each: the result and, unsplit, the sum that is normalised
+        assert (native.gemm_layernorm(x, w, bias, r, g, b, 1e-12).double() - ref).norm() / ref.norm() < 2.0 ** -7

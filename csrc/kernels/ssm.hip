@@ -310,36 +310,33 @@ __global__ __launch_bounds__(256, NP <= 128 ? 2 : 1) void scan_chunk_kernel(Chun
   constexpr int BV = CQ * NP / 8 / 256, XV = (CQ * PS / 8 + 255) / 256;
   u32x4 rb[BV], rx[XV];
   bf16x8 cf[CB::KS];
-  float rdt = 0.f;
+  unsigned short rdt = 0;
   const u32x4 zero4 = (u32x4){0u, 0u, 0u, 0u};
-  auto fetch = [&](int c0) {  // chunk rows into registers (zeros past the sequence or past N / P)
+  // Chunk rows into registers, as they are: rows past the sequence and columns past N / P come from the last ones and are
+  // zeroed where they are used, so that neither a branch nor a conversion waits for a load here (the step delta converted at
+  // its load held up every chunk for the whole fetch).
+  auto fetch = [&](int c0) {
 #pragma unroll
     for (int i = 0; i < BV; ++i) {
       const int v = tid + 256 * i, t = v / (NP / 8), c = (v % (NP / 8)) * 8;
-      rb[i] = (c0 + t < n && c < a.N)
-                  ? *reinterpret_cast<const u32x4*>(a.xbc + (size_t)(t0 + c0 + t) * a.ch + offB + c) : zero4;
+      rb[i] = *reinterpret_cast<const u32x4*>(a.xbc + (size_t)(t0 + min(c0 + t, n - 1)) * a.ch + offB + min(c, a.N - 8));
     }
 #pragma unroll
     for (int i = 0; i < XV; ++i) {
       const int v = tid + 256 * i, t = v / (PS / 8), c = (v % (PS / 8)) * 8;
-      rx[i] = (t < CQ && c0 + t < n && p0 + c < a.P)
-                  ? *reinterpret_cast<const u32x4*>(a.xbc + (size_t)(t0 + c0 + t) * a.ch + h * a.P + p0 + c) : zero4;
+      rx[i] = *reinterpret_cast<const u32x4*>(a.xbc + (size_t)(t0 + min(c0 + t, n - 1)) * a.ch + h * a.P + min(p0 + c, a.P - 8));
     }
-    const int tq = c0 + 16 * wid + fr;
+    const int tq = min(c0 + 16 * wid + fr, n - 1);
 #pragma unroll
-    for (int s = 0; s < CB::KS; ++s) {
-      const int c = 32 * s + 8 * fh;
-      cf[s] = (tq < n && c < a.N)
-                  ? *reinterpret_cast<const bf16x8*>(a.xbc + (size_t)(t0 + tq) * a.ch + offC + c)
-                  : (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
-    }
-    rdt = c0 + lane < n ? bf2f(a.row[(size_t)(t0 + c0 + lane) * a.ld + a.off_dt + h]) : 0.f;
+    for (int s = 0; s < CB::KS; ++s)
+      cf[s] = *reinterpret_cast<const bf16x8*>(a.xbc + (size_t)(t0 + tq) * a.ch + offC + min(32 * s + 8 * fh, a.N - 8));
+    rdt = a.row[(size_t)(t0 + min(c0 + lane, n - 1)) * a.ld + a.off_dt + h];
   };
   fetch(0);
 
   for (int c0 = 0; c0 < n; c0 += CQ) {
     // every wave forms the chunk's running log-decay (lane = token) and keeps what it needs of it
-    const float dt = c0 + lane < n ? softplusf(rdt + dbias) : 0.f;
+    const float dt = c0 + lane < n ? softplusf(bf2f(rdt) + dbias) : 0.f;
     const float cum = wave_scan(-decay_rate * dt);
     const float c_end = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cum), 63));
     const float wgt = __builtin_amdgcn_exp2f(c_end - cum) * dt;  // what this lane's token leaves in the state
@@ -350,11 +347,11 @@ __global__ __launch_bounds__(256, NP <= 128 ? 2 : 1) void scan_chunk_kernel(Chun
 #pragma unroll
     for (int i = 0; i < BV; ++i) {
       const int v = tid + 256 * i, t = v / (NP / 8), c = v % (NP / 8);
-      *reinterpret_cast<u32x4*>(sB + t * CB::ROWB + 16 * (c ^ kswz<NP>(t))) = rb[i];
+      *reinterpret_cast<u32x4*>(sB + t * CB::ROWB + 16 * (c ^ kswz<NP>(t))) = c0 + t < n && 8 * c < a.N ? rb[i] : zero4;
     }
     bf16x8 cq[CB::KS];
 #pragma unroll
-    for (int s = 0; s < CB::KS; ++s) cq[s] = cf[s];
+    for (int s = 0; s < CB::KS; ++s) cq[s] = 32 * s + 8 * fh < a.N ? cf[s] : (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < XV; ++i) {
       const int v = tid + 256 * i, t = v / (PS / 8), c = v % (PS / 8);
@@ -362,12 +359,13 @@ __global__ __launch_bounds__(256, NP <= 128 ? 2 : 1) void scan_chunk_kernel(Chun
       if (t < CQ) {
         const int off = t * CX::ROWB + 16 * (c ^ vswz<PS>(t));
         float f[8];
-        unpack8(rx[i], f);
+        const u32x4 xr = c0 + t < n && p0 + 8 * c < a.P ? rx[i] : zero4;
+        unpack8(xr, f);
 #pragma unroll
         for (int e = 0; e < 8; ++e) f[e] *= wt;
         u32x4 hi, lo;
         split8(f, hi, lo);
-        *reinterpret_cast<u32x4*>(sX + off) = rx[i];
+        *reinterpret_cast<u32x4*>(sX + off) = xr;
         *reinterpret_cast<u32x4*>(sXh + off) = hi;
         *reinterpret_cast<u32x4*>(sXl + off) = lo;
       }
@@ -737,8 +735,9 @@ RAGK_API int ragk_ssm_scan_chunk(const int* cu_q, const int* kv_lens, const int*
     return (int)hipErrorInvalidValue;
   const ChunkArgs a{{cu_q, kv_lens, states, T, S}, (const bf16_t*)xbc, ch, (const bf16_t*)row, ld, off_dt, dt_bias, A, D,
                     ssm_state, (bf16_t*)y, H, P, N, G};
-  // narrow column slices when one block per (head, sequence) would leave CUs idle
-  const bool narrow = P <= 32 || (g_scan_cols ? g_scan_cols == 32 : (long long)H * S * ((P + 63) / 64) <= 256);
+  // narrow column slices while three of their blocks a CU are resident together: 320 (head, sequence) pairs of 1900 tokens
+  // 154 us against 171, 64 of 4000 199 against 279
+  const bool narrow = P <= 32 || (g_scan_cols ? g_scan_cols == 32 : (long long)H * S * ((P + 63) / 64) <= 384);
 #define RAGK_SC(NPV) return narrow ? launch_scan_chunk<NPV, 32>(a, st) : launch_scan_chunk<NPV, 64>(a, st)
   if (N <= 32) RAGK_SC(32);
   if (N <= 64) RAGK_SC(64);

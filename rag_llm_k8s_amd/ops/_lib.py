@@ -257,7 +257,11 @@ class EncoderCall(ctypes.Structure):
 
 
 def stream_ptr(device=None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle. Asked for at every launch, so without the Stream object that torch.cuda.current_stream
+    makes (2.7 us against 0.3)."""
+    if device is not None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def check(rc: int, what: str):

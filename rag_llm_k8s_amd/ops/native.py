@@ -546,6 +546,13 @@ def slab_count(M, N, K):
     return _slab_best(M, N, K, _cu_count())[0]
 
 
+@functools.lru_cache(maxsize=4096)
+def _splitk_tile(M, N, K, nsplit, cus):
+    """(gemm_mid's tile, whether gemm_w4 is ahead of it) for nsplit slabs."""
+    t, mi = min((_tiles_us(M, N, K, m, nsplit, cus), m) for m in MID_US)
+    return mi, _tiles_us(M, N, K, 0, nsplit, cus) < t
+
+
 def gemm_splitk(x, w, nsplit, out=None):
     """fp32 split-K slabs P[nsplit, M, N] with P.sum(0) = x @ w^T in one launch, consumed by add_partials_rmsnorm (residual
     add + norm). gemm_mid or gemm_w4's KSPLIT form, whichever the launch model puts first."""
@@ -559,10 +566,8 @@ def gemm_splitk(x, w, nsplit, out=None):
     _req(out.dtype == torch.float32 and out.is_contiguous() and out.numel() >= nsplit * M * N, "gemm_splitk out")
     if M == 0:
         return out
-    cus = _cu_count()
-    t, mi = min((_tiles_us(M, N, K, m, nsplit, cus), m) for m in MID_US)
-    fits = x.stride(0) * M * 2 < 2 ** 31 and w.stride(0) * N * 2 < 2 ** 31
-    if fits and _tiles_us(M, N, K, 0, nsplit, cus) < t:
+    mi, w4 = _splitk_tile(M, N, K, nsplit, _cu_count())
+    if w4 and x.stride(0) * M * 2 < 2 ** 31 and w.stride(0) * N * 2 < 2 ** 31:
         check(_lib.lib().ragk_gemm_w4_splitk(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), M, N, K,
                                              nsplit, stream_ptr()), "ragk_gemm_w4_splitk")
     else:

@@ -1,8 +1,8 @@
 """Sublayers of residual-stream decoders: shaped attention, latent attention, Mamba-2 state space, gated MLPs.
 
 Each mixer owns its device weights and its cache (paged K/V, or per-slot state) and maps normed rows to
-either the sublayer's output rows (prefill) or fp32 split-K slabs of them (decode), which the following
-residual_norm kernel sums. A model composes them; nothing here knows a model's name.
+either the sublayer's output rows (prefill) or fp32 split-K slabs of them (decode, and prompts of few rows), which the
+following residual_norm kernel sums. A model composes them; nothing here knows a model's name.
 
 Activations are in the weights' type (bf16 when serving, fp32 for exact replay); the residual stream,
 norms, scores, decays and states are fp32 in both.
@@ -102,7 +102,7 @@ class AttentionMixer:
             row = be.gemm(xn, self.wqkv, bias=self.bqkv, epi="bias")
             own = be.shaped_kv_store(row, s, inp.slots, self.kc, self.vc, v_first, lam)
             be.shaped_attn_prefill(row, s, self.table, self.kc, self.vc, meta, out)
-            y = be.gemm(out, self.wo)
+            y = be.out_rows(out, self.wo)
         if self.v_source:
             shared["v_first"] = own
         return y
@@ -146,7 +146,8 @@ class LatentAttentionMixer:
             self.pages = torch.zeros(num_blocks, 64, self.spec.rp, dtype=dtype, device=device)
 
     def forward(self, be, x, inp, shared):
-        """`shared`: latent rows that layers of one forward hand on, by source layer."""
+        """`shared`: latent rows that layers of one forward hand on, by source layer, and "slabs", whether its output
+        projections come as fp32 slabs."""
         s = self.spec
         pages = self.pages if self.source is None else self.source.pages
         exact = s.out_row == s.heads * s.dvp
@@ -155,7 +156,7 @@ class LatentAttentionMixer:
             be.latent_decode(be.proj_rows(x, self.win)[0], s, self.lw, self.eps, inp, pages, out)
             return be.proj_rows(out, self.wo)[0]
         be.latent_prefill(be.gemm(x, self.win), s, self.lw, self.eps, inp, pages, shared, out)
-        return be.gemm(out, self.wo)
+        return be.out_rows(out, self.wo, shared.get("slabs"))
 
 
 class Mamba2Mixer:
@@ -197,7 +198,7 @@ class Mamba2Mixer:
             return be.proj_rows(out, self.wo)[0]
         row = be.gemm(xn, self.win)
         be.ssm_prefill(row, s, self.w, self.eps, meta, self.conv_state, self.ssm_state, out)
-        return be.gemm(out, self.wo)
+        return be.out_rows(out, self.wo)
 
 
 class GluMlp:
@@ -214,9 +215,9 @@ class GluMlp:
             par = dev(torch.tensor([math.inf, 1.0, 0.0, 0.0]), torch.float32)
         return cls(wgu, dev(pad2(get("down"), wp, fp)), par)
 
-    def forward(self, be, xn, inp):
+    def forward(self, be, xn, inp, slabs=None):
         a = be.gemm_glu(xn, self.wgu, self.par)
-        return be.proj_rows(a, self.wdown)[0] if inp.meta.kind == "decode" else be.gemm(a, self.wdown)
+        return be.proj_rows(a, self.wdown)[0] if inp.meta.kind == "decode" else be.out_rows(a, self.wdown, slabs)
 
 
 class ClippedGluMlp(GluMlp):

@@ -205,8 +205,8 @@ class RolesunModel(DecoderModel):
         return (1, 1) + latent_workspace([m.spec for m in self.mixers], max_kv_len, batch, self.device)
 
     # ---- one step
-    def _gate(self, x, w, inp):
-        return self.be.proj_rows(x, w)[0] if inp.meta.kind == "decode" else self.be.gemm(x, w)
+    def _gate(self, x, w, inp, slabs):
+        return self.be.proj_rows(x, w)[0] if inp.meta.kind == "decode" else self.be.out_rows(x, w, slabs)
 
     def _advance(self, h, y, z, zb, norm, nxt, inp):
         """Close a layer; (rows, shifted rows) for layer `nxt`, or None behind the last one."""
@@ -228,15 +228,16 @@ class RolesunModel(DecoderModel):
         h = be.embed_residual(inp.ids, w.embed, carry=inp.carry, prev=inp.carry_src, scale=c.embed_scale,
                               pos=inp.positions, turns=w.turns, n=n)
         x, xs = self._shift(h, 0, inp)
-        shared = {}
+        slabs = be.splits(h.shape[0], w.layers[0]["rg1"])  # of the gates, so of what they gate too
+        shared = {"slabs": slabs}
         for li, L in enumerate(w.layers):
-            z = self._gate(x, L["rg1"], inp)
+            z = self._gate(x, L["rg1"], inp, slabs)
             y = L["mixer"].forward(be, xs, inp, shared)
             zb, norm = L["rg1b"], L["norm1"]
             if L["mlp"] is not None:
                 x, _ = be.gated_residual(h, y, z, zb, norm, eps, n, dt, keep=True)
-                z = self._gate(x, L["rg2"], inp)
-                y = L["mlp"].forward(be, x, inp)
+                z = self._gate(x, L["rg2"], inp, slabs)
+                y = L["mlp"].forward(be, x, inp, slabs)
                 zb, norm = L["rg2b"], L["norm2"]
             nxt = li + 1 if li + 1 < len(w.layers) else None
             x, xs = self._advance(h, y, z, zb, norm, nxt, inp) or (None, None)

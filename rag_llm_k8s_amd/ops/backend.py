@@ -252,6 +252,14 @@ class TorchBackend:
         """Decode projection rows for a consumer that sums them: fp32 slabs [S, M, N] + the bias still to add."""
         return self.gemm(x, w, out_f32=True).unsqueeze(0), bias
 
+    def splits(self, M, w):
+        """Whether out_rows of M rows would come as slabs."""
+        return False
+
+    def out_rows(self, x, w, slabs=None):
+        """A prompt's projection rows for a residual norm, which takes rows or fp32 slabs [S, M, N] (slabs: None, either)."""
+        return self.gemm(x, w)
+
     def gemm_glu(self, x, w, par):
         """Packed gate/up projection with the clipped GLU (par = [limit, alpha, shift]; None, in bf16: silu(g) * u)."""
         if par is None:
@@ -470,6 +478,26 @@ class NativeBackend(TorchBackend):
         if self.part_ok(x.shape[0], w):
             return self.n.gemm_part(x, w), bias
         return self.n.gemm(x, w, out_f32=True).unsqueeze(0), bias
+
+    def splits(self, M, w):
+        # Up to 64 rows from 2^24 weights on: the register-streaming product with its epilogue reads them on too few blocks
+        # (50 rows of niduvik / rolesun, 4096 wide: 985 / 1102 -> 775 / 826 us). Below, the launches' host time bounds the step
+        # and the slabs' is longer (2048 wide, 30 / 40 rows: 543 / 655 us against 569 / 719).
+        if w.dtype != torch.bfloat16:
+            return False
+        if M <= 64:
+            return w.numel() >= 1 << 24 and self.part_ok(M, w)
+        return self.n.slab_count(M, w.shape[0], w.shape[1]) > 1
+
+    def out_rows(self, x, w, slabs=None):
+        # the slabs' sum is part of the norm's pass, so a split needs no reduction launch (4 us) and pays at fewer rows
+        M = x.shape[0]
+        if w.dtype != torch.bfloat16 or not (self.splits(M, w) if slabs is None else slabs):
+            return self.gemm(x, w)
+        if M <= 64:
+            return self.proj_rows(x, w)[0]
+        S = self.n.slab_count(M, w.shape[0], w.shape[1])
+        return self.n.gemm_splitk(x, w, S) if S > 1 else self.n.gemm(x, w, out_f32=True).unsqueeze(0)
 
     def gemm_glu(self, x, w, par):
         if w.dtype == torch.float32:

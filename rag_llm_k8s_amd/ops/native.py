@@ -356,12 +356,17 @@ PART_MIN_BLOCKS = 512
 _part_cfg = [False]
 
 
-def gemm_part_slabs(M, N, K, ks=None):
-    """(ks_steps, S) of the split-K partial GEMM for this shape (0, 0 if unsupported)."""
+@functools.lru_cache(maxsize=4096)
+def _part_ksteps(M, N, K):
     if not _part_cfg[0]:
         check(_lib.lib().ragk_gemm_part_set_min_blocks(PART_MIN_BLOCKS), "ragk_gemm_part_set_min_blocks")
         _part_cfg[0] = True
-    ks = ks or _lib.lib().ragk_gemm_part_ksteps(M, N, K)
+    return _lib.lib().ragk_gemm_part_ksteps(M, N, K)
+
+
+def gemm_part_slabs(M, N, K, ks=None):
+    """(ks_steps, S) of the split-K partial GEMM for this shape (0, 0 if unsupported)."""
+    ks = ks or _part_ksteps(M, N, K)
     if ks <= 0 or K % (64 * ks):
         return 0, 0
     return ks, K // (64 * ks)
@@ -400,18 +405,23 @@ STREAM_PART_MAX_S = 64  # slabs the consumer sums
 
 
 def stream_part_cfg(M, N, K):
+    """(rows, S) of the slab-mode stream GEMM."""
+    return _stream_part_cfg(N, K, _cu_count(), STREAM_PART_ROWS, STREAM_PART_MAX_S)
+
+
+@functools.lru_cache(maxsize=1024)
+def _stream_part_cfg(N, K, cus, only, max_s):
     """(rows, S) of the slab-mode stream GEMM: the most blocks that are co-resident (128-row tiles one
     block per CU, 64-row tiles two), at least 8 K-steps of 64 per block; (0, 0) if nothing fits."""
-    cus = _cu_count()
     steps = K // 64
     best = (0, 0, 0)
     for rows, per_cu in ((128, 1), (64, 2)):
-        if STREAM_PART_ROWS and rows != STREAM_PART_ROWS:
+        if only and rows != only:
             continue
         tiles = -(-N // rows)
         S = 1
         while (tiles * S * 2 <= per_cu * cus and steps % (S * 2) == 0 and steps // (S * 2) >= 8
-               and S * 2 <= STREAM_PART_MAX_S):
+               and S * 2 <= max_s):
             S *= 2
         blocks = tiles * S
         if blocks <= per_cu * cus and (blocks / per_cu, rows) > (best[2], best[0]):
@@ -425,7 +435,7 @@ def stream_part_cfg(M, N, K):
     # the wider tile is ahead: 4096 x 8192 14.3 against 16.4)
     if best[0] == 128 and (best[2] < cus or steps // best[1] < 16):
         tiles, S = -(-N // 64), 1
-        while tiles * S * 2 <= cus and steps % (S * 2) == 0 and steps // (S * 2) >= 8 and S * 2 <= STREAM_PART_MAX_S:
+        while tiles * S * 2 <= cus and steps % (S * 2) == 0 and steps // (S * 2) >= 8 and S * 2 <= max_s:
             S *= 2
         if 0.9 * cus <= tiles * S <= cus:
             return 64, S
@@ -847,6 +857,11 @@ def _gemm_stream(x, w, wscale, out, bias, resid, ldr, M, N, K, epi, e, out_f32):
                               cnt.data_ptr(), stream_ptr())
 
 
+@functools.lru_cache(maxsize=256)
+def _hold_rows(K, fp8):
+    return _lib.lib().ragk_gemm_hold_rows(K, int(fp8))
+
+
 def use_hold(M, N, K, epi, fp8=False):
     """Packed gate/up projections whose activations fit a block's registers go to gemm_hold.hip: 11264 x 2048 bf16 at 12 / 50
     rows 14.7 / 24 -> 11.8 / 17 us against the register-streaming kernel, 28672 x 4096 fp8 at 11 / 32 rows 38 / 37 -> 27.5 / 33
@@ -857,7 +872,7 @@ def use_hold(M, N, K, epi, fp8=False):
     depth (14336 x 4096 at 48 rows 51 -> 38, but 7168 x 4096 25 against 28)."""
     if not 0 < M <= 64 or K < 2048 or epi not in PAIR_EPI or (fp8 and epi != "silu_mul"):
         return False
-    per = _lib.lib().ragk_gemm_hold_rows(K, int(fp8))
+    per = _hold_rows(K, fp8)
     if per == 0 or not (M <= per or (fp8 and 32 < M <= 2 * per and 2 * N >= 8192)):
         return False
     tiles, cus = N // 8, _cu_count()
@@ -874,7 +889,7 @@ def gemm_hold(x, w, wscale=None, par=None, epi="silu_mul", out=None):
     N = w.shape[0] // 2
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    per = L.ragk_gemm_hold_rows(K, int(wscale is not None))
+    per = _hold_rows(K, wscale is not None)
     _req(per > 0 and w.shape[1] == K and epi in PAIR_EPI and 0 < M <= 64, "gemm_hold shape")
     per = -(-M // -(-M // per))
     for r0 in range(0, M, per):

@@ -220,6 +220,10 @@ struct ChunkArgs {
   float* ssm_state;
   bf16_t* y;
   int H, P, N, G;
+  int nseg, seg_len;  // segments of a sequence, tokens of one (a multiple of CQ)
+  float* seg_state;   // [S][nseg + 1][H][N][P]: state that a segment leaves behind (zero entering it; the first: the sequence's
+                      // own), and last a copy of the sequence's entering state
+  float* seg_decay;   // [S][nseg][H]: what a segment leaves of the state that enters it
 };
 
 constexpr int CQ = 64;  // chunk length
@@ -249,7 +253,13 @@ __device__ __forceinline__ void split8(const float* f, u32x4& hi, u32x4& lo) {
 
 // NP: padded state rows (N <= NP), PS: state columns per block. 4 waves: wave w computes the outputs of chunk
 // tokens 16w .. 16w + 15 and owns state rows 16w, 16(w + 4), ... of the running state (fp32 accumulators).
-template <int NP, int PS>
+//
+// A chunk depends on the state before it, so few (head, sequence) pairs leave a chain of chunks on a part of the chip (64
+// heads of one sequence: half of the CUs, one block each). Then a sequence is cut into nseg segments (grid.y = S * nseg):
+// PASS 1 forms what each segment but the last adds to the state, PASS 2 sums the states before its segment and gives the
+// outputs; PASS 0 is the whole sequence in one. One sequence of 4000 tokens, 64 heads: 199 -> 29 + 64 us; 2000: 100 -> 17 + 44.
+// Side by side the blocks are bound by their vector instructions, so segments take the wide column slices, which form M once.
+template <int NP, int PS, int PASS>
 __global__ __launch_bounds__(256, NP <= 128 ? 2 : 1) void scan_chunk_kernel(ChunkArgs a) {
   using CB = Cfg<NP>;
   using CX = Cfg<PS>;
@@ -268,44 +278,21 @@ __global__ __launch_bounds__(256, NP <= 128 ? 2 : 1) void scan_chunk_kernel(Chun
 
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tid = threadIdx.x;
   const int fr = lane & 15, fh = lane >> 4;
-  const int h = blockIdx.x, seq = blockIdx.y, p0 = blockIdx.z * PS;
+  const int h = blockIdx.x, seq = PASS ? blockIdx.y / a.nseg : blockIdx.y, seg = PASS ? blockIdx.y % a.nseg : 0;
+  const int p0 = blockIdx.z * PS;
   const int g = h / (a.H / a.G);
   int t0, n;
   bool fresh;
   seq_span(a.q, seq, t0, n, fresh);
-  if (n <= 0) return;
-  float* st = a.ssm_state + ((size_t)a.q.states[seq] * a.H + h) * a.N * a.P;
+  const int c_begin = PASS ? seg * a.seg_len : 0, c_stop = PASS && seg + 1 < a.nseg ? min(n, c_begin + a.seg_len) : n;
+  if (c_begin >= n) return;
+  const bool last = c_stop == n;
+  if (PASS == 1 && last) return;
+  const size_t sz = (size_t)a.N * a.P;
+  float* st = a.ssm_state + ((size_t)a.q.states[seq] * a.H + h) * sz;
+  auto slot = [&](int k) { return a.seg_state + (((size_t)seq * (a.nseg + 1) + k) * a.H + h) * sz; };
   const float decay_rate = a.A[h] * 1.4426950408889634f, dskip = a.D[h], dbias = a.dt_bias[h];
   const int inner = a.H * a.P, offB = inner + g * a.N, offC = inner + (a.G + g) * a.N;
-
-  // running state: S[n][p], row tile i of this wave = rows 16 (wid + 4 i); lane holds rows 4fh + r, column fr
-  f32x4 S[SPW][PT];
-#pragma unroll
-  for (int i = 0; i < SPW; ++i)
-#pragma unroll
-    for (int j = 0; j < PT; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int nn = 16 * (wid + 4 * i) + 4 * fh + r, pp = p0 + 16 * j + fr;
-        S[i][j][r] = (!fresh && nn < a.N && pp < a.P) ? st[(size_t)nn * a.P + pp] : 0.f;
-      }
-  auto store_state = [&]() {  // high / low parts into LDS, [p][n]: four consecutive n per lane
-#pragma unroll
-    for (int i = 0; i < SPW; ++i)
-      if (wid + 4 * i < NT16) {
-#pragma unroll
-        for (int j = 0; j < PT; ++j) {
-          const f32x4 v = S[i][j];
-          const unsigned h0 = pk2bf(v[0], v[1]), h1 = pk2bf(v[2], v[3]);
-          const unsigned l0 = pk2bf(v[0] - __uint_as_float(h0 << 16), v[1] - __uint_as_float(h0 & 0xffff0000u));
-          const unsigned l1 = pk2bf(v[2] - __uint_as_float(h1 << 16), v[3] - __uint_as_float(h1 & 0xffff0000u));
-          const int off = (16 * j + fr) * SROW + (16 * (wid + 4 * i) + 4 * fh) * 2;
-          *reinterpret_cast<uint2*>(sSh + off) = make_uint2(h0, h1);
-          *reinterpret_cast<uint2*>(sSl + off) = make_uint2(l0, l1);
-        }
-      }
-  };
-  store_state();
 
   constexpr int BV = CQ * NP / 8 / 256, XV = (CQ * PS / 8 + 255) / 256;
   u32x4 rb[BV], rx[XV];
@@ -328,13 +315,83 @@ __global__ __launch_bounds__(256, NP <= 128 ? 2 : 1) void scan_chunk_kernel(Chun
     }
     const int tq = min(c0 + 16 * wid + fr, n - 1);
 #pragma unroll
-    for (int s = 0; s < CB::KS; ++s)
+    for (int s = 0; PASS != 1 && s < CB::KS; ++s)
       cf[s] = *reinterpret_cast<const bf16x8*>(a.xbc + (size_t)(t0 + tq) * a.ch + offC + min(32 * s + 8 * fh, a.N - 8));
     rdt = a.row[(size_t)(t0 + min(c0 + lane, n - 1)) * a.ld + a.off_dt + h];
   };
-  fetch(0);
+  fetch(c_begin);
 
-  for (int c0 = 0; c0 < n; c0 += CQ) {
+  // running state: S[n][p], row tile i of this wave = rows 16 (wid + 4 i); lane holds rows 4fh + r, column fr
+  f32x4 S[SPW][PT];
+  // f(value, offset of it in a state) for those inside N x P; e counts them all
+  auto each_e = [&](auto&& f, int& e) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < SPW; ++i)
+#pragma unroll
+      for (int j = 0; j < PT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int nn = 16 * (wid + 4 * i) + 4 * fh + r, pp = p0 + 16 * j + fr;
+          float v = S[i][j][r];
+          if (nn < a.N && pp < a.P) f(v, (size_t)nn * a.P + pp);
+          S[i][j][r] = v;
+          ++e;
+        }
+  };
+  auto each = [&](auto&& f) __attribute__((always_inline)) {
+    int e = 0;
+    each_e(f, e);
+  };
+#pragma unroll
+  for (int i = 0; i < SPW; ++i)
+#pragma unroll
+    for (int j = 0; j < PT; ++j) S[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  if (seg == 0) {
+    // the last segment's block overwrites the state; the first one's, which may run after it, has a copy
+    const float* src = PASS == 2 && !last ? slot(a.nseg) : st;
+    if (!fresh) each([&](float& v, size_t o) { v = src[o]; });
+    if (PASS == 1 && !fresh) each([&](float& v, size_t o) { slot(a.nseg)[o] = v; });
+  } else if (PASS == 2) {
+    constexpr int KU = SPW * PT <= 4 ? 4 : 2;  // segments whose states are in flight
+    for (int k0 = 0; k0 < seg; k0 += KU) {
+      float left[KU], add[KU][SPW * PT * 4];
+#pragma unroll
+      for (int u = 0; u < KU; ++u) {
+        const int k = min(k0 + u, seg - 1);
+        left[u] = a.seg_decay[((size_t)seq * a.nseg + k) * a.H + h];
+        const float* src = slot(k);
+        int e = 0;
+        each_e([&](float&, size_t o) { add[u][e] = src[o]; }, e);
+      }
+#pragma unroll
+      for (int u = 0; u < KU; ++u) {
+        if (k0 + u >= seg) break;
+        int e = 0;
+        each_e([&](float& v, size_t) { v = v * left[u] + add[u][e]; }, e);
+      }
+    }
+  }
+  auto store_state = [&]() {  // high / low parts into LDS, [p][n]: four consecutive n per lane
+#pragma unroll
+    for (int i = 0; i < SPW; ++i)
+      if (wid + 4 * i < NT16) {
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+          const f32x4 v = S[i][j];
+          const unsigned h0 = pk2bf(v[0], v[1]), h1 = pk2bf(v[2], v[3]);
+          const unsigned l0 = pk2bf(v[0] - __uint_as_float(h0 << 16), v[1] - __uint_as_float(h0 & 0xffff0000u));
+          const unsigned l1 = pk2bf(v[2] - __uint_as_float(h1 << 16), v[3] - __uint_as_float(h1 & 0xffff0000u));
+          const int off = (16 * j + fr) * SROW + (16 * (wid + 4 * i) + 4 * fh) * 2;
+          *reinterpret_cast<uint2*>(sSh + off) = make_uint2(h0, h1);
+          *reinterpret_cast<uint2*>(sSl + off) = make_uint2(l0, l1);
+        }
+      }
+  };
+  if constexpr (PASS != 1) store_state();
+  float decay = 0.f;  // log2 of what the segment leaves of its entering state
+
+
+  for (int c0 = c_begin; c0 < c_stop; c0 += CQ) {
     // every wave forms the chunk's running log-decay (lane = token) and keeps what it needs of it
     const float dt = c0 + lane < n ? softplusf(bf2f(rdt) + dbias) : 0.f;
     const float cum = wave_scan(-decay_rate * dt);
@@ -371,7 +428,10 @@ __global__ __launch_bounds__(256, NP <= 128 ? 2 : 1) void scan_chunk_kernel(Chun
       }
     }
     __syncthreads();
-    if (c0 + CQ < n) fetch(c0 + CQ);  // in flight during the products
+    if (c0 + CQ < c_stop) fetch(c0 + CQ);  // in flight during the products
+    decay += c_end;
+
+    if constexpr (PASS != 1) {
 
     // ---- M^T[s][t] = (B_s . C_t) e^(c_t - c_s) dt_s for s <= t; t = 16 wid + fr ----
     const int tq = 16 * wid + fr;
@@ -437,6 +497,7 @@ __global__ __launch_bounds__(256, NP <= 128 ? 2 : 1) void scan_chunk_kernel(Chun
                          pk2bf(__builtin_fmaf(dskip, x2, y[j][2]), __builtin_fmaf(dskip, x3, y[j][3])));
       }
     }
+    }
     // ---- S <- e^(c_end) S + B^T (w x) ----
     const float e_end = __builtin_amdgcn_exp2f(c_end);
 #pragma unroll
@@ -470,17 +531,12 @@ __global__ __launch_bounds__(256, NP <= 128 ? 2 : 1) void scan_chunk_kernel(Chun
       }
     }
     __syncthreads();  // every wave has read this chunk's tiles and the entering state
-    store_state();    // ordered before its readers by the next chunk's barrier
+    if constexpr (PASS != 1) store_state();  // ordered before its readers by the next chunk's barrier
   }
-#pragma unroll
-  for (int i = 0; i < SPW; ++i)
-#pragma unroll
-    for (int j = 0; j < PT; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int nn = 16 * (wid + 4 * i) + 4 * fh + r, pp = p0 + 16 * j + fr;
-        if (nn < a.N && pp < a.P) st[(size_t)nn * a.P + pp] = S[i][j][r];
-      }
+  if (PASS == 2 && !last) return;
+  float* dst = PASS == 1 ? slot(seg) : st;
+  if (PASS == 1 && tid == 0 && p0 == 0) a.seg_decay[((size_t)seq * a.nseg + seg) * a.H + h] = __builtin_amdgcn_exp2f(decay);
+  each([&](float& v, size_t o) { dst[o] = v; });
 }
 
 // ---- decode: one token per sequence from projection slabs P [S][B][ld] ----
@@ -632,7 +688,13 @@ int launch_gate_norm_wave(const TY* y, const bf16_t* row, int ld, const float* w
 
 template <int NP, int PS>
 int launch_scan_chunk(const ChunkArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL((scan_chunk_kernel<NP, PS>), dim3(a.H, a.q.S, (a.P + PS - 1) / PS), dim3(256), 0, st, a);
+  const dim3 grid(a.H, a.q.S * a.nseg, (a.P + PS - 1) / PS);
+  if (a.nseg == 1) {
+    hipLaunchKernelGGL((scan_chunk_kernel<NP, PS, 0>), grid, dim3(256), 0, st, a);
+  } else {
+    hipLaunchKernelGGL((scan_chunk_kernel<NP, PS, 1>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((scan_chunk_kernel<NP, PS, 2>), grid, dim3(256), 0, st, a);
+  }
   return (int)hipGetLastError();
 }
 
@@ -726,18 +788,22 @@ RAGK_API int ragk_ssm_scan_set_cols(int cols) {
   return 0;
 }
 
-// Chunked scan (bf16). y: bf16 [T][H*P]. P % 8 == 0, N % 8 == 0, N <= 256, ch % 8 == 0.
+// Chunked scan (bf16). y: bf16 [T][H*P]. P % 8 == 0, N % 8 == 0, N <= 256, ch % 8 == 0. nseg > 1: every sequence in segments of
+// seg_len tokens (a multiple of 64; the last takes the rest), seg_ws: S ((nseg + 1) N P + nseg) H floats.
 RAGK_API int ragk_ssm_scan_chunk(const int* cu_q, const int* kv_lens, const int* states, int T, int S, const void* xbc,
                                  int ch, const void* row, int ld, int off_dt, const float* dt_bias, const float* A,
-                                 const float* D, float* ssm_state, void* y, int H, int P, int N, int G, hipStream_t st) {
+                                 const float* D, float* ssm_state, void* y, int H, int P, int N, int G, int nseg,
+                                 int seg_len, float* seg_ws, hipStream_t st) {
   if (T <= 0) return 0;
-  if (P % 8 || N % 8 || N > 256 || ch % 8 || H % G || S < 1 || S > 65535 || (!cu_q && S != T))
+  if (P % 8 || N % 8 || N > 256 || ch % 8 || H % G || S < 1 || nseg < 1 || (long long)S * nseg > 65535 || (!cu_q && S != T) ||
+      (nseg > 1 && (!seg_ws || seg_len < CQ || seg_len % CQ)))
     return (int)hipErrorInvalidValue;
   const ChunkArgs a{{cu_q, kv_lens, states, T, S}, (const bf16_t*)xbc, ch, (const bf16_t*)row, ld, off_dt, dt_bias, A, D,
-                    ssm_state, (bf16_t*)y, H, P, N, G};
+                    ssm_state, (bf16_t*)y, H, P, N, G, nseg, seg_len, seg_ws, seg_ws + (size_t)S * (nseg + 1) * H * N * P};
   // narrow column slices while three of their blocks a CU are resident together: 320 (head, sequence) pairs of 1900 tokens
   // 154 us against 171, 64 of 4000 199 against 279
-  const bool narrow = P <= 32 || (g_scan_cols ? g_scan_cols == 32 : (long long)H * S * ((P + 63) / 64) <= 384);
+  // (segments fill the chip, and what two slices both compute then counts)
+  const bool narrow = P <= 32 || (g_scan_cols ? g_scan_cols == 32 : nseg == 1 && (long long)H * S * ((P + 63) / 64) <= 384);
 #define RAGK_SC(NPV) return narrow ? launch_scan_chunk<NPV, 32>(a, st) : launch_scan_chunk<NPV, 64>(a, st)
   if (N <= 32) RAGK_SC(32);
   if (N <= 64) RAGK_SC(64);

@@ -120,7 +120,7 @@ _SIGS = {
     "ragk_latent_decode": [P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, S],
     "ragk_latent_out": [P, I, I, I, I, P, P, P, P, P, I, I, I, I, I, I, I, I, S],
     "ragk_ssm_scan_set_cols": [I],
-    "ragk_ssm_scan_chunk": [P, P, P, I, I, P, I, P, I, I, P, P, P, P, P, I, I, I, I, S],
+    "ragk_ssm_scan_chunk": [P, P, P, I, I, P, I, P, I, I, P, P, P, P, P, I, I, I, I, I, I, P, S],
     "ragk_ssm_decode": [P, I, I, P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, S],
     "ragk_ssm_gate_norm": [P, I, P, I, P, P, I, I, I, I, F, I, S],
     # csrc/comm/allreduce.hip (xGMI peer-mapped all-reduce)

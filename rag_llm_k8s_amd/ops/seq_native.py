@@ -570,6 +570,25 @@ def scan_chunk_ok(spec):
     return spec.vdim % 8 == 0 and spec.state % 8 == 0 and spec.state <= 256
 
 
+SCAN_SEG_MIN_TOKENS = 768
+
+
+def scan_segments(longest, S, spec):
+    """(segments of a sequence, tokens of one) of the chunked scan. A (head, sequence) pair's chunks are a chain, 3.2 us each in
+    a block of its own; as many segments of it as leave two blocks a CU run side by side, for a first pass over their states: one
+    sequence of 4000 / 1500 / 800 tokens, 64 heads, prefill 2541 / 1276 / 924 -> 2339 / 1224 / 885 us, two of 1200 1505 -> 1493;
+    with less than four segments it lost (three and four of 1200: 1810 -> 1859, 2118 -> 2157)."""
+    from .native import _cu_count
+
+    blocks = S * spec.heads * -(-spec.vdim // 64)
+    chunks = -(-longest // 64)
+    n = min((2 if spec.state <= 128 else 1) * _cu_count() // blocks, chunks // 2)
+    if longest < SCAN_SEG_MIN_TOKENS or n < 4:
+        return 1, 0
+    per = -(-chunks // n)
+    return -(-chunks // per), 64 * per
+
+
 def ssm_scan_chunk(xbc, row, spec, w, meta, ssm_state):
     """MFMA chunked scan of packed prompts (bf16)."""
     _req(_act(row, "row") == 0 and xbc.dtype == BF16 and xbc.is_contiguous() and scan_chunk_ok(spec), "chunk scan operands")
@@ -579,10 +598,14 @@ def ssm_scan_chunk(xbc, row, spec, w, meta, ssm_state):
     for k in ("dt_bias", "A", "D"):
         _vec(w[k], spec.heads, F32, k)
     y = torch.empty((T, spec.inner), dtype=BF16, device=row.device)
+    nseg, seg_len = scan_segments(max(meta.host_q_lens) if meta.host_q_lens else T, S, spec)
+    ws = None
+    if nseg > 1:
+        ws = torch.empty(S * spec.heads * ((nseg + 1) * spec.state * spec.vdim + nseg), dtype=F32, device=row.device)
     check(_lib.lib().ragk_ssm_scan_chunk(cu, meta.kv_lens.data_ptr(), meta.states.data_ptr(), T, S, xbc.data_ptr(),
                                          xbc.stride(0), row.data_ptr(), row.stride(0), spec.off_dt, w["dt_bias"].data_ptr(),
                                          w["A"].data_ptr(), w["D"].data_ptr(), ssm_state.data_ptr(), y.data_ptr(),
-                                         spec.heads, spec.vdim, spec.state, spec.groups, stream_ptr()),
+                                         spec.heads, spec.vdim, spec.state, spec.groups, nseg, seg_len, ptr(ws), stream_ptr()),
           "ragk_ssm_scan_chunk")
     return y
 

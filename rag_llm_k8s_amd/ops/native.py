@@ -212,6 +212,11 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
         return _gemm_blas(x, w, resid, out, epi)
     if path is None and M > 64:
         rows = w.shape[0]
+        # gemm_mid addresses a tile's rows with 32-bit offsets: rows megabytes apart are brought together first
+        if x.stride(0) * 512 + 2 * K >= 2 ** 31:
+            x = x.contiguous()
+        if w.stride(0) * 256 + 2 * K >= 2 ** 31:
+            w = w.contiguous()
         # gemm_w4 addresses operands with 32-bit buffer offsets
         fits = x.stride(0) * M * 2 < 2 ** 31 and w.stride(0) * rows * 2 < 2 ** 31
         if not fits and use_pp(M, N, K, epi):
@@ -229,9 +234,10 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
             return out
     if path == 0:
         return gemm_mid(x, w, bias=bias, resid=resid, epi=epi, out=out, out_f32=out_f32)
-    if path is None and use_hold(M, N, K, epi):
+    if path is None and use_hold(M, N, K, epi) and _vec_rows(x, w):
         return gemm_hold(x, w, par=bias, epi=epi, out=out)
-    if path is None and use_vocab(M, N, K, epi) and out_f32 and out.stride(0) == N:
+    if (path is None and use_vocab(M, N, K, epi) and out_f32 and out.stride(0) == N and _vec_rows(x, w)
+            and out.data_ptr() % 16 == 0):
         return gemm_stream_part(x, w, out=out, rows=64, S=1)
     if path is None and STREAM_DEFAULT and use_stream(M, N, K, epi):
         path = 5
@@ -881,6 +887,11 @@ def use_hold(M, N, K, epi, fp8=False):
     return fp8 or not use_stream(M, N, K, epi) or _lib.lib().ragk_gemm_stream_splits(N, K, EPI[epi], 0) > 1
 
 
+def _vec_rows(*ts):
+    """Whether every row starts on 16 bytes (odd strides and offsets stay with the kernels that took them before)."""
+    return all((t.stride(0) * t.element_size()) % 16 == 0 and t.data_ptr() % 16 == 0 for t in ts)
+
+
 def gemm_hold(x, w, wscale=None, par=None, epi="silu_mul", out=None):
     """Packed gate/up projection of at most 64 rows with the activations held in registers (gemm_hold.hip); more rows than
     one launch holds go in equal launches."""
@@ -945,7 +956,7 @@ def gemm_fp8(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False):
     if M == 0:
         return out
     ldr = resid.stride(0) if resid is not None else 0
-    if use_hold(M, N, K, epi, fp8=True):
+    if use_hold(M, N, K, epi, fp8=True) and _vec_rows(x, w8):
         return gemm_hold(x, w8, sw, epi=epi, out=out)
     if M <= DEC_MAX_M and FP8_DEC_STREAM and use_stream(M, N, K, epi, fp8=True):
         rc = _gemm_stream(x, w8, sw, out, bias, resid, ldr, M, N, K, epi, e, out_f32)

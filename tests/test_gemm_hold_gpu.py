@@ -61,3 +61,22 @@ def test_stream_slabs(native, N, K):
     for M in (5, 17, 64):
         x = torch.randn(M, K, device=DEV).bfloat16()
         assert (native.gemm_part(x, w).double().sum(0) - x.double() @ w.double().t()).abs().max().item() < K * 2.0 ** -24 * 8
+
+
+def test_rows_of_any_stride(native):
+    """Rows that start off the 16 bytes of a vector, or megabytes apart, give what their copies give."""
+    w = (torch.randn(2816, 2048, device=DEV) * 2048 ** -0.5).bfloat16()
+    head = (torch.randn(16384, 2048, device=DEV) * 2048 ** -0.5).bfloat16()
+    w8 = quantize_weight(w)
+    base = torch.randn(12, 2053, device=DEV).bfloat16()
+    for x in (base[:, :2048], base[:, 3:2051]):
+        c = x.contiguous()
+        # both round to bf16 once from fp32 sums of another order
+        for a, b in ((native.gemm(x, w, epi="silu_mul"), native.gemm(c, w, epi="silu_mul")),
+                     (native.gemm_fp8(x, w8, epi="silu_mul"), native.gemm_fp8(c, w8, epi="silu_mul")),
+                     (native.gemm(c, head, out_f32=True), native.gemm(c, head, out=torch.empty(12, 16392, device=DEV)[:, :16384],
+                                                                      out_f32=True))):
+            assert ((a.double() - b.double()).norm() / b.double().norm()).item() < 2.0 ** -7
+    far = torch.empty_strided((70, 256), (2 ** 22, 1), dtype=torch.bfloat16, device=DEV)
+    far.copy_(torch.randn(70, 256, device=DEV))
+    assert torch.equal(native.gemm(far, w[:, :256].contiguous()), native.gemm(far.contiguous(), w[:, :256].contiguous()))

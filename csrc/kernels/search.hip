@@ -814,7 +814,10 @@ RAGK_API int ragk_l2_scan_groups(int row_begin, int row_end, int nq) {
 RAGK_API int ragk_l2_search_groups(int row_begin, int row_end, int nq, int k, int d) {
   if (!use_mfma(nq, k, d)) return ragk_l2_scan_groups(row_begin, row_end, nq);
   const int n = max(0, row_end - row_begin);
-  return max(1, min((n + 16 * mfma_rt(n) - 1) / (16 * mfma_rt(n)), 256));  // a block a CU
+  // a block a CU over all query groups, but eight (one an XCD, which then serves its rows to every group from its L2): 1000
+  // queries of 10000 x 1024, 256 blocks a group, each staging its q^T for one tile a wave, 1068 us, so 265
+  const int groups = nq > 16 ? (nq + 31) / 32 : 1;
+  return max(1, min((n + 16 * mfma_rt(n) - 1) / (16 * mfma_rt(n)), max(8, 256 / groups)));
 }
 
 // Exact top-k (k <= 64) over rows [row_begin, row_end) of xt[d][cap]; part_d / part_i hold
@@ -864,10 +867,17 @@ RAGK_API int ragk_l2_search(const float* xt, int cap, int d, int row_begin, int 
   // queries per block, padded to the next count below. Twelve or sixteen spill the scalar registers, and one pass of them loses
   // to two groups of eight that share the L2: 12 queries of 500000 x 1024 594 us, 15 837; in groups of eight 528
   const int QB = nq > 4 ? 8 : (nq > 2 ? 4 : nq);
-  if (QB == 8) launch_scan_s<8>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
-  else if (QB == 4) launch_scan_s<4>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
-  else if (QB == 2) launch_scan_s<2>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
-  else launch_scan_s<1>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, q, nq, k, part_d, part_i, ids_map);
+  // (a grid's second dimension ends at 65535 query groups)
+  for (int q0 = 0, qn; q0 < nq; q0 += qn) {
+    qn = min(nq - q0, 65535 * QB);
+    const float* qs = q + (size_t)q0 * d;
+    float* pd = part_d + (size_t)q0 * G * k;
+    int* pi = part_i + (size_t)q0 * G * k;
+    if (QB == 8) launch_scan_s<8>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, qs, qn, k, pd, pi, ids_map);
+    else if (QB == 4) launch_scan_s<4>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, qs, qn, k, pd, pi, ids_map);
+    else if (QB == 2) launch_scan_s<2>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, qs, qn, k, pd, pi, ids_map);
+    else launch_scan_s<1>(S, G, st, xt, cap, d, row_begin, row_end, ntiles, qs, qn, k, pd, pi, ids_map);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
   hipLaunchKernelGGL(topk_lists_merge_kernel, dim3(nq), dim3(MW * 64), 0, st, part_d, part_i, G, k, out_d, out_i);

@@ -354,7 +354,11 @@ __global__ __launch_bounds__(NT) void gather_rows_kernel(const bf16_t* x, int ld
 
 // h = bf16(h + bf16(sum_s P[s][row]))  (HF: bf16 linear output, then the bf16 residual add), written
 // back to h; out = rmsnorm(h) * w exactly as rmsnorm_kernel. One block of 512 threads per row.
+// ROUNDED = false: h = bf16(h + sum_s P[s][row]), the rounding of a product whose epilogue adds the residual: where a prompt's
+// step may take either form, the one with slabs loses nothing (300 rows, four Llama layers 4096 wide: error of the last values
+// against 64 bits 7.11e-3 with the sum rounded first, 6.80e-3 without and 6.79e-3 from the epilogue).
 constexpr int PNT = 512;
+template <bool ROUNDED>
 __global__ __launch_bounds__(PNT) void add_partials_rmsnorm_kernel(const float* __restrict__ P, int S, int M,
                                                                    bf16_t* h, int ldh,
                                                                    const bf16_t* __restrict__ w, bf16_t* out,
@@ -387,7 +391,7 @@ __global__ __launch_bounds__(PNT) void add_partials_rmsnorm_kernel(const float* 
       add_slabs8(pv[i], P + (size_t)row * H + vi * 8, S, (size_t)M * H, a);
       unpack8(hv[i], v[i]);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[i][e] = bf2f(f2bf(v[i][e] + bf2f(f2bf(a[e]))));
+      for (int e = 0; e < 8; ++e) v[i][e] = bf2f(f2bf(v[i][e] + (ROUNDED ? bf2f(f2bf(a[e])) : a[e])));
       *reinterpret_cast<u32x4*>(hr + vi * 8) = pack8(v[i]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss += v[i][e] * v[i][e];
@@ -550,11 +554,11 @@ RAGK_API int ragk_gather_rows(const void* x, int ldx, const int* idx, void* out,
 }
 
 RAGK_API int ragk_add_partials_rmsnorm(const float* P, int S, int M, void* h, int ldh, const void* w, void* out,
-                                       int ldo, int H, float eps, hipStream_t st) {
+                                       int ldo, int H, float eps, int rounded, hipStream_t st) {
   if (M <= 0) return 0;
   if (H % 8 || H > 8 * PNT * 2 || S < 1) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(add_partials_rmsnorm_kernel, dim3(M), dim3(PNT), 0, st, P, S, M, (bf16_t*)h, ldh,
-                     (const bf16_t*)w, (bf16_t*)out, ldo, H, eps);
+  const auto kernel = rounded ? add_partials_rmsnorm_kernel<true> : add_partials_rmsnorm_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(M), dim3(PNT), 0, st, P, S, M, (bf16_t*)h, ldh, (const bf16_t*)w, (bf16_t*)out, ldo, H, eps);
   return (int)hipGetLastError();
 }
 

@@ -387,11 +387,10 @@ class LlamaModel(DecoderModel):
         return self._final(h, inp)
 
     def hidden_states_splitk(self, inp: StepInput, h, attn, ns_o, ns_d):
-        """TP=1 prefill of a step too small to fill the CUs with 256x256 output tiles (a single ~5k-token
-        RAG prompt): o_proj / down run as split-K GEMMs into fp32 slabs (ops/native.py:prefill_nsplit,
-        gemm_w4c KSPLIT) and the residual add moves into the following RMSNorm kernel
-        (add_partials_rmsnorm), which the layer needs anyway -- same rounding points as the residual
-        epilogue path (bf16 projection output, bf16 residual add)."""
+        """TP=1 prefill of a step whose output tiles leave CUs idle (a few hundred rows): o_proj / down run as split-K GEMMs
+        into fp32 slabs (ops/native.py:slab_count) and the residual add moves into the following RMSNorm kernel
+        (add_partials_rmsnorm), which the layer needs anyway -- rounded where the residual epilogue rounds, once, behind the
+        add."""
         be, w, c = self.be, self.w, self.cfg
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
         layers = w.layers
@@ -401,14 +400,14 @@ class LlamaModel(DecoderModel):
             qkv = be.gemm_rope_kv(xn, L["wqkv"], inp.positions, self.cos, self.sin, inp.slots, kc, vc, Hq, Hkv, D)
             be.attn_prefill(qkv, kc, vc, inp.meta, attn, Hq, Hkv, D)
             if ns_o > 1:
-                xn = be.add_partials_rmsnorm(be.gemm_splitk(attn, L["wo"], ns_o), h, L["ln_post"], c.rms_norm_eps)
+                xn = be.add_partials_rmsnorm(be.gemm_splitk(attn, L["wo"], ns_o), h, L["ln_post"], c.rms_norm_eps, rounded=False)
             else:
                 be.gemm(attn, L["wo"], resid=h, epi="resid", out=h)
                 xn = be.rmsnorm(h, L["ln_post"], c.rms_norm_eps)
             a = be.gemm(xn, L["wgu"], epi="silu_mul")
             nxt = layers[li + 1]["ln_in"] if li + 1 < len(layers) else w.norm
             if ns_d > 1:
-                xn = be.add_partials_rmsnorm(be.gemm_splitk(a, L["wdown"], ns_d), h, nxt, c.rms_norm_eps)
+                xn = be.add_partials_rmsnorm(be.gemm_splitk(a, L["wdown"], ns_d), h, nxt, c.rms_norm_eps, rounded=False)
             else:
                 be.gemm(a, L["wdown"], resid=h, epi="resid", out=h)
                 xn = be.rmsnorm(h, nxt, c.rms_norm_eps)

@@ -60,7 +60,7 @@ _SIGS = {
     "ragk_mlp_engine_split": [I, I, I, I, P],
     "ragk_gemm_part_ksteps": [I, I, I],
     "ragk_gemm_part_set_min_blocks": [I],
-    "ragk_add_partials_rmsnorm": [P, I, I, P, I, P, P, I, I, F, S],
+    "ragk_add_partials_rmsnorm": [P, I, I, P, I, P, P, I, I, F, I, S],
     "ragk_rope_kv_partials": [P, I, I, I, P, I, P, P, P, P, P, P, I, I, I, I, S],
     "ragk_gemm_dec": [P, I, P, I, P, I, P, P, I, I, I, I, I, I, I, P, P, S],
     "ragk_gemm_dec_splits": [I, I, I],

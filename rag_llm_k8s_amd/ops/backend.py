@@ -172,8 +172,9 @@ class TorchBackend:
         """add_partials_rmsnorm (o_proj slabs + residual + post-attention norm) then mlp_engine, one op."""
         return self.mlp_engine(self.add_partials_rmsnorm(P, h, gamma, eps), w_gu, w_down, h)
 
-    def add_partials_rmsnorm(self, P, h, w, eps):
-        h.copy_((h.float() + P.sum(0).to(h.dtype).float()).to(h.dtype))
+    def add_partials_rmsnorm(self, P, h, w, eps, rounded=True):
+        y = P.sum(0)
+        h.copy_((h.float() + (y.to(h.dtype).float() if rounded else y)).to(h.dtype))
         return R.rmsnorm(h, w, eps)
 
     def rope_kv_partials(self, P, q_out, positions, cos_t, sin_t, slots, kc, vc, Hq, Hkv, D):
@@ -410,8 +411,8 @@ class NativeBackend(TorchBackend):
     def gemm_part_silu(self, pgu, w):
         return self.n.gemm_part_silu(pgu, w)
 
-    def add_partials_rmsnorm(self, P, h, w, eps):
-        return self.n.add_partials_rmsnorm(P, h, w, eps)
+    def add_partials_rmsnorm(self, P, h, w, eps, rounded=True):
+        return self.n.add_partials_rmsnorm(P, h, w, eps, rounded=rounded)
 
     def mlp_engine_ok(self, M, w_gu, w_down):
         return self.n.mlp_engine_ok(M, w_gu, w_down)

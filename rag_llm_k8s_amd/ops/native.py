@@ -1042,8 +1042,9 @@ def rope_kv(qkv, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, Hkv, D, a
                                   stream_ptr()), "ragk_rope_kv")
 
 
-def add_partials_rmsnorm(P, h, w, eps, out=None):
-    """h <- bf16(h + bf16(P.sum(0))) in place; returns rmsnorm(h) * w (split-K decode consumer)."""
+def add_partials_rmsnorm(P, h, w, eps, out=None, rounded=True):
+    """h <- bf16(h + bf16(P.sum(0))) in place; returns rmsnorm(h) * w (split-K decode consumer). rounded=False: the sum is
+    added as it is, as a product's residual epilogue does (prompts, whose steps take either)."""
     _bf16_2d(h, "h")
     M, H = h.shape
     _req(P.dtype == torch.float32 and P.is_contiguous() and P.dim() == 3 and P.shape[1:] == (M, H), "partials shape")
@@ -1051,7 +1052,7 @@ def add_partials_rmsnorm(P, h, w, eps, out=None):
     out = torch.empty_like(h) if out is None else out
     _req(out.shape == (M, H) and out.stride(1) == 1, "out")
     check(_lib.lib().ragk_add_partials_rmsnorm(P.data_ptr(), P.shape[0], M, h.data_ptr(), h.stride(0), w.data_ptr(),
-                                               out.data_ptr(), out.stride(0), H, float(eps), stream_ptr()),
+                                               out.data_ptr(), out.stride(0), H, float(eps), int(rounded), stream_ptr()),
           "ragk_add_partials_rmsnorm")
     return out
 

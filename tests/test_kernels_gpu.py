@@ -1020,6 +1020,22 @@ def test_add_partials_rmsnorm(native, S, M, H):
     assert rel_err(y.cpu(), ref) < 4e-3
 
 
+@pytest.mark.parametrize("S,M,H", [(1, 70, 384), (2, 300, 4096), (9, 65, 4096), (3, 80, 8192)])
+def test_add_partials_unrounded(native, S, M, H):
+    """Slabs of a prompt: h <- bf16(h + sum P), no rounding of the sum before the add, as the residual epilogue."""
+    P = torch.randn(S, M, H, device=DEV) * 3
+    h = torch.randn(M, H, device=DEV).bfloat16()
+    w = torch.randn(H, device=DEV).bfloat16()
+    s = P[0].clone()
+    for i in range(1, S):
+        s += P[i]
+    ref = (h.float() + s).bfloat16()
+    y = native.add_partials_rmsnorm(P, h, w, 1e-5, rounded=False)
+    # the slabs' order within the sum is the kernel's: its last fp32 bit may flip a tie of bf16 (of 2^16 spacings, so few)
+    assert (h != ref).float().mean().item() < 1e-3
+    assert rel_err(y.cpu(), R.rmsnorm(h.cpu(), w.cpu(), 1e-5)) < 4e-3
+
+
 @pytest.mark.parametrize("S,T", [(4, 33), (9, 32), (16, 1)])  # S > 8: more than one unrolled slab group
 def test_rope_kv_partials(native, S, T):
     torch.manual_seed(12)

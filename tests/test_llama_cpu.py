@@ -158,6 +158,23 @@ def test_split_k_decode_path_matches_plain_decode(tiny):
     assert outs[0] == outs[1]
 
 
+def test_split_prompt_rounds_where_the_whole_product_does(tiny):
+    """A prompt whose o_proj / down come as slabs (the whole sum and zeros, so that only the rounding is looked at) is the
+    residual epilogue's prompt bit for bit: logits and caches."""
+    cfg, hf, sd = tiny
+    w = LlamaWeights.from_state_dict(cfg, sd, "cpu")
+    g = torch.Generator().manual_seed(2)
+    ids = torch.randint(3, cfg.vocab_size, (70,), generator=g).tolist()
+    outs = []
+    for ns in (1, 2):
+        model = LlamaModel(cfg, w, "cpu", max_positions=512)
+        model.be.prefill_nsplit = lambda M, w: ns
+        model.be.gemm_splitk = lambda x, w, n: torch.stack([x.float() @ w.float().t(), torch.zeros(x.shape[0], w.shape[0])])
+        outs.append((_prefill_logits(model, ids), [t.clone() for kv in model.kv_cache for t in kv]))
+    assert torch.equal(outs[0][0], outs[1][0])
+    assert all(torch.equal(a, b) for a, b in zip(outs[0][1], outs[1][1]))
+
+
 def test_batch1_decode_mlp_engine_path_matches_plain_decode(tiny):
     """Batch-1 split-K decode with the persistent post-attention launch (o_proj slabs + residual + norm +
     gate/up + SiLU + down + residual in one op,

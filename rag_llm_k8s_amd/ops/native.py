@@ -228,7 +228,7 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
                 gemm(x[h:], w, bias=bias, epi=epi, out=out[h:])
                 return out
         else:
-            w4 = fits and K % 64 == 0 and K >= 192 and (N % 128 == 0 if epi in PAIR_EPI else N % 8 == 0)
+            w4 = fits and (N % 128 == 0 if epi in PAIR_EPI else N % 8 == 0)
             for r0, r1, mi, S in gemm_plan(M, rows, K, w4, _cu_count()):
                 _gemm_rows(x, w, bias, resid, epi, out, out_f32, r0, r1, mi, S)
             return out
@@ -340,7 +340,7 @@ def gemm_plan(M, rows, K, w4, cus):
     1777 rows gemm_w4 329 against 365 (its 128 x 128 wave tiles read less LDS per MFMA)."""
     t, mi, S = _mid_best(M, rows, K, cus, SLAB_US, 3.0)
     plan = ((0, M, mi, S),)
-    if not w4:
+    if not w4 or K % 64 or K < 192:  # gemm_w4's ring needs three K-tiles
         return plan
     full = _tiles_us(M, rows, K, 0, 1, cus)
     if full < t:
@@ -544,7 +544,7 @@ def _slab_best(M, N, K, cus):
     o_proj / down at 300 rows: 28 / 88 us whole, 17 / 42 us as 2 / 4 slabs; at 14076 rows the slabs' traffic (212 us in the
     norm) is more than the last round that they would fill."""
     whole = 0.0
-    for r0, r1, mi, S in gemm_plan(M, N, K, K >= 192, cus):
+    for r0, r1, mi, S in gemm_plan(M, N, K, True, cus):
         whole += _tiles_us(r1 - r0, N, K, mi, S, cus) + (3.0 + SLAB_US * S * (r1 - r0) * N if S > 1 else 0)
     best, S, mi = min((t - 0.75 * SLAB_US * M * N, S, mi) for t, mi, S in [_mid_best(M, N, K, cus, SLAB_US, 0.0, even=True)])
     w4 = prefill_nsplit(M, N, K)

@@ -32,6 +32,16 @@ def test_native_forward_is_the_layered_one(native, pooling, kind, lens):
     assert bool((out[0] == 9.0).all()) and bool((out[-1] == 9.0).all())
 
 
+def test_narrow_encoder_of_a_large_batch(native):
+    """128 columns (two K-tiles a product) at the tokens of a full ingest batch."""
+    m = model("mean", hidden=128)
+    lens = [512] * 100
+    ids = np.random.RandomState(4).randint(0, 500, sum(lens)).astype(np.int32)
+    out = torch.zeros(len(lens), 128, device=DEV)
+    m.embed_into(ids, np.asarray(lens, dtype=np.int64), out, np.arange(len(lens)))
+    assert torch.equal(out, m.forward_packed(torch.from_numpy(ids).to(DEV), lens))
+
+
 def test_engine_order_and_odd_outputs(native):
     """Batches cut by tokens, unsorted lengths; an output that the native call does not take (strided columns) still works."""
     m = model("mean")

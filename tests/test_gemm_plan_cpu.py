@@ -28,3 +28,11 @@ def test_launch_model_prefers_full_rounds():
     assert n.gemm_plan(4096, 4096, 4096, True, 256) == ((0, 4096, 0, 1),)
     (a, b) = n.gemm_plan(14076, 4096, 4096, True, 256)
     assert a == (0, 12288, 0, 1) and b[2] > 0
+
+
+def test_short_inner_dimension_stays_off_the_long_ring():
+    """Encoders of 128 columns: gemm_w4 refuses two K-tiles, at the batch sizes too where its tiles would be cheapest."""
+    for H, I in ((128, 512), (128, 1024), (128, 2048)):
+        for T in (65, 300, 4096, 24576, 49152, 65536):
+            for N, K in ((3 * H, H), (H, H), (I, H), (H, I)):
+                assert all(mi in n.MID_US for _, _, mi, _ in n.gemm_plan(T, N, K, True, 256)) or K >= 192

@@ -578,9 +578,12 @@ class NativeBackend(TorchBackend):
     def encoder_forward(self, cfg, w, ids, lens, first_pos, out, rows):
         T = int(lens.sum())
         if (out.dtype != torch.float32 or out.stride(1) != 1 or out.device != w.word.device or T == 0
-                or T * max(3 * cfg.hidden_size, cfg.intermediate_size) * 2 >= 2 ** 31 or not self.n.encoder_forward_ok(cfg, w)):
+                or T * max(3 * cfg.hidden_size, cfg.intermediate_size) * 2 >= 2 ** 31):
             return False
-        self.n.encoder_forward(cfg, w, ids, lens, first_pos, out, rows)
+        weights = self.n.encoder_pointers(cfg, w)
+        if weights is None:
+            return False
+        self.n.encoder_forward(cfg, weights, ids, lens, first_pos, out, rows)
         return True
 
     def topk_candidates(self, logits, K, vocab_offset=0, max_cand=512, chunks=None):

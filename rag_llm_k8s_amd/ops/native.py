@@ -7,7 +7,9 @@ HIP stream, so everything here is capturable in a hipGraph (torch.cuda.CUDAGraph
 from __future__ import annotations
 
 import functools
+import itertools
 import math
+import operator
 import os
 import threading
 
@@ -1088,19 +1090,36 @@ def pool_l2norm(hidden, cu, mode="cls", normalize=True, out=None):
 ENCODER_LAYER = ("wqkv", "bqkv", "wo", "bo", "ln1_g", "ln1_b", "wi", "bi", "wo2", "bo2", "ln2_g", "ln2_b")
 
 
-def encoder_forward_ok(cfg, w):
-    """Whether encoder_forward takes these weights (else: layer by layer through the checked entry points)."""
-    H, I = cfg.hidden_size, cfg.intermediate_size
+def encoder_pointers(cfg, w):
+    """Addresses of what encoder_forward reads of an encoder's weights, [word, pos, ln_g, ln_b, type row (or None), then
+    ENCODER_LAYER of every layer], or None if one of them would be read wrongly by its address (then: layer by layer through
+    the checked entry points). For the call at hand only, a property at a time over all tensors: 77 of them take 35 us."""
+    H, I, T = cfg.hidden_size, cfg.intermediate_size, torch.Tensor
     if H % 128 or I % 128 or H > 2048 or max(3 * H, I) >= STREAM_MIN_ROWS or H // cfg.num_attention_heads not in (32, 64, 128):
-        return False
-    sizes = [2 * n for n in (3 * H * H, 3 * H, H * H, H, H, H, I * H, I, H * I, H, H, H)]
-    return (all([L[k].nbytes for k in ENCODER_LAYER] == sizes and L["wqkv"].dtype == torch.bfloat16 for L in w.layers)
-            and w.word.dtype == torch.bfloat16 and w.word.shape[1] == H and w.pos.shape[1] == H and w.type_row.numel() == H)
+        return None
+    row = w.type_row
+    row = row.view(-1) if row is not None and row.is_contiguous() else row
+    layers = list(itertools.chain.from_iterable(map(operator.itemgetter(*ENCODER_LAYER), w.layers)))
+    ts = [w.word, w.pos, w.ln_g, w.ln_b] + ([row] if row is not None else []) + layers
+    shapes = [(w.word.shape[0], H), (w.pos.shape[0], H)] + [(H,)] * (len(ts) - len(layers) - 2) + [
+        (3 * H, H), (3 * H,), (H, H), (H,), (H,), (H,), (I, H), (I,), (H, I), (H,), (H,), (H,)] * len(w.layers)
+    if (all(map(T.is_contiguous, ts)) and list(map(T.size, ts)) == shapes and [t.dtype for t in ts].count(torch.bfloat16) == len(ts)
+            and list(map(T.get_device, ts)).count(w.word.get_device()) == len(ts)):
+        at = list(map(T.data_ptr, ts))
+        if not any(map((15).__and__, at)):  # the kernels' vectors and LDS-DMA pieces
+            return at if row is not None else at[:4] + [None] + at[4:]
+    return None
 
 
-def encoder_forward(cfg, w, ids, lens, first_pos, out, rows):
+def encoder_forward_ok(cfg, w):
+    """Whether encoder_forward takes these weights."""
+    return encoder_pointers(cfg, w) is not None
+
+
+def encoder_forward(cfg, weights, ids, lens, first_pos, out, rows):
     """Embeddings of packed sequences (host int32 ids, int64 lens) into rows `rows` of out (fp32 on the device): one upload
-    of the step's integers, one workspace, one native call for all launches (csrc/kernels/encoder.hip)."""
+    of the step's integers, one workspace, one native call for all launches (csrc/kernels/encoder.hip). `weights`: their
+    encoder_pointers."""
     import ctypes
 
     import numpy as np
@@ -1115,7 +1134,7 @@ def encoder_forward(cfg, w, ids, lens, first_pos, out, rows):
     pos = np.arange(first_pos, first_pos + T, dtype=np.int32) - np.repeat(cu[:-1], lens)
     tiles = build_prefill_tiles(lens, nh, nh).numpy().reshape(-1)
     parts = [ids, pos, cu, lens, rows, tiles]
-    at = np.cumsum([0] + [len(p) for p in parts]).tolist()
+    at = list(itertools.accumulate(map(len, parts), initial=0))
     ints = torch.from_numpy(np.concatenate(parts).astype(np.int32, copy=False)).to(dev)
     L, cus, c = _lib.lib(), _cu_count(), _lib.EncoderCall()
     slab = 0
@@ -1128,17 +1147,16 @@ def encoder_forward(cfg, w, ids, lens, first_pos, out, rows):
             slab = max(slab, S * (r1 - r0) * N if S > 1 else 0)
     # activations in the order h, a, attn, qkv, f, then the slabs
     sizes = [2 * T * n for n in (H, H, H, 3 * H, I)] + [4 * slab]
-    off = np.cumsum([0] + [-(-n // 256) * 256 for n in sizes]).tolist()
+    off = list(itertools.accumulate([-(-n // 256) * 256 for n in sizes], initial=0))
     buf = torch.empty(off[-1], dtype=torch.uint8, device=dev)
     p, q = buf.data_ptr(), ints.data_ptr()
     c.h, c.a, c.attn, c.qkv, c.f, c.ws = (p + o for o in off[:-1])
     c.ids, c.pos, c.cu, c.lens, c.rows, c.tiles = (q + 4 * o for o in at[:-1])
-    table = [t.data_ptr() for layer in w.layers for t in map(layer.__getitem__, ENCODER_LAYER)]
+    c.word, c.pos_table, c.ln_g, c.ln_b, c.type_row, *table = weights
     ptrs = (ctypes.c_void_p * len(table))(*table)
-    c.layers = ctypes.addressof(ptrs)
-    c.word, c.pos_table, c.type_row = w.word.data_ptr(), w.pos.data_ptr(), w.type_row.data_ptr()
-    c.ln_g, c.ln_b, c.out, c.ldo = w.ln_g.data_ptr(), w.ln_b.data_ptr(), out.data_ptr(), out.stride(0)
-    c.n_layers, c.T, c.B, c.H, c.I, c.heads, c.n_tiles = len(w.layers), T, B, H, I, nh, len(tiles) // 2
+    c.layers, c.n_layers = ctypes.addressof(ptrs), len(table) // len(ENCODER_LAYER)
+    c.out, c.ldo = out.data_ptr(), out.stride(0)
+    c.T, c.B, c.H, c.I, c.heads, c.n_tiles = T, B, H, I, nh, len(tiles) // 2
     c.pooling, c.normalize, c.eps = {"cls": 0, "mean": 1, "last": 2}[cfg.pooling], int(cfg.normalize), float(cfg.layer_norm_eps)
     check(L.ragk_encoder_forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
     return out
@@ -1225,6 +1243,11 @@ def build_prefill_tiles(q_lens, Hq, Hkv):
 
     qt = prefill_qtile(Hq, Hkv)
     ql = np.asarray(q_lens, dtype=np.int64)
+    top = (int(ql.max()) - 1) // qt if len(ql) else -1
+    if len(ql) * (top + 1) <= 64:  # one query's: 10 us as a list, 21 through the arrays below
+        lens = ql.tolist()
+        tiles = [(s, q0) for q0 in range(top * qt, -1, -qt) for s, n in enumerate(lens) if n > q0]
+        return torch.tensor(tiles, dtype=torch.int32).reshape(-1, 2)
     nt = (ql + qt - 1) // qt
     seq = np.repeat(np.arange(len(ql)), nt)
     first = np.repeat(np.cumsum(nt) - nt, nt)

@@ -67,3 +67,47 @@ def test_encoder_matches_transformers(kind, pooling):
     assert cos.min().item() > 0.995, cos
     assert torch.allclose(got.norm(dim=-1), torch.ones(B), atol=1e-3)
     assert ((got - ref).norm() / ref.norm()).item() < 5e-2
+
+
+def _edited(name, f):
+    from rag_llm_k8s_amd.models import encoder as E
+
+    cfg = E.EncoderConfig(model_type="bert", vocab_size=50, hidden_size=128, num_hidden_layers=2, num_attention_heads=4,
+                          intermediate_size=128, max_position_embeddings=64)
+    w = E.EncoderWeights.random(cfg, "cpu")
+    if name in w.layers[1]:
+        w.layers[1][name] = f(w.layers[1][name])
+    else:
+        setattr(w, name, f(getattr(w, name)))
+    return cfg, w
+
+
+def _off16(t):
+    return torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("name", ["word", "pos", "ln_g", "ln_b", "type_row", "wqkv", "bqkv", "wo", "bo", "ln1_g", "ln1_b", "wi",
+                                  "bi", "wo2", "bo2", "ln2_g", "ln2_b"])
+def test_weights_that_the_native_forward_takes(name):
+    """It reads them by address alone: another type, order, size or start of any one goes layer by layer."""
+    from rag_llm_k8s_amd.ops import native
+
+    def strided(t):
+        return torch.stack([t, t], -1)[..., 0]
+
+    assert native.encoder_forward_ok(*_edited(name, lambda t: t.clone()))
+    for f in (lambda t: t.half(), strided, _off16, lambda t: torch.cat([t, t])):
+        if f(torch.zeros(128, 128)).shape[0] == 256 and name in ("word", "pos"):
+            continue  # (any number of rows)
+        assert not native.encoder_forward_ok(*_edited(name, f)), name
+    if name in ("wo", "wi", "wo2"):
+        assert not native.encoder_forward_ok(*_edited(name, lambda t: t.t()))
+
+
+def test_no_token_type_row_is_taken():
+    from rag_llm_k8s_amd.ops import native
+
+    cfg, w = _edited("type_row", lambda t: None)
+    assert native.encoder_pointers(cfg, w)[4] is None and len(native.encoder_pointers(cfg, w)) == 5 + 12 * 2
+    cfg, w = _edited("type_row", lambda t: t[None])
+    assert native.encoder_pointers(cfg, w)[4] == w.type_row.data_ptr()

@@ -56,3 +56,26 @@ def test_engine_order_and_odd_outputs(native):
     ids, lens = np.concatenate(lists).astype(np.int32), np.array([len(x) for x in lists], dtype=np.int32)
     eng.embed_flat(ids, lens, cols)
     assert torch.equal(cols, got)
+
+
+def test_edited_weights(native):
+    """Weights whose addresses alone would mislead the native call: rows with gaps give what they give without, a transposed
+    matrix is refused as the layered path refuses it, one on the host is not taken; no token type row is."""
+    ids, lens, row = np.arange(5, 105, dtype=np.int32), np.array([100], dtype=np.int64), np.array([0])
+    ref, out = torch.zeros(1, 256, device=DEV), torch.zeros(1, 256, device=DEV)
+    m = model("mean")
+    m.embed_into(ids, lens, ref, row)
+    m.w.layers[1]["wi"] = torch.cat([m.w.layers[1]["wi"]] * 2, 1)[:, :256]
+    assert not native.encoder_forward_ok(m.cfg, m.w)
+    m.embed_into(ids, lens, out, row)
+    assert torch.equal(out, ref)
+    m.w.layers[0]["wo"] = m.w.layers[0]["wo"].t()
+    with pytest.raises(ValueError):
+        m.embed_into(ids, lens, out, row)
+    m = model("mean")
+    m.w.type_row = None
+    m.embed_into(ids, lens, out, row)
+    assert native.encoder_forward_ok(m.cfg, m.w) and not torch.equal(out, ref)
+    assert torch.equal(out, m.forward_packed(torch.from_numpy(ids).to(DEV), [100]))
+    m.w.layers[0]["ln1_g"] = m.w.layers[0]["ln1_g"].cpu()
+    assert not native.encoder_forward_ok(m.cfg, m.w)

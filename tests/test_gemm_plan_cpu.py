@@ -36,3 +36,13 @@ def test_short_inner_dimension_stays_off_the_long_ring():
         for T in (65, 300, 4096, 24576, 49152, 65536):
             for N, K in ((3 * H, H), (H, H), (I, H), (H, I)):
                 assert all(mi in n.MID_US for _, _, mi, _ in n.gemm_plan(T, N, K, True, 256)) or K >= 192
+
+
+def test_work_lists_of_prompts():
+    """Every tile of every sequence once, later positions first, sequences in order among equals: short lists and long ones."""
+    r = random.Random(2)
+    for Hq, Hkv in ((32, 8), (12, 12), (16, 8)):
+        qt = n.prefill_qtile(Hq, Hkv)
+        for lens in ([], [0], [1], [qt], [qt + 1, 0, qt], [64 * qt], [64 * qt + 1], [4096, 5, 70], [r.randint(1, 900) for _ in range(9)]):
+            want = sorted(((s, q) for s, L in enumerate(lens) for q in range(0, L, qt)), key=lambda t: -t[1])
+            assert n.build_prefill_tiles(lens, Hq, Hkv).tolist() == [list(t) for t in want]

@@ -173,6 +173,7 @@ def lib():
                 "or __graft_entry__.build()." % LIB_PATH)
         h = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
         _check_stamp(h, only)
+        _check_mirrors(h)
         for name, args in _SIGS.items():
             if only is not None and not hasattr(h, name):
                 setattr(h, name, _absent(name))
@@ -182,6 +183,14 @@ def lib():
             fn.restype = _RESTYPES.get(name, ctypes.c_int)
         _lib = h
         return h
+
+
+def _check_mirrors(h):
+    """The structs that cross as pointers have the size that the library was compiled with (a partial one may lack them)."""
+    for mirror, size in ((EncoderCall, "ragk_encoder_call_bytes"),):
+        if hasattr(h, size) and getattr(h, size)() != ctypes.sizeof(mirror):
+            raise NativeLibraryError("%s is %d bytes here and %d in the library: rebuild it (python -m rag_llm_k8s_amd._build)"
+                                     % (mirror.__name__, ctypes.sizeof(mirror), getattr(h, size)()))
 
 
 def _absent(name):

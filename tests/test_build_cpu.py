@@ -50,3 +50,18 @@ def test_runtime_stamp_matches_tree_and_stale_is_refused(monkeypatch):
         runtime.check_rt_stamp(mod)
     monkeypatch.setenv("RAGK_ALLOW_STALE_LIB", "1")
     runtime.check_rt_stamp(mod)
+
+
+@pytest.mark.skipif(not _lib.available(), reason="kernel library not built")
+def test_struct_mirrors_have_the_library_s_size(monkeypatch):
+    """A struct passed by pointer that differs from the library's is refused when it is loaded."""
+    monkeypatch.setattr(_lib, "_lib", None)
+    assert ctypes.sizeof(_lib.EncoderCall) == _lib.lib().ragk_encoder_call_bytes()
+
+    class Longer(ctypes.Structure):
+        _fields_ = _lib.EncoderCall._fields_ + [("more", ctypes.c_void_p)]
+
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "EncoderCall", Longer)
+    with pytest.raises(_lib.NativeLibraryError, match="bytes here"):
+        _lib.lib()

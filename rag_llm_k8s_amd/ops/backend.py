@@ -15,6 +15,7 @@ import math
 from dataclasses import dataclass, field
 from typing import List, Optional
 
+import numpy as np
 import torch
 
 from . import reference as R
@@ -577,7 +578,7 @@ class NativeBackend(TorchBackend):
 
     def encoder_forward(self, cfg, w, ids, lens, first_pos, out, rows):
         T = int(lens.sum())
-        if (out.dtype != torch.float32 or out.stride(1) != 1 or out.device != w.word.device or T == 0
+        if (ids.dtype != np.int32 or out.dtype != torch.float32 or out.stride(1) != 1 or out.device != w.word.device or T == 0
                 or T * max(3 * cfg.hidden_size, cfg.intermediate_size) * 2 >= 2 ** 31):
             return False
         weights = self.n.encoder_pointers(cfg, w)

@@ -58,6 +58,14 @@ def test_engine_order_and_odd_outputs(native):
     assert torch.equal(cols, got)
 
 
+def test_ids_of_another_type_are_refused(native):
+    m = model("mean")
+    out = torch.zeros(2, 256, device=DEV)
+    with pytest.raises(ValueError):
+        EmbeddingEngine(m, None).embed_flat(np.arange(20, dtype=np.int64), np.array([15, 5], dtype=np.int32), out)
+    assert not out.any()
+
+
 def test_edited_weights(native):
     """Weights whose addresses alone would mislead the native call: rows with gaps give what they give without, a transposed
     matrix is refused as the layered path refuses it, one on the host is not taken; no token type row is."""

@@ -365,6 +365,11 @@ __global__ __launch_bounds__(256) void splitk_rope_kernel(const float* __restric
   mid_rope8(x1, x2, rk, C, ldc, row, hd, d);
 }
 
+// An operand's rows as the DMA takes them: 16-byte pieces, a tile's (at most 256) rows within 32-bit offsets.
+bool mid_rows_ok(const void* p, int ld, int K) {
+  return (uintptr_t)p % 16 == 0 && ld % 8 == 0 && 256LL * ld * 2 + 2LL * K < (1LL << 31);
+}
+
 int mid_grid(int total) {
   static int cus = 0;
   if (!cus) {
@@ -420,7 +425,7 @@ int launch_finish(const float* P, int S, void* C, int ldc, const void* bias, con
   X(EPI_SILU_MUL) X(EPI_GLU_CLIP)
 
 // N = output columns (for the pair epilogues the weight has 2 N rows in the packed [64 gate | 64 up] layout, N % 64 == 0).
-// mi = rows of a tile / 32. S > 1: K-split through the fp32 slabs ws [S][M][weight rows], summed with the epilogue by a
+// Rows of A and B start on 16 bytes. mi = rows of a tile / 32. S > 1: K-split through the fp32 slabs ws [S][M][weight rows], summed with the epilogue by a
 // second launch. S slabs without a consumer here: epi NONE, out_f32 = 2 (C holds the slabs).
 RAGK_API int ragk_gemm_mid(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias,
                            const void* resid, int ldr, int M, int N, int K, int epi, int out_f32, int mi, int S, float* ws,
@@ -430,7 +435,7 @@ RAGK_API int ragk_gemm_mid(const void* A, int lda, const void* B, int ldb, void*
   if (K % MID_BK || S < 1 || S > nk || N % 8) return (int)hipErrorInvalidValue;
   if (epi_pair(epi) && (N % 64 || out_f32)) return (int)hipErrorInvalidValue;
   if (epi == EPI_GLU_CLIP && !bias) return (int)hipErrorInvalidValue;
-  if (256LL * lda * 2 + 2LL * K >= (1LL << 31) || 128LL * ldb * 2 + 2LL * K >= (1LL << 31)) return (int)hipErrorInvalidValue;
+  if (!mid_rows_ok(A, lda, K) || !mid_rows_ok(B, ldb, K)) return (int)hipErrorInvalidValue;
   const int rows = epi_pair(epi) ? 2 * N : N;
   if (out_f32 == 2) {
     if (epi != EPI_NONE || ldc != N) return (int)hipErrorInvalidValue;
@@ -467,7 +472,7 @@ RAGK_API int ragk_gemm_mid_rope_kv(const void* A, int lda, const void* B, int ld
   if (K % MID_BK || K <= 0 || S < 1 || S > K / MID_BK || Hq < 1 || Hkv < 1 || BS < 1 || ldc % 8 || (S > 1 && !ws))
     return (int)hipErrorInvalidValue;
   if (!pos || !slot || !cos_t || !sin_t || !kc || !vc) return (int)hipErrorInvalidValue;
-  if (256LL * lda * 2 + 2LL * K >= (1LL << 31) || 128LL * ldb * 2 + 2LL * K >= (1LL << 31)) return (int)hipErrorInvalidValue;
+  if (!mid_rows_ok(A, lda, K) || !mid_rows_ok(B, ldb, K)) return (int)hipErrorInvalidValue;
   const RopeKV rk{pos, slot, cos_t, sin_t, (bf16_t*)kc, (bf16_t*)vc, Hq, Hkv, BS};
   if (S == 1)
     return dispatch_mid<EPI_ROPE_KV>(mi, A, lda, B, ldb, C, ldc, nullptr, nullptr, 0, M, N, K, 1, 0, st, rk);

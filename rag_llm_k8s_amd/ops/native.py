@@ -156,6 +156,7 @@ def gemm_rope_kv(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, Hkv
         out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     _req(out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "gemm_rope_kv out")
     L = _lib.lib()
+    x, w = _tile_rows(x), _tile_rows(w)
     for r0, r1, mi, S in gemm_plan(M, N, K, True, _cu_count()):
         a = (x.data_ptr() + r0 * x.stride(0) * 2, x.stride(0), w.data_ptr(), w.stride(0),
              out.data_ptr() + r0 * out.stride(0) * 2, out.stride(0), r1 - r0, K, positions.data_ptr() + 4 * r0,
@@ -214,11 +215,7 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
         return _gemm_blas(x, w, resid, out, epi)
     if path is None and M > 64:
         rows = w.shape[0]
-        # gemm_mid addresses a tile's rows with 32-bit offsets: rows megabytes apart are brought together first
-        if x.stride(0) * 512 + 2 * K >= 2 ** 31:
-            x = x.contiguous()
-        if w.stride(0) * 256 + 2 * K >= 2 ** 31:
-            w = w.contiguous()
+        x, w = _tile_rows(x), _tile_rows(w)
         # gemm_w4 addresses operands with 32-bit buffer offsets
         fits = x.stride(0) * M * 2 < 2 ** 31 and w.stride(0) * rows * 2 < 2 ** 31
         if not fits and use_pp(M, N, K, epi):
@@ -282,10 +279,20 @@ def gemm_mid(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, m
     a workspace, summed with the epilogue by a second launch)."""
     M, K = x.shape
     N = w.shape[0] // 2 if epi in PAIR_EPI else w.shape[0]
+    x, w = _tile_rows(x), _tile_rows(w)
     _req(mi in MID_US and 1 <= S <= K // 64 and K % 64 == 0 and w.shape[1] == K, "gemm_mid tile or split")
     _req(out.shape == (M, N) and out.stride(1) == 1, "gemm_mid out")
     _gemm_rows(x, w, bias, resid, epi, out, out_f32, 0, M, mi, S)
     return out
+
+
+def _tile_rows(t):
+    """t, or a copy of rows that gemm_mid and gemm_w4 cannot fetch where they lie: their LDS-DMA pieces start on 16 bytes, and a
+    tile's 256 rows are reached by 32-bit offsets."""
+    ld = t.stride(0)
+    if ld % 8 == 0 and t.data_ptr() % 16 == 0 and ld * 514 < 2 ** 31:
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
 
 
 def _gemm_rows(x, w, bias, resid, epi, out, out_f32, r0, r1, mi, S):
@@ -584,6 +591,7 @@ def gemm_splitk(x, w, nsplit, out=None):
     _req(out.dtype == torch.float32 and out.is_contiguous() and out.numel() >= nsplit * M * N, "gemm_splitk out")
     if M == 0:
         return out
+    x, w = _tile_rows(x), _tile_rows(w)
     mi, w4 = _splitk_tile(M, N, K, nsplit, _cu_count())
     if w4 and x.stride(0) * M * 2 < 2 ** 31 and w.stride(0) * N * 2 < 2 ** 31:
         check(_lib.lib().ragk_gemm_w4_splitk(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), M, N, K,
@@ -890,7 +898,7 @@ def use_hold(M, N, K, epi, fp8=False):
 
 
 def _vec_rows(*ts):
-    """Whether every row starts on 16 bytes (odd strides and offsets stay with the kernels that took them before)."""
+    """Whether every row starts on 16 bytes."""
     return all((t.stride(0) * t.element_size()) % 16 == 0 and t.data_ptr() % 16 == 0 for t in ts)
 
 
@@ -1198,6 +1206,7 @@ def gemm_layernorm(x, w, bias, resid, g, b, eps):
     S, mi = ln_slabs(M, N, K)
     if S == 1:
         return layernorm(gemm(x, w, bias=bias, resid=resid, epi="bias_resid"), g, b, eps)
+    x, w = _tile_rows(x), _tile_rows(w)
     if mi < 0:
         return layernorm_slabs(gemm_part(x, w, out=torch.empty((S, M, N), dtype=torch.float32, device=x.device), ks=K // 64 // S),
                                bias, resid, g, b, eps)

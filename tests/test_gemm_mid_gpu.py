@@ -96,3 +96,55 @@ def test_gemm_routes_agree(native, M, N, K):
     S = native.slab_count(M, N, K)
     if S > 1:
         assert rel_err(native.gemm_splitk(x, w, S).sum(0), x.float() @ w.float().t()) < 1e-5
+
+
+@pytest.mark.parametrize("M", [65, 70, 300, 1100])
+def test_operands_between_vectors(native, M):
+    """x and w with rows off 16 bytes or from a start between vectors, or megabytes apart: what their copies give, bit for bit,
+    through every entry that fetches them in 16-byte pieces. Bias, residual and output lie anywhere."""
+    g = torch.Generator(device=DEV).manual_seed(M)
+
+    def odd(rows, cols, how):
+        t = torch.randn(rows, cols + 16, device=DEV, generator=g).bfloat16()
+        flat = torch.randn(rows * cols + 8, device=DEV, generator=g).bfloat16()
+        return {"stride": torch.randn(rows, cols + 5, device=DEV, generator=g).bfloat16()[:, :cols], "start": t[:, 3:cols + 3],
+                "flat": flat[1:rows * cols + 1].view(rows, cols)}[how]
+
+    N, K = 1024, 1024
+    for how in ("stride", "start", "flat"):
+        x, w, wgu = odd(M, K, how), odd(N, K, how), odd(2 * N, K, how)
+        cx, cw, cgu = (t.clone(memory_format=torch.contiguous_format) for t in (x, w, wgu))
+        b, r = odd(1, N, how)[0], odd(M, N, how)
+        out = odd(M, N, how)
+        native.gemm(x, w, bias=b, resid=r, epi="bias_resid", out=out)
+        assert torch.equal(out, native.gemm(cx, cw, bias=b.clone(), resid=r.contiguous(), epi="bias_resid"))
+        assert torch.equal(native.gemm(x, wgu, epi="silu_mul"), native.gemm(cx, cgu, epi="silu_mul"))
+        assert torch.equal(native.gemm(x, w, path=0), native.gemm(cx, cw, path=0))
+        assert torch.equal(native.gemm_splitk(x, w, 2), native.gemm_splitk(cx, cw, 2))
+        gain, shift = torch.randn(2, N, device=DEV, generator=g).bfloat16()
+        assert torch.equal(native.gemm_layernorm(x, w, b.clone(), cx, gain, shift, 1e-5),
+                           native.gemm_layernorm(cx, cw, b.clone(), cx, gain, shift, 1e-5))
+        few = odd(60, K, how)
+        assert torch.equal(native.gemm_layernorm(few, w, b.clone(), cx[:60], gain, shift, 1e-5),
+                           native.gemm_layernorm(few.clone(memory_format=torch.contiguous_format), cw, b.clone(), cx[:60], gain, shift, 1e-5))
+        cos, sin = (t.to(DEV) for t in R.rope_tables(128, M))
+        pos = torch.arange(M, device=DEV).int()
+        kc = torch.zeros(2, M // 64 + 1, 2, 64, 128, device=DEV).bfloat16()
+        vc = torch.zeros_like(kc)
+        a, c = (native.gemm_rope_kv(p, q, pos, cos, sin, pos, kc[i], vc[i], 4, 2, 128) for i, (p, q) in enumerate(((x, w), (cx, cw))))
+        assert torch.equal(a, c) and torch.equal(kc[0], kc[1]) and torch.equal(vc[0], vc[1])
+    if M <= 70:
+        far = torch.empty_strided((M, K), (2 ** 22, 1), dtype=torch.bfloat16, device=DEV)
+        far.copy_(cx)
+        assert torch.equal(native.gemm_splitk(far, cw, 2), native.gemm_splitk(cx, cw, 2))
+
+
+def test_library_refuses_rows_between_vectors(native):
+    """The C entry itself: nothing is launched."""
+    t = torch.zeros(128 * 136, dtype=torch.bfloat16, device=DEV)
+    out, L = torch.zeros(80, 128, dtype=torch.bfloat16, device=DEV), native._lib.lib()
+    for a, lda, b, ldb in ((0, 129, 0, 128), (2, 128, 0, 128), (0, 128, 0, 132), (0, 128, 4, 128)):
+        assert L.ragk_gemm_mid(t.data_ptr() + a, lda, t.data_ptr() + b, ldb, out.data_ptr(), 128, None, None, 0, 80, 128, 128, 0, 0,
+                               4, 1, None, 0) != 0
+    torch.cuda.synchronize()
+    assert not out.any()

@@ -1,6 +1,8 @@
 """The launch rule of products with more than 64 rows: every row once, splits that the kernels take."""
 import random
 
+import torch
+
 from rag_llm_k8s_amd.ops import native as n
 
 
@@ -46,3 +48,16 @@ def test_work_lists_of_prompts():
         for lens in ([], [0], [1], [qt], [qt + 1, 0, qt], [64 * qt], [64 * qt + 1], [4096, 5, 70], [r.randint(1, 900) for _ in range(9)]):
             want = sorted(((s, q) for s, L in enumerate(lens) for q in range(0, L, qt)), key=lambda t: -t[1])
             assert n.build_prefill_tiles(lens, Hq, Hkv).tolist() == [list(t) for t in want]
+
+
+def test_operand_rows_that_are_copied():
+    """Rows off 16 bytes or megabytes apart, whole tensors that start between vectors; nothing else."""
+    a = torch.arange(80 * 264, dtype=torch.float32).bfloat16().view(80, 264)
+    far = torch.empty_strided((3, 256), (2 ** 22, 1), dtype=torch.bfloat16)
+    far.copy_(a[:3, :256])
+    for t, copied in ((a, False), (a[:, :256], False), (a[:, 8:], False), (a[::2], False), (a[:, 4:260], True), (a[:, :132][1:], False),
+                      (a.view(-1)[:79 * 263].view(79, 263)[:, :256], True), (a.view(-1)[1:1 + 70 * 256].view(70, 256), True),
+                      (far, True), (far[:, :8], True)):
+        got = n._tile_rows(t)
+        assert (got.data_ptr() != t.data_ptr()) == copied and torch.equal(got, t)
+        assert not copied or (got.is_contiguous() and got.data_ptr() % 16 == 0)

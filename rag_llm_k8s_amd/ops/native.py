@@ -178,13 +178,11 @@ def _gemm_blas(x, w, resid, out, epi):
     return torch.mm(x, w.t(), out=out)
 
 
-def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=None):
-    """out[M,N] = epi(x[M,K] @ w[N,K]^T). For epi='silu_mul', w is the packed
-    gate/up weight [2N, K] (see reference.pack_gate_up) and out has N columns."""
+def _gemm_operands(x, w, bias, resid, epi):
+    """(M, N, K) of a product whose operands are fit for any of its kernels."""
     _bf16_2d(x, "x")
     _bf16_2d(w, "w")
     M, K = x.shape
-    e = EPI[epi]
     N = w.shape[0] // 2 if epi in PAIR_EPI else w.shape[0]
     _req(w.shape[1] == K, "K mismatch %s vs %s" % (tuple(x.shape), tuple(w.shape)))
     _req(K % 128 == 0, "K must be a multiple of 128 (got %d)" % K)
@@ -199,6 +197,14 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
     if "resid" in epi:
         _bf16_2d(resid, "resid")
         _req(resid.shape == (M, N), "resid shape")
+    return M, N, K
+
+
+def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=None):
+    """out[M,N] = epi(x[M,K] @ w[N,K]^T). For epi='silu_mul', w is the packed
+    gate/up weight [2N, K] (see reference.pack_gate_up) and out has N columns."""
+    M, N, K = _gemm_operands(x, w, bias, resid, epi)
+    e = EPI[epi]
     odt = torch.float32 if out_f32 else torch.bfloat16
     if out is None:
         out = torch.empty((M, N), dtype=odt, device=x.device)
@@ -1201,8 +1207,7 @@ def ln_slabs(M, N, K):
 
 def gemm_layernorm(x, w, bias, resid, g, b, eps):
     """LN(x @ w^T + bias + resid) * g + b, the sum kept in fp32 where the product is split (ln_slabs)."""
-    M, K = x.shape
-    N = w.shape[0]
+    M, N, K = _gemm_operands(x, w, bias, resid, "bias_resid")
     S, mi = ln_slabs(M, N, K)
     if S == 1:
         return layernorm(gemm(x, w, bias=bias, resid=resid, epi="bias_resid"), g, b, eps)

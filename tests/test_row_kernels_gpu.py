@@ -54,3 +54,17 @@ def test_gemm_layernorm(native, N, K):
         ref = R.layernorm(x.double() @ w.double().t() + bias.double() + r.double(), g.double(), b.double(), 1e-12)
         # roundings to bf16, at most 2^-8 of a value each: the result and, unsplit, the sum that is normalised
         assert (native.gemm_layernorm(x, w, bias, r, g, b, 1e-12).double() - ref).norm() / ref.norm() < 2.0 ** -7
+
+
+@pytest.mark.parametrize("T", [60, 300])
+def test_gemm_layernorm_refuses_what_gemm_does(native, T):
+    """At sizes whose product is split, as at the others."""
+    x, w = torch.zeros(T, 1024, device=DEV).bfloat16(), torch.zeros(1024, 1024, device=DEV).bfloat16()
+    v, r = torch.zeros(1024, device=DEV).bfloat16(), torch.zeros(T, 1024, device=DEV).bfloat16()
+    assert native.ln_slabs(T, 1024, 1024)[0] > 1
+    native.gemm_layernorm(x, w, v, r, v, v, 1e-5)
+    for bad in ((x[:, :896], w, v, r), (x, w[:, :896], v, r), (x.float(), w, v, r), (x, w.half(), v, r), (x, w.t(), v, r),
+                (x[:, :960], w[:, :960], v, r), (x, w, v.float(), r), (x, w, v[:512], r), (x, w, None, r), (x, w, v, r[:5]),
+                (x, w, v, r.float()), (x, w.cpu(), v, r)):
+        with pytest.raises(ValueError):
+            native.gemm_layernorm(*bad, v, v, 1e-5)

@@ -374,20 +374,17 @@ def gemm_plan(M, rows, K, w4, cus):
 
 
 PART_MIN_BLOCKS = 512
-_part_cfg = [False]
 
 
 @functools.lru_cache(maxsize=4096)
-def _part_ksteps(M, N, K):
-    if not _part_cfg[0]:
-        check(_lib.lib().ragk_gemm_part_set_min_blocks(PART_MIN_BLOCKS), "ragk_gemm_part_set_min_blocks")
-        _part_cfg[0] = True
+def _part_ksteps(M, N, K, min_blocks):
+    check(_lib.lib().ragk_gemm_part_set_min_blocks(min_blocks), "ragk_gemm_part_set_min_blocks")
     return _lib.lib().ragk_gemm_part_ksteps(M, N, K)
 
 
 def gemm_part_slabs(M, N, K, ks=None):
     """(ks_steps, S) of the split-K partial GEMM for this shape (0, 0 if unsupported)."""
-    ks = ks or _part_ksteps(M, N, K)
+    ks = ks or _part_ksteps(M, N, K, PART_MIN_BLOCKS)
     if ks <= 0 or K % (64 * ks):
         return 0, 0
     return ks, K // (64 * ks)
@@ -539,7 +536,10 @@ def prefill_nsplit(M, N, K):
     (66 %) -> 2 slabs = 2.6 waves (88 %). The 32k-token bench steps (2048 tiles) never split."""
     if not PREFILL_SPLITK or M < PREFILL_SPLITK_MIN_M:
         return 1
-    cus = _cu_count()
+    return _w4_nsplit(M, N, K, _cu_count())
+
+
+def _w4_nsplit(M, N, K, cus):
     tiles = -(-M // 256) * -(-N // 256)
     best, best_s = 0.0, 1
     for s in (1, 2):
@@ -553,7 +553,7 @@ def prefill_nsplit(M, N, K):
 
 
 @functools.lru_cache(maxsize=4096)
-def _slab_best(M, N, K, cus):
+def _slab_best(M, N, K, cus, w4_min_m=PREFILL_SPLITK_MIN_M):
     """(S, mi) of the cheapest split whose slabs a row norm sums, (1, 0) if the whole product + a plain norm is cheaper.
     Per output value the slabs cost 8 B each through memory, the whole product 6 (bf16 write, residual, norm's read).
     o_proj / down at 300 rows: 28 / 88 us whole, 17 / 42 us as 2 / 4 slabs; at 14076 rows the slabs' traffic (212 us in the
@@ -562,7 +562,7 @@ def _slab_best(M, N, K, cus):
     for r0, r1, mi, S in gemm_plan(M, N, K, True, cus):
         whole += _tiles_us(r1 - r0, N, K, mi, S, cus) + (3.0 + SLAB_US * S * (r1 - r0) * N if S > 1 else 0)
     best, S, mi = min((t - 0.75 * SLAB_US * M * N, S, mi) for t, mi, S in [_mid_best(M, N, K, cus, SLAB_US, 0.0, even=True)])
-    w4 = prefill_nsplit(M, N, K)
+    w4 = _w4_nsplit(M, N, K, cus) if M >= w4_min_m else 1
     if w4 > 1:
         t = _tiles_us(M, N, K, 0, w4, cus) + SLAB_US * (w4 - 0.75) * M * N
         if t < best:
@@ -574,7 +574,7 @@ def slab_count(M, N, K):
     """K-slabs for a prefill projection in front of a row norm (1: the whole product)."""
     if not PREFILL_SPLITK or M <= 64 or K % 128 or N % 8:
         return 1
-    return _slab_best(M, N, K, _cu_count())[0]
+    return _slab_best(M, N, K, _cu_count(), PREFILL_SPLITK_MIN_M)[0]
 
 
 @functools.lru_cache(maxsize=4096)
@@ -1201,7 +1201,9 @@ def ln_slabs(M, N, K):
     if M <= 64:
         ks = 4 if K <= 3072 else 8  # K-steps of a slab: at most twelve slabs of the shorter ones
         return (K // (64 * ks), -1) if K >= 1024 and K % (64 * ks) == 0 and M * K >= 18432 else (1, 0)
-    S, mi = _slab_best(M, N, K, _cu_count())
+    if not PREFILL_SPLITK:
+        return 1, 0
+    S, mi = _slab_best(M, N, K, _cu_count(), PREFILL_SPLITK_MIN_M)
     return (S, mi) if S > 1 and mi else (1, 0)
 
 

@@ -1,8 +1,10 @@
 """The launch rule of products with more than 64 rows: every row once, splits that the kernels take."""
 import random
 
+import pytest
 import torch
 
+from rag_llm_k8s_amd.ops import _lib
 from rag_llm_k8s_amd.ops import native as n
 
 
@@ -61,3 +63,31 @@ def test_operand_rows_that_are_copied():
         got = n._tile_rows(t)
         assert (got.data_ptr() != t.data_ptr()) == copied and torch.equal(got, t)
         assert not copied or (got.is_contiguous() and got.data_ptr() % 16 == 0)
+
+
+def test_plans_follow_their_settings(monkeypatch):
+    """What was worked out under one setting is not kept for another: splits off and on, their least rows, a launch's blocks."""
+    monkeypatch.setattr(n, "_cu_count", lambda: 256)
+    sizes = [(300, 4096, 4096), (700, 1024, 4096), (5000, 4096, 4096)]
+    on = [(n.slab_count(*s), n.ln_slabs(*s), n.prefill_nsplit(*s)) for s in sizes]
+    assert all(a[0] > 1 for a in on[:2]) and all(a[1][0] > 1 for a in on[:2]) and on[2][2] > 1
+    for f in (n._slab_best, n._splitk_tile, n.gemm_plan):
+        f.cache_clear()
+    monkeypatch.setattr(n, "PREFILL_SPLITK", False)
+    assert all((n.slab_count(*s), n.ln_slabs(*s), n.prefill_nsplit(*s)) == (1, (1, 0), 1) for s in sizes)
+    monkeypatch.setattr(n, "PREFILL_SPLITK", True)
+    assert on == [(n.slab_count(*s), n.ln_slabs(*s), n.prefill_nsplit(*s)) for s in sizes]
+    monkeypatch.setattr(n, "PREFILL_SPLITK_MIN_M", 10 ** 6)
+    assert all(n.prefill_nsplit(*s) == 1 for s in sizes)
+    assert n.slab_count(1700, 4096, 14336) == 1
+    monkeypatch.setattr(n, "PREFILL_SPLITK_MIN_M", 1024)
+    assert n.slab_count(1700, 4096, 14336) == 2
+
+
+@pytest.mark.skipif(not _lib.available(), reason="kernel library not built")
+def test_slices_follow_the_block_count(monkeypatch):
+    a = n.gemm_part_slabs(1, 4096, 4096)
+    monkeypatch.setattr(n, "PART_MIN_BLOCKS", 64)
+    b = n.gemm_part_slabs(1, 4096, 4096)
+    monkeypatch.setattr(n, "PART_MIN_BLOCKS", 512)
+    assert a != b and n.gemm_part_slabs(1, 4096, 4096) == a

@@ -799,20 +799,20 @@ static size_t mfma_lds(int d, int QT) { return (size_t)mq_floats(d, QT) * 4; }
 // rows of a wave's tile / 16: tiles for every wave of the chip before wider loads
 static int mfma_rt(int n) { return n >= 196608 ? 4 : (n >= 65536 ? 2 : 1); }
 
-// Number of partial lists per query the scan of rows [row_begin, row_end) emits (size the
-// partial buffers [nq][G][k] with it).
-RAGK_API int ragk_l2_scan_groups(int row_begin, int row_end, int nq) {
+// Partial lists per query that l2_scan emits over rows [row_begin, row_end).
+static int scan_groups(int row_begin, int row_end, int nq) {
   const int n = max(0, row_end - row_begin);
   const int S = scan_slices(n);
-  const int ntiles = (n + 64 * (4 / S) - 1) / (64 * (4 / S));  // (the MFMA path's 256-row tiles: <= this)
+  const int ntiles = (n + 64 * (4 / S) - 1) / (64 * (4 / S));
   const int qgroups = (max(nq, 1) + 15) / 16;
   const int target = max(1, 2048 / qgroups);  // bounded list count: the merge stays short
   return max(1, min(ntiles, target));
 }
 
-// As ragk_l2_scan_groups, for the kernel ragk_l2_search actually launches for (nq, k, d).
+// Partial lists per query that ragk_l2_search emits, by the kernel that it launches for (nq, k, d): size its partial buffers
+// [nq][G][k] with it.
 RAGK_API int ragk_l2_search_groups(int row_begin, int row_end, int nq, int k, int d) {
-  if (!use_mfma(nq, k, d)) return ragk_l2_scan_groups(row_begin, row_end, nq);
+  if (!use_mfma(nq, k, d)) return scan_groups(row_begin, row_end, nq);
   const int n = max(0, row_end - row_begin);
   // a block a CU over all query groups, but eight (one an XCD, which then serves its rows to every group from its L2): 1000
   // queries of 10000 x 1024, 256 blocks a group, each staging its q^T for one tile a wave, 1068 us, so 265
@@ -821,7 +821,7 @@ RAGK_API int ragk_l2_search_groups(int row_begin, int row_end, int nq, int k, in
 }
 
 // Exact top-k (k <= 64) over rows [row_begin, row_end) of xt[d][cap]; part_d / part_i hold
-// nq * ragk_l2_scan_groups(...) * k entries; results -> out_d / out_i [nq][k].
+// nq * ragk_l2_search_groups(row_begin, row_end, nq, k, d) * k entries; results -> out_d / out_i [nq][k].
 RAGK_API int ragk_l2_search(const float* xt, int cap, int d, int row_begin, int row_end, const float* q, int nq,
                             int k, const int* ids_map, float* part_d, int* part_i, float* out_d,
                             long long* out_i, hipStream_t st) {

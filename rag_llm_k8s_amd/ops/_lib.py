@@ -82,7 +82,6 @@ _SIGS = {
     "ragk_topk_candidates": [P, I, I, I, I, I, I, P, P, S],
     "ragk_sample_candidates": [P, P, I, I, P, P, P, P, P, P, P, S],
     "ragk_sample_candidates_lists": [P, P, I, I, I, P, P, P, P, P, P, P, S],
-    "ragk_l2_scan_groups": [I, I, I],
     "ragk_l2_search_groups": [I, I, I, I, I],
     "ragk_l2_search_set_mfma_min_nq": [I],
     "ragk_l2_search": [P, I, I, I, I, P, I, I, P, P, P, P, P, S],

@@ -65,3 +65,12 @@ def test_struct_mirrors_have_the_library_s_size(monkeypatch):
     monkeypatch.setattr(_lib, "EncoderCall", Longer)
     with pytest.raises(_lib.NativeLibraryError, match="bytes here"):
         _lib.lib()
+
+
+@pytest.mark.skipif(not _lib.available(), reason="kernel library not built")
+def test_search_partials_have_one_count():
+    """The lists of a search are those of the kernel it launches: batched queries emit more than the scan would."""
+    h = _lib.lib()
+    assert not hasattr(h, "ragk_l2_scan_groups")
+    scan, batched = (h.ragk_l2_search_groups(0, 10000, nq, 5, 384) for nq in (15, 16))
+    assert scan == -(-10000 // 64) and batched == 256

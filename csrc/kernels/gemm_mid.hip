@@ -85,19 +85,21 @@ __device__ __forceinline__ MidItem mid_item(int it, int total, int tiles_m, int 
   return w;
 }
 
-// values of eight consecutive outputs -> bias, residual, activation (the order and rounding of gemm_w4's epilogue)
+constexpr bool mid_has_bias(int e) { return e == EPI_BIAS || e == EPI_BIAS_RESID || e == EPI_BIAS_GELU || e == EPI_BIAS_GELU_TANH; }
+constexpr bool mid_has_resid(int e) { return e == EPI_RESID || e == EPI_BIAS_RESID; }
+
+// values of eight consecutive outputs + bias, residual (as loaded), activation (the order and rounding of gemm_w4's epilogue)
 template <int EPI>
-__device__ __forceinline__ void mid_finish8(float (&o)[8], const bf16_t* __restrict__ bias, const bf16_t* resid, size_t at,
-                                            int col) {
-  if constexpr (EPI == EPI_BIAS || EPI == EPI_BIAS_RESID || EPI == EPI_BIAS_GELU || EPI == EPI_BIAS_GELU_TANH) {
+__device__ __forceinline__ void mid_finish8(float (&o)[8], u32x4 bias, u32x4 resid) {
+  if constexpr (mid_has_bias(EPI)) {
     float b[8];
-    unpack8(*reinterpret_cast<const u32x4*>(bias + col), b);
+    unpack8(bias, b);
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] += b[e];
   }
-  if constexpr (EPI == EPI_RESID || EPI == EPI_BIAS_RESID) {
+  if constexpr (mid_has_resid(EPI)) {
     float r[8];
-    unpack8(*reinterpret_cast<const u32x4*>(resid + at), r);
+    unpack8(resid, r);
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] += r[e];
   }
@@ -303,6 +305,20 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
       }
     } else {
       void* Cz = out_f32 ? (void*)(reinterpret_cast<float*>(C) + (size_t)w.z * M * ldc) : C;
+      // The tile's bias and residual are requested together, ahead of any use: loaded where they are added, each of the 2 MI
+      // row pieces waited for memory once more (8192 x 3072 x 1024 on 256-row tiles, us: bias 65.4 -> 56.5, without an epilogue
+      // 55.1; GELU 78.2 -> 68.3; 13762 x 1024 x 4096, bias and residual, 160-row tiles 118.7 -> 116.8).
+      u32x4 bv[2] = {}, rv[MI][2] = {};
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int col = min(w.n0 + 64 * wc + 32 * p + 8 * fh, N - 8);
+        if constexpr (mid_has_bias(EPI)) bv[p] = *reinterpret_cast<const u32x4*>(bias + col);
+        if constexpr (mid_has_resid(EPI)) {
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+            rv[i][p] = *reinterpret_cast<const u32x4*>(resid + (size_t)min(w.m0 + wr * 16 * MI + 16 * i + fr, M - 1) * ldr + col);
+        }
+      }
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
         const int row = w.m0 + wr * 16 * MI + 16 * i + fr;
@@ -313,7 +329,7 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
             float o[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] = acc[i][2 * p + (e >> 2)][e & 3];
-            mid_finish8<EPI>(o, bias, resid, (size_t)row * ldr + col, col);
+            mid_finish8<EPI>(o, bv[p], rv[i][p]);
             mid_store8(Cz, (size_t)row * ldc + col, o, out_f32);
           }
         }
@@ -345,8 +361,11 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const float* __restr
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = glu_act<EPI>(g[e], u[e], gp);
   } else {
+    u32x4 bv = {}, rv = {};
+    if constexpr (mid_has_bias(EPI)) bv = *reinterpret_cast<const u32x4*>(bias + col);
+    if constexpr (mid_has_resid(EPI)) rv = *reinterpret_cast<const u32x4*>(resid + (size_t)row * ldr + col);
     sum_slabs8(P + (size_t)row * N + col, S, (size_t)M * N, o);
-    mid_finish8<EPI>(o, bias, resid, (size_t)row * ldr + col, col);
+    mid_finish8<EPI>(o, bv, rv);
   }
   mid_store8(C, (size_t)row * ldc + col, o, out_f32);
 }

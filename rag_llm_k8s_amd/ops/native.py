@@ -318,9 +318,15 @@ def _gemm_rows(x, w, bias, resid, epi, out, out_f32, r0, r1, mi, S):
 
 
 # Microseconds that one 64-deep K-tile of an output tile takes with few blocks running, and what a full machine adds
-# (clocks, L2): tiles of gemm_mid by rows / 32, 0 = gemm_w4's 256 x 256. Fitted to M = 90 .. 13762, N = 1024 .. 28672.
-MID_US = {3: (0.29, 0.13), 4: (0.34, 0.17), 5: (0.40, 0.25), 6: (0.48, 0.15), 8: (0.60, 0.23)}
-W4_US = (1.0, 0.36)
+# (clocks, L2): tiles of gemm_mid by rows / 32, 0 = gemm_w4's 256 x 256; then those of a launch and of a tile's epilogue. Fitted
+# to every tile and split of 20 weights (384 to 28672 rows, K 384 to 14336) at 65 .. 32768 rows of x on two cards, for the
+# choices that follow: they take 0.5 % more than the best launch in the mean, 4 % in one of twenty. (An earlier fit, with 0.25
+# added at 160 rows and one us for either epilogue, took the next tile up there: 1 and 8 %, and 12 % more than gemm_w4 alone at
+# 2600 x 4096 x 14336.)
+MID_US = {3: (0.27, 0.13), 4: (0.34, 0.15), 5: (0.40, 0.17), 6: (0.49, 0.17), 8: (0.62, 0.21)}
+W4_US = (1.01, 0.29)
+LAUNCH_US = (4.5, 1.75)
+W4_LAUNCH_US = (5.25, 4.25)
 SLAB_US = 8 / 5e6  # one fp32 slab value written and read back
 
 
@@ -330,7 +336,8 @@ def _tiles_us(M, rows, K, mi, S, cus):
     items = -(-M // bm) * -(-rows // bn) * S
     rounds = -(-items // cus)
     a, b = MID_US[mi] if mi else W4_US
-    return (4.5 if mi else 7.5) + rounds * (-(-(K // 64) // S) * (a + b * items / (rounds * cus)) + 1.0)
+    launch, epilogue = LAUNCH_US if mi else W4_LAUNCH_US
+    return launch + rounds * (-(-(K // 64) // S) * (a + b * items / (rounds * cus)) + epilogue)
 
 
 def _mid_best(M, rows, K, cus, slab_us, launch_us, even=False):

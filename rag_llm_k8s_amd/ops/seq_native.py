@@ -177,7 +177,9 @@ DECODE_MIN_PAGES = 4
 
 
 def decode_parts(spec, max_kv_len, batch):
-    """Partitions per (sequence, KV head): the pages a query can visit, spread to fill the chip."""
+    """Partitions per (sequence, KV head): the pages a query can visit, spread to fill the chip. Rounded up, unlike
+    native.decode_partitions: 17 rows of 3000 tokens, 8 KV heads, take 44.8 us in 544 blocks and 47.9 in 408, where a third of
+    the slots have nothing to hide this kernel's score work behind."""
     pages = -(-max_kv_len // 64)
     if spec.window > 0:
         pages = min(pages, -(-spec.keep_first // 64) + -(-spec.window // 64) + 1)

@@ -27,22 +27,23 @@ namespace {
 // out[b] = normalize(pool(hidden[cu[b]:cu[b+1]])) in fp32. mode 0 = CLS (first token),
 // mode 1 = masked mean over the sequence, mode 2 = last token. One block a sequence: a thread owns eight columns of every
 // RG-th row (a column a thread and a row at a time before: mean of 80 x 160 rows of 384 columns 45 -> 9.4 us, of 12 x 1146 of 1024
-// 1207 -> 25). VEC = 1 for widths
-// or row strides that are no multiple of eight.
-constexpr int POOL_NT = 1024, POOL_MAXH = 2048;
-template <int VEC>
-__global__ __launch_bounds__(POOL_NT) void pool_l2norm_kernel(const bf16_t* __restrict__ hidden, int ld,
+// 1207 -> 25). Modes 0 and 2 read one row: NT = 256 threads and one row group, not the mean's 1024 (300 sequences of 384
+// columns 5.4 -> 3.6 us).
+// VEC = 1 for widths or row strides that are no multiple of eight.
+constexpr int POOL_MAXH = 2048;
+template <int VEC, int NT>
+__global__ __launch_bounds__(NT) void pool_l2norm_kernel(const bf16_t* __restrict__ hidden, int ld,
                                                               const int* __restrict__ cu, const int* __restrict__ rows,
                                                               float* out, int ldo, int H, int mode, int normalize) {
-  __shared__ float part[POOL_NT * 8];
-  __shared__ float red[POOL_NT / 64];
+  __shared__ float part[NT == 256 ? 1 : NT * 8];
+  __shared__ float red[NT / 64];
   const int b = blockIdx.x;
   const int s0 = cu[b], s1 = cu[b + 1];
   const int len = s1 - s0;
   const int first = mode == 2 ? s1 - 1 : s0, last = mode == 1 ? s1 : first + 1;
   const int groups = (H + VEC - 1) / VEC;            // column groups of VEC
-  const int RG = groups < POOL_NT ? POOL_NT / groups : 1;  // row groups
-  constexpr int CG = VEC == 8 ? 1 : (POOL_MAXH + POOL_NT - 1) / POOL_NT;  // column groups of a thread
+  const int RG = NT > 256 && groups < NT ? NT / groups : 1;  // row groups
+  constexpr int CG = (POOL_MAXH / VEC + NT - 1) / NT;  // column groups of a thread
   const int rg = RG > 1 ? threadIdx.x / groups : 0, c0 = RG > 1 ? threadIdx.x % groups : threadIdx.x;
   float acc[CG][VEC];
 #pragma unroll
@@ -52,7 +53,7 @@ __global__ __launch_bounds__(POOL_NT) void pool_l2norm_kernel(const bf16_t* __re
   if (rg < RG) {
 #pragma unroll
     for (int k = 0; k < CG; ++k) {
-      const int c = c0 + k * POOL_NT;
+      const int c = c0 + k * NT;
       if (c >= groups) continue;
       const bf16_t* col = hidden + (size_t)c * VEC;
 #pragma unroll 4
@@ -97,7 +98,7 @@ __global__ __launch_bounds__(POOL_NT) void pool_l2norm_kernel(const bf16_t* __re
   float* o = out + (size_t)(rows ? rows[b] : b) * ldo;
 #pragma unroll
   for (int k = 0; k < CG; ++k) {
-    const int c = c0 + k * POOL_NT;
+    const int c = c0 + k * NT;
     if (c < groups)
 #pragma unroll
       for (int e = 0; e < VEC; ++e) o[c * VEC + e] = acc[k][e] * scale;
@@ -158,8 +159,10 @@ RAGK_API int ragk_pool_l2norm_rows(const void* hidden, int ld, const int* cu, co
                                    int mode, int normalize, hipStream_t st) {
   if (B <= 0) return 0;
   if (H > POOL_MAXH) return (int)hipErrorInvalidValue;
-  const auto kernel = H % 8 == 0 && ld % 8 == 0 && (uintptr_t)hidden % 16 == 0 ? pool_l2norm_kernel<8> : pool_l2norm_kernel<1>;
-  hipLaunchKernelGGL(kernel, dim3(B), dim3(POOL_NT), 0, st, (const bf16_t*)hidden, ld, cu, rows, out, ldo, H, mode, normalize);
+  const bool vec = H % 8 == 0 && ld % 8 == 0 && (uintptr_t)hidden % 16 == 0;
+  const auto kernel = mode == 1 ? (vec ? pool_l2norm_kernel<8, 1024> : pool_l2norm_kernel<1, 1024>)
+                                : (vec ? pool_l2norm_kernel<8, 256> : pool_l2norm_kernel<1, 256>);
+  hipLaunchKernelGGL(kernel, dim3(B), dim3(mode == 1 ? 1024 : 256), 0, st, (const bf16_t*)hidden, ld, cu, rows, out, ldo, H, mode, normalize);
   return (int)hipGetLastError();
 }
 

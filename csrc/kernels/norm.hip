@@ -258,6 +258,9 @@ hipError_t by_row(int H, F f) {
   if (H <= 512) f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
   else if (H <= 1024) f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
   else if (H <= 2048) f(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+  // two vectors a thread, since one of its four would load again what another has (14000 x 3072
+  // 38.4 -> 29.1 us, 2000 x 4096 10.0 -> 8.6)
+  else if (H <= 4096) f(integral_constant<int, 2>{}, integral_constant<int, 4>{});
   else f(integral_constant<int, 4>{}, integral_constant<int, 4>{});
   return hipGetLastError();
 }

@@ -796,8 +796,21 @@ static bool use_mfma(int nq, int k, int d) {
   return nq >= g_mfma_min_nq && k <= MQ_MK && d % 32 == 0 && d <= MQ_DMAX;
 }
 static size_t mfma_lds(int d, int QT) { return (size_t)mq_floats(d, QT) * 4; }
-// rows of a wave's tile / 16: tiles for every wave of the chip before wider loads
-static int mfma_rt(int n) { return n >= 196608 ? 4 : (n >= 65536 ? 2 : 1); }
+// A block a CU over all query groups, but eight (one an XCD, which then serves its rows to every group from its L2): 1000
+// queries of 10000 x 1024, 256 blocks a group, each staging its q^T for one tile a wave, 1068 us, so 265.
+static int mfma_blocks(int nq) { return max(8, 256 / (nq > 16 ? (nq + 31) / 32 : 1)); }
+// Rows of a wave's tile / 16. Wider tiles load more a lane and share their queries' reads; narrow ones spread few rows over the
+// waves. 16 / 256 queries of 1024 dims on tiles of 16, 32 and 64 rows, us: 10000 rows 34.9 / 90.6, 39.2 / 95.9, 48.9 / 97.4;
+// 20000 44.5 / 145, 39.7 / 136, 50.4 / 142; 60000 88.1 / 380, 57.2 / 335, 61.9 / 311; 140000 x 16 queries - / 128 / 139, where
+// 64-row tiles leave a second round nearly empty. A row costs a quarter more in the 32-row tile, so the rounds of both decide.
+// Over 1000 to 500000 rows, 384 and 1024 dims and 16 to 256 queries that takes 0.5 % more than the best tile in the mean, 10 %
+// at most.
+static int mfma_rt(int n, int nq) {
+  if (n < 16384) return 1;
+  const int waves = MQ_NW * mfma_blocks(nq);
+  const int r2 = ((n + 31) / 32 + waves - 1) / waves, r4 = ((n + 63) / 64 + waves - 1) / waves;
+  return r2 * 2 * 5 <= r4 * 4 * 4 ? 2 : 4;
+}
 
 // Partial lists per query that l2_scan emits over rows [row_begin, row_end).
 static int scan_groups(int row_begin, int row_end, int nq) {
@@ -814,10 +827,8 @@ static int scan_groups(int row_begin, int row_end, int nq) {
 RAGK_API int ragk_l2_search_groups(int row_begin, int row_end, int nq, int k, int d) {
   if (!use_mfma(nq, k, d)) return scan_groups(row_begin, row_end, nq);
   const int n = max(0, row_end - row_begin);
-  // a block a CU over all query groups, but eight (one an XCD, which then serves its rows to every group from its L2): 1000
-  // queries of 10000 x 1024, 256 blocks a group, each staging its q^T for one tile a wave, 1068 us, so 265
-  const int groups = nq > 16 ? (nq + 31) / 32 : 1;
-  return max(1, min((n + 16 * mfma_rt(n) - 1) / (16 * mfma_rt(n)), max(8, 256 / groups)));
+  const int rows = 16 * mfma_rt(n, nq);
+  return max(1, min((n + rows - 1) / rows, mfma_blocks(nq)));
 }
 
 // Exact top-k (k <= 64) over rows [row_begin, row_end) of xt[d][cap]; part_d / part_i hold
@@ -841,7 +852,7 @@ RAGK_API int ragk_l2_search(const float* xt, int cap, int d, int row_begin, int 
     }();
     if (attr != hipSuccess) return (int)attr;
     const int n = max(0, row_end - row_begin);
-    const int RT = mfma_rt(n);
+    const int RT = mfma_rt(n, nq);
     const int ntiles = (n + 16 * RT - 1) / (16 * RT);
     const int G = ragk_l2_search_groups(row_begin, row_end, nq, k, d);
     const int QT = nq > 16 ? 2 : 1;

@@ -7,7 +7,8 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("d", [32, 100, 384, 1024])
-@pytest.mark.parametrize("n,begin,cap", [(7, 0, 7), (15, 0, 15), (65, 3, 66), (1025, 17, 1031), (70001, 5, 70001),
+@pytest.mark.parametrize("n,begin,cap", [(7, 0, 7), (15, 0, 15), (65, 3, 66), (1025, 17, 1031), (16387, 3, 16390),
+                                         (49153, 1, 49153), (70001, 5, 70001),
                                          (200003, 17, 200004)])
 def test_search_tiles(native, n, begin, cap, d):
     """Stores of less than a tile, tiles cut by the end of the store or begun at an odd row; queries on both sides of every

@@ -146,17 +146,17 @@ def gemm_rope_kv_ok(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, 
             and slots.is_contiguous() and positions.numel() == M and slots.numel() == M)
 
 
-def gemm_rope_kv(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, Hkv, D, out=None):
+def gemm_rope_kv(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, Hkv, D, out=None, checked=False):
     """qkv = x @ w^T with RoPE applied to q and k and the k / v rows written to the paged cache at `slots`
-    (gemm + rope_kv in gemm's own launches, bit-identical to both; callers check gemm_rope_kv_ok first)."""
-    _req(gemm_rope_kv_ok(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, Hkv, D), "gemm_rope_kv operands")
+    (gemm + rope_kv in gemm's own launches, bit-identical to both). checked: the caller has asked gemm_rope_kv_ok."""
+    _req(checked or gemm_rope_kv_ok(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, Hkv, D), "gemm_rope_kv operands")
     M, K = x.shape
     N = w.shape[0]
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     _req(out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "gemm_rope_kv out")
     L = _lib.lib()
-    x, w = _tile_rows(x), _tile_rows(w)
+    x, w = _tile_rows(x, w)
     for r0, r1, mi, S in gemm_plan(M, N, K, True, _cu_count()):
         a = (x.data_ptr() + r0 * x.stride(0) * 2, x.stride(0), w.data_ptr(), w.stride(0),
              out.data_ptr() + r0 * out.stride(0) * 2, out.stride(0), r1 - r0, K, positions.data_ptr() + 4 * r0,
@@ -213,15 +213,13 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
         raise ValueError("tile GEMM needs N % 8 == 0")
     if M == 0:
         return out
-    L = _lib.lib()
-    ldr = resid.stride(0) if resid is not None else 0
     if (path is None and PREFILL_BLAS != "none" and not out_f32 and bias is None and use_pp(M, N, K, epi)
             and ((epi == "none" and PREFILL_BLAS in ("plain", "all"))
                  or (epi == "resid" and PREFILL_BLAS in ("resid", "all")))):
         return _gemm_blas(x, w, resid, out, epi)
     if path is None and M > 64:
-        rows = w.shape[0]
-        x, w = _tile_rows(x), _tile_rows(w)
+        rows = 2 * N if epi in PAIR_EPI else N
+        x, w = _tile_rows(x, w)
         # gemm_w4 addresses operands with 32-bit buffer offsets
         fits = x.stride(0) * M * 2 < 2 ** 31 and w.stride(0) * rows * 2 < 2 ** 31
         if not fits and use_pp(M, N, K, epi):
@@ -244,6 +242,8 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
     if (path is None and use_vocab(M, N, K, epi) and out_f32 and out.stride(0) == N and _vec_rows(x, w)
             and out.data_ptr() % 16 == 0):
         return gemm_stream_part(x, w, out=out, rows=64, S=1)
+    L = _lib.lib()
+    ldr = resid.stride(0) if resid is not None else 0
     if path is None and STREAM_DEFAULT and use_stream(M, N, K, epi):
         path = 5
     if path is None and DEC_DEFAULT and use_dec(M, N, K, epi):
@@ -285,20 +285,23 @@ def gemm_mid(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, m
     a workspace, summed with the epilogue by a second launch)."""
     M, K = x.shape
     N = w.shape[0] // 2 if epi in PAIR_EPI else w.shape[0]
-    x, w = _tile_rows(x), _tile_rows(w)
+    x, w = _tile_rows(x, w)
     _req(mi in MID_US and 1 <= S <= K // 64 and K % 64 == 0 and w.shape[1] == K, "gemm_mid tile or split")
     _req(out.shape == (M, N) and out.stride(1) == 1, "gemm_mid out")
     _gemm_rows(x, w, bias, resid, epi, out, out_f32, 0, M, mi, S)
     return out
 
 
-def _tile_rows(t):
-    """t, or a copy of rows that gemm_mid and gemm_w4 cannot fetch where they lie: their LDS-DMA pieces start on 16 bytes, and a
-    tile's 256 rows are reached by 32-bit offsets."""
-    ld = t.stride(0)
-    if ld % 8 == 0 and t.data_ptr() % 16 == 0 and ld * 514 < 2 ** 31:
-        return t
-    return t.clone(memory_format=torch.contiguous_format)
+_TILE_LD = ~(2 ** 21 - 8)  # bits that no row stride has which _tile_rows leaves: starts off 16 bytes, rows from 4 MB on
+
+
+def _tile_rows(x, w):
+    """x and w, or copies of rows that gemm_mid and gemm_w4 cannot fetch where they lie: their LDS-DMA pieces start on 16 bytes,
+    and a tile's 256 rows are reached by 32-bit offsets. (One look at both: this is host time of every product.)"""
+    if not ((x.data_ptr() | w.data_ptr()) & 15 or (x.stride(0) | w.stride(0)) & _TILE_LD):
+        return x, w
+    return tuple(t.clone(memory_format=torch.contiguous_format) if t.data_ptr() & 15 or t.stride(0) & _TILE_LD else t
+                 for t in (x, w))
 
 
 def _gemm_rows(x, w, bias, resid, epi, out, out_f32, r0, r1, mi, S):
@@ -606,7 +609,7 @@ def gemm_splitk(x, w, nsplit, out=None):
     _req(out.dtype == torch.float32 and out.is_contiguous() and out.numel() >= nsplit * M * N, "gemm_splitk out")
     if M == 0:
         return out
-    x, w = _tile_rows(x), _tile_rows(w)
+    x, w = _tile_rows(x, w)
     mi, w4 = _splitk_tile(M, N, K, nsplit, _cu_count())
     if w4 and x.stride(0) * M * 2 < 2 ** 31 and w.stride(0) * N * 2 < 2 ** 31:
         check(_lib.lib().ragk_gemm_w4_splitk(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), M, N, K,
@@ -1139,6 +1142,20 @@ def encoder_forward_ok(cfg, w):
     return encoder_pointers(cfg, w) is not None
 
 
+@functools.lru_cache(maxsize=4096)
+def _encoder_plans(T, H, I, cus, split, w4_min_m):
+    """(launches of the four products of a layer of T rows, floats of the largest one's slabs)."""
+    plans, slab = (_lib.GemmPlan * 4)(), 0
+    for i, (N, K) in enumerate(((3 * H, H), (H, H), (I, H), (H, I))):
+        S, mi = ln_slabs(T, N, K) if i in (1, 3) else (1, 0)
+        plan = ((0, T, mi, S),) if S > 1 else ((0, T, -1, 1),) if T <= 64 else gemm_plan(T, N, K, True, cus)
+        plans[i].n, plans[i].slabs = len(plan), int(S > 1)
+        for j, (r0, r1, mi, S) in enumerate(plan):
+            plans[i].p[j] = _lib.GemmPiece(r0, r1, mi, S)
+            slab = max(slab, S * (r1 - r0) * N if S > 1 else 0)
+    return plans, slab
+
+
 def encoder_forward(cfg, weights, ids, lens, first_pos, out, rows):
     """Embeddings of packed sequences (host int32 ids, int64 lens) into rows `rows` of out (fp32 on the device): one upload
     of the step's integers, one workspace, one native call for all launches (csrc/kernels/encoder.hip). `weights`: their
@@ -1160,14 +1177,7 @@ def encoder_forward(cfg, weights, ids, lens, first_pos, out, rows):
     at = list(itertools.accumulate(map(len, parts), initial=0))
     ints = torch.from_numpy(np.concatenate(parts).astype(np.int32, copy=False)).to(dev)
     L, cus, c = _lib.lib(), _cu_count(), _lib.EncoderCall()
-    slab = 0
-    for i, (N, K) in enumerate(((3 * H, H), (H, H), (I, H), (H, I))):
-        S, mi = ln_slabs(T, N, K) if i in (1, 3) else (1, 0)
-        plan = ((0, T, mi, S),) if S > 1 else ((0, T, -1, 1),) if T <= 64 else gemm_plan(T, N, K, True, cus)
-        c.plans[i].n, c.plans[i].slabs = len(plan), int(S > 1)
-        for j, (r0, r1, mi, S) in enumerate(plan):
-            c.plans[i].p[j] = _lib.GemmPiece(r0, r1, mi, S)
-            slab = max(slab, S * (r1 - r0) * N if S > 1 else 0)
+    c.plans, slab = _encoder_plans(T, H, I, cus, PREFILL_SPLITK, PREFILL_SPLITK_MIN_M)
     # activations in the order h, a, attn, qkv, f, then the slabs
     sizes = [2 * T * n for n in (H, H, H, 3 * H, I)] + [4 * slab]
     off = list(itertools.accumulate([-(-n // 256) * 256 for n in sizes], initial=0))
@@ -1222,7 +1232,7 @@ def gemm_layernorm(x, w, bias, resid, g, b, eps):
     S, mi = ln_slabs(M, N, K)
     if S == 1:
         return layernorm(gemm(x, w, bias=bias, resid=resid, epi="bias_resid"), g, b, eps)
-    x, w = _tile_rows(x), _tile_rows(w)
+    x, w = _tile_rows(x, w)
     if mi < 0:
         return layernorm_slabs(gemm_part(x, w, out=torch.empty((S, M, N), dtype=torch.float32, device=x.device), ks=K // 64 // S),
                                bias, resid, g, b, eps)

@@ -60,7 +60,8 @@ def test_operand_rows_that_are_copied():
     for t, copied in ((a, False), (a[:, :256], False), (a[:, 8:], False), (a[::2], False), (a[:, 4:260], True), (a[:, :132][1:], False),
                       (a.view(-1)[:79 * 263].view(79, 263)[:, :256], True), (a.view(-1)[1:1 + 70 * 256].view(70, 256), True),
                       (far, True), (far[:, :8], True)):
-        got = n._tile_rows(t)
+        (got, same), (same2, got2) = n._tile_rows(t, a), n._tile_rows(a, t)
+        assert same is a and same2 is a and torch.equal(got, got2)
         assert (got.data_ptr() != t.data_ptr()) == copied and torch.equal(got, t)
         assert not copied or (got.is_contiguous() and got.data_ptr() % 16 == 0)
 
@@ -77,6 +78,8 @@ def test_plans_follow_their_settings(monkeypatch):
     assert all((n.slab_count(*s), n.ln_slabs(*s), n.prefill_nsplit(*s)) == (1, (1, 0), 1) for s in sizes)
     monkeypatch.setattr(n, "PREFILL_SPLITK", True)
     assert on == [(n.slab_count(*s), n.ln_slabs(*s), n.prefill_nsplit(*s)) for s in sizes]
+    off = n._encoder_plans(700, 1024, 4096, 256, n.PREFILL_SPLITK, n.PREFILL_SPLITK_MIN_M)
+    assert off[1] > 0 and off[0][3].slabs and [p.r1 for p in off[0][3].p[:1]] == [700]
     monkeypatch.setattr(n, "PREFILL_SPLITK_MIN_M", 10 ** 6)
     assert all(n.prefill_nsplit(*s) == 1 for s in sizes)
     assert n.slab_count(1700, 4096, 14336) == 1

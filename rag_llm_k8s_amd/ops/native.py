@@ -237,7 +237,7 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
             return out
     if path == 0:
         return gemm_mid(x, w, bias=bias, resid=resid, epi=epi, out=out, out_f32=out_f32)
-    if path is None and use_hold(M, N, K, epi) and _vec_rows(x, w):
+    if path is None and not out_f32 and use_hold(M, N, K, epi) and _vec_rows(x, w):
         return gemm_hold(x, w, par=bias, epi=epi, out=out)
     if (path is None and use_vocab(M, N, K, epi) and out_f32 and out.stride(0) == N and _vec_rows(x, w)
             and out.data_ptr() % 16 == 0):
@@ -930,6 +930,7 @@ def gemm_hold(x, w, wscale=None, par=None, epi="silu_mul", out=None):
         out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     per = _hold_rows(K, wscale is not None)
     _req(per > 0 and w.shape[1] == K and epi in PAIR_EPI and 0 < M <= 64, "gemm_hold shape")
+    _req(out.dtype == torch.bfloat16 and out.shape == (M, N) and out.stride(1) == 1, "gemm_hold out")
     per = -(-M // -(-M // per))
     for r0 in range(0, M, per):
         xs, os_ = x[r0:r0 + per], out[r0:r0 + per]

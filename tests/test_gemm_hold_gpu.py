@@ -80,3 +80,18 @@ def test_rows_of_any_stride(native):
     far = torch.empty_strided((70, 256), (2 ** 22, 1), dtype=torch.bfloat16, device=DEV)
     far.copy_(torch.randn(70, 256, device=DEV))
     assert torch.equal(native.gemm(far, w[:, :256].contiguous()), native.gemm(far.contiguous(), w[:, :256].contiguous()))
+
+
+@pytest.mark.parametrize("M", [1, 12, 64, 70])
+def test_gated_units_are_bf16_only(native, M):
+    """fp32 rows of a gated unit are refused at every size, whichever kernel would take the product; so is another output."""
+    x, w = torch.zeros(M, 2048, device=DEV).bfloat16(), torch.zeros(2816, 2048, device=DEV).bfloat16()
+    out = torch.full((M, 1408), 7.0, device=DEV)
+    for args in (dict(epi="silu_mul"), dict(epi="glu_clip", bias=torch.ones(3, device=DEV))):
+        with pytest.raises((ValueError, native._lib.NativeLibraryError)):
+            native.gemm(x, w, out=out, out_f32=True, **args)
+    if M <= 64:
+        for bad in (out, out.bfloat16()[:, ::2], torch.zeros(M, 1344, device=DEV).bfloat16()):
+            with pytest.raises(ValueError):
+                native.gemm_hold(x, w, out=bad)
+    assert out.eq(7.0).all()

@@ -3,7 +3,7 @@
 // A few hundred to a few thousand rows give the 256x256 tiles of gemm_w4.hip too few tiles for 256 CUs (112 at
 // 1777 x 4096), and a 128x128 tile with one K-tile in flight waits for memory on every K-tile. Here:
 //  * tiles of 32*MI x 128 (MI = 3, 4, 5, 6, 8: 96 to 256 rows), chosen with the K-split by a cost model of the whole
-//    launch (ops/native.py mid_plan), so rows are padded little and the last round of tiles is full;
+//    launch (ops/native.py gemm_plan), so rows are padded little and the last round of tiles is full;
 //  * a ring of D K-tiles (64 deep, 3 to 5 of them in LDS), a slot refilled as soon as it is read out; one persistent
 //    block per CU streams the K-tiles of its work items through it as one sequence, so only the first item waits;
 //  * split-K: work item = (slab, tile); fp32 slabs P[S][M][N] go to a consumer that sums them (row norms) or to
@@ -13,8 +13,9 @@
 //
 // Measured (us, cold weights; before: the 128x128 double-buffered tile / gemm_w4 from 1024 rows): 300 x 4096 x 4096
 // 48 -> 24, 300 x 4096 x 14336 193 -> 51, 300 x 28672 x 4096 126 -> 86, 800 x 4096 x 4096 51 -> 31, 1777 x 4096 x 4096
-// 79 -> 55, 1777 x 4096 x 14336 263 -> 181, 3000 x 1024 x 4096 69 -> 28. On few blocks a K-tile takes 0.29 us at MI = 3 and
-// 0.63 at MI = 8 (LDS bound: 0.28 and 0.48); with every CU busy 0.42 and 0.83.
+// 79 -> 55, 1777 x 4096 x 14336 263 -> 181, 3000 x 1024 x 4096 69 -> 28 (on the slowest card seen a tenth more: 24.4, 53,
+// 94, 34, 61, 197, 31). A K-tile takes 0.28 us at MI = 3 and 0.62 at MI = 8 on few blocks (LDS bound: 0.28 and 0.48), with
+// every CU busy 0.40 and 0.83.
 //
 // The weight fragment is the first MFMA operand: a lane holds four consecutive output columns of one row, eight with
 // the staged weight rows permuted (mid_row), so epilogues load and store 16 B straight from registers. K order and
@@ -478,8 +479,8 @@ int launch_finish(const float* P, int S, void* C, int ldc, const void* bias, con
   X(EPI_SILU_MUL) X(EPI_GLU_CLIP)
 
 // N = output columns (for the pair epilogues the weight has 2 N rows in the packed [64 gate | 64 up] layout, N % 64 == 0).
-// Rows of A and B start on 16 bytes. mi = rows of a tile / 32. S > 1: K-split through the fp32 slabs ws [S][M][weight rows], summed with the epilogue by a
-// second launch. S slabs without a consumer here: epi NONE, out_f32 = 2 (C holds the slabs).
+// Rows of A and B start on 16 bytes. mi = rows of a tile / 32. S > 1: K-split through the fp32 slabs ws [S][M][weight rows],
+// summed with the epilogue by a second launch. S slabs without a consumer here: epi NONE, out_f32 = 2 (C holds the slabs).
 RAGK_API int ragk_gemm_mid(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias,
                            const void* resid, int ldr, int M, int N, int K, int epi, int out_f32, int mi, int S, float* ws,
                            hipStream_t st) {

@@ -482,9 +482,13 @@ class NativeBackend(TorchBackend):
         return self.n.gemm(x, w, out_f32=True).unsqueeze(0), bias
 
     def splits(self, M, w):
-        # Up to 64 rows from 2^24 weights on: the register-streaming product with its epilogue reads them on too few blocks
-        # (50 rows of niduvik / rolesun, 4096 wide: 985 / 1102 -> 775 / 826 us). Below, the launches' host time bounds the step
-        # and the slabs' is longer (2048 wide, 30 / 40 rows: 543 / 655 us against 569 / 719).
+        # Up to 64 rows, rows against slabs with the norm behind them: the slabs cost the host 2 us more a projection (18 to 19
+        # -> 20 to 21) and take less on the GPU the more weights and rows there are, since the register-streaming product reads
+        # its weights on too few blocks: 2048 x 2048 at 12 / 50 rows 9.5 / 15.1 -> 8.4 / 10.2 us, 2048 x 5632 15.1 / 28.9 -> 10.8 /
+        # 12.5, 3584 x 3584 12.9 / 22.1 -> 14.3 / 17.5, 4096 x 4096 14.3 / 25.2 -> 12.7 / 14.5, 4096 x 14336 32.0 / 66.6 -> 25.3 /
+        # 29.2. From 2^24 weights on they are ahead at every row count (niduvik / rolesun 4096 wide, 50 rows: 985 / 1102 -> 775 /
+        # 826 us a step). Models 2048 wide, whose steps the host bounds at 30 / 40 rows, lose (543 / 655 -> 569 / 719); the line
+        # lies between the two, and long projections of many rows below it forgo the GPU's gain.
         if w.dtype != torch.bfloat16:
             return False
         if M <= 64:

@@ -115,7 +115,7 @@ def use_pp(M, N, K, epi):
 PREFILL_BLAS = os.environ.get("RAGK_PREFILL_BLAS", "none")
 
 
-# The prefill qkv projection with rope_kv's work in the gemm_w4 epilogue (RoPE on q / k, k and v rows into
+# The prefill qkv projection with rope_kv's work in its epilogue (gemm_w4's, gemm_mid's; RoPE on q / k, k and v rows into
 # the paged cache; bit-identical to gemm + rope_kv): one pass over the 32k-token chunk's qkv fewer.
 PREFILL_ROPE_FUSED = os.environ.get("RAGK_PREFILL_ROPE", "1") != "0"
 
@@ -542,10 +542,10 @@ def _cu_count():
 
 
 def prefill_nsplit(M, N, K):
-    """K-slabs for a prefill GEMM whose 256x256 tile grid fills the CUs poorly (gemm_w4c KSPLIT):
-    the split with the best wave efficiency (tiles / (waves * CUs)), 2 % charged per extra slab for
-    the fp32 slab traffic; 1 = no split. M = 5.2k (a C=1 RAG prompt), N = 4096: 336 tiles = 1.31 waves
-    (66 %) -> 2 slabs = 2.6 waves (88 %). The 32k-token bench steps (2048 tiles) never split."""
+    """K-slabs of gemm_w4 alone (its KSPLIT form) by how full its 256x256 tiles leave the CUs: the split with the best
+    wave efficiency (tiles / (waves * CUs)), 2 % charged per extra slab for the fp32 slab traffic; 1 = no split. 5200 rows,
+    N = 4096: 336 tiles = 1.31 waves (66 %) -> 2 slabs = 2.6 waves (88 %). slab_count weighs it against gemm_mid's tiles: there
+    those rows take no split, gemm_w4 on 4096 of them and gemm_mid on the rest."""
     if not PREFILL_SPLITK or M < PREFILL_SPLITK_MIN_M:
         return 1
     return _w4_nsplit(M, N, K, _cu_count())

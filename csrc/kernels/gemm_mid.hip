@@ -2,20 +2,26 @@
 //
 // A few hundred to a few thousand rows give the 256x256 tiles of gemm_w4.hip too few tiles for 256 CUs (112 at
 // 1777 x 4096), and a 128x128 tile with one K-tile in flight waits for memory on every K-tile. Here:
-//  * tiles of 32*MI x 128 (MI = 3, 4, 5, 6, 8: 96 to 256 rows), chosen with the K-split by a cost model of the whole
-//    launch (ops/native.py gemm_plan), so rows are padded little and the last round of tiles is full;
+//  * tiles of 32*MI x 128 (MI = 3 .. 8: 96 to 256 rows) and of 160 x 256, chosen with the K-split by a cost model of the
+//    whole launch (ops/native.py gemm_plan), so rows are padded little and the last round of tiles is full;
 //  * a ring of D K-tiles (64 deep, 3 to 5 of them in LDS), a slot refilled as soon as it is read out; one persistent
 //    block per CU streams the K-tiles of its work items through it as one sequence, so only the first item waits;
 //  * split-K: work item = (slab, tile); fp32 slabs P[S][M][N] go to a consumer that sums them (row norms) or to
 //    splitk_finish (bias / residual / activation / gated pairs).
-// 4 waves as 2 x 2, wave tile 16*MI x 64: per K-tile a wave reads (16 MI + 64) x 128 B for 8 MI MFMAs. LDS traffic
-// with the DMA writes bounds small MI (768 of 512 MFMA clocks at MI = 4, 1152 of 1024 at MI = 8).
+// 4 waves as 2 x 2, wave tile 16*MI x 16*NJ (NJ = 4: 128 columns, 8: 256): per K-tile a wave reads (16 MI + 16 NJ) x 128 B
+// for 2 MI NJ MFMAs. LDS traffic with the DMA writes bounds small MI (768 of 512 MFMA clocks at MI = 4, 1152 of 1024 at
+// MI = 8); 160 x 256 is the largest tile that leaves a ring of three K-tiles and the one that LDS bounds least (1248 clocks
+// of 1280): two of the 160 x 128 tiles it stands for take 1728. 192 x 192 and 224 x 192 tiles came to the same rates and won
+// where neither size divides well only (1500 x 6144 x 4096 64 us against 66), 96 and 128 rows of 256 columns nowhere.
 //
 // Measured (us, cold weights; before: the 128x128 double-buffered tile / gemm_w4 from 1024 rows): 300 x 4096 x 4096
 // 48 -> 24, 300 x 4096 x 14336 193 -> 51, 300 x 28672 x 4096 126 -> 86, 800 x 4096 x 4096 51 -> 31, 1777 x 4096 x 4096
 // 79 -> 55, 1777 x 4096 x 14336 263 -> 181, 3000 x 1024 x 4096 69 -> 28 (on the slowest card seen a tenth more: 24.4, 53,
-// 94, 34, 61, 197, 31). A K-tile takes 0.28 us at MI = 3 and 0.62 at MI = 8 on few blocks (LDS bound: 0.28 and 0.48), with
-// every CU busy 0.40 and 0.83.
+// 94, 34, 61, 197, 31). With 160 x 256 and 224 x 128 beside the other tiles (both on that card): 300 x 28672 x 4096 89 -> 75,
+// 600 x 28672 x 4096 154 -> 135, 600 x 4096 x 14336 in slabs 81 -> 67, 1500 x 6144 x 4096 81 -> 67, 1777 x 4096 x 4096 56 ->
+// 54, 1777 x 4096 x 14336 183 -> 175, 200 x 28672 x 4096 65 -> 61.
+// A K-tile takes 0.28 us at MI = 3 and 0.62 at MI = 8 on few blocks (LDS bound: 0.28 and 0.48), with
+// every CU busy 0.40 and 0.83; of 160 x 256 0.76 and 0.96.
 //
 // The weight fragment is the first MFMA operand: a lane holds four consecutive output columns of one row, eight with
 // the staged weight rows permuted (mid_row), so epilogues load and store 16 B straight from registers. K order and
@@ -27,24 +33,25 @@ using namespace ragk;
 
 namespace {
 
-constexpr int MID_BN = 128, MID_BK = 64, MID_THREADS = 256;
+constexpr int MID_BK = 64, MID_THREADS = 256;
 constexpr int MID_GROUP_M = 8;
 constexpr int MID_LDS = 160 * 1024;
+constexpr int MID_WIDE = 16;  // added to a tile's rows / 32 in the C entries' `mi`: 256 columns instead of 128
 
-constexpr int mid_stage(int mi) { return (32 * mi + MID_BN) * MID_BK * 2; }
-constexpr int mid_depth(int mi) { return MID_LDS / mid_stage(mi) < 5 ? MID_LDS / mid_stage(mi) : 5; }
+constexpr int mid_stage(int mi, int nj) { return 32 * (mi + nj) * MID_BK * 2; }
+constexpr int mid_depth(int mi, int nj) { return MID_LDS / mid_stage(mi, nj) < 5 ? MID_LDS / mid_stage(mi, nj) : 5; }
 
 __device__ __forceinline__ int mswz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 
-// Weight row (within the 128-row tile) staged at LDS row q, so that lane (fr, fh) of MFMA tiles 2p, 2p + 1 of a wave
-// holds eight consecutive output columns. PAIR: the tile is [64 first | 64 second] (gate / up; the halves of a rotated
-// head): a wave's tiles 0, 1 come from the first half and 2, 3 from the second, so both members of a pair are in one
-// lane.
-template <bool PAIR>
+// Weight row (within the tile) staged at LDS row q, so that lane (fr, fh) of MFMA tiles 2p, 2p + 1 of a wave holds eight
+// consecutive output columns. PAIR: groups of 128 rows are [64 first | 64 second] (gate / up; the halves of a rotated head)
+// and tile j of a wave pairs with tile j + NJ / 2, so both members of a pair are in one lane: 128 columns are one group
+// that two waves share, a wave of the 256-column tile has a group of its own and needs no other order than without pairs.
+template <int NJ, bool PAIR>
 __device__ __forceinline__ int mid_row(int q) {
-  const int h = q >> 6, j = (q >> 4) & 3, c = (q >> 2) & 3, k = q & 3;
-  if constexpr (PAIR) return 64 * (j >> 1) + 32 * h + 8 * c + 4 * (j & 1) + k;
-  return 64 * h + 32 * (j >> 1) + 8 * c + 4 * (j & 1) + k;
+  const int h = q / (16 * NJ), j = (q >> 4) % NJ, c = (q >> 2) & 3, k = q & 3;
+  if constexpr (PAIR && NJ == 4) return 64 * (j >> 1) + 32 * h + 8 * c + 4 * (j & 1) + k;
+  return 16 * NJ * h + 32 * (j >> 1) + 8 * c + 4 * (j & 1) + k;
 }
 
 // Inline asm ties source and destination of an accumulator (with the builtin hipcc rotates them through other registers
@@ -53,13 +60,13 @@ __device__ __forceinline__ int mid_row(int q) {
 __device__ __forceinline__ void mid_mfma(f32x4& c, const bf16x8& w, const bf16x8& x) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
 }
-template <int MI>
-__device__ __forceinline__ void mid_pin(f32x4 (&acc)[MI][4]) {
+template <int MI, int NJ>
+__device__ __forceinline__ void mid_pin(f32x4 (&acc)[MI][NJ]) {
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 1" ::: "memory");
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) asm volatile("" : "+a"(acc[i][j])::"memory");
+    for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j])::"memory");
 }
 
 struct MidItem {
@@ -68,7 +75,8 @@ struct MidItem {
 
 // Work item -> tile. Items are numbered so that each XCD owns a contiguous range (a block keeps its XCD: the grid is
 // a multiple of 8 or one round), M-tiles of one weight panel next to each other.
-__device__ __forceinline__ MidItem mid_item(int it, int total, int tiles_m, int tiles_n, int nk, int S, int bm) {
+__device__ __forceinline__ MidItem mid_item(int it, int total, int tiles_m, int tiles_n, int nk, int S, int bm,
+                                           int bn) {
   const int nt = tiles_m * tiles_n;
   int l = xcd_remap(it, total);
   MidItem w;
@@ -80,7 +88,7 @@ __device__ __forceinline__ MidItem mid_item(int it, int total, int tiles_m, int 
   const int in = l - group * MID_GROUP_M * tiles_n;
   // (uniform; the divisions run on the vector unit)
   w.m0 = __builtin_amdgcn_readfirstlane((first + in % gm) * bm);
-  w.n0 = __builtin_amdgcn_readfirstlane((in / gm) * MID_BN);
+  w.n0 = __builtin_amdgcn_readfirstlane((in / gm) * bn);
   w.k0 = __builtin_amdgcn_readfirstlane((int)((unsigned)(nk * w.z) / (unsigned)S));
   w.k1 = __builtin_amdgcn_readfirstlane((int)((unsigned)(nk * (w.z + 1)) / (unsigned)S));
   return w;
@@ -180,25 +188,26 @@ __device__ __forceinline__ void mid_rope8(float (&x1)[8], float (&x2)[8], const 
   }
 }
 
-template <int MI, int EPI>
+template <int MI, int NJ, int EPI>
 __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ B, int ldb, void* C, int ldc,
     const bf16_t* __restrict__ bias, const bf16_t* resid, int ldr, int M, int N, int K, int S, int out_f32, RopeKV rk) {
   constexpr bool PAIR = epi_pair(EPI) || EPI == EPI_ROPE_KV;
-  constexpr int BM = 32 * MI, STAGE = mid_stage(MI), D = mid_depth(MI), PW = MI + 4;  // DMA pieces (and fragment reads a half) a wave
-  constexpr int DSTEP = 4 * MI / PW;                                             // MFMAs between two pieces
+  constexpr int BM = 32 * MI, BN = 32 * NJ, STAGE = mid_stage(MI, NJ), D = mid_depth(MI, NJ);
+  constexpr int PW = MI + NJ;          // DMA pieces (and fragment reads a half) a wave
+  constexpr int DSTEP = NJ * MI / PW;  // MFMAs between two pieces
   constexpr int OFF_B = BM * 128;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wid >> 1, wc = wid & 1, fr = lane & 15, fh = lane >> 4;
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + MID_BN - 1) / MID_BN;
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const int total = tiles_m * tiles_n * S, nk = K / MID_BK, grid = gridDim.x;
 
   // ---- DMA side: the K-tile that is issued next. Descriptors start at the tile's own rows, so offsets stay small.
   int d_it = blockIdx.x;
-  MidItem dw = mid_item(d_it, total, tiles_m, tiles_n, nk, S, BM);
-  int dk = dw.k0, off_a[MI], off_b[4];
+  MidItem dw = mid_item(d_it, total, tiles_m, tiles_n, nk, S, BM, BN);
+  int dk = dw.k0, off_a[MI], off_b[NJ];
   i32x4 srd_a, srd_b;
   auto origin = [&](const MidItem& w) {
     // rows past the edge read the last valid row: their outputs are never stored
@@ -208,9 +217,9 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
       off_a[i] = min(r, M - 1 - w.m0) * lda * 2 + 16 * mswz(r, lane & 7);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = (wid * 4 + i) * 8 + (lane >> 3);
-      off_b[i] = min(mid_row<PAIR>(r), N - 1 - w.n0) * ldb * 2 + 16 * mswz(r, lane & 7);
+    for (int i = 0; i < NJ; ++i) {
+      const int r = (wid * NJ + i) * 8 + (lane >> 3);
+      off_b[i] = min(mid_row<NJ, PAIR>(r), N - 1 - w.n0) * ldb * 2 + 16 * mswz(r, lane & 7);
     }
     srd_a = make_srd(A + (size_t)w.m0 * lda, 0x7fffffffu);
     srd_b = make_srd(B + (size_t)w.n0 * ldb, 0x7fffffffu);
@@ -222,7 +231,7 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
   auto piece = [&](int q) {
     const int so = dk * (MID_BK * 2);
     if (q < MI) blds16_asm(srd_a, off_a[q], so, d_slot + (wid * MI + q) * 1024);
-    else blds16_asm(srd_b, off_b[q - MI], so, d_slot + OFF_B + (wid * 4 + q - MI) * 1024);
+    else blds16_asm(srd_b, off_b[q - MI], so, d_slot + OFF_B + (wid * NJ + q - MI) * 1024);
   };
   auto advance = [&]() {
     d_slot = d_slot + STAGE == lds0 + D * STAGE ? lds0 : d_slot + STAGE;
@@ -230,7 +239,7 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
       const int nx = d_it + grid;
       if (nx < total) {
         d_it = nx;
-        dw = mid_item(nx, total, tiles_m, tiles_n, nk, S, BM);
+        dw = mid_item(nx, total, tiles_m, tiles_n, nk, S, BM, BN);
         dk = dw.k0;
         origin(dw);
       } else {
@@ -246,21 +255,21 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
   for (int s = 0; s < 2; ++s) {
     const int cs = 16 * ((4 * s + fh) ^ ((fr >> 1) & 7));
     ra[s] = smem + (wr * 16 * MI + fr) * 128 + cs;
-    rb[s] = smem + OFF_B + (wc * 64 + fr) * 128 + cs;
+    rb[s] = smem + OFF_B + (wc * 16 * NJ + fr) * 128 + cs;
   }
-  bf16x8 a0[MI], b0[4], a1[MI], b1[4];
-  auto read = [&](bf16x8 (&a)[MI], bf16x8 (&b)[4], int s, unsigned slot, int q) {
-    if (q < 4) b[q] = *reinterpret_cast<const bf16x8*>(rb[s] + slot + q * 2048);
-    else a[q - 4] = *reinterpret_cast<const bf16x8*>(ra[s] + slot + (q - 4) * 2048);
+  bf16x8 a0[MI], b0[NJ], a1[MI], b1[NJ];
+  auto read = [&](bf16x8 (&a)[MI], bf16x8 (&b)[NJ], int s, unsigned slot, int q) {
+    if (q < NJ) b[q] = *reinterpret_cast<const bf16x8*>(rb[s] + slot + q * 2048);
+    else a[q - NJ] = *reinterpret_cast<const bf16x8*>(ra[s] + slot + (q - NJ) * 2048);
   };
-  f32x4 acc[MI][4];
+  f32x4 acc[MI][NJ];
   // MFMA m of a 32-deep half, then what else goes out there: the order is the written one (one wave a SIMD: nothing
   // else fills the gap that a burst of reads or DMAs leaves)
-  auto half = [&](const bf16x8 (&a)[MI], const bf16x8 (&b)[4], bf16x8 (&na)[MI], bf16x8 (&nb)[4], int ns, unsigned nslot,
+  auto half = [&](const bf16x8 (&a)[MI], const bf16x8 (&b)[NJ], bf16x8 (&na)[MI], bf16x8 (&nb)[NJ], int ns, unsigned nslot,
                   auto dma) {
 #pragma unroll
-    for (int m = 0; m < 4 * MI; ++m) {
-      const int i = m >> 2, j = m & 3;
+    for (int m = 0; m < NJ * MI; ++m) {
+      const int i = m / NJ, j = m % NJ;
       mid_mfma(acc[i][j], b[j], a[i]);
       if (m < PW) read(na, nb, ns, nslot, m);
       if constexpr (decltype(dma)::value) {
@@ -282,11 +291,11 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
   for (int q = 0; q < PW; ++q) read(a0, b0, 0, slot, q);
 
   for (int it = blockIdx.x; it < total; it += grid) {
-    const MidItem w = mid_item(it, total, tiles_m, tiles_n, nk, S, BM);
+    const MidItem w = mid_item(it, total, tiles_m, tiles_n, nk, S, BM, BN);
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < NJ; ++j) {
         acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
         asm volatile("" : "+a"(acc[i][j]));
       }
@@ -306,46 +315,60 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
       // Positions of all rows together, then tables and slots a row ahead of their use, instead of two loads in turn a row:
       // 1300 x 6144 x 4096 on 160-row tiles 78.1 -> 75.4 us, 8192 x 3072 x 2048 on 256-row ones 108.5 -> 99.4 (without the
       // rotation 67.3 and 85.1).
-      const int hd = w.n0 >> 7, d = 32 * wc + 8 * fh, r0 = w.m0 + wr * 16 * MI + fr;
+      // A wave of the 128-column tile turns 32 of a head's column pairs, one of the 256-column tile a whole head (the last such
+      // tile may hold one head only).
+      const int hd = (w.n0 >> 7) + (NJ == 8 ? wc : 0), r0 = w.m0 + wr * 16 * MI + fr;
       int pos[MI];
 #pragma unroll
       for (int i = 0; i < MI; ++i) pos[i] = rk.pos[min(r0 + 16 * i, M - 1)];
-      MidTurn t = mid_turn(rk, pos[0], min(r0, M - 1), hd, d), next = t;
+      if (hd * 128 < N) {
 #pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        const int row = r0 + 16 * i;
-        if (i + 1 < MI) next = mid_turn(rk, pos[i + 1 < MI ? i + 1 : i], min(row + 16, M - 1), hd, d);
-        if (row < M) {
-          float x1[8], x2[8];
+        for (int p = 0; p < NJ / 4; ++p) {
+          const int d = (NJ == 8 ? 32 * p : 32 * wc) + 8 * fh;
+          MidTurn t = mid_turn(rk, pos[0], min(r0, M - 1), hd, d), next = t;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            x1[e] = acc[i][e >> 2][e & 3];
-            x2[e] = acc[i][2 + (e >> 2)][e & 3];
+          for (int i = 0; i < MI; ++i) {
+            const int row = r0 + 16 * i;
+            if (i + 1 < MI) next = mid_turn(rk, pos[i + 1 < MI ? i + 1 : i], min(row + 16, M - 1), hd, d);
+            if (row < M) {
+              float x1[8], x2[8];
+#pragma unroll
+              for (int e = 0; e < 8; ++e) {
+                x1[e] = acc[i][2 * p + (e >> 2)][e & 3];
+                x2[e] = acc[i][2 * p + NJ / 2 + (e >> 2)][e & 3];
+              }
+              mid_rope8(x1, x2, rk, t, reinterpret_cast<bf16_t*>(C), ldc, row, hd, d);
+            }
+            t = next;
           }
-          mid_rope8(x1, x2, rk, t, reinterpret_cast<bf16_t*>(C), ldc, row, hd, d);
         }
-        t = next;
       }
     } else if constexpr (PAIR) {
       const GluPar gp = glu_par<EPI>(bias);
-      const int col = (w.n0 >> 1) + 32 * wc + 8 * fh;
 #pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        const int row = w.m0 + wr * 16 * MI + 16 * i + fr;
-        float o[8];
+      for (int p = 0; p < NJ / 4; ++p) {
+        const int col = (w.n0 >> 1) + (NJ == 8 ? 64 * wc + 32 * p : 32 * wc) + 8 * fh;
+        if (2 * col < N) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = glu_act<EPI>(acc[i][e >> 2][e & 3], acc[i][2 + (e >> 2)][e & 3], gp);
-        if (row < M) *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(C) + (size_t)row * ldc + col) = pack8(o);
+          for (int i = 0; i < MI; ++i) {
+            const int row = w.m0 + wr * 16 * MI + 16 * i + fr;
+            float o[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              o[e] = glu_act<EPI>(acc[i][2 * p + (e >> 2)][e & 3], acc[i][2 * p + NJ / 2 + (e >> 2)][e & 3], gp);
+            if (row < M) *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(C) + (size_t)row * ldc + col) = pack8(o);
+          }
+        }
       }
     } else {
       void* Cz = out_f32 ? (void*)(reinterpret_cast<float*>(C) + (size_t)w.z * M * ldc) : C;
       // The tile's bias and residual are requested together, ahead of any use: loaded where they are added, each of the 2 MI
       // row pieces waited for memory once more (8192 x 3072 x 1024 on 256-row tiles, us: bias 65.4 -> 56.5, without an epilogue
       // 55.1; GELU 78.2 -> 68.3; 13762 x 1024 x 4096, bias and residual, 160-row tiles 118.7 -> 116.8).
-      u32x4 bv[2] = {}, rv[MI][2] = {};
+      u32x4 bv[NJ / 2] = {}, rv[MI][NJ / 2] = {};
 #pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const int col = min(w.n0 + 64 * wc + 32 * p + 8 * fh, N - 8);
+      for (int p = 0; p < NJ / 2; ++p) {
+        const int col = min(w.n0 + 16 * NJ * wc + 32 * p + 8 * fh, N - 8);
         if constexpr (mid_has_bias(EPI)) bv[p] = *reinterpret_cast<const u32x4*>(bias + col);
         if constexpr (mid_has_resid(EPI)) {
 #pragma unroll
@@ -357,8 +380,8 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
       for (int i = 0; i < MI; ++i) {
         const int row = w.m0 + wr * 16 * MI + 16 * i + fr;
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          const int col = w.n0 + 64 * wc + 32 * p + 8 * fh;
+        for (int p = 0; p < NJ / 2; ++p) {
+          const int col = w.n0 + 16 * NJ * wc + 32 * p + 8 * fh;
           if (row < M && col < N) {
             float o[8];
 #pragma unroll
@@ -435,17 +458,17 @@ int mid_grid(int total) {
   return total < cus ? total : cus;
 }
 
-template <int MI, int EPI>
+template <int MI, int NJ, int EPI>
 int launch_mid(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias, const void* resid, int ldr,
                int M, int N, int K, int S, int out_f32, hipStream_t st,
                const RopeKV& rk = RopeKV{}) {
-  constexpr int lds = mid_stage(MI) * mid_depth(MI);
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<MI, EPI>),
+  constexpr int lds = mid_stage(MI, NJ) * mid_depth(MI, NJ);
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<MI, NJ, EPI>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (attr != hipSuccess) return (int)attr;
-  const long long total = (long long)((M + 32 * MI - 1) / (32 * MI)) * ((N + MID_BN - 1) / MID_BN) * S;
+  const long long total = (long long)((M + 32 * MI - 1) / (32 * MI)) * ((N + 32 * NJ - 1) / (32 * NJ)) * S;
   if (total > 0x7fffffff) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL((gemm_mid_kernel<MI, EPI>), dim3(mid_grid((int)total)), dim3(MID_THREADS), lds, st, (const bf16_t*)A, lda,
+  hipLaunchKernelGGL((gemm_mid_kernel<MI, NJ, EPI>), dim3(mid_grid((int)total)), dim3(MID_THREADS), lds, st, (const bf16_t*)A, lda,
                      (const bf16_t*)B, ldb, C, ldc, (const bf16_t*)bias, (const bf16_t*)resid, ldr, M, N, K, S, out_f32, rk);
   return (int)hipGetLastError();
 }
@@ -454,11 +477,16 @@ template <int EPI>
 int dispatch_mid(int mi, const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias, const void* resid,
                  int ldr, int M, int N, int K, int S, int out_f32, hipStream_t st, const RopeKV& rk = RopeKV{}) {
   switch (mi) {
-    case 3: return launch_mid<3, EPI>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, S, out_f32, st, rk);
-    case 4: return launch_mid<4, EPI>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, S, out_f32, st, rk);
-    case 5: return launch_mid<5, EPI>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, S, out_f32, st, rk);
-    case 6: return launch_mid<6, EPI>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, S, out_f32, st, rk);
-    case 8: return launch_mid<8, EPI>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, S, out_f32, st, rk);
+#define RAGK_TILE(CODE, MI, NJ) \
+  case CODE: return launch_mid<MI, NJ, EPI>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, S, out_f32, st, rk);
+    RAGK_TILE(3, 3, 4)
+    RAGK_TILE(4, 4, 4)
+    RAGK_TILE(5, 5, 4)
+    RAGK_TILE(6, 6, 4)
+    RAGK_TILE(7, 7, 4)
+    RAGK_TILE(8, 8, 4)
+    RAGK_TILE(MID_WIDE + 5, 5, 8)
+#undef RAGK_TILE
     default: return (int)hipErrorInvalidValue;
   }
 }

@@ -281,8 +281,8 @@ def gemm_glu(x, w, par):
 
 
 def gemm_mid(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, mi=4, S=1):
-    """gemm() on the 128-column ring tiles of gemm_mid.hip: tiles of 32 mi rows, K cut into S slabs (S > 1: fp32 slabs in
-    a workspace, summed with the epilogue by a second launch)."""
+    """gemm() on the ring tiles of gemm_mid.hip: 32 mi rows of 128 columns (mi = 21: 160 of 256), K cut into S slabs (S > 1:
+    fp32 slabs in a workspace, summed with the epilogue by a second launch)."""
     M, K = x.shape
     N = w.shape[0] // 2 if epi in PAIR_EPI else w.shape[0]
     x, w = _tile_rows(x, w)
@@ -321,12 +321,14 @@ def _gemm_rows(x, w, bias, resid, epi, out, out_f32, r0, r1, mi, S):
 
 
 # Microseconds that one 64-deep K-tile of an output tile takes with few blocks running, and what a full machine adds
-# (clocks, L2): tiles of gemm_mid by rows / 32, 0 = gemm_w4's 256 x 256; then those of a launch and of a tile's epilogue. Fitted
+# (clocks, L2): tiles of gemm_mid by rows / 32 (+ 16: of 256 columns, not 128), 0 = gemm_w4's 256 x 256; then those of a
+# launch and of a tile's epilogue. Fitted
 # to every tile and split of 20 weights (384 to 28672 rows, K 384 to 14336) at 65 .. 32768 rows of x on two cards, for the
 # choices that follow: they take 0.5 % more than the best launch in the mean, 4 % in one of twenty. (An earlier fit, with 0.25
 # added at 160 rows and one us for either epilogue, took the next tile up there: 1 and 8 %, and 12 % more than gemm_w4 alone at
-# 2600 x 4096 x 14336.)
-MID_US = {3: (0.27, 0.13), 4: (0.34, 0.15), 5: (0.40, 0.17), 6: (0.49, 0.17), 8: (0.62, 0.21)}
+# 2600 x 4096 x 14336.) 224 x 128 and 160 x 256 were fitted to 46 products of 90 .. 8000 rows later: with them the choices take
+# 3 % less in the mean, 20 % less at best (600 x 4096 x 14336), and 0.3 % more than the best launch.
+MID_US = {3: (0.27, 0.13), 4: (0.34, 0.15), 5: (0.40, 0.17), 6: (0.49, 0.17), 7: (0.54, 0.21), 8: (0.62, 0.21), 21: (0.76, 0.20)}
 W4_US = (1.01, 0.29)
 LAUNCH_US = (4.5, 1.75)
 W4_LAUNCH_US = (5.25, 4.25)
@@ -335,7 +337,7 @@ SLAB_US = 8 / 5e6  # one fp32 slab value written and read back
 
 def _tiles_us(M, rows, K, mi, S, cus):
     """Model time of one launch: rounds of tiles over the CUs, each K-tiles long plus an epilogue."""
-    bm, bn = (32 * mi, 128) if mi else (256, 256)
+    bm, bn = (32 * (mi & 15), 256 if mi & 16 else 128) if mi else (256, 256)
     items = -(-M // bm) * -(-rows // bn) * S
     rounds = -(-items // cus)
     a, b = MID_US[mi] if mi else W4_US

@@ -148,3 +148,50 @@ def test_library_refuses_rows_between_vectors(native):
                                4, 1, None, 0) != 0
     torch.cuda.synchronize()
     assert not out.any()
+
+
+# 224 x 128 and 160 x 256: edges in rows, a last tile of 8, 136 and 248 columns, rings with as many K-tiles as slots and fewer
+@pytest.mark.parametrize("mi,S,M,N,K", [(7, 1, 225, 136, 192), (7, 2, 223, 384, 128), (7, 3, 449, 640, 704), (21, 1, 161, 264, 192),
+                                         (21, 1, 159, 392, 128), (21, 2, 321, 504, 256), (21, 5, 320, 256, 704), (21, 1, 2000, 5120, 192)])
+def test_gemm_mid_larger_tiles(native, mi, S, M, N, K):
+    x, w, b, r = operands(M, N, K)
+    y = native.gemm_mid(x, w, out=torch.empty_like(r), mi=mi, S=S)
+    assert rel_err(y, x.float() @ w.float().t()) < 4e-3  # bf16 result: 2^-9 per value
+    for epi in ("none", "bias", "bias_resid", "gelu"):
+        y = native.gemm_mid(x, w, bias=b, resid=r, epi=epi, out=torch.empty_like(r), mi=mi, S=S)
+        # another tile's values: the order of K is the same in all of them
+        assert torch.equal(y, native.gemm_mid(x, w, bias=b, resid=r, epi=epi, out=torch.empty_like(r), mi=4, S=S)), epi
+    rows = N // 128 * 128  # gate / up: also one group in the last 256-column tile
+    par = torch.tensor([2.0, 1.702, 1.0, 0.0], device=DEV)
+    for epi, bias in (("silu_mul", None), ("glu_clip", par)):
+        y, z = (native.gemm_mid(x, w[:rows], bias=bias, epi=epi, out=torch.empty(M, rows // 2, device=DEV).bfloat16(), mi=m, S=S)
+                for m in (mi, 3))
+        assert torch.equal(y, z), epi
+    buf = torch.full((M + 2, N + 16), -3.0, device=DEV).bfloat16()
+    native.gemm_mid(x, w, out=buf[1:M + 1, 8:N + 8], mi=mi, S=S)
+    buf[1:M + 1, 8:N + 8] = -3.0
+    assert bool((buf == -3.0).all())
+
+
+@pytest.mark.parametrize("mi", [7, 21])
+@pytest.mark.parametrize("M,Hq,Hkv,S", [(161, 1, 1, 1), (300, 4, 2, 1), (225, 2, 1, 3)])
+def test_rotated_projection_larger_tiles(native, mi, M, Hq, Hkv, S):
+    """The C entry with a given tile against 128 x 128 (which gemm + rope_kv is compared with above); three heads leave half of the
+    last 256 columns."""
+    K, N, L = 640, (Hq + 2 * Hkv) * 128, native._lib.lib()
+    x, w, _, _ = operands(M, N, K)
+    cos, sin = (t.to(DEV) for t in R.rope_tables(128, 512))
+    pos = torch.randint(0, 512, (M,), device=DEV).int()
+    slots = torch.randperm((M // 64 + 2) * 64, device=DEV)[:M].int()
+    slots[::5] = -1
+    ws = torch.empty(S * M * N, device=DEV)
+    got = []
+    for m in (mi, 4):
+        out = torch.zeros(M + 1, N, device=DEV).bfloat16()
+        kc, vc = torch.zeros(2, M // 64 + 2, Hkv, 64, 128, device=DEV).bfloat16()
+        rc = L.ragk_gemm_mid_rope_kv(x.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), N, M, K, pos.data_ptr(), slots.data_ptr(),
+                                     cos.data_ptr(), sin.data_ptr(), kc.data_ptr(), vc.data_ptr(), Hq, Hkv, 64, m, S, ws.data_ptr(),
+                                     native.stream_ptr())
+        assert rc == 0
+        got.append((out, kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and bool(got[0][0][:M].any())

@@ -8,8 +8,8 @@ using namespace ragk;
 
 extern "C" {
 int ragk_gemm(const void*, int, const void*, int, void*, int, const void*, const void*, int, int, int, int, int, int, hipStream_t);
-int ragk_gemm_w4(const void*, int, const void*, int, void*, int, const void*, const void*, int, int, int, int, int, int,
-                 hipStream_t);
+int ragk_gemm_w4_tile(const void*, int, const void*, int, void*, int, const void*, const void*, int, int, int, int, int, int, int,
+                      hipStream_t);
 int ragk_gemm_mid(const void*, int, const void*, int, void*, int, const void*, const void*, int, int, int, int, int, int, int,
                   int, float*, hipStream_t);
 int ragk_attn_prefill(const void*, int, const void*, const void*, int, const int*, int, const int*, const int*, const int*,
@@ -106,7 +106,8 @@ __global__ __launch_bounds__(NT) void pool_l2norm_kernel(const bf16_t* __restric
 }
 
 
-// Launches of one product: rows r0 .. r1 on gemm_mid (tile mi, S slabs), gemm_w4 (mi 0) or the decode kernels (mi -1).
+// Launches of one product: rows r0 .. r1 on gemm_mid (tile mi, S slabs), gemm_w4 (mi 0: 256 rows a tile, or 32 + rows / 32) or the
+// decode kernels (mi -1).
 struct Piece { int r0, r1, mi, S; };
 struct Plan { int n, slabs; Piece p[2]; };  // slabs: p[0].S fp32 slabs of all rows for the norm behind it
 
@@ -131,8 +132,9 @@ int product(const Plan& plan, const void* x, int K, const void* w, int N, const 
     char* po = (char*)out + (size_t)p.r0 * N * 2;
     const int M = p.r1 - p.r0;
     const int rc = p.mi < 0    ? ragk_gemm(px, K, w, K, po, N, bias, pr, N, M, N, K, epi, 0, st)
-                   : p.mi == 0 ? ragk_gemm_w4(px, K, w, K, po, N, bias, pr, N, M, N, K, epi, 0, st)
-                               : ragk_gemm_mid(px, K, w, K, po, N, bias, pr, N, M, N, K, epi, 0, p.mi, p.S, ws, st);
+                   : p.mi == 0 || p.mi > 32
+                       ? ragk_gemm_w4_tile(px, K, w, K, po, N, bias, pr, N, M, N, K, epi, 0, p.mi ? p.mi - 32 : 8, st)
+                       : ragk_gemm_mid(px, K, w, K, po, N, bias, pr, N, M, N, K, epi, 0, p.mi, p.S, ws, st);
     if (rc) return rc;
   }
   return 0;

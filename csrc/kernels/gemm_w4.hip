@@ -1,5 +1,10 @@
 // 256x256x64 bf16 GEMM for the large-M prefill projections: 4 waves x (128x128) per workgroup, one
-// wave per SIMD, one persistent workgroup per CU streaming its tiles' K-tiles as ONE continuous ring.
+// wave per SIMD, one persistent workgroup per CU streaming its tiles' K-tiles as ONE continuous ring. Tiles of
+// 224 and 192 rows (16 IM rows a wave, IM = 8, 7, 6) fill rounds that 256 leaves part empty; the numbers below are IM = 8's.
+// 13764 rows, us at 256 / 224 rows: 3072 x 1024 75 / 69.5, 1024 x 1024 38 / 33, 1024 x 4096 90 / 85, 4096 x 1024 with GELU 128 /
+// 116 (in two launches with gemm_mid 122); 14076 x 28672 x 4096 gated 2283 / 2195, 7917 x 14336 x 2048 367 / 355. At 192 rows
+// 7917 x 3072 x 2048 86 -> 74.5, 5200 x 4096 x 4096 164 -> 138. Which tile: ops/native.py gemm_plan. 224 and 192 rows spill
+// nothing (256: 0 to 8 registers, in the epilogues).
 //
 // C[M,N] = A[M,K] . B[N,K]^T (+ fused epilogue: bias / residual / GELU / SiLU*up / fp32 split-K slabs).
 // A = activations (row-major, K contiguous), B = weights (nn.Linear layout [N][K]).
@@ -38,12 +43,11 @@ using namespace ragk;
 
 namespace {
 
-constexpr int WBM = 256, WBN = 256, WBK = 64;
+constexpr int WBN = 256, WBK = 64;
 constexpr int W4_THREADS = 256;
-constexpr int W_TILE_A = WBM * WBK * 2;  // 32 KiB
-constexpr int W_TILE_B = WBN * WBK * 2;  // 32 KiB
-constexpr int W_BUF = W_TILE_A + W_TILE_B;
-constexpr int W4_LDS = 2 * W_BUF;  // two K-tile buffers; the epilogue needs no LDS
+constexpr int w_tile_a(int im) { return 32 * im * WBK * 2; }  // 32 KiB at 256 rows
+constexpr int W_TILE_B = WBN * WBK * 2;                       // 32 KiB
+constexpr int w_buf(int im) { return w_tile_a(im) + W_TILE_B; }  // a K-tile; two of them, and the epilogue needs no LDS
 constexpr int WGROUP_M = 8;
 constexpr int W4_MIN_KT = 3;  // K-tiles per tile the continuous ring needs (K >= 192)
 
@@ -70,14 +74,14 @@ __device__ __forceinline__ int w4_perm(int q) {
   return 32 * (j >> 1) + 8 * fh + 4 * (j & 1) + k;
 }
 
-// 256 rows x 128 B = 32 pieces of 8 rows; wave w stages pieces 8w..8w+7 of each operand. Per-lane
-// byte offsets of those 8 pieces (row clamped to the last valid row, chunk source-swizzled; PERM: the
+// 32 NP rows x 128 B = 4 NP pieces of 8 rows; wave w stages pieces NP w .. of each operand. Per-lane
+// byte offsets of those NP pieces (row clamped to the last valid row, chunk source-swizzled; PERM: the
 // weight operand's rows in w4_perm order within each 128-row half).
-template <bool PERM>
-__device__ __forceinline__ void w4_offsets(int ld, int row0, int rows_valid, int wid, int lane, int (&off)[8]) {
+template <bool PERM, int NP>
+__device__ __forceinline__ void w4_offsets(int ld, int row0, int rows_valid, int wid, int lane, int (&off)[NP]) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = (wid * 8 + i) * 8 + (lane >> 3);
+  for (int i = 0; i < NP; ++i) {
+    const int r = (wid * NP + i) * 8 + (lane >> 3);
     const int c = wswz(r, lane & 7);
     int gr = row0 + (PERM ? (r & ~127) + w4_perm(r & 127) : r);
     gr = gr < rows_valid ? gr : rows_valid - 1;
@@ -85,9 +89,10 @@ __device__ __forceinline__ void w4_offsets(int ld, int row0, int rows_valid, int
   }
 }
 
-__device__ __forceinline__ void w4_stage(i32x4 srd, const int (&off)[8], int k0, char* lds, int wid) {
+template <int NP>
+__device__ __forceinline__ void w4_stage(i32x4 srd, const int (&off)[NP], int k0, char* lds, int wid) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) blds16(srd, off[i], k0 * 2, lds + (wid * 8 + i) * 1024);
+  for (int i = 0; i < NP; ++i) blds16(srd, off[i], k0 * 2, lds + (wid * NP + i) * 1024);
 }
 
 __device__ __forceinline__ void w4_barrier() {
@@ -96,15 +101,16 @@ __device__ __forceinline__ void w4_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// fragments of one 32-deep sub-step (prologue only): A rows wr*128 + 16i + fr, B rows wc*128 + 16j + fr
-__device__ __forceinline__ void w4_read(const char* buf, int s, int wr, int wc, int fr, int fh, bf16x8 (&a)[8],
+// fragments of one 32-deep sub-step (prologue only): A rows wr*16*IM + 16i + fr, B rows wc*128 + 16j + fr
+template <int IM>
+__device__ __forceinline__ void w4_read(const char* buf, int s, int wr, int wc, int fr, int fh, bf16x8 (&a)[IM],
                                         bf16x8 (&b)[8]) {
   const char* sa = buf;
-  const char* sb = buf + W_TILE_A;
+  const char* sb = buf + w_tile_a(IM);
   const int c = 4 * s + fh;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int R = wr * 128 + 16 * i + fr;
+  for (int i = 0; i < IM; ++i) {
+    const int R = wr * 16 * IM + 16 * i + fr;
     a[i] = *reinterpret_cast<const bf16x8*>(sa + R * 128 + 16 * wswz(R, c));
   }
 #pragma unroll
@@ -121,14 +127,16 @@ __device__ __forceinline__ void w4_read(const char* buf, int s, int wr, int wc, 
 // epilogue reads (w4_pin_acc below). The weight fragment is srcA and the activation fragment srcB, so
 // the accumulator comes out transposed: lane (fr, fh) of acc[i][j] holds C[16i + fr][4 consecutive
 // output columns] (which ones: w4_perm).
-__device__ __forceinline__ void w4_mfma(f32x4 (&acc)[8][8], const bf16x8 (&a)[8], const bf16x8 (&b)[8], int m) {
+template <int IM>
+__device__ __forceinline__ void w4_mfma(f32x4 (&acc)[IM][8], const bf16x8 (&a)[IM], const bf16x8 (&b)[8], int m) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %2, %1, %0"
                : "+a"(acc[m >> 3][m & 7])
                : "v"(a[m >> 3]), "v"(b[m & 7])
                : "memory");
 }
 // the same with srcC = 0 (first K-tile of a tile: no zeroing pass)
-__device__ __forceinline__ void w4_mfma0(f32x4 (&acc)[8][8], const bf16x8 (&a)[8], const bf16x8 (&b)[8], int m) {
+template <int IM>
+__device__ __forceinline__ void w4_mfma0(f32x4 (&acc)[IM][8], const bf16x8 (&a)[IM], const bf16x8 (&b)[8], int m) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %2, %1, 0"
                : "=a"(acc[m >> 3][m & 7])
                : "v"(a[m >> 3]), "v"(b[m & 7])
@@ -137,10 +145,11 @@ __device__ __forceinline__ void w4_mfma0(f32x4 (&acc)[8][8], const bf16x8 (&a)[8
 
 // Orders every accumulator access after an s_nop pad (>= 16 wait states covers MFMA D -> VALU/DS read
 // and v_accvgpr_write -> MFMA srcC).
-__device__ __forceinline__ void w4_pin_acc(f32x4 (&acc)[8][8]) {
+template <int IM>
+__device__ __forceinline__ void w4_pin_acc(f32x4 (&acc)[IM][8]) {
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 1" ::: "memory");
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < IM; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j])::"memory");
 }
@@ -156,12 +165,12 @@ constexpr bool epi_bias(int e) {
   return e == EPI_BIAS || e == EPI_BIAS_RESID || e == EPI_BIAS_GELU || e == EPI_BIAS_GELU_TANH;
 }
 
-template <int EPI, bool OUT_F32>
+template <int EPI, bool OUT_F32, int IM>
 constexpr int w4_epi_vmem() {
   if constexpr (EPI == EPI_ROPE_KV) return 63;    // loads + stores over the counter's range: the bound clamps
-  if constexpr (epi_pair(EPI)) return 16;  // 8 rows x 2 pairs of 16-B stores
-  if constexpr (OUT_F32) return 64 + (epi_res(EPI) ? 64 : 0) + (epi_bias(EPI) ? 8 : 0);
-  return 32 + (epi_res(EPI) ? 32 : 0) + (epi_bias(EPI) ? 4 : 0);
+  if constexpr (epi_pair(EPI)) return 2 * IM;  // IM rows x 2 pairs of 16-B stores
+  if constexpr (OUT_F32) return 8 * IM + (epi_res(EPI) ? 8 * IM : 0) + (epi_bias(EPI) ? 8 : 0);
+  return 4 * IM + (epi_res(EPI) ? 4 * IM : 0) + (epi_bias(EPI) ? 4 : 0);
 }
 
 template <int EPI>
@@ -181,17 +190,17 @@ __device__ __forceinline__ void unpack4(uint2 v, float (&f)[4]) {
 // Full tile, bf16 output: per row 16i + fr and column pair p (tiles 2p, 2p+1), eight consecutive
 // columns n0 + wc*128 + 32p + 8fh .. +7, one 16-B store (SiLU*up: gate pair (2p, 2p+1), up pair
 // (2p+4, 2p+5), output columns (n0 >> 1) + wc*64 + 32p + 8fh).
-template <int EPI>
-__device__ __forceinline__ void w4_epilogue_full_bf16(const f32x4 (&acc)[8][8], int wr, int wc, int fr, int fh,
+template <int EPI, int IM>
+__device__ __forceinline__ void w4_epilogue_full_bf16(const f32x4 (&acc)[IM][8], int wr, int wc, int fr, int fh,
                                                       int m0, int n0, void* C, int ldc,
                                                       const bf16_t* __restrict__ bias, const bf16_t* resid, int ldr) {
-  const int row0 = m0 + wr * 128 + fr;
+  const int row0 = m0 + wr * 16 * IM + fr;
   bf16_t* Cb = reinterpret_cast<bf16_t*>(C);
   if constexpr (epi_pair(EPI)) {
     const GluPar gp = glu_par<EPI>(bias);
     const int colw = (n0 >> 1) + wc * 64 + 8 * fh;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < IM; ++i) {
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         float o[8];
@@ -214,16 +223,16 @@ __device__ __forceinline__ void w4_epilogue_full_bf16(const f32x4 (&acc)[8][8], 
 #pragma unroll
       for (int p = 0; p < 4; ++p) bv[p] = *reinterpret_cast<const u32x4*>(bias + colw + 32 * p);
     }
-    u32x4 rv[RES ? 32 : 1];
+    u32x4 rv[RES ? 4 * IM : 1];
     if constexpr (RES) {  // the lane's whole residual tile in flight before the first use
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < IM; ++i)
 #pragma unroll
         for (int p = 0; p < 4; ++p)
           rv[4 * i + p] = *reinterpret_cast<const u32x4*>(resid + (size_t)(row0 + 16 * i) * ldr + colw + 32 * p);
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < IM; ++i) {
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
         float o[8];
@@ -259,27 +268,27 @@ __device__ __forceinline__ void w4_epilogue_full_bf16(const f32x4 (&acc)[8][8], 
 // row's slot; v heads: C and the cache. Rows two at a time (cos / sin in registers: 64 values), loads
 // never predicated (rows past M clamp; only the stores are guarded).
 
-template <bool FULL>
-__device__ __forceinline__ void w4_epilogue_rope(const f32x4 (&acc)[8][8], int wr, int wc, int fr, int fh, int m0,
+template <bool FULL, int IM>
+__device__ __forceinline__ void w4_epilogue_rope(const f32x4 (&acc)[IM][8], int wr, int wc, int fr, int fh, int m0,
                                                  int n0, bf16_t* C, int ldc, const RopeKV& rk, int M) {
-  const int row0 = m0 + wr * 128 + fr;
+  const int row0 = m0 + wr * 16 * IM + fr;
   const int hd = (n0 + wc * 128) >> 7;
   const int d0 = 8 * fh;
   const bool isq = hd < rk.Hq, isk = !isq && hd < rk.Hq + rk.Hkv, rot = hd < rk.Hq + rk.Hkv;
   const int kvh = isk ? hd - rk.Hq : hd - rk.Hq - rk.Hkv;
   bf16_t* cache = isk ? rk.kc : rk.vc;
-  int pos[8], slot[8];
+  int pos[IM], slot[IM];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < IM; ++i) {
     const int r = FULL ? row0 + 16 * i : min(row0 + 16 * i, M - 1);
     pos[i] = rk.pos[r];
     slot[i] = rk.slot[r];
   }
 #pragma unroll
-  for (int i2 = 0; i2 < 8; i2 += 2) {
+  for (int i2 = 0; i2 < IM; i2 += 2) {
     u32x4 cv[2][2][2], sv[2][2][2];  // [row][p][half]
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < min(2, IM - i2); ++u)
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         const float* ct = rk.cos_t + (size_t)pos[i2 + u] * 64 + d0 + 32 * p;
@@ -290,7 +299,7 @@ __device__ __forceinline__ void w4_epilogue_rope(const f32x4 (&acc)[8][8], int w
         sv[u][p][1] = *reinterpret_cast<const u32x4*>(st + 4);
       }
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < min(2, IM - i2); ++u) {
       const int i = i2 + u;
       const int gr = row0 + 16 * i;
       float o[4][8];
@@ -330,16 +339,16 @@ __device__ __forceinline__ void w4_epilogue_rope(const f32x4 (&acc)[8][8], int w
 // Per-accumulator epilogue: fp32 outputs (full tiles: 16-B stores) and every edge tile (guarded, any
 // output type). Lane (fr, fh) of acc[i][j] owns columns w4_perm(16j + 4fh) .. +3 of its wave tile.
 // Nout = output columns (packed rows / 2 for SiLU*up).
-template <int EPI, bool OUT_F32, bool FULL>
-__device__ __forceinline__ void w4_epilogue_reg(const f32x4 (&acc)[8][8], int wr, int wc, int fr, int fh, int m0,
+template <int EPI, bool OUT_F32, bool FULL, int IM>
+__device__ __forceinline__ void w4_epilogue_reg(const f32x4 (&acc)[IM][8], int wr, int wc, int fr, int fh, int m0,
                                                 int n0, void* C, int ldc, const bf16_t* __restrict__ bias,
                                                 const bf16_t* resid, int ldr, int M, int Nout) {
-  const int row0 = m0 + wr * 128 + fr;
+  const int row0 = m0 + wr * 16 * IM + fr;
   if constexpr (epi_pair(EPI)) {
     const GluPar gp = glu_par<EPI>(bias);
     const int colw = (n0 >> 1) + wc * 64;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < IM; ++i) {
       const int gr = row0 + 16 * i;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -364,14 +373,14 @@ __device__ __forceinline__ void w4_epilogue_reg(const f32x4 (&acc)[8][8], int wr
         bv[j] = *reinterpret_cast<const uint2*>(bias + (FULL ? gc : min(gc, Nout - 4)));
       }
     }
-    // residual row groups in flight: the whole tile (RD = 8, 128 registers) for the residual-only form;
+    // residual row groups in flight: the whole tile (RD = IM, 16 IM registers) for the residual-only form;
     // one 16-row group at a time with a bias too (the whole tile there made this rarely taken path the
     // loop body's register peak: 22 -> 8 spilled values bf16, 38 -> 0 fp32; the residual-only form
     // spills more, 2 -> 4, when grouped)
-    constexpr int RD = BIAS ? 1 : 8;
+    constexpr int RD = BIAS ? 1 : IM;
     uint2 rv[RES ? 8 * RD : 1];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < IM; ++i) {
       const int gr = row0 + 16 * i;
       if constexpr (RES) {
         if (i % RD == 0) {
@@ -420,13 +429,13 @@ __device__ __forceinline__ void w4_epilogue_reg(const f32x4 (&acc)[8][8], int wr
 }
 
 // ---------------------------------------------------------------------------------------------------
-// K-tile schedule. MFMA m = 8i + j (+ 64 in the second 32-deep sub-step) uses a[i] and b[j]; after MFMA m:
-//   R1 + q * R1_STEP      read q of tile t's second sub-step, q = 0..15
+// K-tile schedule. MFMA m = 8i + j (+ 8 IM in the second 32-deep sub-step) uses a[i] and b[j]; after MFMA m:
+//   R1 + q * R1_STEP      read q of tile t's second sub-step, q = 0..IM + 7
 //   FREE_W / FREE         lgkmcnt(0), barrier: buffer t&1 is read out in every wave
-//   D + q * D_STEP        DMA piece q of tile t+2 into it (activation and weight pieces in turn)
+//   D + q * D_STEP        DMA piece q of tile t+2 into it (activation and weight pieces in turn, then the weight's left over)
 //   LAND_W / LAND         vmcnt(pieces of t+2 issued so far), barrier: tile t+1 is in LDS
 //   F0 + q * F0_STEP      read q of tile t+1's first sub-step
-// Reads go in the order of first use: a[0], b[0..7], a[1..7]. The first sub-step's are waited for row by row at
+// Reads go in the order of first use: a[0], b[0..7], a[1..IM - 1]. The first sub-step's are waited for row by row at
 // the head of the next K-tile (row_wait), so the last of them may be issued late.
 __device__ __forceinline__ void h_read(bf16x8& d, unsigned addr, int off_imm) {
   // off_imm is a compile-time constant at every call site (fully unrolled schedule)
@@ -441,13 +450,15 @@ __device__ __forceinline__ void h_m0(unsigned lds, int off_imm) {
 }
 
 struct W4Sched {
-  int r1, r1_step, free_w, d, d_step, land_w, f0, f0_step;
+  int im, r1, r1_step, free_w, d, d_step, land_w, f0, f0_step;
   constexpr int at(int first, int step, int m) const {  // q if read / piece q follows MFMA m, else -1
-    return m >= first && (m - first) % step == 0 && (m - first) / step < 16 ? (m - first) / step : -1;
+    return m >= first && (m - first) % step == 0 && (m - first) / step < im + 8 ? (m - first) / step : -1;
   }
   constexpr int read1(int m) const { return at(r1, r1_step, m); }
   constexpr int piece(int m) const { return at(d, d_step, m); }
   constexpr int read0(int m) const { return at(f0, f0_step, m); }
+  constexpr bool weight(int q) const { return q >= 2 * im || q & 1; }  // whether piece q is the weight's, and which one
+  constexpr int index(int q) const { return q >= 2 * im ? q - im : q >> 1; }
   constexpr int pieces_before(int m) const {
     int n = 0;
     for (int k = 0; k < m; ++k) n += piece(k) >= 0;
@@ -455,21 +466,25 @@ struct W4Sched {
   }
   // LDS reads that may still be in flight before MFMA m = 8i: all but the first sub-step's first 9 + i
   constexpr int row_wait(int m) const {
-    int n = 16 - (9 + m / 8);
+    int n = im + 8 - (9 + m / 8);
     for (int k = 0; k < m; ++k) n += read1(k) >= 0;
     return n < 15 ? n : 15;
   }
   constexpr bool ok() const {
-    return r1 + 15 * r1_step < free_w && free_w < d && d + 15 * d_step < 128 && free_w < 64 && land_w < f0 &&
-           f0 >= 64 && f0 + 15 * f0_step < 128 && d > 0 && d_step > 1;
+    return r1 + (im + 7) * r1_step < free_w && free_w < d && d + (im + 7) * d_step < 16 * im && free_w < 8 * im &&
+           land_w < f0 && f0 >= 8 * im && f0 + (im + 7) * f0_step < 16 * im && d > 0 && d_step > 1;
   }
 };
-constexpr W4Sched SCH{1, 2, 37, 40, 5, 84, 87, 2};
-static_assert(SCH.ok(), "K-tile schedule");
-constexpr int H_VM = SCH.pieces_before(SCH.land_w);  // DMAs of this K-tile issued before the LAND wait
+template <int IM>
+constexpr W4Sched SCH = IM == 8   ? W4Sched{8, 1, 2, 37, 40, 5, 84, 87, 2}
+                        : IM == 7 ? W4Sched{7, 1, 2, 35, 38, 5, 72, 75, 2}
+                                  : W4Sched{6, 1, 2, 33, 36, 4, 60, 63, 2};
+static_assert(SCH<8>.ok() && SCH<7>.ok() && SCH<6>.ok(), "K-tile schedule");
+template <int IM>
+constexpr int H_VM = SCH<IM>.pieces_before(SCH<IM>.land_w);  // DMAs of this K-tile issued before the LAND wait
 
-template <int Q>
-__device__ __forceinline__ void h_fragment(unsigned ra, unsigned rb, bf16x8 (&a)[8], bf16x8 (&b)[8]) {
+template <int Q, int IM>
+__device__ __forceinline__ void h_fragment(unsigned ra, unsigned rb, bf16x8 (&a)[IM], bf16x8 (&b)[8]) {
   if constexpr (Q == 0) h_read(a[0], ra, 0);
   else if constexpr (Q < 9) h_read(b[Q - 1], rb, (Q - 1) * 2048);
   else h_read(a[Q - 8], ra, (Q - 8) * 2048);
@@ -482,34 +497,37 @@ __device__ __forceinline__ void h_fragment(unsigned ra, unsigned rb, bf16x8 (&a)
 // the caller issues them itself, w4_read_f0). rbA / rbB: this lane's read bases (sub-step s, buffer 0)
 // of the activation / weight fragments; fragment i at + 2048 i (the swizzle of row 16 i + fr does not
 // depend on i).
-template <bool ZERO, int VMW, bool F0 = true>
-__device__ __forceinline__ void w4_ktile(char* smem, int g, i32x4 srd_a, i32x4 srd_b, const int (&sa)[8],
+template <int IM, bool ZERO, int VMW, bool F0 = true>
+__device__ __forceinline__ void w4_ktile(char* smem, int g, i32x4 srd_a, i32x4 srd_b, const int (&sa)[IM],
                                          const int (&sb)[8], int kst, int wid, const unsigned (&rbA)[2],
-                                         const unsigned (&rbB)[2], f32x4 (&acc)[8][8], bf16x8 (&a0)[8],
-                                         bf16x8 (&b0)[8], bf16x8 (&a1)[8], bf16x8 (&b1)[8]) {
-  static_assert(VMW >= H_VM && VMW <= 63, "vmcnt bound");
-  const unsigned cur = (unsigned)(g & 1) * W_BUF, nxt = (unsigned)((g + 1) & 1) * W_BUF;
+                                         const unsigned (&rbB)[2], f32x4 (&acc)[IM][8], bf16x8 (&a0)[IM],
+                                         bf16x8 (&b0)[8], bf16x8 (&a1)[IM], bf16x8 (&b1)[8]) {
+  constexpr W4Sched S = SCH<IM>;
+  static_assert(VMW >= H_VM<IM> && VMW <= 63, "vmcnt bound");
+  const unsigned cur = (unsigned)(g & 1) * w_buf(IM), nxt = (unsigned)((g + 1) & 1) * w_buf(IM);
   const unsigned lds_cur = (unsigned)(unsigned long long)(const __attribute__((address_space(3))) char*)smem + cur;
-  const unsigned dst = __builtin_amdgcn_readfirstlane(lds_cur + wid * 8192);  // weight pieces W_TILE_A further
+  const unsigned dst_a = __builtin_amdgcn_readfirstlane(lds_cur + wid * IM * 1024);
+  const unsigned dst_b = __builtin_amdgcn_readfirstlane(lds_cur + w_tile_a(IM) + wid * 8192);
   const int kb = kst * WBK * 2;
   const unsigned rb1 = rbB[1] + cur, ra1 = rbA[1] + cur, rb0 = rbB[0] + nxt, ra0 = rbA[0] + nxt;
-  static_for<128>([&](auto mc) __attribute__((always_inline)) {
+  static_for<16 * IM>([&](auto mc) __attribute__((always_inline)) {
     constexpr int m = decltype(mc)::value;
-    if constexpr (m % 8 == 0 && m < SCH.free_w)
-      asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(SCH.row_wait(m)) : "memory");
-    if constexpr (m == SCH.free_w) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if constexpr (m == SCH.land_w) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(VMW) : "memory");
-    if constexpr (m == SCH.free_w + 1 || m == SCH.land_w + 1) w4_barrier();
-    if constexpr (m < 64) {
+    if constexpr (m % 8 == 0 && m < S.free_w)
+      asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(S.row_wait(m)) : "memory");
+    if constexpr (m == S.free_w) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if constexpr (m == S.land_w) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(VMW) : "memory");
+    if constexpr (m == S.free_w + 1 || m == S.land_w + 1) w4_barrier();
+    if constexpr (m < 8 * IM) {
       if constexpr (ZERO) w4_mfma0(acc, a0, b0, m);
       else w4_mfma(acc, a0, b0, m);
     } else {
-      w4_mfma(acc, a1, b1, m - 64);
+      w4_mfma(acc, a1, b1, m - 8 * IM);
     }
-    constexpr int q = SCH.piece(m), qn = SCH.piece(m + 1);
-    if constexpr (q >= 0) h_dma(q & 1 ? srd_b : srd_a, q & 1 ? sb[q >> 1] : sa[q >> 1], kb);
-    if constexpr (qn >= 0) h_m0(dst, (qn & 1) * W_TILE_A + (qn >> 1) * 1024);
-    constexpr int r1 = SCH.read1(m), r0 = SCH.read0(m);
+    constexpr int q = S.piece(m), qn = S.piece(m + 1);
+    if constexpr (q >= 0 && S.weight(q)) h_dma(srd_b, sb[S.index(q)], kb);
+    if constexpr (q >= 0 && !S.weight(q)) h_dma(srd_a, sa[S.index(q)], kb);
+    if constexpr (qn >= 0) h_m0(S.weight(qn) ? dst_b : dst_a, S.index(qn) * 1024);
+    constexpr int r1 = S.read1(m), r0 = S.read0(m);
     if constexpr (r1 >= 0) h_fragment<r1>(ra1, rb1, a1, b1);
     if constexpr (F0 && r0 >= 0) h_fragment<r0>(ra0, rb0, a0, b0);
   });
@@ -517,11 +535,12 @@ __device__ __forceinline__ void w4_ktile(char* smem, int g, i32x4 srd_a, i32x4 s
 
 // The first reads of the K-tile in ring slot g & 1, in w4_ktile's order, left in flight for the next
 // w4_ktile's counted waits.
+template <int IM>
 __device__ __forceinline__ void w4_read_f0(int g, const unsigned (&rbA)[2], const unsigned (&rbB)[2],
-                                           bf16x8 (&a0)[8], bf16x8 (&b0)[8]) {
-  const unsigned buf = (unsigned)(g & 1) * W_BUF;
+                                           bf16x8 (&a0)[IM], bf16x8 (&b0)[8]) {
+  const unsigned buf = (unsigned)(g & 1) * w_buf(IM);
   const unsigned rb0 = rbB[0] + buf, ra0 = rbA[0] + buf;
-  static_for<16>([&](auto qc) __attribute__((always_inline)) {
+  static_for<IM + 8>([&](auto qc) __attribute__((always_inline)) {
     h_fragment<decltype(qc)::value>(ra0, rb0, a0, b0);
   });
 }
@@ -529,13 +548,14 @@ __device__ __forceinline__ void w4_read_f0(int g, const unsigned (&rbA)[2], cons
 // Output tile `tile` (of nwg) -> origin. Tiles are numbered so that the 8 XCDs each own a contiguous
 // range (xcd_remap; a persistent block keeps its XCD since the grid is a multiple of 8), grouped
 // WGROUP_M M-tiles deep for L2 reuse of the weight tiles.
-__device__ __forceinline__ void w4_origin(int tile, int nwg, int tiles_m, int tiles_n, int& m0, int& n0) {
+__device__ __forceinline__ void w4_origin(int tile, int nwg, int tiles_m, int tiles_n, int bm, int& m0,
+                                          int& n0) {
   const int logical = xcd_remap(tile, nwg);
   const int group = logical / (WGROUP_M * tiles_n);
   const int first_m = group * WGROUP_M;
   const int gm = min(tiles_m - first_m, WGROUP_M);
   const int in_group = logical % (WGROUP_M * tiles_n);
-  m0 = (first_m + in_group % gm) * WBM;
+  m0 = (first_m + in_group % gm) * bm;
   n0 = (in_group / gm) * WBN;
 }
 
@@ -544,18 +564,19 @@ __device__ __forceinline__ void w4_origin(int tile, int nwg, int tiles_m, int ti
 // writes the fp32 partial tile of slab z to C + z * M * ldc (the consumer, e.g. add_partials_rmsnorm,
 // sums the slabs). For prefill shapes whose tile count fills only ~1.3 waves of the CUs (o_proj / down
 // at M ~ 5k: 336 tiles on 256 CUs), two slabs make 2.6 waves.
-template <int EPI, bool OUT_F32, bool KSPLIT = false>
+template <int EPI, bool OUT_F32, bool KSPLIT, int IM>
 __global__ __launch_bounds__(W4_THREADS, 1) void gemm_w4_kernel(const bf16_t* __restrict__ A, int lda,
                                                                 const bf16_t* __restrict__ B, int ldb, void* C,
                                                                 int ldc, const bf16_t* __restrict__ bias,
                                                                 const bf16_t* resid, int ldr, int M, int N, int K,
                                                                 int nsplit, RopeKV rk) {
-  __shared__ __attribute__((aligned(16))) char smem[W4_LDS];
+  constexpr int BM = 32 * IM, W_BUF = w_buf(IM), W_TILE_A = w_tile_a(IM);
+  __shared__ __attribute__((aligned(16))) char smem[2 * W_BUF];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wid >> 1, wc = wid & 1;
   const int fr = lane & 15, fh = lane >> 4;
-  const int tiles_m = (M + WBM - 1) / WBM, tiles_n = (N + WBN - 1) / WBN;
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + WBN - 1) / WBN;
   const int nwg = tiles_m * tiles_n;
   const int nwt = KSPLIT ? nwg * nsplit : nwg;  // work items
   const int nk = K / WBK;
@@ -565,8 +586,8 @@ __global__ __launch_bounds__(W4_THREADS, 1) void gemm_w4_kernel(const bf16_t* __
   const i32x4 srd_b = make_srd(B, (unsigned)N * (unsigned)ldb * 2u);
 
   // epilogue vector-memory ops younger than the next tile's K-tile-1 DMA at its first vmcnt
-  constexpr int EV = w4_epi_vmem<EPI, OUT_F32>();
-  constexpr int VMH0 = H_VM + EV > 63 ? 63 : H_VM + EV;
+  constexpr int EV = w4_epi_vmem<EPI, OUT_F32, IM>();
+  constexpr int VMH0 = H_VM<IM> + EV > 63 ? 63 : H_VM<IM> + EV;
   // The next tile's F0 fragments are read before the epilogue (in the last K-tile, hidden under its
   // MFMAs) only where the epilogue leaves room for their 64 registers: with the bias, GELU or fp32
   // residual epilogues the allocator spilled them to scratch straight after the asm read issued, i.e.
@@ -578,14 +599,14 @@ __global__ __launch_bounds__(W4_THREADS, 1) void gemm_w4_kernel(const bf16_t* __
   int tile = blockIdx.x;
   int z = KSPLIT ? tile / nwg : 0;
   int m0, n0;
-  w4_origin(tile - z * nwg, nwg, tiles_m, tiles_n, m0, n0);
-  int off_a[8], off_b[8];
+  w4_origin(tile - z * nwg, nwg, tiles_m, tiles_n, BM, m0, n0);
+  int off_a[IM], off_b[8];
   w4_offsets<false>(lda, m0, M, wid, lane, off_a);
   w4_offsets<true>(ldb, n0, N, wid, lane, off_b);
   if constexpr (KSPLIT) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      off_a[i] += z * K * 2;
+      if (i < IM) off_a[i] += z * K * 2;
       off_b[i] += z * K * 2;
     }
   }
@@ -595,7 +616,7 @@ __global__ __launch_bounds__(W4_THREADS, 1) void gemm_w4_kernel(const bf16_t* __
   w4_stage(srd_b, off_b, WBK, smem + W_BUF + W_TILE_A, wid);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): K-tiles 0 and 1 (the first iteration's vmcnt then covers K-tile 2)
   w4_barrier();
-  bf16x8 a0[8], b0[8], a1[8], b1[8];
+  bf16x8 a0[IM], b0[8], a1[IM], b1[8];
   w4_read(smem, 0, wr, wc, fr, fh, a0, b0);
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   __builtin_amdgcn_sched_barrier(0);
@@ -607,20 +628,20 @@ __global__ __launch_bounds__(W4_THREADS, 1) void gemm_w4_kernel(const bf16_t* __
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const unsigned cs = (unsigned)(((4 * s + fh) ^ ((fr >> 1) & 7)) * 16);
-      rbA[s] = l0 + (unsigned)((wr * 128 + fr) * 128) + cs;
+      rbA[s] = l0 + (unsigned)((wr * 16 * IM + fr) * 128) + cs;
       rbB[s] = l0 + W_TILE_A + (unsigned)((wc * 128 + fr) * 128) + cs;
     }
   }
 
-  f32x4 acc[8][8];
+  f32x4 acc[IM][8];
   int g = 0;
   for (;;) {
     const int next = tile + (int)gridDim.x;
     const bool has_next = next < nwt;
-    w4_ktile<true, VMH0>(smem, g, srd_a, srd_b, off_a, off_b, 2, wid, rbA, rbB, acc, a0, b0, a1, b1);
+    w4_ktile<IM, true, VMH0>(smem, g, srd_a, srd_b, off_a, off_b, 2, wid, rbA, rbB, acc, a0, b0, a1, b1);
     ++g;
     for (int t = 1; t + 2 < nk; ++t, ++g)
-      w4_ktile<false, H_VM>(smem, g, srd_a, srd_b, off_a, off_b, t + 2, wid, rbA, rbB, acc, a0, b0, a1, b1);
+      w4_ktile<IM, false, H_VM<IM>>(smem, g, srd_a, srd_b, off_a, off_b, t + 2, wid, rbA, rbB, acc, a0, b0, a1, b1);
     // The last two iterations stage (and read the first fragments of) the next tile; on the block's
     // last tile they re-stage this tile's K-tiles 0 / 1 instead (valid addresses, never read), so both
     // cases run the same straight-line code: a branch around the MFMA iterations made the register
@@ -628,7 +649,7 @@ __global__ __launch_bounds__(W4_THREADS, 1) void gemm_w4_kernel(const bf16_t* __
     int nm0, nn0;
     const int ntile = has_next ? next : tile;
     const int nz = KSPLIT ? ntile / nwg : 0;
-    w4_origin(ntile - nz * nwg, nwg, tiles_m, tiles_n, nm0, nn0);
+    w4_origin(ntile - nz * nwg, nwg, tiles_m, tiles_n, BM, nm0, nn0);
     {
       int ln;  // == lane; opaque so the lane-only offset math is not hoisted out of the loop
       asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
@@ -638,33 +659,33 @@ __global__ __launch_bounds__(W4_THREADS, 1) void gemm_w4_kernel(const bf16_t* __
       if constexpr (KSPLIT) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          off_a[i] += nz * K * 2;
+          if (i < IM) off_a[i] += nz * K * 2;
           off_b[i] += nz * K * 2;
         }
       }
     }
-    w4_ktile<false, H_VM>(smem, g, srd_a, srd_b, off_a, off_b, 0, wid, rbA, rbB, acc, a0, b0, a1, b1);
+    w4_ktile<IM, false, H_VM<IM>>(smem, g, srd_a, srd_b, off_a, off_b, 0, wid, rbA, rbB, acc, a0, b0, a1, b1);
     ++g;
-    w4_ktile<false, H_VM, !LATE_F0>(smem, g, srd_a, srd_b, off_a, off_b, 1, wid, rbA, rbB, acc, a0, b0, a1, b1);
+    w4_ktile<IM, false, H_VM<IM>, !LATE_F0>(smem, g, srd_a, srd_b, off_a, off_b, 1, wid, rbA, rbB, acc, a0, b0, a1, b1);
     ++g;
     // the epilogue is compiler-scheduled code: it may move any register, so no asm read is in flight
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     w4_pin_acc(acc);
     void* Cz = KSPLIT ? (void*)(reinterpret_cast<float*>(C) + (size_t)z * M * ldc) : C;
     if constexpr (EPI == EPI_ROPE_KV) {
-      if (m0 + WBM <= M) {
-        w4_epilogue_rope<true>(acc, wr, wc, fr, fh, m0, n0, reinterpret_cast<bf16_t*>(Cz), ldc, rk, M);
+      if (m0 + BM <= M) {
+        w4_epilogue_rope<true, IM>(acc, wr, wc, fr, fh, m0, n0, reinterpret_cast<bf16_t*>(Cz), ldc, rk, M);
       } else {
-        w4_epilogue_rope<false>(acc, wr, wc, fr, fh, m0, n0, reinterpret_cast<bf16_t*>(Cz), ldc, rk, M);
+        w4_epilogue_rope<false, IM>(acc, wr, wc, fr, fh, m0, n0, reinterpret_cast<bf16_t*>(Cz), ldc, rk, M);
         __builtin_amdgcn_s_waitcnt(0x0F70);  // guarded: count unknown, drain (the next K-tile 1 lands too)
       }
-    } else if (m0 + WBM <= M && n0 + WBN <= N) {
+    } else if (m0 + BM <= M && n0 + WBN <= N) {
       if constexpr (OUT_F32)
-        w4_epilogue_reg<EPI, true, true>(acc, wr, wc, fr, fh, m0, n0, Cz, ldc, bias, resid, ldr, M, Nout);
+        w4_epilogue_reg<EPI, true, true, IM>(acc, wr, wc, fr, fh, m0, n0, Cz, ldc, bias, resid, ldr, M, Nout);
       else
-        w4_epilogue_full_bf16<EPI>(acc, wr, wc, fr, fh, m0, n0, Cz, ldc, bias, resid, ldr);
+        w4_epilogue_full_bf16<EPI, IM>(acc, wr, wc, fr, fh, m0, n0, Cz, ldc, bias, resid, ldr);
     } else {
-      w4_epilogue_reg<EPI, OUT_F32, false>(acc, wr, wc, fr, fh, m0, n0, Cz, ldc, bias, resid, ldr, M, Nout);
+      w4_epilogue_reg<EPI, OUT_F32, false, IM>(acc, wr, wc, fr, fh, m0, n0, Cz, ldc, bias, resid, ldr, M, Nout);
       __builtin_amdgcn_s_waitcnt(0x0F70);  // guarded: count unknown, drain (the next K-tile 1 lands too)
     }
     // epilogue accumulator reads -> the next tile's srcC = 0 MFMA writes
@@ -682,7 +703,7 @@ __global__ __launch_bounds__(W4_THREADS, 1) void gemm_w4_kernel(const bf16_t* __
   }
 }
 
-// Persistent grid: one block per CU (the kernel holds 128 KiB of LDS and 4 waves x 512 registers,
+// Persistent grid: one block per CU (the kernel holds 112 to 128 KiB of LDS and 4 waves x 512 registers,
 // so a CU never runs two), rounded down to a multiple of 8 so a block keeps its XCD across tiles.
 // ragk_gemm_w4_set_grid(n > 0) caps the grid at n (tests: many tiles per block), 0 = one block per tile.
 static int g_w4_grid = -1;
@@ -697,14 +718,23 @@ static int w4_grid(int nwg) {
   return (g_w4_grid == 0 || g_w4_grid >= nwg) ? nwg : g_w4_grid;
 }
 
-template <int EPI, bool F32>
-int launch_w4(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias, const void* resid,
-              int ldr, int M, int N, int K, hipStream_t st) {
-  const int nwg = ((M + WBM - 1) / WBM) * ((N + WBN - 1) / WBN);
-  hipLaunchKernelGGL((gemm_w4_kernel<EPI, F32>), dim3(w4_grid(nwg)), dim3(W4_THREADS), 0, st, (const bf16_t*)A, lda,
-                     (const bf16_t*)B, ldb, C, ldc, (const bf16_t*)bias, (const bf16_t*)resid, ldr, M, N, K, 1,
-                     RopeKV{});
+template <int IM, int EPI, bool F32, bool KSPLIT = false>
+int launch_w4_rows(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias, const void* resid,
+                   int ldr, int M, int N, int K, int nsplit, hipStream_t st, const RopeKV& rk) {
+  const int nwg = ((M + 32 * IM - 1) / (32 * IM)) * ((N + WBN - 1) / WBN);
+  hipLaunchKernelGGL((gemm_w4_kernel<EPI, F32, KSPLIT, IM>), dim3(w4_grid(nwg * nsplit)), dim3(W4_THREADS), 0, st,
+                     (const bf16_t*)A, lda, (const bf16_t*)B, ldb, C, ldc, (const bf16_t*)bias, (const bf16_t*)resid, ldr, M,
+                     N, K, nsplit, rk);
   return (int)hipGetLastError();
+}
+
+template <int EPI, bool F32>
+int launch_w4(int im, const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias, const void* resid,
+              int ldr, int M, int N, int K, hipStream_t st, const RopeKV& rk = RopeKV{}) {
+  if (im == 8) return launch_w4_rows<8, EPI, F32>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, 1, st, rk);
+  if (im == 7) return launch_w4_rows<7, EPI, F32>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, 1, st, rk);
+  if (im == 6) return launch_w4_rows<6, EPI, F32>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, 1, st, rk);
+  return (int)hipErrorInvalidValue;
 }
 
 }  // namespace
@@ -717,9 +747,9 @@ RAGK_API int ragk_gemm_w4_set_grid(int g) {
 }
 
 // N = output columns (for EPI_SILU_MUL the weight has 2N rows, N % 128 == 0). Requires K % 64 == 0 and
-// K >= 192 (three K-tiles per tile for the continuous ring).
-RAGK_API int ragk_gemm_w4(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias,
-                          const void* resid, int ldr, int M, int N, int K, int epi, int out_f32, hipStream_t st) {
+// K >= 192 (three K-tiles per tile for the continuous ring). im = rows of a tile / 32 (8, 7 or 6).
+RAGK_API int ragk_gemm_w4_tile(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias,
+                          const void* resid, int ldr, int M, int N, int K, int epi, int out_f32, int im, hipStream_t st) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   if (K % WBK != 0 || K / WBK < W4_MIN_KT) return (int)hipErrorInvalidValue;
   const long long rows_b = epi_pair(epi) ? 2LL * N : (long long)N;
@@ -727,17 +757,17 @@ RAGK_API int ragk_gemm_w4(const void* A, int lda, const void* B, int ldb, void* 
     return (int)hipErrorInvalidValue;  // 32-bit buffer offsets
   if (epi == EPI_SILU_MUL) {
     if (N % 128 != 0 || out_f32) return (int)hipErrorInvalidValue;
-    return launch_w4<EPI_SILU_MUL, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, 2 * N, K, st);
+    return launch_w4<EPI_SILU_MUL, false>(im, A, lda, B, ldb, C, ldc, bias, resid, ldr, M, 2 * N, K, st);
   }
   if (epi == EPI_GLU_CLIP) {
     if (N % 128 != 0 || out_f32 || !bias) return (int)hipErrorInvalidValue;
-    return launch_w4<EPI_GLU_CLIP, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, 2 * N, K, st);
+    return launch_w4<EPI_GLU_CLIP, false>(im, A, lda, B, ldb, C, ldc, bias, resid, ldr, M, 2 * N, K, st);
   }
   if (N % 8 != 0) return (int)hipErrorInvalidValue;
 #define RAGK_W4_CASE(E) \
   case E:               \
-    return out_f32 ? launch_w4<E, true>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st) \
-                   : launch_w4<E, false>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
+    return out_f32 ? launch_w4<E, true>(im, A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st) \
+                   : launch_w4<E, false>(im, A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, st);
   switch (epi) {
     RAGK_W4_CASE(EPI_NONE)
     RAGK_W4_CASE(EPI_BIAS)
@@ -752,6 +782,11 @@ RAGK_API int ragk_gemm_w4(const void* A, int lda, const void* B, int ldb, void* 
 #undef RAGK_W4_CASE
 }
 
+RAGK_API int ragk_gemm_w4(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias,
+                          const void* resid, int ldr, int M, int N, int K, int epi, int out_f32, hipStream_t st) {
+  return ragk_gemm_w4_tile(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, epi, out_f32, 8, st);
+}
+
 // Split-K prefill GEMM into fp32 slabs: P[z][M][N] = A[:, z*Ks:(z+1)*Ks] . B[:, z*Ks:(z+1)*Ks]^T,
 // Ks = K / nsplit, one persistent launch over nsplit x tiles work items (see KSPLIT).
 RAGK_API int ragk_gemm_w4_splitk(const void* A, int lda, const void* B, int ldb, float* P, int M, int N, int K,
@@ -760,11 +795,7 @@ RAGK_API int ragk_gemm_w4_splitk(const void* A, int lda, const void* B, int ldb,
   if (nsplit < 1 || K % nsplit || (K / nsplit) % WBK || (K / nsplit) / WBK < W4_MIN_KT || N % 8 || !P)
     return (int)hipErrorInvalidValue;
   if ((long long)M * lda * 2 >= (1LL << 31) || (long long)N * ldb * 2 >= (1LL << 31)) return (int)hipErrorInvalidValue;
-  const int nwg = ((M + WBM - 1) / WBM) * ((N + WBN - 1) / WBN);
-  hipLaunchKernelGGL((gemm_w4_kernel<EPI_NONE, true, true>), dim3(w4_grid(nwg * nsplit)), dim3(W4_THREADS), 0, st,
-                     (const bf16_t*)A, lda, (const bf16_t*)B, ldb, (void*)P, N, nullptr, nullptr, 0, M, N, K / nsplit,
-                     nsplit, RopeKV{});
-  return (int)hipGetLastError();
+  return launch_w4_rows<8, EPI_NONE, true, true>(A, lda, B, ldb, P, N, nullptr, nullptr, 0, M, N, K / nsplit, nsplit, st, RopeKV{});
 }
 
 // qkv = A . B^T (B = [(Hq + 2 Hkv) * 128][K]) with rope_kv's work in the epilogue (EPI_ROPE_KV above): q and
@@ -772,15 +803,12 @@ RAGK_API int ragk_gemm_w4_splitk(const void* A, int lda, const void* B, int ldb,
 // kc / vc [blocks][Hkv][BS][128] at slot[M] (slot < 0: not cached). Same conditions as ragk_gemm_w4.
 RAGK_API int ragk_gemm_w4_rope_kv(const void* A, int lda, const void* B, int ldb, void* C, int ldc, int M, int K,
                                   const int* pos, const int* slot, const float* cos_t, const float* sin_t, void* kc,
-                                  void* vc, int Hq, int Hkv, int BS, hipStream_t st) {
+                                  void* vc, int Hq, int Hkv, int BS, int im, hipStream_t st) {
   if (M <= 0) return 0;
   const int N = (Hq + 2 * Hkv) * 128;
   if (K % WBK != 0 || K / WBK < W4_MIN_KT || Hq < 1 || Hkv < 1 || BS < 1 || N % WBN != 0) return (int)hipErrorInvalidValue;
   if (!pos || !slot || !cos_t || !sin_t || !kc || !vc || ldc % 8 != 0) return (int)hipErrorInvalidValue;
   if ((long long)M * lda * 2 >= (1LL << 31) || (long long)N * ldb * 2 >= (1LL << 31)) return (int)hipErrorInvalidValue;
-  const int nwg = ((M + WBM - 1) / WBM) * (N / WBN);
   const RopeKV rk{pos, slot, cos_t, sin_t, (bf16_t*)kc, (bf16_t*)vc, Hq, Hkv, BS};
-  hipLaunchKernelGGL((gemm_w4_kernel<EPI_ROPE_KV, false>), dim3(w4_grid(nwg)), dim3(W4_THREADS), 0, st,
-                     (const bf16_t*)A, lda, (const bf16_t*)B, ldb, C, ldc, nullptr, nullptr, 0, M, N, K, 1, rk);
-  return (int)hipGetLastError();
+  return launch_w4<EPI_ROPE_KV, false>(im, A, lda, B, ldb, C, ldc, nullptr, nullptr, 0, M, N, K, st, rk);
 }

@@ -162,8 +162,8 @@ def gemm_rope_kv(x, w, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, Hkv
              out.data_ptr() + r0 * out.stride(0) * 2, out.stride(0), r1 - r0, K, positions.data_ptr() + 4 * r0,
              slots.data_ptr() + 4 * r0, cos_t.data_ptr(), sin_t.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), Hq, Hkv,
              k_cache.shape[2])
-        if mi == 0:
-            check(L.ragk_gemm_w4_rope_kv(*a, stream_ptr()), "ragk_gemm_w4_rope_kv")
+        if mi in W4_TILES:
+            check(L.ragk_gemm_w4_rope_kv(*a, mi & 15 or 8, stream_ptr()), "ragk_gemm_w4_rope_kv")
         else:
             ws = torch.empty(S * (r1 - r0) * N, dtype=torch.float32, device=x.device) if S > 1 else None
             check(L.ragk_gemm_mid_rope_kv(*a, mi, S, ptr(ws), stream_ptr()), "ragk_gemm_mid_rope_kv")
@@ -286,7 +286,7 @@ def gemm_mid(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, m
     M, K = x.shape
     N = w.shape[0] // 2 if epi in PAIR_EPI else w.shape[0]
     x, w = _tile_rows(x, w)
-    _req(mi in MID_US and 1 <= S <= K // 64 and K % 64 == 0 and w.shape[1] == K, "gemm_mid tile or split")
+    _req(mi in MID_TILES and 1 <= S <= K // 64 and K % 64 == 0 and w.shape[1] == K, "gemm_mid tile or split")
     _req(out.shape == (M, N) and out.stride(1) == 1, "gemm_mid out")
     _gemm_rows(x, w, bias, resid, epi, out, out_f32, 0, M, mi, S)
     return out
@@ -305,7 +305,7 @@ def _tile_rows(x, w):
 
 
 def _gemm_rows(x, w, bias, resid, epi, out, out_f32, r0, r1, mi, S):
-    """Rows r0 .. r1 of gemm() on gemm_mid (mi > 0) or gemm_w4 (mi == 0); operands checked by the caller."""
+    """Rows r0 .. r1 of gemm() on gemm_mid's or gemm_w4's tile mi; operands checked by the caller."""
     M, K = r1 - r0, x.shape[1]
     N = w.shape[0] // 2 if epi in PAIR_EPI else w.shape[0]
     ldx, ldo = x.stride(0), out.stride(0)
@@ -313,42 +313,46 @@ def _gemm_rows(x, w, bias, resid, epi, out, out_f32, r0, r1, mi, S):
     px, po = x.data_ptr() + r0 * ldx * 2, out.data_ptr() + r0 * ldo * out.element_size()
     pr = resid.data_ptr() + r0 * ldr * 2 if resid is not None else None
     args = (px, ldx, w.data_ptr(), w.stride(0), po, ldo, ptr(bias), pr, ldr, M, N, K, EPI[epi], int(out_f32))
-    if mi == 0:
-        check(_lib.lib().ragk_gemm_w4(*args, stream_ptr()), "ragk_gemm_w4")
+    if mi in W4_TILES:
+        check(_lib.lib().ragk_gemm_w4_tile(*args, mi & 15 or 8, stream_ptr()), "ragk_gemm_w4_tile")
         return
     ws = torch.empty(S * M * w.shape[0], dtype=torch.float32, device=x.device) if S > 1 else None
     check(_lib.lib().ragk_gemm_mid(*args, mi, S, ptr(ws), stream_ptr()), "ragk_gemm_mid")
 
 
 # Microseconds that one 64-deep K-tile of an output tile takes with few blocks running, and what a full machine adds
-# (clocks, L2): tiles of gemm_mid by rows / 32 (+ 16: of 256 columns, not 128), 0 = gemm_w4's 256 x 256; then those of a
-# launch and of a tile's epilogue. Fitted
-# to every tile and split of 20 weights (384 to 28672 rows, K 384 to 14336) at 65 .. 32768 rows of x on two cards, for the
-# choices that follow: they take 0.5 % more than the best launch in the mean, 4 % in one of twenty. (An earlier fit, with 0.25
-# added at 160 rows and one us for either epilogue, took the next tile up there: 1 and 8 %, and 12 % more than gemm_w4 alone at
-# 2600 x 4096 x 14336.) 224 x 128 and 160 x 256 were fitted to 46 products of 90 .. 8000 rows later: with them the choices take
-# 3 % less in the mean, 20 % less at best (600 x 4096 x 14336), and 0.3 % more than the best launch.
-MID_US = {3: (0.27, 0.13), 4: (0.34, 0.15), 5: (0.40, 0.17), 6: (0.49, 0.17), 7: (0.54, 0.21), 8: (0.62, 0.21), 21: (0.76, 0.20)}
-W4_US = (1.01, 0.29)
+# (clocks, L2). Tiles of gemm_mid by rows / 32 (+ 16: of 256 columns, not 128), gemm_w4's by 32 + rows / 32 (always 256 columns),
+# its 256 x 256 as 0; below, those of a launch and of a tile's epilogue. Fitted to every tile and split of 20 weights (384 to
+# 28672 rows, K 384 to 14336) at 65 .. 32768 rows of x on two cards, for the choices that follow: they take 0.5 % more than the
+# best launch in the mean, 4 % in one of twenty. (An earlier fit, with 0.25 added at 160 rows and one us for either epilogue, took
+# the next tile up there: 1 and 8 %, and 12 % more than gemm_w4 alone at 2600 x 4096 x 14336.) 224 x 128 and 160 x 256 were fitted
+# later to 46 products of 90 .. 8000 rows: with them the choices take 3 % less in the mean, 20 % less at best (600 x 4096 x
+# 14336). gemm_w4's three to 166 of 66 .. 16000 rows (0.4 % over the best launch in the mean): on a full
+# machine all of them reach the same 1.35 to 1.45 PFLOP/s, so what decides is the last round, and the epilogue where K is short.
+MID_US = {3: (0.27, 0.13), 4: (0.34, 0.15), 5: (0.40, 0.17), 6: (0.49, 0.17), 7: (0.54, 0.21), 8: (0.62, 0.21), 21: (0.76, 0.20),
+          38: (0.72, 0.39), 39: (0.84, 0.42), 0: (0.87, 0.55)}
+W4_TILES = (0, 38, 39)
+W4_SPLIT_US = (1.01, 0.29)  # gemm_w4 writing fp32 slabs (256 rows a tile only)
+MID_TILES = tuple(mi for mi in MID_US if mi not in W4_TILES)
 LAUNCH_US = (4.5, 1.75)
-W4_LAUNCH_US = (5.25, 4.25)
+W4_LAUNCH_US = (5.25, {0: 4.25, 38: 2.0, 39: 2.6})
 SLAB_US = 8 / 5e6  # one fp32 slab value written and read back
 
 
 def _tiles_us(M, rows, K, mi, S, cus):
     """Model time of one launch: rounds of tiles over the CUs, each K-tiles long plus an epilogue."""
-    bm, bn = (32 * (mi & 15), 256 if mi & 16 else 128) if mi else (256, 256)
+    bm, bn = 32 * (mi & 15 or 8), 128 if 0 < mi < 16 else 256
     items = -(-M // bm) * -(-rows // bn) * S
     rounds = -(-items // cus)
-    a, b = MID_US[mi] if mi else W4_US
-    launch, epilogue = LAUNCH_US if mi else W4_LAUNCH_US
+    a, b = W4_SPLIT_US if mi == 0 and S > 1 else MID_US[mi]
+    launch, epilogue = (W4_LAUNCH_US[0], W4_LAUNCH_US[1][mi]) if mi in W4_TILES else LAUNCH_US
     return launch + rounds * (-(-(K // 64) // S) * (a + b * items / (rounds * cus)) + epilogue)
 
 
 def _mid_best(M, rows, K, cus, slab_us, launch_us, even=False):
     """(time, mi, S) of the best gemm_mid launch; a split costs launch_us and slab_us per slab value (even: equal slabs)."""
     best = (float("inf"), 0, 1)
-    for mi in MID_US:
+    for mi in MID_TILES:
         for S in range(1, 17):
             if S > 1 and K // 64 // S < 4:
                 break
@@ -361,10 +365,10 @@ def _mid_best(M, rows, K, cus, slab_us, launch_us, even=False):
 
 @functools.lru_cache(maxsize=4096)
 def gemm_plan(M, rows, K, w4, cus):
-    """Launches of one product with M > 64 rows: [(first row, end, mi, S)], mi as in _tiles_us. Candidates: gemm_mid alone;
-    gemm_w4 alone (w4: its operands fit); gemm_w4 on as many rows as fill whole rounds of its tiles and gemm_mid on the
-    rest. Where they meet (us, N = K = 4096): 300 rows 24 against gemm_w4's 69, 1777 rows 54 against 79; at N = 28672 of
-    1777 rows gemm_w4 329 against 365 (its 128 x 128 wave tiles read less LDS per MFMA)."""
+    """Launches of one product with M > 64 rows: [(first row, end, mi, S)], mi as in MID_US. Candidates: gemm_mid alone;
+    gemm_w4 alone (w4: its operands fit), at 256, 224 or 192 rows a tile; its 256-row tiles on as many rows as fill whole rounds
+    and gemm_mid on the rest. Where they meet (us, N = K = 4096): 300 rows 24 against gemm_w4's 69, 1777 rows 53 against 66 (192
+    rows a tile); at N = 28672 of 1777 rows gemm_w4 322 against 350 (its wave tiles read less LDS per MFMA)."""
     t, mi, S = _mid_best(M, rows, K, cus, SLAB_US, 3.0)
     plan = ((0, M, mi, S),)
     if not w4 or K % 64 or K < 192:  # gemm_w4's ring needs three K-tiles
@@ -384,6 +388,10 @@ def gemm_plan(M, rows, K, w4, cus):
         # 1.05 of it (827 x 28672 x 4096 188 us against 180), the others 0.69 to 1.02, 0.88 in the mean
         if t2 < 0.96 * t:
             t, plan = t2, ((0, m1, 0, 1), (m1, M, mi, S))
+    # its smaller tiles; against two launches only well ahead (14076 x 4096 x 4096: both ways 343 us, modelled 0.985)
+    t3, mi = min((_tiles_us(M, rows, K, mi, 1, cus), mi) for mi in W4_TILES[1:])
+    if t3 < (0.97 if len(plan) > 1 else 1) * t:
+        plan = ((0, M, mi, 1),)
     return plan
 
 
@@ -594,7 +602,7 @@ def slab_count(M, N, K):
 @functools.lru_cache(maxsize=4096)
 def _splitk_tile(M, N, K, nsplit, cus):
     """(gemm_mid's tile, whether gemm_w4 is ahead of it) for nsplit slabs."""
-    t, mi = min((_tiles_us(M, N, K, m, nsplit, cus), m) for m in MID_US)
+    t, mi = min((_tiles_us(M, N, K, m, nsplit, cus), m) for m in MID_TILES)
     return mi, _tiles_us(M, N, K, 0, nsplit, cus) < t
 
 

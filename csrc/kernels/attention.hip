@@ -336,6 +336,189 @@ __global__ __launch_bounds__(NWV * 64, 8 / NWV) void attn_prefill_kernel(Prefill
   }
 }
 
+// ------------------------------------------------------------------------------------
+// Encoder attention (bidirectional, K / V rows beside each other in a packed qkv buffer; D 32 and 64).
+// A 64-key tile of 32 queries is 32 exponentials a lane (8 clocks of a SIMD each, measured) and some 125 other vector instructions
+// (fma, sum, maximum, conversion), against 8 D of 32x32x16 MFMA clocks: the vector unit bounds it. So a wave takes one column
+// block of 32 queries, a lane pair each: the maximum is one lane swap a tile, the sum stays in the lane until the end. 32x32x16
+// products hold the issue port 8 of their 32 clocks (16x16x32: 8 of 16); K / V addresses are scalar and a tile's buffer is known
+// when compiling. Four waves a SIMD share the two units: the vector one is busy 75 % of the time, the matrix one 46 %.
+// 12 sequences of 13764 rows, 16 heads of 64: 110 -> 93 us (0.73 us a tile and wave), 64 sequences of 1344 rows 659, one sequence
+// of 1330 25 -> 23; 256 of up to 60 rows, 12 heads of 32: 17.1 -> 16.5. Wave priorities around the products changed nothing;
+// looking for the maximum only where a sum outgrows 2^8 takes 20 instructions off, but the scores computed again beside it cost
+// the fourth wave (94 us). Other head sizes, grouped heads and unaligned rows stay on attn_prefill_kernel.
+// Layouts as in attn_prefill_v3_kernel; V rows are swizzled by pairs of 32-B granules (a transposed read takes four rows of two
+// granules from each half of the banks).
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+
+template <int D>
+__device__ __forceinline__ int vswz32(int row) {
+  return D == 64 ? 4 * ((row >> 1) & 1) : 0;
+}
+
+template <int D>
+__global__ __launch_bounds__(256, 3) void attn_encoder_kernel(PrefillArgs a) {
+  using C = Cfg<D>;
+  constexpr int KS = D / 16, DB = D / 32, PPW = C::PIECES / 4;  // MFMA steps over d, 32-wide blocks of d, DMA pieces a wave
+  __shared__ __attribute__((aligned(16))) char smem[4 * C::TILEB];  // [buf][K | V]
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 31, h = lane >> 5, i16 = lane & 15;
+  int tix, head;
+  prefill_block(a, tix, head);
+  const int seq = a.tiles[2 * tix], q_start = a.tiles[2 * tix + 1];
+  const int q_off = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_off;
+  const int kv_len = a.kv_lens[seq], n_kt = (kv_len + KT - 1) / KT;
+  const int qi = q_start + wid * 32 + n;  // this lane's query
+
+  bf16x8 qf[KS];
+  {
+    const bf16_t* qp = a.q + (size_t)(q_off + min(qi, q_len - 1)) * a.q_stride + head * D + 8 * h;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qp + 16 * s);
+  }
+  // waited for here: left to the compiler, its waits stand at the uses, inside the loop, and wait for the tile's DMAs too
+#pragma unroll
+  for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));
+
+  // per-lane source offsets of the wave's pieces, from the tile's first row
+  const int ldb = a.kv_stride * 2;
+  int prow[PPW], koff[PPW], voff[PPW], kch[PPW], vch[PPW];
+#pragma unroll
+  for (int i = 0; i < PPW; ++i) {
+    const int row = (wid * PPW + i) * C::RPP + lane / C::NC, ph = lane % C::NC;
+    prow[i] = row;
+    kch[i] = 16 * (ph ^ kswz<D>(row));
+    vch[i] = 16 * (ph ^ vswz32<D>(row));
+    koff[i] = row * ldb + kch[i];
+    voff[i] = row * ldb + vch[i];
+  }
+  const size_t kv0 = (size_t)a.cu_kv[seq] * a.kv_stride + head * D;
+  const unsigned lds0 = __builtin_amdgcn_readfirstlane(lds_addr(smem));
+  auto stage = [&](int kt) {
+    const size_t at = kv0 + (size_t)kt * KT * a.kv_stride;
+    const i32x4 srd_k = make_srd(a.k + at, 0x7fffffffu), srd_v = make_srd(a.v + at, 0x7fffffffu);
+    if ((kt + 1) * KT > kv_len) {  // rows past the end read the last one: their scores are masked
+      const int last = kv_len - 1 - kt * KT;
+#pragma unroll
+      for (int i = 0; i < PPW; ++i) {
+        koff[i] = min(prow[i], last) * ldb + kch[i];
+        voff[i] = min(prow[i], last) * ldb + vch[i];
+      }
+    }
+    const unsigned dst = lds0 + (kt & 1) * 2 * C::TILEB + wid * PPW * 1024;
+#pragma unroll
+    for (int i = 0; i < PPW; ++i) {
+      blds16_asm(srd_k, koff[i], 0, dst + i * 1024);
+      blds16_asm(srd_v, voff[i], 0, dst + C::TILEB + i * 1024);
+    }
+  };
+
+  // fragment reads: the swizzles of rows 32 kb + n and 16 ks + 4 h + .. do not depend on kb and ks
+  int kat[KS], vat[DB][2];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) kat[s] = n * C::ROWB + 16 * ((2 * s + h) ^ kswz<D>(n));
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int row = 4 * h + (i16 >> 2) + 8 * u, chunk = 2 * (2 * db + ((lane >> 4) & 1)) + ((i16 >> 1) & 1);
+      vat[db][u] = C::TILEB + row * C::ROWB + 16 * (chunk ^ vswz32<D>(row)) + 8 * (i16 & 1);
+    }
+
+  f32x16 o[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[db][e] = 0.f;
+  // mref: the maximum that the exponents are taken against (0 while every score was -inf), move: the score that moves it
+  float l_i = 0.f, mref = 0.f, move = -INFINITY;
+  bool none = true;
+  const float c = a.scale_log2;
+
+  auto tile_step = [&](int kt, auto buf_tag) __attribute__((always_inline)) {
+    const char* tile = smem + decltype(buf_tag)::value * 2 * C::TILEB;
+    if (kt + 1 < n_kt) stage(kt + 1);  // into the buffer that every wave has read out
+    f32x16 s[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[kb][e] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(tile + kat[ks] + kb * 32 * C::ROWB);
+        s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[kb], 0, 0, 0);
+      }
+    // softmax as in attn_prefill_kernel: maximum of the raw scores, deferred rescale
+    if ((kt + 1) * KT > kv_len) {
+      const int left = kv_len - kt * KT - 4 * h;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (32 * kb + 8 * (e >> 2) + (e & 3) >= left) s[kb][e] = -INFINITY;
+    }
+    float mx = s[0][0];
+#pragma unroll
+    for (int e = 1; e < 32; ++e) mx = fmaxf(mx, s[e >> 4][e & 15]);
+    const float mxs = max_xor32(mx) * c;
+    if (__builtin_amdgcn_ballot_w64(mxs > move)) {
+      if (mxs > move) {
+        const float alpha = none ? 0.f : __builtin_amdgcn_exp2f(mref - mxs);
+        none = false;
+        mref = mxs;
+        move = mxs + RESCALE_LOG2;
+        l_i *= alpha;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) o[db] *= alpha;
+      }
+    }
+    float ls[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][e], c, -mref));
+        s[kb][e] = p;
+        ls[kb] = e ? ls[kb] + p : p;
+      }
+    l_i += ls[0] + ls[1];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      u32x4 pw;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pw[j] = pk2bf(s[ks >> 1][8 * (ks & 1) + 2 * j], s[ks >> 1][8 * (ks & 1) + 2 * j + 1]);
+      const bf16x8 pb = __builtin_bit_cast(bf16x8, pw);
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        const bf16x4 v0 = tr_read(tile + vat[db][0] + ks * 16 * C::ROWB), v1 = tr_read(tile + vat[db][1] + ks * 16 * C::ROWB);
+        const bf16x8 vf = (bf16x8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pb, o[db], 0, 0, 0);
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  if (n_kt > 0) stage(0);
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  for (int kt = 0; kt < n_kt; kt += 2) {  // the buffer of a tile is known when compiling: no address arithmetic
+    tile_step(kt, std::integral_constant<int, 0>{});
+    if (kt + 1 < n_kt) tile_step(kt + 1, std::integral_constant<int, 1>{});
+  }
+
+  l_i += __shfl_xor(l_i, 32, 64);
+  const float inv = l_i > 0.f ? 1.f / l_i : 0.f;
+  if (qi < q_len) {
+    bf16_t* op = a.out + (size_t)(q_off + qi) * a.out_stride + head * D + 4 * h;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        *reinterpret_cast<uint2*>(op + 32 * db + 8 * b) =
+            make_uint2(pk2bf(o[db][4 * b] * inv, o[db][4 * b + 1] * inv), pk2bf(o[db][4 * b + 2] * inv, o[db][4 * b + 3] * inv));
+  }
+}
+
 template <typename F, int... Is>
 __device__ __forceinline__ void pp_static_for_impl(F&& f, std::integer_sequence<int, Is...>) {
   (f(std::integral_constant<int, Is>{}), ...);
@@ -372,7 +555,6 @@ __device__ __forceinline__ void pp_static_for(F&& f) {
 // 32 kb + 8b + 4h + r. P^T fragment of key step ks (16 keys) = acc S[ks / 2][8 (ks % 2) + j] (keys
 // 16 ks + 8 (j / 4) + 4h + j % 4), so V^T is read with the same key order: ds_read_b64_tr_b16 of rows
 // 16 ks + 4h + (i >> 2) and + 8 (i = l & 15) gives lane l the d column 32 db + 16 ((l >> 4) & 1) + i.
-typedef __attribute__((ext_vector_type(16))) float f32x16;
 constexpr int V3_NS = 4;
 constexpr int V3_PF = 4, V3_RING = 8;  // ring size divides the 32 slots (continuity across iterations)
 
@@ -1212,6 +1394,12 @@ hipError_t launch_prefill(PrefillArgs a, int n_tiles, hipStream_t st) {
   if constexpr (D == 128 && GB == 4 && CAUSAL && PAGED) {
     if (a.kv_bytes) {
       hipLaunchKernelGGL((attn_prefill_v3_kernel<8, false, 0, 1, true>), grid, dim3(512), 0, st, a);
+      return hipGetLastError();
+    }
+  }
+  if constexpr (!CAUSAL && !PAGED && GB == 1 && D <= 64) {
+    if (G == 1 && ((uintptr_t)a.k | (uintptr_t)a.v) % 16 == 0 && a.kv_stride % 8 == 0) {
+      hipLaunchKernelGGL((attn_encoder_kernel<D>), grid, dim3(256), 0, st, a);
       return hipGetLastError();
     }
   }

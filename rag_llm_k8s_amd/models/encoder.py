@@ -187,7 +187,7 @@ class EncoderModel:
     def forward_packed(self, ids: torch.Tensor, lens):
         """ids: int32 [T] packed token ids (on device), lens: python list of sequence lengths.
         Returns fp32 [B, H] pooled (+ normalised) sentence embeddings."""
-        from ..ops.native import build_prefill_tiles
+        from ..ops.native import build_encoder_tiles
 
         be, w, c = self.be, self.w, self.cfg
         H, nh, D = c.hidden_size, c.num_attention_heads, c.head_dim
@@ -197,7 +197,7 @@ class EncoderModel:
             cu_host.append(cu_host[-1] + L)
         cu = torch.tensor(cu_host, dtype=torch.int32).to(dev)
         pos = self.position_ids(lens).to(dev)
-        tiles = build_prefill_tiles(lens, nh, nh).to(dev) if dev.type == "cuda" else None
+        tiles = build_encoder_tiles(lens, nh).to(dev) if dev.type == "cuda" else None
         h = be.embed_ln(ids, pos, w.word, w.pos, w.type_row, w.ln_g, w.ln_b, c.layer_norm_eps)
         T = h.shape[0]
         attn = torch.empty((T, H), dtype=h.dtype, device=dev)

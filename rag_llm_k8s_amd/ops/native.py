@@ -1183,7 +1183,7 @@ def encoder_forward(cfg, weights, ids, lens, first_pos, out, rows):
     cu = np.zeros(B + 1, dtype=np.int32)
     np.cumsum(lens, out=cu[1:])
     pos = np.arange(first_pos, first_pos + T, dtype=np.int32) - np.repeat(cu[:-1], lens)
-    tiles = build_prefill_tiles(lens, nh, nh).numpy().reshape(-1)
+    tiles = build_encoder_tiles(lens, nh).numpy().reshape(-1)
     parts = [ids, pos, cu, lens, rows, tiles]
     at = list(itertools.accumulate(map(len, parts), initial=0))
     ints = torch.from_numpy(np.concatenate(parts).astype(np.int32, copy=False)).to(dev)
@@ -1300,6 +1300,24 @@ def build_prefill_tiles(q_lens, Hq, Hkv):
     q0 = (np.arange(int(nt.sum())) - first) * qt
     order = np.argsort(-q0, kind="stable")
     return torch.from_numpy(np.stack([seq[order], q0[order]], 1).astype(np.int32)).reshape(-1, 2)
+
+
+def build_encoder_tiles(lens, heads):
+    """(seq, q_start) work list of bidirectional attention: every block of a sequence reads all of its keys, so its tiles stay
+    together (they share K / V in the L2 of each head's XCD: 64 sequences of 1344 rows 939 us as build_prefill_tiles orders them,
+    671 so, 12 sequences of 13764 rows 100 and 97), longest sequences first."""
+    import numpy as np
+
+    qt = prefill_qtile(heads, heads)
+    if len(lens) <= 8:  # a query's: host time
+        ls = [int(n) for n in lens]
+        tiles = [(s, q0) for s in sorted(range(len(ls)), key=lambda s: -ls[s]) for q0 in range(0, ls[s], qt)]
+        return torch.tensor(tiles, dtype=torch.int32).reshape(-1, 2)
+    ql = np.asarray(lens, dtype=np.int64)
+    order = np.argsort(-ql, kind="stable")
+    nt = (ql[order] + qt - 1) // qt
+    q0 = (np.arange(int(nt.sum())) - np.repeat(np.cumsum(nt) - nt, nt)) * qt
+    return torch.from_numpy(np.stack([np.repeat(order, nt), q0], 1).astype(np.int32))
 
 
 def attn_prefill(q, k, v, cu_q, kv_lens, tiles, out, Hq, Hkv, D, causal=True, paged=True, block_tables=None,

@@ -179,15 +179,32 @@ __device__ __forceinline__ void rope8(const float* x1, const float* x2, const fl
   }
 }
 
+// lane (i + N) % 16 of the lane's row of 16
+template <int N>
+__device__ __forceinline__ float row_ror(float v) {
+  const int i = __float_as_int(v);
+  return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x120 + N, 0xf, 0xf, false));
+}
+// f over the 64 lanes of a wave, on every lane: the butterfly over lane ^ 32, 16, 8, 4, 2, 1, by lane swaps and row rotations (once
+// lanes 8 apart agree, the lane 4 further on holds what lane ^ 4 does, and so on), which cost an instruction each where a
+// __shfl_xor is a trip through the LDS unit (a query encoder's 25 launches with two row norms in half of them 126 -> 119 us, a
+// decode step of recurrent layers 666 -> 662). All lanes take part.
+template <typename F>
+__device__ __forceinline__ float wave_all(float v, F f) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  v = f(v, row_ror<8>(v));
+  v = f(v, row_ror<4>(v));
+  v = f(v, row_ror<2>(v));
+  return f(v, row_ror<1>(v));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return wave_all(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_all(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Block-wide sum for blockDim.x a multiple of 64 (<= 1024). `red` needs

@@ -1,9 +1,10 @@
 // Sentence encoders: pooling + L2 normalise (E7: CLS / masked mean, sentence-transformers Normalize(),
 // /root/reference/llm/rag.py:55 normalize_embeddings=True), and one forward over packed sequences as a single host call.
 //
-// A query's embedding is about 45 launches of 2 to 5 us each (6 layers); issued one by one from Python they took 14 us each and
-// the GPU idled between them. The kernels of the layers are those of gemm*.hip, attention.hip and norm.hip.
-#include "common.h"
+// A short text's embedding is about 45 launches of 2 to 5 us each (6 layers); issued one by one from Python they took 14 us each and
+// the GPU idled between them. The kernels of the layers are those of gemm*.hip, attention.hip and norm.hip; a single sequence of
+// at most 32 rows takes encoder_few.hip's.
+#include "encoder.h"
 using namespace ragk;
 
 extern "C" {
@@ -106,23 +107,6 @@ __global__ __launch_bounds__(NT) void pool_l2norm_kernel(const bf16_t* __restric
 }
 
 
-// Launches of one product: rows r0 .. r1 on gemm_mid (tile mi, S slabs), gemm_w4 (mi 0: 256 rows a tile, or 32 + rows / 32) or the
-// decode kernels (mi -1).
-struct Piece { int r0, r1, mi, S; };
-struct Plan { int n, slabs; Piece p[2]; };  // slabs: p[0].S fp32 slabs of all rows for the norm behind it
-
-// The arguments of one forward (mirrored by ops/_lib.py EncoderCall).
-struct EncoderCall {
-  const void *word, *pos_table, *type_row, *ln_g, *ln_b;
-  const void* const* layers;  // 12 a layer: wqkv bqkv wo bo ln1_g ln1_b wi bi wo2 bo2 ln2_g ln2_b
-  const int *ids, *pos, *cu, *lens, *tiles, *rows;  // rows: output row of every sequence
-  void *h, *a, *qkv, *attn, *f;
-  float *ws, *out;
-  int n_layers, T, B, H, I, heads, n_tiles, pooling, normalize, ldo;
-  float eps;
-  Plan plans[4];  // qkv, attention output, up, down
-};
-
 int product(const Plan& plan, const void* x, int K, const void* w, int N, const void* bias, const void* resid, void* out, int epi,
             float* ws, hipStream_t st) {
   for (int i = 0; i < plan.n; ++i) {
@@ -154,7 +138,26 @@ int product_norm(const EncoderCall& c, const Plan& plan, const void* x, int K, c
   return rc ? rc : ragk_layernorm_slabs(c.ws, p.S, bias, c.h, c.H, g, b, c.h, c.H, c.T, c.H, c.eps, st);
 }
 
+// Host integers as a kernel's argument: no copy engine, no wait for what the stream still has to do.
+constexpr int PUT_N = 960;
+struct PutInts { int v[PUT_N]; };
+__global__ __launch_bounds__(256) void put_ints_kernel(PutInts a, int* out, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = a.v[i];
+}
+
 }  // namespace
+
+// n integers of host memory (read before the call returns) to dst.
+RAGK_API int ragk_put_ints(const int* src, int n, int* dst, hipStream_t st) {
+  for (int at = 0; at < n; at += PUT_N) {
+    PutInts a;
+    const int m = n - at < PUT_N ? n - at : PUT_N;
+    __builtin_memcpy(a.v, src + at, (size_t)m * 4);
+    hipLaunchKernelGGL(put_ints_kernel, dim3((m + 255) / 256), dim3(256), 0, st, a, dst + at, m);
+  }
+  return (int)hipGetLastError();
+}
 
 // The pooled sequence b goes to row rows[b] of out (rows null: row b), row stride ldo.
 RAGK_API int ragk_pool_l2norm_rows(const void* hidden, int ld, const int* cu, const int* rows, float* out, int ldo, int B, int H,
@@ -179,6 +182,7 @@ RAGK_API int ragk_encoder_forward(const EncoderCall* cp, hipStream_t st) {
   const EncoderCall& c = *cp;
   const int H = c.H, D = H / c.heads, T = c.T;
   if (T <= 0 || c.B <= 0) return 0;
+  if (c.few) return encoder_few_forward(c, st);
   const float scale = 1.f / sqrtf((float)D);
 #define RAGK_TRY(x) \
   if (const int rc = (x)) return rc

@@ -192,6 +192,10 @@ class EncoderModel:
         be, w, c = self.be, self.w, self.cfg
         H, nh, D = c.hidden_size, c.num_attention_heads, c.head_dim
         dev = self.device
+        if len(lens) == 1 and lens[0] == len(ids):  # a question: the launches that embed_into takes for it
+            one = be.encoder_few(c, w, ids, self.first_position)
+            if one is not None:
+                return one
         cu_host = [0]
         for L in lens:
             cu_host.append(cu_host[-1] + L)

@@ -72,6 +72,7 @@ _SIGS = {
     "ragk_embed_ln": [P, P, P, P, P, P, P, P, I, I, F, I, S],
     "ragk_rope_kv": [P, I, P, P, P, P, P, P, I, I, I, I, I, I, S],
     "ragk_pool_l2norm": [P, I, P, P, I, I, I, I, S],
+    "ragk_put_ints": [P, I, P, S],
     "ragk_encoder_call_bytes": [],
     "ragk_encoder_forward": [P, S],
     "ragk_silu_mul": [P, I, P, I, I, I, S],
@@ -258,10 +259,11 @@ class GemmPlan(ctypes.Structure):
 
 
 class EncoderCall(ctypes.Structure):
-    """csrc/kernels/encoder.hip EncoderCall."""
+    """csrc/kernels/encoder.h EncoderCall."""
     _fields_ = ([(n, P) for n in ("word", "pos_table", "type_row", "ln_g", "ln_b", "layers", "ids", "pos", "cu", "lens", "tiles",
-                                  "rows", "h", "a", "qkv", "attn", "f", "ws", "out")]
-                + [(n, I) for n in ("n_layers", "T", "B", "H", "I", "heads", "n_tiles", "pooling", "normalize", "ldo")]
+                                  "rows", "ids_host", "h", "a", "qkv", "attn", "f", "ws", "out", "y")]
+                + [(n, I) for n in ("n_layers", "T", "B", "H", "I", "heads", "n_tiles", "pooling", "normalize", "ldo", "few",
+                                    "first_pos")]
                 + [("eps", F), ("plans", GemmPlan * 4)])
 
 

@@ -228,6 +228,10 @@ class TorchBackend:
         """Whole forward of a packed batch given as host integers, into rows of out; False: not offered here."""
         return False
 
+    def encoder_few(self, cfg, w, ids, first_pos):
+        """The whole forward of one short sequence whose ids are on the device, [1, H]; None: not offered here."""
+        return None
+
     # fp32 residual stream, shaped attention, state-space mixers ---------------
     def embed_residual(self, ids, table, carry=None, prev=None, scale=1.0, pos=None, turns=None, n=0):
         """Embedding rows * scale as the fp32 residual stream, plus the sinusoid of `pos` over the first n columns."""
@@ -590,6 +594,17 @@ class NativeBackend(TorchBackend):
             return False
         self.n.encoder_forward(cfg, weights, ids, lens, first_pos, out, rows)
         return True
+
+    def encoder_few(self, cfg, w, ids, first_pos):
+        if not (self.n.encoder_few_ok(cfg, len(ids), 1) and ids.dtype == torch.int32 and ids.is_contiguous()
+                and ids.device == w.word.device):
+            return None
+        weights = self.n.encoder_pointers(cfg, w)
+        if weights is None:
+            return None
+        out = torch.empty((1, cfg.hidden_size), dtype=torch.float32, device=ids.device)
+        self.n.encoder_few(cfg, weights, ids, first_pos, out[0])
+        return out
 
     def topk_candidates(self, logits, K, vocab_offset=0, max_cand=512, chunks=None):
         return self.n.topk_candidates(logits, K, vocab_offset=vocab_offset, max_cand=max_cand, chunks=chunks)

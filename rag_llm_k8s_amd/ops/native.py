@@ -1167,6 +1167,59 @@ def _encoder_plans(T, H, I, cus, split, w4_min_m):
     return plans, slab
 
 
+FEW_ROWS, FEW_COLS = 32, 1024  # csrc/kernels/encoder.h FEW_T, FEW_H
+FEW_SIZE = 16384  # rows x columns: the blocks repeat the rows' work
+# ints that travel as kernel arguments, 960 a launch of 2 us: copied to the device (a wait for the stream, 15 us when it is idle)
+# only where a forward takes milliseconds
+PUT_INTS = 3840
+
+
+def encoder_few_ok(cfg, T, B):
+    """Whether a batch takes the four launches a layer of csrc/kernels/encoder_few.hip. Us a call against seven launches: six
+    layers of 384 columns 104 / 207 at 5 rows, 119 / 215 at 14, 165 / 218 at 32; 24 layers of 1024 621 / 769 at 5 rows, 742 / 797
+    at 16, but 844 / 824 at 17 and 1048 / 873 at 32."""
+    H = cfg.hidden_size
+    return (B == 1 and 1 <= T <= FEW_ROWS and H <= FEW_COLS and T * H <= FEW_SIZE
+            and H // cfg.num_attention_heads in (32, 64))
+
+
+def _encoder_call(cfg, weights, bufs, at, T, B):
+    """(call, what has to outlive it): addresses of `bufs` ((field, bytes) pairs) within one allocation that begins at `at`."""
+    import ctypes
+
+    c = _lib.EncoderCall()
+    for name, size in bufs:
+        setattr(c, name, at)
+        at += -(-size // 256) * 256
+    c.word, c.pos_table, c.ln_g, c.ln_b, c.type_row, *table = weights
+    ptrs = (ctypes.c_void_p * len(table))(*table)
+    c.layers, c.n_layers = ctypes.addressof(ptrs), len(table) // len(ENCODER_LAYER)
+    c.T, c.B, c.H, c.I, c.heads = T, B, cfg.hidden_size, cfg.intermediate_size, cfg.num_attention_heads
+    c.pooling, c.normalize, c.eps = {"cls": 0, "mean": 1, "last": 2}[cfg.pooling], int(cfg.normalize), float(cfg.layer_norm_eps)
+    return c, ptrs
+
+
+def encoder_few(cfg, weights, ids, first_pos, out):
+    """Embedding of one sequence (encoder_few_ok) into the fp32 row `out`; ids: contiguous int32, on the host (they travel as a
+    kernel argument: nothing is uploaded) or on the device."""
+    import ctypes
+
+    H, T = cfg.hidden_size, len(ids)
+    _req(out.dtype == torch.float32 and out.is_cuda and out.is_contiguous() and out.numel() == H, "out fp32 row")
+    bufs = [("h", 2 * T * H), ("qkv", 6 * T * H), ("f", 2 * T * cfg.intermediate_size), ("y", 4 * T * H)]
+    buf = torch.empty(sum(-(-n // 256) * 256 for _, n in bufs), dtype=torch.uint8, device=out.device)
+    c, keep = _encoder_call(cfg, weights, bufs, buf.data_ptr(), T, 1)
+    c.few, c.first_pos, c.out, c.ldo = 1, first_pos, out.data_ptr(), H
+    if isinstance(ids, torch.Tensor):
+        _req(ids.is_cuda and ids.dtype == torch.int32 and ids.is_contiguous(), "ids int32")
+        c.ids = ids.data_ptr()
+    else:
+        _req(ids.dtype == "int32" and ids.flags.c_contiguous, "ids int32")
+        c.ids_host = ids.ctypes.data
+    check(_lib.lib().ragk_encoder_forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
+    return out
+
+
 def encoder_forward(cfg, weights, ids, lens, first_pos, out, rows):
     """Embeddings of packed sequences (host int32 ids, int64 lens) into rows `rows` of out (fp32 on the device): one upload
     of the step's integers, one workspace, one native call for all launches (csrc/kernels/encoder.hip). `weights`: their
@@ -1180,28 +1233,30 @@ def encoder_forward(cfg, weights, ids, lens, first_pos, out, rows):
     _req(T == int(lens.sum()) and len(rows) == B and 0 <= int(rows.min()) and int(rows.max()) < out.shape[0], "lens, rows")
     _req(T * max(3 * H, I) * 2 < 2 ** 31, "packed rows past 2 GiB")
     dev = out.device
+    if encoder_few_ok(cfg, T, B):
+        encoder_few(cfg, weights, np.ascontiguousarray(ids), first_pos, out[int(rows[0])])
+        return out
     cu = np.zeros(B + 1, dtype=np.int32)
     np.cumsum(lens, out=cu[1:])
     pos = np.arange(first_pos, first_pos + T, dtype=np.int32) - np.repeat(cu[:-1], lens)
     tiles = build_encoder_tiles(lens, nh).numpy().reshape(-1)
     parts = [ids, pos, cu, lens, rows, tiles]
     at = list(itertools.accumulate(map(len, parts), initial=0))
-    ints = torch.from_numpy(np.concatenate(parts).astype(np.int32, copy=False)).to(dev)
-    L, cus, c = _lib.lib(), _cu_count(), _lib.EncoderCall()
-    c.plans, slab = _encoder_plans(T, H, I, cus, PREFILL_SPLITK, PREFILL_SPLITK_MIN_M)
-    # activations in the order h, a, attn, qkv, f, then the slabs
-    sizes = [2 * T * n for n in (H, H, H, 3 * H, I)] + [4 * slab]
-    off = list(itertools.accumulate([-(-n // 256) * 256 for n in sizes], initial=0))
-    buf = torch.empty(off[-1], dtype=torch.uint8, device=dev)
-    p, q = buf.data_ptr(), ints.data_ptr()
-    c.h, c.a, c.attn, c.qkv, c.f, c.ws = (p + o for o in off[:-1])
+    host = np.concatenate(parts).astype(np.int32, copy=False)
+    L = _lib.lib()
+    if len(host) <= PUT_INTS:
+        ints = torch.empty(len(host), dtype=torch.int32, device=dev)
+        check(L.ragk_put_ints(host.ctypes.data, len(host), ints.data_ptr(), stream_ptr()), "ragk_put_ints")
+    else:
+        ints = torch.from_numpy(host).to(dev)
+    plans, slab = _encoder_plans(T, H, I, _cu_count(), PREFILL_SPLITK, PREFILL_SPLITK_MIN_M)
+    bufs = [("h", 2 * T * H), ("a", 2 * T * H), ("attn", 2 * T * H), ("qkv", 6 * T * H), ("f", 2 * T * I), ("ws", 4 * slab)]
+    buf = torch.empty(sum(-(-n // 256) * 256 for _, n in bufs), dtype=torch.uint8, device=dev)
+    c, keep = _encoder_call(cfg, weights, bufs, buf.data_ptr(), T, B)
+    c.plans = plans
+    q = ints.data_ptr()
     c.ids, c.pos, c.cu, c.lens, c.rows, c.tiles = (q + 4 * o for o in at[:-1])
-    c.word, c.pos_table, c.ln_g, c.ln_b, c.type_row, *table = weights
-    ptrs = (ctypes.c_void_p * len(table))(*table)
-    c.layers, c.n_layers = ctypes.addressof(ptrs), len(table) // len(ENCODER_LAYER)
-    c.out, c.ldo = out.data_ptr(), out.stride(0)
-    c.T, c.B, c.H, c.I, c.heads, c.n_tiles = T, B, H, I, nh, len(tiles) // 2
-    c.pooling, c.normalize, c.eps = {"cls": 0, "mean": 1, "last": 2}[cfg.pooling], int(cfg.normalize), float(cfg.layer_norm_eps)
+    c.out, c.ldo, c.n_tiles = out.data_ptr(), out.stride(0), len(tiles) // 2
     check(L.ragk_encoder_forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
     return out
 

@@ -937,6 +937,9 @@ RAGK_API int ragk_kmeans_assign(const float* X, int n, int d, const float* C, co
   return (int)hipGetLastError();
 }
 
+// Returns when everything enqueued on the stream is done.
+RAGK_API int ragk_stream_wait(hipStream_t st) { return (int)hipStreamSynchronize(st); }
+
 RAGK_API int ragk_l2_append(float* xt, int cap, int d, int n0, const float* x, int n, hipStream_t st) {
   if (n <= 0) return 0;
   if (n0 + n > cap) return (int)hipErrorInvalidValue;

@@ -1576,11 +1576,32 @@ _search_ws = {}
 _search_lock = threading.Lock()
 
 
+# Results in host memory up to this many are stored there by the merge itself (pinned, 12 bytes each) and only waited for, instead
+# of copied behind it: one query of 10000 x 384 40.4 -> 38.9 us, 256 queries of the k = 10 nearest 119 -> 109, 1000 of 1000 rows
+# 87 -> 78.
+SEARCH_STORE = 16384
+
+
+def _search_out(nq, k, device, host):
+    n = nq * k
+    if host and 0 < n <= SEARCH_STORE:
+        return torch.empty(3 * n, dtype=torch.int32, pin_memory=True)
+    return torch.empty(3 * n, dtype=torch.int32, device=device)
+
+
+def _search_wait(out):
+    """Behind the launches, whatever became of them: a pinned buffer goes back to its pool once nothing can write to it."""
+    if not out.is_cuda:
+        check(_lib.lib().ragk_stream_wait(stream_ptr()), "ragk_stream_wait")
+
+
 def _search_views(buf, nq, k, host):
-    """(D fp32 [nq, k], I int64 [nq, k]) as views of the ONE allocation a search writes, int64 ids first; host: of its copy there
-    (a copy of each result waits for the device twice)."""
-    if host:
+    """(D fp32 [nq, k], I int64 [nq, k]) as views of the ONE allocation a search writes (_search_out), int64 ids first; host: of a
+    copy in pageable memory (a copy of each result waits for the device twice; pinned pages go back to their pool)."""
+    if host and buf.is_cuda:
         buf = buf.cpu()
+    elif host:
+        buf = buf.clone()
     return buf[2 * nq * k:].view(torch.float32).view(nq, k), buf[:2 * nq * k].view(torch.int64).view(nq, k)
 
 
@@ -1612,15 +1633,18 @@ def l2_search(xt, cap, n, q, k, row_begin=0, ids_map=None, host=False):
     _req(xt.shape[1] == cap and 0 <= row_begin <= max(row_begin, n) <= cap, "rows within the store")
     _req(ids_map is None or (ids_map.dtype == torch.int32 and ids_map.is_cuda and ids_map.numel() >= n), "ids_map")
     L = _lib.lib()
-    out = torch.empty(nq * k * 3, dtype=torch.int32, device=q.device)
+    out = _search_out(nq, k, q.device, host)
     if nq == 0:
         return _search_views(out, nq, k, host)
     G = L.ragk_l2_search_groups(row_begin, max(n, row_begin), nq, k, d)
-    with _search_lock:
-        pd, pi = _search_partials(nq * G * k, q.device)
-        check(L.ragk_l2_search(xt.data_ptr(), cap, d, row_begin, max(n, row_begin), q.data_ptr(), nq, k,
-                               ptr(ids_map), pd.data_ptr(), pi.data_ptr(), out.data_ptr() + 8 * nq * k, out.data_ptr(),
-                               stream_ptr()), "ragk_l2_search")
+    try:
+        with _search_lock:
+            pd, pi = _search_partials(nq * G * k, q.device)
+            check(L.ragk_l2_search(xt.data_ptr(), cap, d, row_begin, max(n, row_begin), q.data_ptr(), nq, k,
+                                   ptr(ids_map), pd.data_ptr(), pi.data_ptr(), out.data_ptr() + 8 * nq * k, out.data_ptr(),
+                                   stream_ptr()), "ragk_l2_search")
+    finally:
+        _search_wait(out)
     return _search_views(out, nq, k, host)
 
 
@@ -1636,15 +1660,18 @@ def ivf_search(xt, cap, q, probes, offsets, ids_map, k, max_list=None, ends=None
     d = xt.shape[0]
     nq, nprobe = probes.shape
     _req(1 <= k <= 64 and d <= 2048 and nprobe >= 1, "k <= 64, d <= 2048")
-    out = torch.empty(nq * k * 3, dtype=torch.int32, device=q.device)
+    out = _search_out(nq, k, q.device, host)
     if nq == 0:
         return _search_views(out, nq, k, host)
-    with _search_lock:
-        pd, pi = _search_partials(nq * nprobe * k, q.device)
-        check(_lib.lib().ragk_ivf_search(xt.data_ptr(), cap, d, q.data_ptr(), nq, probes.data_ptr(), nprobe,
-                                         offsets.data_ptr(), ptr(ends), ids_map.data_ptr(), k, pd.data_ptr(),
-                                         pi.data_ptr(), out.data_ptr() + 8 * nq * k, out.data_ptr(), stream_ptr()),
-              "ragk_ivf_search")
+    try:
+        with _search_lock:
+            pd, pi = _search_partials(nq * nprobe * k, q.device)
+            check(_lib.lib().ragk_ivf_search(xt.data_ptr(), cap, d, q.data_ptr(), nq, probes.data_ptr(), nprobe,
+                                             offsets.data_ptr(), ptr(ends), ids_map.data_ptr(), k, pd.data_ptr(),
+                                             pi.data_ptr(), out.data_ptr() + 8 * nq * k, out.data_ptr(), stream_ptr()),
+                  "ragk_ivf_search")
+    finally:
+        _search_wait(out)
     return _search_views(out, nq, k, host)
 
 

@@ -7,12 +7,12 @@
 //   up     rows = norm
 //   down   rows as they lie
 // A block is 16 output columns: it requests its weights (and whatever else does not depend on the rows), then works on the rows
-// while they travel, keeps the rows in LDS as bf16 and multiplies: eight waves share K and meet in LDS. Repeating the rows' work in
+// while they travel, keeps the rows in LDS as bf16 and multiplies: 16 waves share the rows, then K, and meet in LDS. Repeating the rows' work in
 // each of 24 to 256 blocks costs reads from L2 (21 KB a block for 14 fp32 rows of 384) and 0.6 us, the launch it saves 2.4 to 4.
 // Sums of a product, its bias and its residual reach the norm behind it in fp32; block 0 writes the norm's rows out, as the
 // residual of the product after next.
-// Six layers of 384 columns, 14 rows: 220 -> 119 us a call, 25 launches of 4.7 instead of 44; 24 layers of 1024, 14 rows: 796 ->
-// 723. What is left of a launch is its start, one trip to memory for the rows and one through LDS for the sum (a down projection
+// Six layers of 384 columns, 14 rows: 220 -> 111 us a call, 25 launches of 4.4 instead of 44 (with eight waves a
+// block, two rows a wave, 119); 24 layers of 1024, 14 rows: 752 -> 686 (726). What is left of a launch is its start, one trip to memory for the rows and one through LDS for the sum (a down projection
 // alone, without rows to make, takes as long as the others). Past 16384 values of rows the repeated work costs more than it
 // saves (ops/native.py encoder_few_ok).
 #include "attn_tiles.h"
@@ -21,7 +21,7 @@ using namespace ragk;
 
 namespace {
 
-constexpr int FEW_W = 8;  // waves
+constexpr int FEW_W = 16;  // waves
 
 enum { ROWS, EMBED, NORM, ATTEND };
 
@@ -162,7 +162,7 @@ struct FewHead {
   }
 };
 
-// MT = 16-row tiles; NP = K-steps of 32 that a wave requests at once (it takes every eighth). D: head size (ATTEND).
+// MT = 16-row tiles; NP = K-steps of 32 that a wave requests at once (it takes every 16th). D: head size (ATTEND).
 template <int PRO, int EPI, int MT, int NP, int D>
 __global__ __launch_bounds__(FEW_W * 64) void few_kernel(FewArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -204,35 +204,29 @@ __global__ __launch_bounds__(FEW_W * 64) void few_kernel(FewArgs a) {
     few_pairs(a.g, lane, nj, gr);
     few_pairs(a.b, lane, nj, br);
 #pragma unroll
-    for (int i = 0; i < 2 * MT; i += 2) {
-      float v[2][16];
+    for (int i = 0; i < MT; ++i) {
+      const int row = wid + FEW_W * i;
+      if (row < a.T) {
+        float v[16];
+        unsigned o[8];
+        few_row<PRO>(a, row, lane, nj, v);
+        few_norm(v, nj, a.K, a.eps, gr, br, o);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) few_row<PRO>(a, min(wid + FEW_W * (i + u), a.T - 1), lane, nj, v[u]);
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int row = wid + FEW_W * (i + u);
-        if (row < a.T) {
-          unsigned o[8];
-          few_norm(v[u], nj, a.K, a.eps, gr, br, o);
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (j < nj) {
-              *reinterpret_cast<unsigned*>(rows + row * rowb + 4 * lane + 256 * j) = o[j];
-              if (blockIdx.x == 0) *reinterpret_cast<unsigned*>(a.h + (size_t)row * a.K + 2 * lane + 128 * j) = o[j];
-            }
-        }
+        for (int j = 0; j < 8; ++j)
+          if (j < nj) {
+            *reinterpret_cast<unsigned*>(rows + row * rowb + 4 * lane + 256 * j) = o[j];
+            if (blockIdx.x == 0) *reinterpret_cast<unsigned*>(a.h + (size_t)row * a.K + 2 * lane + 128 * j) = o[j];
+          }
       }
     }
   }
   if constexpr (PRO == ATTEND) {
     const bf16_t* qkv = reinterpret_cast<const bf16_t*>(a.x);
     const int heads = a.K / D;
-    for (int hd = wid; hd < heads; hd += 2 * FEW_W) {  // two heads' loads in flight
-      FewHead<MT, D> h0, h1;
-      h0.load(qkv, a.K, a.T, hd, fr, fh);
-      h1.load(qkv, a.K, a.T, min(hd + FEW_W, heads - 1), fr, fh);
-      h0.attend(rows, rowb, a.T, hd, fr, fh, a.scale_log2);
-      if (hd + FEW_W < heads) h1.attend(rows, rowb, a.T, hd + FEW_W, fr, fh, a.scale_log2);
+    for (int hd = wid; hd < heads; hd += FEW_W) {
+      FewHead<MT, D> head;
+      head.load(qkv, a.K, a.T, hd, fr, fh);
+      head.attend(rows, rowb, a.T, hd, fr, fh, a.scale_log2);
     }
   }
   if constexpr (PRO != ROWS) __syncthreads();
@@ -286,20 +280,21 @@ template <int PRO, int EPI, int D = 32>
 int few_dispatch(const FewArgs& a, hipStream_t st) {
   if (a.T < 1 || a.T > FEW_T || a.K % 128 || a.K <= 0 || a.N % 16 || (PRO != ROWS && a.K > FEW_H)) return (int)hipErrorInvalidValue;
 #define RAGK_FEW(NP) return a.T <= 16 ? few_launch<PRO, EPI, 1, NP, D>(a, st) : few_launch<PRO, EPI, 2, NP, D>(a, st)
-  if (a.K <= 512) RAGK_FEW(2);
-  if constexpr (PRO != ROWS) RAGK_FEW(4);
-  if (a.K <= 1024) RAGK_FEW(4);
-  if (a.K <= 2048) RAGK_FEW(8);
-  RAGK_FEW(16);
+  if (a.K <= 512) RAGK_FEW(1);
+  if constexpr (PRO != ROWS) RAGK_FEW(2);
+  if (a.K <= 1024) RAGK_FEW(2);
+  if (a.K <= 2048) RAGK_FEW(4);
+  RAGK_FEW(8);
 #undef RAGK_FEW
 }
 
+constexpr int POOL_W = 8;
 // Norm of the rows, then the pooled row as encoder.hip has it (the norm's rows rounded to bf16). A wave takes every eighth row.
-__global__ __launch_bounds__(FEW_W * 64) void few_pool_kernel(const float* __restrict__ y, const bf16_t* __restrict__ g,
+__global__ __launch_bounds__(POOL_W * 64) void few_pool_kernel(const float* __restrict__ y, const bf16_t* __restrict__ g,
                                                               const bf16_t* __restrict__ b, float* out, int T, int H, float eps,
                                                               int mode, int normalize) {
-  __shared__ float part[FEW_W][FEW_H];
-  __shared__ float red[FEW_W];
+  __shared__ float part[POOL_W][FEW_H];
+  __shared__ float red[POOL_W];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nj = H / 128;
   const int first = mode == 2 ? T - 1 : 0, last = mode == 1 ? T : first + 1;
   unsigned gr[8], br[8];
@@ -311,7 +306,7 @@ __global__ __launch_bounds__(FEW_W * 64) void few_pool_kernel(const float* __res
   FewArgs a{};
   a.x = y;
   a.K = H;
-  for (int row = first + wid; row < last; row += FEW_W) {
+  for (int row = first + wid; row < last; row += POOL_W) {
     float v[16];
     unsigned o[8];
     few_row<NORM>(a, row, lane, nj, v);
@@ -328,14 +323,14 @@ __global__ __launch_bounds__(FEW_W * 64) void few_pool_kernel(const float* __res
     if (j < nj) *reinterpret_cast<float2*>(&part[wid][2 * lane + 128 * j]) = make_float2(acc[2 * j], acc[2 * j + 1]);
   __syncthreads();
   const float inv = mode == 1 ? 1.f / (float)T : 1.f;
-  float v[FEW_H / (FEW_W * 64)], ss = 0.f;
+  float v[FEW_H / (POOL_W * 64)], ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < FEW_H / (FEW_W * 64); ++i) {
-    const int c = threadIdx.x + FEW_W * 64 * i;
+  for (int i = 0; i < FEW_H / (POOL_W * 64); ++i) {
+    const int c = threadIdx.x + POOL_W * 64 * i;
     v[i] = 0.f;
     if (c < H) {
 #pragma unroll
-      for (int w = 0; w < FEW_W; ++w) v[i] += part[w][c];
+      for (int w = 0; w < POOL_W; ++w) v[i] += part[w][c];
       v[i] *= inv;
       ss += v[i] * v[i];
     }
@@ -346,8 +341,8 @@ __global__ __launch_bounds__(FEW_W * 64) void few_pool_kernel(const float* __res
     scale = 1.f / fmaxf(sqrtf(ss), 1e-12f);  // torch.nn.functional.normalize eps
   }
 #pragma unroll
-  for (int i = 0; i < FEW_H / (FEW_W * 64); ++i) {
-    const int c = threadIdx.x + FEW_W * 64 * i;
+  for (int i = 0; i < FEW_H / (POOL_W * 64); ++i) {
+    const int c = threadIdx.x + POOL_W * 64 * i;
     if (c < H) out[c] = v[i] * scale;
   }
 }
@@ -393,7 +388,7 @@ int encoder_few_forward(const EncoderCall& c, hipStream_t st) {
   }
 #undef RAGK_TRY
   const void* const* w = c.layers + 12 * (c.n_layers - 1);
-  hipLaunchKernelGGL(few_pool_kernel, dim3(1), dim3(FEW_W * 64), 0, st, c.y, (const bf16_t*)w[10], (const bf16_t*)w[11], c.out, T, H,
+  hipLaunchKernelGGL(few_pool_kernel, dim3(1), dim3(POOL_W * 64), 0, st, c.y, (const bf16_t*)w[10], (const bf16_t*)w[11], c.out, T, H,
                      c.eps, c.pooling, c.normalize);
   return (int)hipGetLastError();
 }

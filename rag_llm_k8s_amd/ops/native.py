@@ -1176,8 +1176,8 @@ PUT_INTS = 3840
 
 def encoder_few_ok(cfg, T, B):
     """Whether a batch takes the four launches a layer of csrc/kernels/encoder_few.hip. Us a call against seven launches: six
-    layers of 384 columns 104 / 207 at 5 rows, 119 / 215 at 14, 165 / 218 at 32; 24 layers of 1024 621 / 769 at 5 rows, 742 / 797
-    at 16, but 844 / 824 at 17 and 1048 / 873 at 32."""
+    layers of 384 columns 103 / 197 at 5 rows, 111 / 202 at 14, 147 / 205 at 32; 24 layers of 1024 600 / 711 at 5 rows, 705 / 761
+    at 16, 777 / 790 at 17, but 855 / 820 at 24 and 958 / 839 at 32."""
     H = cfg.hidden_size
     return (B == 1 and 1 <= T <= FEW_ROWS and H <= FEW_COLS and T * H <= FEW_SIZE
             and H // cfg.num_attention_heads in (32, 64))

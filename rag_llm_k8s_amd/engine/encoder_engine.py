@@ -57,6 +57,9 @@ class EmbeddingEngine:
             out = torch.empty((n, self.dim), dtype=torch.float32, device=self.device)
         if n == 0:
             return out
+        if n == 1:  # a question: nothing to order or cut (30 us of host time around a forward of 110)
+            self.model.embed_into(ids[:int(lens[0])], np.asarray(lens, dtype=np.int64), out, np.array([row0]))
+            return out
         starts = np.zeros(n + 1, dtype=np.int64)
         np.cumsum(lens, out=starts[1:])
         order = np.argsort(-lens.astype(np.int64), kind="stable")

@@ -585,7 +585,7 @@ class NativeBackend(TorchBackend):
         return self.n.pool_l2norm(hidden, cu, mode=mode, normalize=normalize)
 
     def encoder_forward(self, cfg, w, ids, lens, first_pos, out, rows):
-        T = int(lens.sum())
+        T = int(lens[0]) if len(lens) == 1 else int(lens.sum())
         if (ids.dtype != np.int32 or out.dtype != torch.float32 or out.stride(1) != 1 or out.device != w.word.device or T == 0
                 or T * max(3 * cfg.hidden_size, cfg.intermediate_size) * 2 >= 2 ** 31):
             return False

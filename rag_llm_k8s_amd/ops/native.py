@@ -1230,12 +1230,14 @@ def encoder_forward(cfg, weights, ids, lens, first_pos, out, rows):
 
     H, I, nh, B, T = cfg.hidden_size, cfg.intermediate_size, cfg.num_attention_heads, len(lens), int(len(ids))
     _req(out.dtype == torch.float32 and out.is_cuda and out.stride(1) == 1 and out.shape[1] == H, "out fp32 rows")
+    if encoder_few_ok(cfg, T, B):
+        row = int(rows[0])
+        _req(T == int(lens[0]) and len(rows) == 1 and 0 <= row < out.shape[0], "lens, rows")
+        encoder_few(cfg, weights, np.ascontiguousarray(ids), first_pos, out[row])
+        return out
     _req(T == int(lens.sum()) and len(rows) == B and 0 <= int(rows.min()) and int(rows.max()) < out.shape[0], "lens, rows")
     _req(T * max(3 * H, I) * 2 < 2 ** 31, "packed rows past 2 GiB")
     dev = out.device
-    if encoder_few_ok(cfg, T, B):
-        encoder_few(cfg, weights, np.ascontiguousarray(ids), first_pos, out[int(rows[0])])
-        return out
     cu = np.zeros(B + 1, dtype=np.int32)
     np.cumsum(lens, out=cu[1:])
     pos = np.arange(first_pos, first_pos + T, dtype=np.int32) - np.repeat(cu[:-1], lens)

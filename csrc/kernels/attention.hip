@@ -579,6 +579,7 @@ __device__ __forceinline__ void pin_s(int& x) { asm volatile("" : "+s"(x)); }
 // The asm MFMAs are opaque to the compiler's hazard recognizer: a VALU read of an MFMA result needs
 // the XDL-write -> VALU-read wait states (18 for a 16-pass op), and a VALU write read by an MFMA a few.
 __device__ __forceinline__ void mfma_result_wait() {}
+// NW = 4: 32 query rows, the tile's first or (blockIdx.y) second half.
 // NW = 8: two groups of 4 waves (query rows q_start + [0, 32) and + [32, 64)) share every K / V tile,
 // so each SIMD runs two of these streams and one wave's dependency stalls are the other's issue slots.
 // DIAG (stamp builds only, wrong results): 1 = no softmax chunks in the fast slots, 2 = no fragment reads
@@ -599,7 +600,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_prefill_v3_kernel(Prefil
   const int wid_u = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   int tix, hg;
   prefill_block(a, tix, hg);
-  const int seq = a.tiles[2 * tix], q_start = a.tiles[2 * tix + 1];
+  const int seq = a.tiles[2 * tix], q_start = a.tiles[2 * tix + 1] + (NW == 4 ? 32 * (int)blockIdx.y : 0);
   const int G = a.Hq / a.Hkv;
   const int groups_per_kv = G / 4;
   const int kvh = hg / groups_per_kv;
@@ -608,6 +609,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_prefill_v3_kernel(Prefil
 
   const int q_off = a.cu_q[seq];
   const int q_len = a.cu_q[seq + 1] - q_off;
+  if (NW == 4 && q_start >= q_len) return;  // block-uniform, before any barrier
   const int kv_len = a.kv_lens[seq];
   const int ctx0 = kv_len - q_len;
   // block-uniform tile counts (every wave runs the same iterations and barriers)
@@ -1381,10 +1383,16 @@ __global__ void attn_decode_reduce_kernel(DecodeArgs a, int D) {
 // Kernel per config:
 //   * Llama (D 128, 4 query heads per KV head, causal, paged cache < 4 GiB): the software-pipelined
 //     8-wave kernel with the whole-row LDS epilogue (attn_prefill_v3_kernel<8, ..., WIDE>; 64-query
-//     tiles), tools/attn_pp_ab.py;
+//     tiles), tools/attn_pp_ab.py; few blocks: its 4-wave form, two blocks a tile (V3_HALF);
 //   * every other 4-heads-per-block config: attn_prefill_kernel with 8 waves (64-query tiles, two 32-row
 //     groups sharing each K/V tile);
 //   * 1 or 2 heads per block (encoders, GPT-2, odd GQA ratios): the 4-wave attn_prefill_kernel.
+// Up to this many 64-query blocks the pipelined kernel runs as twice as many of 32 queries: with CUs to spare, a wave that has its
+// SIMD to itself takes a key tile faster than two that share it. 32 query heads over 8, one prompt, us: 64 tokens 7.8 -> 6.8, 300
+// 13.7 -> 11.7, 700 22.2 -> 18.3, 1000 (128 blocks) 29.3 -> 24.8; 16 heads over 4, 2000 tokens 49.3 -> 40.3; 3 of 300 15.0 -> 12.8.
+// Past 128 blocks the halves no longer fit one round: 10 prompts of 100 tokens (160 blocks) 10.5 against 13.4, one of 1300 (168)
+// 36.5 against 30.9; the entry does not know which it has.
+constexpr unsigned V3_HALF = 128;
 template <int D, int GB, bool CAUSAL, bool PAGED>
 hipError_t launch_prefill(PrefillArgs a, int n_tiles, hipStream_t st) {
   const int G = a.Hq / a.Hkv;
@@ -1393,6 +1401,10 @@ hipError_t launch_prefill(PrefillArgs a, int n_tiles, hipStream_t st) {
   const dim3 grid(n_tiles * n_hg);
   if constexpr (D == 128 && GB == 4 && CAUSAL && PAGED) {
     if (a.kv_bytes) {
+      if (grid.x <= V3_HALF) {
+        hipLaunchKernelGGL((attn_prefill_v3_kernel<4, false, 0, 0, true>), dim3(grid.x, 2), dim3(256), 0, st, a);
+        return hipGetLastError();
+      }
       hipLaunchKernelGGL((attn_prefill_v3_kernel<8, false, 0, 1, true>), grid, dim3(512), 0, st, a);
       return hipGetLastError();
     }

@@ -349,13 +349,6 @@ __global__ __launch_bounds__(NWV * 64, 8 / NWV) void attn_prefill_kernel(Prefill
 // the fourth wave (94 us). Other head sizes, grouped heads and unaligned rows stay on attn_prefill_kernel.
 // Layouts as in attn_prefill_v3_kernel; V rows are swizzled by pairs of 32-B granules (a transposed read takes four rows of two
 // granules from each half of the banks).
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-
-template <int D>
-__device__ __forceinline__ int vswz32(int row) {
-  return D == 64 ? 4 * ((row >> 1) & 1) : 0;
-}
-
 template <int D>
 __global__ __launch_bounds__(256, 3) void attn_encoder_kernel(PrefillArgs a) {
   using C = Cfg<D>;

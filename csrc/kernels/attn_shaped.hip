@@ -190,10 +190,19 @@ struct ShapedPrefill {
 // BOUNDED: every score is known to stay within a range whose exponentials fp32 holds (soft cap + largest bias), so
 // the sums need no running maximum: the weights are 2^s, and the extra zero score adds exactly 1.
 enum PrefillMode { GENERAL, BOUNDED, PLAIN };
+// Bound by the score arithmetic (vector unit) with the products behind it: 4 waves a block, a wave 32 queries of one head,
+// 32x32x16 products of keys x queries. A lane pair holds one query, so its maximum, its rescale and its position arithmetic
+// are one per lane, and a key fragment feeds twice the products of a 16x16x32 one. The values are read transposed at pair
+// granularity (vswz32: with the 16-column swizzle half of those reads met in a bank, 64.1 against 61.9 us below). A block's
+// end asks for all its output gates together. Before (16x16x32 products, gates one by one), now, a launch, us:
+//   one gate a value, plain scores: 24 heads, 1777 tokens 70.0 -> 61.9, 2 x 700 29.6 -> 25.1, 300 17.6 -> 15.2
+//   soft cap, bias, window, zero score: 5 x 1900 120.8 -> 113.2, 5000 334.9 -> 323.1, 3 x 400 25.3 -> 24.2
+// Layouts as in attn_prefill_v3_kernel (attention.hip).
 template <int DK, int DV, PrefillMode MODE>
 __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_shaped_prefill_kernel(ShapedPrefill pa) {
   using CK = Cfg<DK>;
   using CV = Cfg<DV>;
+  constexpr int QS = DK / 16, DB = DV / 32;  // products over a key row, 32-wide blocks of a value row
   const ShapedArgs& a = pa.a;
   extern __shared__ __attribute__((aligned(16))) char smem[];  // [buf][K | V], page list, bias tables
   int* s_bt = reinterpret_cast<int*>(smem + 2 * (CK::TILEB + CV::TILEB));
@@ -212,34 +221,28 @@ __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_sh
   const int keep = MODE == PLAIN ? 0 : a.keep, sink = MODE == PLAIN ? 0 : a.sink;
   const Pages pg = visited(ctx0 + q_start, ctx0 + min(q_start + qt_rows, q_len) - 1, a.window, keep);
   const int wave_pmin = ctx0 + pbase, wave_pmax = ctx0 + min(pbase + 31, q_len - 1);
-  const int fr = lane & 15, fh = lane >> 4;
+  const int l32 = lane & 31, h = lane >> 5, i16 = lane & 15;  // this lane's query, half of the keys / columns
+  const int qpos = ctx0 + pbase + l32, qi = pbase + l32;
 
-  bf16x8 qf[2][CK::KS];
+  bf16x8 qf[QS];
+  {
+    const bf16_t* qp = (const bf16_t*)a.q + (size_t)(q_off + min(qi, q_len - 1)) * a.ldq + hq * DK + 8 * h;
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
-    const int qi = min(pbase + 16 * qt + fr, q_len - 1);
-    const bf16_t* qp = (const bf16_t*)a.q + (size_t)(q_off + qi) * a.ldq + hq * DK + 8 * fh;
-#pragma unroll
-    for (int s = 0; s < CK::KS; ++s) qf[qt][s] = *reinterpret_cast<const bf16x8*>(qp + 32 * s);
+    for (int s = 0; s < QS; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qp + 16 * s);
   }
-  f32x4 o[CV::DT][2];
+  f32x16 o[DB];
 #pragma unroll
-  for (int dt = 0; dt < CV::DT; ++dt)
+  for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) o[dt][qt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  // the extra zero score: running max 0, one unit in the sum (one of a query's four lanes holds it)
-  float m_i[2], l_i[2];
-#pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
-    m_i[qt] = sink ? 0.f : -INFINITY;
-    l_i[qt] = sink && fh == 0 ? 1.f : 0.f;
-  }
+    for (int e = 0; e < 16; ++e) o[db][e] = 0.f;
+  // the extra zero score: running max 0, one unit in the sum (one of a query's two lanes holds it)
+  float m_i = sink ? 0.f : -INFINITY, l_i = sink && h == 0 ? 1.f : 0.f;
   const int* bt = a.block_tables + (size_t)seq * a.bt_stride;
   for (int i = threadIdx.x; i < pg.n; i += 256) s_bt[i] = a.entry(bt, seq, pg.page(i));
   if (MODE != PLAIN && a.table && pa.sb_stride)
-    for (int h = 0; h < gb; ++h)
+    for (int b = 0; b < gb; ++b)
       for (int i = threadIdx.x; i <= a.far; i += 256)
-        s_bias[h * pa.sb_stride + i] = a.table[(size_t)(h0 + h) * (a.far + 1) + i] * LOG2E;
+        s_bias[b * pa.sb_stride + i] = a.table[(size_t)(h0 + b) * (a.far + 1) + i] * LOG2E;
   __syncthreads();
   const float* tb = MODE != PLAIN && a.table ? a.table + (size_t)hq * (a.far + 1) : nullptr;
   const float* s_tb = s_bias + hb * pa.sb_stride;  // the same row in LDS, in log2 units
@@ -263,7 +266,7 @@ __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_sh
 #pragma unroll
   for (int i = 0; i < VP; ++i) {
     const int row = (wid_u + 4 * i) * CV::RPP + lane / CV::NC, ph = lane % CV::NC;
-    voff[i] = row * a.v_row * 2 + 16 * (ph ^ vswz<DV>(row));
+    voff[i] = row * a.v_row * 2 + 16 * (ph ^ vswz32<DV>(row));
   }
   const unsigned lds0 = lds_addr(smem);
   auto stage = [&](int entry, int buf) {
@@ -276,29 +279,41 @@ __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_sh
 #pragma unroll
     for (int i = 0; i < VP; ++i) blds16_asm(srd_v, voff[i], 0, l + CK::TILEB + (wid_u + 4 * i) * 1024);
   };
+  // fragment reads: the swizzles of key rows 32 kb + l32 and of value rows 16 ks + 4 h + .. do not depend on kb and ks
+  int kat[QS], vat[DB][2];
+#pragma unroll
+  for (int s = 0; s < QS; ++s) kat[s] = l32 * CK::ROWB + 16 * ((2 * s + h) ^ kswz<DK>(l32));
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int r = 4 * h + (i16 >> 2) + 8 * u, chunk = 2 * (2 * db + ((lane >> 4) & 1)) + ((i16 >> 1) & 1);
+      vat[db][u] = CK::TILEB + r * CV::ROWB + 16 * (chunk ^ vswz32<DV>(r)) + 8 * (i16 & 1);
+    }
+#pragma unroll
+  for (int s = 0; s < QS; ++s) asm volatile("" : "+v"(qf[s]));  // waited for outside the loop
   stage(s_bt[0], 0);  // pg.n >= 1: a query always sees its own page
   wait_vmcnt0();
   __syncthreads();
 
   for (int it = 0; it < pg.n; ++it) {
     const int cur = it & 1, k0 = pg.page(it) * KT;
-    const char* sK = smem + cur * (CK::TILEB + CV::TILEB);
-    const char* sV = sK + CK::TILEB;
+    const char* page = smem + cur * (CK::TILEB + CV::TILEB);
     const bool active = k0 <= wave_pmax && (wave_pmin - (k0 + KT - 1) < win || k0 < keep);
     const int next = s_bt[min(it + 1, pg.n - 1)];
-    f32x4 s[4][2];
+    f32x16 s[2];
     if (active) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        s[t][0] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        s[t][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int ks = 0; ks < CK::KS; ++ks) {
-          const bf16x8 kf = load_k<DK>(sK, t, ks, lane);
-          s[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[0][ks], s[t][0], 0, 0, 0);
-          s[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[1][ks], s[t][1], 0, 0, 0);
+        for (int e = 0; e < 16; ++e) s[kb][e] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < QS; ++ks)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(page + kat[ks] + kb * 32 * CK::ROWB);
+          s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[kb], 0, 0, 0);
         }
-      }
     }
     if (it + 1 < pg.n) stage(next, cur ^ 1);  // DMA of the next page behind the QK^T products
     if (active) {
@@ -306,131 +321,79 @@ __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_sh
       const bool far_only = !tb || wave_pmin - (k0 + KT - 1) >= a.far;  // one bias for the whole page
       // scores in log2 units, with the page-wide bias; wave-uniform branches around whole pages of elements
       const float base = far_only ? far_bias : 0.f;
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        if (capped) {
-          float ax = 0.f;
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) ax = fmaxf(ax, fabsf(s[t][qt][r]));
-          if (!__builtin_amdgcn_ballot_w64(!(ax <= x_lim))) {
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const float x = s[t][qt][r], z = x * x;
-                const float q = __builtin_fmaf(z, __builtin_fmaf(z, __builtin_fmaf(z, q3, q2), q1), q0);
-                s[t][qt][r] = __builtin_fmaf(x, q, base);
-              }
-          } else {
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-              for (int r = 0; r < 4; ++r)
-                s[t][qt][r] = __builtin_fmaf(-2.f * shape.cap2, shape.sigma(s[t][qt][r]), base + shape.cap2);
+      const int d0 = qpos - k0 - 4 * h;  // distance of this lane's key 0; element e of block kb is key 32 kb + 8 (e / 4) + e % 4
+#define RAGK_SCORES(kb, e)  _Pragma("unroll") for (int kb = 0; kb < 2; ++kb) _Pragma("unroll") for (int e = 0; e < 16; ++e)
+      if (capped) {
+        float ax = 0.f;
+        RAGK_SCORES(kb, e) ax = fmaxf(ax, fabsf(s[kb][e]));
+        if (!__builtin_amdgcn_ballot_w64(!(ax <= x_lim))) {
+          RAGK_SCORES(kb, e) {
+            const float x = s[kb][e], z = x * x;
+            const float q = __builtin_fmaf(z, __builtin_fmaf(z, __builtin_fmaf(z, q3, q2), q1), q0);
+            s[kb][e] = __builtin_fmaf(x, q, base);
           }
-        } else if constexpr (MODE != PLAIN) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) s[t][qt][r] = __builtin_fmaf(s[t][qt][r], shape.c, base);
+        } else {
+          RAGK_SCORES(kb, e) s[kb][e] = __builtin_fmaf(-2.f * shape.cap2, shape.sigma(s[kb][e]), base + shape.cap2);
         }
+      } else if constexpr (MODE != PLAIN) {
+        RAGK_SCORES(kb, e) s[kb][e] = __builtin_fmaf(s[kb][e], shape.c, base);
       }
       if (!far_only) {
         if (pa.sb_stride) {
-#pragma unroll
-          for (int qt = 0; qt < 2; ++qt) {
-            const int d0 = ctx0 + pbase + 16 * qt + fr - k0 - 4 * fh;  // distance of this lane's key 0
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) s[t][qt][r] += s_tb[max(0, min(d0 - 16 * t - r, a.far))];
-          }
+          RAGK_SCORES(kb, e) s[kb][e] += s_tb[max(0, min(d0 - 32 * kb - 8 * (e >> 2) - (e & 3), a.far))];
         } else {
-#pragma unroll
-          for (int qt = 0; qt < 2; ++qt) {
-            const int d0 = ctx0 + pbase + 16 * qt + fr - k0 - 4 * fh;
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-              for (int r = 0; r < 4; ++r)
-                s[t][qt][r] = __builtin_fmaf(tb[max(0, min(d0 - 16 * t - r, a.far))], LOG2E, s[t][qt][r]);
-          }
+          RAGK_SCORES(kb, e)
+            s[kb][e] = __builtin_fmaf(tb[max(0, min(d0 - 32 * kb - 8 * (e >> 2) - (e & 3), a.far))], LOG2E, s[kb][e]);
         }
       }
       if (!all_visible) {
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt) {
-          const int qpos = ctx0 + pbase + 16 * qt + fr, d0 = qpos - k0 - 4 * fh;
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int d = d0 - 16 * t - r;
-              const bool ok = (d >= 0) & ((d < win) | (qpos - d < keep));
-              s[t][qt][r] = ok ? s[t][qt][r] : -INFINITY;
-            }
+        RAGK_SCORES(kb, e) {
+          const int d = d0 - 32 * kb - 8 * (e >> 2) - (e & 3);
+          const bool ok = (d >= 0) & ((d < win) | (qpos - d < keep));
+          s[kb][e] = ok ? s[kb][e] : -INFINITY;
         }
       }
+      float ls[2] = {0.f, 0.f};
       if constexpr (MODE == BOUNDED) {
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt)
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const float p = __builtin_amdgcn_exp2f(s[t][qt][r]);
-              s[t][qt][r] = p;
-              l_i[qt] += p;
-            }
-      } else {
-        float alpha[2];
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt) {
-          float mx = -INFINITY;
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[t][qt][r]);
-          mx = max_xor32(max_xor16(mx));
-          if constexpr (MODE == PLAIN) mx *= shape.c;
-          alpha[qt] = 1.f;
-          if (mx > m_i[qt] + RESCALE_LOG2) {
-            alpha[qt] = m_i[qt] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_i[qt] - mx);
-            m_i[qt] = mx;
-          }
-          const float mref = m_i[qt] == -INFINITY ? 0.f : m_i[qt];
-          float ls = 0.f;
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][qt][r], MODE == PLAIN ? shape.c : 1.f, -mref));
-              s[t][qt][r] = p;
-              ls += p;
-            }
-          l_i[qt] = l_i[qt] * alpha[qt] + ls;
+        RAGK_SCORES(kb, e) {
+          s[kb][e] = __builtin_amdgcn_exp2f(s[kb][e]);
+          ls[kb] += s[kb][e];
         }
-        if (__builtin_amdgcn_ballot_w64(alpha[0] != 1.f || alpha[1] != 1.f)) {
+        l_i += ls[0] + ls[1];
+      } else {
+        float mx = -INFINITY;
+        RAGK_SCORES(kb, e) mx = fmaxf(mx, s[kb][e]);
+        mx = max_xor32(mx);
+        if constexpr (MODE == PLAIN) mx *= shape.c;
+        float alpha = 1.f;
+        if (mx > m_i + RESCALE_LOG2) {
+          alpha = m_i == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_i - mx);
+          m_i = mx;
+        }
+        const float mref = m_i == -INFINITY ? 0.f : m_i;
+        RAGK_SCORES(kb, e) {
+          s[kb][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][e], MODE == PLAIN ? shape.c : 1.f, -mref));
+          ls[kb] += s[kb][e];
+        }
+        l_i = l_i * alpha + (ls[0] + ls[1]);
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
 #pragma unroll
-          for (int dt = 0; dt < CV::DT; ++dt)
-#pragma unroll
-            for (int qt = 0; qt < 2; ++qt) o[dt][qt] *= alpha[qt];
+          for (int db = 0; db < DB; ++db) o[db] *= alpha;
         }
       }
+#undef RAGK_SCORES
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        bf16x8 hi[2], lo[2];
+      for (int ks = 0; ks < 4; ++ks) {  // 16 keys: elements 8 (ks % 2) .. of block ks / 2, and the value rows in their order
+        const int kb = ks >> 1, e0 = 8 * (ks & 1);
+        bf16x8 hi, lo;
+        split_p((f32x4){s[kb][e0], s[kb][e0 + 1], s[kb][e0 + 2], s[kb][e0 + 3]},
+                (f32x4){s[kb][e0 + 4], s[kb][e0 + 5], s[kb][e0 + 6], s[kb][e0 + 7]}, hi, lo);
 #pragma unroll
-        for (int qt = 0; qt < 2; ++qt) split_p(s[2 * ks][qt], s[2 * ks + 1][qt], hi[qt], lo[qt]);
-#pragma unroll
-        for (int dt = 0; dt < CV::DT; ++dt) {
-          const bf16x8 vf = load_vt<DV>(sV, dt, ks, lane);
-#pragma unroll
-          for (int qt = 0; qt < 2; ++qt) o[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, hi[qt], o[dt][qt], 0, 0, 0);
-#pragma unroll
-          for (int qt = 0; qt < 2; ++qt) o[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, lo[qt], o[dt][qt], 0, 0, 0);
+        for (int db = 0; db < DB; ++db) {
+          const bf16x4 v0 = tr_read(page + vat[db][0] + ks * 16 * CV::ROWB), v1 = tr_read(page + vat[db][1] + ks * 16 * CV::ROWB);
+          const bf16x8 vf = (bf16x8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+          o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, hi, o[db], 0, 0, 0);
+          o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, lo, o[db], 0, 0, 0);
         }
       }
     }
@@ -438,34 +401,33 @@ __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_sh
     __syncthreads();
   }
 
+  l_i += __shfl_xor(l_i, 32, 64);
+  float inv = l_i > 0.f ? 1.f / l_i : 0.f;
+  // element 4 b + r of block db is column 32 db + 8 b + 4 h + r
+  const bf16_t* gq = (const bf16_t*)a.q + (size_t)(q_off + min(qi, q_len - 1)) * a.ldq + a.off_g;
+  const bool gv = a.off_g >= 0 && a.gate_vec;
+  bf16x4 gate[DB][4];
+  if (gv) {  // all of them together: one by one, where they are used, each was a trip to memory, 16 at the end of a block
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
-    float l = l_i[qt];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    float inv = l > 0.f ? 1.f / l : 0.f;
-    const int qi = pbase + 16 * qt + fr;
-    if (qi < q_len) {
-      const bf16_t* gp = nullptr;
-      if (a.off_g >= 0 && a.gate_vec) {
-        gp = (const bf16_t*)a.q + (size_t)(q_off + qi) * a.ldq + a.off_g + hq * DV + 4 * fh;
-      } else if (a.off_g >= 0) {
-        const float g = bf2f(((const bf16_t*)a.q)[(size_t)(q_off + qi) * a.ldq + a.off_g + hq]);
-        inv *= __builtin_amdgcn_rcpf(1.f + __expf(-g));
-      }
-      bf16_t* op = (bf16_t*)a.out + (size_t)(q_off + qi) * a.ldo + hq * DV + 4 * fh;
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
-      for (int dt = 0; dt < CV::DT; ++dt) {
-        f32x4 v = o[dt][qt] * inv;
-        if (gp) {
-          const bf16x4 g = *reinterpret_cast<const bf16x4*>(gp + 16 * dt);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] *= __builtin_amdgcn_rcpf(1.f + __expf(-bf2f_s(g[r])));
-        }
-        *reinterpret_cast<uint2*>(op + 16 * dt) = make_uint2(pk2bf(v[0], v[1]), pk2bf(v[2], v[3]));
-      }
-    }
+      for (int b = 0; b < 4; ++b) gate[db][b] = *reinterpret_cast<const bf16x4*>(gq + hq * DV + 32 * db + 8 * b + 4 * h);
+  } else if (a.off_g >= 0) {
+    inv *= __builtin_amdgcn_rcpf(1.f + __expf(-bf2f(gq[hq])));
   }
+  if (qi >= q_len) return;
+  bf16_t* op = (bf16_t*)a.out + (size_t)(q_off + qi) * a.ldo + hq * DV + 4 * h;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      f32x4 v = (f32x4){o[db][4 * b], o[db][4 * b + 1], o[db][4 * b + 2], o[db][4 * b + 3]} * inv;
+      if (gv) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] *= __builtin_amdgcn_rcpf(1.f + __expf(-bf2f_s(gate[db][b][r])));
+      }
+      *reinterpret_cast<uint2*>(op + 32 * db + 8 * b) = make_uint2(pk2bf(v[0], v[1]), pk2bf(v[2], v[3]));
+    }
 }
 
 // ---- decode ----

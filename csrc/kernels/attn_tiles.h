@@ -5,6 +5,8 @@
 
 namespace ragk {
 
+typedef __attribute__((ext_vector_type(16))) float f32x16;  // 32x32 MFMA accumulator
+
 constexpr int KT = 64;  // keys per tile == KV-cache page size
 constexpr int MAX_BT = 2048;  // prefill block-table row cached in LDS (128k tokens)
 constexpr float RESCALE_LOG2 = 8.f;  // deferred-rescale threshold (log2 units)
@@ -45,6 +47,13 @@ __device__ __forceinline__ int kswz(int row) {
 template <int D>
 __device__ __forceinline__ int vswz(int row) {
   return 2 * ((row / Cfg<D>::RB) & (Cfg<D>::GR - 1));
+}
+
+// V tile whose transposed reads take 32 columns (32x32 products): such a read takes two granules of four rows from each half
+// of a wave, so granules move by pairs, and the four rows' pairs lie in different banks
+template <int D>
+__device__ __forceinline__ int vswz32(int row) {
+  return 4 * ((row / Cfg<D>::RB) & (Cfg<D>::GR / 2 - 1) & 3);
 }
 
 __device__ __forceinline__ bf16x4 tr_read(const char* p) {

@@ -228,6 +228,27 @@ struct ChunkArgs {
 
 constexpr int CQ = 64;  // chunk length
 
+// Order of a whole scan's blocks: sequences by length, the longest first, so that the work that starts last is the shortest. All
+// of up to three blocks a CU start together, so their order decides what a CU holds: the dispatcher deals them out in rounds of
+// one block a CU, and the rounds run up and down through the lengths, the last full one up, so that an incomplete one adds to
+// the CUs with the least. 64 heads, in the sequences' own order and sorted: 1900, 1253, 1237, 1681, 1846 tokens 138 -> 119 us
+// (sorted down only: 123), 1500, 1086, 1456 88 -> 82, 128 heads of the five 225 -> 205; other mixes within 2 %.
+constexpr int DEALT = 256;  // CUs
+__device__ __forceinline__ int dealt_place(int b, int n) {  // block b's place among n sorted ones
+  const int round = b / DEALT, full = n / DEALT;
+  return round < full && (full - 1 - round) % 2 == 0 ? (2 * round + 1) * DEALT - 1 - b : b;
+}
+// the k-th longest of up to 64 sequences (more of them take the chip many rounds anyway)
+__device__ __forceinline__ int kth_longest(const SeqArgs& q, int k, int lane) {
+  const int len = lane < q.S ? q.cu_q[lane + 1] - q.cu_q[lane] : 0;
+  int rank = 0;
+  for (int j = 0; j < q.S; ++j) {
+    const int other = __builtin_amdgcn_readlane(len, j);
+    rank += other > len || (other == len && j < lane);
+  }
+  return __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < q.S && rank == k));
+}
+
 // inclusive sum over the wave's lanes, on the VALU (row shifts, then the two row broadcasts)
 template <int CTRL, int ROWS>
 __device__ __forceinline__ float dpp_add(float v) {
@@ -278,8 +299,14 @@ __global__ __launch_bounds__(256, NP <= 128 ? 2 : 1) void scan_chunk_kernel(Chun
 
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tid = threadIdx.x;
   const int fr = lane & 15, fh = lane >> 4;
-  const int h = blockIdx.x, seq = PASS ? blockIdx.y / a.nseg : blockIdx.y, seg = PASS ? blockIdx.y % a.nseg : 0;
-  const int p0 = blockIdx.z * PS;
+  int h = blockIdx.x, seq = PASS ? blockIdx.y / a.nseg : blockIdx.y, seg = PASS ? blockIdx.y % a.nseg : 0, slice = blockIdx.z;
+  if (PASS == 0 && a.q.S > 1 && a.q.S <= 64 && a.q.cu_q) {  // sorted blocks run through heads, slices, sequences
+    const int b = h + a.H * (seq + a.q.S * slice), per = a.H * gridDim.z, u = dealt_place(b, per * a.q.S), k = u / per;
+    seq = kth_longest(a.q, k, lane);
+    h = u % a.H;
+    slice = (u - k * per) / a.H;
+  }
+  const int p0 = slice * PS;
   const int g = h / (a.H / a.G);
   int t0, n;
   bool fresh;
@@ -800,8 +827,8 @@ RAGK_API int ragk_ssm_scan_chunk(const int* cu_q, const int* kv_lens, const int*
     return (int)hipErrorInvalidValue;
   const ChunkArgs a{{cu_q, kv_lens, states, T, S}, (const bf16_t*)xbc, ch, (const bf16_t*)row, ld, off_dt, dt_bias, A, D,
                     ssm_state, (bf16_t*)y, H, P, N, G, nseg, seg_len, seg_ws, seg_ws + (size_t)S * (nseg + 1) * H * N * P};
-  // narrow column slices while three of their blocks a CU are resident together: 320 (head, sequence) pairs of 1900 tokens
-  // 154 us against 171, 64 of 4000 199 against 279
+  // narrow column slices while three of their blocks a CU are resident together: 192 (head, sequence) pairs of 1086 to 1500
+  // tokens 82 us against 93, 384 of 300 to 2000 109 against 121, 512 of 1446 to 1900 190 against 127
   // (segments fill the chip, and what two slices both compute then counts)
   const bool narrow = P <= 32 || (g_scan_cols ? g_scan_cols == 32 : nseg == 1 && (long long)H * S * ((P + 63) / 64) <= 384);
 #define RAGK_SC(NPV) return narrow ? launch_scan_chunk<NPV, 32>(a, st) : launch_scan_chunk<NPV, 64>(a, st)

@@ -1179,7 +1179,7 @@ def encoder_few_ok(cfg, T, B):
     layers of 384 columns 103 / 197 at 5 rows, 111 / 202 at 14, 147 / 205 at 32; 24 layers of 1024 600 / 711 at 5 rows, 705 / 761
     at 16, 777 / 790 at 17, but 855 / 820 at 24 and 958 / 839 at 32."""
     H = cfg.hidden_size
-    return (B == 1 and 1 <= T <= FEW_ROWS and H <= FEW_COLS and T * H <= FEW_SIZE
+    return (B == 1 and 1 <= T <= FEW_ROWS and H <= FEW_COLS and T * H <= FEW_SIZE and cfg.num_hidden_layers > 0
             and H // cfg.num_attention_heads in (32, 64))
 
 

@@ -61,6 +61,18 @@ def test_short_sequence(native, monkeypatch, T, hidden, heads, inter, pooling, k
     assert err[0] < 0.01 and err[0] < 1.3 * err[1] + 1e-4, err
 
 
+def test_no_layers(native):
+    """Embeddings, their norm and the pooling only: the launches of a layer have nothing to begin with."""
+    cfg = E.EncoderConfig(model_type="bert", vocab_size=500, hidden_size=128, num_hidden_layers=0, num_attention_heads=4,
+                          intermediate_size=128, max_position_embeddings=64, pooling="mean")
+    m = E.EncoderModel(cfg, E.EncoderWeights.random(cfg, DEV, seed=1), DEV)
+    ids, out = np.arange(5, 12, dtype=np.int32), torch.zeros(1, 128, device=DEV)
+    m.embed_into(ids, np.array([7], dtype=np.int64), out, np.array([0]))
+    ref = exact(cfg, m.w, torch.from_numpy(ids).to(DEV).long(), m.first_position)
+    # rows rounded to bf16 (2^-8 of a value), pooled and scaled
+    assert ((out.to(F64) - ref).norm() / ref.norm()).item() < 2.0 ** -8
+
+
 def test_library_refuses_what_it_cannot_take(native):
     """Nothing is launched for more rows or columns than there is room for, a head size of its own, or no ids."""
     import ctypes

@@ -1,0 +1,54 @@
+"""Products cut into two plans by columns: where the rule cuts (CPU), and that every epilogue's operands follow the cut (GPU)."""
+import pytest
+import torch
+
+from rag_llm_k8s_amd.ops import native as n
+
+
+def test_rule():
+    cut = n.gemm_columns(1777, 28672, 4096, 256)  # three rounds of 256 x 256 tiles and 16 more of them
+    assert cut and cut % 256 == 0
+    assert n.gemm_columns(1777, 28672, 128, 256) == 0  # three K-tiles at least
+    assert n.gemm_columns(2048, 8192, 4096, 256) == 0  # one round exactly
+    for M in (65, 300, 529, 1129, 1777, 2813, 4072, 7917, 14076):
+        for rows, K in ((28672, 4096), (11264, 2048), (8512, 2048), (6144, 4096), (3072, 1024)):
+            c = n.gemm_columns(M, rows, K, 256)
+            assert c % 256 == 0 and 0 <= c < rows
+            if c:
+                whole, a, b = (n._timed_plan(M, r, K, True, 256)[0] for r in (rows, c, rows - c))
+                assert a + b < n.COLUMNS_GAIN * whole
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,rows,cut", [(65, 320, 256), (200, 1152, 512), (257, 1024, 768)])
+@pytest.mark.parametrize("epi", ["none", "bias", "resid", "bias_resid", "bias_gelu", "silu_mul", "glu_clip"])
+def test_operands_follow_the_cut(native, monkeypatch, M, rows, cut, epi):
+    K = 256
+    g = torch.Generator().manual_seed(M)
+    pair = epi in native.PAIR_EPI
+    if pair:
+        rows = -(-rows // 128) * 128
+        N = rows // 2
+    else:
+        N = rows
+    rand = lambda *s: torch.randn(*s, generator=g).cuda()  # noqa: E731
+    x, w = rand(M, K).bfloat16(), (rand(rows, K) * K ** -0.5).bfloat16()
+    bias = rand(N).bfloat16() if "bias" in epi else None
+    if epi == "glu_clip":
+        bias = torch.tensor([7.0, 1.7, 1.0], device="cuda")
+    res = rand(M, N).bfloat16() if "resid" in epi else None
+    for f32 in ((False,) if pair else (False, True)):
+        outs = []
+        for c in (cut, 0):
+            monkeypatch.setattr(native, "gemm_columns", lambda *a, c=c: c)
+            wide = torch.full((M, N + 64), 3.0, device="cuda", dtype=torch.float32 if f32 else torch.bfloat16)
+            out = wide[:, :N]
+            if res is not None and not f32:
+                out.copy_(res)  # in place, as the residual stream is
+            native.gemm(x, w, bias=bias, resid=out if res is not None and not f32 else res, epi=epi, out=out, out_f32=f32)
+            assert bool((wide[:, N:] == 3.0).all())
+            outs.append(out.double())
+        # fp32 sums of 256 products in another order (a K-split may differ): 2^-16 of the values' size, and half a bf16 unit of
+        # either side where the result is rounded (2^-8 each)
+        d = (outs[0] - outs[1]).abs()
+        assert bool((d <= (2.0 ** -16 if f32 else 2.0 ** -7) * outs[1].abs() + 2.0 ** -15).all()), (epi, f32, float(d.max()))

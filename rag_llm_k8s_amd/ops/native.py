@@ -425,9 +425,16 @@ def _timed_plan(M, rows, K, w4, cus):
         # 1.05 of it (827 x 28672 x 4096 188 us against 180), the others 0.69 to 1.02, 0.88 in the mean
         if t2 < 0.96 * t:
             t, plan = t2, ((0, m1, 0, 1), (m1, M, mi, S))
-    # its smaller tiles; against two launches only well ahead (14076 x 4096 x 4096: both ways 343 us, modelled 0.985)
-    t3, mi = min((_tiles_us(M, rows, K, mi, 1, cus), mi) for mi in W4_TILES[1:])
-    if t3 < (0.97 if len(plan) > 1 else 1) * t:
+    # its smaller tiles, where they are well ahead. Against 256 rows: of 70 products of 1500 to 16384 rows those modelled at 0.97
+    # to 1 took 0.985 to 1.10 of it, 192 rows from 0.95 on 0.97 to 1.04, the others 0.88 to 0.96. Where the last round of 256 rows
+    # is all but empty 224 came out a little better than that (14076 x 28672 x 4096, 24 rounds and 16 tiles: modelled 0.989, 2288
+    # -> 2214 us; three more 1.00 to 1.01). Against two launches: 14076 x 4096 x 4096 both ways 343 us, modelled 0.985.
+    limit = {38: 0.97, 39: 0.97} if len(plan) > 1 else {}
+    if plan == ((0, M, 0, 1),):
+        tail = -(-M // 256) * tn % cus
+        limit = {38: 0.95, 39: 0.99 if 0 < tail < cus // 4 else 0.97}
+    score, t3, mi = min((us / limit.get(mi, 1), us, mi) for mi in W4_TILES[1:] for us in [_tiles_us(M, rows, K, mi, 1, cus)])
+    if score < t:
         t, plan = t3, ((0, M, mi, 1),)
     return t, plan
 

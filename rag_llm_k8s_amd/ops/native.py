@@ -239,7 +239,7 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
                     wc, o = w[c0:c1], slice(c0 // 2, c1 // 2) if epi in PAIR_EPI else slice(c0, c1)
                     oc, rc = out[:, o], resid[:, o] if resid is not None else None
                     bc = bias[o] if bias is not None and epi != "glu_clip" else bias  # (glu_clip: the unit's parameters)
-                for r0, r1, mi, S in gemm_plan(M, c1 - c0, K, w4, _cu_count()):
+                for r0, r1, mi, S in gemm_plan(M, c1 - c0, K, w4, _cu_count(), not cols):
                     _gemm_rows(x, wc, bc, rc, epi, oc, out_f32, r0, r1, mi, S)
             return out
     if path == 0:
@@ -356,11 +356,12 @@ def _tiles_us(M, rows, K, mi, S, cus):
     return launch + rounds * (-(-(K // 64) // S) * (a + b * items / (rounds * cus)) + epilogue)
 
 
-def _mid_best(M, rows, K, cus, slab_us, launch_us, even=False):
-    """(time, mi, S) of the best gemm_mid launch; a split costs launch_us and slab_us per slab value (even: equal slabs)."""
+def _mid_best(M, rows, K, cus, slab_us, launch_us, even=False, most=16):
+    """(time, mi, S) of the best gemm_mid launch of up to `most` slabs; a split costs launch_us and slab_us per slab value (even:
+    equal slabs)."""
     best = (float("inf"), 0, 1)
     for mi in MID_TILES:
-        for S in range(1, 17):
+        for S in range(1, most + 1):
             if S > 1 and K // 64 // S < 4:
                 break
             if even and K // 64 % S:
@@ -371,30 +372,35 @@ def _mid_best(M, rows, K, cus, slab_us, launch_us, even=False):
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_plan(M, rows, K, w4, cus):
-    """Launches of one product with M > 64 rows: [(first row, end, mi, S)], mi as in MID_US. Candidates: gemm_mid alone;
-    gemm_w4 alone (w4: its operands fit), at 256, 224 or 192 rows a tile; its 256-row tiles on as many rows as fill whole rounds
-    and gemm_mid on the rest. Where they meet (us, N = K = 4096): 300 rows 24 against gemm_w4's 69, 1777 rows 53 against 66 (192
-    rows a tile); at N = 28672 of 1777 rows gemm_w4 322 against 350 (its wave tiles read less LDS per MFMA)."""
-    return _timed_plan(M, rows, K, w4, cus)[1]
+def gemm_plan(M, rows, K, w4, cus, split=True):
+    """Launches of one product with M > 64 rows: [(first row, end, mi, S)], mi as in MID_US (split: S may be above 1). Candidates:
+    gemm_mid alone; gemm_w4 alone (w4: its operands fit), at 256, 224 or 192 rows a tile; its 256-row tiles on as many rows as
+    fill whole rounds and gemm_mid on the rest. Where they meet (us, N = K = 4096): 300 rows 24 against gemm_w4's 69, 1777 rows 53
+    against 66 (192 rows a tile); at N = 28672 of 1777 rows gemm_w4 322 against 350 (its wave tiles read less LDS per MFMA)."""
+    return _timed_plan(M, rows, K, w4, cus, split)[1]
 
 
 @functools.lru_cache(maxsize=4096)
 def gemm_columns(M, rows, K, cus):
     """Weight rows (a multiple of 256) that one plan takes, the others a second one, or 0: where all tiles are little more than
     whole rounds (1777 x 28672: 784 of 256 x 256, three rounds and 16), gemm_w4 on as many columns of tiles as fill the rounds
-    and the best plan for the rest. Us: 1777 x 28672 x 4096 322 -> 307, 7917 x 11264 x 2048 280 -> 274, 1548 x 28672 x 4096
-    302 -> 276. It cuts 107 of 4000 products drawn from 13 weights at 66 to 16000 rows; 40 of these took 0.87 to 1.02 of the
-    time, 0.94 in the mean (those modelled at 0.95 to 0.96: 0.92 to 1.02). Within a prompt's other work the card's power takes a
-    part of that back: four layers of the first 3636 -> 3599 us, of the second 3606 both ways."""
-    t, n1 = COLUMNS_GAIN * _timed_plan(M, rows, K, True, cus)[0], 0
+    and the best plan for the rest. Only products that are summed over K in one piece, with and without the cut: then it changes
+    no bit, and gemm_rope_kv and the native encoder forward, which do not ask here, agree with gemm. (Encoders of 384 and 1024
+    columns are never cut, of the widths that gemm_rope_kv serves 6144 x 4096 at 2690 .. 2880 rows, for 2 %.) Us: 1777 x 28672 x
+    4096 322 -> 310, 1548 x 28672 x 4096 301 -> 281, 1297 x 11264 x 2048 62 -> 56. It cuts 30 of 1284 products drawn from 12
+    weights at 66 to 16000 rows; these took 0.81 to 1.015 of the time, 0.95 in the mean (those modelled at 0.95 to 0.96: 0.95 to
+    1.015)."""
     if K % 64 or K < 192:
         return 0
+    t, plan = _timed_plan(M, rows, K, True, cus)
+    if any(S > 1 for _, _, _, S in plan):
+        return 0
+    t, n1 = COLUMNS_GAIN * t, 0
     for mi in W4_TILES:
         tiles_m = -(-M // (32 * (mi & 15 or 8)))
         c = tiles_m * -(-rows // 256) // cus * cus // tiles_m * 256
         if 0 < c < rows:
-            t2 = _timed_plan(M, c, K, True, cus)[0] + _timed_plan(M, rows - c, K, True, cus)[0]
+            t2 = _timed_plan(M, c, K, True, cus, False)[0] + _timed_plan(M, rows - c, K, True, cus, False)[0]
             if t2 < t:
                 t, n1 = t2, c
     return n1
@@ -404,9 +410,10 @@ COLUMNS_GAIN = 0.96  # modelled time that a second launch has to save
 
 
 @functools.lru_cache(maxsize=8192)
-def _timed_plan(M, rows, K, w4, cus):
+def _timed_plan(M, rows, K, w4, cus, split=True):
     """(modelled time, launches) of gemm_plan."""
-    t, mi, S = _mid_best(M, rows, K, cus, SLAB_US, 3.0)
+    most = 16 if split else 1
+    t, mi, S = _mid_best(M, rows, K, cus, SLAB_US, 3.0, most=most)
     plan = ((0, M, mi, S),)
     if not w4 or K % 64 or K < 192:  # gemm_w4's ring needs three K-tiles
         return t, plan
@@ -419,7 +426,7 @@ def _timed_plan(M, rows, K, w4, cus):
         m1 = r * cus // tn * 256
         if not 0 < m1 < M:
             continue
-        t2, mi, S = _mid_best(M - m1, rows, K, cus, SLAB_US, 3.0)
+        t2, mi, S = _mid_best(M - m1, rows, K, cus, SLAB_US, 3.0, most=most)
         t2 += _tiles_us(m1, rows, K, 0, 1, cus)
         # two launches have to earn their keep: of 57 such plans the five modelled at 0.96 to 0.97 of gemm_w4 alone took 0.99 to
         # 1.05 of it (827 x 28672 x 4096 188 us against 180), the others 0.69 to 1.02, 0.88 in the mean

@@ -1,8 +1,11 @@
 """Products cut into two plans by columns: where the rule cuts (CPU), and that every epilogue's operands follow the cut (GPU)."""
+import random
+
 import pytest
 import torch
 
 from rag_llm_k8s_amd.ops import native as n
+from rag_llm_k8s_amd.ops import reference as R
 
 
 def test_rule():
@@ -15,8 +18,41 @@ def test_rule():
             c = n.gemm_columns(M, rows, K, 256)
             assert c % 256 == 0 and 0 <= c < rows
             if c:
-                whole, a, b = (n._timed_plan(M, r, K, True, 256)[0] for r in (rows, c, rows - c))
+                whole, a, b = (n._timed_plan(M, r, K, True, 256, s)[0] for r, s in ((rows, True), (c, False), (rows - c, False)))
                 assert a + b < n.COLUMNS_GAIN * whole
+
+
+def test_a_cut_splits_no_sum():
+    """Every launch of a cut product, and every launch that it would have without the cut, sums over K in one piece."""
+    r = random.Random(4)
+    cuts = 0
+    for _ in range(3000):
+        M, (rows, K) = int(2 ** r.uniform(6.05, 14)), r.choice(((28672, 4096), (6144, 4096), (16704, 4096), (11264, 2048), (8512, 2048)))
+        c = n.gemm_columns(M, rows, K, 256)
+        plans = [n.gemm_plan(M, rows, K, True, 256)]
+        if c:
+            cuts += 1
+            plans += [n.gemm_plan(M, m, K, True, 256, False) for m in (c, rows - c)]
+            assert all(S == 1 for p in plans for _, _, _, S in p), (M, rows, K, c)
+    assert cuts > 20
+
+
+# cut at 9216 of 11264 columns; at 4352 of 6144 (once at 5888, with the last two heads' sums split); not cut
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,Hq,Hkv,K", [(1297, 72, 8, 2048), (2692, 32, 8, 4096), (1500, 32, 8, 4096)])
+def test_rotated_projection_agrees_with_a_cut_product(native, M, Hq, Hkv, K):
+    """gemm_rope_kv, whose launches are not cut, is gemm followed by rope_kv bit for bit, cached rows included."""
+    N, g = (Hq + 2 * Hkv) * 128, torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    cos, sin = (t.cuda() for t in R.rope_tables(128, 4096))
+    pos = torch.arange(M, device="cuda").int()
+    slots = torch.randperm((M // 64 + 2) * 64, device="cuda", generator=g)[:M].int()
+    kc, vc, kc2, vc2 = torch.zeros(4, M // 64 + 2, Hkv, 64, 128, device="cuda").bfloat16()
+    assert (native.gemm_columns(M, N, K, 256) > 0) == (M != 1500)
+    got, ref = native.gemm_rope_kv(x, w, pos, cos, sin, slots, kc, vc, Hq, Hkv, 128), native.gemm(x, w)
+    native.rope_kv(ref, pos, cos, sin, slots, kc2, vc2, Hq, Hkv, 128)
+    assert torch.equal(got, ref) and torch.equal(kc, kc2) and torch.equal(vc, vc2)
 
 
 @pytest.mark.gpu

@@ -58,7 +58,8 @@ class EmbeddingEngine:
         if n == 0:
             return out
         if n == 1:  # a question: nothing to order or cut (30 us of host time around a forward of 110)
-            self.model.embed_into(ids[:int(lens[0])], np.asarray(lens, dtype=np.int64), out, np.array([row0]))
+            # (a numpy array of whatever holds the ids, as for several texts)
+            self.model.embed_into(np.concatenate([ids[:lens[0]]]), lens.astype(np.int64), out, np.array([row0]))
             return out
         starts = np.zeros(n + 1, dtype=np.int64)
         np.cumsum(lens, out=starts[1:])

@@ -28,3 +28,18 @@ def test_pipelined_embed_equals_one_by_one(tmp_path, monkeypatch):
     assert got.shape == (300, 64)
     assert torch.allclose(got, ref, atol=2e-3), (got - ref).abs().max()
     assert torch.allclose(emb.embed_ids(emb.tokenize(texts)), got, atol=1e-5)
+
+
+def test_one_text_takes_the_ids_that_two_take():
+    """int32 token ids as a numpy array, a tensor on the host, or every other element of an array: the same embeddings."""
+    from rag_llm_k8s_amd.engine import encoder_engine as EE
+    from rag_llm_k8s_amd.models import encoder as E
+
+    cfg = E.EncoderConfig(vocab_size=100, hidden_size=64, num_hidden_layers=1, num_attention_heads=4, intermediate_size=128)
+    emb = EE.EmbeddingEngine(E.EncoderModel(cfg, E.EncoderWeights.random(cfg, "cpu", seed=3), "cpu"), None)
+    ids = np.arange(5, 25, dtype=np.int32)
+    for lens in ([20], [12, 8]):
+        lens = np.array(lens, dtype=np.int32)
+        want = emb.embed_flat(ids, lens)
+        for same in (torch.from_numpy(ids), np.repeat(ids, 2)[::2]):
+            assert torch.equal(emb.embed_flat(same, lens), want)

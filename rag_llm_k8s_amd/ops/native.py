@@ -1225,6 +1225,13 @@ FEW_SIZE = 16384  # rows x columns: the blocks repeat the rows' work
 PUT_INTS = 3840
 
 
+def _req_no_capture():
+    """Integers of host memory that travel as kernel arguments would be frozen into a graph, which repeats them whatever the
+    caller's memory holds by then; a copy of that memory refuses a capture by itself."""
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("an encoder forward of ids in host memory cannot be captured")
+
+
 def encoder_few_ok(cfg, T, B):
     """Whether a batch takes the four launches a layer of csrc/kernels/encoder_few.hip. Us a call against seven launches: six
     layers of 384 columns 103 / 197 at 5 rows, 111 / 202 at 14, 147 / 205 at 32; 24 layers of 1024 600 / 711 at 5 rows, 705 / 761
@@ -1266,6 +1273,7 @@ def encoder_few(cfg, weights, ids, first_pos, out):
         c.ids = ids.data_ptr()
     else:
         _req(ids.dtype == "int32" and ids.flags.c_contiguous, "ids int32")
+        _req_no_capture()
         c.ids_host = ids.ctypes.data
     check(_lib.lib().ragk_encoder_forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
     return out
@@ -1298,6 +1306,7 @@ def encoder_forward(cfg, weights, ids, lens, first_pos, out, rows):
     host = np.concatenate(parts).astype(np.int32, copy=False)
     L = _lib.lib()
     if len(host) <= PUT_INTS:
+        _req_no_capture()
         ints = torch.empty(len(host), dtype=torch.int32, device=dev)
         check(L.ragk_put_ints(host.ctypes.data, len(host), ints.data_ptr(), stream_ptr()), "ragk_put_ints")
     else:

@@ -87,3 +87,21 @@ def test_edited_weights(native):
     assert torch.equal(out, m.forward_packed(torch.from_numpy(ids).to(DEV), [100]))
     m.w.layers[0]["ln1_g"] = m.w.layers[0]["ln1_g"].cpu()
     assert not native.encoder_forward_ok(m.cfg, m.w)
+
+
+@pytest.mark.parametrize("lens", [[14], [14, 30], [300] * 4])
+def test_host_ids_are_not_frozen_into_a_graph(native, lens):
+    """Ids read from host memory when the call is made: a graph would repeat them whatever the caller's buffer holds by then, so
+    a capture is refused (and given up by its owner); the same call afterwards works."""
+    m = model("mean")
+    ids, out = np.arange(5, 5 + sum(lens), dtype=np.int32) % 500, torch.zeros(len(lens), 256, device=DEV)
+    args = ids, np.asarray(lens, dtype=np.int64), out, np.arange(len(lens))
+    m.embed_into(*args)
+    want = out.clone()
+    out.zero_()
+    torch.cuda.synchronize()
+    with pytest.raises(RuntimeError):
+        with torch.cuda.graph(torch.cuda.CUDAGraph()):
+            m.embed_into(*args)
+    m.embed_into(*args)
+    assert torch.equal(out, want)

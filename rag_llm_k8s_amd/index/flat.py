@@ -31,6 +31,7 @@ class FlatL2Index:
 
             self._n = native
             self._xt = torch.zeros(self.d, self._cap, dtype=torch.float32, device=self.device)
+            native.search_block()  # into the pool, ahead of the first search
         else:
             self._n = None
             self._xb = torch.zeros(self._cap, self.d, dtype=torch.float32)

@@ -174,6 +174,7 @@ class IVFFlatIndex:
         need = self._size + counts
         if self._xt is None or bool((need > self._lcap).any()):
             self._regrow(need)
+            native.search_block()  # into the pool, ahead of the first search
         order = np.argsort(a, kind="stable")
         first = np.concatenate([[0], np.cumsum(counts)[:-1]])
         rank = np.empty(len(a), np.int64)

@@ -388,7 +388,7 @@ def gemm_columns(M, rows, K, cus):
     no bit, and gemm_rope_kv and the native encoder forward, which do not ask here, agree with gemm. (Encoders of 384 and 1024
     columns are never cut, of the widths that gemm_rope_kv serves 6144 x 4096 at 2690 .. 2880 rows, for 2 %.) Us: 1777 x 28672 x
     4096 322 -> 310, 1548 x 28672 x 4096 301 -> 281, 1297 x 11264 x 2048 62 -> 56. It cuts 30 of 1284 products drawn from 12
-    weights at 66 to 16000 rows; these took 0.81 to 1.015 of the time, 0.95 in the mean (those modelled at 0.95 to 0.96: 0.95 to
+    weights at 66 to 16000 rows; these took 0.81 to 1.015 of the time, 0.95 in the mean (those modelled at 0.95 to 0.96: 0.96 to
     1.015)."""
     if K % 64 or K < 192:
         return 0
@@ -433,13 +433,12 @@ def _timed_plan(M, rows, K, w4, cus, split=True):
         if t2 < 0.96 * t:
             t, plan = t2, ((0, m1, 0, 1), (m1, M, mi, S))
     # its smaller tiles, where they are well ahead. Against 256 rows: of 70 products of 1500 to 16384 rows those modelled at 0.97
-    # to 1 took 0.985 to 1.10 of it, 192 rows from 0.95 on 0.97 to 1.04, the others 0.88 to 0.96. Where the last round of 256 rows
-    # is all but empty 224 came out a little better than that (14076 x 28672 x 4096, 24 rounds and 16 tiles: modelled 0.989, 2288
-    # -> 2214 us; three more 1.00 to 1.01). Against two launches: 14076 x 4096 x 4096 both ways 343 us, modelled 0.985.
+    # to 1 took 0.985 to 1.10 of it, 192 rows from 0.95 on 0.97 to 1.04, the others 0.88 to 0.96; 44 more of 5348 to 16092 rows
+    # whose last round of 256 rows is all but empty, 224 rows modelled at 0.97 to 0.99, took 0.98 to 1.08 of it, 1.009 in the mean
+    # (14076 x 28672 x 4096 2282 against 2255 us). Against two launches: 14076 x 4096 x 4096 both ways 343 us, modelled 0.985.
     limit = {38: 0.97, 39: 0.97} if len(plan) > 1 else {}
     if plan == ((0, M, 0, 1),):
-        tail = -(-M // 256) * tn % cus
-        limit = {38: 0.95, 39: 0.99 if 0 < tail < cus // 4 else 0.97}
+        limit = {38: 0.95, 39: 0.97}
     score, t3, mi = min((us / limit.get(mi, 1), us, mi) for mi in W4_TILES[1:] for us in [_tiles_us(M, rows, K, mi, 1, cus)])
     if score < t:
         t, plan = t3, ((0, M, mi, 1),)

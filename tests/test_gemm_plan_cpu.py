@@ -94,3 +94,16 @@ def test_slices_follow_the_block_count(monkeypatch):
     b = n.gemm_part_slabs(1, 4096, 4096)
     monkeypatch.setattr(n, "PART_MIN_BLOCKS", 512)
     assert a != b and n.gemm_part_slabs(1, 4096, 4096) == a
+
+
+def test_smaller_tiles_only_well_ahead():
+    """224 and 192 rows a tile instead of 256 from one modelled gain on for every product, also where the last round is all but
+    empty (14076 x 28672 x 4096: 24 rounds and 16 tiles)."""
+    r = random.Random(5)
+    sizes = [(14076, 28672, 4096), (15284, 18560, 4096), (8908, 16704, 4096)]
+    sizes += [(r.randint(1500, 16384), 256 * r.randint(4, 112), 64 * r.randint(16, 64)) for _ in range(500)]
+    for M, rows, K in sizes:
+        (_, _, mi, _), *rest = n.gemm_plan(M, rows, K, True, 256)
+        t = n._tiles_us(M, rows, K, 0, 1, 256)
+        if mi in (38, 39) and not rest and n._mid_best(M, rows, K, 256, n.SLAB_US, 3.0)[0] >= t:
+            assert n._tiles_us(M, rows, K, mi, 1, 256) < {38: 0.95, 39: 0.97}[mi] * t, (M, rows, K)

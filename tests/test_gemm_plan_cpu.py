@@ -19,10 +19,10 @@ def test_plans_cover_every_row_with_legal_launches():
             for r0, r1, mi, S in plan:
                 assert r0 == at < r1
                 at = r1
-                assert (mi in n.MID_US or (mi == 0 and w4 and S == 1)) and 1 <= S <= max(1, K // 256)
+                assert (mi in n.MID_TILES or (mi in n.W4_TILES and w4 and S == 1)) and 1 <= S <= max(1, K // 256)
             assert at == M
         S, mi = n._slab_best(M, rows, K, 256)
-        assert S == 1 or (K % (64 * S) == 0 and K // S >= 256 and (mi in n.MID_US or mi == 0))
+        assert S == 1 or (K % (64 * S) == 0 and K // S >= 256 and (mi in n.MID_TILES or mi == 0))
 
 
 def test_launch_model_prefers_full_rounds():
@@ -39,7 +39,7 @@ def test_short_inner_dimension_stays_off_the_long_ring():
     for H, I in ((128, 512), (128, 1024), (128, 2048)):
         for T in (65, 300, 4096, 24576, 49152, 65536):
             for N, K in ((3 * H, H), (H, H), (I, H), (H, I)):
-                assert all(mi in n.MID_US for _, _, mi, _ in n.gemm_plan(T, N, K, True, 256)) or K >= 192
+                assert all(mi in n.MID_TILES for _, _, mi, _ in n.gemm_plan(T, N, K, True, 256)) or K >= 192
 
 
 def test_work_lists_of_prompts():

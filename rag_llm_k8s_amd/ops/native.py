@@ -234,11 +234,7 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
             w4 = fits and (N % 128 == 0 if epi in PAIR_EPI else N % 8 == 0)
             cols = gemm_columns(M, rows, K, _cu_count()) if w4 else 0
             for c0, c1 in ((0, cols), (cols, rows)) if cols else ((0, rows),):
-                wc, bc, rc, oc = w, bias, resid, out
-                if cols:
-                    wc, o = w[c0:c1], slice(c0 // 2, c1 // 2) if epi in PAIR_EPI else slice(c0, c1)
-                    oc, rc = out[:, o], resid[:, o] if resid is not None else None
-                    bc = bias[o] if bias is not None and epi != "glu_clip" else bias  # (glu_clip: the unit's parameters)
+                wc, bc, rc, oc = _columns(w, bias, resid, out, epi, c0, c1) if cols else (w, bias, resid, out)
                 for r0, r1, mi, S in gemm_plan(M, c1 - c0, K, w4, _cu_count(), not cols):
                     _gemm_rows(x, wc, bc, rc, epi, oc, out_f32, r0, r1, mi, S)
             return out
@@ -297,6 +293,13 @@ def gemm_mid(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, m
     _req(out.shape == (M, N) and out.stride(1) == 1, "gemm_mid out")
     _gemm_rows(x, w, bias, resid, epi, out, out_f32, 0, M, mi, S)
     return out
+
+
+def _columns(w, bias, resid, out, epi, c0, c1):
+    """What rows c0 .. c1 of a product's weight take of its operands. A bias may have any shape; what the epilogue does not read
+    stays as it is (glu_clip's bias holds the unit's parameters)."""
+    o = slice(c0 // 2, c1 // 2) if epi in PAIR_EPI else slice(c0, c1)
+    return (w[c0:c1], bias.view(-1)[o] if "bias" in epi else bias, resid[:, o] if "resid" in epi else resid, out[:, o])
 
 
 _TILE_LD = ~(2 ** 21 - 8)  # bits that no row stride has which _tile_rows leaves: starts off 16 bytes, rows from 4 MB on

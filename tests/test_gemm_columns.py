@@ -37,6 +37,23 @@ def test_a_cut_splits_no_sum():
     assert cuts > 20
 
 
+def test_operands_of_a_cut():
+    """Every piece's operands begin at its columns and hold them all, a bias of shape [N], [1, N] or [N, 1] alike."""
+    M, N, K = 3, 768, 64
+    w, r, out = torch.zeros(N, K).bfloat16(), torch.zeros(M, N + 8).bfloat16()[:, :N], torch.zeros(M, N)
+    for shape in ((N,), (1, N), (N, 1)):
+        b = torch.arange(N).bfloat16().view(shape)
+        for c0, c1 in ((0, 512), (512, N)):
+            wc, bc, rc, oc = n._columns(w, b, r, out, "bias_resid", c0, c1)
+            for part, whole, at in ((wc, w, c0 * K), (bc, b, c0), (rc, r, c0), (oc, out, c0)):
+                assert part.data_ptr() == whole.data_ptr() + at * whole.element_size()
+            assert wc.shape == (c1 - c0, K) and bc.numel() == c1 - c0 and rc.shape == oc.shape == (M, c1 - c0)
+    par, row = torch.zeros(3), torch.zeros(5)  # (not read as a bias; not read at all)
+    wc, bc, rc, oc = n._columns(w, par, row, out[:, :N // 2], "glu_clip", 512, N)
+    assert bc is par and rc is row and wc.shape[0] == 256 and oc.shape == (M, 128)
+    assert oc.data_ptr() == out.data_ptr() + 256 * 4
+
+
 # cut at 9216 of 11264 columns; at 4352 of 6144 (once at 5888, with the last two heads' sums split); not cut
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,Hq,Hkv,K", [(1297, 72, 8, 2048), (2692, 32, 8, 4096), (1500, 32, 8, 4096)])

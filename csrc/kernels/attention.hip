@@ -1403,7 +1403,8 @@ hipError_t launch_prefill(PrefillArgs a, int n_tiles, hipStream_t st) {
     }
   }
   if constexpr (!CAUSAL && !PAGED && GB == 1 && D <= 64) {
-    if (G == 1 && ((uintptr_t)a.k | (uintptr_t)a.v) % 16 == 0 && a.kv_stride % 8 == 0) {
+    // rows on 16 bytes, a tile's 64 within 31-bit offsets
+    if (G == 1 && ((uintptr_t)a.k | (uintptr_t)a.v) % 16 == 0 && a.kv_stride % 8 == 0 && a.kv_stride < 1 << 24) {
       hipLaunchKernelGGL((attn_encoder_kernel<D>), grid, dim3(256), 0, st, a);
       return hipGetLastError();
     }

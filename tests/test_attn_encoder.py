@@ -68,3 +68,24 @@ def test_attn_encoder_keeps_sequences_apart(native):
     for rows in (slice(0, 70), slice(200, 265)):
         assert torch.equal(got[rows], clean[rows])
     assert torch.equal(got.isnan(), general.isnan()) and torch.equal(got.isinf(), general.isinf())
+
+
+@pytest.mark.gpu
+def test_rows_megabytes_apart(native):
+    """Keys and values whose rows of a tile lie further apart than 32-bit offsets reach: what they give side by side."""
+    D, H, lens = 64, 2, [66, 3]
+    T = sum(lens)
+    qkv = torch.randn(T, 3 * H * D, generator=torch.Generator().manual_seed(6)).bfloat16().to(DEV)
+    cu = torch.tensor([0, 66, T], dtype=torch.int32, device=DEV)
+    kl, tiles = torch.tensor(lens, dtype=torch.int32, device=DEV), n.build_encoder_tiles(lens, H).to(DEV)
+    outs = []
+    for ld in (2 * H * D, 2 ** 24 - 8, 2 ** 24, 2 ** 24 + 2 ** 20):
+        kv = torch.empty(T * ld, dtype=torch.bfloat16, device=DEV).view(T, ld)[:, :2 * H * D]
+        kv.copy_(qkv[:, H * D:])
+        out = torch.empty(T, H * D, dtype=torch.bfloat16, device=DEV)
+        native.attn_prefill(qkv, kv, kv[:, H * D:], cu, kl, tiles, out, H, H, D, causal=False, paged=False, cu_kv=cu, kv_stride=ld)
+        outs.append(out.float())
+        del kv
+    assert torch.equal(outs[0], outs[1])
+    for o in outs[2:]:  # the general kernel: bf16 weights and results of both, 2^-9 a rounding
+        assert ((o - outs[0]).norm() / outs[0].norm()).item() < 2 ** -8

@@ -15,9 +15,11 @@ def run(native, q, kc, vc, bt, lens, ctx, Hq, Hkv):
     return out[:-1]
 
 
-# rows short of a half tile, a whole half, one past it, short of and past a tile; contexts before the queries; 8 and 4 KV heads
+# rows short of a half tile, a whole half, one past it, short of and past a tile; contexts before the queries, short ones and such
+# that the ring of four key tiles goes round several times and ends in each of its slots; 8 and 4 KV heads
 @pytest.mark.parametrize("Hq,Hkv", [(32, 8), (16, 4)])
-@pytest.mark.parametrize("rows,ctx", [(1, 0), (31, 0), (32, 65), (33, 0), (63, 3), (64, 0), (65, 130), (97, 0), (300, 0), (200, 77)])
+@pytest.mark.parametrize("rows,ctx", [(1, 0), (31, 0), (32, 65), (33, 0), (63, 3), (64, 0), (65, 130), (97, 0), (300, 0), (200, 77),
+                                      (700, 0), (33, 509), (65, 640), (40, 1000), (40, 1064), (40, 1128), (40, 1192)])
 def test_few_blocks_are_many(native, Hq, Hkv, rows, ctx):
     g = torch.Generator(device=DEV).manual_seed(rows + ctx)
     pages = -(-(rows + ctx) // 64)

@@ -7,14 +7,14 @@
 //   up     rows = norm
 //   down   rows as they lie
 // A block is 16 output columns: it requests its weights (and whatever else does not depend on the rows), then works on the rows
-// while they travel, keeps the rows in LDS as bf16 and multiplies: 16 waves share the rows, then K, and meet in LDS. Repeating the rows' work in
-// each of 24 to 256 blocks costs reads from L2 (21 KB a block for 14 fp32 rows of 384) and 0.6 us, the launch it saves 2.4 to 4.
-// Sums of a product, its bias and its residual reach the norm behind it in fp32; block 0 writes the norm's rows out, as the
-// residual of the product after next.
-// Six layers of 384 columns, 14 rows: 220 -> 111 us a call, 25 launches of 4.4 instead of 44 (with eight waves a
-// block, two rows a wave, 119); 24 layers of 1024, 14 rows: 752 -> 686 (726). What is left of a launch is its start, one trip to memory for the rows and one through LDS for the sum (a down projection
-// alone, without rows to make, takes as long as the others). Past 16384 values of rows the repeated work costs more than it
-// saves (ops/native.py encoder_few_ok).
+// while they travel, keeps the rows in LDS as bf16 and multiplies: 16 waves share the rows, then K, and meet in LDS. Repeating the
+// rows' work in each of 24 to 256 blocks costs reads from L2 (21 KB a block for 14 fp32 rows of 384) and 0.6 us, the launch it
+// saves 2.4 to 4. Sums of a product, its bias and its residual reach the norm behind it in fp32; block 0 writes the norm's rows
+// out, as the residual of the product after next.
+// Six layers of 384 columns, 14 rows: 220 -> 111 us a call, 25 launches of 4.4 instead of 44 (with eight waves a block, two rows a
+// wave, 119); 24 layers of 1024, 14 rows: 752 -> 686 (726). What is left of a launch is its start, one trip to memory for the rows
+// and one through LDS for the sum (a down projection alone, without rows to make, takes as long as the others). Past 16384 values
+// of rows the repeated work costs more than it saves (ops/native.py encoder_few_ok).
 #include "attn_tiles.h"
 #include "encoder.h"
 using namespace ragk;

@@ -2,7 +2,7 @@
 // wave per SIMD, one persistent workgroup per CU streaming its tiles' K-tiles as ONE continuous ring. Tiles of
 // 224 and 192 rows (16 IM rows a wave, IM = 8, 7, 6) fill rounds that 256 leaves part empty; the numbers below are IM = 8's.
 // 13764 rows, us at 256 / 224 rows: 3072 x 1024 75 / 69.5, 1024 x 1024 38 / 33, 1024 x 4096 90 / 85, 4096 x 1024 with GELU 128 /
-// 116 (in two launches with gemm_mid 122); 14076 x 28672 x 4096 gated 2283 / 2195, 7917 x 14336 x 2048 367 / 355. At 192 rows
+// 116 (in two launches with gemm_mid 122); 7917 x 14336 x 2048 367 / 355 (14076 x 28672 x 4096 gated 2282 / 2255). At 192 rows
 // 7917 x 3072 x 2048 86 -> 74.5, 5200 x 4096 x 4096 164 -> 138. Which tile: ops/native.py gemm_plan. 224 and 192 rows spill
 // nothing (256: 0 to 8 registers, in the epilogues).
 //

@@ -1223,7 +1223,8 @@ def _encoder_plans(T, H, I, cus, split, w4_min_m):
 FEW_ROWS, FEW_COLS = 32, 1024  # csrc/kernels/encoder.h FEW_T, FEW_H
 FEW_SIZE = 16384  # rows x columns: the blocks repeat the rows' work
 # ints that travel as kernel arguments, 960 a launch of 2 us: copied to the device (a wait for the stream, 15 us when it is idle)
-# only where a forward takes milliseconds
+# only where a forward takes milliseconds. Copied / as arguments, us a call of six layers of 384 columns among others: two texts of
+# 20 tokens 227 / 220, eight of 14 278 / 246, four of 400 351 / 319; 24 layers of 1024: 919 / 888, 1343 / 1324, 2369 / 2342
 PUT_INTS = 3840
 
 

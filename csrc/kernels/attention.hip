@@ -1306,69 +1306,21 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && !KL) ? 2 : 1) void attn_decode
   attn_decode_block<D, G, NT, NW, DG, KL>(a, blockIdx.z, blockIdx.x, blockIdx.y, smem);
 }
 
-// merge split-K partitions: grid (Hq, B), block D threads. The partition statistics are loaded by
-// all threads at once (thread t: partitions t, t + D, ...) and reduced in LDS, and each output
-// element's partial sums are loaded 8 partitions per batch of independent loads: the previous
-// version walked the partitions in two dependent load chains per thread (~9 us at batch 1 with 32
-// partitions, pure load latency; the decode attention itself took 9.4 us).
-constexpr int RED_MAXP = 256;  // partitions held in LDS (launcher guarantees max_parts <= this)
+// merge split-K partitions: grid (Hq, B), block D threads (join_parts)
+constexpr int RED_MAXP = 256;  // most partitions of a sequence
 __global__ void attn_decode_reduce_kernel(DecodeArgs a, int D) {
-  __shared__ float s_sc[RED_MAXP];
-  __shared__ float s_red[8];
-  __shared__ float s_M, s_L;
   const int hq = blockIdx.x, b = blockIdx.y, t = threadIdx.x;
-  const int nw = (blockDim.x + 63) >> 6, lane = t & 63, wid = t >> 6;
-  const int n_kt = (a.kv_lens[b] + KT - 1) / KT;
-  const int pt = decode_part_tiles(n_kt, a);
-  const int nparts = (n_kt + pt - 1) / pt;
-  if (nparts <= 1) return;  // block-uniform: the partition kernel wrote the output itself
   const size_t p0 = ((size_t)b * a.Hq + hq) * a.max_parts;
-  float m = -INFINITY;
-  for (int p = t; p < nparts; p += blockDim.x) {
-    const float mp = a.part_ml[(p0 + p) * 2];
-    s_sc[p] = mp;
-    m = fmaxf(m, mp);
-  }
-  m = wave_max(m);
-  if (lane == 0) s_red[wid] = m;
-  __syncthreads();
-  if (t == 0) {
-    float M = -INFINITY;
-    for (int w = 0; w < nw; ++w) M = fmaxf(M, s_red[w]);
-    s_M = M == -INFINITY ? 0.f : M;
-  }
-  __syncthreads();
-  const float Mu = s_M;
-  float l = 0.f;
-  for (int p = t; p < nparts; p += blockDim.x) {
-    const float sc = exp2f(s_sc[p] - Mu);
-    s_sc[p] = sc;
-    l += a.part_ml[(p0 + p) * 2 + 1] * sc;
-  }
-  l = wave_sum(l);
-  __syncthreads();
-  if (lane == 0) s_red[wid] = l;
-  __syncthreads();
-  if (t == 0) {
-    float L = 0.f;
-    for (int w = 0; w < nw; ++w) L += s_red[w];
-    s_L = L;
-  }
-  __syncthreads();
-  if (t >= D) return;
-  const float* po = a.part_o + p0 * D + t;
-  float O = 0.f;
-  int p = 0;
-  for (; p + 8 <= nparts; p += 8) {  // 8 independent loads in flight per thread
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = po[(size_t)(p + i) * D];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) O += v[i] * s_sc[p + i];
-  }
-  for (; p < nparts; ++p) O += po[(size_t)p * D] * s_sc[p];
-  const float L = s_L;
-  a.out[(size_t)b * a.out_stride + hq * D + t] = f2bf(L > 0.f ? O / L : 0.f);
+  int nparts = 0;
+  const float2 r = join_parts(
+      a.part_ml + p0 * 2, a.part_o + p0 * D, D, a.max_parts, t, false,
+      [&] {
+        const int n_kt = (a.kv_lens[b] + KT - 1) / KT, pt = decode_part_tiles(n_kt, a);
+        return nparts = (n_kt + pt - 1) / pt;
+      },
+      [](float x) { return exp2f(x); });
+  if (nparts <= 1) return;  // the partition kernel wrote the output itself
+  a.out[(size_t)b * a.out_stride + hq * D + t] = f2bf(r.y > 0.f ? r.x / r.y : 0.f);
 }
 
 // Block order (prefill_block): a 1-D grid, head group fastest, so the heaviest causal tiles of every head

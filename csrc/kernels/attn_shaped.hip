@@ -459,7 +459,15 @@ __device__ __forceinline__ void slab_row8(const ShapedDecode& a, int b, int col,
 __device__ __forceinline__ float slab_gate(const ShapedDecode& a, int b, int h) {
   if (a.off_g < 0) return 1.f;
   float g = a.bias ? bf2f(a.bias[a.off_g + h]) : 0.f;
-  for (int s = 0; s < a.S; ++s) g += a.P[s * a.slab + (size_t)b * a.ldp + a.off_g + h];
+  const float* P = a.P + (size_t)b * a.ldp + a.off_g + h;
+  for (int s0 = 0; s0 < a.S; s0 += PSU) {  // a round of loads, then their sum in order
+    float p[PSU];
+#pragma unroll
+    for (int u = 0; u < PSU; ++u) p[u] = P[min(s0 + u, a.S - 1) * a.slab];
+#pragma unroll
+    for (int u = 0; u < PSU; ++u)
+      if (s0 + u < a.S) g += p[u];
+  }
   return __builtin_amdgcn_rcpf(1.f + __expf(-g));
 }
 // pages per partition: the visited pages spread over all partitions, at least min_tiles each
@@ -672,39 +680,22 @@ __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_sh
   }
 }
 
-// join the partitions of one (head, sequence), add the extra zero score, apply the gate; DV threads
+// join the partitions of one (head, sequence), add the extra zero score, apply the gate; DV threads, at least a wave
 __global__ void attn_shaped_merge_kernel(ShapedDecode a, int DV) {
-  const int h = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
-  const int pos = a.kv_lens[b] - 1;
-  const int n = visited(pos, pos, a.window, a.keep).n, pt = part_pages(n, a), nparts = (n + pt - 1) / pt;
-  if (nparts == 1) return;  // written by the decode kernel
+  const int h = blockIdx.x, b = blockIdx.y, d = min((int)threadIdx.x, DV - 1);
   const size_t p0 = ((size_t)b * a.H + h) * a.max_parts;
-  float M = a.sink ? 0.f : -INFINITY;
-  for (int p = 0; p < nparts; ++p) M = fmaxf(M, a.part_ml[(p0 + p) * 2]);
-  const float Mu = M == -INFINITY ? 0.f : M;
-  float L = a.sink ? __builtin_amdgcn_exp2f(-Mu) : 0.f, O = 0.f;
-  int p = 0;
-  for (; p + 4 <= nparts; p += 4) {
-    float v[4], m[4], l[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[i] = a.part_o[(p0 + p + i) * DV + d];
-      m[i] = a.part_ml[(p0 + p + i) * 2];
-      l[i] = a.part_ml[(p0 + p + i) * 2 + 1];
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float sc = __builtin_amdgcn_exp2f(m[i] - Mu);
-      L += l[i] * sc;
-      O += v[i] * sc;
-    }
-  }
-  for (; p < nparts; ++p) {
-    const float sc = __builtin_amdgcn_exp2f(a.part_ml[(p0 + p) * 2] - Mu);
-    L += a.part_ml[(p0 + p) * 2 + 1] * sc;
-    O += a.part_o[(p0 + p) * DV + d] * sc;
-  }
-  a.out[(size_t)b * a.ldo + h * DV + d] = f2bf(L > 0.f ? O / L * slab_gate(a, b, h) : 0.f);
+  const float gate = slab_gate(a, b, h);
+  int nparts = 0;
+  const float2 r = join_parts(
+      a.part_ml + p0 * 2, a.part_o + p0 * DV, DV, a.max_parts, d, a.sink,
+      [&] {
+        const int pos = a.kv_lens[b] - 1;
+        const int n = visited(pos, pos, a.window, a.keep).n, pt = part_pages(n, a);
+        return nparts = (n + pt - 1) / pt;
+      },
+      [](float x) { return __builtin_amdgcn_exp2f(x); });
+  if (nparts == 1 || (int)threadIdx.x >= DV) return;  // one: written by the decode kernel
+  a.out[(size_t)b * a.ldo + h * DV + d] = f2bf(r.y > 0.f ? r.x / r.y * gate : 0.f);
 }
 
 template <int DK, int DV, PrefillMode MODE>
@@ -734,7 +725,7 @@ int launch_decode(const ShapedDecode& a, hipStream_t st) {
   const int chunks = (a.H / a.G + DEC_HEADS - 1) / DEC_HEADS;
   hipLaunchKernelGGL((attn_shaped_decode_kernel<DK, DV>), dim3(a.max_parts, a.G * chunks, a.B), dim3(256), 0, st, a);
   if (a.max_parts > 1)
-    hipLaunchKernelGGL(attn_shaped_merge_kernel, dim3(a.H, a.B), dim3(DV), 0, st, a, DV);
+    hipLaunchKernelGGL(attn_shaped_merge_kernel, dim3(a.H, a.B), dim3(DV < 64 ? 64 : DV), 0, st, a, DV);
   return (int)hipGetLastError();
 }
 

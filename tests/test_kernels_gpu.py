@@ -433,6 +433,27 @@ def test_attn_decode(native, kv_lens, Hq, Hkv, target):
     assert rel_err(out.cpu().reshape(B, Hq, D), ref) < 2e-2
 
 
+@pytest.mark.parametrize("mp", [2, 7, 8, 9, 63, 64, 65, 130, 256])
+def test_attn_decode_partition_counts(native, mp):
+    """Joins of few, of a round of loads' and of more than a wave's partitions, records past the last holding NaN."""
+    kv_lens, Hq, Hkv, D = [16500, 1, 130], 4, 1, 128
+    torch.manual_seed(mp)
+    kc, vc, bt = _paged_setup(kv_lens, Hkv, D, seed=4)
+    B = len(kv_lens)
+    q = torch.randn(B, Hq * D).bfloat16()
+    kvl = torch.tensor(kv_lens, dtype=torch.int32)
+    out = torch.empty(B, Hq * D, device=DEV).bfloat16()
+    ws_o = torch.full((B, Hq, mp, D), float("nan"), device=DEV)
+    ws_ml = torch.full((B, Hq, mp, 2), float("nan"), device=DEV)
+    native.attn_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), kvl.to(DEV), out, Hq, Hkv, D, 1, mp, ws_o, ws_ml)
+    cu = torch.arange(B + 1, dtype=torch.int32)
+    ref = R.attention_varlen(q.reshape(B, Hq, D), None, None, cu, kvl, True, 1 / math.sqrt(D),
+                             k_full=lambda s: R.paged_kv_view(kc, bt[s], kv_lens[s], 64),
+                             v_full=lambda s: R.paged_kv_view(vc, bt[s], kv_lens[s], 64))
+    # weights and outputs are rounded to bf16 (2^-8 of a value at most, independent: well under 2^-7 of the norm)
+    assert rel_err(out.cpu().reshape(B, Hq, D), ref) < 2 ** -7
+
+
 @pytest.mark.parametrize("kv_lens,Hq,Hkv", [([5200, 1, 64, 4100], 32, 8), ([65, 3000, 700], 4, 1), ([1], 32, 8),
                                              ([8100] * 3 + [5], 32, 8)])
 @pytest.mark.parametrize("nt", [0, 1])

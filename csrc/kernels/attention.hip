@@ -16,9 +16,10 @@
 //    from a packed qkv buffer (bidirectional encoders). One block = 4 waves =
 //    GB query heads sharing one KV head x (4/GB) groups of 32 query rows.
 //  * attn_decode<D, G>: one query token per sequence, split-K over the context
-//    (flash-decoding). Each wave streams its own 64-key tiles (K straight to
-//    VGPRs, V through a wave-private LDS tile for the transposed read); 4 waves
-//    combine in LDS; partitions merged by attn_decode_reduce.
+//    (flash-decoding). Each wave streams its own 64-key tiles, the next one
+//    requested behind the present one (K to VGPRs, V through VGPRs into a
+//    wave-private LDS tile for the transposed read); 4 waves combine in LDS;
+//    partitions merged by attn_decode_reduce.
 //
 // Replaces reference ops K5/K6 (causal GQA attention in transformers' Llama SDPA path,
 // [dep] modeling_llama.py:191-215) and E3 (XLM-R/BERT bidirectional attention).
@@ -1003,7 +1004,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void attn_prefill_v3_kernel(Prefil
 struct DecodeArgs {
   const bf16_t* q; int q_stride;           // [B] rows, head h at +h*D
   const bf16_t* kc; const bf16_t* vc;      // paged caches
-  const int* block_tables; int bt_stride;
+  const int* block_tables; int bt_stride, bt_cols;
   const int* kv_lens;                      // [B]
   float* part_o;                           // [B][Hq][max_parts][D]
   float* part_ml;                          // [B][Hq][max_parts][2]
@@ -1033,6 +1034,11 @@ __device__ __forceinline__ int decode_part_tiles(int n_kt, const DecodeArgs& a) 
 template <int D, int G, int NW = 4, bool KL = false>
 constexpr int decode_lds_bytes() { return NW * Cfg<D>::TILEB * (KL ? 2 : 1) + G * D * 2; }
 
+// The K / V stream bounds it, and for short contexts the trips to memory in front of it. Both lengths and page table are one trip,
+// the queries' slabs and the first tile another (four in a row before: length, page, tile, and the slabs behind the tile, since
+// vector loads return in order), and a wave's next tile is on its way while it works on one. One layer, 128-wide heads, us with the
+// join: 11 rows of 2000 tokens, 8 KV heads 28.6 -> 26.1; 3 of 4000 19.3 -> 15.5; 20 of 5000 68.0 -> 63.7; 1 of 5267 13.3 -> 11.9;
+// 2 rows of 2000, 4 KV heads 11.3 -> 10.7; 32 of 4200 in one partition (KL) 96 -> 92.5, 5.97 TB/s.
 // One split-K partition block of decode attention: partition `part` of KV head `kvh` of sequence `b`.
 // NW: waves per block (4; 8 for the batch-32 grid with one partition per sequence: one 8-wave block per
 // CU keeps the same KV bytes in flight as two 4-wave blocks and needs no merge launch). A multi-partition
@@ -1047,11 +1053,14 @@ constexpr int decode_lds_bytes() { return NW * Cfg<D>::TILEB * (KL ? 2 : 1) + G 
 template <int D, int G, bool NT = false, int NW = 4, int DG = 0, bool KL = false>
 __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part, int kvh, int b, char* smem) {
   constexpr int NTH = NW * 64;
+  constexpr bool REGS = !KL && DG != 2;    // K and V tiles through registers
+  constexpr bool AHEAD = REGS && DG == 0;  // ... and requested a tile ahead
   using C = Cfg<D>;
   static_assert(G <= 16, "at most 16 query heads per KV head");
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int wid_u = __builtin_amdgcn_readfirstlane(wid);
-  const int kv_len = a.kv_lens[b];
+  PageRow<2> table(a.block_tables + (size_t)b * a.bt_stride, a.bt_cols, lane);
+  const int kv_len = ld_uniform(a.kv_lens + b), pos = ld_uniform((a.qkv_p ? a.positions : a.kv_lens) + b);
   const int n_kt = (kv_len + KT - 1) / KT;
   const int pt = decode_part_tiles(n_kt, a);
   const int kt0 = part * pt;
@@ -1059,151 +1068,196 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
   const int kt1 = min(kt0 + pt, n_kt);
   const int nparts = (n_kt + pt - 1) / pt;
   const int fr = lane & 15, fh = lane >> 4;
-  const int* bt = a.block_tables + (size_t)b * a.bt_stride;
+  table.wait();
 
   bf16x8 qf[C::KS];
-  // Fused-RoPE path: this wave's first KV tile is requested BEFORE the q prologue (K straight to
-  // registers, V to the wave's LDS tile), so its HBM latency overlaps the qkv partial-slab loads instead
-  // of following them -- at batch 1 a wave handles a single tile and the two latencies were in series.
-  // Not for the sequence's last tile: the new token's k / v is appended into it during the prologue.
   char* sV = smem + wid * C::TILEB;
   char* sK = smem + (NW + wid) * C::TILEB;  // KL only
-  const bool pre = a.qkv_p != nullptr && kt0 + wid_u < kt1 && kt0 + wid_u != n_kt - 1;  // wave-uniform
-  bf16x8 kf0[4][C::KS];
-  if (pre) {
-    const size_t base = ((size_t)bt[kt0 + wid_u] * a.Hkv + kvh) * KT * D;
-    const bf16_t* kb = a.kc + base;
-    const bf16_t* vb = a.vc + base;
-    if constexpr (KL) stage_kv<D, false, NT, 1>(sK, 0, 1, lane, [&](int r) { return kb + (size_t)r * D; });
-    stage_kv<D, true, NT, 1>(sV, 0, 1, lane, [&](int r) { return vb + (size_t)r * D; });
+  bf16x8 kf[4][C::KS];
+  auto page = [&](int kt) { return ((size_t)table(kt) * a.Hkv + kvh) * KT * D; };
+  // (lanes' places as 32-bit offsets from a scalar address: a pair of registers a load otherwise)
+  constexpr int VP = C::RPP < C::RB * C::GR ? C::RB * C::GR / C::RPP : 1;  // pieces until the swizzle repeats
+  const unsigned k_lane = (fr * D + 8 * fh) * 2;
+  unsigned v_lane[VP];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+  for (int i = 0; i < VP; ++i)
+    v_lane[i] = lane / C::NC * C::ROWB + 16 * ((lane % C::NC) ^ vswz<D>(i * C::RPP + lane / C::NC));
+  auto request_k = [&](int kt) {
+    const bf16_t* kb = a.kc + page(kt);
+    if constexpr (KL) {
+      stage_kv<D, false, NT, 1>(sK, 0, 1, lane, [&](int r) { return kb + (size_t)r * D; });
+    } else {
 #pragma unroll
-      for (int s = 0; s < C::KS; ++s)
-        if constexpr (!KL)
-          kf0[t][s] = NT ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(kb + (size_t)(16 * t + fr) * D +
-                                                                                     32 * s + 8 * fh))
-                         : *reinterpret_cast<const bf16x8*>(kb + (size_t)(16 * t + fr) * D + 32 * s + 8 * fh);
-  }
-  if (a.qkv_p != nullptr) {
-    // q = RoPE(bf16(sum_s P[s][b])) for this KV head's G query heads, one (d, d + D/2) rotate_half
-    // pair of 8-vectors per thread (G * D/16 threads, all slab loads of a thread in flight together),
-    // staged through LDS; in the block owning the last KV tile, other threads append the new
-    // token's k (rotated) and v meanwhile. One barrier covers both.
-    bf16_t* s_q = reinterpret_cast<bf16_t*>(smem + NW * C::TILEB * (KL ? 2 : 1));
-    constexpr int NV = D / 16;  // pairs per head
-    const int pos = a.positions[b];
-    const float* prow = a.qkv_p + (size_t)b * a.ldp;
-    const float* ct = a.cos_t + (size_t)pos * (D / 2);
-    const float* st = a.sin_t + (size_t)pos * (D / 2);
-    const int tid = threadIdx.x;
-    const bool append = kt1 == n_kt;  // block-uniform
-    constexpr int KV0 = (G * NV + 63) / 64 * 64;  // append threads start on a fresh wave
-    if (tid < G * NV) {
-      const int g = tid / NV, v = tid % NV;
-      const float* ph = prow + (size_t)(kvh * G + g) * D + 8 * v;
-      float x1[8], x2[8], o1[8], o2[8];
-      sum_partials8x2(ph, ph + D / 2, a.S, (size_t)a.p_slab, x1, x2);
-      rope8(x1, x2, ct + 8 * v, st + 8 * v, o1, o2);
-      *reinterpret_cast<u32x4*>(s_q + g * D + 8 * v) = pack8(o1);
-      *reinterpret_cast<u32x4*>(s_q + g * D + D / 2 + 8 * v) = pack8(o2);
-    } else if (append && tid >= KV0 && tid < KV0 + 2 * NV) {  // [KV0, KV0+NV): k, [KV0+NV, KV0+2NV): v
-      const int isv = tid - KV0 >= NV, v = (tid - KV0) % NV;
-      const int slot = a.slots[b];
-      const size_t kvo = (((size_t)(slot / KT) * a.Hkv + kvh) * KT + (slot % KT)) * D;
-      const float* ph = prow + (size_t)(a.Hq + (isv ? a.Hkv : 0) + kvh) * D + 8 * v;
-      float x1[8], x2[8];
-      sum_partials8x2(ph, ph + D / 2, a.S, (size_t)a.p_slab, x1, x2);
-      bf16_t* dst = (isv ? const_cast<bf16_t*>(a.vc) : const_cast<bf16_t*>(a.kc)) + kvo;
-      if (isv) {
-        *reinterpret_cast<u32x4*>(dst + 8 * v) = pack8(x1);
-        *reinterpret_cast<u32x4*>(dst + D / 2 + 8 * v) = pack8(x2);
-      } else {
-        float o1[8], o2[8];
-        rope8(x1, x2, ct + 8 * v, st + 8 * v, o1, o2);
-        *reinterpret_cast<u32x4*>(dst + 8 * v) = pack8(o1);
-        *reinterpret_cast<u32x4*>(dst + D / 2 + 8 * v) = pack8(o2);
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int s = 0; s < C::KS; ++s) {
+          const bf16x8* p = reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(kb + 16 * t * D + 32 * s) + k_lane);
+          kf[t][s] = NT ? __builtin_nontemporal_load(p) : *p;
+        }
+    }
+  };
+  // V: whole 1-KiB pieces, by LDS-DMA (KL) or through registers, so that the tile behind it can be on its way while this one is
+  // read from LDS (the compiler drains every load in flight around LDS-DMA pieces, K's with them)
+  u32x4 vr[C::PIECES];
+  auto request_v = [&](int kt) {
+    const bf16_t* vb = a.vc + page(kt);
+    if constexpr (!REGS) {
+      stage_kv<D, true, NT, 1>(sV, 0, 1, lane, [&](int r) { return vb + (size_t)r * D; });
+    } else {
+#pragma unroll
+      for (int i = 0; i < C::PIECES; ++i) {
+        const u32x4* p = reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vb) + i * 1024 + v_lane[i % VP]);
+        vr[i] = NT ? __builtin_nontemporal_load(p) : *p;
       }
     }
-    __syncthreads();  // q in LDS; the appended row visible to every wave of this block (same CU)
+  };
+  // Rotating path (qkv_p): q = RoPE(bf16(sum_s P[s][b])) for this KV head's G query heads, staged through LDS; in the block owning
+  // the last KV tile the new token's k (rotated) and v are appended meanwhile. Every wave takes whole heads, a rotate_half pair
+  // (d, d + D / 2) a lane.
+  bf16_t* s_q = reinterpret_cast<bf16_t*>(smem + NW * C::TILEB * (KL ? 2 : 1));
+  constexpr int PL = D / 2, IPW = 64 / PL;  // pairs of a head, heads of a wave at a time
+  const bool rope = a.qkv_p != nullptr, append = rope && kt1 == n_kt;  // block-uniform
+  const int n_items = G + (append ? 2 : 0);                            // query heads, then k and v
+  const int p = lane % PL, it0 = wid * IPW + lane / PL;
+  float x1[PSU], x2[PSU], cs = 0.f, sn = 0.f;
+  auto column = [&](int it) {
+    it = min(it, G + 1);
+    return a.qkv_p + (size_t)b * a.ldp + (size_t)(it < G ? kvh * G + it : (it == G ? a.Hq : a.Hq + a.Hkv) + kvh) * D + p;
+  };
+  auto request_item = [&](int it) {
+    const float* ph = column(it);
 #pragma unroll
-    for (int s = 0; s < C::KS; ++s)
-      qf[s] = fr < G ? *reinterpret_cast<const bf16x8*>(s_q + fr * D + 32 * s + 8 * fh)
-                     : (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
+    for (int u = 0; u < PSU; ++u) {
+      const size_t o = (size_t)min(u, a.S - 1) * a.p_slab;
+      x1[u] = ph[o];
+      x2[u] = ph[o + PL];
+    }
+    cs = a.cos_t[(size_t)pos * PL + p];
+    sn = a.sin_t[(size_t)pos * PL + p];
+  };
+  auto finish_item = [&](int it) {
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int u = 0; u < PSU; ++u)
+      if (u < a.S) {
+        s1 += x1[u];
+        s2 += x2[u];
+      }
+    for (int u = PSU; u < a.S; ++u) {
+      s1 += column(it)[(size_t)u * a.p_slab];
+      s2 += column(it)[(size_t)u * a.p_slab + PL];
+    }
+    s1 = bf2f(f2bf(s1));
+    s2 = bf2f(f2bf(s2));
+    const bf16_t r1 = f2bf(bf2f(f2bf(s1 * cs)) + bf2f(f2bf(-s2 * sn)));  // rope8's formula and roundings
+    const bf16_t r2 = f2bf(bf2f(f2bf(s2 * cs)) + bf2f(f2bf(s1 * sn)));
+    asm volatile("" ::"v"((unsigned)r1), "v"((unsigned)r2));  // every load is used on every path
+    if (it < G) {
+      s_q[it * D + p] = r1;
+      s_q[it * D + PL + p] = r2;
+    } else if (it < n_items) {
+      const int slot = ld_uniform(a.slots + b);
+      bf16_t* dst = (it == G ? const_cast<bf16_t*>(a.kc) : const_cast<bf16_t*>(a.vc)) +
+                    (((size_t)(slot / KT) * a.Hkv + kvh) * KT + (slot % KT)) * D + p;
+      dst[0] = it == G ? r1 : f2bf(s1);
+      dst[PL] = it == G ? r2 : f2bf(s2);
+    }
+  };
+  // One trip to memory for the queries and the wave's first tile, the queries first: vector loads return in order, so behind the
+  // tile their sums waited for it. Requests are unconditional (a wave without a tile asks for the block's last one, which another
+  // wave reads): where paths with and without them meet, the compiler waits for every load in flight. The tile that the new token
+  // goes into is asked for again behind the barrier.
+  const int kt_first = min(kt0 + wid_u, kt1 - 1);
+  if (rope) {
+    request_item(it0);
   } else {
     const int g = fr < G ? fr : 0;
     const bf16_t* qp = a.q + (size_t)b * a.q_stride + (kvh * G + g) * D + 8 * fh;
 #pragma unroll
-    for (int s = 0; s < C::KS; ++s) {
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>(qp + 32 * s);
-      qf[s] = fr < G ? v : (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
-    }
+    for (int s = 0; s < C::KS; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qp + 32 * s);
   }
+  __builtin_amdgcn_sched_barrier(0);
+  request_k(kt_first);
+  __builtin_amdgcn_sched_barrier(0);  // K before V: the scores and the softmax run while V is landing
+  request_v(kt_first);
+  __builtin_amdgcn_sched_barrier(0);
+  if (rope) {
+    finish_item(it0);
+    for (int i0 = NW * IPW; i0 < n_items; i0 += NW * IPW) {  // block-uniform
+      request_item(i0 + it0);
+      finish_item(i0 + it0);
+    }
+    if (append) {
+      __syncthreads();  // q in LDS; the appended row visible to every wave of this block (same CU)
+      if (kt_first == n_kt - 1) {
+        if constexpr (!REGS) wait_vmcnt0();  // (into the LDS that its first request fills)
+        request_k(kt_first);
+        __builtin_amdgcn_sched_barrier(0);
+        request_v(kt_first);
+      }
+    } else {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int s = 0; s < C::KS; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(s_q + min(fr, G - 1) * D + 32 * s + 8 * fh);
+  }
+#pragma unroll
+  for (int s = 0; s < C::KS; ++s)
+    if (fr >= G) qf[s] = (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
   f32x4 o[C::DT];
 #pragma unroll
   for (int dt = 0; dt < C::DT; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
   float m_i = -INFINITY, l_i = 0.f;
   unsigned dsink = 0;
 
-  for (int kt = kt0 + wid_u; kt < kt1; kt += NW) {
-    bf16x8 kf[4][C::KS];
+  // One tile. MORE: the wave's next one is requested meanwhile (a form of its own: behind a branch around the requests the
+  // compiler would wait for them where it waits for this tile's values).
+  auto tile = [&](int kt, auto more_t) {
+    constexpr bool MORE = decltype(more_t)::value;
+    const bool have = kt == kt0 + wid_u;  // requested above
     if constexpr (KL) {
-      if (!(pre && kt == kt0 + wid_u)) {  // else staged before the prologue
-        const size_t base = ((size_t)bt[kt] * a.Hkv + kvh) * KT * D;
-        const bf16_t* kb = a.kc + base;
-        const bf16_t* vb = a.vc + base;
+      if (!have) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // previous tile's K / V reads retired
-        stage_kv<D, false, NT, 1>(sK, 0, 1, lane, [&](int r) { return kb + (size_t)r * D; });
-        stage_kv<D, true, NT, 1>(sV, 0, 1, lane, [&](int r) { return vb + (size_t)r * D; });
+        request_k(kt);
+        request_v(kt);
       }
       // K first: QK^T and the softmax run while the V tile (the 16 youngest LDS-DMAs) is still landing. The
       // builtin wait (not inline asm) updates the compiler's own counter model, so it adds no vmcnt(0) of its own.
-      static_assert(Cfg<D>::PIECES < 64, "vmcnt range");
-      __builtin_amdgcn_s_waitcnt((Cfg<D>::PIECES & 15) | (((Cfg<D>::PIECES >> 4) & 3) << 14) | (0x7 << 4) | (0xF << 8));
+      static_assert(C::PIECES < 64, "vmcnt range");
+      __builtin_amdgcn_s_waitcnt((C::PIECES & 15) | (((C::PIECES >> 4) & 3) << 14) | (0x7 << 4) | (0xF << 8));
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int s = 0; s < C::KS; ++s) kf[t][s] = load_k<D>(sK, t, s, lane);
-    } else if (pre && kt == kt0 + wid_u) {  // requested before the prologue
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int s = 0; s < C::KS; ++s) kf[t][s] = kf0[t][s];
-    } else if (DG == 2) {
-      const size_t base = ((size_t)bt[kt] * a.Hkv + kvh) * KT * D;
-      const bf16_t* kb = a.kc + base;
-      const bf16_t* vb = a.vc + base;
+    } else if constexpr (DG == 2) {
+      const bf16_t* kb = a.kc + page(kt);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      stage_kv<D, true, NT, 1>(sV, 0, 1, lane, [&](int r) { return vb + (size_t)r * D; });
+      request_v(kt);
       stage_kv<D, false, NT, 1>(sV, 0, 1, lane, [&](int r) { return kb + (size_t)r * D; });
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int s = 0; s < C::KS; ++s) kf[t][s] = (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
-    } else {
-      const size_t base = ((size_t)bt[kt] * a.Hkv + kvh) * KT * D;
-      const bf16_t* kb = a.kc + base;
-      const bf16_t* vb = a.vc + base;
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // previous tile's V reads retired
-      // V tile -> wave-private LDS (transposed reads later)
-      stage_kv<D, true, NT, 1>(sV, 0, 1, lane, [&](int r) { return vb + (size_t)r * D; });
-      // K fragments straight to VGPRs
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int s = 0; s < C::KS; ++s)
-          kf[t][s] = NT ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(kb + (size_t)(16 * t + fr) * D +
-                                                                                    32 * s + 8 * fh))
-                        : *reinterpret_cast<const bf16x8*>(kb + (size_t)(16 * t + fr) * D + 32 * s + 8 * fh);
+    } else if (DG == 1 && !have) {
+      request_k(kt);
+      request_v(kt);
     }
     if constexpr (DG != 0) {
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int s = 0; s < C::KS; ++s) dsink ^= __builtin_bit_cast(u32x4, kf[t][s])[0];
-      wait_vmcnt0();
-      dsink ^= *reinterpret_cast<const unsigned*>(sV + 4 * lane);
-      continue;
+      if constexpr (REGS) {
+#pragma unroll
+        for (int i = 0; i < C::PIECES; ++i) dsink ^= vr[i][0];
+      } else {
+        wait_vmcnt0();
+        dsink ^= *reinterpret_cast<const unsigned*>(sV + 4 * lane);
+      }
+      return;
     }
     f32x4 s4[4];
 #pragma unroll
@@ -1211,6 +1265,11 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
       s4[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < C::KS; ++s) s4[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][s], qf[s], s4[t], 0, 0, 0);
+    }
+    if constexpr (MORE) {  // the next tile's K travels behind this one's softmax and P.V
+      __builtin_amdgcn_sched_barrier(0);
+      request_k(kt + NW);
+      __builtin_amdgcn_sched_barrier(0);
     }
     const int k0 = kt * KT;
     float mx = -INFINITY;
@@ -1245,57 +1304,78 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
     for (int dt = 0; dt < C::DT; ++dt) o[dt] *= alpha;
     const bf16x8 pb0 = pack_p(s4[0], s4[1]);
     const bf16x8 pb1 = pack_p(s4[2], s4[3]);
-    if constexpr (KL)
+    if constexpr (REGS) {
+#pragma unroll
+      for (int i = 0; i < C::PIECES; ++i) *reinterpret_cast<u32x4*>(sV + i * 1024 + lane * 16) = vr[i];
+      if constexpr (MORE) request_v(kt + NW);
+      // (the wave's own LDS accesses stay in order: written above, read below, written again in the next iteration)
+    } else {
       __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));  // V tile landed (vmcnt(0), seen by the compiler)
-    else
-      wait_vmcnt0();  // V tile landed in this wave's LDS
+    }
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) {
       o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load_vt<D>(sV, dt, 0, lane), pb0, o[dt], 0, 0, 0);
       o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load_vt<D>(sV, dt, 1, lane), pb1, o[dt], 0, 0, 0);
     }
+  };
+  int kt = kt0 + wid_u;
+  if constexpr (AHEAD) {
+    if (kt < kt1) {
+      for (; kt + NW < kt1; kt += NW) tile(kt, std::true_type{});
+      tile(kt, std::false_type{});
+    }
+  } else {
+    for (; kt < kt1; kt += NW) tile(kt, std::false_type{});
   }
 
   if constexpr (DG != 0) {
     if (dsink == 0x9e3779b9u) a.out[(size_t)b * a.out_stride + lane] = 0;  // keeps the loads alive
     return;
   }
-  // ---- combine the 4 waves in LDS ----
-  __syncthreads();
-  float* sm = reinterpret_cast<float*>(smem);    // [4][16] max
-  float* sl = sm + NW * 16;                      // [NW][64] partial l (per lane)
-  float* so = sl + NW * 64;                      // [NW][16][D] O
-  if (fh == 0) sm[wid * 16 + fr] = m_i;
-  sl[wid * 64 + lane] = l_i;
+  // ---- combine the waves in LDS: each puts its G rows and their statistics where its V tile lay, rows 16 bytes apart in the
+  // banks (as 16 rows of D floats behind a barrier, one float a lane, this was 1 us of a block) ----
+  constexpr int OS = D + 4, PER = C::TILEB / 4;  // floats of a row, of a wave
+  static_assert((G * OS + 2 * G) * 4 <= C::TILEB, "a wave's rows fit its V tile");
+  float* so = reinterpret_cast<float*>(smem);
+  if constexpr (!REGS) wait_vmcnt0();  // pieces that no tile waited for
+  l_i += __shfl_xor(l_i, 16, 64);
+  l_i += __shfl_xor(l_i, 32, 64);
+  if (fr < G) {
+    float* w = so + wid_u * PER;
 #pragma unroll
-  for (int dt = 0; dt < C::DT; ++dt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) so[(wid * 16 + fr) * D + 16 * dt + 4 * fh + r] = o[dt][r];
+    for (int dt = 0; dt < C::DT; ++dt) *reinterpret_cast<f32x4*>(w + fr * OS + 16 * dt + 4 * fh) = o[dt];
+    if (fh == 0) *reinterpret_cast<float2*>(w + G * OS + 2 * fr) = make_float2(m_i, l_i);
+  }
   __syncthreads();
-  // thread -> (g, d) pairs
-  for (int e = threadIdx.x; e < G * D; e += NTH) {
-    const int g = e / D, d = e % D;
+  for (int e = threadIdx.x; e < G * D / 4; e += NTH) {
+    const int g = e / (D / 4), d = e % (D / 4) * 4;
+    float2 ml[NW];
+    f32x4 ov[NW];
     float M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) M = fmaxf(M, sm[w * 16 + g]);
+    for (int w = 0; w < NW; ++w) {
+      ml[w] = *reinterpret_cast<const float2*>(so + w * PER + G * OS + 2 * g);
+      ov[w] = *reinterpret_cast<const f32x4*>(so + w * PER + g * OS + d);
+      M = fmaxf(M, ml[w].x);
+    }
     const float Mu = M == -INFINITY ? 0.f : M;
-    float L = 0.f, O = 0.f;
+    float L = 0.f;
+    f32x4 O = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const float sc = exp2f(sm[w * 16 + g] - Mu);
-      L += (sl[w * 64 + g] + sl[w * 64 + g + 16] + sl[w * 64 + g + 32] + sl[w * 64 + g + 48]) * sc;
-      O += so[(w * 16 + g) * D + d] * sc;
+      const float sc = exp2f(ml[w].x - Mu);
+      L += ml[w].y * sc;
+      O += ov[w] * sc;
     }
     const int hq = kvh * G + g;
     if (nparts == 1) {
-      a.out[(size_t)b * a.out_stride + hq * D + d] = f2bf(L > 0.f ? O / L : 0.f);
+      if (!(L > 0.f)) O = (f32x4){0.f, 0.f, 0.f, 0.f}, L = 1.f;
+      *reinterpret_cast<u32x2_a2*>(a.out + (size_t)b * a.out_stride + hq * D + d) =
+          (u32x2_a2){pk2bf(O[0] / L, O[1] / L), pk2bf(O[2] / L, O[3] / L)};
     } else {
       const size_t pi = ((size_t)b * a.Hq + hq) * a.max_parts + part;
-      a.part_o[pi * D + d] = O;
-      if (d == 0) {
-        a.part_ml[pi * 2] = M;
-        a.part_ml[pi * 2 + 1] = L;
-      }
+      *reinterpret_cast<f32x4_a4*>(a.part_o + pi * D + d) = O;
+      if (d == 0) *reinterpret_cast<f32x2_a4*>(a.part_ml + pi * 2) = (f32x2_a4){M, L};
     }
   }
 }
@@ -1446,12 +1526,12 @@ RAGK_API int ragk_attn_decode_set_defer(int on) {
 }
 
 RAGK_API int ragk_attn_decode(const void* q, int q_stride, const void* kc, const void* vc, const int* block_tables,
-                              int bt_stride, const int* kv_lens, float* part_o, float* part_ml, void* out,
+                              int bt_stride, int bt_cols, const int* kv_lens, float* part_o, float* part_ml, void* out,
                               int out_stride, int B, int Hq, int Hkv, int D, int part_tiles, int max_parts,
                               float scale, hipStream_t st) {
   if (B <= 0) return 0;
   if (Hq % Hkv || part_tiles < 1 || max_parts < 1 || max_parts > RED_MAXP) return (int)hipErrorInvalidValue;
-  DecodeArgs a{(const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, block_tables, bt_stride, kv_lens,
+  DecodeArgs a{(const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, block_tables, bt_stride, bt_cols, kv_lens,
                part_o, part_ml, (bf16_t*)out, out_stride, Hq, Hkv, part_tiles, max_parts,
                scale * 1.4426950408889634f};
   return launch_attn_decode(a, B, D, max_parts, st);
@@ -1462,14 +1542,14 @@ RAGK_API int ragk_attn_decode(const void* q, int q_stride, const void* kc, const
 // rope_kv_partials + attn_decode). Cache blocks hold KT tokens.
 RAGK_API int ragk_attn_decode_rope(const float* P, int S, int ldp, const int* positions, const int* slots,
                                    const float* cos_t, const float* sin_t, void* kc, void* vc,
-                                   const int* block_tables, int bt_stride, const int* kv_lens, float* part_o,
+                                   const int* block_tables, int bt_stride, int bt_cols, const int* kv_lens, float* part_o,
                                    float* part_ml, void* out, int out_stride, int B, int Hq, int Hkv, int D,
                                    int part_tiles, int max_parts, float scale, hipStream_t st) {
   if (B <= 0) return 0;
   if (Hq % Hkv || part_tiles < 1 || max_parts < 1 || max_parts > RED_MAXP || S < 1 || D % 64 ||
       ldp < (Hq + 2 * Hkv) * D || !P || !positions || !slots || !cos_t || !sin_t)
     return (int)hipErrorInvalidValue;
-  DecodeArgs a{nullptr, 0, (const bf16_t*)kc, (const bf16_t*)vc, block_tables, bt_stride, kv_lens,
+  DecodeArgs a{nullptr, 0, (const bf16_t*)kc, (const bf16_t*)vc, block_tables, bt_stride, bt_cols, kv_lens,
                part_o, part_ml, (bf16_t*)out, out_stride, Hq, Hkv, part_tiles, max_parts,
                scale * 1.4426950408889634f, P, (long long)B * ldp, ldp, S, positions, slots, cos_t, sin_t};
   return launch_attn_decode(a, B, D, max_parts, st);

@@ -105,8 +105,37 @@ __device__ __forceinline__ bf16x8 pack_p(const f32x4& a, const f32x4& b) {
                   f2bf_s(b[0]), f2bf_s(b[1]), f2bf_s(b[2]), f2bf_s(b[3])};
 }
 
-// Records whose owner promises no more than their elements' alignment
+// One value at a wave-uniform address that this kernel does not write: a scalar load, which no counted vector wait includes
+__device__ __forceinline__ int ld_uniform(const int* p) { return *(const __attribute__((address_space(4))) int*)p; }
+
+// A sequence's row of the block table: its first 64 N entries are requested at once, N a lane, so that finding a page does not wait
+// for the sequence's length and then for the entry (a trip to memory each). Indices are wave-uniform.
+template <int N>
+struct PageRow {
+  const int* row;
+  int v[N];
+  __device__ __forceinline__ PageRow(const int* r, int cols, int lane) : row(r) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = cols > 0 ? r[min(64 * i + lane, cols - 1)] : 0;
+  }
+  // Waits for them, so that no later path has to allow for their being in flight
+  __device__ __forceinline__ void wait() {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
+  }
+  __device__ __forceinline__ int operator()(int page) const {
+    if (page >= 64 * N) return ld_uniform(row + page);
+    int x = v[0];
+#pragma unroll
+    for (int i = 1; i < N; ++i) x = page >= 64 * i ? v[i] : x;
+    return __builtin_amdgcn_readlane(x, page & 63);
+  }
+};
+
+// Rows and records whose owners promise no more than their elements' alignment
+typedef __attribute__((ext_vector_type(2), aligned(2))) unsigned u32x2_a2;
 typedef __attribute__((ext_vector_type(2), aligned(4))) float f32x2_a4;
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_a4;
 
 // Join of a decode query's split-K partitions: (sum of their outputs' column t, sum of their weights), both scaled to the common
 // maximum; records ml[p] = (maximum, sum), po[p][D]. count() gives how many there are; at most max_parts, which the records' arrays

@@ -1534,8 +1534,8 @@ def attn_decode(q, k_cache, v_cache, block_tables, kv_lens, out, Hq, Hkv, D, par
     _set_decode_nt(B, Hkv)
     check(_lib.lib().ragk_attn_decode(
         q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(),
-        block_tables.stride(0), kv_lens.data_ptr(), ptr(ws_o), ptr(ws_ml), out.data_ptr(), out.stride(0), B, Hq, Hkv,
-        D, part_tiles, max_parts, float(scale), stream_ptr()), "ragk_attn_decode")
+        block_tables.stride(0), block_tables.shape[1], kv_lens.data_ptr(), ptr(ws_o), ptr(ws_ml), out.data_ptr(), out.stride(0),
+        B, Hq, Hkv, D, part_tiles, max_parts, float(scale), stream_ptr()), "ragk_attn_decode")
     return out
 
 
@@ -1571,7 +1571,7 @@ def attn_decode_rope(P, positions, cos_t, sin_t, slots, k_cache, v_cache, block_
         check(lib.ragk_attn_decode_rope(
             P.data_ptr(), S, ldp, positions.data_ptr(), slots.data_ptr(), cos_t.data_ptr(), sin_t.data_ptr(),
             k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(), block_tables.stride(0),
-            kv_lens.data_ptr(), ptr(ws_o), ptr(ws_ml), out.data_ptr(), out.stride(0), B, Hq, Hkv, D, part_tiles,
+            block_tables.shape[1], kv_lens.data_ptr(), ptr(ws_o), ptr(ws_ml), out.data_ptr(), out.stride(0), B, Hq, Hkv, D, part_tiles,
             max_parts, float(scale), stream_ptr()), "ragk_attn_decode_rope")
     finally:
         if defer_merge:

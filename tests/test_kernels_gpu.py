@@ -564,6 +564,36 @@ def test_attn_decode_rope_matches_unfused(native, kv_lens, target, Hq, Hkv):
     assert torch.equal(out, ref)
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,S", [(64, 4, 4, 1), (64, 16, 4, 9), (128, 2, 2, 17), (128, 2, 1, 8), (128, 8, 1, 9)])
+@pytest.mark.parametrize("kv_lens,target", [([8193, 8256, 12001, 65], 64), ([8193, 64, 2], 1)])
+def test_attn_decode_rope_long_tables_and_slabs(native, kv_lens, target, D, Hq, Hkv, S):
+    """As above beyond 128 pages a sequence (a lane holds two table entries), for more slabs than a round of loads, and where a
+    wave's queries are half a head, a head, two and more."""
+    torch.manual_seed(15)
+    kc, vc, bt = _paged_setup(kv_lens, Hkv, D, seed=6)
+    B = len(kv_lens)
+    kc, vc, bt = kc.to(DEV), vc.to(DEV), bt.to(DEV)
+    kvl = torch.tensor(kv_lens, dtype=torch.int32, device=DEV)
+    pos = kvl - 1
+    slots = (bt[torch.arange(B, device=DEV), (pos // 64).long()] * 64 + pos % 64).int()
+    P = torch.randn(S, B, (Hq + 2 * Hkv) * D, device=DEV)
+    cos, sin = (t.to(DEV) for t in R.rope_tables(D, 16384, theta=500000.0))
+    pt, mp = native.decode_partitions(max(kv_lens), B, Hkv, target_blocks=target)
+    kc2, vc2 = kc.clone(), vc.clone()
+    q, ref, out = (torch.empty(B, Hq * D, device=DEV).bfloat16() for _ in range(3))
+    native.rope_kv_partials(P, q, pos, cos, sin, slots, kc2, vc2, Hq, Hkv, D)
+    native.attn_decode(q, kc2, vc2, bt, kvl, ref, Hq, Hkv, D, pt, mp)
+    native.attn_decode_rope(P, pos, cos, sin, slots, kc, vc, bt, kvl, out, Hq, Hkv, D, pt, mp)
+    assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    assert torch.equal(out, ref)
+    qh = q.cpu().reshape(B, Hq, D)
+    oracle = R.attention_varlen(qh, None, None, torch.arange(B + 1, dtype=torch.int32), kvl.cpu(), True, 1 / math.sqrt(D),
+                                k_full=lambda s: R.paged_kv_view(kc.cpu(), bt.cpu()[s], kv_lens[s], 64),
+                                v_full=lambda s: R.paged_kv_view(vc.cpu(), bt.cpu()[s], kv_lens[s], 64))
+    # weights and outputs are rounded to bf16 (2^-8 of a value at most, independent: well under 2^-7 of the norm)
+    assert rel_err(out.cpu().reshape(B, Hq, D), oracle) < 2 ** -7
+
+
 @pytest.mark.parametrize("M,N,K,ns", [(5207, 4096, 4096, 2), (5207, 4096, 14336, 2), (300, 4096, 4096, 4),
                                        (1000, 1024, 2048, 2), (256, 520, 1024, 4)])
 def test_gemm_splitk_slabs(native, M, N, K, ns):

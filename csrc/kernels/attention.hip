@@ -16,7 +16,7 @@
 //    from a packed qkv buffer (bidirectional encoders). One block = 4 waves =
 //    GB query heads sharing one KV head x (4/GB) groups of 32 query rows.
 //  * attn_decode<D, G>: one query token per sequence, split-K over the context
-//    (flash-decoding). Each wave streams its own 64-key tiles, the next one
+//    (flash-decoding). Each wave streams its own 32-key units, the next one
 //    requested behind the present one (K to VGPRs, V through VGPRs into a
 //    wave-private LDS tile for the transposed read); 4 waves combine in LDS;
 //    partitions merged by attn_decode_reduce.
@@ -1020,25 +1020,31 @@ struct DecodeArgs {
   const float* cos_t; const float* sin_t;
 };
 
-// Tiles per partition of one sequence: its KV tiles spread evenly over all max_parts partitions
-// (never fewer than part_tiles per partition). The grid is sized once for max_parts (hipGraph
+constexpr int DEC_U = 32;  // keys of a unit: what a wave takes at a time where tiles come through registers
+
+// Units per partition of one sequence: its keys spread evenly over all max_parts partitions (never fewer
+// than part_tiles tiles per partition). The grid is sized once for max_parts (hipGraph
 // capture), so sizing the split from the actual length keeps every launched block busy with the
 // same amount of KV: splitting a 5.3k-token context by a fixed 32-tile partition left 1 of 4
 // partitions idle and 8 vs 5 tiles per wave on the others.
-__device__ __forceinline__ int decode_part_tiles(int n_kt, const DecodeArgs& a) {
-  return max(a.part_tiles, (n_kt + a.max_parts - 1) / a.max_parts);
+__device__ __forceinline__ int decode_part_units(int n, const DecodeArgs& a, int unit = DEC_U) {
+  return max(a.part_tiles * (KT / unit), (n + a.max_parts - 1) / a.max_parts);
 }
 
 // LDS of one decode-attention block: one V tile per wave (KL: and one K tile per wave after them), then the
 // block's rotated q (G x D bf16).
-template <int D, int G, int NW = 4, bool KL = false>
-constexpr int decode_lds_bytes() { return NW * Cfg<D>::TILEB * (KL ? 2 : 1) + G * D * 2; }
+template <int D, int G, int NW = 4, bool KL = false, int DG = 0>
+constexpr int decode_lds_bytes() {
+  return NW * Cfg<D>::TILEB * (KL ? 2 : 1) / (!KL && DG == 0 ? KT / DEC_U : 1) + G * D * 2;
+}
 
 // The K / V stream bounds it, and for short contexts the trips to memory in front of it. Both lengths and page table are one trip,
-// the queries' slabs and the first tile another (four in a row before: length, page, tile, and the slabs behind the tile, since
-// vector loads return in order), and a wave's next tile is on its way while it works on one. One layer, 128-wide heads, us with the
-// join: 11 rows of 2000 tokens, 8 KV heads 28.6 -> 26.1; 3 of 4000 19.3 -> 15.5; 20 of 5000 68.0 -> 63.7; 1 of 5267 13.3 -> 11.9;
-// 2 rows of 2000, 4 KV heads 11.3 -> 10.7; 32 of 4200 in one partition (KL) 96 -> 92.5, 5.97 TB/s.
+// the queries' slabs and the first unit another (four in a row before: length, page, tile, and the slabs behind the tile, since
+// vector loads return in order), and a wave's next unit is on its way while it works on one. Units of half a page: few pages
+// spread over more waves and blocks, and many end closer together (with whole pages, a wave of two beside three of one). One
+// layer, 128-wide heads, us with the join, page by page before / page by page ahead / in units: 11 rows of 2000 tokens, 8 KV heads
+// 28.6 / 26.1 / 23.3; 3 of 4000 19.3 / 15.5 / 14.4; 20 of 5000 68.0 / 63.7 / 59.4; 25 of 2400 60 / - / 53.7; 1 of 5267 13.3 / 11.9
+// / 10.5; 2 rows of 2000, 4 KV heads 11.3 / 10.7 / 8.4; 32 of 4200 in one partition (KL, whole pages) 96 / 92.5, 5.97 TB/s.
 // One split-K partition block of decode attention: partition `part` of KV head `kvh` of sequence `b`.
 // NW: waves per block (4; 8 for the batch-32 grid with one partition per sequence: one 8-wave block per
 // CU keeps the same KV bytes in flight as two 4-wave blocks and needs no merge launch). A multi-partition
@@ -1056,13 +1062,15 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
   constexpr bool REGS = !KL && DG != 2;    // K and V tiles through registers
   constexpr bool AHEAD = REGS && DG == 0;  // ... and requested a tile ahead
   using C = Cfg<D>;
+  constexpr int KU = AHEAD ? DEC_U : KT, UPT = KT / KU;  // keys of a unit, units of a page
+  constexpr int VB = C::TILEB / UPT, VPC = C::PIECES / UPT;  // bytes and 1-KiB pieces of its values
   static_assert(G <= 16, "at most 16 query heads per KV head");
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int wid_u = __builtin_amdgcn_readfirstlane(wid);
   PageRow<2> table(a.block_tables + (size_t)b * a.bt_stride, a.bt_cols, lane);
   const int kv_len = ld_uniform(a.kv_lens + b), pos = ld_uniform((a.qkv_p ? a.positions : a.kv_lens) + b);
-  const int n_kt = (kv_len + KT - 1) / KT;
-  const int pt = decode_part_tiles(n_kt, a);
+  const int n_kt = (kv_len + KU - 1) / KU;  // (all counts below in units)
+  const int pt = decode_part_units(n_kt, a, KU);
   const int kt0 = part * pt;
   if (kt0 >= n_kt) return;  // block-uniform early exit (before any barrier)
   const int kt1 = min(kt0 + pt, n_kt);
@@ -1071,10 +1079,10 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
   table.wait();
 
   bf16x8 qf[C::KS];
-  char* sV = smem + wid * C::TILEB;
+  char* sV = smem + wid * VB;
   char* sK = smem + (NW + wid) * C::TILEB;  // KL only
-  bf16x8 kf[4][C::KS];
-  auto page = [&](int kt) { return ((size_t)table(kt) * a.Hkv + kvh) * KT * D; };
+  bf16x8 kf[KU / 16][C::KS];
+  auto page = [&](int kt) { return (((size_t)table(kt / UPT) * a.Hkv + kvh) * KT + kt % UPT * KU) * D; };
   // (lanes' places as 32-bit offsets from a scalar address: a pair of registers a load otherwise)
   constexpr int VP = C::RPP < C::RB * C::GR ? C::RB * C::GR / C::RPP : 1;  // pieces until the swizzle repeats
   const unsigned k_lane = (fr * D + 8 * fh) * 2;
@@ -1088,7 +1096,7 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
       stage_kv<D, false, NT, 1>(sK, 0, 1, lane, [&](int r) { return kb + (size_t)r * D; });
     } else {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < KU / 16; ++t)
 #pragma unroll
         for (int s = 0; s < C::KS; ++s) {
           const bf16x8* p = reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(kb + 16 * t * D + 32 * s) + k_lane);
@@ -1098,14 +1106,14 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
   };
   // V: whole 1-KiB pieces, by LDS-DMA (KL) or through registers, so that the tile behind it can be on its way while this one is
   // read from LDS (the compiler drains every load in flight around LDS-DMA pieces, K's with them)
-  u32x4 vr[C::PIECES];
+  u32x4 vr[VPC];
   auto request_v = [&](int kt) {
     const bf16_t* vb = a.vc + page(kt);
     if constexpr (!REGS) {
       stage_kv<D, true, NT, 1>(sV, 0, 1, lane, [&](int r) { return vb + (size_t)r * D; });
     } else {
 #pragma unroll
-      for (int i = 0; i < C::PIECES; ++i) {
+      for (int i = 0; i < VPC; ++i) {
         const u32x4* p = reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vb) + i * 1024 + v_lane[i % VP]);
         vr[i] = NT ? __builtin_nontemporal_load(p) : *p;
       }
@@ -1114,7 +1122,7 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
   // Rotating path (qkv_p): q = RoPE(bf16(sum_s P[s][b])) for this KV head's G query heads, staged through LDS; in the block owning
   // the last KV tile the new token's k (rotated) and v are appended meanwhile. Every wave takes whole heads, a rotate_half pair
   // (d, d + D / 2) a lane.
-  bf16_t* s_q = reinterpret_cast<bf16_t*>(smem + NW * C::TILEB * (KL ? 2 : 1));
+  bf16_t* s_q = reinterpret_cast<bf16_t*>(smem + NW * VB * (KL ? 2 : 1));
   constexpr int PL = D / 2, IPW = 64 / PL;  // pairs of a head, heads of a wave at a time
   const bool rope = a.qkv_p != nullptr, append = rope && kt1 == n_kt;  // block-uniform
   const int n_items = G + (append ? 2 : 0);                            // query heads, then k and v
@@ -1229,7 +1237,7 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
       static_assert(C::PIECES < 64, "vmcnt range");
       __builtin_amdgcn_s_waitcnt((C::PIECES & 15) | (((C::PIECES >> 4) & 3) << 14) | (0x7 << 4) | (0xF << 8));
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < KU / 16; ++t)
 #pragma unroll
         for (int s = 0; s < C::KS; ++s) kf[t][s] = load_k<D>(sK, t, s, lane);
     } else if constexpr (DG == 2) {
@@ -1238,7 +1246,7 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
       request_v(kt);
       stage_kv<D, false, NT, 1>(sV, 0, 1, lane, [&](int r) { return kb + (size_t)r * D; });
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < KU / 16; ++t)
 #pragma unroll
         for (int s = 0; s < C::KS; ++s) kf[t][s] = (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
     } else if (DG == 1 && !have) {
@@ -1247,21 +1255,21 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
     }
     if constexpr (DG != 0) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < KU / 16; ++t)
 #pragma unroll
         for (int s = 0; s < C::KS; ++s) dsink ^= __builtin_bit_cast(u32x4, kf[t][s])[0];
       if constexpr (REGS) {
 #pragma unroll
-        for (int i = 0; i < C::PIECES; ++i) dsink ^= vr[i][0];
+        for (int i = 0; i < VPC; ++i) dsink ^= vr[i][0];
       } else {
         wait_vmcnt0();
         dsink ^= *reinterpret_cast<const unsigned*>(sV + 4 * lane);
       }
       return;
     }
-    f32x4 s4[4];
+    f32x4 s4[KU / 16];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < KU / 16; ++t) {
       s4[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < C::KS; ++s) s4[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][s], qf[s], s4[t], 0, 0, 0);
@@ -1271,10 +1279,10 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
       request_k(kt + NW);
       __builtin_amdgcn_sched_barrier(0);
     }
-    const int k0 = kt * KT;
+    const int k0 = kt * KU;
     float mx = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < KU / 16; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int kj = k0 + 16 * t + 4 * fh + r;
@@ -1291,7 +1299,7 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
     const float alpha = __builtin_amdgcn_exp2f(m_i - m_use);
     float ls = 0.f;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < KU / 16; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float p = __builtin_amdgcn_exp2f(s4[t][r] - m_use);
@@ -1302,21 +1310,22 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
     m_i = m_new;
 #pragma unroll
     for (int dt = 0; dt < C::DT; ++dt) o[dt] *= alpha;
-    const bf16x8 pb0 = pack_p(s4[0], s4[1]);
-    const bf16x8 pb1 = pack_p(s4[2], s4[3]);
+    bf16x8 pb[KU / 32];
+#pragma unroll
+    for (int ks = 0; ks < KU / 32; ++ks) pb[ks] = pack_p(s4[2 * ks], s4[2 * ks + 1]);
     if constexpr (REGS) {
 #pragma unroll
-      for (int i = 0; i < C::PIECES; ++i) *reinterpret_cast<u32x4*>(sV + i * 1024 + lane * 16) = vr[i];
+      for (int i = 0; i < VPC; ++i) *reinterpret_cast<u32x4*>(sV + i * 1024 + lane * 16) = vr[i];
       if constexpr (MORE) request_v(kt + NW);
       // (the wave's own LDS accesses stay in order: written above, read below, written again in the next iteration)
     } else {
       __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));  // V tile landed (vmcnt(0), seen by the compiler)
     }
 #pragma unroll
-    for (int dt = 0; dt < C::DT; ++dt) {
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load_vt<D>(sV, dt, 0, lane), pb0, o[dt], 0, 0, 0);
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load_vt<D>(sV, dt, 1, lane), pb1, o[dt], 0, 0, 0);
-    }
+    for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+      for (int ks = 0; ks < KU / 32; ++ks)
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load_vt<D>(sV, dt, ks, lane), pb[ks], o[dt], 0, 0, 0);
   };
   int kt = kt0 + wid_u;
   if constexpr (AHEAD) {
@@ -1334,8 +1343,8 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
   }
   // ---- combine the waves in LDS: each puts its G rows and their statistics where its V tile lay, rows 16 bytes apart in the
   // banks (as 16 rows of D floats behind a barrier, one float a lane, this was 1 us of a block) ----
-  constexpr int OS = D + 4, PER = C::TILEB / 4;  // floats of a row, of a wave
-  static_assert((G * OS + 2 * G) * 4 <= C::TILEB, "a wave's rows fit its V tile");
+  constexpr int OS = D + 4, PER = VB / 4;  // floats of a row, of a wave
+  static_assert((G * OS + 2 * G) * 4 <= VB, "a wave's rows fit its V tile");
   float* so = reinterpret_cast<float*>(smem);
   if constexpr (!REGS) wait_vmcnt0();  // pieces that no tile waited for
   l_i += __shfl_xor(l_i, 16, 64);
@@ -1382,7 +1391,7 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
 
 template <int D, int G, bool NT = false, int NW = 4, int DG = 0, bool KL = false>
 __global__ __launch_bounds__(NW * 64, (NW == 4 && !KL) ? 2 : 1) void attn_decode_kernel(DecodeArgs a) {
-  __shared__ __attribute__((aligned(16))) char smem[decode_lds_bytes<D, G, NW, KL>()];
+  __shared__ __attribute__((aligned(16))) char smem[decode_lds_bytes<D, G, NW, KL, DG>()];
   attn_decode_block<D, G, NT, NW, DG, KL>(a, blockIdx.z, blockIdx.x, blockIdx.y, smem);
 }
 
@@ -1395,8 +1404,8 @@ __global__ void attn_decode_reduce_kernel(DecodeArgs a, int D) {
   const float2 r = join_parts(
       a.part_ml + p0 * 2, a.part_o + p0 * D, D, a.max_parts, t, false,
       [&] {
-        const int n_kt = (a.kv_lens[b] + KT - 1) / KT, pt = decode_part_tiles(n_kt, a);
-        return nparts = (n_kt + pt - 1) / pt;
+        const int n = (a.kv_lens[b] + DEC_U - 1) / DEC_U, pt = decode_part_units(n, a);
+        return nparts = (n + pt - 1) / pt;
       },
       [](float x) { return exp2f(x); });
   if (nparts <= 1) return;  // the partition kernel wrote the output itself

@@ -1469,23 +1469,29 @@ DECODE_MIN_TILES = 4
 
 
 def decode_partitions(max_kv_len, batch, Hkv, target_blocks=None, min_tiles=None):
-    """(part_tiles, max_parts) for split-K decode: grid = max_parts x Hkv x batch <= target_blocks, the two blocks a CU that
-    are resident at once. A few more run as a round of their own behind the first: 11 rows of 2000 tokens in 528 blocks took
-    33.5 us, in 440 27.5; 30 rows of 600 in 720 27.4, in 480 21.6. Over the 69 of 95 batches (1 to 31 rows, 1 to 8 KV heads)
-    whose blocks do not divide, rounding down takes 6 % less at 2500 tokens and 8 % less at 5200 in the mean, 18 % at best; a
-    grid that it leaves a third empty (176 pairs, 352 blocks) takes what rounding up does, within 4 %. The shaped kernel's
-    blocks lose by it (seq_native.decode_parts).
+    """(part_tiles, max_parts) for split-K decode: grid = max_parts x Hkv x batch <= target_blocks, two blocks a CU. More than fit
+    at once run as a round of their own behind the first (20 rows of 5000 tokens, 8 KV heads: 59.4 us in 480 blocks, 63.4 in 640),
+    and fewer, larger ones beat a third of a CU's slots (16 rows of 6000, 4 KV heads: 33.7 in 512, 34.7 in 768). The shaped
+    kernel's blocks lose by rounding down (seq_native.decode_parts).
 
-    The kernel spreads each sequence's actual KV tiles evenly over the max_parts partitions
-    (at least ``part_tiles`` = min_tiles tiles each, attention.hip:decode_part_tiles), so the grid can
-    be sized once for the longest allowed context (hipGraph capture) without idle partitions."""
+    Once batch x KV heads would fill the CUs by itself, one partition per pair (attention.hip KL) where its rounds of one block a
+    CU are at least four fifths full, else three: 264 pairs of 1600 tokens 52.4 -> 45.2 us, 320 of 560 28.0 -> 23.7, 384 of 2400
+    87.5 -> 86.0, 400 of 1250 52.6 -> 51.1; 512 full ones of 3200 tokens 134 in one, 146 in three.
+
+    The kernel spreads each sequence's actual KV tiles evenly over the max_parts partitions (at least ``part_tiles`` tiles each,
+    attention.hip:decode_part_units), so the grid can be sized once for the longest allowed context (hipGraph capture) without
+    idle partitions. part_tiles is half of min_tiles, which caps max_parts: one unit a wave (one row of 500 tokens, 8 KV heads 8.4
+    -> 7.4 us, 2 of 2000 with 4 8.7 -> 8.4, 3 of 4000 with 8 14.7 -> 14.4; 5 of 1000, 320 blocks instead of 160, 9.6 -> 10.3),
+    while a join of more than 32 partitions costs what they save (one of 5267: 10.2 in 28, 13.3 in 42)."""
     target_blocks = DECODE_TARGET_BLOCKS if target_blocks is None else target_blocks
     min_tiles = DECODE_MIN_TILES if min_tiles is None else min_tiles
+    part_tiles = max(1, min_tiles // 2)
     max_kt = max(1, (max_kv_len + 63) // 64)
-    if DECODE_NW8_MIN_PAIRS > 0 and batch * Hkv >= DECODE_NW8_MIN_PAIRS:
-        return min_tiles, 1  # one 8-wave block per (sequence, KV head), no merge (attention.hip NW = 8)
-    mp = max(1, min(target_blocks // (batch * Hkv), -(-max_kt // min_tiles)))
-    return min_tiles, mp
+    pairs = batch * Hkv
+    if DECODE_NW8_MIN_PAIRS > 0 and pairs >= DECODE_NW8_MIN_PAIRS:
+        rounds = -(-pairs // DECODE_NW8_MIN_PAIRS)
+        return part_tiles, 1 if 5 * pairs >= 4 * rounds * DECODE_NW8_MIN_PAIRS else 3
+    return part_tiles, max(1, min(target_blocks // pairs, -(-max_kt // min_tiles)))
 
 
 # One partition per (sequence, KV head) in 8-wave blocks once batch x KV heads reaches this (>= one block

@@ -21,6 +21,7 @@
 // The MFMA kernels keep the softmax weights at 16 significant bits for P.V (bf16 high + low part, two products).
 #include "attn_tiles.h"
 #include "seq_common.h"
+#include <type_traits>
 using namespace ragk;
 
 namespace {
@@ -435,7 +436,7 @@ struct ShapedDecode {
   const float* P; int S; int ldp; size_t slab;  // projection slabs [S][B][ldp]
   const bf16_t* bias;                            // [ldp] or null
   bf16_t* kc; bf16_t* vc;
-  const int* block_tables; int bt_stride;
+  const int* block_tables; int bt_stride, bt_cols;
   const int* kv_lens; const int* slots;
   const float* table;
   const float* v_first; const float* lam;        // [B][G * DV] values to mix in, or null
@@ -447,15 +448,6 @@ struct ShapedDecode {
   float scale, softcap;
 };
 
-__device__ __forceinline__ void slab_row8(const ShapedDecode& a, int b, int col, float* f) {
-  sum_slabs8(a.P + (size_t)b * a.ldp + col, a.S, a.slab, f);
-  if (a.bias) {
-    float w[8];
-    ld8(a.bias + col, w);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] += w[e];
-  }
-}
 __device__ __forceinline__ float slab_gate(const ShapedDecode& a, int b, int h) {
   if (a.off_g < 0) return 1.f;
   float g = a.bias ? bf2f(a.bias[a.off_g + h]) : 0.f;
@@ -470,136 +462,208 @@ __device__ __forceinline__ float slab_gate(const ShapedDecode& a, int b, int h) 
   }
   return __builtin_amdgcn_rcpf(1.f + __expf(-g));
 }
-// pages per partition: the visited pages spread over all partitions, at least min_tiles each
-__device__ __forceinline__ int part_pages(int n, const ShapedDecode& a) {
-  return max(a.min_tiles, (n + a.max_parts - 1) / a.max_parts);
+constexpr int DEC_U = 32;                // keys of a unit: what a wave takes at a time
+constexpr int DEC_UPT = KT / DEC_U;      // units of a page
+// units that a new token at `pos` visits (the last page's second half may lie past it)
+__device__ __forceinline__ int units(const Pages& pg, int pos) { return pg.n * DEC_UPT - (pos % KT < DEC_U ? 1 : 0); }
+// units per partition: the visited ones spread over all partitions, at least min_tiles pages each
+__device__ __forceinline__ int part_units(int n, const ShapedDecode& a) {
+  return max(a.min_tiles * DEC_UPT, (n + a.max_parts - 1) / a.max_parts);
 }
 
 constexpr int DEC_HEADS = 16;  // query heads per decode block (one MFMA column each)
 
-// grid: (max_parts, KV heads x groups of 16 query heads, batch), 4 waves; a wave takes every 4th page
+// grid: (KV heads x groups of 16 query heads, batch, max_parts), 4 waves; a wave takes every 4th unit. What bounds it, its two trips
+// to memory ahead of the stream, units of half a page and the next one behind the present one: as attn_decode_block (attention.hip).
+// Us with the join, before and now: 17 rows of 2400 tokens, 32 heads over 8, 43.8 -> 40.3; 1 of 5000 14.6 -> 11.3; 25 of 4700 97.7
+// -> 83.3 (5.9 TB/s); 16 heads over 4: 4 of 1000 14.9 -> 9.9, 20 of 2400 35.3 -> 22.9, 50 of 1250 39.8 -> 28.7.
 template <int DK, int DV>
 __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_shaped_decode_kernel(ShapedDecode a) {
   using CK = Cfg<DK>;
   using CV = Cfg<DV>;
-  __shared__ __attribute__((aligned(16))) char smem[4 * CV::TILEB + DEC_HEADS * DK * 2 + 4 * (16 + 64) * 4];
+  constexpr int KB = DEC_U / 16, VPC = CV::PIECES / DEC_UPT;  // key blocks of a unit, 1-KiB pieces of its values
+  constexpr int OS = DV + 4;                                   // floats between the combined rows
+  constexpr int ROWS = DEC_HEADS * (OS + 2) * 4, PW = CV::TILEB / DEC_UPT > ROWS ? CV::TILEB / DEC_UPT : ROWS;  // LDS of a wave
+  __shared__ __attribute__((aligned(16))) char smem[4 * PW + DEC_HEADS * DK * 2];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int wid_u = __builtin_amdgcn_readfirstlane(wid);
-  const int part = blockIdx.x, b = blockIdx.z;
+  const int part = blockIdx.z, b = blockIdx.y;
   const int Gq = a.H / a.G, chunks = (Gq + DEC_HEADS - 1) / DEC_HEADS;
-  const int kvh = blockIdx.y / chunks, hc = blockIdx.y % chunks;
+  const int kvh = blockIdx.x / chunks, hc = blockIdx.x % chunks;
   const int h0 = kvh * Gq + hc * DEC_HEADS, nh = min(DEC_HEADS, Gq - hc * DEC_HEADS);
-  const int pos = a.kv_lens[b] - 1;
+  PageRow<2> table(a.block_tables + (size_t)b * a.bt_stride, a.bt_cols, lane);
+  const int pos = ld_uniform(a.kv_lens + b) - 1;
   const Pages pg = visited(pos, pos, a.window, a.keep);
-  const int pt = part_pages(pg.n, a);
+  const int n = units(pg, pos), pt = part_units(n, a);
   const int it0 = part * pt;
-  if (it0 >= pg.n) return;  // block-uniform, before any barrier
-  const int it1 = min(it0 + pt, pg.n), nparts = (pg.n + pt - 1) / pt;
+  if (it0 >= n) return;  // block-uniform, before any barrier
+  const int it1 = min(it0 + pt, n), nparts = (n + pt - 1) / pt;
   const int fr = lane & 15, fh = lane >> 4;
-  const int* bt = a.block_tables + (size_t)b * a.bt_stride;
-  char* sV = smem + wid_u * CV::TILEB;
-  bf16_t* s_q = reinterpret_cast<bf16_t*>(smem + 4 * CV::TILEB);
+  table.wait();
+  char* sV = smem + wid_u * PW;
+  bf16_t* s_q = reinterpret_cast<bf16_t*>(smem + 4 * PW);
 
-  // the wave's first page is requested before the prologue (not the page that the new token goes into)
-  const bool pre = it0 + wid_u < it1 && it0 + wid_u != pg.n - 1;
-  bf16x8 kf[4][CK::KS];
-  auto request = [&](int it) {
-    const size_t pgi = (size_t)bt[pg.page(it)] * a.G + kvh;
-    const bf16_t* kb = a.kc + pgi * KT * DK;
-    const bf16_t* vb = a.vc + pgi * KT * DV;
+  bf16x8 kf[KB][CK::KS];
+  u32x4 vr[VPC];
+  constexpr int VP = CV::RPP < CV::RB * CV::GR ? CV::RB * CV::GR / CV::RPP : 1;  // pieces until the swizzle repeats
+  const unsigned k_lane = (fr * DK + 8 * fh) * 2;
+  unsigned v_lane[VP];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int s = 0; s < CK::KS; ++s)
-        kf[t][s] = *reinterpret_cast<const bf16x8*>(kb + (size_t)(16 * t + fr) * DK + 32 * s + 8 * fh);
-    __builtin_amdgcn_sched_barrier(0);  // K before V: the scores and the softmax run while V is landing
-    stage_kv<DV, true, false, 1>(sV, 0, 1, lane, [&](int r) { return vb + (size_t)r * DV; });
+  for (int i = 0; i < VP; ++i)
+    v_lane[i] = lane / CV::NC * CV::ROWB + 16 * ((lane % CV::NC) ^ vswz<DV>(i * CV::RPP + lane / CV::NC));
+  auto first_key = [&](int it) {  // (row of the cache pages, all heads of a page behind each other)
+    return ((size_t)table(pg.page(it / DEC_UPT)) * a.G + kvh) * KT + it % DEC_UPT * DEC_U;
   };
-  if (pre) request(it0 + wid_u);
-
-  constexpr int QV = DK / 8, VV = DV / 8;
-  const bool append = it1 == pg.n;
-  const int n_q = nh * QV, n_all = n_q + (append ? QV + VV : 0);
-  for (int i = threadIdx.x; i < n_all; i += 256) {
-    float f[8];
-    if (i < n_q) {
-      slab_row8(a, b, h0 * DK + i * 8, f);
-      st8(s_q + i * 8, f);
-    } else {
-      const int slot = a.slots[b];
-      const size_t row = ((size_t)(slot >> 6) * a.G + kvh) * KT + (slot & 63);
-      const int j = i - n_q;
-      if (j < QV) {
-        slab_row8(a, b, a.off_k + kvh * DK + j * 8, f);
-        st8(a.kc + row * DK + j * 8, f);
-      } else {
-        const int c = (j - QV) * 8;
-        slab_row8(a, b, a.off_v + kvh * DV + c, f);
-        const size_t vo = ((size_t)b * a.G + kvh) * DV + c;
-        if (a.v_own) st8(a.v_own + vo, f);
-        if (a.v_first) {
-          const float lm = a.lam[0];
-          float w[8];
-          ld8(a.v_first + vo, w);
+  auto request_k = [&](int it) {
+    const char* kb = reinterpret_cast<const char*>(a.kc + first_key(it) * DK);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) f[e] = (1.f - lm) * f[e] + lm * w[e];
-        }
-        st8(a.vc + row * DV + c, f);
+    for (int t = 0; t < KB; ++t)
+#pragma unroll
+      for (int s = 0; s < CK::KS; ++s) kf[t][s] = *reinterpret_cast<const bf16x8*>(kb + (16 * t * DK + 32 * s) * 2 + k_lane);
+  };
+  auto request_v = [&](int it) {
+    const char* vb = reinterpret_cast<const char*>(a.vc + first_key(it) * DV);
+#pragma unroll
+    for (int i = 0; i < VPC; ++i) vr[i] = *reinterpret_cast<const u32x4*>(vb + i * 1024 + v_lane[i % VP]);
+  };
+
+  // Projection rows, four columns a thread: the heads' queries, then (in the block that takes the last unit) the new token's k and v
+  const bool append = it1 == n;  // block-uniform
+  const int n_q = nh * DK / 4, n_all = n_q + (append ? (DK + DV) / 4 : 0);
+  f32x4 x[PSU], first;
+  uint2 bias;
+  auto column = [&](int i) {
+    const int j = i - n_q;
+    return j < 0 ? h0 * DK + 4 * i : j < DK / 4 ? a.off_k + kvh * DK + 4 * j : a.off_v + kvh * DV + 4 * min(j - DK / 4, DV / 4 - 1);
+  };
+  auto slab = [&](int i, int u) {
+    return *reinterpret_cast<const f32x4*>(a.P + (size_t)u * a.slab + (size_t)b * a.ldp + column(i));
+  };
+  auto value = [&](int i) {  // place of a value item among the tokens' values
+    return ((size_t)b * a.G + kvh) * DV + 4 * max(0, min(i - n_q - DK / 4, DV / 4 - 1));
+  };
+  const float lm = a.v_first ? a.lam[0] : 0.f;
+  auto request_item = [&](int i) {
+#pragma unroll
+    for (int u = 0; u < PSU; ++u) x[u] = slab(i, min(u, a.S - 1));
+    bias = a.bias ? *reinterpret_cast<const uint2*>(a.bias + column(i)) : make_uint2(0u, 0u);
+    first = a.v_first ? *reinterpret_cast<const f32x4*>(a.v_first + value(i)) : (f32x4){0.f, 0.f, 0.f, 0.f};
+  };
+  auto finish_item = [&](int i) {
+    f32x4 f = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < PSU; ++u)
+      if (u < a.S) f += x[u];
+    for (int u = PSU; u < a.S; ++u) f += slab(i, u);
+    if (a.bias)
+      f += (f32x4){__uint_as_float(bias.x << 16), __uint_as_float(bias.x & 0xffff0000u), __uint_as_float(bias.y << 16),
+                   __uint_as_float(bias.y & 0xffff0000u)};
+    const f32x4 own = f;
+    if (a.v_first && i >= n_q + DK / 4) f = (1.f - lm) * f + lm * first;
+    const uint2 r = make_uint2(pk2bf(f[0], f[1]), pk2bf(f[2], f[3]));
+    asm volatile("" ::"v"(r.x), "v"(r.y), "v"(first));  // every load is used on every path
+    if (i < n_q) {
+      *reinterpret_cast<uint2*>(s_q + 4 * i) = r;
+    } else if (i < n_all) {
+      const int slot = ld_uniform(a.slots + b), j = i - n_q;
+      const size_t row = ((size_t)(slot >> 6) * a.G + kvh) * KT + (slot & 63);
+      if (j < DK / 4) {
+        *reinterpret_cast<uint2*>(a.kc + row * DK + 4 * j) = r;
+      } else {
+        if (a.v_own) *reinterpret_cast<f32x4*>(a.v_own + value(i)) = own;
+        *reinterpret_cast<uint2*>(a.vc + row * DV + 4 * (j - DK / 4)) = r;
       }
     }
-  }
-  __syncthreads();  // q in LDS; the appended row visible to the whole block
-  bf16x8 qf[CK::KS];
-#pragma unroll
-  for (int s = 0; s < CK::KS; ++s)
-    qf[s] = fr < nh ? *reinterpret_cast<const bf16x8*>(s_q + fr * DK + 32 * s + 8 * fh) : (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
-
-  const Shape shape = make_shape(a.scale, a.softcap);
+  };
   const float* tb = a.table ? a.table + (size_t)(h0 + min(fr, nh - 1)) * (a.far + 1) : nullptr;
   const float far_bias = tb ? tb[a.far] * LOG2E : 0.f;
+  // (requested whether the wave has a unit or not, and in this order: attn_decode_block)
+  const int first_it = min(it0 + wid_u, it1 - 1);
+  request_item(threadIdx.x);
+  __builtin_amdgcn_sched_barrier(0);
+  request_k(first_it);
+  __builtin_amdgcn_sched_barrier(0);
+  request_v(first_it);
+  __builtin_amdgcn_sched_barrier(0);
+  finish_item(threadIdx.x);
+  for (int i0 = 256; i0 < n_all; i0 += 256) {  // block-uniform
+    request_item(i0 + threadIdx.x);
+    finish_item(i0 + threadIdx.x);
+  }
+  if (append) {
+    __syncthreads();  // q in LDS; the appended row visible to the whole block
+    if (first_it == n - 1) {
+      request_k(first_it);
+      __builtin_amdgcn_sched_barrier(0);
+      request_v(first_it);
+    }
+  } else {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  bf16x8 qf[CK::KS];
+#pragma unroll
+  for (int s = 0; s < CK::KS; ++s) {
+    qf[s] = *reinterpret_cast<const bf16x8*>(s_q + min(fr, nh - 1) * DK + 32 * s + 8 * fh);
+    if (fr >= nh) qf[s] = (bf16x8){0, 0, 0, 0, 0, 0, 0, 0};
+  }
+
+  const Shape shape = make_shape(a.scale, a.softcap);
   const bool capped = shape.cap2 > 0.f;
   const int win = a.window > 0 ? a.window : 0x7fffffff;
   f32x4 o[CV::DT];
 #pragma unroll
   for (int dt = 0; dt < CV::DT; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
   float m_i = -INFINITY, l_i = 0.f;
-  for (int it = it0 + wid_u; it < it1; it += 4) {
-    if (!(pre && it == it0 + wid_u)) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the previous page's V reads have retired
-      request(it);
-    }
-    const int k0 = pg.page(it) * KT;
-    f32x4 s4[4];
+  auto unit = [&](int it, auto more_t) {
+    constexpr bool MORE = decltype(more_t)::value;
+    const int k0 = pg.page(it / DEC_UPT) * KT + it % DEC_UPT * DEC_U;
+    f32x4 s4[KB];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < KB; ++t) {
       s4[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < CK::KS; ++s) s4[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][s], qf[s], s4[t], 0, 0, 0);
     }
     const int d0 = pos - k0 - 4 * fh;  // distance of this lane's key 0
-    const bool far_only = !tb || pos - (k0 + KT - 1) >= a.far;
+    const bool far_only = !tb || pos - (k0 + DEC_U - 1) >= a.far;
+    f32x4 near[KB];  // biases of keys nearer than the table's end (ahead of the next unit: loads return in order)
+#pragma unroll
+    for (int t = 0; t < KB; ++t) near[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (!far_only) {
+#pragma unroll
+      for (int t = 0; t < KB; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) near[t][r] = tb[max(0, min(d0 - 16 * t - r, a.far))] * LOG2E;
+#pragma unroll
+      for (int t = 0; t < KB; ++t) asm volatile("" ::"v"(near[t]));
+    }
+    if constexpr (MORE) {
+      __builtin_amdgcn_sched_barrier(0);
+      request_k(it + 4);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     const float base = (capped ? shape.cap2 : 0.f) + (far_only ? far_bias : 0.f);
     if (capped) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < KB; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) s4[t][r] = __builtin_fmaf(-2.f * shape.cap2, shape.sigma(s4[t][r]), base);
     } else {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < KB; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) s4[t][r] = __builtin_fmaf(s4[t][r], shape.c, base);
     }
     if (!far_only) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          s4[t][r] = __builtin_fmaf(tb[max(0, min(d0 - 16 * t - r, a.far))], LOG2E, s4[t][r]);
+      for (int t = 0; t < KB; ++t) s4[t] += near[t];
     }
-    if (!(k0 + KT - 1 <= pos && (pos - k0 < win || k0 + KT <= a.keep))) {
+    if (!(k0 + DEC_U - 1 <= pos && (pos - k0 < win || k0 + DEC_U <= a.keep))) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < KB; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int d = d0 - 16 * t - r;
@@ -609,7 +673,7 @@ __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_sh
     }
     float mx = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < KB; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s4[t][r]);
     mx = max_xor32(max_xor16(mx));
@@ -617,7 +681,7 @@ __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_sh
     const float alpha = __builtin_amdgcn_exp2f(m_i - m_use);
     float ls = 0.f;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < KB; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float p = __builtin_amdgcn_exp2f(s4[t][r] - m_use);
@@ -628,54 +692,64 @@ __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_sh
     m_i = m_new;
 #pragma unroll
     for (int dt = 0; dt < CV::DT; ++dt) o[dt] *= alpha;
-    bf16x8 hi[2], lo[2];
-    split_p(s4[0], s4[1], hi[0], lo[0]);
-    split_p(s4[2], s4[3], hi[1], lo[1]);
-    wait_vmcnt0();  // the V page is in this wave's LDS
+    bf16x8 hi, lo;
+    split_p(s4[0], s4[1], hi, lo);
 #pragma unroll
-    for (int dt = 0; dt < CV::DT; ++dt)
+    for (int i = 0; i < VPC; ++i) *reinterpret_cast<u32x4*>(sV + i * 1024 + lane * 16) = vr[i];
+    if constexpr (MORE) request_v(it + 4);
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        const bf16x8 vf = load_vt<DV>(sV, dt, ks, lane);
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, hi[ks], o[dt], 0, 0, 0);
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, lo[ks], o[dt], 0, 0, 0);
-      }
+    for (int dt = 0; dt < CV::DT; ++dt) {
+      const bf16x8 vf = load_vt<DV>(sV, dt, 0, lane);
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, hi, o[dt], 0, 0, 0);
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, lo, o[dt], 0, 0, 0);
+    }
+  };
+  int it = it0 + wid_u;
+  if (it < it1) {
+    for (; it + 4 < it1; it += 4) unit(it, std::true_type{});
+    unit(it, std::false_type{});
   }
 
-  // combine the 4 waves: O [4][16][DV] reuses the V pages, statistics sit behind the q rows
-  __syncthreads();
+  // combine the 4 waves: each puts its rows and their statistics where its values lay
   float* so = reinterpret_cast<float*>(smem);
-  float* sm = reinterpret_cast<float*>(smem + 4 * CV::TILEB + DEC_HEADS * DK * 2);
-  float* sl = sm + 64;
-  if (fh == 0) sm[wid * 16 + fr] = m_i;
-  sl[wid * 64 + lane] = l_i;
+  l_i += __shfl_xor(l_i, 16, 64);
+  l_i += __shfl_xor(l_i, 32, 64);
+  if (fr < nh) {
+    float* w = so + wid_u * (PW / 4);
 #pragma unroll
-  for (int dt = 0; dt < CV::DT; ++dt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) so[(wid * 16 + fr) * DV + 16 * dt + 4 * fh + r] = o[dt][r];
+    for (int dt = 0; dt < CV::DT; ++dt) *reinterpret_cast<f32x4*>(w + fr * OS + 16 * dt + 4 * fh) = o[dt];
+    if (fh == 0) *reinterpret_cast<float2*>(w + DEC_HEADS * OS + 2 * fr) = make_float2(m_i, l_i);
+  }
   __syncthreads();
-  for (int e = threadIdx.x; e < nh * DV; e += 256) {
-    const int g = e / DV, d = e % DV, h = h0 + g;
+  for (int e = threadIdx.x; e < nh * (DV / 4); e += 256) {
+    const int g = e / (DV / 4), d = e % (DV / 4) * 4, h = h0 + g;
+    float2 ml[4];
+    f32x4 ov[4];
     float M = nparts == 1 && a.sink ? 0.f : -INFINITY;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) M = fmaxf(M, sm[w * 16 + g]);
+    for (int w = 0; w < 4; ++w) {
+      ml[w] = *reinterpret_cast<const float2*>(so + w * (PW / 4) + DEC_HEADS * OS + 2 * g);
+      ov[w] = *reinterpret_cast<const f32x4*>(so + w * (PW / 4) + g * OS + d);
+      M = fmaxf(M, ml[w].x);
+    }
     const float Mu = M == -INFINITY ? 0.f : M;
-    float L = nparts == 1 && a.sink ? __builtin_amdgcn_exp2f(-Mu) : 0.f, O = 0.f;
+    float L = nparts == 1 && a.sink ? __builtin_amdgcn_exp2f(-Mu) : 0.f;
+    f32x4 O = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-      const float sc = __builtin_amdgcn_exp2f(sm[w * 16 + g] - Mu);
-      L += (sl[w * 64 + g] + sl[w * 64 + g + 16] + sl[w * 64 + g + 32] + sl[w * 64 + g + 48]) * sc;
-      O += so[(w * 16 + g) * DV + d] * sc;
+      const float sc = __builtin_amdgcn_exp2f(ml[w].x - Mu);
+      L += ml[w].y * sc;
+      O += ov[w] * sc;
     }
     if (nparts == 1) {
-      a.out[(size_t)b * a.ldo + h * DV + d] = f2bf(L > 0.f ? O / L * slab_gate(a, b, h) : 0.f);
+      const float gate = slab_gate(a, b, h);
+      if (!(L > 0.f)) O = (f32x4){0.f, 0.f, 0.f, 0.f}, L = 1.f;
+      *reinterpret_cast<u32x2_a2*>(a.out + (size_t)b * a.ldo + h * DV + d) =
+          (u32x2_a2){pk2bf(O[0] / L * gate, O[1] / L * gate), pk2bf(O[2] / L * gate, O[3] / L * gate)};
     } else {
       const size_t pi = ((size_t)b * a.H + h) * a.max_parts + part;
-      a.part_o[pi * DV + d] = O;
-      if (d == 0) {
-        a.part_ml[pi * 2] = M;
-        a.part_ml[pi * 2 + 1] = L;
-      }
+      *reinterpret_cast<f32x4_a4*>(a.part_o + pi * DV + d) = O;
+      if (d == 0) *reinterpret_cast<f32x2_a4*>(a.part_ml + pi * 2) = (f32x2_a4){M, L};
     }
   }
 }
@@ -690,7 +764,7 @@ __global__ void attn_shaped_merge_kernel(ShapedDecode a, int DV) {
       a.part_ml + p0 * 2, a.part_o + p0 * DV, DV, a.max_parts, d, a.sink,
       [&] {
         const int pos = a.kv_lens[b] - 1;
-        const int n = visited(pos, pos, a.window, a.keep).n, pt = part_pages(n, a);
+        const int n = units(visited(pos, pos, a.window, a.keep), pos), pt = part_units(n, a);
         return nparts = (n + pt - 1) / pt;
       },
       [](float x) { return __builtin_amdgcn_exp2f(x); });
@@ -723,7 +797,7 @@ int launch_prefill(ShapedPrefill pa, int n_tiles, int bounded, hipStream_t st) {
 template <int DK, int DV>
 int launch_decode(const ShapedDecode& a, hipStream_t st) {
   const int chunks = (a.H / a.G + DEC_HEADS - 1) / DEC_HEADS;
-  hipLaunchKernelGGL((attn_shaped_decode_kernel<DK, DV>), dim3(a.max_parts, a.G * chunks, a.B), dim3(256), 0, st, a);
+  hipLaunchKernelGGL((attn_shaped_decode_kernel<DK, DV>), dim3(a.G * chunks, a.B, a.max_parts), dim3(256), 0, st, a);
   if (a.max_parts > 1)
     hipLaunchKernelGGL(attn_shaped_merge_kernel, dim3(a.H, a.B), dim3(DV < 64 ? 64 : DV), 0, st, a, DV);
   return (int)hipGetLastError();
@@ -826,8 +900,8 @@ RAGK_API int ragk_row_attn_rows(const void* q, int ldq, const void* kv, int ldk,
 
 // bf16 caches, fp32 slabs P [S][B][ldp] (+ bias). The new token's k / v go to `slots`; out [B][ldo].
 RAGK_API int ragk_shaped_attn_decode(const float* P, int S, int ldp, const void* bias, void* kc, void* vc,
-                                     const int* block_tables, int bt_stride, const int* kv_lens, const int* slots,
-                                     const float* table, const float* v_first, const float* lam, float* v_own, void* out,
+                                     const int* block_tables, int bt_stride, int bt_cols, const int* kv_lens,
+                                     const int* slots, const float* table, const float* v_first, const float* lam, float* v_own, void* out,
                                      int ldo, float* part_o, float* part_ml, int B, int H, int G, int DK, int DV,
                                      int off_k, int off_v, int off_g, int window, int keep, int far, int sink,
                                      int min_tiles, int max_parts, float scale, float softcap, hipStream_t st) {
@@ -836,7 +910,7 @@ RAGK_API int ragk_shaped_attn_decode(const float* P, int S, int ldp, const void*
       (max_parts > 1 && (!part_o || !part_ml)) || B > 65535 || window < 0 || keep < 0 || far < 0)
     return (int)hipErrorInvalidValue;
   const ShapedDecode a{P, S, ldp, (size_t)B * ldp, (const bf16_t*)bias, (bf16_t*)kc, (bf16_t*)vc, block_tables, bt_stride,
-                       kv_lens, slots, table, v_first, lam, v_own, (bf16_t*)out, ldo, part_o, part_ml, B, H, G, off_k,
+                       bt_cols, kv_lens, slots, table, v_first, lam, v_own, (bf16_t*)out, ldo, part_o, part_ml, B, H, G, off_k,
                        off_v, off_g, window, keep, far, sink, min_tiles, max_parts, scale, softcap};
   RAGK_SHAPED_DISPATCH(launch_decode, a, st);
 }

@@ -110,7 +110,7 @@ _SIGS = {
     "ragk_ssm_conv": [P, P, P, I, I, P, I, I, P, P, P, P, I, I, I, S],
     "ragk_ssm_scan_seq": [P, P, P, I, I, P, I, P, I, I, P, P, P, P, P, I, I, I, I, I, S],
     "ragk_shaped_attn_prefill": [P, I, P, P, P, I, P, P, P, I, I, P, P, I, I, I, I, I, I, I, I, I, I, I, F, F, S],
-    "ragk_shaped_attn_decode": [P, I, I, P, P, P, P, I, P, P, P, P, P, P, P, I, P, P, I, I, I, I, I, I, I, I, I, I, I, I,
+    "ragk_shaped_attn_decode": [P, I, I, P, P, P, P, I, I, P, P, P, P, P, P, P, I, P, P, I, I, I, I, I, I, I, I, I, I, I, I,
                                 I, I, F, F, S],
     "ragk_row_attn_prefill": [P, I, P, I, I, P, P, P, P, I, P, I, I, I, I, I, I, I, F, S],
     "ragk_row_attn_rows": [P, I, P, I, I, P, P, P, P, I, I, I, I, I, I, I, I, F, I, S],

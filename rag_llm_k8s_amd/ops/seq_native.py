@@ -173,27 +173,31 @@ def query_tiles(q_lens, qt):
 
 
 DECODE_TARGET_BLOCKS = 512  # decode attention grid: partitions x KV heads x batch
-DECODE_MIN_PAGES = 4
+DECODE_MIN_PAGES = 4  # of a partition when every page is visited: more partitions cost their join what they save
+DECODE_PART_PAGES = 2  # of a shorter sequence's partition: a unit a wave (one row of 200 tokens 267 -> 263 us a step)
 
 
 def decode_parts(spec, max_kv_len, batch):
-    """Partitions per (sequence, KV head): the pages a query can visit, spread to fill the chip. Rounded up, unlike
-    native.decode_partitions: 17 rows of 3000 tokens, 8 KV heads, take 44.8 us in 544 blocks and 47.9 in 408, where a third of
-    the slots have nothing to hide this kernel's score work behind."""
+    """Partitions per (sequence, KV head): the pages a query can visit, spread to fill the chip, two blocks a CU. Rounded down
+    while that leaves a quarter of those places at most: decode steps of 25 rows of 4700 tokens 788 us in 400 blocks, 796 in 600;
+    20 of 2400, 4 KV heads 338 in 480, 346 in 560; 17 of 2400 the same in 408 as in 544; 40 of 1600 820 in 320, 810 in 640."""
     pages = -(-max_kv_len // 64)
     if spec.window > 0:
         pages = min(pages, -(-spec.keep_first // 64) + -(-spec.window // 64) + 1)
     rows = batch * spec.kv_heads * -(-spec.group // 16)
-    return max(1, min(-(-DECODE_TARGET_BLOCKS // rows), -(-pages // DECODE_MIN_PAGES)))
+    parts = max(1, DECODE_TARGET_BLOCKS // rows)
+    if 4 * parts * rows < 3 * DECODE_TARGET_BLOCKS:
+        parts += 1
+    return min(parts, -(-pages // DECODE_MIN_PAGES))
 
 
 def decode_split(specs, max_kv_len, batch, device):
     """(min pages per partition, 1, partition sums, partition statistics): one workspace all layers share."""
     need = [(batch * s.heads * p, s.dvp) for s in specs for p in [decode_parts(s, max_kv_len, batch)] if p > 1]
     if not need:
-        return DECODE_MIN_PAGES, 1, None, None
+        return DECODE_PART_PAGES, 1, None, None
     f32 = dict(dtype=F32, device=device)
-    return (DECODE_MIN_PAGES, 1, torch.empty(max(r * d for r, d in need), **f32),
+    return (DECODE_PART_PAGES, 1, torch.empty(max(r * d for r, d in need), **f32),
             torch.empty(max(r for r, _ in need) * 2, **f32))
 
 
@@ -300,10 +304,10 @@ def attn_decode(P, bias, spec, table, slots, kc, vc, meta, out, v_first=None, la
              "decode workspace too small")
     check(_lib.lib().ragk_shaped_attn_decode(
         P.data_ptr(), S, N, ptr(bias), kc.data_ptr(), vc.data_ptr(), meta.block_tables.data_ptr(),
-        meta.block_tables.stride(0), meta.kv_lens.data_ptr(), slots.data_ptr(), ptr(table), ptr(v_first),
+        meta.block_tables.stride(0), meta.block_tables.shape[1], meta.kv_lens.data_ptr(), slots.data_ptr(), ptr(table), ptr(v_first),
         ptr(lam) if v_first is not None else None, own.data_ptr(), out.data_ptr(), out.stride(0), ptr(meta.ws_o),
         ptr(meta.ws_ml), B, spec.heads, spec.kv_heads, spec.dkp, spec.dvp, spec.off_k, spec.off_v,
-        spec.off_g if spec.gate else -1, spec.window, spec.keep_first, spec.far, int(spec.sink), DECODE_MIN_PAGES, parts,
+        spec.off_g if spec.gate else -1, spec.window, spec.keep_first, spec.far, int(spec.sink), DECODE_PART_PAGES, parts,
         float(spec.scale), float(spec.softcap), stream_ptr()), "ragk_shaped_attn_decode")
     return own
 

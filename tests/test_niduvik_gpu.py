@@ -214,6 +214,41 @@ def test_attention_decode_partitions_agree(be):
         close(heads_of(spec, out), want[-1:], 0.01, max_kv)
 
 
+@pytest.mark.parametrize("window,keep,vdim", [(0, 0, 64), (1000, 70, 128), (130, 0, 256)])
+def test_attention_decode_units(be, window, keep, vdim):
+    """Lengths around the 32-key units that a wave takes, contexts beyond the 128 pages whose table entries a block holds, and more
+    slabs than one round of loads, against plain fp64 attention of the new tokens."""
+    spec = AttnSpec(heads=8, kv_heads=2, dim=64, vdim=vdim, window=window, keep_first=keep, far=90, scale=0.125, softcap=12.0,
+                    sink=True, gate=True)
+    lens = [8300, 1, 31, 32, 33, 64, 65, 96, 97, 1100, 8193]
+    g = torch.Generator().manual_seed(window + vdim)
+    pages = Pages(spec, lens, BF16)
+    for c in (pages.kc, pages.vc):
+        c.copy_(torch.randn(c.shape, generator=g))
+    B, S = len(lens), 9
+    table = torch.randn(spec.heads, spec.far + 1, generator=g).to(DEV)
+    P = (torch.randn(S, B, spec.row, generator=g) / 3).to(DEV)
+    slots = torch.cat([pages.slots(i, n - 1, n) for i, n in enumerate(lens)]).to(DEV)
+    out = torch.zeros(B, spec.out_row, dtype=BF16, device=DEV)
+    be.shaped_attn_decode(P, None, spec, table, slots, pages.kc, pages.vc, decode_meta(spec, pages, lens, 8320), out)
+    row = P.sum(0).cpu()
+    kc, vc, got = pages.kc.cpu(), pages.vc.cpu(), heads_of(spec, out)
+    want = torch.zeros(B, spec.heads, vdim, dtype=torch.float64)
+    for i, n in enumerate(lens):
+        p = torch.arange(n)
+        blk = pages.bt[i, p // 64].long()
+        k, v = (c[blk, :, p % 64].double().transpose(0, 1) for c in (kc, vc))
+        d = n - 1 - p
+        seen = (d < window) | (p < keep) if window else d >= 0
+        q = row[i, :spec.off_k].to(BF16).double().view(2, 4, 64)
+        x = torch.matmul(q, k.transpose(1, 2)).view(8, n) * spec.scale
+        s = spec.softcap * torch.tanh(x / spec.softcap) + table.cpu().double()[:, d.clamp(max=spec.far)]
+        w = torch.softmax(torch.cat([s[:, seen], torch.zeros(8, 1, dtype=torch.float64)], 1), 1)[:, :-1]
+        gate = torch.sigmoid(row[i, spec.off_g:spec.off_g + 8].double())[:, None]
+        want[i] = torch.matmul(w.view(2, 4, -1), v[:, seen]).view(8, vdim) * gate
+    close(got, want, 0.01)
+
+
 def test_attention_options_off(be):
     """No soft cap, bias, sink, gate or window: plain causal attention."""
     spec = AttnSpec(heads=4, kv_heads=2, dim=64, vdim=64, scale=0.125)

@@ -18,6 +18,8 @@
 //              machinery (64 candidates per step, skip test first).
 // Small indexes split each row tile's dimensions over S waves (S = 4 below 64k rows) so that
 // a 10k-row index still spreads over ~160 blocks; the partial sums are added in slice order.
+#include <chrono>
+#include <climits>
 #include "common.h"
 #include <float.h>
 using namespace ragk;
@@ -608,9 +610,10 @@ __global__ __launch_bounds__(MW * 64) void topk_lists_merge_kernel(const float* 
     if (w < h) wave_merge64(bv, bi, mv[w + h][lane], mi[w + h][lane], lane);
     __syncthreads();
   }
-  if (w == 0 && lane < k) {
-    out_d[(size_t)qi * k + lane] = bv;
-    out_i[(size_t)qi * k + lane] = bi;  // int64 ids: the caller's final type, no widening launch
+  if (w == 0 && lane < k) {  // (through to memory: a host may be watching the results arrive)
+    __hip_atomic_store(out_d + (size_t)qi * k + lane, bv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    // int64 ids: the caller's final type, no widening launch
+    __hip_atomic_store(out_i + (size_t)qi * k + lane, (long long)bi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -935,6 +938,58 @@ RAGK_API int ragk_kmeans_assign(const float* X, int n, int d, const float* C, co
     hipLaunchKernelGGL(kmeans_assign_kernel<false>, dim3((n + KA_ROWS - 1) / KA_ROWS), dim3(256), lds, st, X, n, d, C,
                        cnorm, k, assign, dist, scores);
   return (int)hipGetLastError();
+}
+
+// Results watched in host memory. A search's merge stores them into pinned memory itself, and the host needs no more than those
+// stores: waiting for the stream instead adds the kernel's end, its signal and the runtime's way back, 5.5 us behind a result that
+// has arrived (a kernel of one store: seen after 5.4 us, hipStreamSynchronize back after 11.0). Every entry is marked beforehand
+// with an id and a distance that no search gives, and taken once neither is left, so the order of the stores does not matter.
+namespace {
+constexpr long long PENDING_ID = LLONG_MIN;
+constexpr unsigned PENDING_D = 0xffc0deadu;  // a NaN that no arithmetic gives (should one be handed through: the stream is waited for)
+constexpr auto WATCH_LIMIT = std::chrono::milliseconds(5);  // then the stream is waited for, which also reports what went wrong
+}  // namespace
+
+// block: pinned, n int64 ids and behind them n distances. Ahead of the search's launches; refused while the stream is captured (a
+// graph's results would not be there to be watched).
+RAGK_API int ragk_search_arm(void* block, int n, hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  const hipError_t e = hipStreamIsCapturing(st, &cs);
+  if (e != hipSuccess) return (int)e;
+  if (cs != hipStreamCaptureStatusNone) return (int)hipErrorStreamCaptureUnsupported;
+  long long* ids = (long long*)block;
+  unsigned* d = (unsigned*)(ids + n);
+  for (int i = 0; i < n; ++i) {
+    __atomic_store_n(ids + i, PENDING_ID, __ATOMIC_RELAXED);
+    __atomic_store_n(d + i, PENDING_D, __ATOMIC_RELAXED);
+  }
+  __atomic_thread_fence(__ATOMIC_SEQ_CST);
+  return 0;
+}
+
+// Behind the launches: the n results into host memory as they arrive.
+RAGK_API int ragk_search_collect(const void* block, int n, long long* out_i, float* out_d, hipStream_t st) {
+  const long long* ids = (const long long*)block;
+  const unsigned* d = (const unsigned*)(ids + n);
+  const auto until = std::chrono::steady_clock::now() + WATCH_LIMIT;
+  bool watch = true;
+  for (int i = 0; i < n; ++i) {
+    long long id;
+    unsigned v;
+    for (int spin = 0;; ++spin) {
+      id = __atomic_load_n(ids + i, __ATOMIC_RELAXED);
+      v = __atomic_load_n(d + i, __ATOMIC_RELAXED);
+      if (!watch || (id != PENDING_ID && v != PENDING_D)) break;
+      if ((spin & 63) == 63 && std::chrono::steady_clock::now() > until) {
+        const hipError_t e = hipStreamSynchronize(st);
+        if (e != hipSuccess) return (int)e;
+        watch = false;
+      }
+    }
+    out_i[i] = id;
+    __builtin_memcpy(out_d + i, &v, 4);
+  }
+  return 0;
 }
 
 // Returns when everything enqueued on the stream is done.

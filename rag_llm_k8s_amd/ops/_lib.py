@@ -74,6 +74,8 @@ _SIGS = {
     "ragk_pool_l2norm": [P, I, P, P, I, I, I, I, S],
     "ragk_put_ints": [P, I, P, S],
     "ragk_stream_wait": [S],
+    "ragk_search_arm": [P, I, S],
+    "ragk_search_collect": [P, I, P, P, S],
     "ragk_encoder_call_bytes": [],
     "ragk_encoder_forward": [P, S],
     "ragk_silu_mul": [P, I, P, I, I, I, S],

@@ -1647,9 +1647,9 @@ _search_ws = {}
 _search_lock = threading.Lock()
 
 
-# Results in host memory up to this many are stored there by the merge itself (pinned, 12 bytes each) and only waited for, instead
-# of copied behind it: one query of 10000 x 384 40.4 -> 38.9 us, 256 queries of the k = 10 nearest 119 -> 109, 1000 of 1000 rows
-# 87 -> 78.
+# Results in host memory up to this many are stored there by the merge itself (pinned, 12 bytes each) and watched arriving
+# (search.hip ragk_search_collect), instead of copied behind it: one query of 10000 x 384 40.4 us copied, 38.0 stored and the stream
+# waited for, 26 watched; 5 of 2000 x 384 47 -> 37, 256 of 10000 x 384 110 -> 102, 32 of 500000 x 1024 411 -> 402.
 SEARCH_STORE = 16384
 
 
@@ -1661,40 +1661,52 @@ def search_block():
     return torch.empty(3 * SEARCH_STORE, dtype=torch.int32, pin_memory=True)
 
 
-def _search_out(nq, k, device, host):
-    n = nq * k
-    if host and 0 < n <= SEARCH_STORE:
-        return search_block()
-    return torch.empty(3 * n, dtype=torch.int32, device=device)
-
-
-def _search_wait(out):
-    """Behind the launches, whatever became of them: a pinned buffer goes back to its pool once nothing can write to it."""
-    if not out.is_cuda:
-        check(_lib.lib().ragk_stream_wait(stream_ptr()), "ragk_stream_wait")
+def _search_to_host(nq, k, launch):
+    """(D, I) of a search that launch(ids' address, distances' address) enqueues, in pageable memory of their own."""
+    L, n, block = _lib.lib(), nq * k, search_block()
+    at, st = block.data_ptr(), stream_ptr()
+    check(L.ragk_search_arm(at, n, st), "ragk_search_arm")
+    try:
+        launch(at, at + 8 * n)
+    except BaseException:
+        L.ragk_stream_wait(st)  # the block goes back to its pool once nothing can write to it
+        raise
+    D, I = torch.empty(nq, k), torch.empty(nq, k, dtype=torch.int64)  # (while the search runs)
+    check(L.ragk_search_collect(at, n, I.data_ptr(), D.data_ptr(), st), "ragk_search_collect")
+    return D, I
 
 
 def _search_views(buf, nq, k, host):
-    """(D fp32 [nq, k], I int64 [nq, k]) as views of the ONE allocation a search writes (_search_out), int64 ids first; host: of a
-    copy in pageable memory (a copy of each result waits for the device twice; pinned pages go back to their pool)."""
-    if host and buf.is_cuda:
+    """(D fp32 [nq, k], I int64 [nq, k]) as views of the ONE allocation a search writes, int64 ids first; host: of a copy in
+    pageable memory (a copy of each result waits for the device twice)."""
+    if host:
         buf = buf.cpu()
-    elif host:
-        buf = buf.as_strided((3 * nq * k,), (1,)).clone()
     return (buf.as_strided((nq, k), (k, 1), 2 * nq * k).view(torch.float32),
             buf.as_strided((nq, 2 * k), (2 * k, 1)).view(torch.int64))
 
 
+def _search(nq, k, device, host, launch):
+    """Results of launch(ids' address, distances' address), on the device or (host) in host memory."""
+    n = nq * k
+    if host and 0 < n <= SEARCH_STORE:
+        return _search_to_host(nq, k, launch)
+    out = torch.empty(3 * n, dtype=torch.int32, device=device)
+    if n:
+        launch(out.data_ptr(), out.data_ptr() + 8 * n)
+    return _search_views(out, nq, k, host)
+
+
 def _search_partials(n_entries, device):
-    """Per-(device, stream) grow-only partial-list workspace (fp32 distances + int32 ids). Callers hold
+    """Addresses of the partial lists (fp32 distances, int32 ids) in a grow-only workspace of this device and stream. Callers hold
     _search_lock from here until both kernels of the search are enqueued, so two searches on one stream
     never interleave their scan / merge pair over the same buffer."""
-    key = (str(device), stream_ptr())
+    key = (device.index, stream_ptr())
     ws = _search_ws.get(key)
     if ws is None or ws.numel() < 2 * n_entries:
         ws = torch.empty(max(2 * n_entries, 1 << 16), dtype=torch.int32, device=device)
         _search_ws[key] = ws
-    return ws[:n_entries].view(torch.float32), ws[n_entries:2 * n_entries]
+    at = ws.data_ptr()
+    return at, at + 4 * n_entries
 
 
 def l2_search(xt, cap, n, q, k, row_begin=0, ids_map=None, host=False):
@@ -1702,8 +1714,8 @@ def l2_search(xt, cap, n, q, k, row_begin=0, ids_map=None, host=False):
     (csrc/kernels/search.hip: l2_scan with wave-resident running top lists + one list merge; batches
     of >= 16 queries with k <= 8 on the fp32-MFMA distance GEMM, faiss' BLAS form).
     Returns (D fp32 [nq,k], I int64 [nq,k]) with faiss padding semantics (-1, FLT_MAX), on the device or (host) in host memory.
-    Host cost per call: one output block from a pool, two ctypes calls (the partial lists live in a cached
-    workspace) and, for results in host memory, a wait and a copy of them."""
+    Host cost per call: one output block, two ctypes calls (the partial lists live in a cached
+    workspace) and, for results in host memory, the marks ahead of them and the watch for them."""
     _req(xt.is_cuda and xt.dtype == torch.float32 and xt.is_contiguous() and xt.dim() == 2, "xt fp32 [d, cap]")
     _req(q.is_cuda and q.dtype == torch.float32 and q.is_contiguous() and q.dim() == 2, "q fp32 [nq, d]")
     d = xt.shape[0]
@@ -1713,19 +1725,15 @@ def l2_search(xt, cap, n, q, k, row_begin=0, ids_map=None, host=False):
     _req(xt.shape[1] == cap and 0 <= row_begin <= max(row_begin, n) <= cap, "rows within the store")
     _req(ids_map is None or (ids_map.dtype == torch.int32 and ids_map.is_cuda and ids_map.numel() >= n), "ids_map")
     L = _lib.lib()
-    out = _search_out(nq, k, q.device, host)
-    if nq == 0:
-        return _search_views(out, nq, k, host)
-    G = L.ragk_l2_search_groups(row_begin, max(n, row_begin), nq, k, d)
-    try:
+
+    def launch(ids, dist):
+        G = L.ragk_l2_search_groups(row_begin, max(n, row_begin), nq, k, d)
         with _search_lock:
             pd, pi = _search_partials(nq * G * k, q.device)
-            check(L.ragk_l2_search(xt.data_ptr(), cap, d, row_begin, max(n, row_begin), q.data_ptr(), nq, k,
-                                   ptr(ids_map), pd.data_ptr(), pi.data_ptr(), out.data_ptr() + 8 * nq * k, out.data_ptr(),
-                                   stream_ptr()), "ragk_l2_search")
-    finally:
-        _search_wait(out)
-    return _search_views(out, nq, k, host)
+            check(L.ragk_l2_search(xt.data_ptr(), cap, d, row_begin, max(n, row_begin), q.data_ptr(), nq, k, ptr(ids_map), pd, pi,
+                                   dist, ids, stream_ptr()), "ragk_l2_search")
+
+    return _search(nq, k, q.device, host, launch)
 
 
 def ivf_search(xt, cap, q, probes, offsets, ids_map, k, max_list=None, ends=None, host=False):
@@ -1740,19 +1748,15 @@ def ivf_search(xt, cap, q, probes, offsets, ids_map, k, max_list=None, ends=None
     d = xt.shape[0]
     nq, nprobe = probes.shape
     _req(1 <= k <= 64 and d <= 2048 and nprobe >= 1, "k <= 64, d <= 2048")
-    out = _search_out(nq, k, q.device, host)
-    if nq == 0:
-        return _search_views(out, nq, k, host)
-    try:
+
+    def launch(ids, dist):
         with _search_lock:
             pd, pi = _search_partials(nq * nprobe * k, q.device)
             check(_lib.lib().ragk_ivf_search(xt.data_ptr(), cap, d, q.data_ptr(), nq, probes.data_ptr(), nprobe,
-                                             offsets.data_ptr(), ptr(ends), ids_map.data_ptr(), k, pd.data_ptr(),
-                                             pi.data_ptr(), out.data_ptr() + 8 * nq * k, out.data_ptr(), stream_ptr()),
-                  "ragk_ivf_search")
-    finally:
-        _search_wait(out)
-    return _search_views(out, nq, k, host)
+                                             offsets.data_ptr(), ptr(ends), ids_map.data_ptr(), k, pd, pi, dist, ids,
+                                             stream_ptr()), "ragk_ivf_search")
+
+    return _search(nq, k, q.device, host, launch)
 
 
 def kmeans_assign(x, c, cnorm=None, scores=None):

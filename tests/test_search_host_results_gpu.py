@@ -34,3 +34,53 @@ def test_searches_allocate_no_host_memory(native):
         for index in (flat, ivf):
             index.search(x[:nq], k)
     assert torch.cuda.host_memory_stats()["num_host_alloc"] == made
+
+
+def test_results_later_than_the_watch(native):
+    """A stream that is busy for longer than results are watched for: the stream is waited for instead."""
+    g = torch.Generator(device=DEV).manual_seed(2)
+    xt, q = torch.randn(32, 512, device=DEV, generator=g), torch.randn(5, 32, device=DEV, generator=g)
+    want = native.l2_search(xt, 512, 500, q, 3)
+    torch.cuda._sleep(60_000_000)  # some 25 ms
+    dist, ids = native.l2_search(xt, 512, 500, q, 3, host=True)
+    assert torch.equal(dist, want[0].cpu()) and torch.equal(ids, want[1].cpu())
+
+
+def test_searches_beside_each_other(native):
+    """Threads with streams of their own, and two on one stream: each gets its own query's results."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    g = torch.Generator(device=DEV).manual_seed(3)
+    xt, q = torch.randn(32, 4096, device=DEV, generator=g), torch.randn(64, 32, device=DEV, generator=g)
+    want = [[t.cpu() for t in native.l2_search(xt, 4096, 4000, q[j:j + 1], 4)] for j in range(64)]
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+
+    def run(t):
+        with torch.cuda.stream(streams[t % 3]):
+            for j in range(t, 64, 4):
+                dist, ids = native.l2_search(xt, 4096, 4000, q[j:j + 1], 4, host=True)
+                if not (torch.equal(dist, want[j][0]) and torch.equal(ids, want[j][1])):
+                    return j
+        return None
+
+    with ThreadPoolExecutor(4) as ex:
+        assert list(ex.map(run, range(4))) == [None] * 4
+
+
+def test_host_results_are_refused_under_capture(native):
+    xt, q = torch.randn(32, 512, device=DEV), torch.randn(1, 32, device=DEV)
+    native.l2_search(xt, 512, 500, q, 3, host=True)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        native.l2_search(xt, 512, 500, q, 3, host=True)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            with pytest.raises(RuntimeError):
+                native.l2_search(xt, 512, 500, q, 3, host=True)
+            got = native.l2_search(xt, 512, 500, q, 3)
+        graph.replay()
+        want = native.l2_search(xt, 512, 500, q, 3)
+    s.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

@@ -11,89 +11,98 @@
 // rows' work in each of 24 to 256 blocks costs reads from L2 (21 KB a block for 14 fp32 rows of 384) and 0.6 us, the launch it
 // saves 2.4 to 4. Sums of a product, its bias and its residual reach the norm behind it in fp32; block 0 writes the norm's rows
 // out, as the residual of the product after next.
-// Six layers of 384 columns, 14 rows: 220 -> 111 us a call, 25 launches of 4.4 instead of 44 (with eight waves a block, two rows a
-// wave, 119); 24 layers of 1024, 14 rows: 752 -> 686 (726). What is left of a launch is its start, one trip to memory for the rows
-// and one through LDS for the sum (a down projection alone, without rows to make, takes as long as the others). Past 16384 values
-// of rows the repeated work costs more than it saves (ops/native.py encoder_few_ok).
+// Six layers of 384 columns, 14 rows: 220 us a call in seven launches a layer, 111 in these, 108.7 of it the chain on the device and
+// 88 the host's launches beside 31 of checks (119 a call where the host is not ahead). With the rows' loads in front of the weights,
+// column groups known when compiling and 64 bytes of arguments 101 and 68; 30 rows 142 -> 135; 24 layers of 1024, 14 rows 691 ->
+// 630. A launch on the device is 1.4 us behind the one before, 1.3 to 2 for the rows' (or the down projection's operands') trip to
+// memory and 1 through LDS for the sum. Past 16384 values of rows the repeated work costs more than it saves (ops/native.py
+// encoder_few_ok).
 #include "attn_tiles.h"
 #include "encoder.h"
+#include <type_traits>
 using namespace ragk;
 
 namespace {
 
 constexpr int FEW_W = 16;  // waves
 
-enum { ROWS, EMBED, NORM, ATTEND };
+enum FewPro : int { ROWS, EMBED, NORM, ATTEND };  // (named: it is part of the kernels' names, which host and device have to agree on)
 
+// 64 bytes: the host pays for a launch by the lines of its arguments (3.3 us for one, 3.8 from two on; one struct for all launches
+// had 248 bytes), and 25 of them are what a call of six layers is on its side.
 struct FewArgs {
   const void* x;          // ROWS: bf16 [T][K]; NORM: fp32 [T][K]; ATTEND: bf16 qkv [T][3 K]
-  const bf16_t *g, *b;    // EMBED, NORM: gain and shift
-  bf16_t* h;              // ... and where the rows go (null: nowhere)
-  const bf16_t *word, *places, *type;  // EMBED
-  const int* ids_dev;     // token ids on the device, or (null) by value
+  const bf16_t *w, *bias;  // [N][K], [N]
+  void* out;              // ROWS and ATTEND: fp32 [T][N], else bf16
+  const bf16_t *p, *q;    // ROWS and ATTEND: residual [T][N]; EMBED, NORM: gain and shift
+  bf16_t* h;              // EMBED, NORM: the rows for the residual of the product after next
+  unsigned sizes;         // T, K / 128, N / 16 in 6, 10 and 16 bits
+  float f;                // ATTEND: scale in log2 units; EMBED, NORM: eps
+  __host__ __device__ int T() const { return sizes & 63; }
+  __host__ __device__ int K() const { return (sizes >> 6 & 1023) * 128; }
+  __host__ __device__ int N() const { return (sizes >> 16) * 16; }
+};
+static_assert(sizeof(FewArgs) == 64, "one line of arguments");
+struct EmbedArgs : FewArgs {
+  const bf16_t *word, *places, *type;
+  const int* ids_dev;  // token ids on the device, or (null) by value
   int ids[FEW_T];
   int first_pos;
-  float scale_log2;       // ATTEND
-  const bf16_t *w, *bias, *resid;  // [N][K], [N], ROWS and ATTEND: [T][N]
-  void* out;              // ROWS and ATTEND: fp32 [T][N], else bf16
-  int T, N, K;
-  float eps;
 };
 
-// One row in a wave: lane l holds columns 2 l + 128 j and the one after. norm.hip's formula and order of roundings.
-__device__ __forceinline__ void few_norm(float (&v)[16], int nj, int K, float eps, const unsigned (&gr)[8], const unsigned (&br)[8],
-                                         unsigned (&o)[8]) {
+// One row in a wave: lane l holds columns 2 l + 128 j and the one after, j < NJ = K / 128 (known when compiling: behind a branch a
+// column group each, the first one's load was waited for before the others went out). norm.hip's formula and order of roundings.
+template <int NJ>
+__device__ __forceinline__ void few_norm(float (&v)[2 * NJ], float eps, const unsigned (&gr)[NJ], const unsigned (&br)[NJ],
+                                         unsigned (&o)[NJ]) {
+  constexpr int K = 128 * NJ;
   float s = 0.f, sq = 0.f;
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
-    if (j < nj) s += v[2 * j] + v[2 * j + 1];
+  for (int j = 0; j < NJ; ++j) s += v[2 * j] + v[2 * j + 1];
   const float mean = wave_sum(s) / (float)K;
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
-    if (j < nj) {
-      const float d0 = v[2 * j] - mean, d1 = v[2 * j + 1] - mean;
-      sq += d0 * d0 + d1 * d1;
-    }
+  for (int j = 0; j < NJ; ++j) {
+    const float d0 = v[2 * j] - mean, d1 = v[2 * j + 1] - mean;
+    sq += d0 * d0 + d1 * d1;
+  }
   const float inv = rsqrtf(wave_sum(sq) / (float)K + eps);
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
-    if (j < nj)
-      o[j] = pk2bf((v[2 * j] - mean) * inv * __uint_as_float(gr[j] << 16) + __uint_as_float(br[j] << 16),
-                   (v[2 * j + 1] - mean) * inv * __uint_as_float(gr[j] & 0xffff0000u) + __uint_as_float(br[j] & 0xffff0000u));
+  for (int j = 0; j < NJ; ++j)
+    o[j] = pk2bf((v[2 * j] - mean) * inv * __uint_as_float(gr[j] << 16) + __uint_as_float(br[j] << 16),
+                 (v[2 * j + 1] - mean) * inv * __uint_as_float(gr[j] & 0xffff0000u) + __uint_as_float(br[j] & 0xffff0000u));
 }
 
-__device__ __forceinline__ void few_pairs(const bf16_t* p, int lane, int nj, unsigned (&r)[8]) {
+template <int NJ>
+__device__ __forceinline__ void few_pairs(const bf16_t* p, int lane, unsigned (&r)[NJ]) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
-    if (j < nj) r[j] = *reinterpret_cast<const unsigned*>(p + 2 * lane + 128 * j);
+  for (int j = 0; j < NJ; ++j) r[j] = *reinterpret_cast<const unsigned*>(p + 2 * lane + 128 * j);
 }
 
-template <int PRO>
-__device__ __forceinline__ void few_row(const FewArgs& a, int row, int lane, int nj, float (&v)[16]) {
-  if constexpr (PRO == NORM) {
-    const float2* p = reinterpret_cast<const float2*>(reinterpret_cast<const float*>(a.x) + (size_t)row * a.K) + lane;
+template <int NJ>
+__device__ __forceinline__ void few_row(const float* x, int row, int lane, float (&v)[2 * NJ]) {
+  const float2* p = reinterpret_cast<const float2*>(x + (size_t)row * 128 * NJ) + lane;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j < nj) {
-        const float2 t = p[64 * j];
-        v[2 * j] = t.x;
-        v[2 * j + 1] = t.y;
-      }
-  } else {
-    unsigned wv[8], pv[8], tv[8];
-    few_pairs(a.word + (size_t)(a.ids_dev ? a.ids_dev[row] : a.ids[row]) * a.K, lane, nj, wv);
-    few_pairs(a.places + (size_t)(a.first_pos + row) * a.K, lane, nj, pv);
-    if (a.type) few_pairs(a.type, lane, nj, tv);
+  for (int j = 0; j < NJ; ++j) {
+    const float2 t = p[64 * j];
+    v[2 * j] = t.x;
+    v[2 * j + 1] = t.y;
+  }
+}
+template <int NJ>
+__device__ __forceinline__ void few_row(const EmbedArgs& a, int row, int lane, float (&v)[2 * NJ]) {
+  constexpr int K = 128 * NJ;
+  unsigned wv[NJ], pv[NJ], tv[NJ];
+  few_pairs(a.word + (size_t)(a.ids_dev ? a.ids_dev[row] : a.ids[row]) * K, lane, wv);
+  few_pairs(a.places + (size_t)(a.first_pos + row) * K, lane, pv);
+  if (a.type) few_pairs(a.type, lane, tv);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j < nj) {
-        v[2 * j] = __uint_as_float(wv[j] << 16) + __uint_as_float(pv[j] << 16);
-        v[2 * j + 1] = __uint_as_float(wv[j] & 0xffff0000u) + __uint_as_float(pv[j] & 0xffff0000u);
-        if (a.type) {
-          v[2 * j] += __uint_as_float(tv[j] << 16);
-          v[2 * j + 1] += __uint_as_float(tv[j] & 0xffff0000u);
-        }
-      }
+  for (int j = 0; j < NJ; ++j) {
+    v[2 * j] = __uint_as_float(wv[j] << 16) + __uint_as_float(pv[j] << 16);
+    v[2 * j + 1] = __uint_as_float(wv[j] & 0xffff0000u) + __uint_as_float(pv[j] & 0xffff0000u);
+    if (a.type) {
+      v[2 * j] += __uint_as_float(tv[j] << 16);
+      v[2 * j + 1] += __uint_as_float(tv[j] & 0xffff0000u);
+    }
   }
 }
 
@@ -162,71 +171,80 @@ struct FewHead {
   }
 };
 
-// MT = 16-row tiles; NP = K-steps of 32 that a wave requests at once (it takes every 16th). D: head size (ATTEND).
+// MT = 16-row tiles; NP = K-steps of 32 that a wave requests at once (it takes every 16th). D: head size (ATTEND), K / 128 (EMBED, NORM).
 template <int PRO, int EPI, int MT, int NP, int D>
-__global__ __launch_bounds__(FEW_W * 64) void few_kernel(FewArgs a) {
+__global__ __launch_bounds__(FEW_W * 64) void few_kernel(std::conditional_t<PRO == EMBED, EmbedArgs, FewArgs> a) {
+  const int T = a.T(), K = PRO == EMBED || PRO == NORM ? 128 * D : a.K(), N = a.N();
   extern __shared__ __attribute__((aligned(16))) char smem[];
   f32x4(*red)[MT][64] = reinterpret_cast<f32x4(*)[MT][64]>(smem);  // [wave][tile][lane]
   char* rows = smem + FEW_W * MT * 1024;
-  const int rowb = a.K * 2 + 16;  // rows 16 bytes apart in the banks
+  const int rowb = K * 2 + 16;  // rows 16 bytes apart in the banks
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int fr = lane & 15, fh = lane >> 4, n0 = blockIdx.x * 16, nk = a.K / 32;
+  const int fr = lane & 15, fh = lane >> 4, n0 = blockIdx.x * 16, nk = K / 32;
 
-  // ---- what does not depend on the rows
-  const bf16_t* wp = a.w + (size_t)(n0 + fr) * a.K + 8 * fh;
+  // ---- requests, the rows ahead of what waits for them: loads come back in order, and with the weights in front a row waited for
+  // 20 KB of them (all indices clamped, so that no request stands behind a branch, where the compiler would wait for all)
+  constexpr bool MAKES = PRO == EMBED || PRO == NORM;
+  constexpr int NJ = MAKES ? D : 1;
+  float v[MT][2 * NJ];
+  unsigned gr[NJ], br[NJ];
+  FewHead<MT, PRO == ATTEND ? D : 32> head;
+  if constexpr (MAKES) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int row = min(wid + FEW_W * i, T - 1);
+      if constexpr (PRO == EMBED) few_row<NJ>(a, row, lane, v[i]);
+      else few_row<NJ>(reinterpret_cast<const float*>(a.x), row, lane, v[i]);
+    }
+    few_pairs(a.p, lane, gr);
+    few_pairs(a.q, lane, br);
+  }
+  if constexpr (PRO == ATTEND) head.load(reinterpret_cast<const bf16_t*>(a.x), K, T, min(wid, K / D - 1), fr, fh);
+  __builtin_amdgcn_sched_barrier(0);
+  const bf16_t* wp = a.w + (size_t)(n0 + fr) * K + 8 * fh;
   bf16x8 wf[NP], xf[MT][NP];
   auto request = [&](int base) {
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const int s = base + wid + FEW_W * i;
-      if (s < nk) wf[i] = *reinterpret_cast<const bf16x8*>(wp + 32 * s);
+      const int s = min(base + wid + FEW_W * i, nk - 1);
+      wf[i] = *reinterpret_cast<const bf16x8*>(wp + 32 * s);
       if constexpr (PRO == ROWS) {
 #pragma unroll
         for (int t = 0; t < MT; ++t)
-          if (s < nk)
-            xf[t][i] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const bf16_t*>(a.x) +
-                                                        (size_t)min(16 * t + fr, a.T - 1) * a.K + 8 * fh + 32 * s);
+          xf[t][i] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const bf16_t*>(a.x) + (size_t)min(16 * t + fr, T - 1) * K +
+                                                      8 * fh + 32 * s);
       }
     }
   };
   request(0);
   const int orow = threadIdx.x >> 4, ocol = n0 + (threadIdx.x & 15);  // this thread's output
-  const bool mine = orow < a.T && orow < 16 * MT;
-  float add = bf2f(a.bias[ocol]);
-  if constexpr (EPI == EPI_BIAS_RESID) {
-    if (mine) add += bf2f(a.resid[(size_t)orow * a.N + ocol]);
-  }
+  const bool mine = orow < T && orow < 16 * MT;
+  const bf16_t bias = a.bias[ocol];
+  bf16_t resid = 0;
+  if constexpr (EPI == EPI_BIAS_RESID) resid = a.p[(size_t)min(orow, T - 1) * N + ocol];
+  __builtin_amdgcn_sched_barrier(0);
 
   // ---- the rows
-  if constexpr (PRO == EMBED || PRO == NORM) {
-    const int nj = a.K / 128;
-    unsigned gr[8], br[8];
-    few_pairs(a.g, lane, nj, gr);
-    few_pairs(a.b, lane, nj, br);
+  if constexpr (MAKES) {
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       const int row = wid + FEW_W * i;
-      if (row < a.T) {
-        float v[16];
-        unsigned o[8];
-        few_row<PRO>(a, row, lane, nj, v);
-        few_norm(v, nj, a.K, a.eps, gr, br, o);
+      unsigned o[NJ];
+      few_norm(v[i], a.f, gr, br, o);
+      if (row < T) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (j < nj) {
-            *reinterpret_cast<unsigned*>(rows + row * rowb + 4 * lane + 256 * j) = o[j];
-            if (blockIdx.x == 0) *reinterpret_cast<unsigned*>(a.h + (size_t)row * a.K + 2 * lane + 128 * j) = o[j];
-          }
+        for (int j = 0; j < NJ; ++j) *reinterpret_cast<unsigned*>(rows + row * rowb + 4 * lane + 256 * j) = o[j];
+        if (blockIdx.x == 0)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) *reinterpret_cast<unsigned*>(a.h + (size_t)row * K + 2 * lane + 128 * j) = o[j];
       }
     }
   }
   if constexpr (PRO == ATTEND) {
-    const bf16_t* qkv = reinterpret_cast<const bf16_t*>(a.x);
-    const int heads = a.K / D;
+    const int heads = K / D;
     for (int hd = wid; hd < heads; hd += FEW_W) {
-      FewHead<MT, D> head;
-      head.load(qkv, a.K, a.T, hd, fr, fh);
-      head.attend(rows, rowb, a.T, hd, fr, fh, a.scale_log2);
+      if (hd != wid) head.load(reinterpret_cast<const bf16_t*>(a.x), K, T, hd, fr, fh);
+      head.attend(rows, rowb, T, hd, fr, fh, a.f);
     }
   }
   if constexpr (PRO != ROWS) __syncthreads();
@@ -258,81 +276,95 @@ __global__ __launch_bounds__(FEW_W * 64) void few_kernel(FewArgs a) {
     float v = 0.f;
 #pragma unroll
     for (int w = 0; w < FEW_W; ++w) v += red[w][t][ln][r];
-    v += add;
+    v += EPI == EPI_BIAS_RESID ? bf2f(bias) + bf2f(resid) : bf2f(bias);
     if constexpr (EPI == EPI_BIAS_GELU) v = gelu_erf(v);
-    if constexpr (EPI == EPI_BIAS_RESID) reinterpret_cast<float*>(a.out)[(size_t)orow * a.N + ocol] = v;
-    else reinterpret_cast<bf16_t*>(a.out)[(size_t)orow * a.N + ocol] = f2bf(v);
+    if constexpr (EPI == EPI_BIAS_RESID) reinterpret_cast<float*>(a.out)[(size_t)orow * N + ocol] = v;
+    else reinterpret_cast<bf16_t*>(a.out)[(size_t)orow * N + ocol] = f2bf(v);
   }
 }
 
 template <int PRO, int EPI, int MT, int NP, int D>
-int few_launch(const FewArgs& a, hipStream_t st) {
-  const int lds = FEW_W * MT * 1024 + (PRO == ROWS ? 0 : 16 * MT * (a.K * 2 + 16));
+int few_launch(const std::conditional_t<PRO == EMBED, EmbedArgs, FewArgs>& a, hipStream_t st) {
+  const int lds = FEW_W * MT * 1024 + (PRO == ROWS ? 0 : 16 * MT * (a.K() * 2 + 16));
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&few_kernel<PRO, EPI, MT, NP, D>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize,
                                                      FEW_W * MT * 1024 + (PRO == ROWS ? 0 : 16 * MT * (FEW_H * 2 + 16)));
   if (attr != hipSuccess) return (int)attr;
-  hipLaunchKernelGGL((few_kernel<PRO, EPI, MT, NP, D>), dim3(a.N / 16), dim3(FEW_W * 64), lds, st, a);
+  hipLaunchKernelGGL((few_kernel<PRO, EPI, MT, NP, D>), dim3(a.N() / 16), dim3(FEW_W * 64), lds, st, a);
   return (int)hipGetLastError();
 }
 
-template <int PRO, int EPI, int D = 32>
-int few_dispatch(const FewArgs& a, hipStream_t st) {
-  if (a.T < 1 || a.T > FEW_T || a.K % 128 || a.K <= 0 || a.N % 16 || (PRO != ROWS && a.K > FEW_H)) return (int)hipErrorInvalidValue;
-#define RAGK_FEW(NP) return a.T <= 16 ? few_launch<PRO, EPI, 1, NP, D>(a, st) : few_launch<PRO, EPI, 2, NP, D>(a, st)
-  if (a.K <= 512) RAGK_FEW(1);
-  if constexpr (PRO != ROWS) RAGK_FEW(2);
-  if (a.K <= 1024) RAGK_FEW(2);
-  if (a.K <= 2048) RAGK_FEW(4);
-  RAGK_FEW(8);
-#undef RAGK_FEW
+template <int PRO, int EPI, int NP, int D>
+int few_rows(const std::conditional_t<PRO == EMBED, EmbedArgs, FewArgs>& a, hipStream_t st) {
+  return a.T() <= 16 ? few_launch<PRO, EPI, 1, NP, D>(a, st) : few_launch<PRO, EPI, 2, NP, D>(a, st);
+}
+// EMBED, NORM: rows of K = 128 NJ columns
+template <int PRO, int EPI, int NJ = FEW_H / 128>
+int few_made(const std::conditional_t<PRO == EMBED, EmbedArgs, FewArgs>& a, hipStream_t st) {
+  if (a.K() == 128 * NJ) return few_rows<PRO, EPI, NJ <= 4 ? 1 : 2, NJ>(a, st);
+  if constexpr (NJ > 1) return few_made<PRO, EPI, NJ - 1>(a, st);
+  else return (int)hipErrorInvalidValue;
+}
+template <int EPI, int D>
+int few_attend(const FewArgs& a, hipStream_t st) {
+  if (a.K() > FEW_H) return (int)hipErrorInvalidValue;
+  return a.K() <= 512 ? few_rows<ATTEND, EPI, 1, D>(a, st) : few_rows<ATTEND, EPI, 2, D>(a, st);
+}
+template <int EPI>
+int few_plain(const FewArgs& a, hipStream_t st) {
+  return a.K() <= 512    ? few_rows<ROWS, EPI, 1, 1>(a, st)
+         : a.K() <= 1024 ? few_rows<ROWS, EPI, 2, 1>(a, st)
+         : a.K() <= 2048 ? few_rows<ROWS, EPI, 4, 1>(a, st)
+                       : few_rows<ROWS, EPI, 8, 1>(a, st);
 }
 
 constexpr int POOL_W = 8;
 // Norm of the rows, then the pooled row as encoder.hip has it (the norm's rows rounded to bf16). A wave takes every eighth row.
+template <int NJ>
 __global__ __launch_bounds__(POOL_W * 64) void few_pool_kernel(const float* __restrict__ y, const bf16_t* __restrict__ g,
-                                                              const bf16_t* __restrict__ b, float* out, int T, int H, float eps,
-                                                              int mode, int normalize) {
-  __shared__ float part[POOL_W][FEW_H];
+                                                              const bf16_t* __restrict__ b, float* out, int T, float eps, int mode,
+                                                              int normalize) {
+  constexpr int H = 128 * NJ;
+  __shared__ float part[POOL_W][H];
   __shared__ float red[POOL_W];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nj = H / 128;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int first = mode == 2 ? T - 1 : 0, last = mode == 1 ? T : first + 1;
-  unsigned gr[8], br[8];
-  few_pairs(g, lane, nj, gr);
-  few_pairs(b, lane, nj, br);
-  float acc[16];
+  unsigned gr[NJ], br[NJ];
+  few_pairs(g, lane, gr);
+  few_pairs(b, lane, br);
+  float acc[2 * NJ];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-  FewArgs a{};
-  a.x = y;
-  a.K = H;
-  for (int row = first + wid; row < last; row += POOL_W) {
-    float v[16];
-    unsigned o[8];
-    few_row<NORM>(a, row, lane, nj, v);
-    few_norm(v, nj, H, eps, gr, br, o);
+  for (int e = 0; e < 2 * NJ; ++e) acc[e] = 0.f;
+  constexpr int AT_ONCE = (FEW_T + POOL_W - 1) / POOL_W;  // a wave's rows, requested together
+  float v[AT_ONCE][2 * NJ];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j < nj) {
-        acc[2 * j] += __uint_as_float(o[j] << 16);
-        acc[2 * j + 1] += __uint_as_float(o[j] & 0xffff0000u);
-      }
+  for (int i = 0; i < AT_ONCE; ++i) few_row<NJ>(y, min(first + wid + POOL_W * i, last - 1), lane, v[i]);
+#pragma unroll
+  for (int i = 0; i < AT_ONCE; ++i) {
+    if (first + wid + POOL_W * i >= last) continue;
+    unsigned o[NJ];
+    few_norm(v[i], eps, gr, br, o);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      acc[2 * j] += __uint_as_float(o[j] << 16);
+      acc[2 * j + 1] += __uint_as_float(o[j] & 0xffff0000u);
+    }
   }
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
-    if (j < nj) *reinterpret_cast<float2*>(&part[wid][2 * lane + 128 * j]) = make_float2(acc[2 * j], acc[2 * j + 1]);
+  for (int j = 0; j < NJ; ++j) *reinterpret_cast<float2*>(&part[wid][2 * lane + 128 * j]) = make_float2(acc[2 * j], acc[2 * j + 1]);
   __syncthreads();
   const float inv = mode == 1 ? 1.f / (float)T : 1.f;
-  float v[FEW_H / (POOL_W * 64)], ss = 0.f;
+  constexpr int NC = (H + POOL_W * 64 - 1) / (POOL_W * 64);
+  float c[NC], ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < FEW_H / (POOL_W * 64); ++i) {
-    const int c = threadIdx.x + POOL_W * 64 * i;
-    v[i] = 0.f;
-    if (c < H) {
+  for (int i = 0; i < NC; ++i) {
+    const int col = threadIdx.x + POOL_W * 64 * i;
+    c[i] = 0.f;
+    if (col < H) {
 #pragma unroll
-      for (int w = 0; w < POOL_W; ++w) v[i] += part[w][c];
-      v[i] *= inv;
-      ss += v[i] * v[i];
+      for (int w = 0; w < POOL_W; ++w) c[i] += part[w][col];
+      c[i] *= inv;
+      ss += c[i] * c[i];
     }
   }
   float scale = 1.f;
@@ -341,10 +373,20 @@ __global__ __launch_bounds__(POOL_W * 64) void few_pool_kernel(const float* __re
     scale = 1.f / fmaxf(sqrtf(ss), 1e-12f);  // torch.nn.functional.normalize eps
   }
 #pragma unroll
-  for (int i = 0; i < FEW_H / (POOL_W * 64); ++i) {
-    const int c = threadIdx.x + POOL_W * 64 * i;
-    if (c < H) out[c] = v[i] * scale;
+  for (int i = 0; i < NC; ++i) {
+    const int col = threadIdx.x + POOL_W * 64 * i;
+    if (col < H) out[col] = c[i] * scale;
   }
+}
+
+template <int NJ = FEW_H / 128>
+int few_pool(const EncoderCall& c, const bf16_t* g, const bf16_t* b, hipStream_t st) {
+  if (c.H == 128 * NJ) {
+    hipLaunchKernelGGL(few_pool_kernel<NJ>, dim3(1), dim3(POOL_W * 64), 0, st, c.y, g, b, c.out, c.T, c.eps, c.pooling, c.normalize);
+    return (int)hipGetLastError();
+  }
+  if constexpr (NJ > 1) return few_pool<NJ - 1>(c, g, b, st);
+  else return (int)hipErrorInvalidValue;
 }
 
 }  // namespace
@@ -355,42 +397,39 @@ namespace ragk {
 int encoder_few_forward(const EncoderCall& c, hipStream_t st) {
   const int H = c.H, T = c.T, D = c.heads > 0 ? H / c.heads : 0;
   if (c.B != 1 || T < 1 || T > FEW_T || H > FEW_H || H % 128 || c.I % 128 || D * c.heads != H || (D != 32 && D != 64) ||
-      c.n_layers < 1 || (!c.ids && !c.ids_host))
+      c.n_layers < 1 || c.I < 128 || c.I >= 128 * 1024 || (!c.ids && !c.ids_host))
     return (int)hipErrorInvalidValue;
+  auto sizes = [&](int K, int N) { return (unsigned)T | (unsigned)(K / 128) << 6 | (unsigned)(N / 16) << 16; };
 #define RAGK_TRY(x) \
   if (const int rc = (x)) return rc
   for (int l = 0; l < c.n_layers; ++l) {
     const void* const* w = c.layers + 12 * l;
     auto b16 = [&](int i) { return (const bf16_t*)w[i]; };
-    FewArgs a{};
-    a.T = T, a.eps = c.eps, a.scale_log2 = 1.4426950408889634f / sqrtf((float)D);
+    const float scale = 1.4426950408889634f / sqrtf((float)D);
     // qkv
-    a.K = H, a.N = 3 * H, a.h = (bf16_t*)c.h, a.w = b16(0), a.bias = b16(1), a.out = c.qkv;
     if (l == 0) {
-      a.g = (const bf16_t*)c.ln_g, a.b = (const bf16_t*)c.ln_b;
+      EmbedArgs a{};
+      static_cast<FewArgs&>(a) = FewArgs{nullptr, b16(0), b16(1), c.qkv, (const bf16_t*)c.ln_g, (const bf16_t*)c.ln_b, (bf16_t*)c.h,
+                                         sizes(H, 3 * H), c.eps};
       a.word = (const bf16_t*)c.word, a.places = (const bf16_t*)c.pos_table, a.type = (const bf16_t*)c.type_row;
       a.ids_dev = c.ids, a.first_pos = c.first_pos;
       if (!c.ids) __builtin_memcpy(a.ids, c.ids_host, (size_t)T * 4);
-      RAGK_TRY((few_dispatch<EMBED, EPI_BIAS>(a, st)));
-    } else {
-      a.x = c.y, a.g = b16(-2), a.b = b16(-1);  // the norm that ends the layer before
-      RAGK_TRY((few_dispatch<NORM, EPI_BIAS>(a, st)));
+      RAGK_TRY((few_made<EMBED, EPI_BIAS>(a, st)));
+    } else {  // behind the norm that ends the layer before
+      const FewArgs a{c.y, b16(0), b16(1), c.qkv, b16(-2), b16(-1), (bf16_t*)c.h, sizes(H, 3 * H), c.eps};
+      RAGK_TRY((few_made<NORM, EPI_BIAS>(a, st)));
     }
     // attention and its projection
-    a.x = c.qkv, a.N = H, a.w = b16(2), a.bias = b16(3), a.resid = (const bf16_t*)c.h, a.out = c.y;
-    RAGK_TRY(D == 32 ? (few_dispatch<ATTEND, EPI_BIAS_RESID, 32>(a, st)) : (few_dispatch<ATTEND, EPI_BIAS_RESID, 64>(a, st)));
-    // up
-    a.x = c.y, a.g = b16(4), a.b = b16(5), a.N = c.I, a.w = b16(6), a.bias = b16(7), a.out = c.f;
-    RAGK_TRY((few_dispatch<NORM, EPI_BIAS_GELU>(a, st)));
-    // down
-    a.x = c.f, a.K = c.I, a.N = H, a.w = b16(8), a.bias = b16(9), a.out = c.y;
-    RAGK_TRY((few_dispatch<ROWS, EPI_BIAS_RESID>(a, st)));
+    const FewArgs out{c.qkv, b16(2), b16(3), c.y, (const bf16_t*)c.h, nullptr, nullptr, sizes(H, H), scale};
+    RAGK_TRY(D == 32 ? (few_attend<EPI_BIAS_RESID, 32>(out, st)) : (few_attend<EPI_BIAS_RESID, 64>(out, st)));
+    const FewArgs up{c.y, b16(6), b16(7), c.f, b16(4), b16(5), (bf16_t*)c.h, sizes(H, c.I), c.eps};
+    RAGK_TRY((few_made<NORM, EPI_BIAS_GELU>(up, st)));
+    const FewArgs down{c.f, b16(8), b16(9), c.y, (const bf16_t*)c.h, nullptr, nullptr, sizes(c.I, H), 0.f};
+    RAGK_TRY(few_plain<EPI_BIAS_RESID>(down, st));
   }
 #undef RAGK_TRY
   const void* const* w = c.layers + 12 * (c.n_layers - 1);
-  hipLaunchKernelGGL(few_pool_kernel, dim3(1), dim3(POOL_W * 64), 0, st, c.y, (const bf16_t*)w[10], (const bf16_t*)w[11], c.out, T, H,
-                     c.eps, c.pooling, c.normalize);
-  return (int)hipGetLastError();
+  return few_pool(c, (const bf16_t*)w[10], (const bf16_t*)w[11], st);
 }
 
 }  // namespace ragk

@@ -61,6 +61,13 @@ def test_short_sequence(native, monkeypatch, T, hidden, heads, inter, pooling, k
     assert err[0] < 0.01 and err[0] < 1.3 * err[1] + 1e-4, err
 
 
+# the widths between (a kernel for each), and as many columns of a down projection as the arguments can name
+@pytest.mark.parametrize("T", [3, 17])
+@pytest.mark.parametrize("hidden,heads,inter", [(256, 8, 256), (768, 12, 3072), (896, 14, 1152), (128, 2, 32768)])
+def test_every_width(native, monkeypatch, T, hidden, heads, inter):
+    test_short_sequence(native, monkeypatch, T, hidden, heads, inter, "mean", "bert")
+
+
 def test_no_layers(native):
     """Embeddings, their norm and the pooling only: the launches of a layer have nothing to begin with."""
     cfg = E.EncoderConfig(model_type="bert", vocab_size=500, hidden_size=128, num_hidden_layers=0, num_attention_heads=4,

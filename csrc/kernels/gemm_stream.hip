@@ -351,7 +351,10 @@ int g_stream_diag = 0;
 // 28672-row Llama gate/up grid (448 tiles) occupies all 256 CUs; 128 = one block per CU, 224 tiles.
 int g_stream_pair_rows = 64;
 
-inline int stream_rows(int epi) { return (epi_pair(epi) && g_stream_pair_rows == 64) ? 64 : WROWS; }
+// Everything else: bf16 weights, from 16384 rows, in 64-row tiles, so that two blocks share a CU and one's epilogue and short
+// last round run under the other's stream (18560 x 4096 at 8 / 64 rows: 128-row tiles and two slabs 55 / 75 us, now 37 / 46;
+// 32000 x 2048 32 / 37 -> 25 / 30); fp8 ones in 128-row tiles.
+inline int stream_rows(int epi, bool fp8) { return (epi_pair(epi) ? g_stream_pair_rows == 64 : !fp8) ? 64 : WROWS; }
 
 template <int MT, int EPI, bool F32, bool FP8>
 int launch_stream(const void* X, int ldx, const void* W, int ldw, const float* wscale, void* C, int ldc,
@@ -382,13 +385,14 @@ int launch_stream(const void* X, int ldx, const void* W, int ldw, const float* w
 #undef RAGK_ST_PAIR
     return (int)hipGetLastError();
   }
-  const dim3 grid((Nrows + WROWS - 1) / WROWS, S);
-  if (g_stream_nt && Nrows >= 65536)  // vocab-sized weights, read once per step: non-temporal
-    hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI, F32, FP8, true>), grid, dim3(ST_THREADS), 0, st, (const bf16_t*)X,
+  constexpr int R = FP8 ? WROWS : 64;
+  const dim3 grid((Nrows + R - 1) / R, S);
+  if (g_stream_nt && (!FP8 || Nrows >= 65536))  // weights of more than the caches hold, read once per step: non-temporal
+    hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI, F32, FP8, true, R>), grid, dim3(ST_THREADS), 0, st, (const bf16_t*)X,
                        ldx, W, ldw, wscale, C, ldc, (const bf16_t*)bias, (const bf16_t*)resid, ldr, M, N, K, S, ws, cnt);
   else
-    hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI, F32, FP8>), grid, dim3(ST_THREADS), 0, st, (const bf16_t*)X, ldx,
-                       W, ldw, wscale, C, ldc, (const bf16_t*)bias, (const bf16_t*)resid, ldr, M, N, K, S, ws, cnt);
+    hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI, F32, FP8, false, R>), grid, dim3(ST_THREADS), 0, st, (const bf16_t*)X,
+                       ldx, W, ldw, wscale, C, ldc, (const bf16_t*)bias, (const bf16_t*)resid, ldr, M, N, K, S, ws, cnt);
   return (int)hipGetLastError();
 }
 
@@ -422,8 +426,6 @@ int dispatch_stream(const void* X, int ldx, const void* W, int ldw, const float*
 
 }  // namespace
 
-// Split count for the stream decode GEMM: enough blocks for 256 CUs (one block per CU), at least
-// 8 K-steps per block, S | K-steps.
 RAGK_API int ragk_gemm_stream_set_diag(int dg) {
   g_stream_diag = (dg >= 1 && dg <= 3) ? dg : 0;
   return 0;
@@ -440,13 +442,16 @@ RAGK_API int ragk_gemm_stream_set_pair_rows(int rows) {
   return 0;
 }
 
+// Split count for the stream decode GEMM: enough blocks for 256 CUs, at least 8 K-steps per block, S | K-steps. No split for
+// bf16 weights that have a 64-row tile for every CU: two slabs fill the second block of each CU, but the reduction costs more
+// (16384 x 4096 at 8 / 64 rows 47 / 54 us in two slabs, 27 / 30 in one).
 RAGK_API int ragk_gemm_stream_splits(int N, int K, int epi, int fp8) {
   const int Nrows = epi_pair(epi) ? 2 * N : N;
-  const int rows = stream_rows(epi);
+  const int rows = stream_rows(epi, fp8 != 0);
   const int tiles = (Nrows + rows - 1) / rows;
   const int steps = K / (fp8 ? 128 : 64);
   int S = 1;
-  const int slots = rows == 64 ? 640 : 320;  // 64-row tiles: two blocks per CU
+  const int slots = rows == 64 && epi_pair(epi) ? 640 : 320;
   while (tiles * S * 2 <= slots && steps % (S * 2) == 0 && steps / (S * 2) >= 8) S *= 2;
   return S;
 }

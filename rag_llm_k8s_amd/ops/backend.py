@@ -493,7 +493,7 @@ class NativeBackend(TorchBackend):
         # 29.2. From 2^24 weights on they are ahead at every row count (niduvik / rolesun 4096 wide, 50 rows: 985 / 1102 -> 775 /
         # 826 us a step). Models 2048 wide, whose steps the host bounds at 30 / 40 rows, lose (543 / 655 -> 569 / 719); the line
         # lies between the two, and long projections of many rows below it forgo the GPU's gain.
-        if w.dtype != torch.bfloat16:
+        if isinstance(w, Fp8Weight) or w.dtype != torch.bfloat16:
             return False
         if M <= 64:
             return w.numel() >= 1 << 24 and self.part_ok(M, w)

@@ -88,6 +88,19 @@ def use_stream(M, N, K, epi, fp8=False):
     return M > 16 if fp8 else True
 
 
+def use_slabs(M, N, K, epi):
+    """Long projections of large weights at 17 to 64 rows: the LDS-DMA weight stream in fp32 slabs and a pass that sums them
+    (gemm_mid.hip ragk_gemm_slabs), where the register-streaming kernel keeps its weights on too few blocks and reads the
+    activations again for every 16 columns. 17 / 64 rows: 4096 x 14336 40 / 66 us -> 24 / 28, 14336 x 4096 37 / 74 -> 29 / 32,
+    33 / 64 rows: 6144 x 4096 28 / 39 -> 15 / 18; 64 rows of 4096 x 4096 23 -> 13. The second launch, the slabs' allocation and
+    this rule cost the host 7 us, so not where the GPU gains little more (20 rows: 6144 x 4096 22 against 14, 4096 x 4096 14
+    against 11; a rolesun step of 694 us became 723), nor below 2^24 weights, where the step's launches bound it (2048 x 5632 at
+    20 rows 16.6 against 9.4, but the steps that hold it 368 -> 409 and 508 -> 557 us); up to 16 rows the second launch takes
+    what the first gains."""
+    return (16 < M <= 64 and K >= 4096 and K % 128 == 0 and N % 8 == 0 and epi not in PAIR_EPI and N * K >= 1 << 24
+            and M * N * K >= 8e8 and stream_part_cfg(M, N, K)[1] > 1)
+
+
 def use_vocab(M, N, K, epi):
     """fp32 logits go to the slab form of the stream GEMM with one slab: its 64-row tiles keep two blocks a CU and no K-split
     ends in a reduction (32000 x 4096, 4 / 32 rows: stream GEMM 64 / 64 us -> 49 / 48; 32768 x 4096, 11 rows: register-streaming
@@ -251,6 +264,9 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
         path = 5
     if path is None and DEC_DEFAULT and use_dec(M, N, K, epi):
         path = 4
+    if path is None and use_slabs(M, N, K, epi) and _vec_rows(
+            x, w, out, *(() if resid is None else (resid,))) and (bias is None or bias.data_ptr() % 16 == 0):
+        return _gemm_slabs(x, w, out, bias, resid, ldr, M, N, K, e, out_f32)
     if path == 5:
         rc = _gemm_stream(x, w, None, out, bias, resid, ldr, M, N, K, epi, e, out_f32)
     elif path == 4:
@@ -952,6 +968,16 @@ def _gemm_stream(x, w, wscale, out, bias, resid, ldr, M, N, K, epi, e, out_f32):
     return L.ragk_gemm_stream(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), ptr(wscale), out.data_ptr(),
                               out.stride(0), ptr(bias), ptr(resid), ldr, M, N, K, e, int(out_f32), S, ws.data_ptr(),
                               cnt.data_ptr(), stream_ptr())
+
+
+def _gemm_slabs(x, w, out, bias, resid, ldr, M, N, K, e, out_f32):
+    """gemm() of at most 64 rows through the stream GEMM's fp32 slabs."""
+    rows, S = stream_part_cfg(M, N, K)
+    ws = torch.empty(S * M * N, dtype=torch.float32, device=x.device)
+    check(_lib.lib().ragk_gemm_slabs(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
+                                     ptr(bias), ptr(resid), ldr, M, N, K, e, int(out_f32), S, rows, ws.data_ptr(),
+                                     stream_ptr()), "ragk_gemm_slabs")
+    return out
 
 
 @functools.lru_cache(maxsize=256)

@@ -1,0 +1,103 @@
+"""Products of at most 64 rows through fp32 slabs, and a short prompt's step on them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _bound(x, w, y, out_f32):
+    """Rounding of a K-long fp32 sum in any order, and of the result: K 2^-24 of the terms' magnitudes, half a bf16 step."""
+    K = x.shape[1]
+    return K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + (0 if out_f32 else 2.0 ** -8) * y.abs() + 1e-6
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 4096, 14336), (20, 14344, 4096), (33, 6152, 4096), (48, 5000, 8192), (64, 4096, 4096)])
+def test_slabs(native, M, N, K):
+    """Row counts around the 16-row fragments, columns that end within a tile, every epilogue, in place and strided."""
+    assert native.use_slabs(M, N, K, "none") and not native.use_slabs(16, N, K, "none")
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, K + 64, device=DEV, generator=g).bfloat16()[:, :K]
+    w = (torch.randn(N, K, device=DEV, generator=g) / K ** 0.5).bfloat16()
+    b = torch.randn(N, device=DEV, generator=g).bfloat16()
+    r = torch.randn(M, N, device=DEV, generator=g).bfloat16()
+    y = x.double() @ w.double().t()
+    for epi, ref in (("none", y), ("bias", y + b.double()), ("resid", y + r.double()), ("bias_resid", y + b.double() + r.double())):
+        for f32 in (False, True):
+            out = torch.full((M + 1, N + 8), 7.0, device=DEV, dtype=torch.float32 if f32 else torch.bfloat16)
+            got = native.gemm(x, w, bias=b, resid=r, epi=epi, out=out[:M, :N], out_f32=f32)
+            assert bool(((got.double() - ref).abs() <= _bound(x, w, ref, f32)).all()), epi
+            assert bool((out[M] == 7).all()) and bool((out[:, N:] == 7).all())
+    for epi, act in (("gelu", lambda v: torch.nn.functional.gelu(v)), ("bias_gelu", lambda v: torch.nn.functional.gelu(v + b.double())),
+                     ("bias_gelu_tanh", lambda v: torch.nn.functional.gelu(v + b.double(), approximate="tanh"))):
+        ref = act(y)  # |gelu'| <= 1.13; the function itself in fp32
+        got = native.gemm(x, w, bias=b, epi=epi)
+        assert bool(((got.double() - ref).abs() <= 1.13 * _bound(x, w, y, True) + 2.0 ** -8 * ref.abs() + 1e-5).all()), epi
+    want = native.gemm(x, w, resid=r, epi="resid")
+    assert torch.equal(native.gemm(x, w, resid=r, epi="resid", out=r), want)  # the residual in place
+
+
+def test_unaligned_rows_keep_their_kernel(native):
+    """Rows off 16 bytes, which the slabs' loads and stores cannot take, go where they went."""
+    M, N, K = 33, 6144, 4096
+    x, w = torch.randn(M, K, device=DEV).bfloat16(), (torch.randn(N, K, device=DEV) / 64).bfloat16()
+    want = native.gemm(x, w, path=1)
+    out = torch.empty(M, N + 4, device=DEV, dtype=torch.bfloat16)[:, 4:]
+    assert torch.equal(native.gemm(x, w, out=out), want)
+
+
+@pytest.mark.parametrize("M", [1, 16, 33, 64])
+@pytest.mark.parametrize("N,K", [(16384, 512), (16424, 1024), (18560, 2048)])
+def test_wide_stream_tiles(native, M, N, K):
+    """bf16 weights from 16384 rows in 64-row tiles: a tile a CU, a last tile that is cut."""
+    assert native.use_stream(M, N, K, "bias")
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    w = (torch.randn(N, K, device=DEV, generator=g) / K ** 0.5).bfloat16()
+    b = torch.randn(N, device=DEV, generator=g).bfloat16()
+    ref = x.double() @ w.double().t() + b.double()
+    for f32 in (False, True):
+        out = torch.full((M + 1, N), 7.0, device=DEV, dtype=torch.float32 if f32 else torch.bfloat16)
+        got = native.gemm(x, w, bias=b, epi="bias", out=out[:M], out_f32=f32)
+        assert bool(((got.double() - ref).abs() <= _bound(x, w, ref, f32)).all()) and bool((out[M] == 7).all())
+
+
+@pytest.mark.parametrize("lens", [[1], [5], [20], [7, 30, 27]])
+def test_short_prompt(native, lens, monkeypatch):
+    """A prompt of at most 64 tokens on slabs against the step on whole products: logits, and the cache rows of layer 0."""
+    from rag_llm_k8s_amd.models import llama as L
+    from rag_llm_k8s_amd.models.base import StepInput
+    from rag_llm_k8s_amd.ops.backend import AttnMeta
+    from rag_llm_k8s_amd.utils.synthetic import llama_state_dict
+
+    cfg = L.llama31_8b()
+    cfg.vocab_size, cfg.num_hidden_layers = 512, 2
+    m = L.LlamaModel(cfg, L.LlamaWeights.from_state_dict(cfg, llama_state_dict(cfg, seed=0, std=0.02), DEV), DEV,
+                     max_positions=256)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    pos = [p for n in lens for p in range(n)]
+    slots = [s * 64 + p for s, n in enumerate(lens) for p in range(n)]
+    cu = [sum(lens[:i]) for i in range(len(lens) + 1)]
+    steps = []
+    for few in (True, False):
+        m.allocate_kv_cache(len(lens))
+        tiles, qtiles = m.prefill_work(lens, DEV)
+        meta = AttnMeta("prefill", i32(lens), i32([[s] for s in range(len(lens))]), cu_q=i32(cu), tiles=tiles, qtiles=qtiles,
+                        host_kv_lens=lens, host_q_lens=lens)
+        calls = []
+        if few:
+            run = m.hidden_states_few
+            monkeypatch.setattr(m, "hidden_states_few", lambda *a: (calls.append(1), run(*a))[1])
+        else:
+            monkeypatch.setattr(m.be, "splits", lambda M, w: False)
+        ids = i32([3 + 7 * i % 500 for i in range(len(pos))])
+        lg = m.forward(StepInput(ids, i32(pos), i32(slots), meta, i32([c - 1 for c in cu[1:]])))
+        assert len(calls) == int(few)
+        rows = [t[torch.tensor(slots) // 64, :, torch.tensor(slots) % 64].double() for t in m.kv_cache[0]]
+        steps.append((lg.double(), *rows))
+    # layer 0's rows are sums in another order, rounded to bf16: a step of 2^-7, through the rotation one of either half
+    (k, v), (k0, v0) = steps[0][1:], steps[1][1:]
+    assert bool(((v - v0).abs() <= 2.0 ** -7 * v0.abs() + 1e-4).all())
+    assert bool(((k - k0).abs() <= 2.0 ** -5 * (k0.abs() + k0.roll(64, -1).abs()) + 1e-4).all())
+    # logits: two layers of such steps
+    assert float((steps[0][0] - steps[1][0]).norm() / steps[1][0].norm()) < 2e-2

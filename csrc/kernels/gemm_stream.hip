@@ -166,11 +166,17 @@ __global__ __launch_bounds__(ST_THREADS, ROWS == 64 ? 2 : 1) void gemm_stream_ke
   const int nst = steps_total / S;
   const int k0 = slice * nst * G::KSTEP;
 
-  f32x4 acc[MT][J];
+  // bf16: a K-step's halves in sums of their own, so that no sum is longer than the register-streaming kernel's, which cuts K
+  // over its waves (normal numbers, rms error of the fp32 results: 64 x 6144 x 4096
+  // in four slabs 1.89e-7 -> 1.34e-7, the other kernel 1.37e-7; 8 x 18560 x 4096 in one 3.96e-7 -> 2.72e-7; as fast)
+  constexpr int AC = FP8 ? 1 : 2;
+  f32x4 acc[AC][MT][J];
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
+  for (int a = 0; a < AC; ++a)
 #pragma unroll
-    for (int j = 0; j < J; ++j) acc[t][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[a][t][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   // prologue: NS-1 stages in flight
 #pragma unroll
@@ -209,7 +215,8 @@ __global__ __launch_bounds__(ST_THREADS, ROWS == 64 ? 2 : 1) void gemm_stream_ke
           const int R = 16 * m + fr;
           const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xt + R * 128 + 16 * swz(R, c));
 #pragma unroll
-          for (int j = 0; j < J; ++j) acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, wf[j], acc[m][j], 0, 0, 0);
+          for (int j = 0; j < J; ++j)
+            acc[s][m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, wf[j], acc[s][m][j], 0, 0, 0);
         }
       }
     } else {
@@ -230,7 +237,8 @@ __global__ __launch_bounds__(ST_THREADS, ROWS == 64 ? 2 : 1) void gemm_stream_ke
           const int R = 16 * m + fr;
           const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xh + R * 128 + 16 * swz(R, c));
 #pragma unroll
-          for (int j = 0; j < J; ++j) acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, wf[j], acc[m][j], 0, 0, 0);
+          for (int j = 0; j < J; ++j)
+            acc[0][m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, wf[j], acc[0][m][j], 0, 0, 0);
         }
       }
     }
@@ -247,7 +255,7 @@ __global__ __launch_bounds__(ST_THREADS, ROWS == 64 ? 2 : 1) void gemm_stream_ke
     for (int j = 0; j < J; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        sC[(16 * m + 4 * fh + r) * G::EPI_LD + wid * (ROWS / 4) + 16 * j + fr] = acc[m][j][r];
+        sC[(16 * m + 4 * fh + r) * G::EPI_LD + wid * (ROWS / 4) + 16 * j + fr] = AC == 2 ? acc[0][m][j][r] + acc[AC - 1][m][j][r] : acc[0][m][j][r];
   __syncthreads();
   if constexpr (SLAB) {
     float* ps = reinterpret_cast<float*>(C) + (size_t)slice * M * N;

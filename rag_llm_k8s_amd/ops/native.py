@@ -88,7 +88,7 @@ def use_stream(M, N, K, epi, fp8=False):
     return M > 16 if fp8 else True
 
 
-def use_slabs(M, N, K, epi):
+def use_slabs(M, N, K, epi, out_f32=False):
     """Long projections of large weights at 17 to 64 rows: the LDS-DMA weight stream in fp32 slabs and a pass that sums them
     (gemm_mid.hip ragk_gemm_slabs), where the register-streaming kernel keeps its weights on too few blocks and reads the
     activations again for every 16 columns. 17 / 64 rows: 4096 x 14336 40 / 66 us -> 24 / 28, 14336 x 4096 37 / 74 -> 29 / 32,
@@ -96,9 +96,10 @@ def use_slabs(M, N, K, epi):
     this rule cost the host 7 us, so not where the GPU gains little more (20 rows: 6144 x 4096 22 against 14, 4096 x 4096 14
     against 11; a rolesun step of 694 us became 723), nor below 2^24 weights, where the step's launches bound it (2048 x 5632 at
     20 rows 16.6 against 9.4, but the steps that hold it 368 -> 409 and 508 -> 557 us); up to 16 rows the second launch takes
-    what the first gains."""
+    what the first gains. Two slabs are longer sums than the other kernel's eight (40 x 14336 x 4096, rms error of fp32 results
+    1.9e-7 against 1.4e-7; rounded to bf16 1.66e-3 both): not for fp32 results."""
     return (16 < M <= 64 and K >= 4096 and K % 128 == 0 and N % 8 == 0 and epi not in PAIR_EPI and N * K >= 1 << 24
-            and M * N * K >= 8e8 and stream_part_cfg(M, N, K)[1] > 1)
+            and M * N * K >= 8e8 and stream_part_cfg(M, N, K)[1] > (3 if out_f32 else 1))
 
 
 def use_vocab(M, N, K, epi):
@@ -264,7 +265,7 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
         path = 5
     if path is None and DEC_DEFAULT and use_dec(M, N, K, epi):
         path = 4
-    if path is None and use_slabs(M, N, K, epi) and _vec_rows(
+    if path is None and use_slabs(M, N, K, epi, out_f32) and _vec_rows(
             x, w, out, *(() if resid is None else (resid,))) and (bias is None or bias.data_ptr() % 16 == 0):
         return _gemm_slabs(x, w, out, bias, resid, ldr, M, N, K, e, out_f32)
     if path == 5:

@@ -254,7 +254,7 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
             return out
     if path == 0:
         return gemm_mid(x, w, bias=bias, resid=resid, epi=epi, out=out, out_f32=out_f32)
-    if path is None and not out_f32 and use_hold(M, N, K, epi) and _vec_rows(x, w):
+    if path is None and not out_f32 and use_hold(M, N, K, epi) and _vec_rows(x, w) and w.stride(0) < 1 << 24:
         return gemm_hold(x, w, par=bias, epi=epi, out=out)
     if (path is None and use_vocab(M, N, K, epi) and out_f32 and out.stride(0) == N and _vec_rows(x, w)
             and out.data_ptr() % 16 == 0):
@@ -590,6 +590,8 @@ def gemm_part(x, w, out=None, ks=None):
     if (STREAM_PART and not fp8 and ks is None and out is None and M >= STREAM_PART_MIN_M and K % 64 == 0
             and N % 4 == 0 and stream_part_cfg(M, N, K)[1] > 0):
         return gemm_stream_part(x, wt)
+    if fp8 and ks is None and out is None and use_hold_slabs(M, N, K) and _vec_rows(x, wt):
+        return gemm_hold_slabs(x, wt, w.scale)
     ks, S = gemm_part_slabs(M, N, K, ks)
     _req(S > 0, "gemm_part: unsupported K=%d" % K)
     if out is None:
@@ -988,12 +990,12 @@ def _hold_rows(K, fp8):
 
 def use_hold(M, N, K, epi, fp8=False):
     """Packed gate/up projections whose activations fit a block's registers go to gemm_hold.hip: 11264 x 2048 bf16 at 12 / 50
-    rows 14.7 / 24 -> 11.8 / 17 us against the register-streaming kernel, 28672 x 4096 fp8 at 11 / 32 rows 38 / 37 -> 27.5 / 33
+    rows 14.7 / 24 -> 11.1 / 16.5 us against the register-streaming kernel, 28672 x 4096 fp8 at 11 / 32 rows 38 / 37 -> 26 / 31
     (gemm_fp8_dec / gemm_stream). Not where they lose: K of 1024 (a barrier for every 16 KB of weights: 28672 rows 10.3 against
     8.7); row tiles that leave the last of a CU's few rounds mostly empty (6144 x 3072 bf16, 1.5 rounds: 11.9 against 11.4);
     bf16 weights that the LDS ring streams without a K-split (28672 x 4096: 43 against 42); and more rows than one launch
-    holds, but for 8192 rows of fp8 and up, whose second launch reads the Infinity Cache while the ring is down to half its
-    depth (14336 x 4096 at 48 rows 51 -> 38, but 7168 x 4096 25 against 28)."""
+    holds, but for 8192 rows of fp8 and up that use_hold_slabs_silu leaves (K = 3072), whose second launch reads the Infinity
+    Cache while the ring is down to half its depth."""
     if not 0 < M <= 64 or K < 2048 or epi not in PAIR_EPI or (fp8 and epi != "silu_mul"):
         return False
     per = _hold_rows(K, fp8)
@@ -1031,6 +1033,34 @@ def gemm_hold(x, w, wscale=None, par=None, epi="silu_mul", out=None):
 
 
 # ----------------------------------------------------------------------------- fp8 GEMM
+def use_hold_slabs(M, N, K):
+    """fp8 split-K products whose slabs go through gemm_hold.hip (a slab per 2048 of K) instead of gemm_part.hip, which stages
+    the activations of a K-slice in every block of 64 columns: 4096 x 14336 at 17 / 33 / 64 rows 19 / 26 / 33 us -> 16 / 19 / 23,
+    5120 x 18432 32 / 38 / 49 -> 23 / 26 / 31, 4096 x 8192 at 33 / 64 rows 14.9 / 18.5 -> 13.9 / 18.1. Smaller weights leave a
+    block too few rows for the 128 KB of x that it loads first (4096 x 8192 at 17 rows 10.7 against 12.0, 4096 x 4096 at 33 / 64
+    7.8 / 9.5 against 9.9 / 13), and up to 16 rows the two are equal."""
+    return 16 < M <= 64 and K % 2048 == 0 and N % 16 == 0 and N * K >= (5 << 23 if M <= 32 else 1 << 25)
+
+
+def gemm_hold_slabs(x, w8, scale, out=None):
+    """fp32 slabs P[K / 2048, M, N] of x @ dequant(w8)^T with the activations of a slab held in registers (gemm_hold.hip)."""
+    M, K = x.shape
+    N = w8.shape[0]
+    _req(0 < M <= 64 and K % 2048 == 0 and N % 16 == 0 and w8.shape[1] == K, "gemm_hold_slabs shape")
+    if out is None:
+        out = torch.empty((K // 2048, M, N), dtype=torch.float32, device=x.device)
+    check(_lib.lib().ragk_gemm_hold_slabs(x.data_ptr(), x.stride(0), w8.data_ptr(), w8.stride(0), scale.data_ptr(),
+                                          out.data_ptr(), M, N, K, _cu_count(), stream_ptr()), "ragk_gemm_hold_slabs")
+    return out
+
+
+def use_hold_slabs_silu(M, K):
+    """fp8 gate/up projections of more rows than a launch of gemm_hold holds: slabs of 2048 of K and a pass that sums and pairs
+    them, 28672 x 4096 at 33 / 64 rows 54 / 61 us (two launches) -> 33 / 38, 7168 x 4096 22 / 26 (gemm_stream) -> 17 / 21, 16384
+    x 6144 at 17 / 64 rows 38 / 72 -> 29 / 37. Up to 16 rows the pass takes what the slabs gain (8192 x 6144 18.6 against 18.1)."""
+    return 16 < M <= 64 and K % 2048 == 0 and M > _hold_rows(K, True)
+
+
 def quant_fp8_rows(x, q=None, scale=None):
     """bf16 [M,K] -> (e4m3fn [M,K], fp32 [M]) with one dynamic scale per row."""
     _bf16_2d(x, "x")
@@ -1075,6 +1105,12 @@ def gemm_fp8(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False):
     if M == 0:
         return out
     ldr = resid.stride(0) if resid is not None else 0
+    if epi == "silu_mul" and use_hold_slabs_silu(M, K) and _vec_rows(x, w8, out):
+        ws = torch.empty(K // 2048 * M * 2 * N, dtype=torch.float32, device=x.device)
+        check(_lib.lib().ragk_gemm_hold_slabs_silu(x.data_ptr(), x.stride(0), w8.data_ptr(), w8.stride(0), sw.data_ptr(),
+                                                   out.data_ptr(), out.stride(0), M, N, K, _cu_count(), ws.data_ptr(),
+                                                   stream_ptr()), "ragk_gemm_hold_slabs_silu")
+        return out
     if use_hold(M, N, K, epi, fp8=True) and _vec_rows(x, w8):
         return gemm_hold(x, w8, sw, epi=epi, out=out)
     if M <= DEC_MAX_M and FP8_DEC_STREAM and use_stream(M, N, K, epi, fp8=True):

@@ -166,10 +166,10 @@ __global__ __launch_bounds__(ST_THREADS, ROWS == 64 ? 2 : 1) void gemm_stream_ke
   const int nst = steps_total / S;
   const int k0 = slice * nst * G::KSTEP;
 
-  // bf16: a K-step's halves in sums of their own, so that no sum is longer than the register-streaming kernel's, which cuts K
-  // over its waves (normal numbers, rms error of the fp32 results: 64 x 6144 x 4096
-  // in four slabs 1.89e-7 -> 1.34e-7, the other kernel 1.37e-7; 8 x 18560 x 4096 in one 3.96e-7 -> 2.72e-7; as fast)
-  constexpr int AC = FP8 ? 1 : 2;
+  // bf16 without slabs: a K-step's halves in sums of their own, so that a sum over all of K is no longer than where K was cut in
+  // two (normal numbers, rms error of fp32 results: 8 x 18560 x 4096 3.96e-7 -> 2.72e-7, as fast). Slabs, whose sums are short,
+  // keep one: two cost them 1 % at 33 rows and more.
+  constexpr int AC = FP8 || SLAB ? 1 : 2;
   f32x4 acc[AC][MT][J];
 #pragma unroll
   for (int a = 0; a < AC; ++a)
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(ST_THREADS, ROWS == 64 ? 2 : 1) void gemm_stream_ke
           const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xt + R * 128 + 16 * swz(R, c));
 #pragma unroll
           for (int j = 0; j < J; ++j)
-            acc[s][m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, wf[j], acc[s][m][j], 0, 0, 0);
+            acc[s % AC][m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, wf[j], acc[s % AC][m][j], 0, 0, 0);
         }
       }
     } else {

@@ -96,10 +96,10 @@ def use_slabs(M, N, K, epi, out_f32=False):
     this rule cost the host 7 us, so not where the GPU gains little more (20 rows: 6144 x 4096 22 against 14, 4096 x 4096 14
     against 11; a rolesun step of 694 us became 723), nor below 2^24 weights, where the step's launches bound it (2048 x 5632 at
     20 rows 16.6 against 9.4, but the steps that hold it 368 -> 409 and 508 -> 557 us); up to 16 rows the second launch takes
-    what the first gains. Two slabs are longer sums than the other kernel's eight (40 x 14336 x 4096, rms error of fp32 results
-    1.9e-7 against 1.4e-7; rounded to bf16 1.66e-3 both): not for fp32 results."""
-    return (16 < M <= 64 and K >= 4096 and K % 128 == 0 and N % 8 == 0 and epi not in PAIR_EPI and N * K >= 1 << 24
-            and M * N * K >= 8e8 and stream_part_cfg(M, N, K)[1] > (3 if out_f32 else 1))
+    what the first gains. Slabs are longer sums than the other kernel's, which cuts K eight times (64 x 6144 x 4096, rms
+    error of fp32 results 1.9e-7 against 1.4e-7; rounded to bf16 1.6605e-3 both): not for fp32 results."""
+    return (not out_f32 and 16 < M <= 64 and K >= 4096 and K % 128 == 0 and N % 8 == 0 and epi not in PAIR_EPI
+            and N * K >= 1 << 24 and M * N * K >= 8e8 and stream_part_cfg(M, N, K)[1] > 1)
 
 
 def use_vocab(M, N, K, epi):

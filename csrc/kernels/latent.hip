@@ -398,12 +398,22 @@ struct OutArgs {
   int B, H, DV, window, min_tiles, max_parts;
 };
 
-// grid: (H * ceil(DV / 64), batch / NB): joins the partitions of one head for NB sequences, 64 rows of its value map, gate
+// grid: (H * ceil(DV / 64), batch / NB): joins the partitions of one head for NB sequences, 64 rows of its value map, gate.
+// Bound by the trips to memory in turn. Two of them, where few sequences leave the chip to few blocks: lengths, maxima and sums,
+// the first partitions, weights and gate slabs are asked for together (whatever lies past a sequence's partitions is dropped),
+// further partitions behind the weights of the join, which are exponentials of values read once (they were read three times).
+// One sequence's few columns are joined by several threads each. Steps of four layers, us before and after: 1 x 4000 tokens,
+// 4096 wide 620.6 -> 613.5, 3 x 2000 639.5 -> 636.2, 2048 wide 50 x 1000 370 -> 365. From eight sequences a block the
+// partitions' stream bounds it, and asking ahead for what may not be there loses (40 x 3000 820 -> 832).
 template <typename TP, int NR, int NB>
 __global__ __launch_bounds__(256) void latent_out_kernel(OutArgs<TP> a) {
   constexpr int Rp = 128 * NR, KS = Rp / 32, ST = Rp + 8, TT = LatentTile<NR>::TT;
-  constexpr int U = NB <= 4 ? 16 : 8;  // partitions requested at a time
+  constexpr int NI = NB * (Rp / 4), PER = (NI + 255) / 256;  // joined 16-byte columns; of a thread
+  constexpr int JP = NI <= 128 ? 256 / NI : 1;               // threads of a column
+  constexpr int U = PER <= 2 ? 16 : 8;                       // partitions requested at a time
+  constexpr bool AHEAD = NB <= 4;
   __shared__ __attribute__((aligned(16))) bf16_t s_c[NB * ST];
+  __shared__ __attribute__((aligned(16))) f32x4 s_j[JP > 1 ? 256 : 1];
   __shared__ float s_w[NB * MAX_PARTS];  // exp2(m_p - M) / L
   __shared__ int s_n[NB];                // partitions
   const int nd = (a.DV + 63) / 64, h = blockIdx.x / nd, d0 = (blockIdx.x % nd) * 64;
@@ -412,65 +422,108 @@ __global__ __launch_bounds__(256) void latent_out_kernel(OutArgs<TP> a) {
   const int dr = d0 + 16 * wid;  // this wave's 16 value rows
   const bool live = dr < a.DV;   // DV is a multiple of 16
   const int col = h * a.DV + dr + 4 * fh;
+  // partition maxima and sums: 16 lanes per sequence
+  constexpr int QP = MAX_PARTS / 16;
+  const int wb = threadIdx.x >> 4, wq = threadIdx.x & 15;
+  f32x2 ml[QP];
+  int len = 0;
+  if (threadIdx.x < 16 * NB) {
+    len = a.kv_lens[b0 + min(wb, nb - 1)];
+    const f32x2_a4* p = reinterpret_cast<const f32x2_a4*>(a.part_ml) + ((size_t)(b0 + min(wb, nb - 1)) * a.H + h) * a.max_parts;
+#pragma unroll
+    for (int j = 0; j < QP; ++j) ml[j] = p[min(wq + 16 * j, a.max_parts - 1)];
+  }
+  const int jp = JP > 1 ? threadIdx.x / NI : 0, j0 = JP > 1 ? threadIdx.x % NI : threadIdx.x;
+  auto column = [&](int i) {  // first partition of a thread's column i
+    const int b = min((j0 + 256 * i) / (Rp / 4), nb - 1), c = ((j0 + 256 * i) % (Rp / 4)) * 4;
+    return a.part_o + ((size_t)(b0 + b) * a.H + h) * a.max_parts * Rp + c;
+  };
+  f32x4 u[AHEAD ? PER : 1][U];
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (k / 4 * 4 < a.max_parts)
+          u[i][k] = *reinterpret_cast<const f32x4*>(column(i) + (size_t)min(jp * U + k, a.max_parts - 1) * Rp);
+  }
   bf16x8 wf[KS];
-  f32x4 z = {0.f, 0.f, 0.f, 0.f};
-  if (live) {  // requested before the join
+  f32x4 zs[PSU];
+  if (live) {
 #pragma unroll
     for (int s = 0; s < KS; ++s)
       wf[s] = *reinterpret_cast<const bf16x8*>(a.wuv + ((size_t)h * a.DV + dr + fr) * Rp + 32 * s + 8 * fh);
     if (a.off_g >= 0) {
       const TP* g = a.P.P + (size_t)(b0 + min(fr, nb - 1)) * a.P.ld + a.off_g + col;
       if constexpr (sizeof(TP) == 4) {
-        for (int s0 = 0; s0 < a.P.S; s0 += PSU) {
-          f32x4 u[PSU];
 #pragma unroll
-          for (int k = 0; k < PSU; ++k) u[k] = *reinterpret_cast<const f32x4*>(g + (size_t)min(s0 + k, a.P.S - 1) * a.P.slab);
-#pragma unroll
-          for (int k = 0; k < PSU; ++k)
-            if (s0 + k < a.P.S) z += u[k];
-        }
+        for (int k = 0; k < PSU; ++k) zs[k] = *reinterpret_cast<const f32x4*>(g + (size_t)min(k, a.P.S - 1) * a.P.slab);
       } else {
         const bf16x4 zz = *reinterpret_cast<const bf16x4*>(g);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) z[r] = bf2f_s(zz[r]);
+        for (int r = 0; r < 4; ++r) zs[0][r] = bf2f_s(zz[r]);
       }
     }
   }
-  // partition weights: 16 lanes per sequence
   if (threadIdx.x < 16 * NB) {
-    const int b = threadIdx.x >> 4, q = threadIdx.x & 15;
-    int n = 0;
-    if (b < nb) n = Split(a.kv_lens[b0 + b] - 1, a.window, TT, a.min_tiles, a.max_parts).parts();
-    const float* ml = a.part_ml + ((size_t)(b0 + min(b, nb - 1)) * a.H + h) * a.max_parts * 2;
+    const int n = wb < nb ? Split(len - 1, a.window, TT, a.min_tiles, a.max_parts).parts() : 0;
     float M = -INFINITY, L = 0.f;
-    for (int p = q; p < n; p += 16) M = fmaxf(M, ml[2 * p]);
+#pragma unroll
+    for (int j = 0; j < QP; ++j)
+      if (wq + 16 * j < n) M = fmaxf(M, ml[j][0]);
 #pragma unroll
     for (int x = 1; x < 16; x <<= 1) M = fmaxf(M, __shfl_xor(M, x, 64));
     const float Mu = M == -INFINITY ? 0.f : M;
-    for (int p = q; p < n; p += 16) L += ml[2 * p + 1] * __builtin_amdgcn_exp2f(ml[2 * p] - Mu);
+#pragma unroll
+    for (int j = 0; j < QP; ++j) {
+      ml[j][0] = wq + 16 * j < n ? __builtin_amdgcn_exp2f(ml[j][0] - Mu) : 0.f;
+      if (wq + 16 * j < n) L += ml[j][1] * ml[j][0];
+    }
 #pragma unroll
     for (int x = 1; x < 16; x <<= 1) L += __shfl_xor(L, x, 64);
     const float inv = L > 0.f ? 1.f / L : 0.f;
-    for (int p = q; p < MAX_PARTS; p += 16)
-      s_w[b * MAX_PARTS + p] = p < n ? __builtin_amdgcn_exp2f(ml[2 * p] - Mu) * inv : 0.f;
-    if (q == 0) s_n[b] = n;
+#pragma unroll
+    for (int j = 0; j < QP; ++j) s_w[wb * MAX_PARTS + wq + 16 * j] = ml[j][0] * inv;
+    if (wq == 0) s_n[wb] = n;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < NB * (Rp / 4); i += 256) {
-    const int b = i / (Rp / 4), c = (i % (Rp / 4)) * 4, n = s_n[b];
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    const float* po = a.part_o + ((size_t)(b0 + min(b, nb - 1)) * a.H + h) * a.max_parts * Rp + c;
-    for (int p = 0; p < n; p += U) {
-      f32x4 u[U];
 #pragma unroll
-      for (int k = 0; k < U; ++k) u[k] = *reinterpret_cast<const f32x4*>(po + (size_t)min(p + k, n - 1) * Rp);
+  for (int i = 0; i < PER; ++i) {
+    const int ji = j0 + 256 * i, b = ji / (Rp / 4), c = (ji % (Rp / 4)) * 4;
+    if (ji >= NI || jp >= JP) break;
+    const int n = s_n[b];
+    const float* po = column(i);
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    auto add = [&](const f32x4 (&x)[U], int p) __attribute__((always_inline)) {
 #pragma unroll
       for (int k = 0; k < U; ++k)
-        if (p + k < n) v += u[k] * s_w[b * MAX_PARTS + p + k];
+        if (p + k < n) v += x[k] * s_w[b * MAX_PARTS + p + k];
+    };
+    int p = jp * U;
+    if constexpr (AHEAD) {
+      add(u[i], p);
+      p += JP * U;
     }
-    *reinterpret_cast<uint2*>(s_c + b * ST + c) = make_uint2(pk2bf(v[0], v[1]), pk2bf(v[2], v[3]));
+    for (; p < n; p += JP * U) {
+      f32x4 y[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) y[k] = *reinterpret_cast<const f32x4*>(po + (size_t)min(p + k, n - 1) * Rp);
+      add(y, p);
+    }
+    if constexpr (JP > 1) s_j[threadIdx.x] = v;
+    else *reinterpret_cast<uint2*>(s_c + b * ST + c) = make_uint2(pk2bf(v[0], v[1]), pk2bf(v[2], v[3]));
   }
   __syncthreads();
+  if constexpr (JP > 1) {
+    if (threadIdx.x < NI) {
+      f32x4 v = s_j[threadIdx.x];
+#pragma unroll
+      for (int k = 1; k < JP; ++k) v += s_j[threadIdx.x + k * NI];
+      const int b = threadIdx.x / (Rp / 4), c = (threadIdx.x % (Rp / 4)) * 4;
+      *reinterpret_cast<uint2*>(s_c + b * ST + c) = make_uint2(pk2bf(v[0], v[1]), pk2bf(v[2], v[3]));
+    }
+    __syncthreads();
+  }
   if (!live) return;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -480,6 +533,14 @@ __global__ __launch_bounds__(256) void latent_out_kernel(OutArgs<TP> a) {
   }
   if (fr >= nb) return;
   if (a.off_g >= 0) {
+    f32x4 z = zs[0];
+    if constexpr (sizeof(TP) == 4) {
+      const TP* g = a.P.P + (size_t)(b0 + fr) * a.P.ld + a.off_g + col;
+#pragma unroll
+      for (int k = 1; k < PSU; ++k)
+        if (k < a.P.S) z += zs[k];
+      for (int k = PSU; k < a.P.S; ++k) z += *reinterpret_cast<const f32x4*>(g + (size_t)k * a.P.slab);
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[r] *= __builtin_amdgcn_rcpf(1.f + __expf(-z[r]));
   }
@@ -517,7 +578,8 @@ int launch_out(const OutArgs<TP>& a, hipStream_t st) {
   const int gx = a.H * ((a.DV + 63) / 64);  // fewer sequences a block where that is what fills the chip
   if (gx * ((a.B + 15) / 16) >= 256) hipLaunchKernelGGL((latent_out_kernel<TP, NR, 16>), dim3(gx, (a.B + 15) / 16), dim3(256), 0, st, a);
   else if (gx * ((a.B + 7) / 8) >= 256) hipLaunchKernelGGL((latent_out_kernel<TP, NR, 8>), dim3(gx, (a.B + 7) / 8), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((latent_out_kernel<TP, NR, 4>), dim3(gx, (a.B + 3) / 4), dim3(256), 0, st, a);
+  else if (a.B > 1) hipLaunchKernelGGL((latent_out_kernel<TP, NR, 4>), dim3(gx, (a.B + 3) / 4), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((latent_out_kernel<TP, NR, 1>), dim3(gx), dim3(256), 0, st, a);
   return (int)hipGetLastError();
 }
 

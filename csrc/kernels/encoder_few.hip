@@ -13,7 +13,7 @@
 // out, as the residual of the product after next.
 // Six layers of 384 columns, 14 rows: 220 us a call in seven launches a layer, 111 in these, 108.7 of it the chain on the device and
 // 88 the host's launches beside 31 of checks (119 a call where the host is not ahead). With the rows' loads in front of the weights,
-// column groups known when compiling and 64 bytes of arguments 101 and 68; 30 rows 142 -> 135; 24 layers of 1024, 14 rows 691 ->
+// column groups known when compiling, no spare K-steps and 64 bytes of arguments 96 and 68; 30 rows 142 -> 128; 24 layers of 1024, 14 rows 691 ->
 // 630. A launch on the device is 1.4 us behind the one before, 1.3 to 2 for the rows' (or the down projection's operands') trip to
 // memory and 1 through LDS for the sum. Past 16384 values of rows the repeated work costs more than it saves (ops/native.py
 // encoder_few_ok).
@@ -310,12 +310,18 @@ int few_attend(const FewArgs& a, hipStream_t st) {
   if (a.K() > FEW_H) return (int)hipErrorInvalidValue;
   return a.K() <= 512 ? few_rows<ATTEND, EPI, 1, D>(a, st) : few_rows<ATTEND, EPI, 2, D>(a, st);
 }
+// As many K-steps at once as a wave has (of K = 1536 three): a spare one is the last again, and its loads take their time (with
+// four, the chain of six such layers 101.1 us for 96.4 at 14 rows, 135.4 for 128.4 at 30).
 template <int EPI>
 int few_plain(const FewArgs& a, hipStream_t st) {
-  return a.K() <= 512    ? few_rows<ROWS, EPI, 1, 1>(a, st)
-         : a.K() <= 1024 ? few_rows<ROWS, EPI, 2, 1>(a, st)
-         : a.K() <= 2048 ? few_rows<ROWS, EPI, 4, 1>(a, st)
-                       : few_rows<ROWS, EPI, 8, 1>(a, st);
+  switch ((a.K() + 511) / 512) {
+    case 1: return few_rows<ROWS, EPI, 1, 1>(a, st);
+    case 2: return few_rows<ROWS, EPI, 2, 1>(a, st);
+    case 3: return few_rows<ROWS, EPI, 3, 1>(a, st);
+    case 4: return few_rows<ROWS, EPI, 4, 1>(a, st);
+    case 5: case 6: return few_rows<ROWS, EPI, 6, 1>(a, st);
+    default: return few_rows<ROWS, EPI, 8, 1>(a, st);
+  }
 }
 
 constexpr int POOL_W = 8;

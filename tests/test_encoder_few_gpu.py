@@ -63,7 +63,7 @@ def test_short_sequence(native, monkeypatch, T, hidden, heads, inter, pooling, k
 
 # the widths between (a kernel for each), and as many columns of a down projection as the arguments can name
 @pytest.mark.parametrize("T", [3, 17])
-@pytest.mark.parametrize("hidden,heads,inter", [(256, 8, 256), (768, 12, 3072), (896, 14, 1152), (128, 2, 32768)])
+@pytest.mark.parametrize("hidden,heads,inter", [(256, 8, 256), (768, 12, 3072), (896, 14, 1152), (384, 6, 2048), (128, 2, 32768)])
 def test_every_width(native, monkeypatch, T, hidden, heads, inter):
     test_short_sequence(native, monkeypatch, T, hidden, heads, inter, "mean", "bert")
 

@@ -188,7 +188,17 @@ __device__ __forceinline__ void mid_rope8(float (&x1)[8], float (&x2)[8], const 
   }
 }
 
-template <int MI, int NJ, int EPI>
+// Weights that one row of tiles reads once, by the streaming policy: 28672 x 4096 at 66 / 140 / 256 rows 50.8 / 56.2 / 66.2 -> 46.9 /
+// 53.4 / 61.9 us, 22528 x 2048 25.4 / 29.1 / 33.8 -> 23.4 / 27.6 / 31.3. Where tiles share them (several rows of tiles, a K-split) it
+// costs 2 to 11 % instead, and weights that the caches hold from call to call keep the other policy.
+__device__ __forceinline__ void blds16_nt_asm(i32x4 srd, int voff, int soff, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds_addr), "v"(voff), "s"(srd),
+               "s"(soff));
+}
+constexpr bool mid_has_nt(int e) { return e == EPI_NONE || epi_pair(e); }
+constexpr long long MID_NT_BYTES = 64LL << 20;  // twice the L2s
+
+template <int MI, int NJ, int EPI, bool NT = false>
 __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ B, int ldb, void* C, int ldc,
     const bf16_t* __restrict__ bias, const bf16_t* resid, int ldr, int M, int N, int K, int S, int out_f32, RopeKV rk) {
@@ -231,6 +241,7 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_mid_kernel(
   auto piece = [&](int q) {
     const int so = dk * (MID_BK * 2);
     if (q < MI) blds16_asm(srd_a, off_a[q], so, d_slot + (wid * MI + q) * 1024);
+    else if constexpr (NT) blds16_nt_asm(srd_b, off_b[q - MI], so, d_slot + OFF_B + (wid * NJ + q - MI) * 1024);
     else blds16_asm(srd_b, off_b[q - MI], so, d_slot + OFF_B + (wid * NJ + q - MI) * 1024);
   };
   auto advance = [&]() {
@@ -458,18 +469,21 @@ int mid_grid(int total) {
   return total < cus ? total : cus;
 }
 
-template <int MI, int NJ, int EPI>
+template <int MI, int NJ, int EPI, bool NT = false>
 int launch_mid(const void* A, int lda, const void* B, int ldb, void* C, int ldc, const void* bias, const void* resid, int ldr,
                int M, int N, int K, int S, int out_f32, hipStream_t st,
                const RopeKV& rk = RopeKV{}) {
+  if constexpr (!NT && mid_has_nt(EPI))
+    if (M <= 32 * MI && S == 1 && 2LL * N * K >= MID_NT_BYTES)
+      return launch_mid<MI, NJ, EPI, true>(A, lda, B, ldb, C, ldc, bias, resid, ldr, M, N, K, S, out_f32, st, rk);
   constexpr int lds = mid_stage(MI, NJ) * mid_depth(MI, NJ);
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<MI, NJ, EPI>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<MI, NJ, EPI, NT>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (attr != hipSuccess) return (int)attr;
   const long long total = (long long)((M + 32 * MI - 1) / (32 * MI)) * ((N + 32 * NJ - 1) / (32 * NJ)) * S;
   if (total > 0x7fffffff) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL((gemm_mid_kernel<MI, NJ, EPI>), dim3(mid_grid((int)total)), dim3(MID_THREADS), lds, st, (const bf16_t*)A, lda,
-                     (const bf16_t*)B, ldb, C, ldc, (const bf16_t*)bias, (const bf16_t*)resid, ldr, M, N, K, S, out_f32, rk);
+  hipLaunchKernelGGL((gemm_mid_kernel<MI, NJ, EPI, NT>), dim3(mid_grid((int)total)), dim3(MID_THREADS), lds, st, (const bf16_t*)A,
+                     lda, (const bf16_t*)B, ldb, C, ldc, (const bf16_t*)bias, (const bf16_t*)resid, ldr, M, N, K, S, out_f32, rk);
   return (int)hipGetLastError();
 }
 

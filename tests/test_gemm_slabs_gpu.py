@@ -14,13 +14,13 @@ def _bound(x, w, y, out_f32):
 
 @pytest.mark.parametrize("M,N,K", [(17, 4096, 14336), (20, 14344, 4096), (33, 6152, 4096), (48, 5000, 8192), (64, 4096, 4096)])
 def test_slabs(native, M, N, K):
-    """Row counts around the 16-row fragments, columns that end within a tile, every epilogue, in place and strided."""
+    """Row counts around the 16-row fragments, columns that end within a tile, every epilogue, in place, strided operands."""
     assert native.use_slabs(M, N, K, "none") and not native.use_slabs(16, N, K, "none")
     g = torch.Generator(device=DEV).manual_seed(M + N)
     x = torch.randn(M, K + 64, device=DEV, generator=g).bfloat16()[:, :K]
-    w = (torch.randn(N, K, device=DEV, generator=g) / K ** 0.5).bfloat16()
+    w = (torch.randn(N, K + 8, device=DEV, generator=g) / K ** 0.5).bfloat16()[:, 8:]
     b = torch.randn(N, device=DEV, generator=g).bfloat16()
-    r = torch.randn(M, N, device=DEV, generator=g).bfloat16()
+    r = torch.randn(M, N + 16, device=DEV, generator=g).bfloat16()[:, 16:]
     y = x.double() @ w.double().t()
     for epi, ref in (("none", y), ("bias", y + b.double()), ("resid", y + r.double()), ("bias_resid", y + b.double() + r.double())):
         for f32 in (False, True):
@@ -34,6 +34,7 @@ def test_slabs(native, M, N, K):
         got = native.gemm(x, w, bias=b, epi=epi)
         assert bool(((got.double() - ref).abs() <= 1.13 * _bound(x, w, y, True) + 2.0 ** -8 * ref.abs() + 1e-5).all()), epi
     want = native.gemm(x, w, resid=r, epi="resid")
+    assert torch.equal(native.gemm(x.contiguous(), w.contiguous(), resid=r.contiguous(), epi="resid"), want)
     assert torch.equal(native.gemm(x, w, resid=r, epi="resid", out=r), want)  # the residual in place
 
 

@@ -1731,11 +1731,11 @@ def _search_to_host(nq, k, launch):
     check(L.ragk_search_arm(at, n, st), "ragk_search_arm")
     try:
         launch(at, at + 8 * n)
-    except BaseException:
+        D, I = torch.empty(nq, k), torch.empty(nq, k, dtype=torch.int64)  # (while the search runs)
+        check(L.ragk_search_collect(at, n, I.data_ptr(), D.data_ptr(), st), "ragk_search_collect")
+    except BaseException:  # (an interrupt too, wherever it comes)
         L.ragk_stream_wait(st)  # the block goes back to its pool once nothing can write to it
         raise
-    D, I = torch.empty(nq, k), torch.empty(nq, k, dtype=torch.int64)  # (while the search runs)
-    check(L.ragk_search_collect(at, n, I.data_ptr(), D.data_ptr(), st), "ragk_search_collect")
     return D, I
 
 

@@ -1079,8 +1079,8 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
   table.wait();
 
   bf16x8 qf[C::KS];
-  char* sV = smem + wid * VB;
-  char* sK = smem + (NW + wid) * C::TILEB;  // KL only
+  char* sV = smem + wid_u * VB;
+  char* sK = smem + (NW + wid_u) * C::TILEB;  // KL only
   bf16x8 kf[KU / 16][C::KS];
   auto page = [&](int kt) { return (((size_t)table(kt / UPT) * a.Hkv + kvh) * KT + kt % UPT * KU) * D; };
   // (lanes' places as 32-bit offsets from a scalar address: a pair of registers a load otherwise)
@@ -1090,10 +1090,36 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
 #pragma unroll
   for (int i = 0; i < VP; ++i)
     v_lane[i] = lane / C::NC * C::ROWB + 16 * ((lane % C::NC) ^ vswz<D>(i * C::RPP + lane / C::NC));
+  constexpr int KP = C::RPP < 16 ? 16 / C::RPP : 1;  // K pieces likewise
+  unsigned kd_lane[KP];
+#pragma unroll
+  for (int i = 0; i < KP; ++i)
+    kd_lane[i] = lane / C::NC * C::ROWB + 16 * ((lane % C::NC) ^ kswz<D>(i * C::RPP + lane / C::NC));
+  if constexpr (KL) {  // held: worked out again in front of the loop they cost 0.2 us
+#pragma unroll
+    for (int i = 0; i < VP; ++i) asm volatile("" : "+v"(v_lane[i]));
+#pragma unroll
+    for (int i = 0; i < KP; ++i) asm volatile("" : "+v"(kd_lane[i]));
+  }
+  // (the instruction's offset counts for both addresses: four pieces to a scalar base and an LDS base. With each piece's own bases,
+  // the LDS one from vector registers, a tile's 32 requests were 200 instructions more: 256 pairs of 1000 / 2000 tokens 23.6 / 39.4
+  // us, now 22.4 / 38.0)
+  auto piece = [&](const bf16_t* tile, int i, unsigned at, char* lds) __attribute__((always_inline)) {
+    const auto* g = (const __attribute__((address_space(1))) char*)tile + i / 4 * 4096 + at;
+    auto* l = (__attribute__((address_space(3))) char*)lds + i / 4 * 4096;
+    constexpr int AUX = NT ? 2 : 0;
+    switch (i % 4) {
+      case 0: __builtin_amdgcn_global_load_lds(g, l, 16, 0, AUX); break;
+      case 1: __builtin_amdgcn_global_load_lds(g, l, 16, 1024, AUX); break;
+      case 2: __builtin_amdgcn_global_load_lds(g, l, 16, 2048, AUX); break;
+      default: __builtin_amdgcn_global_load_lds(g, l, 16, 3072, AUX); break;
+    }
+  };
   auto request_k = [&](int kt) {
     const bf16_t* kb = a.kc + page(kt);
     if constexpr (KL) {
-      stage_kv<D, false, NT, 1>(sK, 0, 1, lane, [&](int r) { return kb + (size_t)r * D; });
+#pragma unroll
+      for (int i = 0; i < C::PIECES; ++i) piece(kb, i, kd_lane[i % KP], sK);
     } else {
 #pragma unroll
       for (int t = 0; t < KU / 16; ++t)
@@ -1110,7 +1136,8 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
   auto request_v = [&](int kt) {
     const bf16_t* vb = a.vc + page(kt);
     if constexpr (!REGS) {
-      stage_kv<D, true, NT, 1>(sV, 0, 1, lane, [&](int r) { return vb + (size_t)r * D; });
+#pragma unroll
+      for (int i = 0; i < C::PIECES; ++i) piece(vb, i, v_lane[i % VP], sV);
     } else {
 #pragma unroll
       for (int i = 0; i < VPC; ++i) {
@@ -1175,6 +1202,9 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
   // tile their sums waited for it. Requests are unconditional (a wave without a tile asks for the block's last one, which another
   // wave reads): where paths with and without them meet, the compiler waits for every load in flight. The tile that the new token
   // goes into is asked for again behind the barrier.
+  // KL asks for a wave's own tile, once: its pieces go to LDS, in front of whose next access the compiler waits for all that is in
+  // flight anyway, and whole pages by waves without a tile, and again behind the barrier, were most of a short context's loads
+  // (512 pairs of 12 to 20 / 60 to 100 tokens 18.1 / 18.3 us, now 11.5 / 13.4).
   const int kt_first = min(kt0 + wid_u, kt1 - 1);
   if (rope) {
     request_item(it0);
@@ -1185,11 +1215,16 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
     for (int s = 0; s < C::KS; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qp + 32 * s);
   }
   __builtin_amdgcn_sched_barrier(0);
-  request_k(kt_first);
-  __builtin_amdgcn_sched_barrier(0);  // K before V: the scores and the softmax run while V is landing
-  request_v(kt_first);
-  __builtin_amdgcn_sched_barrier(0);
-  if (rope) {
+  auto request_first = [&]() __attribute__((always_inline)) {
+    request_k(kt_first);
+    __builtin_amdgcn_sched_barrier(0);  // K before V: the scores and the softmax run while V is landing
+    request_v(kt_first);
+  };
+  // now: asked for in front of the queries' sums; again: behind the append
+  auto prologue = [&](bool now, bool again) __attribute__((always_inline)) {
+    if (now) request_first();
+    __builtin_amdgcn_sched_barrier(0);
+    if (!rope) return;
     finish_item(it0);
     for (int i0 = NW * IPW; i0 < n_items; i0 += NW * IPW) {  // block-uniform
       request_item(i0 + it0);
@@ -1197,11 +1232,9 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
     }
     if (append) {
       __syncthreads();  // q in LDS; the appended row visible to every wave of this block (same CU)
-      if (kt_first == n_kt - 1) {
-        if constexpr (!REGS) wait_vmcnt0();  // (into the LDS that its first request fills)
-        request_k(kt_first);
-        __builtin_amdgcn_sched_barrier(0);
-        request_v(kt_first);
+      if (again) {
+        if constexpr (!REGS && !KL) wait_vmcnt0();  // (into the LDS that its first request fills)
+        request_first();
       }
     } else {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1209,6 +1242,10 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
     }
+  };
+  const bool mine = !KL || kt0 + wid_u < kt1, late = append && kt_first == n_kt - 1;
+  prologue(mine && (!KL || !late), mine && late);
+  if (rope) {
 #pragma unroll
     for (int s = 0; s < C::KS; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(s_q + min(fr, G - 1) * D + 32 * s + 8 * fh);
   }

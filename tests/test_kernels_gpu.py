@@ -532,6 +532,38 @@ def test_attn_decode_rope_single_partition_kl(native, kl, monkeypatch):
     assert rel_err(out.cpu().reshape(B, Hq, D), oracle) < 2e-2
 
 
+def _decode_against_oracle(native, kv_lens, Hq, Hkv, D, pt, mp):
+    """Both entry points of decode attention, the rotating one's appended rows among them."""
+    B = len(kv_lens)
+    torch.manual_seed(B)
+    kc, vc, bt = _paged_setup(kv_lens, Hkv, D, seed=7)
+    kvl = torch.tensor(kv_lens, dtype=torch.int32)
+    pos = kvl - 1
+    slots = (bt[torch.arange(B), (pos // 64).long()] * 64 + pos % 64).int().to(DEV)
+    P = torch.randn(2, B, (Hq + 2 * Hkv) * D, device=DEV)
+    cos, sin = (t.to(DEV) for t in R.rope_tables(D, 1024, theta=500000.0, scaling=None))
+    dev = [t.to(DEV) for t in (kc, vc, bt, kvl, pos)]
+    q, ref, out = (torch.full((B, Hq * D), float("nan"), device=DEV).bfloat16() for _ in range(3))
+    k2, v2 = dev[0].clone(), dev[1].clone()
+    native.rope_kv_partials(P, q, dev[4], cos, sin, slots, k2, v2, Hq, Hkv, D)
+    native.attn_decode(q, k2, v2, *dev[2:4], ref, Hq, Hkv, D, pt, mp)
+    native.attn_decode_rope(P, dev[4], cos, sin, slots, *dev[:4], out, Hq, Hkv, D, pt, mp)
+    assert torch.equal(dev[0], k2) and torch.equal(dev[1], v2)
+    k2, v2 = k2.cpu(), v2.cpu()
+    want = R.attention_varlen(q.cpu().reshape(B, Hq, D), None, None, torch.arange(B + 1, dtype=torch.int32), kvl, True,
+                              1 / math.sqrt(D), k_full=lambda s: R.paged_kv_view(k2, bt[s], kv_lens[s], 64),
+                              v_full=lambda s: R.paged_kv_view(v2, bt[s], kv_lens[s], 64))
+    # weights and outputs are rounded to bf16 (2^-8 of a value at most, independent: well under 2^-7 of the norm)
+    assert rel_err(ref.cpu().reshape(B, Hq, D), want) < 2 ** -7 and rel_err(out.cpu().reshape(B, Hq, D), want) < 2 ** -7
+
+
+@pytest.mark.parametrize("kv_lens", [[1], [64, 65, 128, 129], [192, 193, 256, 257, 320, 321]])
+def test_attn_decode_few_tiles_in_one_partition(native, kv_lens, monkeypatch):
+    """KL blocks of one tile to one more than they have waves: a wave without a tile, a first tile that the new token goes into."""
+    monkeypatch.setattr(native, "DECODE_NW8_MIN_PAIRS", 1)
+    _decode_against_oracle(native, kv_lens, 32, 8, 128, *native.decode_partitions(max(kv_lens), len(kv_lens), 8))
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(32, 8), (4, 1), (8, 1)])
 @pytest.mark.parametrize("kv_lens,target", [([1], 1024), ([5200, 1, 64, 65, 3000, 700], 1024), ([777, 129], 8)])
 def test_attn_decode_rope_matches_unfused(native, kv_lens, target, Hq, Hkv):

@@ -1538,8 +1538,9 @@ def decode_partitions(max_kv_len, batch, Hkv, target_blocks=None, min_tiles=None
     kernel's blocks lose by rounding down (seq_native.decode_parts).
 
     Once batch x KV heads would fill the CUs by itself, one partition per pair (attention.hip KL) where its rounds of one block a
-    CU are at least four fifths full, else three: 264 pairs of 1600 tokens 52.4 -> 45.2 us, 320 of 560 28.0 -> 23.7, 384 of 2400
-    87.5 -> 86.0, 400 of 1250 52.6 -> 51.1; 512 full ones of 3200 tokens 134 in one, 146 in three.
+    CU are at least four fifths full, else three, or as many as the longest context has keys for: 264 pairs of 1600 tokens 52.4 ->
+    45.2 us, 320 of 560 28.0 -> 23.7, 384 of 2400 87.5 -> 86.0, 400 of 1250 52.6 -> 51.1; 512 full ones of 3200 tokens 134 in one,
+    146 in three. A context without keys for the third leaves those blocks, two thirds of the workspace and the join to nothing.
 
     The kernel spreads each sequence's actual KV tiles evenly over the max_parts partitions (at least ``part_tiles`` tiles each,
     attention.hip:decode_part_units), so the grid can be sized once for the longest allowed context (hipGraph capture) without
@@ -1553,7 +1554,9 @@ def decode_partitions(max_kv_len, batch, Hkv, target_blocks=None, min_tiles=None
     pairs = batch * Hkv
     if DECODE_NW8_MIN_PAIRS > 0 and pairs >= DECODE_NW8_MIN_PAIRS:
         rounds = -(-pairs // DECODE_NW8_MIN_PAIRS)
-        return part_tiles, 1 if 5 * pairs >= 4 * rounds * DECODE_NW8_MIN_PAIRS else 3
+        if 5 * pairs >= 4 * rounds * DECODE_NW8_MIN_PAIRS:
+            return part_tiles, 1
+        return part_tiles, min(3, -(-max_kt // min_tiles))
     return part_tiles, max(1, min(target_blocks // pairs, -(-max_kt // min_tiles)))
 
 

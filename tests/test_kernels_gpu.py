@@ -564,6 +564,17 @@ def test_attn_decode_few_tiles_in_one_partition(native, kv_lens, monkeypatch):
     _decode_against_oracle(native, kv_lens, 32, 8, 128, *native.decode_partitions(max(kv_lens), len(kv_lens), 8))
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,B,longest,parts", [(128, 32, 8, 33, 700, 3), (128, 8, 4, 80, 900, 3), (64, 16, 4, 66, 513, 3),
+                                                      (128, 32, 8, 33, 500, 2), (128, 32, 8, 33, 256, 1)])
+def test_attn_decode_more_pairs_than_cus(native, D, Hq, Hkv, B, longest, parts):
+    """From 256 (sequence, KV head) pairs on whose last round of one block a CU would be mostly empty: three partitions, fewer
+    where the longest context has no keys for them. Lengths around the units' and pages' ends, both entry points."""
+    kv_lens = ([longest, 1, 32, 33, 64, 65, 95, 97, 128, 129, 192, 193, 255, 256] + [1 + 53 * i % longest for i in range(B)])[:B]
+    pt, mp = native.decode_partitions(longest, B, Hkv)
+    assert mp == parts
+    _decode_against_oracle(native, kv_lens, Hq, Hkv, D, pt, mp)
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(32, 8), (4, 1), (8, 1)])
 @pytest.mark.parametrize("kv_lens,target", [([1], 1024), ([5200, 1, 64, 65, 3000, 700], 1024), ([777, 129], 8)])
 def test_attn_decode_rope_matches_unfused(native, kv_lens, target, Hq, Hkv):

@@ -77,16 +77,19 @@ def test_split_chunks_partitions_the_token_stream(ns, parts):
 @settings(max_examples=300, deadline=None)
 @given(max_len=st.integers(1, 131072), batch=st.integers(1, 256), hkv=st.sampled_from([1, 2, 4, 8]),
        kv_len=st.integers(1, 131072))
-def test_decode_partitions_cover_every_tile(max_len, batch, hkv, kv_len):
-    """attention.hip:decode_part_tiles: with the planner's (part_tiles, max_parts), every sequence's
-    KV tiles fall in the launched partitions, each partition non-empty."""
+def test_decode_partitions_cover_every_unit(max_len, batch, hkv, kv_len):
+    """attention.hip:decode_part_units: with the planner's (part_tiles, max_parts), every sequence's keys fall in the launched
+    partitions, each partition non-empty: units of 32 keys, and of 64 where one partition takes whole tiles (KL)."""
     from rag_llm_k8s_amd.ops.native import decode_partitions
 
     kv_len = min(kv_len, max_len)
     pt, mp = decode_partitions(max_len, batch, hkv)
     assert pt >= 1 and mp >= 1
-    n_kt = -(-kv_len // 64)
-    eff = max(pt, -(-n_kt // mp))
-    nparts = -(-n_kt // eff)
-    assert 1 <= nparts <= mp
-    assert (nparts - 1) * eff < n_kt <= nparts * eff
+    for unit in (32, 64) if mp == 1 else (32,):
+        n = -(-kv_len // unit)
+        eff = max(pt * (64 // unit), -(-n // mp))
+        nparts = -(-n // eff)
+        assert 1 <= nparts <= mp
+        assert (nparts - 1) * eff < n <= nparts * eff
+    # no partition that only a longer context than the longest could fill
+    assert mp == 1 or (mp - 1) * pt * 64 < max_len

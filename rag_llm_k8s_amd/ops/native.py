@@ -1541,6 +1541,9 @@ def decode_partitions(max_kv_len, batch, Hkv, target_blocks=None, min_tiles=None
     CU are at least four fifths full, else three, or as many as the longest context has keys for: 264 pairs of 1600 tokens 52.4 ->
     45.2 us, 320 of 560 28.0 -> 23.7, 384 of 2400 87.5 -> 86.0, 400 of 1250 52.6 -> 51.1; 512 full ones of 3200 tokens 134 in one,
     146 in three. A context without keys for the third leaves those blocks, two thirds of the workspace and the join to nothing.
+    Where all three are at work in more than two and a quarter rounds, short contexts fill fewer, larger ones: three tiles at least,
+    not two (384 pairs of 150 / 300 / 600 tokens 17.0 / 21.5 / 26.3 us -> 13.0 / 18.2 / 26.3, 408 of 200 / 300 20.1 / 22.7 -> 16.8
+    / 21.1; below, 264 of 200 / 600 14.7 / 19.8 against 16.2 / 21.6).
 
     The kernel spreads each sequence's actual KV tiles evenly over the max_parts partitions (at least ``part_tiles`` tiles each,
     attention.hip:decode_part_units), so the grid can be sized once for the longest allowed context (hipGraph capture) without
@@ -1556,6 +1559,8 @@ def decode_partitions(max_kv_len, batch, Hkv, target_blocks=None, min_tiles=None
         rounds = -(-pairs // DECODE_NW8_MIN_PAIRS)
         if 5 * pairs >= 4 * rounds * DECODE_NW8_MIN_PAIRS:
             return part_tiles, 1
+        if 4 * 3 * pairs >= 9 * target_blocks:
+            part_tiles = max(1, 3 * min_tiles // 4)
         return part_tiles, min(3, -(-max_kt // min_tiles))
     return part_tiles, max(1, min(target_blocks // pairs, -(-max_kt // min_tiles)))
 

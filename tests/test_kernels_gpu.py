@@ -565,7 +565,8 @@ def test_attn_decode_few_tiles_in_one_partition(native, kv_lens, monkeypatch):
 
 
 @pytest.mark.parametrize("D,Hq,Hkv,B,longest,parts", [(128, 32, 8, 33, 700, 3), (128, 8, 4, 80, 900, 3), (64, 16, 4, 66, 513, 3),
-                                                      (128, 32, 8, 33, 500, 2), (128, 32, 8, 33, 256, 1)])
+                                                      (128, 32, 8, 33, 500, 2), (128, 32, 8, 33, 256, 1),
+                                                      (128, 32, 8, 48, 700, 3)])
 def test_attn_decode_more_pairs_than_cus(native, D, Hq, Hkv, B, longest, parts):
     """From 256 (sequence, KV head) pairs on whose last round of one block a CU would be mostly empty: three partitions, fewer
     where the longest context has no keys for them. Lengths around the units' and pages' ends, both entry points."""

@@ -46,6 +46,7 @@ def test_short_sequence(native, monkeypatch, T, hidden, heads, inter, pooling, k
     if T == 2:
         m.w.type_row = None
     monkeypatch.setattr(native, "FEW_SIZE", 10 ** 9)
+    assert native.encoder_pointers(cfg, m.w) is not None  # else the call below goes layer by layer
     ids = np.random.RandomState(T).randint(0, 500, T + 1).astype(np.int32)[1:]
     assert native.encoder_few_ok(cfg, T, 1) and not native.encoder_few_ok(cfg, 33, 1) and not native.encoder_few_ok(cfg, T, 2)
     out = torch.full((3, hidden), 9.0, device=DEV)
@@ -61,11 +62,22 @@ def test_short_sequence(native, monkeypatch, T, hidden, heads, inter, pooling, k
     assert err[0] < 0.01 and err[0] < 1.3 * err[1] + 1e-4, err
 
 
-# the widths between (a kernel for each), and as many columns of a down projection as the arguments can name
+# the widths between (a kernel for each), and as many columns of a down projection as the call takes (encoder_pointers)
 @pytest.mark.parametrize("T", [3, 17])
-@pytest.mark.parametrize("hidden,heads,inter", [(256, 8, 256), (768, 12, 3072), (896, 14, 1152), (384, 6, 2048), (128, 2, 32768)])
+@pytest.mark.parametrize("hidden,heads,inter", [(256, 8, 256), (768, 12, 3072), (896, 14, 1152), (384, 6, 2048), (128, 2, 16256)])
 def test_every_width(native, monkeypatch, T, hidden, heads, inter):
     test_short_sequence(native, monkeypatch, T, hidden, heads, inter, "mean", "bert")
+
+
+@pytest.mark.parametrize("T", [3, 17])
+def test_more_columns_than_the_call_takes(native, T):
+    cfg = E.EncoderConfig(model_type="bert", vocab_size=500, hidden_size=128, num_hidden_layers=2, num_attention_heads=2,
+                          intermediate_size=32768, max_position_embeddings=64, pooling="mean")
+    m = E.EncoderModel(cfg, E.EncoderWeights.random(cfg, DEV, seed=T), DEV)
+    assert native.encoder_pointers(cfg, m.w) is None
+    ids = torch.from_numpy(np.random.RandomState(T).randint(0, 500, T).astype(np.int32)).to(DEV)
+    ref = exact(cfg, m.w, ids.long(), m.first_position)
+    assert ((m.forward_packed(ids, [T]).to(F64) - ref).norm() / ref.norm()).item() < 0.01  # (test_short_sequence)
 
 
 def test_no_layers(native):

@@ -559,7 +559,7 @@ RAGK_API int ragk_gemm_mid(const void* A, int lda, const void* B, int ldb, void*
 }
 
 RAGK_API int ragk_gemm_stream_part(const void* X, int ldx, const void* W, int ldw, float* P, int M, int N, int K, int S,
-                                   int rows, hipStream_t st);
+                                   int rows, int short_sums, hipStream_t st);
 
 // C = epilogue of the sum of P's S fp32 slabs [M][weight rows]. C, bias and resid rows start on 16 bytes, N % 8 == 0.
 RAGK_API int ragk_slabs_finish(const float* P, int S, void* C, int ldc, const void* bias, const void* resid, int ldr, int M,
@@ -583,7 +583,7 @@ RAGK_API int ragk_gemm_slabs(const void* X, int ldx, const void* W, int ldw, voi
                              hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
   if (N % 8 || epi_pair(epi) || !ws) return (int)hipErrorInvalidValue;
-  const int rc = ragk_gemm_stream_part(X, ldx, W, ldw, ws, M, N, K, S, rows, st);
+  const int rc = ragk_gemm_stream_part(X, ldx, W, ldw, ws, M, N, K, S, rows, 1, st);
   return rc ? rc : ragk_slabs_finish(ws, S, C, ldc, bias, resid, ldr, M, N, epi, out_f32, st);
 }
 

@@ -144,7 +144,8 @@ __device__ __forceinline__ void stage_load(const bf16_t* __restrict__ X, int ldx
 // DG = 1 (diagnostic, tools/stream_gemm_probe.py): the ring, its waits and barriers, no fragment reads or MFMA
 // (results meaningless) -- how fast the weight stream itself runs in this kernel's structure. DG = 2: also
 // no activation staging (weights only); DG = 3: as 2 without the per-stage barrier.
-template <int MT, int EPI, bool OUT_F32, bool FP8, bool NT = false, int ROWS = WROWS, bool SLAB = false, int DG = 0>
+// SEG (slabs): so many K-steps to a sum, the sums added up at their ends.
+template <int MT, int EPI, bool OUT_F32, bool FP8, bool NT = false, int ROWS = WROWS, bool SLAB = false, int DG = 0, int SEG = 0>
 __global__ __launch_bounds__(ST_THREADS, ROWS == 64 ? 2 : 1) void gemm_stream_kernel(
     const bf16_t* __restrict__ X, int ldx, const void* __restrict__ Wv, int ldw, const float* __restrict__ wscale,
     void* C, int ldc, const bf16_t* __restrict__ bias, const bf16_t* resid, int ldr, int M, int N, int K, int S,
@@ -167,16 +168,18 @@ __global__ __launch_bounds__(ST_THREADS, ROWS == 64 ? 2 : 1) void gemm_stream_ke
   const int k0 = slice * nst * G::KSTEP;
 
   // bf16 without slabs: a K-step's halves in sums of their own, so that a sum over all of K is no longer than where K was cut in
-  // two (normal numbers, rms error of fp32 results: 8 x 18560 x 4096 3.96e-7 -> 2.72e-7, as fast). Slabs, whose sums are short,
-  // keep one: two cost them 1 % at 33 rows and more.
+  // two (normal numbers, rms error of fp32 results: 8 x 18560 x 4096 3.96e-7 -> 2.72e-7, as fast). Slabs keep one, or (SEG) one
+  // for every few steps of K.
   constexpr int AC = FP8 || SLAB ? 1 : 2;
-  f32x4 acc[AC][MT][J];
+  f32x4 acc[AC][MT][J], total[SEG ? MT : 1][J];
 #pragma unroll
-  for (int a = 0; a < AC; ++a)
+  for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+    for (int j = 0; j < J; ++j) {
 #pragma unroll
-      for (int j = 0; j < J; ++j) acc[a][t][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int a = 0; a < AC; ++a) acc[a][t][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      if constexpr (SEG) total[t][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
 
   // prologue: NS-1 stages in flight
 #pragma unroll
@@ -242,6 +245,17 @@ __global__ __launch_bounds__(ST_THREADS, ROWS == 64 ? 2 : 1) void gemm_stream_ke
         }
       }
     }
+    if constexpr (SEG) {
+      if (t % SEG == SEG - 1 || t == nst - 1) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int j = 0; j < J; ++j) {
+            total[m][j] += acc[0][m][j];
+            acc[0][m][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+          }
+      }
+    }
   }
 
   // ---------------- epilogue: partial tile -> LDS [16 MT][ROWS] f32 ----------------------
@@ -254,8 +268,10 @@ __global__ __launch_bounds__(ST_THREADS, ROWS == 64 ? 2 : 1) void gemm_stream_ke
 #pragma unroll
     for (int j = 0; j < J; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        sC[(16 * m + 4 * fh + r) * G::EPI_LD + wid * (ROWS / 4) + 16 * j + fr] = AC == 2 ? acc[0][m][j][r] + acc[AC - 1][m][j][r] : acc[0][m][j][r];
+      for (int r = 0; r < 4; ++r) {
+        const float v = SEG ? total[SEG ? m : 0][j][r] : AC == 2 ? acc[0][m][j][r] + acc[AC - 1][m][j][r] : acc[0][m][j][r];
+        sC[(16 * m + 4 * fh + r) * G::EPI_LD + wid * (ROWS / 4) + 16 * j + fr] = v;
+      }
   __syncthreads();
   if constexpr (SLAB) {
     float* ps = reinterpret_cast<float*>(C) + (size_t)slice * M * N;
@@ -404,18 +420,21 @@ int launch_stream(const void* X, int ldx, const void* W, int ldw, const float* w
   return (int)hipGetLastError();
 }
 
-template <int MT>
-int launch_stream_slab(const void* X, int ldx, const void* W, int ldw, float* P, int M, int N, int K, int S, int rows,
+// short_sums: 512 of K to a sum, as the register-streaming kernel cuts K = 4096 (rms error of 64 x 14336 x 4096 in two slabs 2.72e-7
+// -> 1.35e-7; 28.9 / 29.2 us). What decode steps' consumers sum has one sum a slab.
+constexpr int SLAB_SEG = 8;
+
+template <int MT, int R>
+int launch_stream_slab(const void* X, int ldx, const void* W, int ldw, float* P, int M, int N, int K, int S, int short_sums,
                        hipStream_t st) {
-  const dim3 grid((N + rows - 1) / rows, S);
+  const dim3 grid((N + R - 1) / R, S);
   // non-temporal weight stream (each weight byte is read once per step)
-  if (rows == 64)
-    hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI_NONE, true, false, true, 64, true>), grid, dim3(ST_THREADS), 0, st,
+  if (short_sums)
+    hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI_NONE, true, false, true, R, true, 0, SLAB_SEG>), grid, dim3(ST_THREADS), 0, st,
                        (const bf16_t*)X, ldx, W, ldw, nullptr, P, N, nullptr, nullptr, 0, M, N, K, S, nullptr, nullptr);
   else
-    hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI_NONE, true, false, true, WROWS, true>), grid, dim3(ST_THREADS), 0,
-                       st, (const bf16_t*)X, ldx, W, ldw, nullptr, P, N, nullptr, nullptr, 0, M, N, K, S, nullptr,
-                       nullptr);
+    hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI_NONE, true, false, true, R, true>), grid, dim3(ST_THREADS), 0, st,
+                       (const bf16_t*)X, ldx, W, ldw, nullptr, P, N, nullptr, nullptr, 0, M, N, K, S, nullptr, nullptr);
   return (int)hipGetLastError();
 }
 
@@ -514,15 +533,18 @@ RAGK_API int ragk_gemm_stream(const void* X, int ldx, const void* W, int ldw, co
 // Split-K partial slabs P[S][M][N] (fp32) of X[M,K] . W[N,K]^T through the LDS-DMA weight ring (SLAB
 // above): bf16 weights, M <= 64, N % 4 == 0, S | K / 64, rows = 64 (two blocks per CU) or 128.
 RAGK_API int ragk_gemm_stream_part(const void* X, int ldx, const void* W, int ldw, float* P, int M, int N, int K,
-                                   int S, int rows, hipStream_t st) {
+                                   int S, int rows, int short_sums, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 64 || K % 64 || S < 1 || (K / 64) % S || N % 4 || (rows != 64 && rows != 128) || ldx % 8 || ldw % 8)
     return (int)hipErrorInvalidValue;
+#define RAGK_SLAB(MT)                                                                                    \
+  return rows == 64 ? launch_stream_slab<MT, 64>(X, ldx, W, ldw, P, M, N, K, S, short_sums, st)          \
+                    : launch_stream_slab<MT, WROWS>(X, ldx, W, ldw, P, M, N, K, S, short_sums, st)
   switch ((M + 15) / 16) {
-    case 1: return launch_stream_slab<1>(X, ldx, W, ldw, P, M, N, K, S, rows, st);
-    case 2: return launch_stream_slab<2>(X, ldx, W, ldw, P, M, N, K, S, rows, st);
-    case 3: return launch_stream_slab<3>(X, ldx, W, ldw, P, M, N, K, S, rows, st);
-    case 4: return launch_stream_slab<4>(X, ldx, W, ldw, P, M, N, K, S, rows, st);
-    default: return (int)hipErrorInvalidValue;
+    case 1: RAGK_SLAB(1);
+    case 2: RAGK_SLAB(2);
+    case 3: RAGK_SLAB(3);
+    default: RAGK_SLAB(4);
   }
+#undef RAGK_SLAB
 }

@@ -14,6 +14,7 @@ MI355X-first design:
 """
 from __future__ import annotations
 
+import functools
 import json
 import math
 import os
@@ -398,16 +399,17 @@ class LlamaModel(DecoderModel):
         be, w, c = self.be, self.w, self.cfg
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
         layers = w.layers
+        part = functools.partial(be.gemm_part, short_sums=True)
         q = torch.empty_like(attn)
         xn = be.rmsnorm(h, layers[0]["ln_in"], c.rms_norm_eps)
         for li, L in enumerate(layers):
             kc, vc = self.kv_cache[li]
-            be.rope_kv_partials(be.gemm_part(xn, L["wqkv"]), q, inp.positions, self.cos, self.sin, inp.slots, kc, vc, Hq, Hkv, D)
+            be.rope_kv_partials(part(xn, L["wqkv"]), q, inp.positions, self.cos, self.sin, inp.slots, kc, vc, Hq, Hkv, D)
             be.attn_prefill(q, kc, vc, inp.meta, attn, Hq, Hkv, D)
-            xn = be.add_partials_rmsnorm(be.gemm_part(attn, L["wo"]), h, L["ln_post"], c.rms_norm_eps, rounded=False)
+            xn = be.add_partials_rmsnorm(part(attn, L["wo"]), h, L["ln_post"], c.rms_norm_eps, rounded=False)
             a = be.gemm(xn, L["wgu"], epi="silu_mul")
             nxt = layers[li + 1]["ln_in"] if li + 1 < len(layers) else w.norm
-            xn = be.add_partials_rmsnorm(be.gemm_part(a, L["wdown"]), h, nxt, c.rms_norm_eps, rounded=False)
+            xn = be.add_partials_rmsnorm(part(a, L["wdown"]), h, nxt, c.rms_norm_eps, rounded=False)
         return xn if inp.logits_idx is None else be.gather_rows(xn, inp.logits_idx)
 
     def hidden_states_splitk(self, inp: StepInput, h, attn, ns_o, ns_d):

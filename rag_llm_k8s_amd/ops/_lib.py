@@ -50,7 +50,7 @@ _SIGS = {
     "ragk_gemm_hold_slabs": [P, I, P, I, P, P, I, I, I, I, S],
     "ragk_gemm_hold_slabs_silu": [P, I, P, I, P, P, I, I, I, I, I, P, S],
     "ragk_gemm_slabs": [P, I, P, I, P, I, P, P, I, I, I, I, I, I, I, I, P, S],
-    "ragk_gemm_stream_part": [P, I, P, I, P, I, I, I, I, I, S],
+    "ragk_gemm_stream_part": [P, I, P, I, P, I, I, I, I, I, I, S],
     "ragk_gemm_part_silu": [P, I, P, I, P, I, I, I, I, S],
     "ragk_gemm_part_silu_ok": [I, I, I, I],
     "ragk_mlp_engine_ok": [I, I, I, I],

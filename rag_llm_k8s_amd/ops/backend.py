@@ -134,7 +134,7 @@ class TorchBackend:
     def part_ok(self, M, w):
         return self.enable_part and M <= 64
 
-    def gemm_part(self, x, w):
+    def gemm_part(self, x, w, short_sums=False):
         wf = w.dequant() if isinstance(w, Fp8Weight) else w.float()
         return (x.float() @ wf.t()).unsqueeze(0)
 
@@ -398,8 +398,8 @@ class NativeBackend(TorchBackend):
             return False
         return self.n.gemm_part_slabs(M, w.shape[0], w.shape[1])[1] > 0
 
-    def gemm_part(self, x, w):
-        return self.n.gemm_part(x, w)
+    def gemm_part(self, x, w, short_sums=False):
+        return self.n.gemm_part(x, w, short_sums=short_sums)
 
     def part_norm_ok(self, M, w):
         return self.enable_part and M <= 4 and not isinstance(w, Fp8Weight) and w.shape[1] in (4096, 8192)

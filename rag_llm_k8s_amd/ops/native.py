@@ -96,8 +96,9 @@ def use_slabs(M, N, K, epi, out_f32=False):
     this rule cost the host 7 us, so not where the GPU gains little more (20 rows: 6144 x 4096 22 against 14, 4096 x 4096 14
     against 11; a rolesun step of 694 us became 723), nor below 2^24 weights, where the step's launches bound it (2048 x 5632 at
     20 rows 16.6 against 9.4, but the steps that hold it 368 -> 409 and 508 -> 557 us); up to 16 rows the second launch takes
-    what the first gains. Slabs are longer sums than the other kernel's, which cuts K eight times (64 x 6144 x 4096, rms
-    error of fp32 results 1.9e-7 against 1.4e-7; rounded to bf16 1.6605e-3 both): not for fp32 results."""
+    what the first gains. The other kernel cuts K eight times; a slab is a sum of sums over 512 of K here, so that it is no further
+    off (rms error of fp32 sums, other kernel / slabs / slabs of one sum: 64 x 6144 x 4096 1.37 / 1.34 / 1.89e-7, 14336 x 4096
+    1.37 / 1.35 / 2.72e-7, 10240 x 8192 1.93 / 1.40 / 3.96e-7; 2 to 4 % of the stream's time). fp32 results keep the one launch."""
     return (not out_f32 and 16 < M <= 64 and K >= 4096 and K % 128 == 0 and N % 8 == 0 and epi not in PAIR_EPI
             and N * K >= 1 << 24 and M * N * K >= 8e8 and stream_part_cfg(M, N, K)[1] > 1)
 
@@ -552,8 +553,9 @@ def _stream_part_cfg(N, K, cus, only, max_s):
     return best[0], best[1]
 
 
-def gemm_stream_part(x, w, out=None, rows=None, S=None):
-    """Partial slabs P[S, M, N] (fp32) with P.sum(0) = x @ w^T from the LDS-DMA stream GEMM (bf16 weights)."""
+def gemm_stream_part(x, w, out=None, rows=None, S=None, short_sums=False):
+    """Partial slabs P[S, M, N] (fp32) with P.sum(0) = x @ w^T from the LDS-DMA stream GEMM (bf16 weights). short_sums: a slab is
+    the sum of sums over 512 of K."""
     _bf16_2d(x, "x")
     _bf16_2d(w, "w")
     M, K = x.shape
@@ -565,15 +567,16 @@ def gemm_stream_part(x, w, out=None, rows=None, S=None):
     if out is None:
         out = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
     check(_lib.lib().ragk_gemm_stream_part(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), M, N,
-                                           K, S, rows, stream_ptr()), "ragk_gemm_stream_part")
+                                           K, S, rows, int(short_sums), stream_ptr()), "ragk_gemm_stream_part")
     return out
 
 
-def gemm_part(x, w, out=None, ks=None):
+def gemm_part(x, w, out=None, ks=None, short_sums=False):
     """Decode GEMM v5 (csrc/kernels/gemm_part.hip): fp32 split-K partials P[S, M, N] with
     P.sum(0) = x @ w^T. The consumer (add_partials_rmsnorm / rope_kv_partials) does the reduction.
     w: bf16 [N, K], or an :class:`ops.fp8.Fp8Weight` (W8A16: e4m3fn rows, per-row scale applied to
-    the partials)."""
+    the partials). short_sums: for results that were products of rows before, whose sums were no longer than 512 of K = 4096
+    (gemm_stream_part)."""
     from .fp8 import Fp8Weight
 
     _bf16_2d(x, "x")
@@ -589,7 +592,7 @@ def gemm_part(x, w, out=None, ks=None):
     _req(wt.shape[1] == K and M <= 64, "gemm_part shape %s x %s" % (tuple(x.shape), tuple(wt.shape)))
     if (STREAM_PART and not fp8 and ks is None and out is None and M >= STREAM_PART_MIN_M and K % 64 == 0
             and N % 4 == 0 and stream_part_cfg(M, N, K)[1] > 0):
-        return gemm_stream_part(x, wt)
+        return gemm_stream_part(x, wt, short_sums=short_sums)
     if fp8 and ks is None and out is None and use_hold_slabs(M, N, K) and _vec_rows(x, wt):
         return gemm_hold_slabs(x, wt, w.scale)
     ks, S = gemm_part_slabs(M, N, K, ks)

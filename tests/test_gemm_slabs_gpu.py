@@ -38,6 +38,23 @@ def test_slabs(native, M, N, K):
     assert torch.equal(native.gemm(x, w, resid=r, epi="resid", out=r), want)  # the residual in place
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 14336, 4096), (33, 6144, 4096), (64, 10240, 8192), (50, 4096, 14336), (20, 5120, 5120)])
+def test_slab_sums(native, M, N, K):
+    """Sums of products of rows are no further off in slabs than in one launch (gemm), and gemm's slabs are these."""
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+    w = (torch.randn(N, K, device=DEV, generator=g) / K ** 0.5).bfloat16()
+    ref = x.double() @ w.double().t()
+    P = native.gemm_part(x, w, short_sums=True)
+    err = [float((y.double() - ref).norm()) for y in (P.sum(0), native.gemm(x, w, out_f32=True))]
+    assert err[0] < 1.02 * err[1]  # (a hundred thousand sums: their rms error is known to well under 1 %)
+    if native.use_slabs(M, N, K, "none"):
+        y = P[0]
+        for p in P[1:]:
+            y = y + p
+        assert torch.equal(native.gemm(x, w), y.bfloat16())
+
+
 def test_unaligned_rows_keep_their_kernel(native):
     """Rows off 16 bytes, which the slabs' loads and stores cannot take, go where they went."""
     M, N, K = 33, 6144, 4096

@@ -18,7 +18,9 @@
 // before and after: fp8 28672 x 4096 (117 MB) at 11 / 32 rows 26.8 / 32.5 -> 25.8 / 31.2 (4.6 TB/s), 14336 x 4096 17.1 / 21.6 ->
 // 15.4 / 20.5, 11264 x 2048 8.1 / 10.6 -> 7.5 / 10.0; bf16 11264 x 2048 (46 MB) at 12 / 32 / 64 rows 11.6 / 14.3 / 17.7 -> 11.1 /
 // 13.1 / 17.7 (a block has three tiles there, and a spare load of a fourth would cost 0.5 us: it keeps the branch). Two tiles of
-// 64 KB in flight, not three: 27.4 -> 25.9.
+// 64 KB in flight, not three: 27.4 -> 25.9. No more tiles are in flight than a block has, since each spare one is loaded all the
+// same: bf16 1024 x 4096 at 1 / 16 rows 10.2 / 12.9 -> 6.9 / 9.6, 4096 x 4096 12.1 / 14.9 -> 9.4 / 11.1, fp8 2048 x 2048 5.4 / 6.7
+// -> 4.2 / 5.5, 16384 x 3072 (four tiles, two in flight for three) 12.5 / 13.5 -> 10.3 / 11.4.
 //
 // More rows than the registers hold (64 of K = 4096 would be a CU's whole register file): SLAB deals the blocks to slabs of 2048
 // of K, each with its part of x, and writes fp32 partials of plain weight rows. fp8 28672 x 4096 at 33 / 64 rows: two launches
@@ -56,14 +58,13 @@ constexpr int hold_depth(int MT, int KI, bool FP8) {
   return hold_regs(MT, KI, FP8, 3) <= HREGS && KI * (FP8 ? 1 : 2) < 4 ? 3 : 2;
 }
 
-// KI = K / 1024 of a launch (SLAB: of a slab). par: fp32 {limit, alpha, shift} of EPI_GLU_CLIP. SLAB: fp32 slabs P[S][M][ldc]
-// of plain weight rows instead, slab blockIdx.y.
-template <int MT, int KI, bool FP8, int EPI, bool SLAB>
+// KI = K / 1024 of a launch (SLAB: of a slab), NB tiles in flight. par: fp32 {limit, alpha, shift} of EPI_GLU_CLIP. SLAB: fp32 slabs
+// P[S][M][ldc] of plain weight rows instead, slab blockIdx.y.
+template <int MT, int KI, bool FP8, int EPI, bool SLAB, int NB>
 __global__ __launch_bounds__(HW * 64, 2) void gemm_hold_kernel(const bf16_t* __restrict__ X, int ldx,
                                                               const unsigned char* __restrict__ W, size_t ldw_bytes,
                                                               const float* __restrict__ sw, void* C, int ldc,
                                                               const bf16_t* __restrict__ par, int M, int tiles, int share) {
-  constexpr int NB = hold_depth(MT, KI, FP8);
   constexpr int L = FP8 ? 2 : 4;     // 16-byte loads of a chunk: 64 contiguous bytes of each row
   constexpr int EB = FP8 ? 1 : 2;
   __shared__ __attribute__((aligned(16))) f32x4 red[2][HW][MT][64];
@@ -105,12 +106,12 @@ __global__ __launch_bounds__(HW * 64, 2) void gemm_hold_kernel(const bf16_t* __r
   }
 #pragma unroll
   for (int b = 1; b < NB; ++b) load(wv[b], min(t0 + b, t1 - 1));  // behind x: the first tile waits for neither
-  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (NB > 1) __builtin_amdgcn_sched_barrier(0);
   if constexpr (FP8)
 #pragma unroll
     for (int j = 0; j < HTILES / 32; ++j) scale[32 * j + (threadIdx.x >> 4)][fr] = sc[j];
   const GluPar gp = glu_par<EPI>(par);
-  if constexpr (!FP8) {  // x is here before the loop, whose waits would else be for the prologue's order of loads
+  if (!FP8 && NB > 1 && t0 + NB < t1) {  // x is here before the loop, whose waits would else be for the prologue's order of loads
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -171,14 +172,26 @@ __global__ __launch_bounds__(HW * 64, 2) void gemm_hold_kernel(const bf16_t* __r
 // Blocks that share the tiles: one a CU, more where theirs would be more than HTILES.
 int hold_share(int tiles, int blocks) { return max(min(tiles, blocks), (tiles + HTILES - 1) / HTILES); }
 
+// Tiles in flight, at most hold_depth: no more than the largest share has, and two of four where three would ask for two spare ones.
+template <int DEPTH, typename F>
+int hold_with_depth(int tiles, int share, F f) {
+  const int per = (tiles + share - 1) / share;
+  if (per == 1) f(std::integral_constant<int, 1>{});
+  else if (DEPTH == 2 || per == 2 || per == 4) f(std::integral_constant<int, 2>{});
+  else f(std::integral_constant<int, DEPTH>{});
+  return (int)hipGetLastError();
+}
+
 template <int MT, int KI, bool FP8, int EPI>
 int launch_hold(const void* X, int ldx, const void* W, int ldw, const float* sw, void* C, int ldc, const void* par, int M,
                 int N, int blocks, hipStream_t st) {
   if constexpr (hold_regs(MT, KI, FP8, 2) <= HREGS) {
     const int tiles = N / 8, share = hold_share(tiles, blocks);
-    hipLaunchKernelGGL((gemm_hold_kernel<MT, KI, FP8, EPI, false>), dim3(share), dim3(HW * 64), 0, st, (const bf16_t*)X, ldx,
-                       (const unsigned char*)W, (size_t)ldw * (FP8 ? 1 : 2), sw, C, ldc, (const bf16_t*)par, M, tiles, share);
-    return (int)hipGetLastError();
+    return hold_with_depth<hold_depth(MT, KI, FP8)>(tiles, share, [&](auto nb) {
+      hipLaunchKernelGGL((gemm_hold_kernel<MT, KI, FP8, EPI, false, decltype(nb)::value>), dim3(share), dim3(HW * 64), 0, st,
+                         (const bf16_t*)X, ldx, (const unsigned char*)W, (size_t)ldw * (FP8 ? 1 : 2), sw, C, ldc, (const bf16_t*)par,
+                         M, tiles, share);
+    });
   } else {
     return (int)hipErrorInvalidValue;
   }
@@ -246,17 +259,19 @@ RAGK_API int ragk_gemm_hold_slabs(const void* X, int ldx, const void* W, int ldw
   const int S = K / 2048;
   if (M > 64 || K <= 0 || K % 2048 || N % 16 || S > blocks || ldx % 8 || ldw % 16 || ldw >= HOLD_LDW || !sw) return (int)hipErrorInvalidValue;
   const int share = hold_share(N / 16, blocks / S);
-#define RAGK_HS(MT)                                                                                                          \
-  hipLaunchKernelGGL((gemm_hold_kernel<MT, 2, true, EPI_NONE, true>), dim3(share, S), dim3(HW * 64), 0, st, (const bf16_t*)X, \
-                     ldx, (const unsigned char*)W, (size_t)ldw, sw, P, N, nullptr, M, N / 16, share)
+  auto launch = [&](auto mt) {
+    constexpr int MT = decltype(mt)::value;
+    return hold_with_depth<hold_depth(MT, 2, true)>(N / 16, share, [&](auto nb) {
+      hipLaunchKernelGGL((gemm_hold_kernel<MT, 2, true, EPI_NONE, true, decltype(nb)::value>), dim3(share, S), dim3(HW * 64), 0, st,
+                         (const bf16_t*)X, ldx, (const unsigned char*)W, (size_t)ldw, sw, P, N, nullptr, M, N / 16, share);
+    });
+  };
   switch ((M + 15) / 16) {
-    case 1: RAGK_HS(1); break;
-    case 2: RAGK_HS(2); break;
-    case 3: RAGK_HS(3); break;
-    default: RAGK_HS(4); break;
+    case 1: return launch(std::integral_constant<int, 1>{});
+    case 2: return launch(std::integral_constant<int, 2>{});
+    case 3: return launch(std::integral_constant<int, 3>{});
+    default: return launch(std::integral_constant<int, 4>{});
   }
-#undef RAGK_HS
-  return (int)hipGetLastError();
 }
 
 // The packed gate/up projection (2 N rows of W) through those slabs and a pass that sums and pairs them.

@@ -63,7 +63,7 @@ def test_gate_up(native, N, K):
 
 
 @pytest.mark.parametrize("fp8", [True, False])
-@pytest.mark.parametrize("N", [64, 192, 1088, 4160])
+@pytest.mark.parametrize("N", [64, 192, 256, 1088, 4160])
 def test_pair_shares(native, N, fp8):
     """The paired form over few blocks: tiles that fill their rounds or leave some."""
     L = native._lib.lib()

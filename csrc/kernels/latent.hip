@@ -404,14 +404,14 @@ struct OutArgs {
 // further partitions behind the weights of the join, which are exponentials of values read once (they were read three times).
 // One sequence's few columns are joined by several threads each. Steps of four layers, us before and after: 1 x 4000 tokens,
 // 4096 wide 620.6 -> 613.5, 3 x 2000 639.5 -> 636.2, 2048 wide 50 x 1000 370 -> 365. From eight sequences a block the
-// partitions' stream bounds it, and asking ahead for what may not be there loses (40 x 3000 820 -> 832).
-template <typename TP, int NR, int NB>
+// partitions' stream bounds it, and asking ahead for what may not be there loses (40 x 3000 820 -> 832), and so do the registers that
+// it takes where there are more blocks than CUs (AHEAD: not there; 17 x 300, 4096 wide, 320 blocks: 676 ahead, 648).
+template <typename TP, int NR, int NB, bool AHEAD = false>
 __global__ __launch_bounds__(256) void latent_out_kernel(OutArgs<TP> a) {
   constexpr int Rp = 128 * NR, KS = Rp / 32, ST = Rp + 8, TT = LatentTile<NR>::TT;
   constexpr int NI = NB * (Rp / 4), PER = (NI + 255) / 256;  // joined 16-byte columns; of a thread
   constexpr int JP = NI <= 128 ? 256 / NI : 1;               // threads of a column
   constexpr int U = PER <= 2 ? 16 : 8;                       // partitions requested at a time
-  constexpr bool AHEAD = NB <= 4;
   __shared__ __attribute__((aligned(16))) bf16_t s_c[NB * ST];
   __shared__ __attribute__((aligned(16))) f32x4 s_j[JP > 1 ? 256 : 1];
   __shared__ float s_w[NB * MAX_PARTS];  // exp2(m_p - M) / L
@@ -578,8 +578,9 @@ int launch_out(const OutArgs<TP>& a, hipStream_t st) {
   const int gx = a.H * ((a.DV + 63) / 64);  // fewer sequences a block where that is what fills the chip
   if (gx * ((a.B + 15) / 16) >= 256) hipLaunchKernelGGL((latent_out_kernel<TP, NR, 16>), dim3(gx, (a.B + 15) / 16), dim3(256), 0, st, a);
   else if (gx * ((a.B + 7) / 8) >= 256) hipLaunchKernelGGL((latent_out_kernel<TP, NR, 8>), dim3(gx, (a.B + 7) / 8), dim3(256), 0, st, a);
-  else if (a.B > 1) hipLaunchKernelGGL((latent_out_kernel<TP, NR, 4>), dim3(gx, (a.B + 3) / 4), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((latent_out_kernel<TP, NR, 1>), dim3(gx), dim3(256), 0, st, a);
+  else if (gx * ((a.B + 3) / 4) > 256) hipLaunchKernelGGL((latent_out_kernel<TP, NR, 4>), dim3(gx, (a.B + 3) / 4), dim3(256), 0, st, a);
+  else if (a.B > 1) hipLaunchKernelGGL((latent_out_kernel<TP, NR, 4, true>), dim3(gx, (a.B + 3) / 4), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((latent_out_kernel<TP, NR, 1, true>), dim3(gx), dim3(256), 0, st, a);
   return (int)hipGetLastError();
 }
 

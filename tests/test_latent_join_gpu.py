@@ -11,7 +11,7 @@ DEV = "cuda"
 
 @pytest.mark.parametrize("S", [1, 3, 12])  # gate slabs: fewer and more than are asked for together
 @pytest.mark.parametrize("rank", [100, 256, 384, 512, 640, 1000])  # one to eight threads of a column for one sequence
-@pytest.mark.parametrize("B,max_kv", [(1, 8192), (1, 100), (2, 8192), (3, 1500), (9, 2500), (40, 700)])
+@pytest.mark.parametrize("B,max_kv", [(1, 8192), (1, 100), (2, 8192), (3, 1500), (9, 2500), (40, 700), (53, 700)])
 def test_join(native, B, max_kv, rank, S):
     from rag_llm_k8s_amd.ops import seq_native as Q
 

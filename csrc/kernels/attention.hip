@@ -1201,7 +1201,7 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
   // One trip to memory for the queries and the wave's first tile, the queries first: vector loads return in order, so behind the
   // tile their sums waited for it. Requests are unconditional (a wave without a tile asks for the block's last one, which another
   // wave reads): where paths with and without them meet, the compiler waits for every load in flight. The tile that the new token
-  // goes into is asked for again behind the barrier.
+  // goes into is asked for again behind the barrier, by its wave.
   // KL asks for a wave's own tile, once: its pieces go to LDS, in front of whose next access the compiler waits for all that is in
   // flight anyway, and whole pages by waves without a tile, and again behind the barrier, were most of a short context's loads
   // (512 pairs of 12 to 20 / 60 to 100 tokens 18.1 / 18.3 us, now 11.5 / 13.4).
@@ -1243,8 +1243,8 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  const bool mine = !KL || kt0 + wid_u < kt1, late = append && kt_first == n_kt - 1;
-  prologue(mine && (!KL || !late), mine && late);
+  const bool mine = kt0 + wid_u < kt1, late = append && kt_first == n_kt - 1;
+  prologue(!KL || (mine && !late), mine && late);
   if (rope) {
 #pragma unroll
     for (int s = 0; s < C::KS; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(s_q + min(fr, G - 1) * D + 32 * s + 8 * fh);

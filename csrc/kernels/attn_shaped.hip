@@ -592,7 +592,7 @@ __global__ __launch_bounds__(256, (DK <= 128 && DV <= 128) ? 2 : 1) void attn_sh
   }
   if (append) {
     __syncthreads();  // q in LDS; the appended row visible to the whole block
-    if (first_it == n - 1) {
+    if (it0 + wid_u == n - 1) {  // this wave's first unit is the one that was appended to
       request_k(first_it);
       __builtin_amdgcn_sched_barrier(0);
       request_v(first_it);

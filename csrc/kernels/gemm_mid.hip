@@ -520,6 +520,21 @@ int launch_finish(const float* P, int S, void* C, int ldc, const void* bias, con
   X(EPI_NONE) X(EPI_BIAS) X(EPI_RESID) X(EPI_BIAS_RESID) X(EPI_BIAS_GELU) X(EPI_GELU) X(EPI_BIAS_GELU_TANH) \
   X(EPI_SILU_MUL) X(EPI_GLU_CLIP)
 
+// C = epilogue of the sum of P's S fp32 slabs [M][weight rows]. C, bias and resid rows start on 16 bytes, N % 8 == 0.
+RAGK_API int ragk_slabs_finish(const float* P, int S, void* C, int ldc, const void* bias, const void* resid, int ldr, int M,
+                               int N, int epi, int out_f32, hipStream_t st) {
+  if (M <= 0 || N <= 0) return 0;
+  if (S < 1 || !P || N % (epi_pair(epi) ? 64 : 8) || (epi_pair(epi) && out_f32)) return (int)hipErrorInvalidValue;
+  if (((mid_has_bias(epi) || epi == EPI_GLU_CLIP) && !bias) || (mid_has_resid(epi) && !resid)) return (int)hipErrorInvalidValue;
+#define RAGK_FIN(E) \
+  case E: return launch_finish<E>(P, S, C, ldc, bias, resid, ldr, M, N, out_f32, st);
+  switch (epi) {
+    RAGK_MID_EPIS(RAGK_FIN)
+    default: return (int)hipErrorInvalidValue;
+  }
+#undef RAGK_FIN
+}
+
 // N = output columns (for the pair epilogues the weight has 2 N rows in the packed [64 gate | 64 up] layout, N % 64 == 0).
 // Rows of A and B start on 16 bytes. mi = rows of a tile / 32. S > 1: K-split through the fp32 slabs ws [S][M][weight rows],
 // summed with the epilogue by a second launch. S slabs without a consumer here: epi NONE, out_f32 = 2 (C holds the slabs).
@@ -540,14 +555,7 @@ RAGK_API int ragk_gemm_mid(const void* A, int lda, const void* B, int ldb, void*
   if (S > 1) {
     if (!ws) return (int)hipErrorInvalidValue;
     const int rc = dispatch_mid<EPI_NONE>(mi, A, lda, B, ldb, ws, rows, nullptr, nullptr, 0, M, rows, K, S, 1, st);
-    if (rc) return rc;
-#define RAGK_FIN(E) \
-  case E: return launch_finish<E>(ws, S, C, ldc, bias, resid, ldr, M, N, out_f32, st);
-    switch (epi) {
-      RAGK_MID_EPIS(RAGK_FIN)
-      default: return (int)hipErrorInvalidValue;
-    }
-#undef RAGK_FIN
+    return rc ? rc : ragk_slabs_finish(ws, S, C, ldc, bias, resid, ldr, M, N, epi, out_f32, st);
   }
 #define RAGK_MID(E) \
   case E: return dispatch_mid<E>(mi, A, lda, B, ldb, C, ldc, bias, resid, ldr, M, rows, K, 1, out_f32, st);
@@ -561,30 +569,14 @@ RAGK_API int ragk_gemm_mid(const void* A, int lda, const void* B, int ldb, void*
 RAGK_API int ragk_gemm_stream_part(const void* X, int ldx, const void* W, int ldw, float* P, int M, int N, int K, int S,
                                    int rows, int short_sums, hipStream_t st);
 
-// C = epilogue of the sum of P's S fp32 slabs [M][weight rows]. C, bias and resid rows start on 16 bytes, N % 8 == 0.
-RAGK_API int ragk_slabs_finish(const float* P, int S, void* C, int ldc, const void* bias, const void* resid, int ldr, int M,
-                               int N, int epi, int out_f32, hipStream_t st) {
-  if (M <= 0 || N <= 0) return 0;
-  if (S < 1 || !P || N % (epi_pair(epi) ? 64 : 8) || (epi_pair(epi) && out_f32)) return (int)hipErrorInvalidValue;
-  if (((mid_has_bias(epi) || epi == EPI_GLU_CLIP) && !bias) || (mid_has_resid(epi) && !resid)) return (int)hipErrorInvalidValue;
-#define RAGK_FIN(E) \
-  case E: return launch_finish<E>(P, S, C, ldc, bias, resid, ldr, M, N, out_f32, st);
-  switch (epi) {
-    RAGK_MID_EPIS(RAGK_FIN)
-    default: return (int)hipErrorInvalidValue;
-  }
-#undef RAGK_FIN
-}
-
 // At most 64 rows: the LDS-DMA weight stream's fp32 slabs ws [S][M][N] (gemm_stream.hip; `rows` of a tile, S | K / 64) and
 // their sum with the epilogue, as above; no pair epilogues.
 RAGK_API int ragk_gemm_slabs(const void* X, int ldx, const void* W, int ldw, void* C, int ldc, const void* bias,
-                             const void* resid, int ldr, int M, int N, int K, int epi, int out_f32, int S, int rows, float* ws,
-                             hipStream_t st) {
+                             const void* resid, int ldr, int M, int N, int K, int epi, int S, int rows, float* ws, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
   if (N % 8 || epi_pair(epi) || !ws) return (int)hipErrorInvalidValue;
   const int rc = ragk_gemm_stream_part(X, ldx, W, ldw, ws, M, N, K, S, rows, 1, st);
-  return rc ? rc : ragk_slabs_finish(ws, S, C, ldc, bias, resid, ldr, M, N, epi, out_f32, st);
+  return rc ? rc : ragk_slabs_finish(ws, S, C, ldc, bias, resid, ldr, M, N, epi, 0, st);
 }
 
 // qkv = A . B^T, B = [(Hq + 2 Hkv) * 128][K], with rope_kv's work in the epilogue: q and k rotated (positions pos[M], tables

@@ -46,10 +46,9 @@ _SIGS = {
     "ragk_attn_decode_set_kl": [I],
     "ragk_gemm_part_merge": [P, P, P, I, P, I, I, I, P, I, P, P, I, I, I, I, S],
     "ragk_gemm_part_merge_ok": [I, I, I, I, I],
-    "ragk_slabs_finish": [P, I, P, I, P, P, I, I, I, I, I, S],
     "ragk_gemm_hold_slabs": [P, I, P, I, P, P, I, I, I, I, S],
     "ragk_gemm_hold_slabs_silu": [P, I, P, I, P, P, I, I, I, I, I, P, S],
-    "ragk_gemm_slabs": [P, I, P, I, P, I, P, P, I, I, I, I, I, I, I, I, P, S],
+    "ragk_gemm_slabs": [P, I, P, I, P, I, P, P, I, I, I, I, I, I, I, P, S],
     "ragk_gemm_stream_part": [P, I, P, I, P, I, I, I, I, I, I, S],
     "ragk_gemm_part_silu": [P, I, P, I, P, I, I, I, I, S],
     "ragk_gemm_part_silu_ok": [I, I, I, I],

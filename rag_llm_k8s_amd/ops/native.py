@@ -268,7 +268,7 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
         path = 4
     if path is None and use_slabs(M, N, K, epi, out_f32) and _vec_rows(
             x, w, out, *(() if resid is None else (resid,))) and (bias is None or bias.data_ptr() % 16 == 0):
-        return _gemm_slabs(x, w, out, bias, resid, ldr, M, N, K, e, out_f32)
+        return _gemm_slabs(x, w, out, bias, resid, ldr, M, N, K, e)
     if path == 5:
         rc = _gemm_stream(x, w, None, out, bias, resid, ldr, M, N, K, epi, e, out_f32)
     elif path == 4:
@@ -976,13 +976,13 @@ def _gemm_stream(x, w, wscale, out, bias, resid, ldr, M, N, K, epi, e, out_f32):
                               cnt.data_ptr(), stream_ptr())
 
 
-def _gemm_slabs(x, w, out, bias, resid, ldr, M, N, K, e, out_f32):
+def _gemm_slabs(x, w, out, bias, resid, ldr, M, N, K, e):
     """gemm() of at most 64 rows through the stream GEMM's fp32 slabs."""
     rows, S = stream_part_cfg(M, N, K)
     ws = torch.empty(S * M * N, dtype=torch.float32, device=x.device)
     check(_lib.lib().ragk_gemm_slabs(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
-                                     ptr(bias), ptr(resid), ldr, M, N, K, e, int(out_f32), S, rows, ws.data_ptr(),
-                                     stream_ptr()), "ragk_gemm_slabs")
+                                     ptr(bias), ptr(resid), ldr, M, N, K, e, S, rows, ws.data_ptr(), stream_ptr()),
+          "ragk_gemm_slabs")
     return out
 
 

@@ -23,11 +23,17 @@ def test_slabs(native, M, N, K):
     r = torch.randn(M, N + 16, device=DEV, generator=g).bfloat16()[:, 16:]
     y = x.double() @ w.double().t()
     for epi, ref in (("none", y), ("bias", y + b.double()), ("resid", y + r.double()), ("bias_resid", y + b.double() + r.double())):
-        for f32 in (False, True):
-            out = torch.full((M + 1, N + 8), 7.0, device=DEV, dtype=torch.float32 if f32 else torch.bfloat16)
-            got = native.gemm(x, w, bias=b, resid=r, epi=epi, out=out[:M, :N], out_f32=f32)
-            assert bool(((got.double() - ref).abs() <= _bound(x, w, ref, f32)).all()), epi
-            assert bool((out[M] == 7).all()) and bool((out[:, N:] == 7).all())
+        out = torch.full((M + 1, N + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+        got = native.gemm(x, w, bias=b, resid=r, epi=epi, out=out[:M, :N])
+        assert bool(((got.double() - ref).abs() <= _bound(x, w, ref, False)).all()), epi
+        assert bool((out[M] == 7).all()) and bool((out[:, N:] == 7).all())
+    # fp32 results keep the one launch
+    assert not native.use_slabs(M, N, K, "none", True)
+    out = torch.full((M + 1, N + 8), 7.0, device=DEV)
+    got = native.gemm(x, w, bias=b, resid=r, epi="bias_resid", out=out[:M, :N], out_f32=True)
+    ref = y + b.double() + r.double()
+    assert bool(((got.double() - ref).abs() <= _bound(x, w, ref, True)).all())
+    assert bool((out[M] == 7).all()) and bool((out[:, N:] == 7).all())
     for epi, act in (("gelu", lambda v: torch.nn.functional.gelu(v)), ("bias_gelu", lambda v: torch.nn.functional.gelu(v + b.double())),
                      ("bias_gelu_tanh", lambda v: torch.nn.functional.gelu(v + b.double(), approximate="tanh"))):
         ref = act(y)  # |gelu'| <= 1.13; the function itself in fp32

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(FEW_W * 64) void few_kernel(std::conditional_t<PRO 
   const int fr = lane & 15, fh = lane >> 4, n0 = blockIdx.x * 16, nk = K / 32;
 
   // ---- requests, the rows ahead of what waits for them: loads come back in order, and with the weights in front a row waited for
-  // 20 KB of them (all indices clamped, so that no request stands behind a branch, where the compiler would wait for all)
+  // 20 KB of them (indices clamped, so that few requests stand behind a branch, where the compiler would wait for all)
   constexpr bool MAKES = PRO == EMBED || PRO == NORM;
   constexpr int NJ = MAKES ? D : 1;
   float v[MT][2 * NJ];
@@ -192,6 +192,7 @@ __global__ __launch_bounds__(FEW_W * 64) void few_kernel(std::conditional_t<PRO 
   if constexpr (MAKES) {
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
+      if (i && wid + FEW_W * i >= T) break;
       const int row = min(wid + FEW_W * i, T - 1);
       if constexpr (PRO == EMBED) few_row<NJ>(a, row, lane, v[i]);
       else few_row<NJ>(reinterpret_cast<const float*>(a.x), row, lane, v[i]);
@@ -229,15 +230,14 @@ __global__ __launch_bounds__(FEW_W * 64) void few_kernel(std::conditional_t<PRO 
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       const int row = wid + FEW_W * i;
+      if (row >= T) break;
       unsigned o[NJ];
       few_norm(v[i], a.f, gr, br, o);
-      if (row < T) {
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) *reinterpret_cast<unsigned*>(rows + row * rowb + 4 * lane + 256 * j) = o[j];
-        if (blockIdx.x == 0)
+      for (int j = 0; j < NJ; ++j) *reinterpret_cast<unsigned*>(rows + row * rowb + 4 * lane + 256 * j) = o[j];
+      if (blockIdx.x == 0)
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) *reinterpret_cast<unsigned*>(a.h + (size_t)row * K + 2 * lane + 128 * j) = o[j];
-      }
+        for (int j = 0; j < NJ; ++j) *reinterpret_cast<unsigned*>(a.h + (size_t)row * K + 2 * lane + 128 * j) = o[j];
     }
   }
   if constexpr (PRO == ATTEND) {

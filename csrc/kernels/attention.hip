@@ -1237,10 +1237,7 @@ __device__ __forceinline__ void attn_decode_block(const DecodeArgs& a, int part,
         request_first();
       }
     } else {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // no LDS access moves to either side
     }
   };
   const bool mine = kt0 + wid_u < kt1, late = append && kt_first == n_kt - 1;

@@ -375,6 +375,11 @@ int g_stream_diag = 0;
 // 28672-row Llama gate/up grid (448 tiles) occupies all 256 CUs; 128 = one block per CU, 224 tiles.
 int g_stream_pair_rows = 64;
 
+// bf16 weights of at least twice the L2s, and vocabularies, by the non-temporal policy: read once a step, and others lie between two
+// steps. Smaller ones may be what a small model leaves in the caches from call to call (8 rows, us from memory / from the caches,
+// non-temporal 16384 x 512 5.4 / 5.1, 32000 x 512 7.6 / 6.8, 32768 x 1024 12.1 / 10.8; plain 5.8 / 4.2, 8.2 / 5.1, 13.3 / 13.0).
+constexpr long long STREAM_NT_BYTES = 64LL << 20;
+
 // Everything else: bf16 weights, from 16384 rows, in 64-row tiles, so that two blocks share a CU and one's epilogue and short
 // last round run under the other's stream (18560 x 4096 at 8 / 64 rows: 128-row tiles and two slabs 55 / 75 us, now 37 / 46;
 // 32000 x 2048 32 / 37 -> 25 / 30); fp8 ones in 128-row tiles.
@@ -411,7 +416,7 @@ int launch_stream(const void* X, int ldx, const void* W, int ldw, const float* w
   }
   constexpr int R = FP8 ? WROWS : 64;
   const dim3 grid((Nrows + R - 1) / R, S);
-  if (g_stream_nt && (!FP8 || Nrows >= 65536))  // weights of more than the caches hold, read once per step: non-temporal
+  if (g_stream_nt && (Nrows >= 65536 || (!FP8 && 2LL * Nrows * K >= STREAM_NT_BYTES)))
     hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI, F32, FP8, true, R>), grid, dim3(ST_THREADS), 0, st, (const bf16_t*)X,
                        ldx, W, ldw, wscale, C, ldc, (const bf16_t*)bias, (const bf16_t*)resid, ldr, M, N, K, S, ws, cnt);
   else

@@ -189,8 +189,10 @@ __device__ __forceinline__ void mid_rope8(float (&x1)[8], float (&x2)[8], const 
 }
 
 // Weights that one row of tiles reads once, by the streaming policy: 28672 x 4096 at 66 / 140 / 256 rows 50.8 / 56.2 / 66.2 -> 46.9 /
-// 53.4 / 61.9 us, 22528 x 2048 25.4 / 29.1 / 33.8 -> 23.4 / 27.6 / 31.3. Where tiles share them (several rows of tiles, a K-split) it
-// costs 2 to 11 % instead, and weights that the caches hold from call to call keep the other policy.
+// 53.4 / 61.9 us, 22528 x 2048 25.4 / 29.1 / 33.8 -> 23.4 / 27.6 / 31.3; also behind whole rounds of larger tiles that have just read
+// them (700 / 3000 rows, the last 188 / 184 here, 146 / 503 -> 141 / 502; 5192 of 22528 x 2048, the last 72, 344 -> 340). Where tiles
+// share them (several rows of tiles, a K-split) it costs 2 to 11 % instead, and weights that the caches hold from call to call keep
+// the other policy.
 __device__ __forceinline__ void blds16_nt_asm(i32x4 srd, int voff, int soff, unsigned lds_addr) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds_addr), "v"(voff), "s"(srd),
                "s"(soff));

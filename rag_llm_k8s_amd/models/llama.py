@@ -378,7 +378,8 @@ class LlamaModel(DecoderModel):
         if self.comm is None and inp.meta is not None and inp.meta.kind != "decode":
             L0 = w.layers[0]
             if h.shape[0] <= 64:
-                if inp.slots is not None and all(be.splits(h.shape[0], L0[n]) for n in ("wqkv", "wo", "wdown")):
+                M = h.shape[0]
+                if inp.slots is not None and be.splits(M, L0["wqkv"]) and be.splits(M, L0["wo"]) and be.splits(M, L0["wdown"]):
                     return self.hidden_states_few(inp, h, attn)
             else:
                 ns = (be.prefill_nsplit(h.shape[0], L0["wo"]), be.prefill_nsplit(h.shape[0], L0["wdown"]))

@@ -266,7 +266,7 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
         path = 5
     if path is None and DEC_DEFAULT and use_dec(M, N, K, epi):
         path = 4
-    if path is None and use_slabs(M, N, K, epi, out_f32) and _vec_rows(
+    if path is None and M > 16 and use_slabs(M, N, K, epi, out_f32) and _vec_rows(
             x, w, out, *(() if resid is None else (resid,))) and (bias is None or bias.data_ptr() % 16 == 0):
         return _gemm_slabs(x, w, out, bias, resid, ldr, M, N, K, e)
     if path == 5:

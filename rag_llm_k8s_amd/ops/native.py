@@ -593,7 +593,7 @@ def gemm_part(x, w, out=None, ks=None, short_sums=False):
     if (STREAM_PART and not fp8 and ks is None and out is None and M >= STREAM_PART_MIN_M and K % 64 == 0
             and N % 4 == 0 and stream_part_cfg(M, N, K)[1] > 0):
         return gemm_stream_part(x, wt, short_sums=short_sums)
-    if fp8 and ks is None and out is None and use_hold_slabs(M, N, K) and _vec_rows(x, wt):
+    if fp8 and ks is None and out is None and use_hold_slabs(M, N, K) and _vec_rows(x, wt) and wt.stride(0) < 1 << 24:
         return gemm_hold_slabs(x, wt, w.scale)
     ks, S = gemm_part_slabs(M, N, K, ks)
     _req(S > 0, "gemm_part: unsupported K=%d" % K)
@@ -1042,7 +1042,8 @@ def use_hold_slabs(M, N, K):
     5120 x 18432 32 / 38 / 49 -> 23 / 26 / 31, 4096 x 8192 at 33 / 64 rows 14.9 / 18.5 -> 13.9 / 18.1. Smaller weights leave a
     block too few rows for the 128 KB of x that it loads first (4096 x 8192 at 17 rows 10.7 against 12.0, 4096 x 4096 at 33 / 64
     7.8 / 9.5 against 9.9 / 13), and up to 16 rows the two are equal."""
-    return 16 < M <= 64 and K % 2048 == 0 and N % 16 == 0 and N * K >= (5 << 23 if M <= 32 else 1 << 25)
+    return (16 < M <= 64 and K % 2048 == 0 and K // 2048 <= _cu_count() and N % 16 == 0
+            and N * K >= (5 << 23 if M <= 32 else 1 << 25))
 
 
 def gemm_hold_slabs(x, w8, scale, out=None):
@@ -1061,7 +1062,7 @@ def use_hold_slabs_silu(M, K):
     """fp8 gate/up projections of more rows than a launch of gemm_hold holds: slabs of 2048 of K and a pass that sums and pairs
     them, 28672 x 4096 at 33 / 64 rows 54 / 61 us (two launches) -> 33 / 38, 7168 x 4096 22 / 26 (gemm_stream) -> 17 / 21, 16384
     x 6144 at 17 / 64 rows 38 / 72 -> 29 / 37. Up to 16 rows the pass takes what the slabs gain (8192 x 6144 18.6 against 18.1)."""
-    return 16 < M <= 64 and K % 2048 == 0 and M > _hold_rows(K, True)
+    return 16 < M <= 64 and K % 2048 == 0 and K // 2048 <= _cu_count() and M > _hold_rows(K, True)
 
 
 def quant_fp8_rows(x, q=None, scale=None):

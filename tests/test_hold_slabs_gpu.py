@@ -31,6 +31,26 @@ def test_partials(native, N, K):
         assert bool(((P.double().sum(0) - x.double() @ wd.t()).abs() <= _bound(x, wd)).all()), M
 
 
+@pytest.mark.parametrize("N,K,ld", [(32, 1 << 20, 1 << 20), (64, 1 << 19, 1 << 24)])
+def test_rows_too_long_or_too_far_apart(native, N, K, ld):
+    """More slabs than there are CUs, and rows past a lane's 32-bit offset, go where they went."""
+    from rag_llm_k8s_amd.ops.fp8 import Fp8Weight
+
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.randn(33, K, device=DEV, generator=g).bfloat16()
+    q = quantize_weight((torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).bfloat16())
+    rows = torch.zeros((N - 1) * ld + K, dtype=torch.uint8, device=DEV).view(torch.float8_e4m3fn).as_strided((N, K), (ld, 1))
+    rows.view(torch.uint8).copy_(q.w8.view(torch.uint8))
+    wd = q.w8.double() * q.scale.double()[:, None]
+    P = native.gemm_part(x, Fp8Weight(rows, q.scale))
+    assert bool(((P.double().sum(0) - x.double() @ wd.t()).abs() <= _bound(x, wd)).all())
+    if ld == K:
+        w2 = Fp8Weight(torch.cat([q.w8.view(torch.uint8)] * 4).view(torch.float8_e4m3fn), q.scale.repeat(4))
+        z = (x.double() @ wd.t()).repeat(1, 4).view(33, 2, 64)
+        ref = torch.nn.functional.silu(z[:, 0]) * z[:, 1]
+        assert float((native.gemm_fp8(x, w2, epi="silu_mul").double() - ref).norm()) < 2.0 ** -8 * float(ref.norm())
+
+
 @pytest.mark.parametrize("tiles", [1, 2, 3, 4, 5, 7, 63, 64, 65, 200])
 def test_shares(native, tiles):
     """Blocks with one to 64 tiles, fewer and more than are in flight, a share that needs more blocks than asked for."""

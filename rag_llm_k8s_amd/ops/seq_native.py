@@ -188,7 +188,7 @@ def decode_parts(spec, max_kv_len, batch):
     parts = max(1, DECODE_TARGET_BLOCKS // rows)
     if 4 * parts * rows < 3 * DECODE_TARGET_BLOCKS:
         parts += 1
-    return min(parts, -(-pages // DECODE_MIN_PAGES))
+    return max(1, min(parts, -(-pages // DECODE_MIN_PAGES)))
 
 
 def decode_split(specs, max_kv_len, batch, device):

@@ -93,3 +93,15 @@ def test_decode_partitions_cover_every_unit(max_len, batch, hkv, kv_len):
         assert (nparts - 1) * eff < n <= nparts * eff
     # no partition that only a longer context than the longest could fill
     assert mp == 1 or (mp - 1) * pt * 64 < max_len
+
+
+@settings(max_examples=200, deadline=None)
+@given(max_kv=st.integers(0, 131072), batch=st.integers(1, 256), groups=st.sampled_from([1, 2, 4, 8]),
+       window=st.sampled_from([0, 64, 4096]))
+def test_shaped_decode_parts(max_kv, batch, groups, window):
+    """At least one partition, and none that only a longer context could fill; no context at all is one, too."""
+    from rag_llm_k8s_amd.ops.seq_native import DECODE_PART_PAGES, decode_parts
+    from rag_llm_k8s_amd.ops.specs import AttnSpec
+
+    parts = decode_parts(AttnSpec(heads=groups * 4, kv_heads=groups, dim=128, vdim=128, scale=1.0, window=window), max_kv, batch)
+    assert parts >= 1 and (parts == 1 or (parts - 1) * DECODE_PART_PAGES * 64 < max_kv)

@@ -1020,7 +1020,7 @@ struct DecodeArgs {
   const float* cos_t; const float* sin_t;
 };
 
-constexpr int DEC_U = 32;  // keys of a unit: what a wave takes at a time where tiles come through registers
+static_assert(KT == DEC_TILE, "a page");  // DEC_U: what a wave takes at a time where tiles come through registers
 
 // Units per partition of one sequence: its keys spread evenly over all max_parts partitions (never fewer
 // than part_tiles tiles per partition). The grid is sized once for max_parts (hipGraph
@@ -1028,7 +1028,7 @@ constexpr int DEC_U = 32;  // keys of a unit: what a wave takes at a time where 
 // same amount of KV: splitting a 5.3k-token context by a fixed 32-tile partition left 1 of 4
 // partitions idle and 8 vs 5 tiles per wave on the others.
 __device__ __forceinline__ int decode_part_units(int n, const DecodeArgs& a, int unit = DEC_U) {
-  return max(a.part_tiles * (KT / unit), (n + a.max_parts - 1) / a.max_parts);
+  return decode_share(n, a.part_tiles, a.max_parts, unit);
 }
 
 // LDS of one decode-attention block: one V tile per wave (KL: and one K tile per wave after them), then the
@@ -1050,9 +1050,9 @@ constexpr int decode_lds_bytes() {
 // CU keeps the same KV bytes in flight as two 4-wave blocks and needs no merge launch). A multi-partition
 // sequence writes its partition records; attn_decode_reduce_kernel (or, deferred, the o_proj GEMM's
 // gemm_part_merge) merges them.
-// DG = 1 (diagnostic build, tools/attn_decode_probe.py): the same K / V loads and waits, no QK^T / softmax / PV
-// -- how much of the kernel's time the KV access pattern alone takes. DG = 2: as 1, but K also arrives by
-// LDS-DMA (1 KiB per instruction, into the V buffer: results meaningless) instead of 64-B row pieces.
+// DG = 1 (diagnostic build, tools/attn_decode_probe.py): the loads of whole pages, one behind the other, without QK^T / softmax /
+// PV -- what the access pattern takes without the kernel's units and look-ahead. DG = 2: as 1, but K also arrives by LDS-DMA
+// (1 KiB per instruction, into the V buffer: results meaningless) instead of 64-B row pieces.
 // KL: K tiles arrive by LDS-DMA too (whole 1 KiB pieces instead of 64-B row pieces per lane: the pure access
 // pattern streams 4-5 % faster, tools/attn_decode_probe.py) and the QK^T fragments are read from LDS; a
 // wave then holds 32 KB of LDS, so the single-partition grid uses 4-wave blocks (one per CU).

@@ -462,13 +462,13 @@ __device__ __forceinline__ float slab_gate(const ShapedDecode& a, int b, int h) 
   }
   return __builtin_amdgcn_rcpf(1.f + __expf(-g));
 }
-constexpr int DEC_U = 32;                // keys of a unit: what a wave takes at a time
-constexpr int DEC_UPT = KT / DEC_U;      // units of a page
+static_assert(KT == DEC_TILE, "a page");
+constexpr int DEC_UPT = KT / DEC_U;  // units of a page
 // units that a new token at `pos` visits (the last page's second half may lie past it)
 __device__ __forceinline__ int units(const Pages& pg, int pos) { return pg.n * DEC_UPT - (pos % KT < DEC_U ? 1 : 0); }
 // units per partition: the visited ones spread over all partitions, at least min_tiles pages each
 __device__ __forceinline__ int part_units(int n, const ShapedDecode& a) {
-  return max(a.min_tiles * DEC_UPT, (n + a.max_parts - 1) / a.max_parts);
+  return decode_share(n, a.min_tiles, a.max_parts);
 }
 
 constexpr int DEC_HEADS = 16;  // query heads per decode block (one MFMA column each)

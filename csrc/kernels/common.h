@@ -220,6 +220,14 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return t;
 }
 
+// Split of a sequence's keys in decode attention, on which its kernels, the joins and the o_proj product that joins by itself
+// (gemm_part.hip) have to agree: units of DEC_U keys, the units of a partition where n are spread over at most max_parts, of
+// min_tiles pages of DEC_TILE keys at least.
+constexpr int DEC_TILE = 64, DEC_U = 32;
+__device__ __forceinline__ int decode_share(int n, int min_tiles, int max_parts, int unit = DEC_U) {
+  return max(min_tiles * (DEC_TILE / unit), (n + max_parts - 1) / max_parts);
+}
+
 // Bijective XCD-aware block remap (MI355X: 8 XCDs, blocks dealt round-robin).
 // Blocks b, b+8, b+16... share an XCD; remap so each XCD gets a contiguous range
 // of logical tile ids (neighbouring tiles share operand panels in its L2).

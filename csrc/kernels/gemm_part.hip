@@ -73,7 +73,6 @@ struct MergeArgs {
   int Hq, part_tiles, max_parts;
 };
 constexpr int MG_D = 128;    // head dim
-constexpr int MG_U = 32;     // keys per unit of a partition (attention.hip DEC_U), two to a KV tile
 constexpr int MG_MAXPP = 32; // partition records merged per thread (host check)
 constexpr int MG_CHUNK = 4;  // records in flight per thread
 constexpr int MG_MAXR = 4;   // rows
@@ -173,9 +172,7 @@ __global__ __launch_bounds__(PT_THREADS + (MG ? MG_THREADS : 0), MG ? 2 : 1) voi
           const int v = mg.kv_lens[min(rr, M - 1)];
           kvl = r == rr ? v : kvl;
         }
-        const int n = (kvl + MG_U - 1) / MG_U;
-        const int pt = max(mg.part_tiles * 2, (n + mg.max_parts - 1) / mg.max_parts);
-        const int np = (n + pt - 1) / pt;
+        const int n = (kvl + DEC_U - 1) / DEC_U, pt = decode_share(n, mg.part_tiles, mg.max_parts), np = (n + pt - 1) / pt;
         const size_t pb = ((size_t)r * mg.Hq + hq) * mg.max_parts;
         const uint2 one = *reinterpret_cast<const uint2*>(mg.out + (size_t)r * mg.out_stride + hq * MG_D + 4 * d4);
         // online max-rescaled merge of this lane's partitions pg, pg + npg, ... in chunks of MG_CHUNK

@@ -395,8 +395,9 @@ class LlamaModel(DecoderModel):
     def hidden_states_few(self, inp: StepInput, h, attn):
         """TP=1 prefill of at most 64 tokens: the decode step's split-K products, whose slabs the rotation and the norms that
         follow sum: as many launches as with products of rows, and the weights at the memory's rate (four layers 4096 wide,
-        9 / 20 / 64 tokens: 515 / 611 / 854 us -> 467 / 477 / 536). The residual rounds where the product's epilogue rounds it,
-        once, behind the add."""
+        9 / 20 / 64 tokens: 507 / 601 / 847 us -> 462 / 470 / 531). Where NativeBackend.splits holds: 2048 wide, where the host bounds
+        the step and the slabs' allocations cost it, 9 / 20 / 48 tokens take 350 / 350 / 351 in rows and 380 / 385 / 386 in slabs. The
+        residual rounds where the product's epilogue rounds it, once, behind the add."""
         be, w, c = self.be, self.w, self.cfg
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
         layers = w.layers

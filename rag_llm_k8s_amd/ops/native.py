@@ -1539,12 +1539,14 @@ def decode_partitions(max_kv_len, batch, Hkv, target_blocks=None, min_tiles=None
     """(part_tiles, max_parts) for split-K decode: grid = max_parts x Hkv x batch <= target_blocks, two blocks a CU. More than fit
     at once run as a round of their own behind the first (20 rows of 5000 tokens, 8 KV heads: 59.4 us in 480 blocks, 63.4 in 640),
     and fewer, larger ones beat a third of a CU's slots (16 rows of 6000, 4 KV heads: 33.7 in 512, 34.7 in 768). The shaped
-    kernel's blocks lose by rounding down (seq_native.decode_parts).
+    kernel's blocks follow a rule of their own (seq_native.decode_parts).
 
     Once batch x KV heads would fill the CUs by itself, one partition per pair (attention.hip KL) where its rounds of one block a
     CU are at least four fifths full, else three, or as many as the longest context has keys for: 264 pairs of 1600 tokens 52.4 ->
     45.2 us, 320 of 560 28.0 -> 23.7, 384 of 2400 87.5 -> 86.0, 400 of 1250 52.6 -> 51.1; 512 full ones of 3200 tokens 134 in one,
-    146 in three. A context without keys for the third leaves those blocks, two thirds of the workspace and the join to nothing.
+    146 in three (eight query heads a KV head, which have no KL: 264 of 60 / 300 / 1000 / 4000 tokens 10.3 / 19.4 / 36.1 / 125 ->
+    12.2 / 18.9 / 29.5 / 87; the shortest pay for the join's launch). A context without keys for the third leaves those blocks, two
+    thirds of the workspace and the join to nothing.
     Where all three are at work in more than two and a quarter rounds, short contexts fill fewer, larger ones: three tiles at least,
     not two (384 pairs of 150 / 300 / 600 tokens 17.0 / 21.5 / 26.3 us -> 13.0 / 18.2 / 26.3, 408 of 200 / 300 20.1 / 22.7 -> 16.8
     / 21.1; below, 264 of 200 / 600 14.7 / 19.8 against 16.2 / 21.6).
@@ -1569,9 +1571,9 @@ def decode_partitions(max_kv_len, batch, Hkv, target_blocks=None, min_tiles=None
     return part_tiles, max(1, min(target_blocks // pairs, -(-max_kt // min_tiles)))
 
 
-# One partition per (sequence, KV head) in 8-wave blocks once batch x KV heads reaches this (>= one block
-# per CU): the same KV bytes in flight as two 4-wave partition blocks, and no merge launch (0 = off).
-# Batch 32: decode step 6.96 -> 6.86-6.90 ms (profiles/decode_nw8_ab_r4.log).
+# From this many (sequence, KV head) pairs on, a block a CU, decode_partitions weighs one partition a pair, without a merge
+# launch, against three (0 = off). One, with 128 columns and four query heads a KV head, runs as below, in 8-wave blocks without
+# DECODE_KL; batch 32: decode step 6.96 -> 6.86-6.90 ms (profiles/decode_nw8_ab_r4.log).
 DECODE_NW8_MIN_PAIRS = 256
 
 

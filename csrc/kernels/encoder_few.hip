@@ -230,14 +230,16 @@ __global__ __launch_bounds__(FEW_W * 64) void few_kernel(std::conditional_t<PRO 
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       const int row = wid + FEW_W * i;
-      if (row >= T) break;
+      if (i && row >= T) break;  // (the first one's norm in front of a branch: 24 layers of 1024, 14 rows 636 -> 630)
       unsigned o[NJ];
       few_norm(v[i], a.f, gr, br, o);
+      if (row < T) {
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) *reinterpret_cast<unsigned*>(rows + row * rowb + 4 * lane + 256 * j) = o[j];
-      if (blockIdx.x == 0)
+        for (int j = 0; j < NJ; ++j) *reinterpret_cast<unsigned*>(rows + row * rowb + 4 * lane + 256 * j) = o[j];
+        if (blockIdx.x == 0)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) *reinterpret_cast<unsigned*>(a.h + (size_t)row * K + 2 * lane + 128 * j) = o[j];
+          for (int j = 0; j < NJ; ++j) *reinterpret_cast<unsigned*>(a.h + (size_t)row * K + 2 * lane + 128 * j) = o[j];
+      }
     }
   }
   if constexpr (PRO == ATTEND) {

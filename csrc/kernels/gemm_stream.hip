@@ -426,7 +426,8 @@ int launch_stream(const void* X, int ldx, const void* W, int ldw, const float* w
 }
 
 // short_sums: 512 of K to a sum, as the register-streaming kernel cuts K = 4096 (rms error of 64 x 14336 x 4096 in two slabs 2.72e-7
-// -> 1.35e-7; 28.9 / 29.2 us). What decode steps' consumers sum has one sum a slab.
+// -> 1.35e-7; 28.9 / 29.2 us), 256 of K up to 2048, which it cuts as often (1 x 32768 x 2048 2.70e-7 -> 0.96e-7). What decode steps'
+// consumers sum has one sum a slab.
 constexpr int SLAB_SEG = 8;
 
 template <int MT, int R>
@@ -434,7 +435,10 @@ int launch_stream_slab(const void* X, int ldx, const void* W, int ldw, float* P,
                        hipStream_t st) {
   const dim3 grid((N + R - 1) / R, S);
   // non-temporal weight stream (each weight byte is read once per step)
-  if (short_sums)
+  if (short_sums && K <= 2048)
+    hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI_NONE, true, false, true, R, true, 0, SLAB_SEG / 2>), grid, dim3(ST_THREADS), 0, st,
+                       (const bf16_t*)X, ldx, W, ldw, nullptr, P, N, nullptr, nullptr, 0, M, N, K, S, nullptr, nullptr);
+  else if (short_sums)
     hipLaunchKernelGGL((gemm_stream_kernel<MT, EPI_NONE, true, false, true, R, true, 0, SLAB_SEG>), grid, dim3(ST_THREADS), 0, st,
                        (const bf16_t*)X, ldx, W, ldw, nullptr, P, N, nullptr, nullptr, 0, M, N, K, S, nullptr, nullptr);
   else

@@ -81,7 +81,7 @@ struct MlpArgs {
   const bf16_t* gamma;     // [H] post-attention norm weight (with P)
   float eps;
   int S;
-  const bf16_t* wgu;       // [2I][H] packed [64 gate | 64 up] per 128 rows
+  const bf16_t* wgu;       // [2I][H] packed [64 gate | 64 up] per 128 rows, rows ldgu apart
   const bf16_t* wd;        // [H][I]
   bf16_t* h;               // [H] residual, updated in place
   bf16_t* act;             // [I] hand-off workspace
@@ -90,7 +90,7 @@ struct MlpArgs {
   unsigned* err_host;      // device address of a host-mapped pinned word (the engine polls it per step)
   const unsigned* tmo;     // deadline in s_memrealtime ticks (0 = ME_TIMEOUT_TICKS); a test hook forces timeouts
   unsigned long long* stamps;  // optional [G][8] s_memrealtime stamps (tools/mlp_engine_bench.py ME_STAMPS=1)
-  int H, I;
+  int H, I, ldgu;
   int w_even, w_odd;       // phase-A work weights of workgroups on even / odd XCDs
 };
 
@@ -201,9 +201,9 @@ __device__ __forceinline__ void me_issue_slot(const MlpArgs& a, const SlotMap& m
   if (cu.s < m.nA) {
     const int j0 = 8 * (m.a0 + cu.g);
     const int prow0 = (j0 >> 6) * 128 + (j0 & 63);
-    base = reinterpret_cast<const char*>(a.wgu) + (long long)prow0 * a.H * 2 + cu.kc * (ME_KC * 2);
-    stride = 2ll * a.H;
-    jump = 112ll * a.H;
+    stride = 2ll * a.ldgu;
+    base = reinterpret_cast<const char*>(a.wgu) + prow0 * stride + cu.kc * (ME_KC * 2);
+    jump = 56 * stride;
   } else {
     base = reinterpret_cast<const char*>(a.wd) + (long long)(16 * (m.d0 + cu.g)) * a.I * 2 + cu.kc * (ME_KC * 2);
     stride = 2ll * a.I;
@@ -575,14 +575,15 @@ RAGK_API int ragk_mlp_engine_set_stamps(void* p) {
 // err: device error word; err_host: device address of a host-mapped word (may be null); tmo: device word
 // holding the deadline in s_memrealtime ticks (0 = default).
 RAGK_API int ragk_mlp_engine(const void* xn, const float* P, int S, const void* gamma, float eps, const void* wgu,
-                             const void* wd, void* h, void* act, void* ctr, void* err, void* err_host, const void* tmo,
+                             int ldgu, const void* wd, void* h, void* act, void* ctr, void* err, void* err_host, const void* tmo,
                              int M, int H, int I, int G, hipStream_t st) {
   if (!ragk_mlp_engine_ok(M, H, I, G)) return (int)hipErrorInvalidValue;
-  if (!wgu || !wd || !h || !act || !ctr || !err || !tmo || (!xn && (!P || !gamma || S < 1 || H % 4)))
+  if (!wgu || ldgu < H || ldgu % 8 || !wd || !h || !act || !ctr || !err || !tmo || (!xn && (!P || !gamma || S < 1 || H % 4)))
     return (int)hipErrorInvalidValue;
+  const bool gap = ldgu != H;  // (the XCDs' rates differ where rows lie 8 KB apart: 3 : 4 and 1 : 1 66.0 and 65.9 us, with the gap 68.4 and 65.7)
   MlpArgs a{(const bf16_t*)xn, xn ? nullptr : P, (const bf16_t*)gamma, eps, S, (const bf16_t*)wgu,
             (const bf16_t*)wd, (bf16_t*)h, (bf16_t*)act, (unsigned long long*)ctr, (unsigned*)err,
-            (unsigned*)err_host, (const unsigned*)tmo, g_me_stamps, H, I, g_me_w_even, g_me_w_odd};
+            (unsigned*)err_host, (const unsigned*)tmo, g_me_stamps, H, I, ldgu, gap ? 1 : g_me_w_even, gap ? 1 : g_me_w_odd};
   if (g_me_nt)
     hipLaunchKernelGGL(mlp_engine_kernel<true>, dim3(G), dim3(ME_THREADS), 0, st, a);
   else

@@ -18,7 +18,7 @@ using namespace ragk;
 namespace {
 
 template <typename T>
-__global__ __launch_bounds__(256) void embed_residual_kernel(int* __restrict__ ids, const T* __restrict__ table, float* h,
+__global__ __launch_bounds__(256) void embed_residual_kernel(int* __restrict__ ids, const T* __restrict__ table, int ldt, float* h,
                                                              int W, int vocab, const int* __restrict__ carry,
                                                              const int* __restrict__ prev, float scale, int n,
                                                              const int* __restrict__ pos,
@@ -36,7 +36,7 @@ __global__ __launch_bounds__(256) void embed_residual_kernel(int* __restrict__ i
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
   for (int v = threadIdx.x; v < (W >> 3); v += 256) {
     float f[8];
-    ld8(table + (size_t)id * W + v * 8, f);
+    ld8(table + (size_t)id * ldt + v * 8, f);
 #pragma unroll
     for (int e = 0; e < 8; ++e) f[e] *= scale;
     if (pos != nullptr) {  // columns 2i / 2i + 1: sin / cos of pos * turns[i] whole turns
@@ -346,18 +346,18 @@ __global__ __launch_bounds__(256) void glu_clip_kernel(const float* __restrict__
 
 }  // namespace
 
-// table: [vocab][W] bf16 (f32 = 0) or fp32; h: fp32 [T][W], W % 8 == 0. carry / prev may be null. pos [T] and turns
+// table: [vocab][W] bf16 (f32 = 0) or fp32, rows ldt apart; h: fp32 [T][W], W % 8 == 0. carry / prev may be null. pos [T] and turns
 // [(n + 1) / 2] (fp64, turns per position of each column pair), or null: no sinusoid.
-RAGK_API int ragk_embed_residual(int* ids, const void* table, float* h, int T, int W, int vocab, const int* carry,
+RAGK_API int ragk_embed_residual(int* ids, const void* table, int ldt, float* h, int T, int W, int vocab, const int* carry,
                                  const int* prev, float scale, int n, const int* pos, const double* turns, int f32,
                                  hipStream_t st) {
   if (T <= 0) return 0;
-  if (W % 8 || n > W || (pos && !turns)) return (int)hipErrorInvalidValue;
+  if (W % 8 || ldt < W || ldt % 8 || n > W || (pos && !turns)) return (int)hipErrorInvalidValue;
   if (f32)
-    hipLaunchKernelGGL(embed_residual_kernel<float>, dim3(T), dim3(256), 0, st, ids, (const float*)table, h, W, vocab,
+    hipLaunchKernelGGL(embed_residual_kernel<float>, dim3(T), dim3(256), 0, st, ids, (const float*)table, ldt, h, W, vocab,
                        carry, prev, scale, n, pos, turns);
   else
-    hipLaunchKernelGGL(embed_residual_kernel<bf16_t>, dim3(T), dim3(256), 0, st, ids, (const bf16_t*)table, h, W, vocab,
+    hipLaunchKernelGGL(embed_residual_kernel<bf16_t>, dim3(T), dim3(256), 0, st, ids, (const bf16_t*)table, ldt, h, W, vocab,
                        carry, prev, scale, n, pos, turns);
   return (int)hipGetLastError();
 }

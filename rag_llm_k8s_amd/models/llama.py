@@ -24,6 +24,7 @@ from typing import List, Optional
 import torch
 
 from ..ops.backend import AttnMeta, get_backend  # noqa: F401
+from ..ops.pitch import pitched
 from ..ops.reference import pack_gate_up, rope_tables
 from .base import DecoderModel, StepInput
 
@@ -147,7 +148,8 @@ class LlamaWeights:
             dn = get(p + "mlp.down_proj.weight", cols=(r * I, (r + 1) * I))
             w.layers.append(dict(
                 ln_in=dev(get(p + "input_layernorm.weight")), ln_post=dev(get(p + "post_attention_layernorm.weight")),
-                wqkv=dev(torch.cat([q, k, v], 0)), wo=dev(o), wgu=dev(pack_gate_up(gt, up)), wdown=dev(dn)))
+                wqkv=dev(torch.cat([q, k, v], 0)), wo=dev(o), wgu=pitched(dev(pack_gate_up(gt, up))),
+                wdown=dev(dn)))
         w.norm = dev(get("model.norm.weight"))
         V = cfg.vocab_size
         lo, hi = r * Vl, min(V, (r + 1) * Vl)
@@ -155,7 +157,7 @@ class LlamaWeights:
         lm = get(name, rows=(lo, hi))
         if lm.shape[0] < Vl:  # pad the last vocab shard
             lm = torch.cat([lm, torch.zeros(Vl - lm.shape[0], lm.shape[1], dtype=lm.dtype, device=lm.device)], 0)
-        w.lm_head = dev(lm)
+        w.lm_head = dev(lm) if cfg.tie_word_embeddings else pitched(dev(lm))  # (a tied one shares its memory)
         w.vocab_offset = lo
         w.vocab_valid = hi - lo
         return w
@@ -201,9 +203,9 @@ class LlamaWeights:
         w.embed = rnd(cfg.vocab_size, H)
         for _ in range(cfg.num_hidden_layers):
             w.layers.append(dict(ln_in=ones(H), ln_post=ones(H), wqkv=rnd((Hq + 2 * Hkv) * D, H),
-                                 wo=rnd(H, Hq * D), wgu=rnd(2 * I, H), wdown=rnd(H, I)))
+                                 wo=rnd(H, Hq * D), wgu=pitched(rnd(2 * I, H)), wdown=rnd(H, I)))
         w.norm = ones(H)
-        w.lm_head = rnd(Vl, H)
+        w.lm_head = pitched(rnd(Vl, H))
         w.vocab_offset = tp_rank * Vl
         w.vocab_valid = min(cfg.vocab_size - tp_rank * Vl, Vl)
         return w
@@ -216,6 +218,7 @@ class LlamaWeights:
         for L in self.layers:
             for k in ("wqkv", "wo", "wgu", "wdown"):
                 L[k] = quantize_weight(L[k])
+                L[k].w8 = pitched(L[k].w8)
         if lm_head:
             self.lm_head = quantize_weight(self.lm_head)
         self.dtype = "fp8"

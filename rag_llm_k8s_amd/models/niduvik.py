@@ -17,6 +17,7 @@ from typing import List, Optional
 import torch
 
 from ..ops.backend import get_backend
+from ..ops.pitch import pitched
 from ..ops.specs import AttnSpec, SsmSpec, ceil_to
 from .base import DecoderModel
 from .mixers import AttentionMixer, ClippedGluMlp, Mamba2Mixer, pad1, pad2
@@ -99,7 +100,7 @@ class NiduvikWeights:
         device = torch.device(device)
 
         def dev(t, dt=dtype):
-            return t.to(device=device, dtype=dt).contiguous()
+            return pitched(t.to(device=device, dtype=dt).contiguous())
 
         def norm(name):
             return dev(pad1(get(name).float(), wp), torch.float32)

@@ -19,6 +19,7 @@ from typing import List, Optional
 import torch
 
 from ..ops.backend import get_backend
+from ..ops.pitch import pitched
 from ..ops.specs import LatentSpec, ceil_to
 from .base import DecoderModel
 from .mixers import GluMlp, LatentAttentionMixer, pad1, pad2
@@ -103,7 +104,7 @@ class RolesunWeights:
         device = torch.device(device)
 
         def dev(t, dt=dtype):
-            return t.to(device=device, dtype=dt).contiguous()
+            return pitched(t.to(device=device, dtype=dt).contiguous())
 
         def vec(name):
             return dev(pad1(get(name).float(), wp), torch.float32)

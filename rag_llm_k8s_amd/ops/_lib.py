@@ -56,7 +56,7 @@ _SIGS = {
     "ragk_mlp_engine_set_nt": [I],
     "ragk_mlp_engine_set_stamps": [P],
     "ragk_mlp_engine_set_xcd_weights": [I, I],
-    "ragk_mlp_engine": [P, P, I, P, F, P, P, P, P, P, P, P, P, I, I, I, I, S],
+    "ragk_mlp_engine": [P, P, I, P, F, P, I, P, P, P, P, P, P, P, I, I, I, I, S],
     "ragk_host_word_alloc": [],
     "ragk_host_word_dev": [P],
     "ragk_host_word_free": [P],
@@ -103,7 +103,7 @@ _SIGS = {
     "ragk_quant_fp8_rows": [P, I, P, I, P, I, I, S],
     "ragk_gemm_fp8": [P, I, P, I, P, P, I, P, P, I, P, P, I, I, I, I, I, I, S],
     # residual.hip / gemm_f32.hip / attn_shaped.hip / ssm.hip
-    "ragk_embed_residual": [P, P, P, I, I, I, P, P, F, I, P, P, I, S],
+    "ragk_embed_residual": [P, P, I, P, I, I, I, P, P, F, I, P, P, I, S],
     "ragk_gated_residual": [P, P, I, P, I, I, P, P, P, P, P, P, P, P, I, I, I, I, F, S],
     "ragk_token_shift": [P, I, I, P, P, P, P, P, I, P, P, I, S],
     "ragk_residual_norm": [P, P, I, I, I, P, P, P, I, I, I, I, F, S],

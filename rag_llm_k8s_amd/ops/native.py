@@ -103,12 +103,14 @@ def use_slabs(M, N, K, epi, out_f32=False):
             and N * K >= 1 << 24 and M * N * K >= 8e8 and stream_part_cfg(M, N, K)[1] > 1)
 
 
-def use_vocab(M, N, K, epi):
+def use_vocab(M, N, K, epi, gap=False):
     """fp32 logits go to the slab form of the stream GEMM with one slab: its 64-row tiles keep two blocks a CU and no K-split
     ends in a reduction (32000 x 4096, 4 / 32 rows: stream GEMM 64 / 64 us -> 49 / 48; 32768 x 4096, 11 rows: register-streaming
     kernel, which reads the activations for every 16 columns, 58.6 -> 48.3, 32 rows: 65.7 -> 49.6). The register-streaming
-    kernel keeps vocabularies from 32768 on below 8 rows (128256 x 4096 at 5 rows: 173 us against 184, at 8: 191 against 182)."""
-    return (epi == "none" and (1 if N < 32768 else 8) <= M <= 64 and N >= STREAM_MIN_ROWS and N % 4 == 0
+    kernel keeps vocabularies from 32768 on below 8 rows (128256 x 4096 at 5 rows: 173 us against 184, at 8: 191 against 182) where
+    the weight's rows lie without a gap between them (`gap`, ops/pitch.py; with it 32768 x 4096 at 1 / 4 / 7 rows 48 / 50 / 55 -> 43 / 43 / 43,
+    128256 x 4096 175 / 182 / 202 -> 159 / 159 / 160; in sums no longer than that kernel's, rms error 1.37e-7 on both sides)."""
+    return (epi == "none" and (1 if N < 32768 or gap else 8) <= M <= 64 and N >= STREAM_MIN_ROWS and N % 4 == 0
             and K % 64 == 0)
 
 
@@ -257,9 +259,9 @@ def gemm(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False, path=
         return gemm_mid(x, w, bias=bias, resid=resid, epi=epi, out=out, out_f32=out_f32)
     if path is None and not out_f32 and use_hold(M, N, K, epi) and _vec_rows(x, w) and w.stride(0) < 1 << 24:
         return gemm_hold(x, w, par=bias, epi=epi, out=out)
-    if (path is None and use_vocab(M, N, K, epi) and out_f32 and out.stride(0) == N and _vec_rows(x, w)
+    if (path is None and use_vocab(M, N, K, epi, w.stride(0) != K) and out_f32 and out.stride(0) == N and _vec_rows(x, w)
             and out.data_ptr() % 16 == 0):
-        return gemm_stream_part(x, w, out=out, rows=64, S=1)
+        return gemm_stream_part(x, w, out=out, rows=64, S=1, short_sums=M < 8 and N >= 32768)
     L = _lib.lib()
     ldr = resid.stride(0) if resid is not None else 0
     if path is None and STREAM_DEFAULT and use_stream(M, N, K, epi):
@@ -555,7 +557,7 @@ def _stream_part_cfg(N, K, cus, only, max_s):
 
 def gemm_stream_part(x, w, out=None, rows=None, S=None, short_sums=False):
     """Partial slabs P[S, M, N] (fp32) with P.sum(0) = x @ w^T from the LDS-DMA stream GEMM (bf16 weights). short_sums: a slab is
-    the sum of sums over 512 of K."""
+    the sum of sums over 512 of K (256 up to 2048)."""
     _bf16_2d(x, "x")
     _bf16_2d(w, "w")
     M, K = x.shape
@@ -879,7 +881,7 @@ def mlp_engine_ok(M, w_gu, w_down):
     if w_gu.dtype != torch.bfloat16 or w_down.dtype != torch.bfloat16 or not w_gu.is_cuda:
         return False
     H, I = w_down.shape
-    if w_gu.shape != (2 * I, H) or not (w_gu.is_contiguous() and w_down.is_contiguous()):
+    if w_gu.shape != (2 * I, H) or not (_vec_rows(w_gu) and w_gu.stride(1) == 1 and w_gu.stride(0) >= H and w_down.is_contiguous()):
         return False
     return bool(_lib.lib().ragk_mlp_engine_ok(M, H, I, _cu_count()))
 
@@ -907,8 +909,8 @@ def _mlp_engine_launch(xn_ptr, P_ptr, S, g_ptr, eps, w_gu, w_down, h):
     _req(h.shape == (1, H) and h.is_contiguous(), "h [1, H]")
     _req(mlp_engine_ok(1, w_gu, w_down), "mlp_engine shape")
     ws = _me_workspace(h.device, I)
-    check(_lib.lib().ragk_mlp_engine(xn_ptr, P_ptr, S, g_ptr, eps, w_gu.data_ptr(), w_down.data_ptr(), h.data_ptr(),
-                                     ws.act.data_ptr(), ws.words.data_ptr(), ws.err_ptr, ws.host_dev, ws.tmo_ptr, 1,
+    check(_lib.lib().ragk_mlp_engine(xn_ptr, P_ptr, S, g_ptr, eps, w_gu.data_ptr(),
+                                     w_gu.stride(0), w_down.data_ptr(), h.data_ptr(), ws.act.data_ptr(), ws.words.data_ptr(), ws.err_ptr, ws.host_dev, ws.tmo_ptr, 1,
                                      H, I, _cu_count(), stream_ptr()),
           "ragk_mlp_engine")
     return h
@@ -1089,7 +1091,7 @@ def gemm_fp8(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False):
     _bf16_2d(x, "x")
     M, K = x.shape
     w8, sw = w.w8, w.scale
-    _req(w8.dtype == torch.float8_e4m3fn and w8.is_cuda and w8.is_contiguous() and w8.shape[1] == K, "fp8 weight")
+    _req(w8.dtype == torch.float8_e4m3fn and w8.is_cuda and w8.stride(1) == 1 and w8.shape[1] == K, "fp8 weight")
     _req(sw.dtype == torch.float32 and sw.numel() == w8.shape[0], "fp8 scale")
     _req(K % 128 == 0, "K must be a multiple of 128")
     e = EPI[epi]

@@ -33,7 +33,8 @@ def _vec(t, n, dtype, name):
 def embed_residual(ids, table, carry=None, prev=None, scale=1.0, pos=None, turns=None, n=0):
     """fp32 rows table[ids] * scale, plus the sinusoid of `pos` over the first n columns (turns: fp64 turns per
     position of every column pair)."""
-    _req(ids.dtype == I32 and ids.is_cuda and ids.is_contiguous() and table.is_contiguous(), "ids int32, table dense")
+    _req(ids.dtype == I32 and ids.is_cuda and ids.is_contiguous() and table.stride(1) == 1
+         and table.stride(0) % 8 == 0 and table.data_ptr() % 16 == 0, "ids int32, table rows")
     V, W = table.shape
     f32 = _act(table, "table")
     if carry is not None:
@@ -42,7 +43,7 @@ def embed_residual(ids, table, carry=None, prev=None, scale=1.0, pos=None, turns
         _vec(pos, ids.numel(), I32, "pos")
         _vec(turns, (n + 1) // 2, torch.float64, "turns")
     h = torch.empty((ids.numel(), W), dtype=F32, device=table.device)
-    check(_lib.lib().ragk_embed_residual(ids.data_ptr(), table.data_ptr(), h.data_ptr(), ids.numel(), W, V, ptr(carry),
+    check(_lib.lib().ragk_embed_residual(ids.data_ptr(), table.data_ptr(), table.stride(0), h.data_ptr(), ids.numel(), W, V, ptr(carry),
                                          ptr(prev) if carry is not None else None, float(scale), n, ptr(pos),
                                          ptr(turns) if pos is not None else None, f32, stream_ptr()),
           "ragk_embed_residual")

@@ -1,0 +1,96 @@
+"""Large weights whose rows lie 128 bytes further apart (ops/pitch.py): the same products and embeddings as from dense rows."""
+import pytest
+import torch
+
+from rag_llm_k8s_amd.ops import pitch
+
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("rows,row_bytes,itemsize,gap", [
+    (8192, 8192, 2, True), (8191, 8192, 2, False), (28672, 12288, 2, True), (28672, 14336, 2, False), (16384, 4096, 2, True),
+    (28672, 16384, 2, False), (4096, 4096, 1, True), (4095, 4096, 1, False), (28672, 8192, 1, False), (28672, 8192, 4, False)])
+def test_rule(rows, row_bytes, itemsize, gap):
+    assert pitch.wants_gap(rows, row_bytes, itemsize) == gap
+
+
+def test_host_weights_stay_dense():
+    w = torch.zeros(32768, 2048, dtype=torch.bfloat16)
+    assert pitch.pitched(w) is w
+
+
+def _with_gap(w):
+    out = torch.zeros(w.shape[0], w.shape[1] + pitch.GAP // w.element_size(), dtype=w.dtype, device=w.device)[:, :w.shape[1]]
+    return out.copy_(w)
+
+
+def _randn(*shape, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(sum(shape))
+    return (torch.randn(*shape, generator=g, device=DEV) * scale).bfloat16()
+
+
+@pytest.mark.gpu
+def test_pitched_copy():
+    w = _randn(16384, 2048)
+    p = pitch.pitched(w)
+    assert p.stride() == (2048 + 64, 1) and torch.equal(p, w) and pitch.pitched(p) is p
+    small = w[:16383]
+    assert pitch.pitched(small) is small and pitch.pitched(w[None]).dim() == 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 3, 4, 5, 16, 17, 64, 65, 200, 600])
+def test_products_from_rows_with_a_gap(M):
+    from rag_llm_k8s_amd.ops import native
+    from rag_llm_k8s_amd.ops.fp8 import Fp8Weight, quantize_weight
+
+    x, w = _randn(M, 2048), _randn(4096, 2048, scale=2048 ** -0.5)
+    p = _with_gap(w)
+    for kw in (dict(), dict(out_f32=True), dict(epi="silu_mul"), dict(epi="resid", resid=_randn(M, 4096))):
+        assert torch.equal(native.gemm(x, w, **kw), native.gemm(x, p, **kw)), kw
+    q = quantize_weight(w)
+    qp = Fp8Weight(_with_gap(q.w8.view(torch.uint8)).view(torch.float8_e4m3fn), q.scale)
+    assert torch.equal(native.gemm_fp8(x, q, epi="silu_mul"), native.gemm_fp8(x, qp, epi="silu_mul"))
+    assert torch.equal(native.gemm_fp8(x, q), native.gemm_fp8(x, qp))
+    if M <= 64:
+        assert torch.equal(native.gemm_part(x, w), native.gemm_part(x, p))
+        assert torch.equal(native.gemm_part(x, q), native.gemm_part(x, qp))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 7, 8, 64])
+@pytest.mark.parametrize("N,K", [(32768, 2048), (32776, 4096)])
+def test_vocabulary_with_a_gap(M, N, K):
+    """fp32 logits take the weight stream at any row count then, in sums no longer than the kernel's that dense rows take below
+    eight: its error against 64 bits, with a tenth of room for another order of the sums."""
+    from rag_llm_k8s_amd.ops import native
+
+    x, w = _randn(M, K), _randn(N, K, scale=K ** -0.5)
+    ref = x.double() @ w.double().t()
+    err = [((native.gemm(x, t, out_f32=True).double() - ref).norm() / ref.norm()).item() for t in (w, _with_gap(w))]
+    assert err[1] <= 1.1 * err[0] < 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_embedding_rows_with_a_gap(dtype):
+    from rag_llm_k8s_amd.ops import seq_native
+
+    t = _randn(100, 256).to(dtype)
+    ids = torch.tensor([0, 99, 5, -3, 1000], dtype=torch.int32, device=DEV)
+    assert torch.equal(seq_native.embed_residual(ids.clone(), t), seq_native.embed_residual(ids.clone(), _with_gap(t)))
+    with pytest.raises(ValueError):
+        seq_native.embed_residual(ids.clone(), t[:, 2:250])
+
+
+@pytest.mark.gpu
+def test_mlp_engine_with_a_gap():
+    from rag_llm_k8s_amd.ops import native
+
+    H, I = 4096, 14336
+    w, d = _randn(2 * I, H, scale=H ** -0.5), _randn(H, I, scale=I ** -0.5)
+    p, x, h = _with_gap(w), _randn(1, H), _randn(1, H)
+    if not native.mlp_engine_ok(1, w, d):
+        pytest.skip("no MLP engine on this device")
+    assert native.mlp_engine_ok(1, p, d) and not native.mlp_engine_ok(1, p.t()[:, :H].t()[:, 1:], d)
+    assert torch.equal(native.mlp_engine(x, w, d, h.clone()), native.mlp_engine(x, p, d, h.clone()))

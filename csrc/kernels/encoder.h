@@ -22,6 +22,7 @@ struct EncoderCall {
   float* y;  // few: [T][H]
   int n_layers, T, B, H, I, heads, n_tiles, pooling, normalize, ldo;
   int few, first_pos;  // few: encoder_few.hip's launches, into the row that out points at
+  int l0, l1;          // few: this call's layers of n_layers (l1 0: the last), calls in order sharing their buffers
   float eps;
   Plan plans[4];  // qkv, attention output, up, down
 };

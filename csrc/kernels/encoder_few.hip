@@ -403,14 +403,14 @@ namespace ragk {
 
 // c.few: one sequence of T <= FEW_T rows, H <= FEW_H, head size 32 or 64 (checked again here).
 int encoder_few_forward(const EncoderCall& c, hipStream_t st) {
-  const int H = c.H, T = c.T, D = c.heads > 0 ? H / c.heads : 0;
+  const int H = c.H, T = c.T, D = c.heads > 0 ? H / c.heads : 0, l1 = c.l1 ? c.l1 : c.n_layers;
   if (c.B != 1 || T < 1 || T > FEW_T || H > FEW_H || H % 128 || c.I % 128 || D * c.heads != H || (D != 32 && D != 64) ||
-      c.n_layers < 1 || c.I < 128 || c.I >= 128 * 1024 || (!c.ids && !c.ids_host))
+      c.l0 < 0 || l1 <= c.l0 || c.n_layers < l1 || c.I < 128 || c.I >= 128 * 1024 || (!c.ids && !c.ids_host))
     return (int)hipErrorInvalidValue;
   auto sizes = [&](int K, int N) { return (unsigned)T | (unsigned)(K / 128) << 6 | (unsigned)(N / 16) << 16; };
 #define RAGK_TRY(x) \
   if (const int rc = (x)) return rc
-  for (int l = 0; l < c.n_layers; ++l) {
+  for (int l = c.l0; l < l1; ++l) {
     const void* const* w = c.layers + 12 * l;
     auto b16 = [&](int i) { return (const bf16_t*)w[i]; };
     const float scale = 1.4426950408889634f / sqrtf((float)D);
@@ -436,6 +436,7 @@ int encoder_few_forward(const EncoderCall& c, hipStream_t st) {
     RAGK_TRY(few_plain<EPI_BIAS_RESID>(down, st));
   }
 #undef RAGK_TRY
+  if (l1 < c.n_layers) return 0;
   const void* const* w = c.layers + 12 * (c.n_layers - 1);
   return few_pool(c, (const bf16_t*)w[10], (const bf16_t*)w[11], st);
 }

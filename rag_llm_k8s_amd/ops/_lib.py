@@ -269,7 +269,7 @@ class EncoderCall(ctypes.Structure):
     _fields_ = ([(n, P) for n in ("word", "pos_table", "type_row", "ln_g", "ln_b", "layers", "ids", "pos", "cu", "lens", "tiles",
                                   "rows", "ids_host", "h", "a", "qkv", "attn", "f", "ws", "out", "y")]
                 + [(n, I) for n in ("n_layers", "T", "B", "H", "I", "heads", "n_tiles", "pooling", "normalize", "ldo", "few",
-                                    "first_pos")]
+                                    "first_pos", "l0", "l1")]
                 + [("eps", F), ("plans", GemmPlan * 4)])
 
 

@@ -589,22 +589,14 @@ class NativeBackend(TorchBackend):
         if (ids.dtype != np.int32 or out.dtype != torch.float32 or out.stride(1) != 1 or out.device != w.word.device or T == 0
                 or T * max(3 * cfg.hidden_size, cfg.intermediate_size) * 2 >= 2 ** 31):
             return False
-        weights = self.n.encoder_pointers(cfg, w)
-        if weights is None:
-            return False
-        self.n.encoder_forward(cfg, weights, ids, lens, first_pos, out, rows)
-        return True
+        return self.n.encoder_forward(cfg, w, ids, lens, first_pos, out, rows)
 
     def encoder_few(self, cfg, w, ids, first_pos):
         if not (self.n.encoder_few_ok(cfg, len(ids), 1) and ids.dtype == torch.int32 and ids.is_contiguous()
                 and ids.device == w.word.device):
             return None
-        weights = self.n.encoder_pointers(cfg, w)
-        if weights is None:
-            return None
         out = torch.empty((1, cfg.hidden_size), dtype=torch.float32, device=ids.device)
-        self.n.encoder_few(cfg, weights, ids, first_pos, out[0])
-        return out
+        return out if self.n.encoder_few(cfg, w, ids, first_pos, out[0]) else None
 
     def topk_candidates(self, logits, K, vocab_offset=0, max_cand=512, chunks=None):
         return self.n.topk_candidates(logits, K, vocab_offset=vocab_offset, max_cand=max_cand, chunks=chunks)

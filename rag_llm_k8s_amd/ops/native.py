@@ -1249,24 +1249,28 @@ def pool_l2norm(hidden, cu, mode="cls", normalize=True, out=None):
 ENCODER_LAYER = ("wqkv", "bqkv", "wo", "bo", "ln1_g", "ln1_b", "wi", "bi", "wo2", "bo2", "ln2_g", "ln2_b")
 
 
-def encoder_pointers(cfg, w):
+def encoder_pointers(cfg, w, l0=0, l1=None):
     """Addresses of what encoder_forward reads of an encoder's weights, [word, pos, ln_g, ln_b, type row (or None), then
     ENCODER_LAYER of every layer], or None if one of them would be read wrongly by its address (then: layer by layer through
-    the checked entry points). For the call at hand only, a property at a time over all tensors: 77 of them take 35 us."""
+    the checked entry points). Of layers l0 to l1, the first five with layer 0. For the call at hand only, a property at a time over
+    all tensors: 77 of them take 35 us."""
     H, I, T = cfg.hidden_size, cfg.intermediate_size, torch.Tensor
     if H % 128 or I % 128 or H > 2048 or max(3 * H, I) >= STREAM_MIN_ROWS or H // cfg.num_attention_heads not in (32, 64, 128):
         return None
-    row = w.type_row
-    row = row.view(-1) if row is not None and row.is_contiguous() else row
-    layers = list(itertools.chain.from_iterable(map(operator.itemgetter(*ENCODER_LAYER), w.layers)))
-    ts = [w.word, w.pos, w.ln_g, w.ln_b] + ([row] if row is not None else []) + layers
-    shapes = [(w.word.shape[0], H), (w.pos.shape[0], H)] + [(H,)] * (len(ts) - len(layers) - 2) + [
-        (3 * H, H), (3 * H,), (H, H), (H,), (H,), (H,), (I, H), (I,), (H, I), (H,), (H,), (H,)] * len(w.layers)
+    ts = list(itertools.chain.from_iterable(map(operator.itemgetter(*ENCODER_LAYER), w.layers[l0:l1])))
+    shapes = [(3 * H, H), (3 * H,), (H, H), (H,), (H,), (H,), (I, H), (I,), (H, I), (H,), (H,), (H,)] * (len(ts) // len(ENCODER_LAYER))
+    row = None
+    if l0 == 0:
+        row = w.type_row
+        row = row.view(-1) if row is not None and row.is_contiguous() else row
+        first = [w.word, w.pos, w.ln_g, w.ln_b] + ([row] if row is not None else [])
+        shapes = [(w.word.shape[0], H), (w.pos.shape[0], H)] + [(H,)] * (len(first) - 2) + shapes
+        ts = first + ts
     if (all(map(T.is_contiguous, ts)) and list(map(T.size, ts)) == shapes and [t.dtype for t in ts].count(torch.bfloat16) == len(ts)
             and list(map(T.get_device, ts)).count(w.word.get_device()) == len(ts)):
         at = list(map(T.data_ptr, ts))
         if not any(map((15).__and__, at)):  # the kernels' vectors and LDS-DMA pieces
-            return at if row is not None else at[:4] + [None] + at[4:]
+            return at if row is not None or l0 else at[:4] + [None] + at[4:]
     return None
 
 
@@ -1329,16 +1333,26 @@ def _encoder_call(cfg, weights, bufs, at, T, B):
     return c, ptrs
 
 
-def encoder_few(cfg, weights, ids, first_pos, out):
+# Layers whose weights are checked and whose launches are made at a time: the device begins behind the first three's, not behind all
+# (4 us of checks a layer, 15 to 27 of launches and kernels). A call of one text, waited for, us: 24 layers of 1024, 5 / 16 tokens
+# 748 / 836 -> 645 / 734; 6 of 384, 14 / 30 tokens 164 / 203 -> 164 / 184. Calls behind each other 119 / 560 on both sides.
+FEW_LAYERS = 3
+
+
+def encoder_few(cfg, w, ids, first_pos, out):
     """Embedding of one sequence (encoder_few_ok) into the fp32 row `out`; ids: contiguous int32, on the host (they travel as a
-    kernel argument: nothing is uploaded) or on the device."""
+    kernel argument: nothing is uploaded) or on the device. False, with the row untouched, if encoder_pointers refuses a weight."""
     import ctypes
 
-    H, T = cfg.hidden_size, len(ids)
+    H, T, n = cfg.hidden_size, len(ids), len(w.layers)
+    weights = encoder_pointers(cfg, w, 0, FEW_LAYERS)
+    if weights is None:
+        return False
     _req(out.dtype == torch.float32 and out.is_cuda and out.is_contiguous() and out.numel() == H, "out fp32 row")
     bufs = [("h", 2 * T * H), ("qkv", 6 * T * H), ("f", 2 * T * cfg.intermediate_size), ("y", 4 * T * H)]
     buf = torch.empty(sum(-(-n // 256) * 256 for _, n in bufs), dtype=torch.uint8, device=out.device)
-    c, keep = _encoder_call(cfg, weights, bufs, buf.data_ptr(), T, 1)
+    size = len(ENCODER_LAYER)
+    c, table = _encoder_call(cfg, weights + [None] * (size * n + 5 - len(weights)), bufs, buf.data_ptr(), T, 1)
     c.few, c.first_pos, c.out, c.ldo = 1, first_pos, out.data_ptr(), H
     if isinstance(ids, torch.Tensor):
         _req(ids.is_cuda and ids.dtype == torch.int32 and ids.is_contiguous(), "ids int32")
@@ -1347,25 +1361,36 @@ def encoder_few(cfg, weights, ids, first_pos, out):
         _req(ids.dtype == "int32" and ids.flags.c_contiguous, "ids int32")
         _req_no_capture()
         c.ids_host = ids.ctypes.data
-    check(_lib.lib().ragk_encoder_forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
-    return out
+    c.l1 = min(n, FEW_LAYERS)
+    while True:
+        check(_lib.lib().ragk_encoder_forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
+        if c.l1 == n:
+            return True
+        c.l0, c.l1 = c.l1, min(n, c.l1 + FEW_LAYERS)
+        weights = encoder_pointers(cfg, w, c.l0, c.l1)
+        if weights is None:  # (the last launch writes the row)
+            return False
+        table[size * c.l0:size * c.l1] = weights
 
 
-def encoder_forward(cfg, weights, ids, lens, first_pos, out, rows):
+def encoder_forward(cfg, w, ids, lens, first_pos, out, rows):
     """Embeddings of packed sequences (host int32 ids, int64 lens) into rows `rows` of out (fp32 on the device): one upload
-    of the step's integers, one workspace, one native call for all launches (csrc/kernels/encoder.hip). `weights`: their
-    encoder_pointers."""
+    of the step's integers, one workspace, one native call for all launches (csrc/kernels/encoder.hip). False, with nothing written, if
+    encoder_pointers refuses a weight."""
     import ctypes
 
     import numpy as np
 
     H, I, nh, B, T = cfg.hidden_size, cfg.intermediate_size, cfg.num_attention_heads, len(lens), int(len(ids))
+    few = encoder_few_ok(cfg, T, B)
+    weights = None if few else encoder_pointers(cfg, w)
+    if weights is None and not few:
+        return False
     _req(out.dtype == torch.float32 and out.is_cuda and out.stride(1) == 1 and out.shape[1] == H, "out fp32 rows")
-    if encoder_few_ok(cfg, T, B):
+    if few:
         row = int(rows[0])
         _req(T == int(lens[0]) and len(rows) == 1 and 0 <= row < out.shape[0], "lens, rows")
-        encoder_few(cfg, weights, np.ascontiguousarray(ids), first_pos, out[row])
-        return out
+        return encoder_few(cfg, w, np.ascontiguousarray(ids), first_pos, out[row])
     _req(T == int(lens.sum()) and len(rows) == B and 0 <= int(rows.min()) and int(rows.max()) < out.shape[0], "lens, rows")
     _req(T * max(3 * H, I) * 2 < 2 ** 31, "packed rows past 2 GiB")
     dev = out.device
@@ -1392,7 +1417,7 @@ def encoder_forward(cfg, weights, ids, lens, first_pos, out, rows):
     c.ids, c.pos, c.cu, c.lens, c.rows, c.tiles = (q + 4 * o for o in at[:-1])
     c.out, c.ldo, c.n_tiles = out.data_ptr(), out.stride(0), len(tiles) // 2
     check(L.ragk_encoder_forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
-    return out
+    return True
 
 
 def layernorm_slabs(P, bias, resid, g, b, eps, out=None):

@@ -111,3 +111,38 @@ def test_integers_as_arguments(native):
         dst = torch.full((n + 2,), 7, dtype=torch.int32, device=DEV)
         assert native._lib.lib().ragk_put_ints(src.ctypes.data, n, dst.data_ptr() + 4, native.stream_ptr()) == 0
         assert dst[1:-1].tolist() == src.tolist() and int(dst[0]) == int(dst[-1]) == 7
+
+
+# one call of layers and several, the last of one layer, two, three
+@pytest.mark.parametrize("layers", [1, 3, 4, 5, 6])
+def test_layers_in_several_calls(native, monkeypatch, layers):
+    cfg = E.EncoderConfig(model_type="bert", vocab_size=500, hidden_size=128, num_hidden_layers=layers, num_attention_heads=4,
+                          intermediate_size=256, max_position_embeddings=64, pooling="mean")
+    m = E.EncoderModel(cfg, E.EncoderWeights.random(cfg, DEV, seed=layers), DEV)
+    ids, row, lens = np.arange(5, 17, dtype=np.int32), np.array([0]), np.array([12], dtype=np.int64)
+    out, once = torch.zeros(1, 128, device=DEV), torch.zeros(1, 128, device=DEV)
+    m.embed_into(ids, lens, out, row)
+    monkeypatch.setattr(native, "FEW_LAYERS", layers)
+    m.embed_into(ids, lens, once, row)
+    assert torch.equal(out, once) and bool(out.any())
+    ref = exact(cfg, m.w, torch.from_numpy(ids).to(DEV).long(), m.first_position)
+    assert ((out.to(F64) - ref).norm() / ref.norm()).item() < 0.01  # (test_short_sequence; a layer's roundings grow with their number)
+
+
+def test_a_weight_of_a_later_call_that_is_not_taken(native):
+    """Launches made by then are given up, and the layers go through the checked entry points."""
+    cfg = E.EncoderConfig(model_type="bert", vocab_size=500, hidden_size=128, num_hidden_layers=5, num_attention_heads=4,
+                          intermediate_size=256, max_position_embeddings=64, pooling="mean")
+    m = E.EncoderModel(cfg, E.EncoderWeights.random(cfg, DEV, seed=1), DEV)
+    ids, row, lens = np.arange(5, 17, dtype=np.int32), np.array([0]), np.array([12], dtype=np.int64)
+    out = torch.zeros(1, 128, device=DEV)
+    m.w.layers[4]["wi"] = torch.cat([m.w.layers[4]["wi"]] * 2, 1)[:, :128]
+    assert native.encoder_pointers(cfg, m.w, 0, 3) is not None and native.encoder_pointers(cfg, m.w, 3, 5) is None
+    m.embed_into(ids, lens, out, row)
+    ref = exact(cfg, m.w, torch.from_numpy(ids).to(DEV).long(), m.first_position)
+    assert ((out.to(F64) - ref).norm() / ref.norm()).item() < 0.01
+    m.w.layers[4]["wi"] = m.w.layers[4]["wi"].half()
+    out.fill_(9.0)
+    with pytest.raises(ValueError):
+        m.embed_into(ids, lens, out, row)
+    assert bool((out == 9.0).all())

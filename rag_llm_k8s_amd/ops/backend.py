@@ -493,7 +493,12 @@ class NativeBackend(TorchBackend):
         # 29.2. From 2^24 weights on they are ahead at every row count (niduvik / rolesun 4096 wide, 50 rows: 985 / 1102 -> 775 /
         # 826 us a step). Models 2048 wide, whose steps the host bounds at 30 / 40 rows, lose (543 / 655 -> 569 / 719); the line
         # lies between the two, and long projections of many rows below it forgo the GPU's gain.
-        if isinstance(w, Fp8Weight) or w.dtype != torch.bfloat16:
+        # One byte a weight: whole products read the activations once a few columns, so they cost by rows, slabs hardly (four layers
+        # 4096 wide, 5 / 9 / 16 / 17 / 24 / 33 / 48 / 64 tokens 372 / 387 / 428 / 473 / 524 / 656 / 749 / 869 us in rows, 397 / 392 / 393 / 399 /
+        # 397 / 418 / 443 / 489 in slabs); the line lies where the two cross.
+        if isinstance(w, Fp8Weight):
+            return 12 < M <= 64 and w.shape[0] * w.shape[1] >= 1 << 24 and self.part_ok(M, w)
+        if w.dtype != torch.bfloat16:
             return False
         if M <= 64:
             return w.numel() >= 1 << 24 and self.part_ok(M, w)

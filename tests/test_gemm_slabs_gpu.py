@@ -125,3 +125,58 @@ def test_short_prompt(native, lens, monkeypatch):
     assert bool(((k - k0).abs() <= 2.0 ** -5 * (k0.abs() + k0.roll(64, -1).abs()) + 1e-4).all())
     # logits: two layers of such steps
     assert float((steps[0][0] - steps[1][0]).norm() / steps[1][0].norm()) < 2e-2
+
+
+@pytest.mark.parametrize("lens", [[13], [17], [7, 30, 27]])
+def test_short_prompt_fp8(native, lens, monkeypatch):
+    """From 13 tokens on fp8 prompts go in slabs: the logits are as far from the dequantised weights' in fp32 as with products of
+    rows, give or take their spread."""
+    from rag_llm_k8s_amd.models import llama as L
+    from rag_llm_k8s_amd.models.base import StepInput
+    from rag_llm_k8s_amd.ops.backend import AttnMeta
+    from rag_llm_k8s_amd.utils.synthetic import llama_state_dict
+
+    cfg = L.llama31_8b()
+    cfg.vocab_size, cfg.num_hidden_layers = 512, 2
+    w = L.LlamaWeights.from_state_dict(cfg, llama_state_dict(cfg, seed=0, std=0.02), DEV).quantize_fp8()
+    m = L.LlamaModel(cfg, w, DEV, max_positions=256)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    pos = [p for n in lens for p in range(n)]
+    slots = [s * 64 + p for s, n in enumerate(lens) for p in range(n)]
+    cu = [sum(lens[:i]) for i in range(len(lens) + 1)]
+    ids = [3 + 7 * i % 500 for i in range(len(pos))]
+
+    def step():
+        calls, run = [], L.LlamaModel.hidden_states_few
+        monkeypatch.setattr(m, "hidden_states_few", lambda *a: (calls.append(1), run(m, *a))[1])
+        m.allocate_kv_cache(len(lens))
+        tiles, qtiles = m.prefill_work(lens, DEV)
+        meta = AttnMeta("prefill", i32(lens), i32([[s] for s in range(len(lens))]), cu_q=i32(cu), tiles=tiles, qtiles=qtiles,
+                        host_kv_lens=lens, host_q_lens=lens)
+        lg = m.forward(StepInput(i32(ids), i32(pos), i32(slots), meta, i32([c - 1 for c in cu[1:]])))
+        return lg.double(), len(calls)
+
+    few, n = step()
+    assert n == 1 and not m.be.splits(12, w.layers[0]["wo"]) and not m.be.splits(65, w.layers[0]["wo"])
+    monkeypatch.setattr(m.be, "splits", lambda M, w: False)
+    rows, n = step()
+    assert n == 0
+    # two layers of sums in another order, rounded to bf16 (test_short_prompt)
+    assert float((few - rows).norm() / rows.norm()) < 2e-2
+
+
+@pytest.mark.parametrize("M", [13, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,K", [(6144, 4096), (4096, 4096), (4096, 14336)])
+def test_fp8_slabs_sum_as_closely(native, M, N, K):
+    """Slabs of an fp8 product against 64 bits: fp32 sums no further off than the product of rows has them."""
+    from rag_llm_k8s_amd.ops.fp8 import quantize_weight
+
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    q = quantize_weight(torch.randn(N, K, generator=g, device=DEV) * K ** -0.5)
+    ref = x.double() @ (q.w8.double() * q.scale.double()[:, None]).t()
+    slabs = native.gemm_part(x, q, short_sums=True).double().sum(0)
+    rows = native.gemm_fp8(x, q, out_f32=True).double()
+    err = [float((y - ref).norm() / ref.norm()) for y in (slabs, rows)]
+    print("fp8 slabs", M, N, K, err)
+    assert err[0] <= 1.1 * err[1]

@@ -512,7 +512,7 @@ def gemm_part_norm(h, gamma, eps, w, out=None, ks=None):
 # Batch 32: decode step 7.35 / 7.33 -> 6.91 / 6.98 ms, bench 1568 / 1570 -> 1597 / 1595 tok/s (same box,
 # alternating; profiles/bench_stream_part_ab_r4.log).
 STREAM_PART = True
-STREAM_PART_MIN_M = 5  # batch 8 / 16 -3 %, batch 4 +0.6 %
+STREAM_PART_MIN_M = 5  # batch 8 / 16 -3 %, batch 4 +0.6 %; below, where _part_stream says
 STREAM_PART_ROWS = 0  # 0: by occupancy (ties: 128)
 STREAM_PART_MAX_S = 64  # slabs the consumer sums
 
@@ -555,6 +555,45 @@ def _stream_part_cfg(N, K, cus, only, max_s):
     return best[0], best[1]
 
 
+def _deep_slabs(N, K, cus, only, max_s, few):
+    """Slabs of 64-row tiles where stream_part_cfg's blocks, one round of them, leave more than a third of the CUs without work for
+    slices of 32 K-steps and more: several rounds of slices half as long and shorter, dealt as places come free. 0: not here. Us, one
+    round -> these, at 8 / 17 / 33 / 64 rows: 18688 x 4096 31.9 / 34.0 / 37.9 / 44.4 -> 27.4 / 28.1 / 31.9 / 36.9, 17408 x 4096 31.6 /
+    33.4 / 33.3 / 37.8 -> 26.5 / 26.8 / 30.6 / 35.2, 18688 x 8192 69 / 68 / 72 / 78 -> 62 / 62 / 70 / 76, 18688 x 2048 18.9 / 20.1 /
+    22.6 / 25.8 -> 17.8 / 17.7 / 19.4 / 22.0; two slabs only up to 32 rows (`few`): 10240 x 8192 38.2 / 39.3 / 38.2 / 41.8 -> 35.4 /
+    35.7 / 39.1 / 42.5, 9216 x 4096 18.8 / 20.0 -> 17.8 / 17.6. From 22528 x 4096 on one round is ahead at 33 rows (36.0 against
+    38.6), and at half-full slices of 16 steps always (9344 x 2048 10.8 against 11.3)."""
+    rows, S = _stream_part_cfg(N, K, cus, only, max_s)
+    steps = K // 64
+    if rows != 128 or -(-N // 128) * S > 0.64 * cus or steps // S < 32 or not (S == 1 or (S == 2 and few)):
+        return 0
+    deep = S
+    while steps % (2 * deep) == 0 and steps // (2 * deep) >= 14 and 2 * deep <= max_s:
+        deep *= 2
+    return deep if deep > S else 0
+
+
+@functools.lru_cache(maxsize=4096)
+def _part_stream(M, N, K, cus, min_m, only, max_s, min_blocks):
+    """(rows, S, whether in short sums) of gemm_part's bf16 products on the LDS-DMA weight stream, S 0: gemm_part.hip's.
+
+    Below STREAM_PART_MIN_M rows they go there only where gemm_part.hip's slices are 28 K-steps long and more, in sums over 512 of K,
+    which are no further off (1 / 4 rows, us and rms error in 1e-7: 4096 x 14336 24.9 / 25.2, 1.7 -> 22.0 / 22.0, 1.3; 18688 x 4096
+    35.3 / 35.8, 1.9 -> 28.2 / 27.1, 1.3; 8192 x 28672 92.5 / 93.8, 1.8 -> 75 / 75, 1.4; 6144 x 14336 44 -> 32). Shorter slices are as
+    fast there, in shorter sums, and so are whole rounds of two blocks a CU over rows a multiple of 16 KB apart (8192 x 8192 31.3
+    against 32.6, 4096 x 16384 32.5 against 34.8, 16384 x 8192 56 against 66, but 10240 x 8192 in 1.25 rounds 39 -> 36). Slabs of
+    _deep_slabs are short sums, too: 18688 x 4096 in one 3.9e-7, in four of 1024 1.8, of 512 1.3, for 0 to 3 % of the time."""
+    few = M < min_m
+    if K % 64 or N % 4:
+        return 0, 0, False
+    if few:
+        ks = _part_ksteps(M, N, K, min_blocks)
+        if ks < 28 or (K % 8192 == 0 and -(-N // 64) * (K // (64 * ks)) % (2 * cus) == 0):
+            return 0, 0, False
+    deep = _deep_slabs(N, K, cus, only, max_s, M <= 32)
+    return (64, deep, True) if deep else _stream_part_cfg(N, K, cus, only, max_s) + (few,)
+
+
 def gemm_stream_part(x, w, out=None, rows=None, S=None, short_sums=False):
     """Partial slabs P[S, M, N] (fp32) with P.sum(0) = x @ w^T from the LDS-DMA stream GEMM (bf16 weights). short_sums: a slab is
     the sum of sums over 512 of K (256 up to 2048)."""
@@ -592,9 +631,10 @@ def gemm_part(x, w, out=None, ks=None, short_sums=False):
     M, K = x.shape
     N = wt.shape[0]
     _req(wt.shape[1] == K and M <= 64, "gemm_part shape %s x %s" % (tuple(x.shape), tuple(wt.shape)))
-    if (STREAM_PART and not fp8 and ks is None and out is None and M >= STREAM_PART_MIN_M and K % 64 == 0
-            and N % 4 == 0 and stream_part_cfg(M, N, K)[1] > 0):
-        return gemm_stream_part(x, wt, short_sums=short_sums)
+    if STREAM_PART and not fp8 and ks is None and out is None:
+        rows, S, short = _part_stream(M, N, K, _cu_count(), STREAM_PART_MIN_M, STREAM_PART_ROWS, STREAM_PART_MAX_S, PART_MIN_BLOCKS)
+        if S > 0 and (M >= STREAM_PART_MIN_M or _vec_rows(x, wt)):
+            return gemm_stream_part(x, wt, rows=rows, S=S, short_sums=short_sums or short)
     if fp8 and ks is None and out is None and use_hold_slabs(M, N, K) and _vec_rows(x, wt) and wt.stride(0) < 1 << 24:
         return gemm_hold_slabs(x, wt, w.scale)
     ks, S = gemm_part_slabs(M, N, K, ks)

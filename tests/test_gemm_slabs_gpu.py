@@ -180,3 +180,25 @@ def test_fp8_slabs_sum_as_closely(native, M, N, K):
     err = [float((y - ref).norm() / ref.norm()) for y in (slabs, rows)]
     print("fp8 slabs", M, N, K, err)
     assert err[0] <= 1.1 * err[1]
+
+
+# slabs of several rounds (one slab before, two of a wide product up to 32 rows), few rows whose register-streamed slices are long
+@pytest.mark.parametrize("N,K,M", [(18688, 4096, 1), (18688, 4096, 4), (18688, 4096, 5), (18692, 4096, 17), (18688, 4096, 64),
+                                   (16640, 2048, 64), (9216, 4096, 32), (4096, 14336, 1), (4100, 14336, 4)])
+def test_slabs_of_decode_products(native, monkeypatch, N, K, M):
+    """Sums over no more of K than those that they replace had: no further off from 64 bits, and the whole product."""
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).bfloat16()
+    ref = x.double() @ w.double().t()
+    err = lambda P: float((P.double().sum(0) - ref).norm() / ref.norm())
+    P = native.gemm_part(x, w)
+    if M < native.STREAM_PART_MIN_M:
+        off = torch.cat([x.new_zeros(M, 4), x], 1)[:, 4:]  # rows off 16 bytes stay where they were
+        assert torch.equal(native.gemm_part(x, w, ks=native.gemm_part_slabs(M, N, K)[0]), native.gemm_part(off, w))
+        monkeypatch.setattr(native, "STREAM_PART", False)
+        old = native.gemm_part(x, w)
+    else:
+        assert P.shape[0] > native.stream_part_cfg(M, N, K)[1]
+        old = native.gemm_stream_part(x, w)
+    assert P.shape[1:] == (M, N) and err(P) <= err(old) < 1e-6

@@ -1,0 +1,22 @@
+"""Which split-K slabs a decode step's products take (ops/native.py _deep_slabs)."""
+import pytest
+from hypothesis import given, settings
+from hypothesis import strategies as st
+
+from rag_llm_k8s_amd.ops import native
+
+
+@pytest.mark.parametrize("N,K,few,S", [(18688, 4096, True, 4), (18688, 4096, False, 4), (20480, 4096, True, 4), (22528, 4096, True, 0),
+                                       (16384, 4096, True, 0), (18688, 8192, True, 8), (18688, 3584, True, 4), (18688, 2048, True, 2),
+                                       (9216, 4096, True, 4), (9216, 4096, False, 0), (12288, 4096, True, 0), (9344, 2048, True, 0),
+                                       (10240, 8192, True, 8), (6144, 4096, True, 0), (4096, 14336, True, 0), (28672, 4096, True, 0)])
+def test_where_rounds_of_short_slices_are_ahead(N, K, few, S):
+    assert native._deep_slabs(N, K, 256, 0, 64, few) == S
+
+
+@settings(max_examples=300, deadline=None)
+@given(N=st.integers(1, 40000), steps=st.integers(1, 512), cus=st.sampled_from([64, 256, 304]), few=st.booleans())
+def test_slabs_divide_the_product(N, steps, cus, few):
+    rows, S = native._stream_part_cfg(N, steps * 64, cus, 0, 64)
+    deep = native._deep_slabs(N, steps * 64, cus, 0, 64, few)
+    assert deep == 0 or (deep > S >= 1 and deep <= 64 and steps % deep == 0 and steps // deep >= 14 and -(-N // rows) * S <= cus)

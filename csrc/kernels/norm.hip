@@ -24,10 +24,10 @@ constexpr int NT = 256;
 // (fused residual add: resid holds the new residual stream).
 __global__ __launch_bounds__(NT) void rmsnorm_kernel(const bf16_t* x, int ldx, bf16_t* resid, int ldr,
                                                      const bf16_t* __restrict__ w, bf16_t* out, int ldo,
-                                                     int H, float eps) {
+                                                     int H, float eps, const int* __restrict__ rows) {
   __shared__ float red[NT / 64];
   const int row = blockIdx.x;
-  const bf16_t* xr = x + (size_t)row * ldx;
+  const bf16_t* xr = x + (size_t)(rows ? rows[row] : row) * ldx;
   bf16_t* rr = resid ? resid + (size_t)row * ldr : nullptr;
   bf16_t* orow = out + (size_t)row * ldo;
   constexpr int MAXV = 4;  // up to 4 x 8 x 256 = 8192 columns held in registers
@@ -191,9 +191,13 @@ __global__ __launch_bounds__(NT) void layernorm_slabs_kernel(const float* __rest
 // carry (optional, asynchronous decode): carry[t] >= 0 takes the token id from prev[carry[t]] (the
 // previous decode step's sampled tokens, still on the device) instead of ids[t]; the resolved id is
 // written back to ids[t] so the step's inputs stay self-describing.
+// NORM: and xn[t] = rmsnorm(out[t]) * w as rmsnorm_kernel has it, from the row in registers: the first layer's input, a launch
+// of its own before (four Llama layers 4096 wide, 11 sequences of 2500 tokens in fp8: 406.9 -> 404.3 us a step).
+template <bool NORM>
 __global__ __launch_bounds__(NT) void embed_kernel(int* __restrict__ ids, const bf16_t* __restrict__ table,
                                                    bf16_t* out, int H, int vocab, const int* __restrict__ carry,
-                                                   const int* __restrict__ prev) {
+                                                   const int* __restrict__ prev, const bf16_t* __restrict__ w, bf16_t* xn,
+                                                   float eps) {
   const int t = blockIdx.x;
   int id = ids[t];
   if (carry != nullptr) {
@@ -207,7 +211,47 @@ __global__ __launch_bounds__(NT) void embed_kernel(int* __restrict__ ids, const 
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
   const u32x4* src = reinterpret_cast<const u32x4*>(table + (size_t)id * H);
   u32x4* dst = reinterpret_cast<u32x4*>(out + (size_t)t * H);
-  for (int i = threadIdx.x; i < (H >> 3); i += NT) dst[i] = src[i];
+  if constexpr (!NORM) {
+    for (int i = threadIdx.x; i < (H >> 3); i += NT) dst[i] = src[i];
+  } else {
+    __shared__ float red[NT / 64];
+    constexpr int MAXV = 4;  // as rmsnorm_kernel
+    u32x4 x[MAXV], g[MAXV];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < MAXV; ++i) {
+      const int vi = threadIdx.x + i * NT;
+      if (vi < (H >> 3)) {
+        x[i] = src[vi];
+        g[i] = reinterpret_cast<const u32x4*>(w)[vi];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < MAXV; ++i) {
+      const int vi = threadIdx.x + i * NT;
+      if (vi < (H >> 3)) {
+        dst[vi] = x[i];
+        float v[8];
+        unpack8(x[i], v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+      }
+    }
+    ss = block_sum(ss, red);
+    const float inv = rsqrtf(ss / (float)H + eps);
+#pragma unroll
+    for (int i = 0; i < MAXV; ++i) {
+      const int vi = threadIdx.x + i * NT;
+      if (vi < (H >> 3)) {
+        float v[8], wv[8], o[8];
+        unpack8(x[i], v);
+        unpack8(g[i], wv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = wv[e] * bf2f(f2bf(v[e] * inv));
+        reinterpret_cast<u32x4*>(xn + (size_t)t * H)[vi] = pack8(o);
+      }
+    }
+  }
 }
 
 // BERT / XLM-R embeddings: LN(word[id] + pos[pos_id] + type[type_id]) (+ optional GPT-2 style no-LN), 4 / W rows a block
@@ -360,14 +404,16 @@ __global__ __launch_bounds__(NT) void gather_rows_kernel(const bf16_t* x, int ld
 // ROUNDED = false: h = bf16(h + sum_s P[s][row]), the rounding of a product whose epilogue adds the residual: where a prompt's
 // step may take either form, the one with slabs loses nothing (300 rows, four Llama layers 4096 wide: error of the last values
 // against 64 bits 7.11e-3 with the sum rounded first, 6.80e-3 without and 6.79e-3 from the epilogue).
+// idx: only the rows idx[i], to out[i], and h stays as it is (behind a prompt's last layer nothing reads it): the norm of all 300 rows
+// and a gather behind it before (with the launch saved in front: 300 tokens 856 -> 846 us, 2048 wide, bound by the host, 400 466 -> 449).
 constexpr int PNT = 512;
 template <bool ROUNDED>
 __global__ __launch_bounds__(PNT) void add_partials_rmsnorm_kernel(const float* __restrict__ P, int S, int M,
                                                                    bf16_t* h, int ldh,
                                                                    const bf16_t* __restrict__ w, bf16_t* out,
-                                                                   int ldo, int H, float eps) {
+                                                                   int ldo, int H, float eps, const int* __restrict__ idx) {
   __shared__ float red[PNT / 64];
-  const int row = blockIdx.x;
+  const int row = idx ? idx[blockIdx.x] : blockIdx.x;
   bf16_t* hr = h + (size_t)row * ldh;
   constexpr int MAXV = 2;  // up to 2 x 8 x 512 = 8192 columns in registers
   float v[MAXV][8];
@@ -395,7 +441,7 @@ __global__ __launch_bounds__(PNT) void add_partials_rmsnorm_kernel(const float* 
       unpack8(hv[i], v[i]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[i][e] = bf2f(f2bf(v[i][e] + (ROUNDED ? bf2f(f2bf(a[e])) : a[e])));
-      *reinterpret_cast<u32x4*>(hr + vi * 8) = pack8(v[i]);
+      if (!idx) *reinterpret_cast<u32x4*>(hr + vi * 8) = pack8(v[i]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss += v[i][e] * v[i][e];
     }
@@ -410,7 +456,7 @@ __global__ __launch_bounds__(PNT) void add_partials_rmsnorm_kernel(const float* 
       unpack8(gv[i], wv);
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = wv[e] * bf2f(f2bf(v[i][e] * inv));
-      *reinterpret_cast<u32x4*>(out + (size_t)row * ldo + vi * 8) = pack8(o);
+      *reinterpret_cast<u32x4*>(out + (size_t)blockIdx.x * ldo + vi * 8) = pack8(o);
     }
   }
 }
@@ -470,7 +516,17 @@ RAGK_API int ragk_rmsnorm(const void* x, int ldx, void* resid, int ldr, const vo
   if (rows <= 0) return 0;
   if (H % 8 || H > 8 * NT * 4) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(rmsnorm_kernel, dim3(rows), dim3(NT), 0, st, (const bf16_t*)x, ldx, (bf16_t*)resid, ldr,
-                     (const bf16_t*)w, (bf16_t*)out, ldo, H, eps);
+                     (const bf16_t*)w, (bf16_t*)out, ldo, H, eps, (const int*)nullptr);
+  return (int)hipGetLastError();
+}
+
+// out[i] = rmsnorm(x[rows[i]]) * w
+RAGK_API int ragk_rmsnorm_rows(const void* x, int ldx, const int* rows, const void* w, void* out, int ldo, int n, int H, float eps,
+                               hipStream_t st) {
+  if (n <= 0) return 0;
+  if (H % 8 || H > 8 * NT * 4 || !rows) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(rmsnorm_kernel, dim3(n), dim3(NT), 0, st, (const bf16_t*)x, ldx, (bf16_t*)nullptr, 0, (const bf16_t*)w,
+                     (bf16_t*)out, ldo, H, eps, rows);
   return (int)hipGetLastError();
 }
 
@@ -502,8 +558,8 @@ RAGK_API int ragk_layernorm_slabs(const float* P, int S, const void* bias, const
 RAGK_API int ragk_embed(const int* ids, const void* table, void* out, int T, int H, int vocab, hipStream_t st) {
   if (T <= 0) return 0;
   if (H % 8) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(embed_kernel, dim3(T), dim3(NT), 0, st, const_cast<int*>(ids), (const bf16_t*)table,
-                     (bf16_t*)out, H, vocab, (const int*)nullptr, (const int*)nullptr);
+  hipLaunchKernelGGL(embed_kernel<false>, dim3(T), dim3(NT), 0, st, const_cast<int*>(ids), (const bf16_t*)table,
+                     (bf16_t*)out, H, vocab, (const int*)nullptr, (const int*)nullptr, (const bf16_t*)nullptr, (bf16_t*)nullptr, 0.f);
   return (int)hipGetLastError();
 }
 
@@ -513,8 +569,18 @@ RAGK_API int ragk_embed_carry(int* ids, const int* carry, const int* prev, const
                               int H, int vocab, hipStream_t st) {
   if (T <= 0) return 0;
   if (H % 8 || !carry || !prev) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(embed_kernel, dim3(T), dim3(NT), 0, st, ids, (const bf16_t*)table, (bf16_t*)out, H, vocab,
-                     carry, prev);
+  hipLaunchKernelGGL(embed_kernel<false>, dim3(T), dim3(NT), 0, st, ids, (const bf16_t*)table, (bf16_t*)out, H, vocab,
+                     carry, prev, (const bf16_t*)nullptr, (bf16_t*)nullptr, 0.f);
+  return (int)hipGetLastError();
+}
+
+// Both (carry null: ids as they are), and xn = rmsnorm(out) * w.
+RAGK_API int ragk_embed_rmsnorm(int* ids, const int* carry, const int* prev, const void* table, void* out, const void* w, void* xn,
+                                int T, int H, int vocab, float eps, hipStream_t st) {
+  if (T <= 0) return 0;
+  if (H % 8 || H > 8 * NT * 4 || (carry && !prev) || !w || !xn) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(embed_kernel<true>, dim3(T), dim3(NT), 0, st, ids, (const bf16_t*)table, (bf16_t*)out, H, vocab, carry, prev,
+                     (const bf16_t*)w, (bf16_t*)xn, eps);
   return (int)hipGetLastError();
 }
 
@@ -557,11 +623,12 @@ RAGK_API int ragk_gather_rows(const void* x, int ldx, const int* idx, void* out,
 }
 
 RAGK_API int ragk_add_partials_rmsnorm(const float* P, int S, int M, void* h, int ldh, const void* w, void* out,
-                                       int ldo, int H, float eps, int rounded, hipStream_t st) {
-  if (M <= 0) return 0;
+                                       int ldo, int H, float eps, int rounded, const int* idx, int n, hipStream_t st) {
+  if (M <= 0 || (idx && n <= 0)) return 0;
   if (H % 8 || H > 8 * PNT * 2 || S < 1) return (int)hipErrorInvalidValue;
   const auto kernel = rounded ? add_partials_rmsnorm_kernel<true> : add_partials_rmsnorm_kernel<false>;
-  hipLaunchKernelGGL(kernel, dim3(M), dim3(PNT), 0, st, P, S, M, (bf16_t*)h, ldh, (const bf16_t*)w, (bf16_t*)out, ldo, H, eps);
+  hipLaunchKernelGGL(kernel, dim3(idx ? n : M), dim3(PNT), 0, st, P, S, M, (bf16_t*)h, ldh, (const bf16_t*)w, (bf16_t*)out, ldo, H,
+                     eps, idx);
   return (int)hipGetLastError();
 }
 

@@ -259,12 +259,12 @@ class LlamaModel(DecoderModel):
             self.comm.all_reduce(x)
 
     # one decoder layer in two halves, so tensor-parallel prefill can interleave micro-batches
-    def _attn_block(self, li, L, h, inp: StepInput, attn):
-        """h <- (rank 0: h +) o_proj(attention(rmsnorm(h))): this rank's partial sum before the all-reduce."""
+    def _attn_block(self, li, L, h, inp: StepInput, attn, xn=None):
+        """h <- (rank 0: h +) o_proj(attention(rmsnorm(h))): this rank's partial sum before the all-reduce. xn: the norm, if known."""
         be, c = self.be, self.cfg
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
         kc, vc = self.kv_cache[li]
-        xn = be.rmsnorm(h, L["ln_in"], c.rms_norm_eps)
+        xn = be.rmsnorm(h, L["ln_in"], c.rms_norm_eps) if xn is None else xn
         qkv = be.gemm_rope_kv(xn, L["wqkv"], inp.positions, self.cos, self.sin, inp.slots, kc, vc, Hq, Hkv, D)
         if inp.meta.kind == "decode":
             be.attn_decode(qkv, kc, vc, inp.meta, attn, Hq, Hkv, D)
@@ -286,7 +286,7 @@ class LlamaModel(DecoderModel):
 
     def _final(self, h, inp: StepInput):
         if inp.logits_idx is not None:
-            h = self.be.gather_rows(h, inp.logits_idx)
+            return self.be.rmsnorm_rows(h, inp.logits_idx, self.w.norm, self.cfg.rms_norm_eps)
         return self.be.rmsnorm(h, self.w.norm, self.cfg.rms_norm_eps)
 
     def _tp(self):
@@ -300,8 +300,8 @@ class LlamaModel(DecoderModel):
             return False
         return self.be.part_ok(M, L["wqkv"]) and self.be.part_ok(M, L["wo"]) and self.be.part_ok(M, L["wdown"])
 
-    def hidden_states_decode_part(self, inp: StepInput, h):
-        """Decode step with the split-K partial GEMM (csrc/kernels/gemm_part.hip) for the three
+    def hidden_states_decode_part(self, inp: StepInput, hn):
+        """hn: the embedded rows and their norm for the first layer. Decode step with the split-K partial GEMM (csrc/kernels/gemm_part.hip) for the three
         small-N projections: qkv / o_proj / down write fp32 partial slabs and the following row
         kernel reduces them -- rope_kv_partials (qkv) and add_partials_rmsnorm (o_proj -> post-attention
         norm, down -> next layer's input norm / the final norm), so the reduction adds no launch and
@@ -319,6 +319,7 @@ class LlamaModel(DecoderModel):
         residual into the down GEMM need the full-rank sum first, so they stay TP=1-only.)"""
         be, w, c = self.be, self.w, self.cfg
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
+        h, xn = hn
         M = h.shape[0]
         tp = self._tp()
 
@@ -334,7 +335,6 @@ class LlamaModel(DecoderModel):
         # batch <= 4 (TP): silu(gate) * up inside the down GEMM; the down partials then go through the
         # reduce + norm consumer, so the next layer's input norm is not fused into its qkv GEMM
         silu_fused = tp and be.part_silu_ok(M, layers[0]["wgu"], layers[0]["wdown"])
-        xn = None if fuse_norm else be.rmsnorm(h, layers[0]["ln_in"], c.rms_norm_eps)
         merge = M <= DECODE_OPROJ_MERGE_MAX_M and be.part_merge_ok(M, inp.meta, layers[0]["wo"], Hq, D)
         # batch 1: gate/up + SiLU + down + residual as ONE persistent launch (csrc/kernels/mlp_engine.hip)
         mlp_eng = M == 1 and not tp and be.mlp_engine_ok(M, layers[0]["wgu"], layers[0]["wdown"])
@@ -374,28 +374,28 @@ class LlamaModel(DecoderModel):
     def hidden_states(self, inp: StepInput):
         """Run the decoder stack; returns the final-norm'ed rows selected by logits_idx."""
         be, w = self.be, self.w
-        h = be.embed(inp.ids, w.embed, carry=inp.carry, prev=inp.carry_src)
+        h, xn = be.embed_rmsnorm(inp.ids, w.embed, w.layers[0]["ln_in"], self.cfg.rms_norm_eps, carry=inp.carry, prev=inp.carry_src)
         if self._decode_part_ok(inp, h):
-            return self.hidden_states_decode_part(inp, h)
+            return self.hidden_states_decode_part(inp, (h, xn))
         attn = torch.empty((h.shape[0], self.Hq * self.D), dtype=h.dtype, device=h.device)
         if self.comm is None and inp.meta is not None and inp.meta.kind != "decode":
             L0 = w.layers[0]
             if h.shape[0] <= 64:
                 M = h.shape[0]
                 if inp.slots is not None and be.splits(M, L0["wqkv"]) and be.splits(M, L0["wo"]) and be.splits(M, L0["wdown"]):
-                    return self.hidden_states_few(inp, h, attn)
+                    return self.hidden_states_few(inp, h, xn, attn)
             else:
                 ns = (be.prefill_nsplit(h.shape[0], L0["wo"]), be.prefill_nsplit(h.shape[0], L0["wdown"]))
                 if max(ns) > 1:
-                    return self.hidden_states_splitk(inp, h, attn, *ns)
+                    return self.hidden_states_splitk(inp, h, xn, attn, *ns)
         for li, L in enumerate(w.layers):
-            self._attn_block(li, L, h, inp, attn)
+            self._attn_block(li, L, h, inp, attn, xn if li == 0 else None)
             self._allreduce(h)
             self._mlp_block(L, h)
             self._allreduce(h)
         return self._final(h, inp)
 
-    def hidden_states_few(self, inp: StepInput, h, attn):
+    def hidden_states_few(self, inp: StepInput, h, xn, attn):
         """TP=1 prefill of at most 64 tokens: the decode step's split-K products, whose slabs the rotation and the norms that
         follow sum: as many launches as with products of rows, and the weights at the memory's rate (four layers 4096 wide,
         9 / 20 / 64 tokens: 507 / 601 / 847 us -> 462 / 470 / 531). Where NativeBackend.splits holds: 2048 wide, where the host bounds
@@ -406,7 +406,6 @@ class LlamaModel(DecoderModel):
         layers = w.layers
         part = functools.partial(be.gemm_part, short_sums=True)
         q = torch.empty_like(attn)
-        xn = be.rmsnorm(h, layers[0]["ln_in"], c.rms_norm_eps)
         for li, L in enumerate(layers):
             kc, vc = self.kv_cache[li]
             be.rope_kv_partials(part(xn, L["wqkv"]), q, inp.positions, self.cos, self.sin, inp.slots, kc, vc, Hq, Hkv, D)
@@ -414,10 +413,11 @@ class LlamaModel(DecoderModel):
             xn = be.add_partials_rmsnorm(part(attn, L["wo"]), h, L["ln_post"], c.rms_norm_eps, rounded=False)
             a = be.gemm(xn, L["wgu"], epi="silu_mul")
             nxt = layers[li + 1]["ln_in"] if li + 1 < len(layers) else w.norm
-            xn = be.add_partials_rmsnorm(part(a, L["wdown"]), h, nxt, c.rms_norm_eps, rounded=False)
-        return xn if inp.logits_idx is None else be.gather_rows(xn, inp.logits_idx)
+            rows = inp.logits_idx if li + 1 == len(layers) else None
+            xn = be.add_partials_rmsnorm(part(a, L["wdown"]), h, nxt, c.rms_norm_eps, rounded=False, rows=rows)
+        return xn
 
-    def hidden_states_splitk(self, inp: StepInput, h, attn, ns_o, ns_d):
+    def hidden_states_splitk(self, inp: StepInput, h, xn, attn, ns_o, ns_d):
         """TP=1 prefill of a step whose output tiles leave CUs idle (a few hundred rows): o_proj / down run as split-K GEMMs
         into fp32 slabs (ops/native.py:slab_count) and the residual add moves into the following RMSNorm kernel
         (add_partials_rmsnorm), which the layer needs anyway -- rounded where the residual epilogue rounds, once, behind the
@@ -425,7 +425,6 @@ class LlamaModel(DecoderModel):
         be, w, c = self.be, self.w, self.cfg
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
         layers = w.layers
-        xn = be.rmsnorm(h, layers[0]["ln_in"], c.rms_norm_eps)
         for li, L in enumerate(layers):
             kc, vc = self.kv_cache[li]
             qkv = be.gemm_rope_kv(xn, L["wqkv"], inp.positions, self.cos, self.sin, inp.slots, kc, vc, Hq, Hkv, D)
@@ -437,13 +436,12 @@ class LlamaModel(DecoderModel):
                 xn = be.rmsnorm(h, L["ln_post"], c.rms_norm_eps)
             a = be.gemm(xn, L["wgu"], epi="silu_mul")
             nxt = layers[li + 1]["ln_in"] if li + 1 < len(layers) else w.norm
+            rows = inp.logits_idx if li + 1 == len(layers) else None
             if ns_d > 1:
-                xn = be.add_partials_rmsnorm(be.gemm_splitk(a, L["wdown"], ns_d), h, nxt, c.rms_norm_eps, rounded=False)
+                xn = be.add_partials_rmsnorm(be.gemm_splitk(a, L["wdown"], ns_d), h, nxt, c.rms_norm_eps, rounded=False, rows=rows)
             else:
                 be.gemm(a, L["wdown"], resid=h, epi="resid", out=h)
-                xn = be.rmsnorm(h, nxt, c.rms_norm_eps)
-        if inp.logits_idx is not None:
-            xn = be.gather_rows(xn, inp.logits_idx)
+                xn = be.rmsnorm(h, nxt, c.rms_norm_eps) if rows is None else be.rmsnorm_rows(h, rows, nxt, c.rms_norm_eps)
         return xn
 
     def hidden_states_sp(self, inp: StepInput):

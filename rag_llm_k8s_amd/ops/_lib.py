@@ -64,11 +64,13 @@ _SIGS = {
     "ragk_mlp_engine_split": [I, I, I, I, P],
     "ragk_gemm_part_ksteps": [I, I, I],
     "ragk_gemm_part_set_min_blocks": [I],
-    "ragk_add_partials_rmsnorm": [P, I, I, P, I, P, P, I, I, F, I, S],
+    "ragk_add_partials_rmsnorm": [P, I, I, P, I, P, P, I, I, F, I, P, I, S],
     "ragk_rope_kv_partials": [P, I, I, I, P, I, P, P, P, P, P, P, I, I, I, I, S],
     "ragk_gemm_dec": [P, I, P, I, P, I, P, P, I, I, I, I, I, I, I, P, P, S],
     "ragk_gemm_dec_splits": [I, I, I],
     "ragk_rmsnorm": [P, I, P, I, P, P, I, I, I, F, S],
+    "ragk_rmsnorm_rows": [P, I, P, P, P, I, I, I, F, S],
+    "ragk_embed_rmsnorm": [P, P, P, P, P, P, P, I, I, I, F, S],
     "ragk_layernorm": [P, I, P, I, P, P, P, I, I, I, F, S],
     "ragk_embed": [P, P, P, I, I, I, S],
     "ragk_embed_carry": [P, P, P, P, P, I, I, I, S],

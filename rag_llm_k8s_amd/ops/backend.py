@@ -69,6 +69,9 @@ class TorchBackend:
             return out
         return y
 
+    def rmsnorm_rows(self, x, rows, w, eps):
+        return self.rmsnorm(self.gather_rows(x, rows), w, eps)
+
     def layernorm(self, x, g, b, eps, out=None, resid=None):
         y = R.layernorm(x, g, b, eps, resid=resid)
         if out is not None:
@@ -97,6 +100,11 @@ class TorchBackend:
         if do_ln:
             h = torch.nn.functional.layer_norm(h, (h.shape[-1],), g.float(), b.float(), eps)
         return h.to(word.dtype)
+
+    def embed_rmsnorm(self, ids, table, w, eps, carry=None, prev=None):
+        """(embedding rows, their norm)"""
+        h = self.embed(ids, table, carry=carry, prev=prev)
+        return h, self.rmsnorm(h, w, eps)
 
     def gather_rows(self, x, idx):
         return x[idx.long()]
@@ -173,9 +181,12 @@ class TorchBackend:
         """add_partials_rmsnorm (o_proj slabs + residual + post-attention norm) then mlp_engine, one op."""
         return self.mlp_engine(self.add_partials_rmsnorm(P, h, gamma, eps), w_gu, w_down, h)
 
-    def add_partials_rmsnorm(self, P, h, w, eps, rounded=True):
+    def add_partials_rmsnorm(self, P, h, w, eps, rounded=True, rows=None):
         y = P.sum(0)
-        h.copy_((h.float() + (y.to(h.dtype).float() if rounded else y)).to(h.dtype))
+        s = (h.float() + (y.to(h.dtype).float() if rounded else y)).to(h.dtype)
+        if rows is not None:
+            return R.rmsnorm(s[rows.long()], w, eps)
+        h.copy_(s)
         return R.rmsnorm(h, w, eps)
 
     def rope_kv_partials(self, P, q_out, positions, cos_t, sin_t, slots, kc, vc, Hq, Hkv, D):
@@ -361,6 +372,9 @@ class NativeBackend(TorchBackend):
     def rmsnorm(self, x, w, eps, out=None):
         return self.n.rmsnorm(x, w, eps, out=out)
 
+    def rmsnorm_rows(self, x, rows, w, eps):
+        return self.n.rmsnorm_rows(x, rows, w, eps)
+
     def layernorm(self, x, g, b, eps, out=None, resid=None):
         return self.n.layernorm(x, g, b, eps, out=out, resid=resid)
 
@@ -369,6 +383,9 @@ class NativeBackend(TorchBackend):
 
     def embed(self, ids, table, out=None, carry=None, prev=None):
         return self.n.embed(ids, table, out=out, carry=carry, prev=prev)
+
+    def embed_rmsnorm(self, ids, table, w, eps, carry=None, prev=None):
+        return self.n.embed_rmsnorm(ids, table, w, eps, carry=carry, prev=prev)
 
     def embed_ln(self, ids, pos_ids, word, pos, type_row, g, b, eps, do_ln=True):
         return self.n.embed_ln(ids, pos_ids, word, pos, type_row, g, b, eps, do_ln=do_ln)
@@ -416,8 +433,8 @@ class NativeBackend(TorchBackend):
     def gemm_part_silu(self, pgu, w):
         return self.n.gemm_part_silu(pgu, w)
 
-    def add_partials_rmsnorm(self, P, h, w, eps, rounded=True):
-        return self.n.add_partials_rmsnorm(P, h, w, eps, rounded=rounded)
+    def add_partials_rmsnorm(self, P, h, w, eps, rounded=True, rows=None):
+        return self.n.add_partials_rmsnorm(P, h, w, eps, rounded=rounded, rows=rows)
 
     def mlp_engine_ok(self, M, w_gu, w_down):
         return self.n.mlp_engine_ok(M, w_gu, w_down)

@@ -1190,6 +1190,19 @@ def rmsnorm(x, w, eps, out=None, resid=None):
     return out
 
 
+def rmsnorm_rows(x, rows, w, eps):
+    """rmsnorm(x[rows]) * w."""
+    _bf16_2d(x, "x")
+    H = x.shape[1]
+    _req(w.numel() == H and w.dtype == torch.bfloat16, "weight")
+    _req(H % 8 == 0 and H <= 8192, "H must be a multiple of 8, <= 8192")
+    _req(rows.dtype == torch.int32 and rows.is_cuda, "rows int32")
+    out = torch.empty((rows.numel(), H), dtype=x.dtype, device=x.device)
+    check(_lib.lib().ragk_rmsnorm_rows(x.data_ptr(), x.stride(0), rows.data_ptr(), w.data_ptr(), out.data_ptr(), H, rows.numel(), H,
+                                       float(eps), stream_ptr()), "ragk_rmsnorm_rows")
+    return out
+
+
 def layernorm(x, g, b, eps, out=None, resid=None):
     _bf16_2d(x, "x")
     T, H = x.shape
@@ -1215,6 +1228,21 @@ def embed(ids, table, out=None, carry=None, prev=None):
     check(_lib.lib().ragk_embed_carry(ids.data_ptr(), carry.data_ptr(), prev.data_ptr(), table.data_ptr(),
                                       out.data_ptr(), ids.numel(), H, V, stream_ptr()), "ragk_embed_carry")
     return out
+
+
+def embed_rmsnorm(ids, table, w, eps, carry=None, prev=None):
+    """(embed(ids, table, carry, prev), its rmsnorm * w) in one launch."""
+    _req(ids.dtype == torch.int32 and ids.is_cuda and ids.is_contiguous(), "ids int32")
+    V, H = table.shape
+    _req(table.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.numel() == H, "weight")
+    _req(H % 8 == 0 and H <= 8192, "H must be a multiple of 8, <= 8192")
+    if carry is not None:
+        _req(carry.dtype == torch.int32 and prev.dtype == torch.int32 and carry.numel() >= ids.numel(), "carry int32")
+    h, xn = torch.empty((2, ids.numel(), H), dtype=table.dtype, device=table.device)
+    check(_lib.lib().ragk_embed_rmsnorm(ids.data_ptr(), ptr(carry), ptr(prev) if carry is not None else None, table.data_ptr(),
+                                        h.data_ptr(), w.data_ptr(), xn.data_ptr(), ids.numel(), H, V, float(eps), stream_ptr()),
+          "ragk_embed_rmsnorm")
+    return h, xn
 
 
 def embed_ln(ids, pos_ids, word, pos, type_row, g, b, eps, do_ln=True, out=None):
@@ -1243,18 +1271,23 @@ def rope_kv(qkv, positions, cos_t, sin_t, slots, k_cache, v_cache, Hq, Hkv, D, a
                                   stream_ptr()), "ragk_rope_kv")
 
 
-def add_partials_rmsnorm(P, h, w, eps, out=None, rounded=True):
+def add_partials_rmsnorm(P, h, w, eps, out=None, rounded=True, rows=None):
     """h <- bf16(h + bf16(P.sum(0))) in place; returns rmsnorm(h) * w (split-K decode consumer). rounded=False: the sum is
-    added as it is, as a product's residual epilogue does (prompts, whose steps take either)."""
+    added as it is, as a product's residual epilogue does (prompts, whose steps take either). rows: of these rows only, and h
+    stays as it is."""
     _bf16_2d(h, "h")
     M, H = h.shape
     _req(P.dtype == torch.float32 and P.is_contiguous() and P.dim() == 3 and P.shape[1:] == (M, H), "partials shape")
     _req(w.is_cuda and w.dtype == torch.bfloat16 and w.numel() == H, "norm weight")
-    out = torch.empty_like(h) if out is None else out
-    _req(out.shape == (M, H) and out.stride(1) == 1, "out")
+    n = M
+    if rows is not None:
+        _req(rows.dtype == torch.int32 and rows.is_cuda, "rows int32")
+        n = rows.numel()
+    out = torch.empty((n, H), dtype=h.dtype, device=h.device) if out is None else out
+    _req(out.shape == (n, H) and out.stride(1) == 1, "out")
     check(_lib.lib().ragk_add_partials_rmsnorm(P.data_ptr(), P.shape[0], M, h.data_ptr(), h.stride(0), w.data_ptr(),
-                                               out.data_ptr(), out.stride(0), H, float(eps), int(rounded), stream_ptr()),
-          "ragk_add_partials_rmsnorm")
+                                               out.data_ptr(), out.stride(0), H, float(eps), int(rounded), ptr(rows), n,
+                                               stream_ptr()), "ragk_add_partials_rmsnorm")
     return out
 
 

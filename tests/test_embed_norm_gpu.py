@@ -1,0 +1,49 @@
+"""Launches that took two before, bit for bit: embedding and first norm, norms of selected rows."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def native():
+    from rag_llm_k8s_amd.ops import native
+
+    return native
+
+
+def _i32(v):
+    return torch.tensor(v, dtype=torch.int32, device=DEV)
+
+
+# one vector, a thread's one, two and four of them, a remainder
+@pytest.mark.parametrize("H", [8, 384, 2048, 4104, 8192])
+@pytest.mark.parametrize("carry", [False, True])
+def test_embed_rmsnorm(native, H, carry):
+    table, w = (torch.randn(50, H, device=DEV).bfloat16(), torch.randn(H, device=DEV).bfloat16())
+    ids = _i32([0, 49, 7, 7, -3, 1000])  # (clamped)
+    kw = dict(carry=_i32([-1, 2, -1, 0, -1, 1]), prev=_i32([11, 60, 13])) if carry else {}
+    ids2 = ids.clone()
+    h = native.embed(ids, table, **kw)
+    h2, xn = native.embed_rmsnorm(ids2, table, w, 1e-5, **kw)
+    assert torch.equal(h, h2) and torch.equal(ids, ids2) and torch.equal(xn, native.rmsnorm(h, w, 1e-5))
+
+
+def test_embed_rmsnorm_refuses_wide_rows(native):
+    with pytest.raises(ValueError):
+        native.embed_rmsnorm(_i32([0]), torch.zeros(2, 8200, device=DEV).bfloat16(), torch.zeros(8200, device=DEV).bfloat16(), 1e-5)
+
+
+@pytest.mark.parametrize("H", [384, 4096, 8192])
+@pytest.mark.parametrize("rows", [[0], [69, 3, 3, 0]])
+def test_norms_of_rows(native, H, rows):
+    x, w = torch.randn(70, H, device=DEV).bfloat16(), torch.randn(H, device=DEV).bfloat16()
+    idx = _i32(rows)
+    assert torch.equal(native.rmsnorm_rows(x, idx, w, 1e-5), native.rmsnorm(native.gather_rows(x, idx), w, 1e-5))
+    for S in (1, 3, 9):
+        for rounded in (True, False):
+            P, h = torch.randn(S, 70, H, device=DEV), x.clone()
+            part = native.add_partials_rmsnorm(P, h, w, 1e-5, rounded=rounded, rows=idx)
+            assert torch.equal(h, x)
+            assert torch.equal(part, native.add_partials_rmsnorm(P, h, w, 1e-5, rounded=rounded)[idx.long()])

@@ -1238,7 +1238,8 @@ def embed_rmsnorm(ids, table, w, eps, carry=None, prev=None):
     _req(H % 8 == 0 and H <= 8192, "H must be a multiple of 8, <= 8192")
     if carry is not None:
         _req(carry.dtype == torch.int32 and prev.dtype == torch.int32 and carry.numel() >= ids.numel(), "carry int32")
-    h, xn = torch.empty((2, ids.numel(), H), dtype=table.dtype, device=table.device)
+    h = torch.empty((ids.numel(), H), dtype=table.dtype, device=table.device)
+    xn = torch.empty_like(h)
     check(_lib.lib().ragk_embed_rmsnorm(ids.data_ptr(), ptr(carry), ptr(prev) if carry is not None else None, table.data_ptr(),
                                         h.data_ptr(), w.data_ptr(), xn.data_ptr(), ids.numel(), H, V, float(eps), stream_ptr()),
           "ragk_embed_rmsnorm")

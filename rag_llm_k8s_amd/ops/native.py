@@ -485,6 +485,16 @@ def gemm_part_slabs(M, N, K, ks=None):
     return ks, K // (64 * ks)
 
 
+def _fp8_halves(M, N, ks, S):
+    """Whether fp8 products take slices half as long as (ks, S): up to 16 rows, where their blocks are little more than whole rounds of
+    two a CU, the last of which so leaves most of the chip without work. Us at 1 / 4 / 11 / 16 rows: 9216 x 4096 11.1 / 11.7 / 12.2 /
+    12.6 -> 10.0 / 10.5 / 10.7 / 11.3, 18688 x 4096 20.7 / 21.6 / 22.3 / 22.7 -> 18.1 / 19.8 / 19.5 / 20.1, 7168 x 5120 11.4 / 11.9 /
+    12.5 / 13.0 -> 10.0 / 10.5 / 11.1 / 11.7, 10240 x 8192 20.8 / 22.1 / 22.5 / 22.7 -> 18.6 / 22.6 / 21.4 / 21.5; in full rounds they
+    lose (12288 x 4096 13.6 against 15.0 at 11 rows). More rows read more of x for shorter slices: 18688 x 4096 at 17 21.8, 23.9."""
+    blocks = -(-N // 64) * S
+    return M <= 16 and ks in (16, 32) and blocks < 0.65 * -(-blocks // PART_MIN_BLOCKS) * PART_MIN_BLOCKS
+
+
 def gemm_part_norm(h, gamma, eps, w, out=None, ks=None):
     """gemm_part of rmsnorm(h) * gamma (the norm applied inside the GEMM's activation staging, same
     math as rmsnorm): decode batches <= 4, bf16 weights, K <= 8192."""
@@ -637,8 +647,11 @@ def gemm_part(x, w, out=None, ks=None, short_sums=False):
             return gemm_stream_part(x, wt, rows=rows, S=S, short_sums=short_sums or short)
     if fp8 and ks is None and out is None and use_hold_slabs(M, N, K) and _vec_rows(x, wt) and wt.stride(0) < 1 << 24:
         return gemm_hold_slabs(x, wt, w.scale)
+    chosen = ks is None and out is None
     ks, S = gemm_part_slabs(M, N, K, ks)
     _req(S > 0, "gemm_part: unsupported K=%d" % K)
+    if fp8 and chosen and _fp8_halves(M, N, ks, S):
+        ks, S = ks // 2, 2 * S
     if out is None:
         out = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
     _req(out.dtype == torch.float32 and out.is_contiguous() and out.numel() >= S * M * N, "gemm_part out")

@@ -202,3 +202,20 @@ def test_slabs_of_decode_products(native, monkeypatch, N, K, M):
         assert P.shape[0] > native.stream_part_cfg(M, N, K)[1]
         old = native.gemm_stream_part(x, w)
     assert P.shape[1:] == (M, N) and err(P) <= err(old) < 1e-6
+
+
+@pytest.mark.parametrize("M", [1, 16, 17])
+@pytest.mark.parametrize("N,K,ks", [(9216, 4096, 16), (18688, 4096, 32), (6144, 8192, 16)])
+def test_fp8_slices_where_a_round_is_mostly_empty(native, M, N, K, ks):
+    """Half as long up to 16 rows, and so no further off from 64 bits."""
+    from rag_llm_k8s_amd.ops.fp8 import quantize_weight
+
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    q = quantize_weight(torch.randn(N, K, generator=g, device=DEV) * K ** -0.5)
+    ref = x.double() @ (q.w8.double() * q.scale.double()[:, None]).t()
+    err = lambda P: float((P.double().sum(0) - ref).norm() / ref.norm())
+    P, whole = native.gemm_part(x, q), native.gemm_part(x, q, ks=ks)
+    if M <= 16 and N != 6144:  # (768 blocks of two rounds: full enough)
+        assert P.shape[0] == 2 * whole.shape[0] and err(P) <= err(whole)
+    assert P.shape[1:] == (M, N) and err(P) < 2e-7

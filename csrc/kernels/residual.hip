@@ -57,6 +57,42 @@ __global__ __launch_bounds__(256) void embed_residual_kernel(int* __restrict__ i
   }
 }
 
+// h[t] = table[ids[t]] and out[t] = rmsnorm(h[t]) * w, as embed_residual_kernel and residual_norm_kernel have them: rows of at most a
+// vector a thread, from registers. A launch's way to memory bounds either (steps of four layers in two launches / one, us: 17 x 3000 tokens
+// 621.8 / 619.3, 1 x 300 489.6 / 486.3, 2048 wide 9 x 600 251.7 / 249.5).
+template <typename T, typename TO, int NT>
+__global__ __launch_bounds__(NT) void embed_norm_kernel(int* __restrict__ ids, const T* __restrict__ table, int ldt, float* h, int W,
+                                                        int vocab, const int* __restrict__ carry, const int* __restrict__ prev,
+                                                        const float* __restrict__ w, TO* out, float n, float eps) {
+  __shared__ float red[NT / 64];
+  const int t = blockIdx.x, v = min((int)threadIdx.x, (W >> 3) - 1);
+  float wv[8], f[8], ss = 0.f;
+  ld8(w + v * 8, wv);
+  int id = ids[t];
+  if (carry != nullptr) {
+    const int c = carry[t];
+    if (c >= 0) {
+      id = prev[c];
+      __syncthreads();  // every lane has read ids[t] before lane 0 overwrites it
+      if (threadIdx.x == 0) ids[t] = id;
+    }
+  }
+  id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
+  ld8(table + (size_t)id * ldt + v * 8, f);
+  const bool mine = (int)threadIdx.x < (W >> 3);
+  if (mine) {
+    st8(h + (size_t)t * W + v * 8, f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
+  }
+  const float inv = rsqrtf(block_sum(ss, red) / n + eps);
+  if (!mine) return;
+  float o[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = f[e] * inv * wv[e];
+  st8(out + (size_t)t * W + v * 8, o);
+}
+
 // new row of one vector of the stream -> the shifted row (prev: the row before it)
 template <typename TO>
 __device__ __forceinline__ void put_shifted(TO* dst, const float* x, const float* prev, const float* mix) {
@@ -406,6 +442,26 @@ RAGK_API int ragk_residual_norm(float* h, const void* y, int ldy, int S, int y_b
                    : launch_residual_norm<bf16_t, bf16_t>(h, y, ldy, 1, slab, w_post, w_next, out, M, W, fn, eps, st);
   return out_f32 ? launch_residual_norm<float, float>(h, y, ldy, S, slab, w_post, w_next, out, M, W, fn, eps, st)
                  : launch_residual_norm<float, bf16_t>(h, y, ldy, S, slab, w_post, w_next, out, M, W, fn, eps, st);
+}
+
+// table: [vocab][W] bf16 (f32 = 0) or fp32, rows ldt apart; h: fp32 [T][W], W <= 4096; out: its norm over the first n columns times w,
+// in the table's type. carry / prev may be null.
+RAGK_API int ragk_embed_norm(int* ids, const void* table, int ldt, float* h, int T, int W, int vocab, const int* carry, const int* prev,
+                             const float* w, void* out, int n, float eps, int f32, hipStream_t st) {
+  if (T <= 0) return 0;
+  if (W % 8 || W < 8 || W > 4096 || ldt < W || ldt % 8 || !w || !out || (carry && !prev)) return (int)hipErrorInvalidValue;
+#define RAGK_EN(TT, NT) \
+  hipLaunchKernelGGL((embed_norm_kernel<TT, TT, NT>), dim3(T), dim3(NT), 0, st, ids, (const TT*)table, ldt, h, W, vocab, carry, prev, w, \
+                     (TT*)out, (float)n, eps)
+  if (W <= 2048) {  // (threads as launch_residual_norm has them: the sums are in its order)
+    if (f32) RAGK_EN(float, 256);
+    else RAGK_EN(bf16_t, 256);
+  } else {
+    if (f32) RAGK_EN(float, 512);
+    else RAGK_EN(bf16_t, 512);
+  }
+#undef RAGK_EN
+  return (int)hipGetLastError();
 }
 
 // x: fp32 [M][2F] in packed gate/up tiles, out: fp32 [M][F], F % 64 == 0; par = {limit, alpha, shift} on the device.

@@ -200,8 +200,7 @@ class NiduvikModel(DecoderModel):
         """Final-normed rows selected by logits_idx. `trace` (a list) receives the residual after every layer."""
         be, w, c = self.be, self.w, self.cfg
         n, eps, dt = c.width, c.eps, self.dtype
-        h = be.embed_residual(inp.ids, w.embed, carry=inp.carry, prev=inp.carry_src)
-        xn = be.residual_norm(h, None, None, w.layers[0]["norm1"], eps, n, dt)
+        h, xn = be.embed_norm(inp.ids, w.embed, w.layers[0]["norm1"], eps, n, carry=inp.carry, prev=inp.carry_src)
         shared = {}
         last = w.norm if inp.logits_idx is None else None  # a prompt's final norm runs on the selected rows only
         for li, L in enumerate(w.layers):

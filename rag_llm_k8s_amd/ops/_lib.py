@@ -106,6 +106,7 @@ _SIGS = {
     "ragk_gemm_fp8": [P, I, P, I, P, P, I, P, P, I, P, P, I, I, I, I, I, I, S],
     # residual.hip / gemm_f32.hip / attn_shaped.hip / ssm.hip
     "ragk_embed_residual": [P, P, I, P, I, I, I, P, P, F, I, P, P, I, S],
+    "ragk_embed_norm": [P, P, I, P, I, I, I, P, P, P, P, I, F, I, S],
     "ragk_gated_residual": [P, P, I, P, I, I, P, P, P, P, P, P, P, P, I, I, I, I, F, S],
     "ragk_token_shift": [P, I, I, P, P, P, P, P, I, P, P, I, S],
     "ragk_residual_norm": [P, P, I, I, I, P, P, P, I, I, I, I, F, S],

@@ -249,6 +249,11 @@ class TorchBackend:
         h = self.embed(ids, table, carry=carry, prev=prev).float() * scale
         return h if pos is None else h + RS.sinusoid(pos, turns, n, h.shape[1])
 
+    def embed_norm(self, ids, table, w, eps, n, carry=None, prev=None):
+        """(embedding rows as the fp32 residual stream, their norm over n columns * w in the table's type)"""
+        h = self.embed_residual(ids, table, carry=carry, prev=prev)
+        return h, self.residual_norm(h, None, None, w, eps, n, table.dtype)
+
     def residual_norm(self, h, y, w_post, w_next, eps, n, out_dtype):
         return RS.residual_norm(h, y, w_post, w_next, eps, n, out_dtype)
 
@@ -481,6 +486,9 @@ class NativeBackend(TorchBackend):
     # fp32 residual stream, shaped attention, state-space mixers ---------------
     def embed_residual(self, ids, table, carry=None, prev=None, scale=1.0, pos=None, turns=None, n=0):
         return self.q.embed_residual(ids, table, carry, prev, scale, pos, turns, n)
+
+    def embed_norm(self, ids, table, w, eps, n, carry=None, prev=None):
+        return self.q.embed_norm(ids, table, w, eps, n, carry=carry, prev=prev)
 
     def gated_residual(self, h, y, z, zb, w, eps, n, out_dtype, keep=False, shift=None, meta=None):
         if out_dtype == torch.float32 and keep:  # the stream itself is the fp32 activation

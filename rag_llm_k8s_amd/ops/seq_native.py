@@ -50,6 +50,30 @@ def embed_residual(ids, table, carry=None, prev=None, scale=1.0, pos=None, turns
     return h
 
 
+EMBED_NORM_COLS = 4096  # a vector a thread
+
+
+def embed_norm(ids, table, w, eps, n, carry=None, prev=None):
+    """(embed_residual(ids, table, carry, prev), its norm over n columns * w in the table's type), rows of up to EMBED_NORM_COLS
+    in one launch."""
+    V, W = table.shape
+    f32 = _act(table, "table")
+    if W > EMBED_NORM_COLS:
+        h = embed_residual(ids, table, carry=carry, prev=prev)
+        return h, residual_norm(h, None, None, w, eps, n, table.dtype)
+    _req(ids.dtype == I32 and ids.is_cuda and ids.is_contiguous() and W % 8 == 0
+         and table.stride(0) % 8 == 0 and table.data_ptr() % 16 == 0, "ids int32, table rows")
+    if carry is not None:
+        _req(carry.dtype == I32 and prev.dtype == I32 and carry.numel() >= ids.numel(), "carry int32")
+    _vec(w, W, F32, "w")
+    h = torch.empty((ids.numel(), W), dtype=F32, device=table.device)
+    out = torch.empty((ids.numel(), W), dtype=table.dtype, device=table.device)
+    check(_lib.lib().ragk_embed_norm(ids.data_ptr(), table.data_ptr(), table.stride(0), h.data_ptr(), ids.numel(), W, V, ptr(carry),
+                                     ptr(prev) if carry is not None else None, w.data_ptr(), out.data_ptr(), n, float(eps), f32,
+                                     stream_ptr()), "ragk_embed_norm")
+    return h, out
+
+
 def _slabs(y, M, W, name):
     """(rows are bf16, number of slabs) of rows [M, W] or fp32 slabs [S, M, W]."""
     _req(y.is_cuda and y.dtype in (BF16, F32) and y.is_contiguous() and y.shape[-2:] == (M, W) and y.dim() in (2, 3), name)

@@ -47,3 +47,20 @@ def test_norms_of_rows(native, H, rows):
             part = native.add_partials_rmsnorm(P, h, w, 1e-5, rounded=rounded, rows=idx)
             assert torch.equal(h, x)
             assert torch.equal(part, native.add_partials_rmsnorm(P, h, w, 1e-5, rounded=rounded)[idx.long()])
+
+
+# a vector, a thread's one on 256 and 512 threads, padded columns, rows wider than one launch takes
+@pytest.mark.parametrize("W,n", [(8, 8), (384, 380), (2048, 2048), (2056, 2050), (4096, 4096), (4224, 4200)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("carry", [False, True])
+def test_embed_norm(W, n, dtype, carry):
+    from rag_llm_k8s_amd.ops import seq_native
+
+    table, w = torch.randn(50, W + 64, device=DEV).to(dtype)[:, :W], torch.randn(W, device=DEV)
+    ids = _i32([0, 49, 7, 7, -3, 1000])
+    kw = dict(carry=_i32([-1, 2, -1, 0, -1, 1]), prev=_i32([11, 60, 13])) if carry else {}
+    ids2 = ids.clone()
+    h = seq_native.embed_residual(ids, table, **kw)
+    h2, xn = seq_native.embed_norm(ids2, table, w, 1e-5, n, **kw)
+    assert torch.equal(h, h2) and torch.equal(ids, ids2)
+    assert torch.equal(xn, seq_native.residual_norm(h, None, None, w, 1e-5, n, dtype))

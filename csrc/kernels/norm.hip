@@ -622,9 +622,11 @@ RAGK_API int ragk_gather_rows(const void* x, int ldx, const int* idx, void* out,
   return (int)hipGetLastError();
 }
 
+// idx null: all M rows, n = M. A selection without rows has no address either, so that one alone does not say which of the two is meant.
 RAGK_API int ragk_add_partials_rmsnorm(const float* P, int S, int M, void* h, int ldh, const void* w, void* out,
                                        int ldo, int H, float eps, int rounded, const int* idx, int n, hipStream_t st) {
-  if (M <= 0 || (idx && n <= 0)) return 0;
+  if (!idx && n != M) return (int)hipErrorInvalidValue;
+  if (M <= 0 || n <= 0) return 0;
   if (H % 8 || H > 8 * PNT * 2 || S < 1) return (int)hipErrorInvalidValue;
   const auto kernel = rounded ? add_partials_rmsnorm_kernel<true> : add_partials_rmsnorm_kernel<false>;
   hipLaunchKernelGGL(kernel, dim3(idx ? n : M), dim3(PNT), 0, st, P, S, M, (bf16_t*)h, ldh, (const bf16_t*)w, (bf16_t*)out, ldo, H,

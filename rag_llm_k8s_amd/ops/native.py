@@ -1209,7 +1209,7 @@ def rmsnorm_rows(x, rows, w, eps):
     H = x.shape[1]
     _req(w.numel() == H and w.dtype == torch.bfloat16, "weight")
     _req(H % 8 == 0 and H <= 8192, "H must be a multiple of 8, <= 8192")
-    _req(rows.dtype == torch.int32 and rows.is_cuda, "rows int32")
+    _req(rows.dtype == torch.int32 and rows.is_cuda and rows.is_contiguous(), "rows int32")
     out = torch.empty((rows.numel(), H), dtype=x.dtype, device=x.device)
     check(_lib.lib().ragk_rmsnorm_rows(x.data_ptr(), x.stride(0), rows.data_ptr(), w.data_ptr(), out.data_ptr(), H, rows.numel(), H,
                                        float(eps), stream_ptr()), "ragk_rmsnorm_rows")
@@ -1295,10 +1295,12 @@ def add_partials_rmsnorm(P, h, w, eps, out=None, rounded=True, rows=None):
     _req(w.is_cuda and w.dtype == torch.bfloat16 and w.numel() == H, "norm weight")
     n = M
     if rows is not None:
-        _req(rows.dtype == torch.int32 and rows.is_cuda, "rows int32")
+        _req(rows.dtype == torch.int32 and rows.is_cuda and rows.is_contiguous(), "rows int32")
         n = rows.numel()
     out = torch.empty((n, H), dtype=h.dtype, device=h.device) if out is None else out
     _req(out.shape == (n, H) and out.stride(1) == 1, "out")
+    if n == 0:
+        return out
     check(_lib.lib().ragk_add_partials_rmsnorm(P.data_ptr(), P.shape[0], M, h.data_ptr(), h.stride(0), w.data_ptr(),
                                                out.data_ptr(), out.stride(0), H, float(eps), int(rounded), ptr(rows), n,
                                                stream_ptr()), "ragk_add_partials_rmsnorm")

@@ -400,7 +400,7 @@ RAGK_API int ragk_gemm_fp8(const void* x_bf16, int ldx, const void* A8, int lda,
                            int ldb, const float* sb, void* C, int ldc, const void* bias, const void* resid, int ldr,
                            int M, int N, int K, int epi, int out_f32, hipStream_t st) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  if (K % 128) return (int)hipErrorInvalidValue;
+  if (K % 128 || ldb % 16) return (int)hipErrorInvalidValue;  // (rows in 16-byte pieces)
   const bool dec = x_bf16 != nullptr;
   if (dec && M > 64) return (int)hipErrorInvalidValue;
   if (epi == EPI_SILU_MUL) {

@@ -501,7 +501,7 @@ RAGK_API int ragk_gemm_stream(const void* X, int ldx, const void* W, int ldw, co
   if (M <= 0 || N <= 0) return 0;
   const bool fp8 = wscale != nullptr;
   const int kstep = fp8 ? 128 : 64;
-  if (M > 64 || K % kstep || S < 1 || (K / kstep) % S) return (int)hipErrorInvalidValue;
+  if (M > 64 || K % kstep || S < 1 || (K / kstep) % S || (fp8 && ldw % 16)) return (int)hipErrorInvalidValue;
   if (S > 1 && (!ws || !counters)) return (int)hipErrorInvalidValue;
   if (epi == EPI_SILU_MUL) {
     if (N % 64 || out_f32) return (int)hipErrorInvalidValue;

@@ -1144,7 +1144,10 @@ def gemm_fp8(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False):
     _bf16_2d(x, "x")
     M, K = x.shape
     w8, sw = w.w8, w.scale
-    _req(w8.dtype == torch.float8_e4m3fn and w8.is_cuda and w8.stride(1) == 1 and w8.shape[1] == K, "fp8 weight")
+    _req(w8.dtype == torch.float8_e4m3fn and w8.is_cuda and w8.dim() == 2 and w8.shape[1] == K
+         and (w8.is_contiguous() or (w8.stride(1) == 1 and w8.stride(0) >= K and w8.stride(0) % 16 == 0)), "fp8 weight")
+    if (w8.data_ptr() | w8.stride(0)) & 15:  # (the kernels' LDS-DMA pieces start on 16 bytes)
+        w8 = w8.clone(memory_format=torch.contiguous_format)
     _req(sw.dtype == torch.float32 and sw.numel() == w8.shape[0], "fp8 scale")
     _req(K % 128 == 0, "K must be a multiple of 128")
     e = EPI[epi]
@@ -1164,13 +1167,14 @@ def gemm_fp8(x, w, bias=None, resid=None, epi="none", out=None, out_f32=False):
     if M == 0:
         return out
     ldr = resid.stride(0) if resid is not None else 0
-    if epi == "silu_mul" and use_hold_slabs_silu(M, K) and _vec_rows(x, w8, out):
+    near = w8.stride(0) < 1 << 24  # a lane's row is a 32-bit offset in gemm_hold
+    if epi == "silu_mul" and use_hold_slabs_silu(M, K) and near and _vec_rows(x, w8, out):
         ws = torch.empty(K // 2048 * M * 2 * N, dtype=torch.float32, device=x.device)
         check(_lib.lib().ragk_gemm_hold_slabs_silu(x.data_ptr(), x.stride(0), w8.data_ptr(), w8.stride(0), sw.data_ptr(),
                                                    out.data_ptr(), out.stride(0), M, N, K, _cu_count(), ws.data_ptr(),
                                                    stream_ptr()), "ragk_gemm_hold_slabs_silu")
         return out
-    if use_hold(M, N, K, epi, fp8=True) and _vec_rows(x, w8):
+    if use_hold(M, N, K, epi, fp8=True) and near and _vec_rows(x, w8):
         return gemm_hold(x, w8, sw, epi=epi, out=out)
     if M <= DEC_MAX_M and FP8_DEC_STREAM and use_stream(M, N, K, epi, fp8=True):
         rc = _gemm_stream(x, w8, sw, out, bias, resid, ldr, M, N, K, epi, e, out_f32)

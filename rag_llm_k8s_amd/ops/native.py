@@ -1235,6 +1235,7 @@ def embed(ids, table, out=None, carry=None, prev=None):
     """Embedding gather. carry/prev (asynchronous decode): rows with carry[t] >= 0 take their token id
     from prev[carry[t]] (the previous step's sampled tokens on the device) and store it into ids[t]."""
     _req(ids.dtype == torch.int32 and ids.is_cuda and ids.is_contiguous(), "ids int32")
+    _req(table.is_contiguous(), "table rows without gaps")
     V, H = table.shape
     out = torch.empty((ids.numel(), H), dtype=table.dtype, device=table.device) if out is None else out
     if carry is None:
@@ -1251,7 +1252,8 @@ def embed_rmsnorm(ids, table, w, eps, carry=None, prev=None):
     """(embed(ids, table, carry, prev), its rmsnorm * w) in one launch."""
     _req(ids.dtype == torch.int32 and ids.is_cuda and ids.is_contiguous(), "ids int32")
     V, H = table.shape
-    _req(table.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.numel() == H, "weight")
+    _req(table.dtype == torch.bfloat16 and table.is_contiguous(), "bf16 table rows without gaps")
+    _req(w.dtype == torch.bfloat16 and w.numel() == H, "weight")
     _req(H % 8 == 0 and H <= 8192, "H must be a multiple of 8, <= 8192")
     if carry is not None:
         _req(carry.dtype == torch.int32 and prev.dtype == torch.int32 and carry.numel() >= ids.numel(), "carry int32")

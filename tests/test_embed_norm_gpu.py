@@ -35,6 +35,17 @@ def test_embed_rmsnorm_refuses_wide_rows(native):
         native.embed_rmsnorm(_i32([0]), torch.zeros(2, 8200, device=DEV).bfloat16(), torch.zeros(8200, device=DEV).bfloat16(), 1e-5)
 
 
+def test_embeddings_refuse_rows_with_gaps(native):
+    """Both read row id at id * H."""
+    wide, w = torch.randn(50, 448, device=DEV).bfloat16(), torch.randn(384, device=DEV).bfloat16()
+    for table in (wide[:, :384], wide[:, :384].t().contiguous().t()):
+        with pytest.raises(ValueError):
+            native.embed(_i32([0, 3]), table)
+        with pytest.raises(ValueError):
+            native.embed_rmsnorm(_i32([0, 3]), table, w, 1e-5)
+    assert torch.equal(native.embed_rmsnorm(_i32([0, 0]), wide[7:8, :384], w, 1e-5)[0], wide[7, :384].expand(2, -1))  # one row has none
+
+
 @pytest.mark.parametrize("H", [384, 4096, 8192])
 @pytest.mark.parametrize("rows", [[0], [69, 3, 3, 0]])
 def test_norms_of_rows(native, H, rows):

@@ -30,20 +30,28 @@ def _vec(t, n, dtype, name):
 
 
 # ------------------------------------------------------------------------------------- residual stream
+def _table_pitch(table):
+    """Values between the starts of an embedding's rows: dense ones may start anywhere, others in whole vectors."""
+    if table.is_contiguous():
+        return table.shape[1]
+    _req(table.stride(0) % 8 == 0 and table.data_ptr() % 16 == 0, "table rows")
+    return table.stride(0)
+
+
 def embed_residual(ids, table, carry=None, prev=None, scale=1.0, pos=None, turns=None, n=0):
     """fp32 rows table[ids] * scale, plus the sinusoid of `pos` over the first n columns (turns: fp64 turns per
     position of every column pair)."""
-    _req(ids.dtype == I32 and ids.is_cuda and ids.is_contiguous() and table.stride(1) == 1
-         and table.stride(0) % 8 == 0 and table.data_ptr() % 16 == 0, "ids int32, table rows")
-    V, W = table.shape
+    _req(ids.dtype == I32 and ids.is_cuda and ids.is_contiguous(), "ids int32")
     f32 = _act(table, "table")
+    V, W = table.shape
+    ldt = _table_pitch(table)
     if carry is not None:
         _req(carry.dtype == I32 and prev.dtype == I32 and carry.numel() >= ids.numel(), "carry int32")
     if pos is not None:
         _vec(pos, ids.numel(), I32, "pos")
         _vec(turns, (n + 1) // 2, torch.float64, "turns")
     h = torch.empty((ids.numel(), W), dtype=F32, device=table.device)
-    check(_lib.lib().ragk_embed_residual(ids.data_ptr(), table.data_ptr(), table.stride(0), h.data_ptr(), ids.numel(), W, V, ptr(carry),
+    check(_lib.lib().ragk_embed_residual(ids.data_ptr(), table.data_ptr(), ldt, h.data_ptr(), ids.numel(), W, V, ptr(carry),
                                          ptr(prev) if carry is not None else None, float(scale), n, ptr(pos),
                                          ptr(turns) if pos is not None else None, f32, stream_ptr()),
           "ragk_embed_residual")
@@ -56,19 +64,19 @@ EMBED_NORM_COLS = 4096  # a vector a thread
 def embed_norm(ids, table, w, eps, n, carry=None, prev=None):
     """(embed_residual(ids, table, carry, prev), its norm over n columns * w in the table's type), rows of up to EMBED_NORM_COLS
     in one launch."""
-    V, W = table.shape
     f32 = _act(table, "table")
+    V, W = table.shape
     if W > EMBED_NORM_COLS:
         h = embed_residual(ids, table, carry=carry, prev=prev)
         return h, residual_norm(h, None, None, w, eps, n, table.dtype)
-    _req(ids.dtype == I32 and ids.is_cuda and ids.is_contiguous() and W % 8 == 0
-         and table.stride(0) % 8 == 0 and table.data_ptr() % 16 == 0, "ids int32, table rows")
+    _req(ids.dtype == I32 and ids.is_cuda and ids.is_contiguous() and W % 8 == 0, "ids int32, table rows")
+    ldt = _table_pitch(table)
     if carry is not None:
         _req(carry.dtype == I32 and prev.dtype == I32 and carry.numel() >= ids.numel(), "carry int32")
     _vec(w, W, F32, "w")
     h = torch.empty((ids.numel(), W), dtype=F32, device=table.device)
     out = torch.empty((ids.numel(), W), dtype=table.dtype, device=table.device)
-    check(_lib.lib().ragk_embed_norm(ids.data_ptr(), table.data_ptr(), table.stride(0), h.data_ptr(), ids.numel(), W, V, ptr(carry),
+    check(_lib.lib().ragk_embed_norm(ids.data_ptr(), table.data_ptr(), ldt, h.data_ptr(), ids.numel(), W, V, ptr(carry),
                                      ptr(prev) if carry is not None else None, w.data_ptr(), out.data_ptr(), n, float(eps), f32,
                                      stream_ptr()), "ragk_embed_norm")
     return h, out

@@ -60,6 +60,26 @@ def test_norms_of_rows(native, H, rows):
             assert torch.equal(part, native.add_partials_rmsnorm(P, h, w, 1e-5, rounded=rounded)[idx.long()])
 
 
+@pytest.mark.parametrize("W", [384, 4096, 4224])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_dense_tables_may_start_anywhere(W, dtype):
+    from rag_llm_k8s_amd.ops import seq_native
+
+    t, w, ids = torch.randn(20, W, device=DEV).to(dtype), torch.randn(W, device=DEV), _i32([0, 19, 7])
+    off = 8 // t.element_size()  # 8 bytes
+    moved = torch.cat([t.new_zeros(off), t.flatten()])[off:].view(20, W)
+    one = torch.as_strided(moved, (1, W), (4, 1), moved.storage_offset() + 7 * W)  # a single row has no distance to another
+    assert moved.data_ptr() % 16 and torch.equal(seq_native.embed_residual(ids, moved), seq_native.embed_residual(ids, t))
+    assert torch.equal(seq_native.embed_residual(_i32([0]), one), t[7:8].float())
+    for a, b in zip(seq_native.embed_norm(ids, moved, w, 1e-5, W), seq_native.embed_norm(ids, t, w, 1e-5, W)):
+        assert torch.equal(a, b)
+    for table in (torch.as_strided(t, (9, W), (W + 4, 1)), torch.as_strided(t, (9, W), (8, 1)), moved[:, :W - 8]):
+        with pytest.raises((ValueError, RuntimeError)):
+            seq_native.embed_residual(ids, table)
+        with pytest.raises((ValueError, RuntimeError)):
+            seq_native.embed_norm(ids, table, w[:table.shape[1]], 1e-5, 8)
+
+
 # a vector, a thread's one on 256 and 512 threads, padded columns, rows wider than one launch takes
 @pytest.mark.parametrize("W,n", [(8, 8), (384, 380), (2048, 2048), (2056, 2050), (4096, 4096), (4224, 4200)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

@@ -293,15 +293,22 @@ class LlamaModel(DecoderModel):
         return self.comm is not None and self.comm.size > 1
 
     def _decode_part_ok(self, inp: StepInput, h):
+        return self._part_rows_ok(inp, *h.shape)
+
+    def _part_rows_ok(self, inp: StepInput, M, H):
         if inp.meta is None or inp.meta.kind != "decode" or inp.slots is None:
             return False
-        L, M = self.w.layers[0], h.shape[0]
-        if self._tp() and not self.comm.fused_decode_ok(M, h.shape[1]):
+        L = self.w.layers[0]
+        if self._tp() and not self.comm.fused_decode_ok(M, H):
             return False
         return self.be.part_ok(M, L["wqkv"]) and self.be.part_ok(M, L["wo"]) and self.be.part_ok(M, L["wdown"])
 
+    def _norm_fused(self, M):
+        """Whether a decode step's input norms run inside the qkv GEMM (gemm_part_norm): batch <= 4, one launch fewer a layer."""
+        return M <= DECODE_DOWN_SKINNY_MAX_M and not self._tp() and self.be.part_norm_ok(M, self.w.layers[0]["wqkv"])
+
     def hidden_states_decode_part(self, inp: StepInput, hn):
-        """hn: the embedded rows and their norm for the first layer. Decode step with the split-K partial GEMM (csrc/kernels/gemm_part.hip) for the three
+        """hn: the embedded rows and, unless _norm_fused, their norm for the first layer. Decode step with the split-K partial GEMM (csrc/kernels/gemm_part.hip) for the three
         small-N projections: qkv / o_proj / down write fp32 partial slabs and the following row
         kernel reduces them -- rope_kv_partials (qkv) and add_partials_rmsnorm (o_proj -> post-attention
         norm, down -> next layer's input norm / the final norm), so the reduction adds no launch and
@@ -330,8 +337,7 @@ class LlamaModel(DecoderModel):
 
         attn = torch.empty((M, Hq * D), dtype=h.dtype, device=h.device)
         layers = w.layers
-        # batch <= 4: the input norm runs inside the qkv GEMM (gemm_part_norm) -- one launch fewer per layer
-        fuse_norm = M <= DECODE_DOWN_SKINNY_MAX_M and not tp and be.part_norm_ok(M, layers[0]["wqkv"])
+        fuse_norm = self._norm_fused(M)
         # batch <= 4 (TP): silu(gate) * up inside the down GEMM; the down partials then go through the
         # reduce + norm consumer, so the next layer's input norm is not fused into its qkv GEMM
         silu_fused = tp and be.part_silu_ok(M, layers[0]["wgu"], layers[0]["wdown"])
@@ -374,8 +380,12 @@ class LlamaModel(DecoderModel):
     def hidden_states(self, inp: StepInput):
         """Run the decoder stack; returns the final-norm'ed rows selected by logits_idx."""
         be, w = self.be, self.w
+        M = inp.ids.numel()
+        part = self._part_rows_ok(inp, M, w.embed.shape[1])
+        if part and self._norm_fused(M):
+            return self.hidden_states_decode_part(inp, (be.embed(inp.ids, w.embed, carry=inp.carry, prev=inp.carry_src), None))
         h, xn = be.embed_rmsnorm(inp.ids, w.embed, w.layers[0]["ln_in"], self.cfg.rms_norm_eps, carry=inp.carry, prev=inp.carry_src)
-        if self._decode_part_ok(inp, h):
+        if part:
             return self.hidden_states_decode_part(inp, (h, xn))
         attn = torch.empty((h.shape[0], self.Hq * self.D), dtype=h.dtype, device=h.device)
         if self.comm is None and inp.meta is not None and inp.meta.kind != "decode":

@@ -229,7 +229,8 @@ __global__ __launch_bounds__(ME_THREADS, 1) void mlp_engine_kernel(MlpArgs a) {
   m.KB = a.I / ME_KC;
   // activation groups split in proportion to per-XCD stream rate (dispatch order w % 8 = XCD): the
   // workgroups on even XCDs streamed the same phase-A work ~15 % slower, repeatably (correlation 0.97
-  // launch to launch, profiles/mlp_engine_skew_r5.log), and the hand-off waits for the slowest
+  // launch to launch, profiles/mlp_engine_skew_r5.log) where gate/up rows lie 8 KB apart, and the hand-off
+  // waits for the slowest (me_weights)
   int rng[4];
   me_split(G, w, NA, ND, a.w_even, a.w_odd, rng);
   m.a0 = rng[0];
@@ -523,37 +524,51 @@ __global__ __launch_bounds__(ME_THREADS, 1) void mlp_engine_kernel(MlpArgs a) {
 int g_me_nt = 1;
 // measured per-XCD rate ratio ~0.84; for Llama-3.1-8B on 256 CUs (7 groups per workgroup on average)
 // 27 : 32 and 3 : 4 give the same integer split, 6 : 8 groups (profiles/mlp_engine_xcd_weights_r5.log)
-int g_me_w_even = 3, g_me_w_odd = 4;
+// where rows lie 8 KB apart; with a gap between them the even split is as good or better (3 : 4 and 1 : 1, us: dense 66.0 and 65.9,
+// gap 68.4 and 65.7, on another card 64.9 and 64.7)
+int g_me_w_even = 0, g_me_w_odd = 0;  // 0: by the rows' distance
 unsigned long long* g_me_stamps = nullptr;
+
+void me_weights(int H, int ldgu, int& we, int& wo) {
+  we = g_me_w_even ? g_me_w_even : ldgu == H ? 3 : 1;
+  wo = g_me_w_odd ? g_me_w_odd : ldgu == H ? 4 : 1;
+}
 
 }  // namespace
 
-// Whether the engine takes this shape on a grid of G workgroups (G = CU count).
-RAGK_API int ragk_mlp_engine_ok(int M, int H, int I, int G) {
-  if (M != 1 || G < 1 || H <= 0 || I <= 0) return 0;
+// Whether the engine takes this shape on a grid of G workgroups (G = CU count), gate/up rows ldgu apart.
+RAGK_API int ragk_mlp_engine_rows_ok(int M, int H, int I, int G, int ldgu) {
+  if (M != 1 || G < 1 || H <= 0 || I <= 0 || ldgu < H || ldgu % 8) return 0;
   if (H % ME_KC || I % ME_KC || I % 64 || H % 16) return 0;
   if (2 * H > ME_VEC || 2 * I > ME_VEC) return 0;
   const int NA = I / 8, ND = H / 16;
-  const long long T = me_cum(G, g_me_w_even, g_me_w_odd);
-  const int wmax = g_me_w_even > g_me_w_odd ? g_me_w_even : g_me_w_odd;
+  int we, wo;
+  me_weights(H, ldgu, we, wo);
+  const long long T = me_cum(G, we, wo);
+  const int wmax = we > wo ? we : wo;
   const int maxA = (int)(((long long)NA * wmax + T - 1) / T), maxB = (ND + G - 1) / G;  // floor-difference bound
   if (maxA * (H / ME_KC) > ME_MAXA || maxB * (I / ME_KC) > ME_MAXB || maxA * 8 > 64 || maxB * 16 > 64) return 0;
   return 1;
 }
 
+RAGK_API int ragk_mlp_engine_ok(int M, int H, int I, int G) { return ragk_mlp_engine_rows_ok(M, H, I, G, H); }
+
 // The kernel's work split for workgroup w of G (CPU-tested: every activation group and down row group
 // owned exactly once, per-workgroup slot counts within the LDS partial capacity).
-RAGK_API int ragk_mlp_engine_split(int G, int w, int H, int I, int* out4) {
+RAGK_API int ragk_mlp_engine_rows_split(int G, int w, int H, int I, int ldgu, int* out4) {
   if (G < 1 || w < 0 || w >= G || !out4) return (int)hipErrorInvalidValue;
-  int r[4];
-  me_split(G, w, I / 8, H / 16, g_me_w_even, g_me_w_odd, r);
+  int r[4], we, wo;
+  me_weights(H, ldgu, we, wo);
+  me_split(G, w, I / 8, H / 16, we, wo, r);
   for (int i = 0; i < 4; ++i) out4[i] = r[i];
   return 0;
 }
 
-// phase-A weights of workgroups on even / odd XCDs (A/B tooling: 1, 1 = the even split)
+RAGK_API int ragk_mlp_engine_split(int G, int w, int H, int I, int* out4) { return ragk_mlp_engine_rows_split(G, w, H, I, H, out4); }
+
+// phase-A weights of workgroups on even / odd XCDs (A/B tooling: 1, 1 = the even split; 0, 0 = by the rows' distance)
 RAGK_API int ragk_mlp_engine_set_xcd_weights(int we, int wo) {
-  if (we < 1 || wo < 1 || we > 1000 || wo > 1000) return (int)hipErrorInvalidValue;
+  if (we < 0 || wo < 0 || (we == 0) != (wo == 0) || we > 1000 || wo > 1000) return (int)hipErrorInvalidValue;
   g_me_w_even = we;
   g_me_w_odd = wo;
   return 0;
@@ -577,13 +592,14 @@ RAGK_API int ragk_mlp_engine_set_stamps(void* p) {
 RAGK_API int ragk_mlp_engine(const void* xn, const float* P, int S, const void* gamma, float eps, const void* wgu,
                              int ldgu, const void* wd, void* h, void* act, void* ctr, void* err, void* err_host, const void* tmo,
                              int M, int H, int I, int G, hipStream_t st) {
-  if (!ragk_mlp_engine_ok(M, H, I, G)) return (int)hipErrorInvalidValue;
-  if (!wgu || ldgu < H || ldgu % 8 || !wd || !h || !act || !ctr || !err || !tmo || (!xn && (!P || !gamma || S < 1 || H % 4)))
+  if (!ragk_mlp_engine_rows_ok(M, H, I, G, ldgu)) return (int)hipErrorInvalidValue;
+  if (!wgu || !wd || !h || !act || !ctr || !err || !tmo || (!xn && (!P || !gamma || S < 1 || H % 4)))
     return (int)hipErrorInvalidValue;
-  const bool gap = ldgu != H;  // (the XCDs' rates differ where rows lie 8 KB apart: 3 : 4 and 1 : 1 66.0 and 65.9 us, with the gap 68.4 and 65.7)
+  int we, wo;
+  me_weights(H, ldgu, we, wo);
   MlpArgs a{(const bf16_t*)xn, xn ? nullptr : P, (const bf16_t*)gamma, eps, S, (const bf16_t*)wgu,
             (const bf16_t*)wd, (bf16_t*)h, (bf16_t*)act, (unsigned long long*)ctr, (unsigned*)err,
-            (unsigned*)err_host, (const unsigned*)tmo, g_me_stamps, H, I, ldgu, gap ? 1 : g_me_w_even, gap ? 1 : g_me_w_odd};
+            (unsigned*)err_host, (const unsigned*)tmo, g_me_stamps, H, I, ldgu, we, wo};
   if (g_me_nt)
     hipLaunchKernelGGL(mlp_engine_kernel<true>, dim3(G), dim3(ME_THREADS), 0, st, a);
   else

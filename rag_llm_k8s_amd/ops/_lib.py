@@ -53,6 +53,8 @@ _SIGS = {
     "ragk_gemm_part_silu": [P, I, P, I, P, I, I, I, I, S],
     "ragk_gemm_part_silu_ok": [I, I, I, I],
     "ragk_mlp_engine_ok": [I, I, I, I],
+    "ragk_mlp_engine_rows_ok": [I, I, I, I, I],
+    "ragk_mlp_engine_rows_split": [I, I, I, I, I, P],
     "ragk_mlp_engine_set_nt": [I],
     "ragk_mlp_engine_set_stamps": [P],
     "ragk_mlp_engine_set_xcd_weights": [I, I],

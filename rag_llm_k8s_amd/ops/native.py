@@ -936,7 +936,7 @@ def mlp_engine_ok(M, w_gu, w_down):
     H, I = w_down.shape
     if w_gu.shape != (2 * I, H) or not (_vec_rows(w_gu) and w_gu.stride(1) == 1 and w_gu.stride(0) >= H and w_down.is_contiguous()):
         return False
-    return bool(_lib.lib().ragk_mlp_engine_ok(M, H, I, _cu_count()))
+    return bool(_lib.lib().ragk_mlp_engine_rows_ok(M, H, I, _cu_count(), w_gu.stride(0)))
 
 
 def mlp_engine(xn, w_gu, w_down, h):
@@ -962,9 +962,9 @@ def _mlp_engine_launch(xn_ptr, P_ptr, S, g_ptr, eps, w_gu, w_down, h):
     _req(h.shape == (1, H) and h.is_contiguous(), "h [1, H]")
     _req(mlp_engine_ok(1, w_gu, w_down), "mlp_engine shape")
     ws = _me_workspace(h.device, I)
-    check(_lib.lib().ragk_mlp_engine(xn_ptr, P_ptr, S, g_ptr, eps, w_gu.data_ptr(),
-                                     w_gu.stride(0), w_down.data_ptr(), h.data_ptr(), ws.act.data_ptr(), ws.words.data_ptr(), ws.err_ptr, ws.host_dev, ws.tmo_ptr, 1,
-                                     H, I, _cu_count(), stream_ptr()),
+    check(_lib.lib().ragk_mlp_engine(xn_ptr, P_ptr, S, g_ptr, eps, w_gu.data_ptr(), w_gu.stride(0), w_down.data_ptr(), h.data_ptr(),
+                                     ws.act.data_ptr(), ws.words.data_ptr(), ws.err_ptr, ws.host_dev, ws.tmo_ptr, 1, H, I,
+                                     _cu_count(), stream_ptr()),
           "ragk_mlp_engine")
     return h
 

@@ -21,6 +21,7 @@ def main():
     from rag_llm_k8s_amd import _build
     from rag_llm_k8s_amd.ops import native
     from rag_llm_k8s_amd.ops import reference as R
+    from rag_llm_k8s_amd.ops.pitch import pitched
 
     _build.build_hip()
     native.MLP_ENGINE = True
@@ -33,7 +34,7 @@ def main():
     for _ in range(L):
         g = (torch.randn(I, H, device=dev) / math.sqrt(H)).bfloat16()
         u = (torch.randn(I, H, device=dev) / math.sqrt(H)).bfloat16()
-        layers.append((R.pack_gate_up(g, u), (torch.randn(H, I, device=dev) / math.sqrt(I)).bfloat16()))
+        layers.append((pitched(R.pack_gate_up(g, u)), (torch.randn(H, I, device=dev) / math.sqrt(I)).bfloat16()))
         del g, u
     x = torch.randn(1, H, device=dev).bfloat16()
     h = torch.randn(1, H, device=dev).bfloat16()

@@ -109,8 +109,10 @@ def use_vocab(M, N, K, epi, gap=False):
     kernel, which reads the activations for every 16 columns, 58.6 -> 48.3, 32 rows: 65.7 -> 49.6). The register-streaming
     kernel keeps vocabularies from 32768 on below 8 rows (128256 x 4096 at 5 rows: 173 us against 184, at 8: 191 against 182) where
     the weight's rows lie without a gap between them (`gap`, ops/pitch.py; with it 32768 x 4096 at 1 / 4 / 7 rows 48 / 50 / 55 -> 43 / 43 / 43,
-    128256 x 4096 175 / 182 / 202 -> 159 / 159 / 160; in sums no longer than that kernel's, rms error 1.37e-7 on both sides)."""
-    return (epi == "none" and (1 if N < 32768 or gap else 8) <= M <= 64 and N >= STREAM_MIN_ROWS and N % 4 == 0
+    128256 x 4096 175 / 182 / 202 -> 159 / 159 / 160). It cuts K into eight sums; the slab's, over 256 up to K = 2048 and 512 from there
+    on, are no longer at multiples of 2048 (rms error in 1e-7, that kernel's and these, K = 2048 / 4096 / 6144 / 8192: 1.02 / 1.37 / 1.67 /
+    1.91 and 1.02 / 1.37 / 1.42 / 1.47) and would be in between (1024 / 3072: 0.81 / 1.20 and 0.94 / 1.34)."""
+    return (epi == "none" and (1 if N < 32768 or (gap and K % 2048 == 0) else 8) <= M <= 64 and N >= STREAM_MIN_ROWS and N % 4 == 0
             and K % 64 == 0)
 
 

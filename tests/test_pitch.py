@@ -72,6 +72,23 @@ def test_vocabulary_with_a_gap(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 4, 7])
+@pytest.mark.parametrize("K", [1024, 3072, 6144])
+def test_vocabulary_sums_with_a_gap_are_no_longer(M, K):
+    """Widths at which the weight stream would sum over more of K keep the dense weight's kernel, bit for bit."""
+    from rag_llm_k8s_amd.ops import native
+
+    x, w = _randn(M, K), _randn(32768, K, scale=K ** -0.5)
+    y, z = native.gemm(x, w, out_f32=True), native.gemm(x, _with_gap(w), out_f32=True)
+    if K % 2048:
+        assert torch.equal(y, z)
+    else:
+        ref = x.double() @ w.double().t()
+        err = [((t.double() - ref).norm() / ref.norm()).item() for t in (z, y)]
+        assert err[0] <= err[1] < 1e-6
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_embedding_rows_with_a_gap(dtype):
     from rag_llm_k8s_amd.ops import seq_native

@@ -492,9 +492,14 @@ def _fp8_halves(M, N, ks, S):
     two a CU, the last of which so leaves most of the chip without work. Us at 1 / 4 / 11 / 16 rows: 9216 x 4096 11.1 / 11.7 / 12.2 /
     12.6 -> 10.0 / 10.5 / 10.7 / 11.3, 18688 x 4096 20.7 / 21.6 / 22.3 / 22.7 -> 18.1 / 19.8 / 19.5 / 20.1, 7168 x 5120 11.4 / 11.9 /
     12.5 / 13.0 -> 10.0 / 10.5 / 11.1 / 11.7, 10240 x 8192 20.8 / 22.1 / 22.5 / 22.7 -> 18.6 / 22.6 / 21.4 / 21.5; in full rounds they
-    lose (12288 x 4096 13.6 against 15.0 at 11 rows). More rows read more of x for shorter slices: 18688 x 4096 at 17 21.8, 23.9."""
+    lose (12288 x 4096 13.6 against 15.0 at 11 rows). More rows read more of x for shorter slices: 18688 x 4096 at 17 21.8, 23.9.
+    At four to six rows of weights 8 KB and more apart the halves' gain shrinks with their number, as nowhere else: 8448 x 8192, 528
+    blocks, 19.5 / 19.5 / 19.6 -> 18.0 / 18.1 / 18.1, 576 of 9216 x 8192 and 4608 x 16384 19.8 / 19.8 / 19.9 -> 20.1 / 19.6 / 18.9 and 19.7 /
+    19.2 / 18.9, 640 of 10240 x 8192 and 5120 x 16384 20.5 / 20.6 / 20.8 against 21.3 / 21.4 / 21.0 (three and seven rows 20.3 -> 18.4,
+    20.8 -> 20.6; 576 of 6144 x 12288 and 640 of 20480 x 4096 gain 7 and 6 % there): they end at 0.6 of a round."""
     blocks = -(-N // 64) * S
-    return M <= 16 and ks in (16, 32) and blocks < 0.65 * -(-blocks // PART_MIN_BLOCKS) * PART_MIN_BLOCKS
+    most = 0.6 if 4 <= M <= 6 and 64 * ks * S % 8192 == 0 else 0.65
+    return M <= 16 and ks in (16, 32) and blocks < most * -(-blocks // PART_MIN_BLOCKS) * PART_MIN_BLOCKS
 
 
 def gemm_part_norm(h, gamma, eps, w, out=None, ks=None):

@@ -1,4 +1,4 @@
-"""Which split-K slabs a decode step's products take (ops/native.py _deep_slabs)."""
+"""Which split-K slabs a decode step's products take (ops/native.py _deep_slabs, _part_stream, _fp8_halves)."""
 import pytest
 from hypothesis import given, settings
 from hypothesis import strategies as st
@@ -20,3 +20,13 @@ def test_slabs_divide_the_product(N, steps, cus, few):
     rows, S = native._stream_part_cfg(N, steps * 64, cus, 0, 64)
     deep = native._deep_slabs(N, steps * 64, cus, 0, 64, few)
     assert deep == 0 or (deep > S >= 1 and deep <= 64 and steps % deep == 0 and steps // deep >= 14 and -(-N // rows) * S <= cus)
+
+
+@pytest.mark.parametrize("N,K,ks,rows", [
+    (10240, 8192, 32, [1, 3, 7, 16]), (5120, 16384, 32, [1, 3, 7, 16]), (9216, 8192, 32, [1, 4, 6, 16]), (8448, 8192, 32, [1, 4, 6, 16]),
+    (20480, 4096, 32, [1, 4, 6, 16]), (6144, 12288, 32, [1, 4, 6, 16]), (9216, 4096, 16, [1, 4, 6, 16]), (12288, 4096, 16, []),
+    (4096, 14336, 28, [])])
+def test_where_fp8_slices_are_halved(N, K, ks, rows):
+    tried = [1, 3, 4, 6, 7, 16, 17]
+    took = [M for M in tried if native._fp8_halves(M, N, ks, K // (64 * ks))]
+    assert took == [M for M in tried if rows and rows[0] <= M <= rows[-1] and (4 in rows or M not in (4, 6))]

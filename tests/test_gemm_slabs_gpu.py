@@ -127,10 +127,35 @@ def test_short_prompt(native, lens, monkeypatch):
     assert float((steps[0][0] - steps[1][0]).norm() / steps[1][0].norm()) < 2e-2
 
 
+def _llama_exact(m, ids, pos, lens):
+    """Last rows' logits of a Llama prompt batch in 64 bits, from the model's weights as they are (fp8 ones dequantised)."""
+    c, w, F = m.cfg, m.w, torch.float64
+    full = lambda t: t.dequant(F) if hasattr(t, "dequant") else t.to(F)
+    rms = lambda x, g: x * torch.rsqrt((x * x).mean(-1, keepdim=True) + c.rms_norm_eps) * g.to(F)
+    Hq, Hkv, D, T = m.Hq, m.Hkv, m.D, len(ids)
+    cos, sin = (torch.cat([t[pos].to(F)] * 2, -1)[:, None] for t in (m.cos, m.sin))
+    turn = lambda x: x * cos + torch.cat([-x[..., D // 2:], x[..., :D // 2]], -1) * sin
+    h = w.embed[ids].to(F)
+    for L in w.layers:
+        q, k, v = (rms(h, L["ln_in"]) @ full(L["wqkv"]).t()).view(T, -1, D).split([Hq, Hkv, Hkv], 1)
+        q, k, at, out = turn(q), turn(k), 0, []
+        for n in lens:
+            qs, ks, vs = q[at:at + n], *(t[at:at + n].repeat_interleave(Hq // Hkv, 1) for t in (k, v))
+            s = (qs.transpose(0, 1) @ ks.permute(1, 2, 0)) * D ** -0.5
+            s = s.masked_fill(torch.ones(n, n, dtype=torch.bool, device=DEV).triu(1), -torch.inf).softmax(-1)
+            out.append((s @ vs.transpose(0, 1)).transpose(0, 1).reshape(n, -1))
+            at += n
+        h = h + torch.cat(out) @ full(L["wo"]).t()
+        gu = (rms(h, L["ln_post"]) @ full(L["wgu"]).t()).view(T, -1, 2, 64)
+        h = h + (torch.nn.functional.silu(gu[:, :, 0]) * gu[:, :, 1]).reshape(T, -1) @ full(L["wdown"]).t()
+    last = [sum(lens[:i + 1]) - 1 for i in range(len(lens))]
+    return rms(h[last], w.norm) @ full(w.lm_head).t()
+
+
 @pytest.mark.parametrize("lens", [[13], [17], [7, 30, 27]])
 def test_short_prompt_fp8(native, lens, monkeypatch):
-    """From 13 tokens on fp8 prompts go in slabs: the logits are as far from the dequantised weights' in fp32 as with products of
-    rows, give or take their spread."""
+    """From 13 tokens on fp8 prompts go in slabs: the logits are as far from the dequantised weights' in 64 bits as with products
+    of rows, give or take their spread."""
     from rag_llm_k8s_amd.models import llama as L
     from rag_llm_k8s_amd.models.base import StepInput
     from rag_llm_k8s_amd.ops.backend import AttnMeta
@@ -163,6 +188,11 @@ def test_short_prompt_fp8(native, lens, monkeypatch):
     assert n == 0
     # two layers of sums in another order, rounded to bf16 (test_short_prompt)
     assert float((few - rows).norm() / rows.norm()) < 2e-2
+    ref = _llama_exact(m, torch.tensor(ids, device=DEV), torch.tensor(pos, device=DEV), lens)
+    err = [float((t - ref).norm() / ref.norm()) for t in (few, rows)]
+    print("fp8 prompt", lens, err)
+    # the error of one row's 512 logits is known to 3 % (one in sqrt(2 * 512)), the quotient of two such to 4.4 %; three of these
+    assert err[0] <= 1.13 * err[1] < 2e-2
 
 
 @pytest.mark.parametrize("M", [13, 16, 17, 33, 64])
@@ -179,7 +209,7 @@ def test_fp8_slabs_sum_as_closely(native, M, N, K):
     rows = native.gemm_fp8(x, q, out_f32=True).double()
     err = [float((y - ref).norm() / ref.norm()) for y in (slabs, rows)]
     print("fp8 slabs", M, N, K, err)
-    assert err[0] <= 1.1 * err[1]
+    assert err[0] <= err[1]
 
 
 # slabs of several rounds (one slab before, two of a wide product up to 32 rows), few rows whose register-streamed slices are long
@@ -194,6 +224,8 @@ def test_slabs_of_decode_products(native, monkeypatch, N, K, M):
     err = lambda P: float((P.double().sum(0) - ref).norm() / ref.norm())
     P = native.gemm_part(x, w)
     if M < native.STREAM_PART_MIN_M:
+        took = native._part_stream(M, N, K, native._cu_count(), native.STREAM_PART_MIN_M, 0, native.STREAM_PART_MAX_S, native.PART_MIN_BLOCKS)
+        assert took[1] and took[2] and torch.equal(P, native.gemm_stream_part(x, w, rows=took[0], S=took[1], short_sums=True))
         off = torch.cat([x.new_zeros(M, 4), x], 1)[:, 4:]  # rows off 16 bytes stay where they were
         assert torch.equal(native.gemm_part(x, w, ks=native.gemm_part_slabs(M, N, K)[0]), native.gemm_part(off, w))
         monkeypatch.setattr(native, "STREAM_PART", False)

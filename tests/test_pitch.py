@@ -57,18 +57,36 @@ def test_products_from_rows_with_a_gap(M):
         assert torch.equal(native.gemm_part(x, q), native.gemm_part(x, qp))
 
 
+# weights from 16384 rows on (the weight stream's gate/up and wide products), each of the rule's distances
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 5, 16, 17, 33, 64, 65, 300])
+@pytest.mark.parametrize("N,K", [(16384, 2048), (16512, 4096), (16384, 6144)])
+def test_wide_products_from_rows_with_a_gap(M, N, K):
+    from rag_llm_k8s_amd.ops import native
+
+    x, w = _randn(M, K), _randn(N, K, scale=K ** -0.5)
+    p, par = _with_gap(w), torch.tensor([2.0, 1.2, 0.5, 0.0], device=DEV)
+    assert native.use_stream(M, N // 2, K, "silu_mul") == native.use_stream(M, N // 2, K, "glu_clip") == (M <= 64)
+    for kw in (dict(), dict(epi="silu_mul"), dict(epi="glu_clip", bias=par)):
+        assert torch.equal(native.gemm(x, w, **kw), native.gemm(x, p, **kw)), kw
+        if kw.get("epi") and M <= 64:  # (some of these go to the held activations)
+            assert torch.equal(native.gemm(x, w, path=5, **kw), native.gemm(x, p, path=5, **kw)), kw
+    if M <= 64:
+        assert torch.equal(native.gemm_part(x, w), native.gemm_part(x, p))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 7, 8, 64])
 @pytest.mark.parametrize("N,K", [(32768, 2048), (32776, 4096)])
 def test_vocabulary_with_a_gap(M, N, K):
     """fp32 logits take the weight stream at any row count then, in sums no longer than the kernel's that dense rows take below
-    eight: its error against 64 bits, with a tenth of room for another order of the sums."""
+    eight: its error against 64 bits, give or take what a mean of 32768 squares says of it (0.4 %) and x, which they share."""
     from rag_llm_k8s_amd.ops import native
 
     x, w = _randn(M, K), _randn(N, K, scale=K ** -0.5)
     ref = x.double() @ w.double().t()
     err = [((native.gemm(x, t, out_f32=True).double() - ref).norm() / ref.norm()).item() for t in (w, _with_gap(w))]
-    assert err[1] <= 1.1 * err[0] < 1e-6
+    assert err[1] <= 1.03 * err[0] < 1e-6
 
 
 @pytest.mark.gpu
@@ -109,5 +127,7 @@ def test_mlp_engine_with_a_gap():
     p, x, h = _with_gap(w), _randn(1, H), _randn(1, H)
     if not native.mlp_engine_ok(1, w, d):
         pytest.skip("no MLP engine on this device")
-    assert native.mlp_engine_ok(1, p, d) and not native.mlp_engine_ok(1, p.t()[:, :H].t()[:, 1:], d)
+    off = lambda gap, start: torch.zeros(2 * I, H + gap, dtype=torch.bfloat16, device=DEV)[:, start:start + H]
+    assert native.mlp_engine_ok(1, p, d) and native.mlp_engine_ok(1, off(8, 0), d) and native.mlp_engine_ok(1, off(8, 8), d)
+    assert not native.mlp_engine_ok(1, off(8, 1), d) and not native.mlp_engine_ok(1, off(4, 0), d)  # rows off 16 bytes
     assert torch.equal(native.mlp_engine(x, w, d, h.clone()), native.mlp_engine(x, p, d, h.clone()))

@@ -24,7 +24,7 @@ from typing import List, Optional
 import torch
 
 from ..ops.backend import AttnMeta, get_backend  # noqa: F401
-from ..ops.pitch import pitched
+from ..ops.pitch import empty_rows, pitched
 from ..ops.reference import pack_gate_up, rope_tables
 from .base import DecoderModel, StepInput
 
@@ -148,8 +148,8 @@ class LlamaWeights:
             dn = get(p + "mlp.down_proj.weight", cols=(r * I, (r + 1) * I))
             w.layers.append(dict(
                 ln_in=dev(get(p + "input_layernorm.weight")), ln_post=dev(get(p + "post_attention_layernorm.weight")),
-                wqkv=dev(torch.cat([q, k, v], 0)), wo=dev(o), wgu=pitched(dev(pack_gate_up(gt, up))),
-                wdown=dev(dn)))
+                wqkv=dev(torch.cat([q, k, v], 0)), wo=dev(o),
+                wgu=pack_gate_up(gt, up, out=empty_rows(2 * I, gt.shape[1], dtype, device)), wdown=dev(dn)))
         w.norm = dev(get("model.norm.weight"))
         V = cfg.vocab_size
         lo, hi = r * Vl, min(V, (r + 1) * Vl)
@@ -157,7 +157,7 @@ class LlamaWeights:
         lm = get(name, rows=(lo, hi))
         if lm.shape[0] < Vl:  # pad the last vocab shard
             lm = torch.cat([lm, torch.zeros(Vl - lm.shape[0], lm.shape[1], dtype=lm.dtype, device=lm.device)], 0)
-        w.lm_head = dev(lm) if cfg.tie_word_embeddings else pitched(dev(lm))  # (a tied one shares its memory)
+        w.lm_head = dev(lm) if cfg.tie_word_embeddings else pitched(dev(lm))  # (a tied one may lie in the embedding's memory)
         w.vocab_offset = lo
         w.vocab_valid = hi - lo
         return w

@@ -27,13 +27,17 @@ def wants_gap(rows, row_bytes, itemsize):
     return itemsize == 2 and row_bytes in ROW_BYTES and rows * row_bytes >= MIN_BYTES
 
 
+def empty_rows(rows, columns, dtype, device):
+    """A weight to be filled, laid out as pitched() does it."""
+    size = dtype.itemsize
+    gap = torch.device(device).type == "cuda" and dtype.is_floating_point and wants_gap(rows, columns * size, size)
+    return torch.empty((rows, columns + gap * GAP // size), dtype=dtype, device=device)[:, :columns]
+
+
 def pitched(w):
     """The weight [rows, columns], or a copy of it whose rows lie GAP bytes further apart, where its products read that faster."""
     size = w.element_size()
     if not (w.is_cuda and w.dim() == 2 and w.is_contiguous() and w.is_floating_point()
             and wants_gap(w.shape[0], w.shape[1] * size, size)):
         return w
-    buf = torch.empty((w.shape[0], w.shape[1] + GAP // size), dtype=w.dtype, device=w.device)
-    out = buf[:, :w.shape[1]]
-    out.copy_(w)
-    return out
+    return empty_rows(*w.shape, w.dtype, w.device).copy_(w)

@@ -19,13 +19,18 @@ EPI = {"none": 0, "bias": 1, "resid": 2, "bias_resid": 3, "bias_gelu": 4, "silu_
        "bias_gelu_tanh": 7, "glu_clip": 9}
 
 
-def pack_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
+def pack_gate_up(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """Pack [I,K] gate and up weights into the kernel layout: 128-row tiles of
-    [64 gate rows | 64 up rows]. Requires I % 64 == 0."""
+    [64 gate rows | 64 up rows]. Requires I % 64 == 0. out: where to (rows may have gaps, on any device, in any type)."""
     I, K = gate.shape
     assert up.shape == gate.shape and I % 64 == 0, (gate.shape, up.shape)
     g = gate.reshape(I // 64, 64, K)
     u = up.reshape(I // 64, 64, K)
+    if out is not None:
+        t = out.view(I // 64, 2, 64, K)
+        t[:, 0].copy_(g)
+        t[:, 1].copy_(u)
+        return out
     return torch.stack([g, u], dim=1).reshape(2 * I, K).contiguous()
 
 

@@ -29,6 +29,29 @@ def _randn(*shape, scale=1.0):
     return (torch.randn(*shape, generator=g, device=DEV) * scale).bfloat16()
 
 
+def test_gate_and_up_rows_packed_in_place():
+    from rag_llm_k8s_amd.ops.reference import pack_gate_up
+
+    g, u = torch.randn(192, 40), torch.randn(192, 40)
+    for out in (torch.zeros(384, 40), torch.full((384, 104), 7.0)[:, :40], torch.zeros(384, 40, dtype=torch.bfloat16)):
+        assert pack_gate_up(g, u, out=out) is out and torch.equal(out, pack_gate_up(g, u).to(out.dtype))
+    assert pitch.empty_rows(32768, 2048, torch.bfloat16, "cpu").is_contiguous()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("source", ["cpu", DEV])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_loaded_gate_and_up_rows(source, dtype):
+    """Into rows with a gap from any device and type, and nowhere else."""
+    from rag_llm_k8s_amd.ops.reference import pack_gate_up
+
+    g, u = torch.randn(8192, 2048).to(source, dtype), torch.randn(8192, 2048).to(source, dtype)
+    out = pitch.empty_rows(16384, 2048, torch.bfloat16, DEV)
+    whole = out.as_strided((16384, 2112), (2112, 1)).fill_(7.0)
+    assert out.stride() == (2112, 1) and torch.equal(pack_gate_up(g, u, out=out), pack_gate_up(g, u).to(DEV, torch.bfloat16))
+    assert bool((whole[:, 2048:] == 7.0).all())
+
+
 @pytest.mark.gpu
 def test_pitched_copy():
     w = _randn(16384, 2048)

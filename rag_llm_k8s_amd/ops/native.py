@@ -591,9 +591,8 @@ def _deep_slabs(N, K, cus, only, max_s, few):
 
 
 @functools.lru_cache(maxsize=4096)
-def _part_stream(M, N, K, cus, min_m, only, max_s, min_blocks, gap=False):
-    """(rows, S, whether in short sums) of gemm_part's bf16 products on the LDS-DMA weight stream, S 0: gemm_part.hip's. gap: the
-    weight's rows do not lie back to back (ops/pitch.py).
+def _part_stream(M, N, K, cus, min_m, only, max_s, min_blocks):
+    """(rows, S, whether in short sums) of gemm_part's bf16 products on the LDS-DMA weight stream, S 0: gemm_part.hip's.
 
     Below STREAM_PART_MIN_M rows they go there only where gemm_part.hip's slices are 28 K-steps long and more, in sums over 512 of K,
     which are no further off (1 / 4 rows, us and rms error in 1e-7: 4096 x 14336 24.9 / 25.2, 1.7 -> 22.0 / 22.0, 1.3; 18688 x 4096
@@ -608,18 +607,8 @@ def _part_stream(M, N, K, cus, min_m, only, max_s, min_blocks, gap=False):
         ks = _part_ksteps(M, N, K, min_blocks)
         if ks < 28 or (K % 8192 == 0 and -(-N // 64) * (K // (64 * ks)) % (2 * cus) == 0):
             return 0, 0, False
-    rows, S = _stream_part_cfg(N, K, cus, only, max_s)
     deep = _deep_slabs(N, K, cus, only, max_s, M <= 32)
-    # one round of more than 0.6 blocks a CU is ahead of these where rows are many: 160 blocks (20480 rows of weights) at 24 / 33 / 64
-    # rows -7 / -2 / +4 % at K = 4096 and -6 / 0 / +4 at 5120 in four slabs, in eight +1 / +2 / +6 at 8192, +5 / +7 / +7 at 7168 (12 rows
-    # -1 and 0); 152 blocks of 19456 x 8192 -2 / -1 / +2
-    if deep and S == 1 and -(-N // 128) > 0.6 * cus and M > (32 if deep <= 4 else 12):
-        deep = 0
-    # and so is one round of short slices up to 16 rows where the rows' gap lets it stream (5 / 8 / 16 / 17 rows: 9216 x 4096 +3 / +2 / +1 /
-    # -3 %, 18688 x 2048 +3 / +2 / 0 / -3, 9216 x 6144 +3 / +2 / 0 / -3, but 8448 x 5120 without a gap -1 / -2 / -4 / -7)
-    if deep and gap and M <= 16 and K // 64 // S <= 48:
-        deep = 0
-    return (64, deep, True) if deep else (rows, S, few)
+    return (64, deep, True) if deep else _stream_part_cfg(N, K, cus, only, max_s) + (few,)
 
 
 def gemm_stream_part(x, w, out=None, rows=None, S=None, short_sums=False):
@@ -660,8 +649,7 @@ def gemm_part(x, w, out=None, ks=None, short_sums=False):
     N = wt.shape[0]
     _req(wt.shape[1] == K and M <= 64, "gemm_part shape %s x %s" % (tuple(x.shape), tuple(wt.shape)))
     if STREAM_PART and not fp8 and ks is None and out is None:
-        rows, S, short = _part_stream(M, N, K, _cu_count(), STREAM_PART_MIN_M, STREAM_PART_ROWS, STREAM_PART_MAX_S, PART_MIN_BLOCKS,
-                                      wt.stride(0) != K)
+        rows, S, short = _part_stream(M, N, K, _cu_count(), STREAM_PART_MIN_M, STREAM_PART_ROWS, STREAM_PART_MAX_S, PART_MIN_BLOCKS)
         if S > 0 and (M >= STREAM_PART_MIN_M or _vec_rows(x, wt)):
             return gemm_stream_part(x, wt, rows=rows, S=S, short_sums=short_sums or short)
     if fp8 and ks is None and out is None and use_hold_slabs(M, N, K) and _vec_rows(x, wt) and wt.stride(0) < 1 << 24:

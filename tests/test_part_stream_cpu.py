@@ -30,20 +30,3 @@ def test_where_fp8_slices_are_halved(N, K, ks, rows):
     tried = [1, 3, 4, 6, 7, 16, 17]
     took = [M for M in tried if native._fp8_halves(M, N, ks, K // (64 * ks))]
     assert took == [M for M in tried if rows and rows[0] <= M <= rows[-1] and (4 in rows or M not in (4, 6))]
-
-
-@pytest.mark.parametrize("N,K,gap,M,took", [
-    # slices of 28 K-steps and more of a few rows, shorter ones, whole rounds of rows 16 KB apart
-    (4096, 14336, False, 1, (128, 8, True)), (4096, 14336, False, 4, (128, 8, True)), (4096, 14336, False, 5, (128, 8, False)),
-    (6144, 4096, False, 4, (0, 0, False)), (18688, 2048, True, 4, (0, 0, False)), (9728, 5120, False, 4, (0, 0, False)),
-    (8192, 8192, False, 4, (0, 0, False)), (4096, 16384, False, 4, (0, 0, False)), (16384, 8192, False, 1, (0, 0, False)),
-    (8192, 8192, False, 5, (128, 4, False)), (10240, 8192, False, 4, (64, 8, True)), (8192, 12288, False, 4, (128, 4, True)),
-    # several rounds of short slices: by rows, by how full one round is, with a gap
-    (18688, 4096, True, 1, (64, 4, True)), (18688, 4096, True, 64, (64, 4, True)), (20480, 4096, True, 32, (64, 4, True)),
-    (20480, 4096, True, 33, (128, 1, False)), (20480, 8192, False, 12, (64, 8, True)), (20480, 8192, False, 13, (128, 1, False)),
-    (19456, 8192, False, 64, (64, 8, True)), (9216, 4096, True, 16, (128, 2, False)), (9216, 4096, True, 17, (64, 4, True)),
-    (9216, 4096, False, 16, (64, 4, True)), (9216, 4096, True, 33, (128, 2, False)), (18688, 2048, True, 16, (128, 1, False)),
-    (18688, 2048, True, 17, (64, 2, True)), (18688, 2048, False, 5, (64, 2, True)), (18688, 6144, True, 5, (64, 4, True)),
-    (4098, 14336, False, 5, (0, 0, False))])
-def test_where_decode_products_go(N, K, gap, M, took):
-    assert native._part_stream(M, N, K, 256, 5, 0, 64, 512, gap) == took

@@ -30,3 +30,15 @@ def test_where_fp8_slices_are_halved(N, K, ks, rows):
     tried = [1, 3, 4, 6, 7, 16, 17]
     took = [M for M in tried if native._fp8_halves(M, N, ks, K // (64 * ks))]
     assert took == [M for M in tried if rows and rows[0] <= M <= rows[-1] and (4 in rows or M not in (4, 6))]
+
+
+@pytest.mark.parametrize("N,K,M,took", [
+    # slices of 28 K-steps and more of a few rows, shorter ones, whole rounds of rows 16 KB apart
+    (4096, 14336, 1, (128, 8, True)), (4096, 14336, 4, (128, 8, True)), (4096, 14336, 5, (128, 8, False)), (6144, 4096, 4, (0, 0, False)),
+    (18688, 2048, 4, (0, 0, False)), (9728, 5120, 4, (0, 0, False)), (8192, 8192, 4, (0, 0, False)), (4096, 16384, 4, (0, 0, False)),
+    (16384, 8192, 1, (0, 0, False)), (8192, 8192, 5, (128, 4, False)), (10240, 8192, 4, (64, 8, True)), (8192, 12288, 4, (128, 4, True)),
+    # several rounds of short slices
+    (18688, 4096, 1, (64, 4, True)), (18688, 4096, 64, (64, 4, True)), (20480, 8192, 33, (64, 8, True)), (9216, 4096, 32, (64, 4, True)),
+    (9216, 4096, 33, (128, 2, False)), (18688, 2048, 5, (64, 2, True)), (18688, 6144, 5, (64, 4, True)), (4098, 14336, 5, (0, 0, False))])
+def test_where_decode_products_go(N, K, M, took):
+    assert native._part_stream(M, N, K, 256, 5, 0, 64, 512) == took

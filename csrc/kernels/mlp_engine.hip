@@ -524,8 +524,8 @@ __global__ __launch_bounds__(ME_THREADS, 1) void mlp_engine_kernel(MlpArgs a) {
 int g_me_nt = 1;
 // measured per-XCD rate ratio ~0.84; for Llama-3.1-8B on 256 CUs (7 groups per workgroup on average)
 // 27 : 32 and 3 : 4 give the same integer split, 6 : 8 groups (profiles/mlp_engine_xcd_weights_r5.log)
-// where rows lie 8 KB apart; with a gap between them the even split is as good or better (3 : 4 and 1 : 1, us: dense 66.0 and 65.9,
-// gap 68.4 and 65.7, on another card 64.9 and 64.7)
+// where rows lie 8 KB apart; with a gap between them the even split is never far from the best (3 : 4 and 1 : 1, us: dense 66.0 and
+// 65.9, gap 68.4 and 65.7; on another card dense 64.1 and 65.1, gap 64.4 and 64.6)
 int g_me_w_even = 0, g_me_w_odd = 0;  // 0: by the rows' distance
 unsigned long long* g_me_stamps = nullptr;
 

@@ -225,6 +225,7 @@ class LlamaWeights:
         return self
 
     def nbytes(self):
+        """Bytes of the values, which a step reads (ops/pitch.py's gaps, 1 to 3 % of the large weights, hold none)."""
         t = [self.embed, self.norm, self.lm_head] + [v for l in self.layers for v in l.values()]
         return sum(x.nbytes() if hasattr(x, "dequant") else x.numel() * x.element_size() for x in t)
 
@@ -308,8 +309,8 @@ class LlamaModel(DecoderModel):
         return M <= DECODE_DOWN_SKINNY_MAX_M and not self._tp() and self.be.part_norm_ok(M, self.w.layers[0]["wqkv"])
 
     def hidden_states_decode_part(self, inp: StepInput, hn):
-        """hn: the embedded rows and, unless _norm_fused, their norm for the first layer. Decode step with the split-K partial GEMM (csrc/kernels/gemm_part.hip) for the three
-        small-N projections: qkv / o_proj / down write fp32 partial slabs and the following row
+        """hn: the embedded rows and, unless _norm_fused, their norm for the first layer.
+        Decode step with the split-K partial GEMM (csrc/kernels/gemm_part.hip) for the three small-N projections: qkv / o_proj / down write fp32 partial slabs and the following row
         kernel reduces them -- rope_kv_partials (qkv) and add_partials_rmsnorm (o_proj -> post-attention
         norm, down -> next layer's input norm / the final norm), so the reduction adds no launch and
         the GEMMs stream their weights with every load in flight (qkv 26.7 -> 15 us, o_proj 15 -> 11.6,

@@ -520,7 +520,9 @@ class NativeBackend(TorchBackend):
         # lies between the two, and long projections of many rows below it forgo the GPU's gain.
         # One byte a weight: whole products read the activations once a few columns, so they cost by rows, slabs hardly (four layers
         # 4096 wide, 5 / 9 / 16 / 17 / 24 / 33 / 48 / 64 tokens 372 / 387 / 428 / 473 / 524 / 656 / 749 / 869 us in rows, 397 / 392 / 393 / 399 /
-        # 397 / 418 / 443 / 489 in slabs); the line lies where the two cross.
+        # 397 / 418 / 443 / 489 in slabs); the line lies where the two cross. Wider ones cross earlier (13 / 17 / 33 / 64 tokens, 5120 514 /
+        # 654 / 1143 / 1481 -> 418 / 481 / 700 / 826, 6144 663 / 758 / 1152 / 1561 -> 558 / 527 / 576 / 670, 8192 1182 / 1279 / 1987 / 2688 ->
+        # 1033 / 892 / 969 / 1113; 9 tokens of these 472 -> 409, 602 -> 528, 1068 -> 979).
         if isinstance(w, Fp8Weight):
             return 12 < M <= 64 and w.shape[0] * w.shape[1] >= 1 << 24 and self.part_ok(M, w)
         if w.dtype != torch.bfloat16:

@@ -579,7 +579,10 @@ def _deep_slabs(N, K, cus, only, max_s, few):
     33.4 / 33.3 / 37.8 -> 26.5 / 26.8 / 30.6 / 35.2, 18688 x 8192 69 / 68 / 72 / 78 -> 62 / 62 / 70 / 76, 18688 x 2048 18.9 / 20.1 /
     22.6 / 25.8 -> 17.8 / 17.7 / 19.4 / 22.0; two slabs only up to 32 rows (`few`): 10240 x 8192 38.2 / 39.3 / 38.2 / 41.8 -> 35.4 /
     35.7 / 39.1 / 42.5, 9216 x 4096 18.8 / 20.0 -> 17.8 / 17.6. From 22528 x 4096 on one round is ahead at 33 rows (36.0 against
-    38.6), and at half-full slices of 16 steps always (9344 x 2048 10.8 against 11.3)."""
+    38.6), and at half-full slices of 16 steps always (9344 x 2048 10.8 against 11.3). At the rule's edge, 20480 rows of weights, the two
+    change places from run to run from 24 rows on (x 8192 at 24 / 64 rows +1 / +6 and -3 / -1 %, x 4096 -7 / +4 and -7 / +5); rows with a gap
+    stream better in one round (5 / 8 / 16 / 17 rows of 9216 x 4096 +3 / +2 / +1 / -3 %, 18688 x 2048 +3 / +2 / 0 / -3). Both keep several,
+    whose sums are two to four times as close (1.3 and 0.95e-7 against 2.7e-7); one round in short sums takes up to 12 % more."""
     rows, S = _stream_part_cfg(N, K, cus, only, max_s)
     steps = K // 64
     if rows != 128 or -(-N // 128) * S > 0.64 * cus or steps // S < 32 or not (S == 1 or (S == 2 and few)):
@@ -598,7 +601,8 @@ def _part_stream(M, N, K, cus, min_m, only, max_s, min_blocks):
     which are no further off (1 / 4 rows, us and rms error in 1e-7: 4096 x 14336 24.9 / 25.2, 1.7 -> 22.0 / 22.0, 1.3; 18688 x 4096
     35.3 / 35.8, 1.9 -> 28.2 / 27.1, 1.3; 8192 x 28672 92.5 / 93.8, 1.8 -> 75 / 75, 1.4; 6144 x 14336 44 -> 32). Shorter slices are as
     fast there, in shorter sums, and so are whole rounds of two blocks a CU over rows a multiple of 16 KB apart (8192 x 8192 31.3
-    against 32.6, 4096 x 16384 32.5 against 34.8, 16384 x 8192 56 against 66, but 10240 x 8192 in 1.25 rounds 39 -> 36). Slabs of
+    against 32.6, 4096 x 16384 32.5 against 34.8, 8192 x 16384 61 against 64, 16384 x 8192 56 against 66, but 10240 x 8192 in 1.25 rounds
+    39 -> 36, 17408 x 8192 in 1.1 63 -> 59; such rows never have a gap, ops/pitch.py). Slabs of
     _deep_slabs are short sums, too: 18688 x 4096 in one 3.9e-7, in four of 1024 1.8, of 512 1.3, for 0 to 3 % of the time."""
     few = M < min_m
     if K % 64 or N % 4:

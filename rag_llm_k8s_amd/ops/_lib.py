@@ -197,6 +197,21 @@ def lib():
         return h
 
 
+_held = {}
+
+
+def held(name):
+    """The library's function `name`, called without giving up the interpreter lock: for the first of several short calls that belong
+    together, where a thread of plain Python would keep the lock for its 5 ms after each."""
+    fn = _held.get(name)
+    if fn is None:
+        like = getattr(lib(), name)
+        fn = getattr(ctypes.PyDLL(lib()._name, mode=ctypes.RTLD_GLOBAL), name)
+        fn.argtypes, fn.restype = like.argtypes, like.restype
+        _held[name] = fn
+    return fn
+
+
 def _check_mirrors(h):
     """The structs that cross as pointers have the size that the library was compiled with (a partial one may lack them)."""
     for mirror, size in ((EncoderCall, "ragk_encoder_call_bytes"),):

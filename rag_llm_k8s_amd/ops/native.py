@@ -1441,7 +1441,8 @@ def _encoder_call(cfg, weights, bufs, at, T, B):
 
 # Layers whose weights are checked and whose launches are made at a time: the device begins behind the first three's, not behind all
 # (4 us of checks a layer, 15 to 27 of launches and kernels). A call of one text, waited for, us: 24 layers of 1024, 5 / 16 tokens
-# 748 / 836 -> 645 / 734; 6 of 384, 14 / 30 tokens 164 / 203 -> 164 / 184. Calls behind each other 119 / 560 on both sides.
+# 748 / 836 -> 645 / 734; 6 of 384, 14 / 30 tokens 164 / 203 -> 164 / 184. Calls behind each other 119 / 560 on both sides. The last
+# call alone gives up the interpreter lock, as the one call for all layers did.
 FEW_LAYERS = 3
 
 
@@ -1469,7 +1470,8 @@ def encoder_few(cfg, w, ids, first_pos, out):
         c.ids_host = ids.ctypes.data
     c.l1 = min(n, FEW_LAYERS)
     while True:
-        check(_lib.lib().ragk_encoder_forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
+        forward = _lib.lib().ragk_encoder_forward if c.l1 == n else _lib.held("ragk_encoder_forward")
+        check(forward(ctypes.byref(c), stream_ptr()), "ragk_encoder_forward")
         if c.l1 == n:
             return True
         c.l0, c.l1 = c.l1, min(n, c.l1 + FEW_LAYERS)

@@ -129,6 +129,30 @@ def test_layers_in_several_calls(native, monkeypatch, layers):
     assert ((out.to(F64) - ref).norm() / ref.norm()).item() < 0.01  # (test_short_sequence; a layer's roundings grow with their number)
 
 
+@pytest.mark.parametrize("layers,calls", [(2, 0), (3, 0), (4, 1), (24, 7)])
+def test_the_last_call_alone_gives_up_the_interpreter_lock(native, monkeypatch, layers, calls):
+    """A thread of plain Python keeps the lock for 5 ms each time it is given up: once for all layers, not every three."""
+    cfg = E.EncoderConfig(model_type="bert", vocab_size=500, hidden_size=128, num_hidden_layers=layers, num_attention_heads=4,
+                          intermediate_size=256, max_position_embeddings=64, pooling="mean")
+    m = E.EncoderModel(cfg, E.EncoderWeights.random(cfg, DEV, seed=2), DEV)
+    ids, row, lens, out = np.arange(5, 17, dtype=np.int32), np.array([0]), np.array([12], dtype=np.int64), torch.zeros(1, 128, device=DEV)
+    python_api, real, took = 4, native._lib.lib(), []  # ctypes' flag of functions that keep the lock
+
+    class Watched:
+        def __getattr__(self, name):
+            if name == "ragk_encoder_forward":
+                took.append("given up")
+            return getattr(real, name)
+
+    held = native._lib.held
+    monkeypatch.setattr(native._lib, "held", lambda name: (took.append("held"), held(name))[1])
+    held("ragk_encoder_forward")
+    monkeypatch.setattr(native._lib, "lib", Watched)
+    m.embed_into(ids, lens, out, row)
+    assert took == ["held"] * calls + ["given up"] and bool(out.any())
+    assert held("ragk_encoder_forward")._flags_ & python_api and not real.ragk_encoder_forward._flags_ & python_api
+
+
 def test_a_weight_of_a_later_call_that_is_not_taken(native):
     """Launches made by then are given up, and the layers go through the checked entry points."""
     cfg = E.EncoderConfig(model_type="bert", vocab_size=500, hidden_size=128, num_hidden_layers=5, num_attention_heads=4,
